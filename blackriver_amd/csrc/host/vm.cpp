@@ -337,10 +337,10 @@ void Enviroment::insert_native_word(const std::string& name, NativeCreator* fn) 
     native_words_[name] = fn;
 }
 
-void Enviroment::insert_fusion(const std::vector<std::string>& sequence, const std::string& fused) {
+void Enviroment::insert_fusion(const std::vector<std::string>& sequence, const std::string& fused, bool across_scopes) {
     br_assert(sequence.size() >= 2, "a fusion needs at least two words");
     br_assert(native_words_.count(fused) != 0, "the fused word must be registered first");
-    fusions_.emplace_back(sequence, fused);
+    fusions_.push_back(Fusion{sequence, fused, across_scopes});
 }
 
 // Peephole pass over a linked program (see insert_fusion).
@@ -349,7 +349,7 @@ void Enviroment::fuse(DaG& dag) {
         return s.kind == DaG::Step::PushString || (s.kind == DaG::Step::RunBuiltin && s.str == "@");
     };
     for (const auto& fusion : fusions_) {
-        const std::vector<std::string>& seq = fusion.first;
+        const std::vector<std::string>& seq = fusion.sequence;
         for (size_t i = 0; i < dag.steps_.size(); i++) {
             if (dag.steps_[i].kind != DaG::Step::RunNative || dag.steps_[i].str != seq[0]) continue;
             std::vector<size_t> at{i};
@@ -358,7 +358,7 @@ void Enviroment::fuse(DaG& dag) {
                 const DaG::Step& s = dag.steps_[pc];
                 if (s.kind == DaG::Step::RunNative && s.str == seq[at.size()]) {
                     at.push_back(pc);
-                } else if (s.kind == DaG::Step::PushNumber && pc + 1 < dag.steps_.size() &&
+                } else if (fusion.across_scopes && s.kind == DaG::Step::PushNumber && pc + 1 < dag.steps_.size() &&
                            dag.steps_[pc + 1].kind == DaG::Step::RunBuiltin && dag.steps_[pc + 1].str == "#") {
                     pc++;   // `n #`: a switch of the name scope
                 } else if (!is_push(s)) {
@@ -369,9 +369,9 @@ void Enviroment::fuse(DaG& dag) {
             if (at.size() != seq.size()) continue;
             for (size_t k = 0; k + 1 < at.size(); k++) dag.steps_[at[k]].kind = DaG::Step::Skip;
             DaG::Step& last = dag.steps_[at.back()];
-            last.str = fusion.second;
+            last.str = fusion.fused;
             last.idx = dag.natives_.size();
-            dag.natives_.push_back(native_words_[fusion.second](*this));
+            dag.natives_.push_back(native_words_[fusion.fused](*this));
             i = at.back();
         }
     }

@@ -217,13 +217,13 @@ struct Enviroment {
     void insert_native_word(const std::string& name, NativeCreator* fn);
     // Registers a fusion: wherever a linked program runs the native words
     // `sequence` one after the other with nothing but operand pushes
-    // (strings and `@`) and switches of the name scope (`n #`, which
+    // (strings and `@`) and, where `across_scopes`, switches of the name scope (`n #`, which
     // neither touch a tensor nor leave anything on the stack: operands
     // already pushed are tensors, not names) in between, the earlier words are skipped -- their
     // operands simply stay on the stack -- and the last one is replaced by
     // `fused`, which pops the operands of the whole sequence (first word's
     // deepest) and must produce exactly what the sequence would have.
-    void insert_fusion(const std::vector<std::string>& sequence, const std::string& fused);
+    void insert_fusion(const std::vector<std::string>& sequence, const std::string& fused, bool across_scopes = false);
 
     // compile + link; the caller owns the result and runs it with run()
     DaG* build(const std::string& txt);
@@ -252,7 +252,12 @@ private:
 
     std::map<std::string, UserWord> user_words_;
     std::map<std::string, NativeCreator*> native_words_;
-    std::vector<std::pair<std::vector<std::string>, std::string>> fusions_;
+    struct Fusion {
+        std::vector<std::string> sequence;
+        std::string fused;
+        bool across_scopes;
+    };
+    std::vector<Fusion> fusions_;
     Stack stack_;
     std::vector<Hash> hashes_;
     size_t target_;

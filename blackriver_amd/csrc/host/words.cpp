@@ -530,7 +530,8 @@ void load_nn_words(Enviroment& env) {
     env.insert_fusion({"op.add", "op.add", "op.softmax"}, "op.add_add_softmax");
     env.insert_fusion({"op.layernorm", "op.copy"}, "op.layernorm_copy");
     env.insert_fusion({"op.gelu_backward", "op.linear_backward"}, "op.gelu_linear_backward");
-    env.insert_fusion({"op.layernorm_backward_add", "op.linear_backward"}, "op.layernorm_backward_add_linear_backward");
+    // the pair also stands across a block boundary of a model program
+    env.insert_fusion({"op.layernorm_backward_add", "op.linear_backward"}, "op.layernorm_backward_add_linear_backward", true);
 }
 
 }  // namespace br
