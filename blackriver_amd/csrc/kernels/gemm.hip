@@ -3,11 +3,12 @@
 //   C[b][i,j] = alpha * sum_p opA[b][i,p] * opB[b][p,j] (+ C) (+ bias[j])
 //
 // 16-bit multiplicands (fp16 / bf16, fp32 accumulation) go to the kernel
-// templates in gemm_dtl16.hpp (both operands stored in the MFMA type, aligned:
-// direct-to-LDS loads) and gemm_mfma16.hpp (everything else: fp32 operands
-// converted on load, ragged sizes).  This file holds the argument checking,
-// the staging of fp32 operands into a caller's workspace so that they too can
-// take the direct-to-LDS kernel, and the kernel that keeps fp32 operands and
+// templates in gemm_dtl16.hpp and gemm_flex16.hpp (both operands stored in the
+// MFMA type, aligned: direct-to-LDS loads; gemm_plan.hpp chooses between them)
+// and gemm_mfma16.hpp (fp32 operands converted on load, unaligned rows).  This
+// file holds the argument checking, the staging of fp32 and of unaligned
+// operands into a caller's workspace so that they too can take the
+// direct-to-LDS kernels, and the kernel that keeps fp32 operands and
 // multiplies with v_mfma_f32_32x32x2_f32 for callers that need fp32-faithful
 // products (128x128x16 tiles, 4 wave64s x 2x2 MFMA blocks, register prefetch +
 // LDS double buffering).
@@ -23,8 +24,14 @@
 using namespace brk;
 
 namespace brk {
-int gemm16_launch_f16(const gemm16::GemmArgs& g, const gemm16::Problem& p, long long batch, hipStream_t st);
-int gemm16_launch_bf16(const gemm16::GemmArgs& g, const gemm16::Problem& p, long long batch, hipStream_t st);
+#define BR_GEMM16_ENTRIES(T)                                                                                             \
+    int gemm16_tiles_##T(const gemm16::GemmArgs& g, const gemm16::Problem& p, int kernel, long long batch, hipStream_t st);  \
+    int gemm16_pair_##T(const gemm16::GemmArgs& g, const gemm16::Problem& p, int kernel, int slot, hipStream_t st);          \
+    int gemm16_ragged_##T(const gemm16::GemmArgs& g, const gemm16::Problem& p, int kernel, long long batch, hipStream_t st); \
+    int gemm16_registers_##T(const gemm16::GemmArgs& g, const gemm16::Problem& p, long long batch, hipStream_t st);
+BR_GEMM16_ENTRIES(f16)
+BR_GEMM16_ENTRIES(bf16)
+#undef BR_GEMM16_ENTRIES
 }  // namespace brk
 
 namespace {
@@ -195,11 +202,47 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma32_kernel(GemmArgs g) {
 
 long long elem_size(int dtype) { return dtype == BR_F32 ? 4 : 2; }
 
-// br_hip_gemm with the tensor an accumulating product adds to named separately (null = c itself).
+// A 16-bit product by its plan, operands already checked by dtl_applies.  g.splits > 1: slices of K as batch entries.
+int run_plan(GemmArgs g, const gemm16::Problem& p, const gemm16::Plan& plan, long long batch, int compute, hipStream_t st) {
+    using namespace gemm16;
+    const bool f16 = compute == BR_GEMM_F16;
+    if (plan.pair && g.partials) {
+        const int slot = split_slot_of(st);
+        if (slot >= 0) return f16 ? gemm16_pair_f16(g, p, plan.kernel, slot, st) : gemm16_pair_bf16(g, p, plan.kernel, slot, st);
+    }
+    if (plan.tail_from > 0) {
+        // whole rounds of 256x256 tiles, then the columns left over on 256x128 tiles (see column_tail)
+        GemmArgs head = g, tail = g;
+        head.n = plan.tail_from;
+        const size_t c_size = (size_t)elem_size(p.c_dtype);
+        tail.n = g.n - plan.tail_from;
+        tail.b = static_cast<const unsigned char*>(g.b) + 2 * (p.b_kstr ? plan.tail_from : plan.tail_from * g.ldb);
+        tail.c = static_cast<unsigned char*>(g.c) + c_size * plan.tail_from;
+        if (g.c2) tail.c2 = static_cast<unsigned char*>(g.c2) + c_size * plan.tail_from;
+        if (g.addend) tail.addend = static_cast<const unsigned char*>(g.addend) + c_size * plan.tail_from;
+        if (g.bias) tail.bias = g.bias + plan.tail_from;
+        const int rc = f16 ? gemm16_tiles_f16(head, p, kTile256, 1, st) : gemm16_tiles_bf16(head, p, kTile256, 1, st);
+        if (rc != BR_OK) return rc;
+        return f16 ? gemm16_tiles_f16(tail, p, kTile256x128Groups, 1, st) : gemm16_tiles_bf16(tail, p, kTile256x128Groups, 1, st);
+    }
+    int kernel = plan.kernel;
+    const bool ragged = g.k % 64 != 0 || g.splits > 1;
+    if (ragged && !is_flex(kernel)) {
+        if (kernel == kTile256x128Groups) kernel = kTile256x128;
+        if (!ragged_applies(p)) kernel = flex_kernel(g.m, g.n, g.k, batch);
+    }
+    if (ragged || is_flex(kernel))
+        return f16 ? gemm16_ragged_f16(g, p, kernel, batch, st) : gemm16_ragged_bf16(g, p, kernel, batch, st);
+    return f16 ? gemm16_tiles_f16(g, p, kernel, batch, st) : gemm16_tiles_bf16(g, p, kernel, batch, st);
+}
+
+// br_hip_gemm with the tensor an accumulating product adds to named separately (null = c itself).  `planned`: what a
+// caller with a workspace has planned (null: plan here, nothing split); `padded`: see gemm16::Problem.
 int gemm_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alpha, const void* a, int a_dtype,
               int64_t lda, int64_t stride_a, const void* b, int b_dtype, int64_t ldb, int64_t stride_b, int accumulate,
               const void* addend, void* c, int c_dtype, int64_t ldc, int64_t stride_c, const float* bias, int64_t batch,
-              int compute, br_stream_t stream, float* partials = nullptr, size_t partial_bytes = 0) {
+              int compute, br_stream_t stream, const gemm16::Plan* planned = nullptr, bool padded = false,
+              float* partials = nullptr, size_t partial_bytes = 0) {
     if (m < 0 || n < 0 || k < 0 || batch < 0) return BR_ERR_ATTR;
     if (m == 0 || n == 0 || batch == 0) return BR_OK;
     if (!a || !b) return BR_ERR_INPUT;
@@ -220,7 +263,7 @@ int gemm_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float a
     g.alpha = alpha;
     g.accumulate = accumulate ? 1 : 0;
     g.addend = accumulate ? addend : nullptr;
-    g.partials = partials;   // room for the partial tiles of a K split (the direct-to-LDS kernel decides)
+    g.partials = partials;   // room for the partial tiles of a K split inside the kernel
     g.partial_bytes = partials ? partial_bytes : 0;
     g.tiles_m = (int)((m + BM - 1) / BM);
     g.tiles_n = (int)((n + BN - 1) / BN);
@@ -250,11 +293,19 @@ int gemm_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float a
     p.a_kstr = ak;
     p.b_kstr = bk;
     p.c_dtype = c_dtype;
-    // the fast kernel loads 128 bits at a time and never checks k
+    p.padded = padded;
+    if (gemm16::dtl_applies(g, p)) {
+        if (planned && planned->slices > 1) {
+            // c holds one partial product per slice, `batch` of them
+            g.splits = (int)batch;
+            g.k_slice = (int)gemm16::slice_length(k, planned->slices);
+        }
+        return run_plan(g, p, planned ? *planned : gemm16::gemm_plan(m, n, k, batch, false), batch, compute, st);
+    }
+    // the register-staged kernel; its fast form loads 128 bits at a time and never checks k
     const long long va = p.a_f32 ? 4 : 8, vb = p.b_f32 ? 4 : 8;
     p.guarded = !g.vec_a || !g.vec_b || k % 32 != 0 || (ak && m % va != 0) || (bk && n % vb != 0);
-    if (compute == BR_GEMM_F16) return gemm16_launch_f16(g, p, batch, st);
-    return gemm16_launch_bf16(g, p, batch, st);
+    return compute == BR_GEMM_F16 ? gemm16_registers_f16(g, p, batch, st) : gemm16_registers_bf16(g, p, batch, st);
 }
 
 }  // namespace
@@ -274,7 +325,7 @@ extern "C" int br_hip_linear_gelu(const void* x, const void* w, const float* bia
     if (rows == 0) return BR_OK;
     if (!x || !w) return BR_ERR_INPUT;
     if (!u || !y || u == y) return BR_ERR_OUTPUT;
-    // the GELU epilogue exists in the direct-to-LDS kernel only
+    // the GELU epilogue exists in the direct-to-LDS kernels only
     if (in % 32 != 0 || out % 8 != 0 || !aligned16(x) || !aligned16(w) || !aligned16(u) || !aligned16(y))
         return BR_ERR_TODO;
     GemmArgs g;
@@ -291,43 +342,53 @@ extern "C" int br_hip_linear_gelu(const void* x, const void* w, const float* bia
     p.a_kstr = p.b_kstr = false;
     p.c_dtype = dtype;
     p.guarded = false;
-    hipStream_t st = as_stream(stream);
-    if (dtype == BR_F16) return gemm16_launch_f16(g, p, 1, st);
-    return gemm16_launch_bf16(g, p, 1, st);
+    if (!gemm16::dtl_applies(g, p)) return BR_ERR_TODO;
+    return run_plan(g, p, gemm16::gemm_plan(rows, out, in, 1, false), 1, dtype == BR_F16 ? BR_GEMM_F16 : BR_GEMM_BF16,
+                    as_stream(stream));
 }
 
-// ---- fp32 operands staged as 16-bit copies ----------------------------------
+// ---- operands staged as dense, aligned 16-bit copies ------------------------
 namespace {
 
-// dst[b][r][c] (dense) = convert(src[b*stride + r*ld + c]); cols % 4 == 0 and
-// 16-byte aligned rows take the vector path.
-template <typename DST, bool VEC>
-__global__ __launch_bounds__(256) void stage_rows_kernel(const float* __restrict__ src, long long ld,
-                                                         long long stride, long long rows, long long cols,
-                                                         long long batch, DST* __restrict__ dst) {
-    const long long per_row = VEC ? cols / 4 : cols;
-    const long long total = batch * rows * per_row;
+// dst[b][r][0 .. pitch) = convert(src[b*stride + r*ld + c]) for c < cols, zero from there to the pitch (a multiple
+// of 8): fp32 rows, or 16-bit rows that do not start on 16-byte boundaries.  One 16-byte granule per thread.
+template <bool F32SRC, bool BF>
+__global__ __launch_bounds__(256) void stage_rows_kernel(const void* __restrict__ src, long long ld, long long stride,
+                                                         unsigned rows, unsigned cols, unsigned granules,
+                                                         long long total, gemm16::u32x4* __restrict__ dst) {
+    constexpr int CT = BF ? BR_GEMM_BF16 : BR_GEMM_F16;
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total;
          i += (long long)gridDim.x * blockDim.x) {
-        const long long c = i % per_row, r = (i / per_row) % rows, b = i / (per_row * rows);
-        const float* s = src + b * stride + r * ld;
-        DST* d = dst + (b * rows + r) * cols;
-        if (VEC) {
-            const float4 v = reinterpret_cast<const float4*>(s)[c];
-            gemm16::u32x2 o;
-            if (sizeof(DST) == 2 && __is_same(DST, __half)) {
-                o.x = gemm16::pack2(gemm16::Cvt<BR_GEMM_F16>::from_f32(v.x), gemm16::Cvt<BR_GEMM_F16>::from_f32(v.y));
-                o.y = gemm16::pack2(gemm16::Cvt<BR_GEMM_F16>::from_f32(v.z), gemm16::Cvt<BR_GEMM_F16>::from_f32(v.w));
+        const unsigned c = (unsigned)(i % granules) * 8;
+        const long long row = i / granules;
+        const long long at = row / rows * stride + row % rows * ld + c;
+        gemm16::u32x4 o;
+        if (F32SRC) {
+            const float* s = static_cast<const float*>(src) + at;
+            float v[8];
+            if (c + 8 <= cols) {
+                __builtin_memcpy(v, s, sizeof(v));
             } else {
-                o.x = gemm16::pack2(gemm16::Cvt<BR_GEMM_BF16>::from_f32(v.x), gemm16::Cvt<BR_GEMM_BF16>::from_f32(v.y));
-                o.y = gemm16::pack2(gemm16::Cvt<BR_GEMM_BF16>::from_f32(v.z), gemm16::Cvt<BR_GEMM_BF16>::from_f32(v.w));
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[e] = c + e < cols ? s[e] : 0.f;
             }
-            reinterpret_cast<gemm16::u32x2*>(d)[c] = o;
+            o = gemm16::mk4(gemm16::pack2(gemm16::Cvt<CT>::from_f32(v[0]), gemm16::Cvt<CT>::from_f32(v[1])),
+                            gemm16::pack2(gemm16::Cvt<CT>::from_f32(v[2]), gemm16::Cvt<CT>::from_f32(v[3])),
+                            gemm16::pack2(gemm16::Cvt<CT>::from_f32(v[4]), gemm16::Cvt<CT>::from_f32(v[5])),
+                            gemm16::pack2(gemm16::Cvt<CT>::from_f32(v[6]), gemm16::Cvt<CT>::from_f32(v[7])));
         } else {
-            const unsigned short h = __is_same(DST, __half) ? gemm16::Cvt<BR_GEMM_F16>::from_f32(s[c])
-                                                            : gemm16::Cvt<BR_GEMM_BF16>::from_f32(s[c]);
-            reinterpret_cast<unsigned short*>(d)[c] = h;
+            const gemm16::u16* s = static_cast<const gemm16::u16*>(src) + at;
+            if (c + 8 <= cols) {
+                __builtin_memcpy(&o, s, sizeof(o));
+            } else {
+                gemm16::u16 h[8];
+#pragma unroll
+                for (int e = 0; e < 8; e++) h[e] = c + e < cols ? s[e] : (gemm16::u16)0;
+                o = gemm16::mk4(gemm16::pack2(h[0], h[1]), gemm16::pack2(h[2], h[3]), gemm16::pack2(h[4], h[5]),
+                                gemm16::pack2(h[6], h[7]));
+            }
         }
+        dst[i] = o;
     }
 }
 
@@ -349,51 +410,47 @@ __global__ __launch_bounds__(256) void stage_flat_kernel(const float4* __restric
     }
 }
 
-int stage_rows(const float* src, long long ld, long long stride, long long rows, long long cols, long long batch,
-               void* dst, int compute, hipStream_t st) {
-    const long long total = batch * rows * cols;
-    if (ld == cols && (batch == 1 || stride == rows * cols) && total % 8 == 0 && aligned16(src) && aligned16(dst)) {
-        const unsigned grid = grid_for(total / 8, 256);
-        if (compute == BR_GEMM_F16)
-            stage_flat_kernel<false><<<grid, 256, 0, st>>>(reinterpret_cast<const float4*>(src),
-                                                           static_cast<gemm16::u32x4*>(dst), total / 8);
+// Row length of a staged copy of `cols` columns.
+int64_t staged_pitch(int64_t cols) { return (cols + 7) & ~(int64_t)7; }
+
+int stage_rows(const void* src, bool f32, long long ld, long long stride, long long rows, long long cols,
+               long long batch, void* dst, int compute, hipStream_t st) {
+    const bool bf = compute == BR_GEMM_BF16;
+    if (f32 && ld == cols && cols % 8 == 0 && (batch == 1 || stride == rows * cols) && aligned16(src)) {
+        const long long n8 = batch * rows * cols / 8;
+        const unsigned grid = grid_for(n8, 256);
+        if (bf)
+            stage_flat_kernel<true><<<grid, 256, 0, st>>>(static_cast<const float4*>(src), static_cast<gemm16::u32x4*>(dst), n8);
         else
-            stage_flat_kernel<true><<<grid, 256, 0, st>>>(reinterpret_cast<const float4*>(src),
-                                                          static_cast<gemm16::u32x4*>(dst), total / 8);
+            stage_flat_kernel<false><<<grid, 256, 0, st>>>(static_cast<const float4*>(src), static_cast<gemm16::u32x4*>(dst), n8);
         BR_HIP_LAUNCH_CHECK();
         return BR_OK;
     }
-    const bool vec = cols % 4 == 0 && ld % 4 == 0 && stride % 4 == 0 && aligned16(src) && aligned16(dst);
-    const long long work = batch * rows * (vec ? cols / 4 : cols);
-    const unsigned grid = grid_for(work, 256);
-    if (compute == BR_GEMM_F16) {
-        if (vec) stage_rows_kernel<__half, true><<<grid, 256, 0, st>>>(src, ld, stride, rows, cols, batch, (__half*)dst);
-        else stage_rows_kernel<__half, false><<<grid, 256, 0, st>>>(src, ld, stride, rows, cols, batch, (__half*)dst);
-    } else {
-        if (vec) stage_rows_kernel<__hip_bfloat16, true><<<grid, 256, 0, st>>>(src, ld, stride, rows, cols, batch, (__hip_bfloat16*)dst);
-        else stage_rows_kernel<__hip_bfloat16, false><<<grid, 256, 0, st>>>(src, ld, stride, rows, cols, batch, (__hip_bfloat16*)dst);
-    }
+    const long long granules = staged_pitch(cols) / 8, total = batch * rows * granules;
+    if (rows > 0xffffffffLL || cols > 0xfffffff0LL) return BR_ERR_ATTR;
+    const unsigned grid = grid_for(total, 256);
+    gemm16::u32x4* d = static_cast<gemm16::u32x4*>(dst);
+#define BR_STAGE(F32, BF) \
+    stage_rows_kernel<F32, BF><<<grid, 256, 0, st>>>(src, ld, stride, (unsigned)rows, (unsigned)cols, (unsigned)granules, total, d)
+    if (!f32) BR_STAGE(false, false);   // bits are moved as they are
+    else if (bf) BR_STAGE(true, true);
+    else BR_STAGE(true, false);
+#undef BR_STAGE
     BR_HIP_LAUNCH_CHECK();
     return BR_OK;
 }
 
 // ---- split-K ------------------------------------------------------------------
 // A product with few output tiles and a long K leaves most CUs idle.  Two forms,
-// both deterministic and free of floating-point atomics:
-//  * many slices (products with M = 512 or fewer rows: 4-16 slices): run as a
-//    strided-batched product over `splits` slices of K into fp32 partials (slice
-//    s of A / B is the operand advanced by s * k/splits along k, which the batch
-//    strides express), followed by a fixed-order sum in a second kernel;
-//  * two slices (M = 2048, N = 4096, K >= 12288: 128 tiles of 256 x 256 on 256
-//    CUs): inside the direct-to-LDS kernel, the slice that finishes last adds the
-//    other's partial tile and runs the epilogue (gemm_dtl16.hpp).  Measured on
-//    the same box, the in-kernel form loses to the two-kernel form when four or
-//    more slices exchange partial tiles (its device-coherent accesses move
-//    1.5-3 TB/s, ordinary stores 6-7) and wins with two, where only one of the
-//    two slices writes anything.
-// Which form, how many slices and which tile depend on the problem's sizes only,
-// so a product's bits do not depend on where its operands or its workspace
-// happen to live.
+// both deterministic and free of floating-point atomics; gemm_plan chooses:
+//  * slices of K as batch entries, each leaving an fp32 partial product in the
+//    workspace, followed by a fixed-order sum in a second kernel;
+//  * two slices inside the direct-to-LDS kernel, the slice that finishes last
+//    adds the other's partial tile and runs the epilogue (gemm_dtl16.hpp).
+//    Measured on the same box, this form loses to the first when four or more
+//    slices exchange partial tiles (its device-coherent accesses move 1.5-3
+//    TB/s, ordinary stores 6-7) and wins with two, where only one of the two
+//    slices writes anything.
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float4* __restrict__ part, int splits,
                                                             long long mn4, long long n4, float alpha,
                                                             const float* __restrict__ bias, const void* old,
@@ -431,52 +488,26 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float4* __rest
     }
 }
 
-// Number of K slices (1 = do not split) for an unbatched product on the
-// direct-to-LDS kernel: the split whose estimated time, including the pass
-// over the partials, is smallest.
-int splitk_choice(int64_t m, int64_t n, int64_t k) {
-    if (n % 4 != 0) return 1;
-    double best = gemm16::dtl_tile_plan(m, n, k, 1).seconds;
-    int pick = 1;
-    for (int s = 2; s <= 16; s *= 2) {
-        if (k % (64 * s) != 0 || k / s < 512) break;
-        const double t = gemm16::dtl_tile_plan(m, n, k / s, s).seconds + 6e-6 + (double)(s + 1) * m * n * 4.0 / 4e12;
-        if (t < 0.85 * best) {
-            best = t;
-            pick = s;
-        }
-    }
-    return pick;
-}
-
-
-// Bytes of partial tiles the two-slice in-kernel form wants (0 = it does not apply or does not pay).
-size_t pair_split_room(int64_t m, int64_t n, int64_t k, int64_t batch) {
-    if (batch != 1 || splitk_choice(m, n, k) > 1) return 0;
-    return gemm16::dtl_pair_split_bytes(m, n, k);
-}
-
 size_t staged_bytes(int64_t rows, int64_t cols, int64_t batch) {
-    const size_t b = (size_t)rows * (size_t)cols * (size_t)batch * 2;
+    const size_t b = (size_t)rows * (size_t)staged_pitch(cols) * (size_t)batch * 2;
     return (b + 255) & ~(size_t)255;
 }
+
+// Whether a dense operand is copied before the product: fp32 operands are converted, 16-bit ones whose rows do not
+// start on 16-byte boundaries are moved to rows that do.
+bool wants_staging(int dtype, int64_t cols) { return dtype == BR_F32 || cols % 8 != 0; }
 
 }  // namespace
 
 extern "C" size_t br_hip_gemm_staged_workspace(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, int a_dtype,
                                                int b_dtype, int64_t batch) {
-    (void)trans_a;
-    (void)trans_b;
     if (m <= 0 || n <= 0 || k <= 0 || batch <= 0) return 0;
     size_t need = 0;
-    if (a_dtype == BR_F32) need += staged_bytes(m, k, batch);
-    if (b_dtype == BR_F32) need += staged_bytes(k, n, batch);
-    if (batch == 1) {
-        const int splits = splitk_choice(m, n, k);
-        if (splits > 1) need += (size_t)splits * (size_t)m * (size_t)n * sizeof(float);
-    }
-    need += pair_split_room(m, n, k, batch);
-    return need;
+    if (wants_staging(a_dtype, trans_a ? m : k)) need += staged_bytes(trans_a ? k : m, trans_a ? m : k, batch);
+    if (wants_staging(b_dtype, trans_b ? k : n)) need += staged_bytes(trans_b ? n : k, trans_b ? k : n, batch);
+    const gemm16::Plan plan = gemm16::gemm_plan(m, n, k, batch, true);
+    if (plan.slices > 1) need += (size_t)plan.slices * (size_t)m * (size_t)n * sizeof(float);
+    return need + gemm16::pair_bytes(plan, m, n);
 }
 
 namespace {
@@ -485,72 +516,61 @@ int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
                 int64_t lda, int64_t stride_a, const void* b, int b_dtype, int64_t ldb, int64_t stride_b, int accumulate,
                 const void* addend, void* c, int c_dtype, int64_t ldc, int64_t stride_c, const float* bias,
                 int64_t batch, int compute, void* workspace, size_t workspace_bytes, br_stream_t stream) {
-    const bool f32_a = a_dtype == BR_F32, f32_b = b_dtype == BR_F32;
+    const int native = compute == BR_GEMM_F16 ? BR_F16 : BR_BF16;
     const bool sixteen = compute == BR_GEMM_F16 || compute == BR_GEMM_BF16;
-    // Stage (and consider splitting K) only when the converted problem meets the
-    // direct-to-LDS kernel's rules; every other case is the plain entry point's
-    // business.
     const int64_t a_rows = trans_a ? k : m, a_cols = trans_a ? m : k;
     const int64_t b_rows = trans_b ? n : k, b_cols = trans_b ? k : n;
-    bool stage = sixteen && workspace && aligned16(workspace) && m > 0 && n > 0 && k > 0 && batch > 0 && a && b &&
-                 k % 32 == 0;
-    if (stage) {
-        // dense 16-bit copies: leading dimension = cols, batch stride = rows*cols
-        if (f32_a && a_cols % 8 != 0) stage = false;
-        if (f32_b && b_cols % 8 != 0) stage = false;
-        if (lda < a_cols || ldb < b_cols) stage = false;
-        if (br_hip_gemm_staged_workspace(trans_a, trans_b, m, n, k, a_dtype, b_dtype, batch) > workspace_bytes)
-            stage = false;
-    }
+    // Stage (and consider splitting K) only with the workspace that was asked for; every other case is the plain
+    // entry point's business.
+    const bool stage = sixteen && workspace && aligned16(workspace) && m > 0 && n > 0 && k > 0 && batch > 0 && a && b &&
+                       c && lda >= a_cols && ldb >= b_cols && ldc >= n &&
+                       (a_dtype == BR_F32 || a_dtype == native) && (b_dtype == BR_F32 || b_dtype == native) &&
+                       (c_dtype == BR_F32 || c_dtype == native) &&
+                       br_hip_gemm_staged_workspace(trans_a, trans_b, m, n, k, a_dtype, b_dtype, batch) <= workspace_bytes;
     if (!stage)
         return gemm_impl(trans_a, trans_b, m, n, k, alpha, a, a_dtype, lda, stride_a, b, b_dtype, ldb, stride_b,
                          accumulate, addend, c, c_dtype, ldc, stride_c, bias, batch, compute, stream);
-    const int native = compute == BR_GEMM_F16 ? BR_F16 : BR_BF16;
     hipStream_t st = as_stream(stream);
     char* ws = static_cast<char*>(workspace);
-    if (f32_a) {
-        const int rc = stage_rows(static_cast<const float*>(a), lda, stride_a, a_rows, a_cols, batch, ws, compute, st);
+    // every row of a staged copy is zero-filled up to its pitch
+    if (wants_staging(a_dtype, a_cols)) {
+        const int rc = stage_rows(a, a_dtype == BR_F32, lda, stride_a, a_rows, a_cols, batch, ws, compute, st);
         if (rc != BR_OK) return rc;
         a = ws;
         a_dtype = native;
-        lda = a_cols;
-        stride_a = a_rows * a_cols;
-        ws += staged_bytes(m, k, batch);
+        lda = staged_pitch(a_cols);
+        stride_a = a_rows * lda;
+        ws += staged_bytes(a_rows, a_cols, batch);
     }
-    if (f32_b) {
-        const int rc = stage_rows(static_cast<const float*>(b), ldb, stride_b, b_rows, b_cols, batch, ws, compute, st);
+    if (wants_staging(b_dtype, b_cols)) {
+        const int rc = stage_rows(b, b_dtype == BR_F32, ldb, stride_b, b_rows, b_cols, batch, ws, compute, st);
         if (rc != BR_OK) return rc;
         b = ws;
         b_dtype = native;
-        ldb = b_cols;
-        stride_b = b_rows * b_cols;
-        ws += staged_bytes(k, n, batch);
+        ldb = staged_pitch(b_cols);
+        stride_b = b_rows * ldb;
+        ws += staged_bytes(b_rows, b_cols, batch);
     }
-    const int splits = batch == 1 ? splitk_choice(m, n, k) : 1;
-    if (splits > 1 && c) {
-        // slices of K as batch entries: a k-contiguous operand advances by k/splits
-        // elements per slice, a row-contiguous one by k/splits rows
-        const int64_t ks = k / splits;
+    const gemm16::Plan plan = gemm16::gemm_plan(m, n, k, batch, true);
+    const bool aligned = aligned16(a) && aligned16(b) && lda % 8 == 0 && ldb % 8 == 0;
+    if (plan.slices > 1 && aligned) {
         float* part = reinterpret_cast<float*>(ws);
-        const int rc = br_hip_gemm(trans_a, trans_b, m, n, ks, 1.0f, a, a_dtype, lda, trans_a ? ks * lda : ks, b,
-                                   b_dtype, ldb, trans_b ? ks : ks * ldb, 0, part, BR_F32, n, m * n, nullptr, splits,
-                                   compute, stream);
+        const int rc = gemm_impl(trans_a, trans_b, m, n, k, 1.0f, a, a_dtype, lda, 0, b, b_dtype, ldb, 0, 0, nullptr,
+                                 part, BR_F32, n, m * n, nullptr, plan.slices, compute, stream, &plan, true);
         if (rc != BR_OK) return rc;
         const long long mn4 = m * n / 4;
         splitk_reduce_kernel<<<grid_for(mn4, 256), 256, 0, st>>>(reinterpret_cast<const float4*>(part),
-                                                                        splits, mn4, n / 4, alpha, bias,
+                                                                        plan.slices, mn4, n / 4, alpha, bias,
                                                                         accumulate ? (addend ? addend : c) : nullptr,
                                                                         c, c_dtype, ldc);
         BR_HIP_LAUNCH_CHECK();
         return BR_OK;
     }
-    // two slices inside the kernel: what is left of the workspace holds one partial tile per output tile; the
-    // product is split only if the room the workspace function asked for is really there
-    const size_t room = pair_split_room(m, n, k, batch);
-    const size_t left = workspace_bytes - (size_t)(ws - static_cast<char*>(workspace));
-    float* partials = room > 0 && room <= left ? reinterpret_cast<float*>(ws) : nullptr;
+    // two slices inside the kernel: what is left of the workspace holds one partial tile per output tile
+    float* partials = plan.pair ? reinterpret_cast<float*>(ws) : nullptr;
     return gemm_impl(trans_a, trans_b, m, n, k, alpha, a, a_dtype, lda, stride_a, b, b_dtype, ldb, stride_b, accumulate,
-                     addend, c, c_dtype, ldc, stride_c, bias, batch, compute, stream, partials, room);
+                     addend, c, c_dtype, ldc, stride_c, bias, batch, compute, stream, plan.slices > 1 ? nullptr : &plan,
+                     true, partials, gemm16::pair_bytes(plan, m, n));
 }
 }  // namespace
 

@@ -36,16 +36,21 @@
 // and the vmcnt waits are inline assembly because the compiler would otherwise
 // wait for ALL outstanding direct-to-LDS loads before any LDS read.
 //
-// Requirements (checked by the host dispatcher; everything else takes the
-// register-staged kernel in gemm_mfma16.hpp): K % 32 == 0, 16-byte aligned
-// operand bases / leading dimensions / batch strides, and for row-contiguous
-// operands rows % 8 == 0.  Rows past the end of an operand are redirected to a
-// valid row; their products land in rows / columns of C that are never stored.
+// Requirements (dtl_applies; everything else takes the register-staged kernel in
+// gemm_mfma16.hpp): 16-byte aligned operand bases / leading dimensions / batch
+// strides and, for k-contiguous operands, K % 8 == 0 (or rows zero-filled up to
+// that).  K that is not a multiple of 64 takes the ragged form (RAG: loads
+// through buffer resources with hardware bounds checks).  Measured on bf16
+// weight gradients of 1002 tokens, which ran on the register-staged kernel's
+// element-wise guarded form before: [8192 x 2048] 355 -> 43 us, [6144 x 2048]
+// 194 -> 37 us.  Rows past the end of an operand are redirected to a valid row;
+// their products land in rows / columns of C that are never stored.
 #pragma once
 #include <mutex>
 #include <type_traits>
 
 #include "gemm_mfma16.hpp"
+#include "gemm_plan.hpp"
 #include "lds_direct.hpp"
 
 
@@ -87,6 +92,13 @@ struct DtlTile {
             row = row < rows ? row : row0;
             return (unsigned)((kk * ld + (row - row0)) * 2);
         }
+    }
+
+    // k (relative to the step) of the first element of the chunk this lane fetches in its q-th load
+    static __device__ __forceinline__ int k_of(int q, int wave, int lane) {
+        const int j = q * WAVES + wave;
+        if (KSTR) return j * kKPerInstr + lane / kChunksPerK;
+        return ((lane % kChunksPerRow) ^ ((j * kRowsPerInstr + lane / kChunksPerRow) / kRowsPer256 % kChunksPerRow)) * 8;
     }
 
     // LDS byte offset (inside one tile image) this lane reads the fragment of
@@ -137,7 +149,6 @@ struct DtlTile {
 // no clearing pass.  There is one set per stream (kSplitSlots of them, handed out in the order streams first ask:
 // split_slot_of): products on one stream run one after the other and may share a set, products split at the same
 // time on different streams meet through different sets; a stream beyond the last set gets no split.
-constexpr int kMaxSplitTiles = 8192;
 constexpr int kSplitSlots = 8;
 static __device__ unsigned dtl_tickets[kSplitSlots][kMaxSplitTiles];
 static __device__ unsigned dtl_arrived[kSplitSlots][kMaxSplitTiles];
@@ -165,13 +176,34 @@ __device__ __forceinline__ void load4_device_coherent(f32x4 (&v)[4], const f32x4
         : "memory");
 }
 
+// One element of C through a buffer resource.
+template <typename T>
+__device__ __forceinline__ float buffer_read(__amdgpu_buffer_rsrc_t r, unsigned at) {
+    if constexpr (sizeof(T) == 4) {
+        return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, at, 0, 0));
+    } else {
+        const T h = __builtin_bit_cast(T, (u16)__builtin_amdgcn_raw_buffer_load_b16(r, at, 0, 0));
+        return c_load<T>(&h);
+    }
+}
+template <typename T>
+__device__ __forceinline__ void buffer_write(__amdgpu_buffer_rsrc_t r, unsigned at, float v) {
+    if constexpr (sizeof(T) == 4) {
+        __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, at, 0, 0);
+    } else {
+        T h;
+        c_store<T>(&h, v);
+        __builtin_amdgcn_raw_buffer_store_b16(__builtin_bit_cast(u16, h), r, at, 0, 0);
+    }
+}
+
 // KW = 2: the sixteen-wide sub-steps of every K step are dealt to two groups of waves (group kw takes sub-steps
 // kw * KS/2 ..), each group covering the whole tile with wave tiles twice as large; the groups' accumulators are
 // added through LDS after the K loop (group 1 into group 0, which runs the epilogue).  For tiles too small to give
 // eight waves a 64 x 128 block each: a 256 x 128 tile on eight 64 x 64 waves reads 128 KB of fragments per K step
 // from LDS, on two groups of four 64 x 128 waves 96 KB.
 template <int CT, int BM, int BN, int WM, int WN, int KT, int STAGES, bool A_KSTR, bool B_KSTR, typename TC,
-          bool GELU = false, bool SPLIT = false, int KW = 1>
+          bool GELU = false, bool SPLIT = false, int KW = 1, bool RAG = false>
 __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64) void gemm_dtl_kernel(GemmArgs g) {
     constexpr int WAVES_MN = (BM / WM) * (BN / WN);
     constexpr int WAVES = WAVES_MN * KW;
@@ -200,7 +232,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64) void gemm_dtl_kern
     batch = __builtin_amdgcn_readfirstlane((int)batch);
     // with a K split the slices take the place of the batch index in the tile order (slice-major: the workgroups
     // an XCD runs at a time still cover one block of tiles, of one slice)
-    const int slice = SPLIT ? (int)batch : 0;
+    const int slice = SPLIT || (RAG && g.splits > 1) ? (int)batch : 0;
+    const long long operand_batch = SPLIT || (RAG && g.splits > 1) ? 0 : batch;
     if (SPLIT) batch = 0;
     const long long row0 = (long long)tm * BM, col0 = (long long)tn * BN;
     const int lane = threadIdx.x & 63;
@@ -211,9 +244,9 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64) void gemm_dtl_kern
     // tile origins at K step 0 (wave-uniform, advanced once per step) and the
     // per-lane chunk offsets (fixed for the whole K loop)
     const unsigned char* a_src = reinterpret_cast<const unsigned char*>(g.a) +
-                                 2 * (batch * g.sa + (A_KSTR ? row0 : row0 * g.lda));
+                                 2 * (operand_batch * g.sa + (A_KSTR ? row0 : row0 * g.lda));
     const unsigned char* b_src = reinterpret_cast<const unsigned char*>(g.b) +
-                                 2 * (batch * g.sb + (B_KSTR ? col0 : col0 * g.ldb));
+                                 2 * (operand_batch * g.sb + (B_KSTR ? col0 : col0 * g.ldb));
     const long long a_step = A_KSTR ? 2 * KT * g.lda : 2 * KT;
     const long long b_step = B_KSTR ? 2 * KT * g.ldb : 2 * KT;
     unsigned a_off[TA::kPerWave], b_off[TB::kPerWave];
@@ -232,23 +265,41 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64) void gemm_dtl_kern
     }
 
     // this workgroup's K steps: [k_begin, k_begin + nk) of the g.k / KT steps (all of them without a split)
-    const int nk_all = (int)(g.k / KT);
-    const int k_begin = SPLIT ? slice * nk_all / 2 : 0;
-    const int nk = SPLIT ? (slice + 1) * nk_all / 2 - k_begin : nk_all;
+    const int nk_all = (int)((g.k + KT - 1) / KT);
+    const int rag_begin = RAG ? slice * (g.k_slice / KT) : 0;
+    const int k_begin = SPLIT ? slice * nk_all / 2 : rag_begin;
+    const int nk = SPLIT ? (slice + 1) * nk_all / 2 - k_begin
+                   : RAG && g.splits > 1 && k_begin + g.k_slice / KT < nk_all ? g.k_slice / KT : nk_all - k_begin;
     // step `t` of the loop covers K step k_begin + (t + first) mod nk (see k_walk_start)
-    const int first = SPLIT ? (int)(k_walk_start(row0, col0, g.k) / KT) % nk : (int)(k_walk_start(row0, col0, g.k) / KT);
+    const int first = SPLIT || RAG ? (int)(k_walk_start(row0, col0, g.k) / KT) % nk : (int)(k_walk_start(row0, col0, g.k) / KT);
     a_src += (k_begin + first) * a_step;
     b_src += (k_begin + first) * b_step;
     int until_wrap = nk - first;  // issues left before the walk returns to K step 0
+    // RAG: K is not a multiple of KT.  The loads go through buffer resources that end where the operands end, so
+    // that k-rows past K of a row-contiguous operand read as zero; chunks past K of a k-contiguous one (K a multiple
+    // of 8, or rows zero-filled up to one) are fetched from past the end.  k_left: k-values from the current step on.
+    int k_left = RAG ? (int)g.k - (k_begin + first) * KT : 0;
     auto issue = [&](int tile) {
         const unsigned dst = lds0 + (unsigned)(tile % STAGES) * kStageBytes + (unsigned)wave * 1024u;
+        if constexpr (RAG) {
+            const buffer_rsrc ra = buffer_from(a_src, (((A_KSTR ? (k_left - 1) * g.lda + g.m - row0 : (g.m - 1 - row0) * g.lda + k_left) * 2 + 15) & ~15LL));
+            const buffer_rsrc rb = buffer_from(b_src, (((B_KSTR ? (k_left - 1) * g.ldb + g.n - col0 : (g.n - 1 - col0) * g.ldb + k_left) * 2 + 15) & ~15LL));
 #pragma unroll
-        for (int q = 0; q < TA::kPerWave; q++) dtl_load(dst + q * WAVES * 1024, a_off[q], a_src);
+            for (int q = 0; q < TA::kPerWave; q++)
+                buffer_dtl_load(dst + q * WAVES * 1024, !A_KSTR && TA::k_of(q, wave, lane) >= k_left ? kPastEnd : a_off[q], ra);
 #pragma unroll
-        for (int q = 0; q < TB::kPerWave; q++) dtl_load(dst + TA::kBytes + q * WAVES * 1024, b_off[q], b_src);
+            for (int q = 0; q < TB::kPerWave; q++)
+                buffer_dtl_load(dst + TA::kBytes + q * WAVES * 1024, !B_KSTR && TB::k_of(q, wave, lane) >= k_left ? kPastEnd : b_off[q], rb);
+        } else {
+#pragma unroll
+            for (int q = 0; q < TA::kPerWave; q++) dtl_load(dst + q * WAVES * 1024, a_off[q], a_src);
+#pragma unroll
+            for (int q = 0; q < TB::kPerWave; q++) dtl_load(dst + TA::kBytes + q * WAVES * 1024, b_off[q], b_src);
+        }
         const bool wraps = --until_wrap == 0;
         a_src += wraps ? a_step - nk * a_step : a_step;
         b_src += wraps ? b_step - nk * b_step : b_step;
+        if (RAG) k_left += wraps ? (nk - 1) * KT : -KT;
     };
     auto read_frags = [&](u32x4 (&fa)[FM], u32x4 (&fb)[FN], int tile, int ks) {
         const lds_byte* stage = lds + (tile % STAGES) * kStageBytes;
@@ -516,34 +567,59 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64) void gemm_dtl_kern
         }
         return;
     }
-    // Edge tiles: element-wise guards.  The two forms are separate loops so that the plain one holds no read of C.
-    auto guarded = [&](auto adds) {
+    // Edge tiles: the same straight line, through buffer resources that end with the last element of C: rows past m
+    // lie beyond their end, columns past n are sent there; loads from there read zero, stores to there are dropped.
+    // (With a bounds test around every element, each store waited for the one before: the [1002 x 6144] projection
+    // from K = 2048 went from 43 to 34 us, a [78 x 4096] product from 22 to 16.)
+    const long long tile_at = (row0 + __builtin_amdgcn_readfirstlane(wm) * WM) * g.ldc + col0 + __builtin_amdgcn_readfirstlane(wn) * WN;
+    const long long tile_left = (g.m - 1 - row0 - __builtin_amdgcn_readfirstlane(wm) * WM) * g.ldc + g.n - col0 - __builtin_amdgcn_readfirstlane(wn) * WN;
+    auto c_buffer = [&](const TC* base) {
+        const long long left = tile_left * (long long)sizeof(TC);
+        return __builtin_amdgcn_make_buffer_rsrc(const_cast<TC*>(base) + tile_at, 0, left <= 0 ? 0 : left > (long long)kPastEnd ? (int)kPastEnd : (int)left, 0x00020000);
+    };
+    const auto cb = c_buffer(c_base), c2b = c_buffer(GELU ? c2_base : c_base), oldb = c_buffer(old_base);
+    float bias[FN];
+    unsigned lane_at[FN];
 #pragma unroll
-        for (int j = 0; j < FN; j++) {
-            const long long col = col0 + wn * WN + j * 32 + (lane & 31);
-            if (col >= g.n) continue;
-            const float bias = g.bias ? g.bias[col] : 0.f;
+    for (int j = 0; j < FN; j++) {
+        const long long col = col0 + wn * WN + j * 32 + (lane & 31);
+        bias[j] = g.bias && col < g.n ? g.bias[col] : 0.f;
+        lane_at[j] = col < g.n ? (unsigned)(((lane >> 5) * 4 * g.ldc + j * 32 + (lane & 31)) * (long long)sizeof(TC)) : kPastEnd;
+    }
+    // a row offset added to kPastEnd stays past the end: the tile spans less than 2^31 bytes (dtl_applies)
+    auto at = [&](int blk, int v) {
+        return lane_at[blk % FN] + (unsigned)((blk / FN * 32 + (v >> 2) * 8 + (v & 3)) * (int)g.ldc * (int)sizeof(TC));
+    };
+    auto edge = [&](auto adds) {
+        constexpr bool ADDS = decltype(adds)::value;
+        float alpha = g.alpha;
+        asm volatile("" : "+v"(alpha));
+        float was[2][16];
+        auto fetch = [&](int blk) {
 #pragma unroll
-            for (int i = 0; i < FM; i++) {
+            for (int v = 0; v < 16; v++) was[blk & 1][v] = buffer_read<TC>(oldb, at(blk, v));
+        };
+        if (ADDS) fetch(0);
 #pragma unroll
-                for (int v = 0; v < 16; v++) {
-                    const long long row = row0 + wm * WM + i * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
-                    if (row < g.m) {
-                        TC* p = c_base + row * g.ldc + col;
-                        float o = g.alpha * acc[i][j][v] + bias;
-                        if (decltype(adds)::value) o += c_load<TC>(old_base + row * g.ldc + col);
-                        if (sizeof(TC) == 2) asm volatile("" : "+v"(o));  // as in the interior form
-                        c_store<TC>(p, o);
-                        if (GELU) c_store<TC>(c2_base + row * g.ldc + col, gelu_one(o));
-                    }
-                }
+        for (int blk = 0; blk < FM * FN; blk++) {
+            const int i = blk / FN, j = blk % FN;
+            if (ADDS && blk + 1 < FM * FN) fetch(blk + 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                float o = alpha * acc[i][j][v] + bias[j];
+                if (ADDS) o += was[blk & 1][v];
+                if (sizeof(TC) == 2) asm volatile("" : "+v"(o));  // as in the interior form
+                buffer_write<TC>(cb, at(blk, v), o);
+                if (GELU) buffer_write<TC>(c2b, at(blk, v), gelu_one(o));
             }
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
     if (g.accumulate) {
-        guarded(std::true_type{});
+        edge(std::true_type{});
     } else {
-        guarded(std::false_type{});
+        edge(std::false_type{});
     }
 }
 
@@ -715,11 +791,7 @@ __global__ __launch_bounds__(512) void gemm_dtl_walk_kernel(GemmArgs g) {
 }
 
 // Whether the walking form takes a product the plan has put on 256 x 256 tiles.
-#ifndef BR_DTL_WALK
-#define BR_DTL_WALK 1   // 0: every product on one workgroup per tile (for an A/B build)
-#endif
 inline bool walk_applies(const GemmArgs& g, long long batch) {
-    if (!BR_DTL_WALK) return false;
     const long long tiles = (g.m / 256) * (g.n / 256);
     return batch == 1 && g.m % 256 == 0 && g.n % 256 == 0 && g.k % 64 == 0 && tiles >= 256 && tiles % 8 == 0 &&
            tiles <= 0x7fffffffLL && !g.bias && !g.accumulate && !g.c2 && !g.addend && g.splits == 1;
@@ -750,12 +822,6 @@ int launch_dtl_walk(GemmArgs g, const Problem& p, hipStream_t st) {
 }
 
 // ---- host-side dispatch -------------------------------------------------------
-#ifndef BR_DTL_KW
-#define BR_DTL_KW 1
-#endif
-#ifndef BR_DTL_KW_MIN_STEPS
-#define BR_DTL_KW_MIN_STEPS 24
-#endif
 template <int CT, int BM, int BN, int WM, int WN, int KT, int ST, int KW = 1>
 int launch_dtl_config(GemmArgs g, const Problem& p, long long batch, hipStream_t st) {
     constexpr int THREADS = (BM / WM) * (BN / WN) * KW * 64;
@@ -822,101 +888,56 @@ int launch_dtl_config(GemmArgs g, const Problem& p, long long batch, hipStream_t
     return BR_OK;
 }
 
-// The direct-to-LDS kernel applies when both operands are 16-bit, the fast
-// path's alignment rules hold and every per-lane source offset fits 32 bits.
+// The ragged form (K not a multiple of 64, or slices of K that are not all alike), for the layouts of a linear
+// layer's three products; the weight gradient's layout only with an fp32 C.
+template <int CT, int BM, int BN, int WM, int WN, int ST>
+int launch_dtl_ragged(GemmArgs g, const Problem& p, long long batch, hipStream_t st) {
+    constexpr int THREADS = (BM / WM) * (BN / WN) * 64;
+    using C16 = std::conditional_t<CT == BR_GEMM_F16, __half, __hip_bfloat16>;
+    g.tiles_m = (int)((g.m + BM - 1) / BM);
+    g.tiles_n = (int)((g.n + BN - 1) / BN);
+    const long long blocks = (long long)g.tiles_m * g.tiles_n * (g.splits > 1 ? g.splits : batch);
+    if (blocks > 0x7fffffffLL) return BR_ERR_ATTR;
+    const unsigned grid = (unsigned)blocks;
+    if (g.c2) {
+        if (p.a_kstr || p.b_kstr || p.c_dtype == BR_F32) return BR_ERR_TODO;
+        gemm_dtl_kernel<CT, BM, BN, WM, WN, 64, ST, false, false, C16, true, false, 1, true><<<grid, THREADS, 0, st>>>(g);
+    } else if (p.a_kstr) {
+        if (!p.b_kstr || p.c_dtype != BR_F32) return BR_ERR_TODO;
+        gemm_dtl_kernel<CT, BM, BN, WM, WN, 64, ST, true, true, float, false, false, 1, true><<<grid, THREADS, 0, st>>>(g);
+    } else if (p.b_kstr) {
+        if (p.c_dtype == BR_F32)
+            gemm_dtl_kernel<CT, BM, BN, WM, WN, 64, ST, false, true, float, false, false, 1, true><<<grid, THREADS, 0, st>>>(g);
+        else
+            gemm_dtl_kernel<CT, BM, BN, WM, WN, 64, ST, false, true, C16, false, false, 1, true><<<grid, THREADS, 0, st>>>(g);
+    } else {
+        if (p.c_dtype == BR_F32)
+            gemm_dtl_kernel<CT, BM, BN, WM, WN, 64, ST, false, false, float, false, false, 1, true><<<grid, THREADS, 0, st>>>(g);
+        else
+            gemm_dtl_kernel<CT, BM, BN, WM, WN, 64, ST, false, false, C16, false, false, 1, true><<<grid, THREADS, 0, st>>>(g);
+    }
+    BR_HIP_LAUNCH_CHECK();
+    return BR_OK;
+}
+inline bool ragged_applies(const Problem& p) { return !p.a_kstr || (p.b_kstr && p.c_dtype == BR_F32); }
+
+// The direct-to-LDS kernels apply when both operands are 16-bit and 16-byte aligned, a k-contiguous operand's rows
+// end on a 16-byte granule of their own (K a multiple of 8, or zero-filled up to one), and every per-lane offset fits
+// 32 bits (of the operands, and of a tile of C, which spans up to 256 rows).
 inline bool dtl_applies(const GemmArgs& g, const Problem& p) {
-    if (p.a_f32 || p.b_f32 || p.guarded) return false;
+    if (p.a_f32 || p.b_f32 || !g.vec_a || !g.vec_b || g.k <= 0) return false;
+    if (g.k % 8 != 0 && !p.padded && !(p.a_kstr && p.b_kstr)) return false;
     const long long lim = 1LL << 31;
     const long long a_span = p.a_kstr ? 2 * 64 * g.lda : 2 * 256 * g.lda;
     const long long b_span = p.b_kstr ? 2 * 64 * g.ldb : 2 * 256 * g.ldb;
-    return a_span < lim && b_span < lim && g.ldc < (1LL << 27);
+    return a_span < lim && b_span < lim && g.ldc < (1LL << 21) && g.m < lim && g.n < lim && g.k < lim;
 }
 
-// Tile choice by estimated time: rounds of workgroups over the 256 CUs x the
-// MFMA work of one tile / the rate a workgroup of that configuration reaches
-// (measured on the BLOOM-7B1 linear-layer shapes: ~1000 TFLOP/s chip-wide for
-// 256x256, ~0.9 of that for 256x128, ~0.8 for 128x128 with two workgroups
-// resident per CU).
-struct DtlPlan {
-    int config;      // 0: 256x256, 1: 256x128, 2: 128x128 (64-wide K steps), 3: 128x128 with 32-wide steps
-    double seconds;  // estimate, for comparing plans only
-};
-inline DtlPlan dtl_tile_plan(long long m, long long n, long long k, long long batch) {
-    const double per_cu = 1.0e15 / 256.0;  // flop/s of one CU at the 256x256 rate
-    auto estimate = [&](long long bm, long long bn, long long slots, double rel) {
-        const long long tiles = ((m + bm - 1) / bm) * ((n + bn - 1) / bn) * batch;
-        const double rounds = (double)((tiles + slots - 1) / slots);
-        const double per_block = per_cu * rel * 256.0 / (double)slots;  // co-resident workgroups share the CU
-        return rounds * 2.0 * (double)bm * (double)bn * (double)k / per_block + 4e-6;
-    };
-    if (k % 64 != 0) return DtlPlan{3, estimate(128, 128, 512, 0.65)};
-    DtlPlan best{0, estimate(256, 256, 256, 1.0)};
-    const double t1 = estimate(256, 128, 256, 0.9), t2 = estimate(128, 128, 512, 0.8);
-    if (t1 < best.seconds) best = DtlPlan{1, t1};
-    if (t2 < best.seconds) best = DtlPlan{2, t2};
-    return best;
-}
-
-// A product whose 256x256 tiles fill some rounds of workgroups and then at most half of one more (the q|k|v
-// projection of 2048 tokens: 384 tiles, a round and a half) leaves half the chip idle for a whole tile time, and on
-// 256x128 tiles throughout it pays their lower rate on every round.  Run in two launches -- the columns that make
-// whole rounds on 256x256 tiles, the rest on 256x128 tiles, which then fill one round -- the projection takes 190 us
-// instead of 210 either way.  Returns the first column of the second launch, or 0 where this does not apply or does
-// not beat `best_seconds` (the estimate of the best single-launch plan, same model as dtl_tile_plan).  The split
-// falls on a multiple of 1024 columns, the period of k_walk_start, so every element of C is still summed in the
-// order every other plan sums it in.
-inline long long dtl_column_tail(long long m, long long n, long long k, double best_seconds) {
-    if (k % 64 != 0) return 0;
-    const long long tm = (m + 255) / 256, tn = (n + 255) / 256;
-    long long a = 256, b = tm;
-    while (b) { const long long r = a % b; a = b; b = r; }   // a = gcd(256, tm)
-    long long unit = 256 / a;                                // tile columns that make whole rounds
-    if (unit < 4) unit = 4;                                  // a power of two; and a multiple of 1024 columns
-    const long long tn_main = tn / unit * unit, tn_rest = tn - tn_main;
-    if (tn_main == 0 || tn_rest == 0 || tm * tn_rest > 128) return 0;
-    const double round256 = 2.0 * 256.0 * 256.0 * (double)k / (1.0e15 / 256.0);
-    const double seconds = (double)(tm * tn_main / 256) * round256 + 0.5 * round256 / 0.9 + 6e-6;
-    return seconds < best_seconds ? tn_main * 256 : 0;
-}
-
-// Whether the two-slice K split inside the kernel pays (-1 = no, else the tile configuration to run it with), from
-// per-workgroup times measured on MI355X (fp16, all CUs busy): a 64-wide K step takes 1.8 us on a 256x256 tile and
-// 1.15 us on 256x128; a round of workgroups costs 3 us to fill and drain; C leaves at 6.5 TB/s; the one partial tile
-// per output tile is written and read back through device-coherent accesses at about 3 TB/s.  It pays where 256x256
-// tiles would fill at most half the CUs and K is long: for [2048 x 4096] outputs from K = 12288 up (8-10 % there).
-// Shorter M (few rows: many slices do better, see the caller) and shapes this timing was not taken on are left alone.
-inline int dtl_pair_split(long long m, long long n, long long k) {
-    if (m < 1024 || k % 64 != 0 || k / 64 < 16) return -1;
-    auto estimate = [&](int config, int splits) {
-        const long long bm = config == 0 ? 256 : 256, bn = config == 0 ? 256 : 128;
-        const long long tiles = ((m + bm - 1) / bm) * ((n + bn - 1) / bn);
-        const double rounds = (double)((tiles * splits + 255) / 256);
-        const double steps = (double)(k / splits) / 64.0;
-        double t = rounds * (steps * (config == 0 ? 1.8 : 1.15) + 3.0) * 1e-6 + (double)m * n * 4.0 / 6.5e12 + 4e-6;
-        if (splits > 1) t += 2.0 * (double)tiles * bm * bn * 4.0 / 3e12 + 3e-6;
-        return t;
-    };
-    const double unsplit = estimate(0, 1) < estimate(1, 1) ? estimate(0, 1) : estimate(1, 1);
-    int pick = -1;
-    double best = 0.97 * unsplit;
-    for (int c = 0; c < 2; c++) {
-        const long long bm = 256, bn = c == 0 ? 256 : 128;
-        if (((m + bm - 1) / bm) * ((n + bn - 1) / bn) > kMaxSplitTiles) continue;
-        const double t = estimate(c, 2);
-        if (t < best) {
-            best = t;
-            pick = c;
-        }
-    }
-    return pick;
-}
-// bytes of partial tiles the two-slice split needs in the caller's workspace (one per output tile; 0 when the
-// split does not pay)
-inline size_t dtl_pair_split_bytes(long long m, long long n, long long k) {
-    const int c = dtl_pair_split(m, n, k);
-    if (c < 0) return 0;
-    const long long bm = 256, bn = c == 0 ? 256 : 128;
-    return (size_t)(((m + bm - 1) / bm) * ((n + bn - 1) / bn)) * bm * bn * sizeof(float);
+// bytes of partial tiles the two-slice split wants in the caller's workspace (one per output tile)
+inline size_t pair_bytes(const Plan& plan, long long m, long long n) {
+    if (!plan.pair) return 0;
+    const KernelCost& c = kCost[plan.kernel];
+    return (size_t)(ceil_div(m, c.bm) * ceil_div(n, c.bn)) * c.bm * c.bn * sizeof(float);
 }
 
 // The counter set of a stream (-1: all sets are taken by other streams).
@@ -932,55 +953,23 @@ inline int split_slot_of(hipStream_t st) {
     return used++;
 }
 
+// The two-slice form of a plan with `pair` set.
 template <int CT>
-int launch_dtl(GemmArgs g, const Problem& p, long long batch, hipStream_t st) {
-    g.splits = 1;
-    if (batch == 1 && g.partials) {
-        const int c = dtl_pair_split(g.m, g.n, g.k);
-        const int slot = c >= 0 ? split_slot_of(st) : -1;
-        if (c >= 0 && slot >= 0 && dtl_pair_split_bytes(g.m, g.n, g.k) <= g.partial_bytes) {
-            g.splits = 2;
-            g.split_slot = slot;
-            if (c == 0) return launch_dtl_config<CT, 256, 256, 64, 128, 64, 2>(g, p, batch, st);
-            return launch_dtl_config<CT, 256, 128, 64, 64, 64, 3>(g, p, batch, st);
-        }
-    }
-    const DtlPlan plan = dtl_tile_plan(g.m, g.n, g.k, batch);
-    const long long tail_from = batch == 1 ? dtl_column_tail(g.m, g.n, g.k, plan.seconds) : 0;
-    if (tail_from > 0) {
-        // whole rounds of 256x256 tiles, then the columns left over on 256x128 tiles (see dtl_column_tail)
-        GemmArgs head = g;
-        head.n = tail_from;
-        const int rc = launch_dtl_config<CT, 256, 256, 64, 128, 64, 2>(head, p, batch, st);
-        if (rc != BR_OK) return rc;
-        GemmArgs tail = g;
-        const size_t c_size = p.c_dtype == BR_F32 ? 4 : 2;
-        tail.n = g.n - tail_from;
-        tail.b = static_cast<const unsigned char*>(g.b) + 2 * (p.b_kstr ? tail_from : tail_from * g.ldb);
-        tail.c = static_cast<unsigned char*>(g.c) + c_size * tail_from;
-        if (g.c2) tail.c2 = static_cast<unsigned char*>(g.c2) + c_size * tail_from;
-        if (g.addend) tail.addend = static_cast<const unsigned char*>(g.addend) + c_size * tail_from;
-        if (g.bias) tail.bias = g.bias + tail_from;
-        if (BR_DTL_KW && g.k / 64 >= BR_DTL_KW_MIN_STEPS) return launch_dtl_config<CT, 256, 128, 64, 128, 64, 3, 2>(tail, p, batch, st);
-        return launch_dtl_config<CT, 256, 128, 64, 64, 64, 3>(tail, p, batch, st);
-    }
-    const int pick = plan.config;
-    if (pick == 0 && walk_applies(g, batch)) return launch_dtl_walk<CT>(g, p, st);
-    if (pick == 0) return launch_dtl_config<CT, 256, 256, 64, 128, 64, 2>(g, p, batch, st);
-    if (pick == 1) {
-        // long K: two groups of four 64 x 128 waves per tile (fewer fragment reads, a merge at the end)
-        if (BR_DTL_KW && g.k / 64 >= BR_DTL_KW_MIN_STEPS) return launch_dtl_config<CT, 256, 128, 64, 128, 64, 3, 2>(g, p, batch, st);
-        return launch_dtl_config<CT, 256, 128, 64, 64, 64, 3>(g, p, batch, st);
-    }
-    if (pick == 2) return launch_dtl_config<CT, 128, 128, 64, 64, 64, 2>(g, p, batch, st);
-    return launch_dtl_config<CT, 128, 128, 64, 64, 32, 3>(g, p, batch, st);
+int launch_dtl_pair(GemmArgs g, const Problem& p, int kernel, int slot, hipStream_t st) {
+    g.splits = 2;
+    g.split_slot = slot;
+    if (kernel == kTile256) return launch_dtl_config<CT, 256, 256, 64, 128, 64, 2>(g, p, 1, st);
+    return launch_dtl_config<CT, 256, 128, 64, 64, 64, 3>(g, p, 1, st);
 }
 
+// K a multiple of 64, one workgroup per tile and batch entry.
 template <int CT>
-int launch_any(const GemmArgs& g, const Problem& p, long long batch, hipStream_t st) {
-    if (dtl_applies(g, p)) return launch_dtl<CT>(g, p, batch, st);
-    if (g.c2) return BR_ERR_TODO;  // only the direct-to-LDS kernel has the GELU epilogue
-    return launch<CT>(g, p, batch, st);
+int launch_dtl(const GemmArgs& g, const Problem& p, int kernel, long long batch, hipStream_t st) {
+    if (kernel == kTile256 && walk_applies(g, batch)) return launch_dtl_walk<CT>(g, p, st);
+    if (kernel == kTile256) return launch_dtl_config<CT, 256, 256, 64, 128, 64, 2>(g, p, batch, st);
+    if (kernel == kTile256x128Groups) return launch_dtl_config<CT, 256, 128, 64, 128, 64, 3, 2>(g, p, batch, st);
+    if (kernel == kTile256x128) return launch_dtl_config<CT, 256, 128, 64, 64, 64, 3>(g, p, batch, st);
+    return launch_dtl_config<CT, 128, 128, 64, 64, 64, 2>(g, p, batch, st);
 }
 
 }  // namespace gemm16

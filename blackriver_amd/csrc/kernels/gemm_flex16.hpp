@@ -1,0 +1,307 @@
+// 16-bit MFMA GEMM for small and ragged products: direct-to-LDS loads with
+// hardware bounds checks, waves that split K among themselves.
+//
+//   C[b][i,j] = alpha * sum_p opA[b][i,p] * opB[b][p,j] (+ C) (+ bias[j])
+//
+// A workgroup owns a BM x BN tile of C (64 x 64 or 32 x 32) and EVERY of its
+// KW waves computes the whole tile over its own share of K: wave w takes the
+// 64-wide K steps w, w + KW, w + 2 KW, ...  Each wave loads its steps into LDS
+// buffers of its own and reads them back itself, so the K loop has no barrier:
+// a wave waits for its own loads (vmcnt) and nothing else.  At the end the KW
+// accumulators meet in LDS and are added in wave order.
+//
+// Why: a product of a few hundred rows has few output tiles, and what bounds
+// it is the latency of one workgroup's walk along K and the 64 B per clock a CU
+// takes from L2.  Small tiles give more workgroups, splitting K inside the
+// workgroup shortens the walk KW times without partial tiles in memory, and a
+// wave that owns the whole tile reads half the LDS bytes per MFMA that four
+// waves with a quarter of the tile each would.
+//
+// Loads are buffer loads through a resource that ends where the operand ends:
+// rows of C past m or n and k-values past K read as zero, so K need not be a
+// multiple of anything for a row-contiguous operand and of 8 for a k-contiguous
+// one (whose tail chunk would otherwise run into the next row; a staged copy
+// with zero-filled row ends makes any K qualify).
+//
+// Measured (fp16, before / after; before = 256 x 128 tiles, or the guarded
+// register-staged kernel where K is ragged): [64 x 768] K = 256 12.1 -> 3.4 us,
+// [78 x 1024] K = 4096 20.4 -> 8.7, [1000 x 1024] K = 1024 21.9 -> 8.5,
+// [1024 x 1024] weight gradient of 1000 tokens 106 -> 8.9, [200 x 512] from
+// K = 32008 in eight slices 3490 -> 19.  What bounds it: with 16 or more K steps
+// a wave, the CU's loads into LDS (about 40 B per clock); below that launch,
+// the first loads' latency and the sum through LDS, 3.3 us for a 32 x 32 and 5
+// for a 64 x 64 tile.  A second buffer per wave, or the loads dealt out between
+// the products, measured equal or 5-15 % slower on the 64 x 64 tile.
+#pragma once
+#include <type_traits>
+
+#include "gemm_mfma16.hpp"
+#include "gemm_plan.hpp"
+#include "lds_direct.hpp"
+
+namespace brk {
+namespace gemm16 {
+
+// Operand tile of ROWS x 64 k-values, loaded by one wave.
+template <int ROWS, bool KSTR>
+struct FlexTile {
+    static constexpr int kBytes = ROWS * 64 * 2;
+    static constexpr int kInstr = kBytes / 1024;   // wave-wide loads of a tile
+    static constexpr int kChunksPerK = ROWS / 8;   // row contiguous: 16-byte chunks of a k-row
+    static constexpr int kKPerInstr = 64 / kChunksPerK;
+    // Which chunk of a k-row sits in slot c: the transposing read of a fragment touches 4 k-rows x 64 bytes at a
+    // time, which have to lie in different banks.
+    static __device__ __forceinline__ int swizzle(int kk) {
+        return ROWS == 32 ? 0 : ROWS == 64 ? 4 * ((kk >> 1) & 1) : 4 * (kk & 3);
+    }
+    // k (relative to the step) of the first element of the chunk this lane fetches in its q-th load
+    static __device__ __forceinline__ int k_of(int q, int lane) {
+        if (KSTR) return q * kKPerInstr + lane / kChunksPerK;
+        return ((lane & 7) ^ (((q * 8 + (lane >> 3)) >> 1) & 7)) * 8;
+    }
+    // its byte offset from the tile's origin at the step's first k
+    static __device__ __forceinline__ unsigned source_offset(int q, int lane, long long ld) {
+        if (KSTR) {
+            const int kk = k_of(q, lane), c = (lane % kChunksPerK) ^ swizzle(kk);
+            return (unsigned)((kk * ld + c * 8) * 2);
+        }
+        return (unsigned)(((q * 8 + (lane >> 3)) * ld + k_of(q, lane)) * 2);
+    }
+    // LDS byte offset of the fragment of 32-row block `row_base`, 16-wide sub-step ks
+    static __device__ __forceinline__ unsigned frag_offset(int row_base, int ks, int lane) {
+        if (!KSTR) {
+            const int r = row_base + (lane & 31), c = ks * 2 + (lane >> 5);
+            return (unsigned)(r * 128 + ((c ^ ((r >> 1) & 7)) * 16));
+        }
+        const int i = lane & 15, grp = lane >> 4;
+        const int kk = ks * 16 + (grp >> 1) * 8 + (i >> 2);
+        const int row16 = row_base + (grp & 1) * 16 + (i & 3) * 4;
+        return (unsigned)(kk * (ROWS * 2) + (((row16 >> 3) ^ swizzle(kk)) * 16) + (row16 & 7) * 2);
+    }
+    static __device__ __forceinline__ u32x4 fragment(const lds_byte* tile, unsigned off) {
+        if (!KSTR) return *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(tile + off);
+        typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+        const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tile + off));
+        const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tile + off + 4 * ROWS * 2));
+        const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
+        return mk4(l2.x, l2.y, h2.x, h2.y);
+    }
+};
+
+typedef float flex_f32x4 __attribute__((ext_vector_type(4)));
+
+template <int CT, int BM, int BN, int KW, int ST, bool A_KSTR, bool B_KSTR, typename TC, bool GELU = false>
+__global__ __launch_bounds__(KW * 64) void gemm_flex_kernel(GemmArgs g) {
+    using TA = FlexTile<BM, A_KSTR>;
+    using TB = FlexTile<BN, B_KSTR>;
+    constexpr int FM = BM / 32, FN = BN / 32;
+    constexpr int kStageBytes = TA::kBytes + TB::kBytes;
+    constexpr int kLoads = TA::kInstr + TB::kInstr;
+    constexpr int kWaveBytes = ST * kStageBytes;
+    static_assert(kWaveBytes >= BM * BN * 4, "a wave's buffers hold its accumulators at the end");
+    static_assert(KW * kWaveBytes <= 160 * 1024, "LDS");
+    __shared__ __attribute__((aligned(1024))) unsigned char lds_raw[KW * kWaveBytes];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    long long batch;
+    int tm, tn;
+    tile_coords(g, batch, tm, tn);
+    tm = __builtin_amdgcn_readfirstlane(tm);
+    tn = __builtin_amdgcn_readfirstlane(tn);
+    const int b = __builtin_amdgcn_readfirstlane((int)batch);
+    const int row0 = tm * BM, col0 = tn * BN;
+    // slices of K take the place of the batch index
+    const bool sliced = g.splits > 1;
+    const int k_begin = sliced ? b * g.k_slice : 0;
+    const int k_end = sliced && k_begin + g.k_slice < g.k ? k_begin + g.k_slice : (int)g.k;
+
+    // this wave's first K step, and where each operand ends as seen from it
+    const int k0 = k_begin + wave * 64;
+    const int steps = (k_end - k_begin + 63) >> 6;
+    const int mine = steps > wave ? (steps - wave + KW - 1) / KW : 0;
+    const long long a_at = (sliced ? 0 : b * g.sa) + (A_KSTR ? (long long)k0 * g.lda + row0 : (long long)row0 * g.lda + k0);
+    const long long b_at = (sliced ? 0 : b * g.sb) + (B_KSTR ? (long long)k0 * g.ldb + col0 : (long long)col0 * g.ldb + k0);
+    const unsigned char* a_src = static_cast<const unsigned char*>(g.a) + 2 * a_at;
+    const unsigned char* b_src = static_cast<const unsigned char*>(g.b) + 2 * b_at;
+    // rounded up to the 16-byte granule the last element lies in
+    long long a_left = ((A_KSTR ? (long long)(k_end - 1 - k0) * g.lda + g.m - row0
+                                : (g.m - 1 - row0) * g.lda + (k_end - k0)) * 2 + 15) & ~15LL;
+    long long b_left = ((B_KSTR ? (long long)(k_end - 1 - k0) * g.ldb + g.n - col0
+                                : (g.n - 1 - col0) * g.ldb + (k_end - k0)) * 2 + 15) & ~15LL;
+    const long long a_step = (A_KSTR ? g.lda : 1) * (2LL * 64 * KW);
+    const long long b_step = (B_KSTR ? g.ldb : 1) * (2LL * 64 * KW);
+    int k_left = k_end - k0;
+    unsigned a_off[TA::kInstr], b_off[TB::kInstr];
+#pragma unroll
+    for (int q = 0; q < TA::kInstr; q++) a_off[q] = TA::source_offset(q, lane, g.lda);
+#pragma unroll
+    for (int q = 0; q < TB::kInstr; q++) b_off[q] = TB::source_offset(q, lane, g.ldb);
+    lds_byte* const mem = (lds_byte*)lds_raw + wave * kWaveBytes;
+    const unsigned mem0 = (unsigned)(unsigned long long)mem;
+
+    auto issue = [&](int stage) {
+        const buffer_rsrc ra = buffer_from(a_src, a_left), rb = buffer_from(b_src, b_left);
+        const unsigned dst = mem0 + (unsigned)stage * kStageBytes;
+        // a k-contiguous operand's last step: chunks past K are fetched from past the end of the operand
+        const bool tail = k_left < 64;
+#pragma unroll
+        for (int q = 0; q < TA::kInstr; q++)
+            buffer_dtl_load(dst + q * 1024, !A_KSTR && tail && TA::k_of(q, lane) >= k_left ? kPastEnd : a_off[q], ra);
+#pragma unroll
+        for (int q = 0; q < TB::kInstr; q++)
+            buffer_dtl_load(dst + TA::kBytes + q * 1024, !B_KSTR && tail && TB::k_of(q, lane) >= k_left ? kPastEnd : b_off[q], rb);
+        a_src += a_step; a_left -= a_step;
+        b_src += b_step; b_left -= b_step;
+        k_left -= 64 * KW;
+    };
+
+    f32x16 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+
+#pragma unroll
+    for (int s = 0; s < ST; s++)
+        if (s < mine) issue(s);
+    int stage = 0;
+    for (int t = 0; t < mine; t++) {
+        // the loads of step t are in once at most those of the steps after it are outstanding
+        const int after = mine - 1 - t;
+        if (ST > 1 && after >= ST - 1) wait_vmem<(ST - 1) * kLoads>();
+        else if (ST > 2 && after == 1) wait_vmem<kLoads>();
+        else wait_vmem<0>();
+        const lds_byte* tile = mem + stage * kStageBytes;
+        u32x4 fa[4][FM], fb[4][FN];
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++) {
+#pragma unroll
+            for (int i = 0; i < FM; i++) fa[ks][i] = TA::fragment(tile, TA::frag_offset(i * 32, ks, lane));
+#pragma unroll
+            for (int j = 0; j < FN; j++) fb[ks][j] = TB::fragment(tile + TA::kBytes, TB::frag_offset(j * 32, ks, lane));
+        }
+        // The step is in registers: its buffer takes the loads of step t + ST while the products run.  (In one
+        // burst: dealt out between the products they measured 5-15 % slower.)
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        if (t + ST < mine) issue(stage);
+        stage = stage + 1 == ST ? 0 : stage + 1;
+        // operands swapped: a lane then holds four consecutive columns of one row of C
+#pragma unroll
+        for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+#pragma unroll
+                for (int j = 0; j < FN; j++) acc[i][j] = Cvt<CT>::mfma(fb[ks][j], fa[ks][i], acc[i][j]);
+    }
+
+    // acc[i][j][v] is C[row, col] with row = i*32 + lane%32, col = j*32 + (v/4)*8 + (lane/32)*4 + v%4.  Each wave
+    // leaves its tile in its own buffers, quad c of row r in slot c ^ (r % 8) of the row (writes of 16 rows and
+    // reads along a row both touch every bank once).
+    typedef __attribute__((address_space(3))) flex_f32x4 lds_f32x4;
+    constexpr int QN = BN / 4;
+    lds_f32x4* const sums = (lds_f32x4*)mem;
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int r = i * 32 + (lane & 31), c = j * 8 + q * 2 + (lane >> 5);
+                flex_f32x4 v;
+                v.x = acc[i][j][4 * q]; v.y = acc[i][j][4 * q + 1]; v.z = acc[i][j][4 * q + 2]; v.w = acc[i][j][4 * q + 3];
+                sums[r * QN + (c ^ (r & 7))] = v;
+            }
+    __syncthreads();
+    TC* c_base = static_cast<TC*>(g.c) + b * g.sc;
+    TC* c2_base = GELU ? static_cast<TC*>(g.c2) + b * g.sc : nullptr;
+    const TC* old_base = g.addend ? static_cast<const TC*>(g.addend) + b * g.sc : c_base;
+    const lds_f32x4* const all = (const lds_f32x4*)(lds_byte*)lds_raw;
+    constexpr int kQuads = BM * QN, kThreads = KW * 64;
+#pragma unroll
+    for (int it = 0; it < (kQuads + kThreads - 1) / kThreads; it++) {
+        const int e = it * kThreads + threadIdx.x;
+        if (kQuads % kThreads != 0 && e >= kQuads) break;
+        const int r = e / QN, c = e % QN;
+        const int at = r * QN + (c ^ (r & 7));
+        flex_f32x4 s = all[at];
+#pragma unroll
+        for (int w = 1; w < KW; w++) s += all[w * (kWaveBytes / 16) + at];
+        const int row = row0 + r, col = col0 + c * 4;
+        if (row >= g.m) continue;
+        const long long off = row * g.ldc + col;
+        const int left = (int)(g.n - col);   // columns of C this quad covers
+        float o[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            o[u] = g.alpha * s[u] + (g.bias && u < left ? g.bias[col + u] : 0.f);
+            if (g.accumulate && u < left) o[u] += c_load<TC>(old_base + off + u);
+            if (sizeof(TC) == 2) asm volatile("" : "+v"(o[u]));   // one fp32 value, then one rounding
+        }
+        if (left >= 4 && g.vec_c) {
+            c_store4<TC>(c_base + off, o);
+            if (GELU) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) o[u] = gelu_one(o[u]);
+                c_store4<TC>(c2_base + off, o);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (u < left) {
+                    c_store<TC>(c_base + off + u, o[u]);
+                    if (GELU) c_store<TC>(c2_base + off + u, gelu_one(o[u]));
+                }
+        }
+    }
+}
+
+// ---- host-side dispatch -------------------------------------------------------
+template <int CT, int BM, int BN, int KW, int ST, typename TC>
+int launch_flex_c(const GemmArgs& g, const Problem& p, unsigned grid, hipStream_t st) {
+    if (g.c2) {
+        // as the large kernels': the linear layer's layout with 16-bit outputs
+        if constexpr (sizeof(TC) == 2) {
+            if (p.a_kstr || p.b_kstr) return BR_ERR_TODO;
+            gemm_flex_kernel<CT, BM, BN, KW, ST, false, false, TC, true><<<grid, KW * 64, 0, st>>>(g);
+        } else {
+            return BR_ERR_TODO;
+        }
+    } else if (p.a_kstr && p.b_kstr) {
+        gemm_flex_kernel<CT, BM, BN, KW, ST, true, true, TC><<<grid, KW * 64, 0, st>>>(g);
+    } else if (p.a_kstr) {
+        gemm_flex_kernel<CT, BM, BN, KW, ST, true, false, TC><<<grid, KW * 64, 0, st>>>(g);
+    } else if (p.b_kstr) {
+        gemm_flex_kernel<CT, BM, BN, KW, ST, false, true, TC><<<grid, KW * 64, 0, st>>>(g);
+    } else {
+        gemm_flex_kernel<CT, BM, BN, KW, ST, false, false, TC><<<grid, KW * 64, 0, st>>>(g);
+    }
+    BR_HIP_LAUNCH_CHECK();
+    return BR_OK;
+}
+
+template <int CT, int BM, int BN, int KW, int ST>
+int launch_flex_config(GemmArgs g, const Problem& p, long long batch, hipStream_t st) {
+    g.tiles_m = (int)((g.m + BM - 1) / BM);
+    g.tiles_n = (int)((g.n + BN - 1) / BN);
+    const long long blocks = (long long)g.tiles_m * g.tiles_n * (g.splits > 1 ? g.splits : batch);
+    if (blocks > 0x7fffffffLL) return BR_ERR_ATTR;
+    const long long es = p.c_dtype == BR_F32 ? 4 : 2;
+    auto quads = [&](const void* q) { return (reinterpret_cast<uintptr_t>(q) & (4 * es - 1)) == 0; };
+    g.vec_c = g.ldc % 4 == 0 && g.sc % 4 == 0 && quads(g.c) && (!g.c2 || quads(g.c2));
+    if (p.c_dtype == BR_F32) return launch_flex_c<CT, BM, BN, KW, ST, float>(g, p, (unsigned)blocks, st);
+    return launch_flex_c<CT, BM, BN, KW, ST, std::conditional_t<CT == BR_GEMM_F16, __half, __hip_bfloat16>>(g, p, (unsigned)blocks, st);
+}
+
+// Any K; slices of K as batch entries when g.splits > 1.
+template <int CT>
+int launch_flex(const GemmArgs& g, const Problem& p, int kernel, long long batch, hipStream_t st) {
+    if (kernel == kFlex64) return launch_flex_config<CT, 64, 64, 4, 1>(g, p, batch, st);
+    if (kernel == kFlex64Short) return launch_flex_config<CT, 64, 64, 2, 1>(g, p, batch, st);
+    if (kernel == kFlex32x64) return launch_flex_config<CT, 32, 64, 4, 1>(g, p, batch, st);
+    return launch_flex_config<CT, 32, 32, 4, 2>(g, p, batch, st);
+}
+
+}  // namespace gemm16
+}  // namespace brk

@@ -76,6 +76,8 @@ struct GemmArgs {
     int splits = 1;
     float* partials = nullptr;
     size_t partial_bytes = 0;
+    int k_slice = 0;      // gemm_flex16.hpp: with splits > 1, the k-values of one slice (a multiple of 64)
+    int vec_c = 0;        // gemm_flex16.hpp: rows of C (and of c2) can be written four elements at a time
     int split_slot = 0;   // which set of the library's arrival counters the two slices of a tile meet through (one per stream)
 };
 
@@ -274,6 +276,23 @@ template <>
 __device__ __forceinline__ void c_store<__half>(__half* p, float v) { *p = __float2half_rn(v); }
 template <>
 __device__ __forceinline__ void c_store<__hip_bfloat16>(__hip_bfloat16* p, float v) { *p = __float2bfloat16(v); }
+// four consecutive elements, aligned to their total size
+template <typename T>
+__device__ __forceinline__ void c_store4(T* p, const float (&v)[4]);
+template <>
+__device__ __forceinline__ void c_store4<float>(float* p, const float (&v)[4]) {
+    *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+}
+template <>
+__device__ __forceinline__ void c_store4<__half>(__half* p, const float (&v)[4]) {
+    *reinterpret_cast<u32x2*>(p) = mk2(pack2(Cvt<BR_GEMM_F16>::from_f32(v[0]), Cvt<BR_GEMM_F16>::from_f32(v[1])),
+                                       pack2(Cvt<BR_GEMM_F16>::from_f32(v[2]), Cvt<BR_GEMM_F16>::from_f32(v[3])));
+}
+template <>
+__device__ __forceinline__ void c_store4<__hip_bfloat16>(__hip_bfloat16* p, const float (&v)[4]) {
+    *reinterpret_cast<u32x2*>(p) = mk2(pack2(Cvt<BR_GEMM_BF16>::from_f32(v[0]), Cvt<BR_GEMM_BF16>::from_f32(v[1])),
+                                       pack2(Cvt<BR_GEMM_BF16>::from_f32(v[2]), Cvt<BR_GEMM_BF16>::from_f32(v[3])));
+}
 
 
 // Tile number `rem` (0 .. tiles_m * tiles_n - 1) of one batch in the order workgroups take them.
@@ -442,6 +461,7 @@ struct Problem {
     bool a_f32, a_kstr, b_f32, b_kstr;
     int c_dtype;
     bool guarded;  // sizes / alignment rule out the fast kernel
+    bool padded = false;   // rows of the k-contiguous operands are zero-filled up to a multiple of 8 elements
 };
 
 template <bool GUARD, int CT, int BM, int BN, int WM, int WN, bool AF, bool AK, bool BF, bool BK_>

@@ -30,6 +30,31 @@ __device__ __forceinline__ void dtl_load(unsigned lds_dst, unsigned voff, const 
         : "memory");
 }
 
+// The same through a buffer resource: lane l copies the 16 bytes at offset voff(l) of the buffer, or sixteen zero
+// bytes where the offset lies past the buffer's end.  Same M0 rule as dtl_load.
+typedef unsigned buffer_rsrc __attribute__((ext_vector_type(4)));
+__device__ __forceinline__ void buffer_dtl_load(unsigned lds_dst, unsigned voff, const buffer_rsrc& rsrc) {
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dwordx4 %1, %2, 0 offen lds"
+        :
+        : "s"(lds_dst), "v"(voff), "s"(rsrc)
+        : "memory");
+}
+
+// A raw buffer of `left` bytes (none if negative) at p; kPastEnd lies beyond the end of any.
+constexpr unsigned kPastEnd = 0x7ffffff0u;
+__device__ __forceinline__ buffer_rsrc buffer_from(const unsigned char* p, long long left) {
+    const unsigned long long a = (unsigned long long)p;
+    buffer_rsrc r;
+    r.x = (unsigned)a;
+    r.y = (unsigned)(a >> 32) & 0xffffu;
+    r.z = left <= 0 ? 0u : left > (long long)kPastEnd ? kPastEnd : (unsigned)left;
+    r.w = 0x00020000u;
+    return r;
+}
+
 template <int N>
 __device__ __forceinline__ void wait_vmem() {
     asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");

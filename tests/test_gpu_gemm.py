@@ -422,3 +422,40 @@ def test_linear_gelu_epilogue_writes_both_tensors(dtype, rows, out, inn):
     assert hip.load().br_hip_linear_gelu(ptr(x), ptr(w), None, ptr(u), ptr(y), dtype, rows, out, inn - 8, stream()) == -1
     assert hip.load().br_hip_linear_gelu(ptr(x), ptr(w), None, ptr(u), ptr(u), dtype, rows, out, inn, stream()) == -3
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("c_dt", [F32, F16])
+@pytest.mark.parametrize("m,n,k,batch", [
+    (1, 8, 8, 1),            # one row of one tile, K within a chunk
+    (33, 40, 72, 1),         # 32 x 32 tiles, one past the first; K one chunk past a step
+    (64, 64, 64, 1),
+    (78, 1024, 520, 1),      # 32-row tiles, K dealt unevenly to the four waves
+    (250, 64, 250, 3),       # attention products of 250 tokens: rows that are not 16-byte aligned
+    (31, 65, 7, 2),          # everything odd
+    (1000, 1032, 1000, 1),   # 64 x 64 tiles with ragged edges
+    (1002, 4096, 1002, 1),   # large tiles with a ragged K
+    (200, 512, 12345, 1),    # slices of a ragged K
+])
+def test_gemm_small_and_ragged_products_are_exact_on_integers(ta, tb, c_dt, m, n, k, batch):
+    """The kernels for small and ragged sizes through the staged entry, on operands of small integers: every
+    partial sum is a whole number below 2^24, so the fp32 result is exact whatever the order of summation (and an
+    fp16 result is its rounding).  Any element read past an operand's end, or missed, changes it."""
+    print("case ta=%d tb=%d c=%d m=%d n=%d k=%d batch=%d" % (ta, tb, c_dt, m, n, k, batch), flush=True)
+    rng = np.random.default_rng(m + n + k)
+    a, b = operands(rng, ta, tb, m, n, k, batch)
+    a = rng.integers(-3, 4, a.shape).astype(np.float32)
+    b = rng.integers(-2, 3, b.shape).astype(np.float32)
+    bias = rng.integers(-5, 6, n).astype(np.float32)
+    da, db_, dbias = to_dev(a, F16), to_dev(b, F16), dev(bias)
+    c0 = rng.integers(-9, 10, (batch, m, n)).astype(np.float32)
+    c = to_dev(c0, c_dt)
+    need = hip.load().br_hip_gemm_staged_workspace(ta, tb, m, n, k, F16, F16, batch)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda").fill_(255)   # NaN wherever nothing is written
+    call("br_hip_gemm_staged", ta, tb, m, n, k, 1.0, ptr(da), F16, m if ta else k, m * k, ptr(db_), F16, k if tb else n,
+         n * k, 1, ptr(c), c_dt, n, m * n, ptr(dbias), batch, hip.GEMM_F16, ptr(ws), need, stream())
+    A, B = a.astype(np.float64), b.astype(np.float64)
+    ref = np.matmul(A.transpose(0, 2, 1) if ta else A, B.transpose(0, 2, 1) if tb else B) + bias.astype(np.float64) + c0
+    if c_dt == F16:
+        ref = ref.astype(np.float16).astype(np.float64)
+    assert np.array_equal(to_host64(c).reshape(batch, m, n), ref)
