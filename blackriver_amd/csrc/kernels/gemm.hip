@@ -3,15 +3,14 @@
 //   C[b][i,j] = alpha * sum_p opA[b][i,p] * opB[b][p,j] (+ C) (+ bias[j])
 //
 // 16-bit multiplicands (fp16 / bf16, fp32 accumulation) go to the kernel
-// templates in gemm_dtl16.hpp and gemm_flex16.hpp (both operands stored in the
+// templates in gemm_dtl16.hpp and gemm_flex.hpp (both operands stored in the
 // MFMA type, aligned: direct-to-LDS loads; gemm_plan.hpp chooses between them)
 // and gemm_mfma16.hpp (fp32 operands converted on load, unaligned rows).  This
 // file holds the argument checking, the staging of fp32 and of unaligned
 // operands into a caller's workspace so that they too can take the
-// direct-to-LDS kernels, and the kernel that keeps fp32 operands and
-// multiplies with v_mfma_f32_32x32x2_f32 for callers that need fp32-faithful
-// products (128x128x16 tiles, 4 wave64s x 2x2 MFMA blocks, register prefetch +
-// LDS double buffering).
+// direct-to-LDS kernels, and a kernel for fp32 products whose leading dimensions
+// are too long for the 32-bit offsets of the one in gemm_flex.hpp (128x128x16
+// tiles, 4 wave64s x 2x2 MFMA blocks, register prefetch + LDS double buffering).
 #include "common.hpp"
 
 #include <hip/hip_bf16.h>
@@ -32,6 +31,7 @@ namespace brk {
 BR_GEMM16_ENTRIES(f16)
 BR_GEMM16_ENTRIES(bf16)
 #undef BR_GEMM16_ENTRIES
+int gemm_fp32(const gemm16::GemmArgs& g, const gemm16::Problem& p, int kernel, bool words, long long batch, hipStream_t st);
 }  // namespace brk
 
 namespace {
@@ -279,14 +279,6 @@ int gemm_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float a
     hipStream_t st = as_stream(stream);
     // opA is k-strided in memory when A is stored [k,m]; opB when B is stored [k,n]
     const bool ak = trans_a != 0, bk = trans_b == 0;
-    if (compute == BR_GEMM_F32) {
-        if (ak && bk) gemm_mfma32_kernel<true, true><<<(unsigned)blocks, kThreads, 0, st>>>(g);
-        else if (ak) gemm_mfma32_kernel<true, false><<<(unsigned)blocks, kThreads, 0, st>>>(g);
-        else if (bk) gemm_mfma32_kernel<false, true><<<(unsigned)blocks, kThreads, 0, st>>>(g);
-        else gemm_mfma32_kernel<false, false><<<(unsigned)blocks, kThreads, 0, st>>>(g);
-        BR_HIP_LAUNCH_CHECK();
-        return BR_OK;
-    }
     gemm16::Problem p;
     p.a_f32 = a_dtype == BR_F32;
     p.b_f32 = b_dtype == BR_F32;
@@ -294,6 +286,20 @@ int gemm_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float a
     p.b_kstr = bk;
     p.c_dtype = c_dtype;
     p.padded = padded;
+    if (compute == BR_GEMM_F32) {
+        // the small-tile kernel's per-lane offsets span 64 rows in 32 bits
+        const long long lim = 1LL << 31;
+        if (256 * lda < lim && 256 * ldb < lim && m < lim && n < lim && k < lim && k > 0) {
+            const bool words = !g.vec_a || !g.vec_b || (k % 4 != 0 && !(ak && bk));
+            return gemm_fp32(g, p, gemm16::fp32_kernel(m, n, k, batch), words, batch, st);
+        }
+        if (ak && bk) gemm_mfma32_kernel<true, true><<<(unsigned)blocks, kThreads, 0, st>>>(g);
+        else if (ak) gemm_mfma32_kernel<true, false><<<(unsigned)blocks, kThreads, 0, st>>>(g);
+        else if (bk) gemm_mfma32_kernel<false, true><<<(unsigned)blocks, kThreads, 0, st>>>(g);
+        else gemm_mfma32_kernel<false, false><<<(unsigned)blocks, kThreads, 0, st>>>(g);
+        BR_HIP_LAUNCH_CHECK();
+        return BR_OK;
+    }
     if (gemm16::dtl_applies(g, p)) {
         if (planned && planned->slices > 1) {
             // c holds one partial product per slice, `batch` of them

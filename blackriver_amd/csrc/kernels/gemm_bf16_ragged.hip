@@ -1,7 +1,7 @@
 // bf16-multiplicand instantiations of the GEMM templates for small and ragged products, and of the register-staged
 // kernel for operands none of the direct-to-LDS kernels takes.
 #include "gemm_dtl16.hpp"
-#include "gemm_flex16.hpp"
+#include "gemm_flex.hpp"
 
 namespace brk {
 int gemm16_ragged_bf16(const gemm16::GemmArgs& g, const gemm16::Problem& p, int kernel, long long batch, hipStream_t st) {

@@ -1,11 +1,12 @@
-// 16-bit MFMA GEMM for small and ragged products: direct-to-LDS loads with
-// hardware bounds checks, waves that split K among themselves.
+// MFMA GEMM for small and ragged 16-bit products and for all fp32 ones:
+// direct-to-LDS loads with hardware bounds checks, waves that split K among
+// themselves.
 //
 //   C[b][i,j] = alpha * sum_p opA[b][i,p] * opB[b][p,j] (+ C) (+ bias[j])
 //
 // A workgroup owns a BM x BN tile of C (64 x 64 or 32 x 32) and EVERY of its
 // KW waves computes the whole tile over its own share of K: wave w takes the
-// 64-wide K steps w, w + KW, w + 2 KW, ...  Each wave loads its steps into LDS
+// 128-byte K steps w, w + KW, w + 2 KW, ...  Each wave loads its steps into LDS
 // buffers of its own and reads them back itself, so the K loop has no barrier:
 // a wave waits for its own loads (vmcnt) and nothing else.  At the end the KW
 // accumulators meet in LDS and are added in wave order.
@@ -32,6 +33,13 @@
 // the first loads' latency and the sum through LDS, 3.3 us for a 32 x 32 and 5
 // for a 64 x 64 tile.  A second buffer per wave, or the loads dealt out between
 // the products, measured equal or 5-15 % slower on the 64 x 64 tile.
+//
+// fp32 products run on the same kernel with v_mfma_f32_32x32x2: 64 clocks for
+// two k-values, so the matrix cores bound anything but the smallest and what
+// counts is that all 1024 SIMDs have an equal share (before / after; before =
+// 128 x 128 tiles of four waves): [512 x 1024] K = 1024 97 -> 14.6 us, K = 4096
+// 345 -> 44, [512 x 4096] K = 1024 97 -> 45 (95 TFLOP/s), [1024 x 8192] K = 2048
+// 327 -> 290 (119 TFLOP/s; clock not yet settled in any of these).
 #pragma once
 #include <type_traits>
 
@@ -42,64 +50,99 @@
 namespace brk {
 namespace gemm16 {
 
-// Operand tile of ROWS x 64 k-values, loaded by one wave.
-template <int ROWS, bool KSTR>
+// Operand tile of ROWS rows by 128 bytes of k (64 16-bit or 32 fp32 values), loaded by one wave in 16-byte granules,
+// or in single fp32 values (WORDS) where rows are not aligned to granules.
+template <int CT, int ROWS, bool KSTR, bool WORDS>
 struct FlexTile {
-    static constexpr int kBytes = ROWS * 64 * 2;
-    static constexpr int kInstr = kBytes / 1024;   // wave-wide loads of a tile
-    static constexpr int kChunksPerK = ROWS / 8;   // row contiguous: 16-byte chunks of a k-row
-    static constexpr int kKPerInstr = 64 / kChunksPerK;
-    // Which chunk of a k-row sits in slot c: the transposing read of a fragment touches 4 k-rows x 64 bytes at a
-    // time, which have to lie in different banks.
+    static constexpr int kSize = CT == BR_GEMM_F32 ? 4 : 2;      // bytes of an element
+    static constexpr int kPer = 16 / kSize;                      // elements of a granule
+    static constexpr int kStep = 128 / kSize;                    // k-values of a step
+    static constexpr int kBytes = ROWS * 128;
+    static constexpr int kInstr = kBytes / (WORDS ? 256 : 1024);  // wave-wide loads of a tile
+    static constexpr int kGranulesPerK = ROWS / kPer;             // row contiguous: granules of a k-row
+    static_assert(!WORDS || kSize == 4, "single values are fp32");
+
+    // Row contiguous, where things lie in LDS.  16-bit: the transposing read of a fragment touches 4 k-rows x 64
+    // bytes at a time; fp32: a fragment's reads touch 128 bytes each of k-rows k and k + 4.  Either has to fall on
+    // different banks: by which granule of a k-row sits in slot c (c ^ swizzle), and for 32 fp32 rows (half the
+    // banks wide) by keeping k-rows k and k + 4 side by side.
     static __device__ __forceinline__ int swizzle(int kk) {
+        if (kSize == 4) return ROWS == 32 ? 0 : 8 * ((kk >> 2) & 1);
         return ROWS == 32 ? 0 : ROWS == 64 ? 4 * ((kk >> 1) & 1) : 4 * (kk & 3);
     }
-    // k (relative to the step) of the first element of the chunk this lane fetches in its q-th load
+    static __device__ __forceinline__ int place_of_k(int kk) {
+        return kSize == 4 && ROWS == 32 ? (kk & ~7) + (kk & 3) * 2 + ((kk >> 2) & 1) : kk;
+    }
+    static __device__ __forceinline__ int k_in_place(int place) {
+        return kSize == 4 && ROWS == 32 ? (place & ~7) + ((place & 7) >> 1) + 4 * (place & 1) : place;
+    }
+    static __device__ __forceinline__ int slot(int q, int lane) { return WORDS ? q * 16 + (lane >> 2) : q * 64 + lane; }
+    static __device__ __forceinline__ int word(int lane) { return WORDS ? lane & 3 : 0; }
+    // k (relative to the step) of the first element this lane fetches in its q-th load
     static __device__ __forceinline__ int k_of(int q, int lane) {
-        if (KSTR) return q * kKPerInstr + lane / kChunksPerK;
-        return ((lane & 7) ^ (((q * 8 + (lane >> 3)) >> 1) & 7)) * 8;
+        const int s = slot(q, lane);
+        if (KSTR) return k_in_place(s / kGranulesPerK);
+        return ((s & 7) ^ ((s >> 4) & 7)) * kPer + word(lane);
     }
     // its byte offset from the tile's origin at the step's first k
     static __device__ __forceinline__ unsigned source_offset(int q, int lane, long long ld) {
+        const int s = slot(q, lane);
         if (KSTR) {
-            const int kk = k_of(q, lane), c = (lane % kChunksPerK) ^ swizzle(kk);
-            return (unsigned)((kk * ld + c * 8) * 2);
+            const int kk = k_of(q, lane), c = (s % kGranulesPerK) ^ swizzle(kk);
+            return (unsigned)((kk * ld + c * kPer + word(lane)) * kSize);
         }
-        return (unsigned)(((q * 8 + (lane >> 3)) * ld + k_of(q, lane)) * 2);
+        return (unsigned)(((s >> 3) * ld + k_of(q, lane)) * kSize);
     }
-    // LDS byte offset of the fragment of 32-row block `row_base`, 16-wide sub-step ks
+    // LDS byte offset of the fragment of 32-row block `row_base`, sub-step ks (a quarter of the step)
     static __device__ __forceinline__ unsigned frag_offset(int row_base, int ks, int lane) {
         if (!KSTR) {
             const int r = row_base + (lane & 31), c = ks * 2 + (lane >> 5);
             return (unsigned)(r * 128 + ((c ^ ((r >> 1) & 7)) * 16));
+        }
+        if (kSize == 4) {
+            const int r = row_base + (lane & 31), kk = ks * 8 + (lane >> 5) * 4;
+            return (unsigned)(place_of_k(kk) * (ROWS * 4) + (((r >> 2) ^ swizzle(kk)) * 16) + (r & 3) * 4);
         }
         const int i = lane & 15, grp = lane >> 4;
         const int kk = ks * 16 + (grp >> 1) * 8 + (i >> 2);
         const int row16 = row_base + (grp & 1) * 16 + (i & 3) * 4;
         return (unsigned)(kk * (ROWS * 2) + (((row16 >> 3) ^ swizzle(kk)) * 16) + (row16 & 7) * 2);
     }
+    // 16-bit: row lane % 32, k = 16 ks + 8 (lane / 32) + 0..7;  fp32: k = 8 ks + 4 (lane / 32) + 0..3
     static __device__ __forceinline__ u32x4 fragment(const lds_byte* tile, unsigned off) {
         if (!KSTR) return *reinterpret_cast<const __attribute__((address_space(3))) u32x4*>(tile + off);
+        if (kSize == 4) {
+            typedef __attribute__((address_space(3))) unsigned lds_u32;
+            constexpr int kNext = ROWS == 32 ? 2 * ROWS : ROWS;   // words from k to k + 1
+            const lds_u32* p = (const lds_u32*)(tile + off);
+            return mk4(p[0], p[kNext], p[2 * kNext], p[3 * kNext]);
+        }
         typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
         const s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tile + off));
         const s16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(tile + off + 4 * ROWS * 2));
         const u32x2 l2 = __builtin_bit_cast(u32x2, lo), h2 = __builtin_bit_cast(u32x2, hi);
         return mk4(l2.x, l2.y, h2.x, h2.y);
     }
+    static __device__ __forceinline__ void load(unsigned dst, int q, unsigned off, const buffer_rsrc& r) {
+        if (WORDS) buffer_dtl_load_dword(dst + q * 256, off, r);
+        else buffer_dtl_load(dst + q * 1024, off, r);
+    }
 };
 
 typedef float flex_f32x4 __attribute__((ext_vector_type(4)));
 
-template <int CT, int BM, int BN, int KW, int ST, bool A_KSTR, bool B_KSTR, typename TC, bool GELU = false>
+template <int CT, int BM, int BN, int KW, int ST, bool A_KSTR, bool B_KSTR, typename TC, bool GELU = false, bool WORDS = false>
 __global__ __launch_bounds__(KW * 64) void gemm_flex_kernel(GemmArgs g) {
-    using TA = FlexTile<BM, A_KSTR>;
-    using TB = FlexTile<BN, B_KSTR>;
+    using TA = FlexTile<CT, BM, A_KSTR, WORDS>;
+    using TB = FlexTile<CT, BN, B_KSTR, WORDS>;
+    constexpr int kSize = TA::kSize, KT = TA::kStep;
     constexpr int FM = BM / 32, FN = BN / 32;
     constexpr int kStageBytes = TA::kBytes + TB::kBytes;
     constexpr int kLoads = TA::kInstr + TB::kInstr;
     constexpr int kWaveBytes = ST * kStageBytes;
     static_assert(kWaveBytes >= BM * BN * 4, "a wave's buffers hold its accumulators at the end");
     static_assert(KW * kWaveBytes <= 160 * 1024, "LDS");
+    static_assert((ST - 1) * kLoads <= 63, "loads a partial wait can leave outstanding");
     __shared__ __attribute__((aligned(1024))) unsigned char lds_raw[KW * kWaveBytes];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -116,20 +159,21 @@ __global__ __launch_bounds__(KW * 64) void gemm_flex_kernel(GemmArgs g) {
     const int k_end = sliced && k_begin + g.k_slice < g.k ? k_begin + g.k_slice : (int)g.k;
 
     // this wave's first K step, and where each operand ends as seen from it
-    const int k0 = k_begin + wave * 64;
-    const int steps = (k_end - k_begin + 63) >> 6;
+    const int k0 = k_begin + wave * KT;
+    const int steps = (k_end - k_begin + KT - 1) / KT;
     const int mine = steps > wave ? (steps - wave + KW - 1) / KW : 0;
     const long long a_at = (sliced ? 0 : b * g.sa) + (A_KSTR ? (long long)k0 * g.lda + row0 : (long long)row0 * g.lda + k0);
     const long long b_at = (sliced ? 0 : b * g.sb) + (B_KSTR ? (long long)k0 * g.ldb + col0 : (long long)col0 * g.ldb + k0);
-    const unsigned char* a_src = static_cast<const unsigned char*>(g.a) + 2 * a_at;
-    const unsigned char* b_src = static_cast<const unsigned char*>(g.b) + 2 * b_at;
+    const unsigned char* a_src = static_cast<const unsigned char*>(g.a) + kSize * a_at;
+    const unsigned char* b_src = static_cast<const unsigned char*>(g.b) + kSize * b_at;
     // rounded up to the 16-byte granule the last element lies in
+    constexpr long long kRound = WORDS ? 3 : 15;
     long long a_left = ((A_KSTR ? (long long)(k_end - 1 - k0) * g.lda + g.m - row0
-                                : (g.m - 1 - row0) * g.lda + (k_end - k0)) * 2 + 15) & ~15LL;
+                                : (g.m - 1 - row0) * g.lda + (k_end - k0)) * kSize + kRound) & ~kRound;
     long long b_left = ((B_KSTR ? (long long)(k_end - 1 - k0) * g.ldb + g.n - col0
-                                : (g.n - 1 - col0) * g.ldb + (k_end - k0)) * 2 + 15) & ~15LL;
-    const long long a_step = (A_KSTR ? g.lda : 1) * (2LL * 64 * KW);
-    const long long b_step = (B_KSTR ? g.ldb : 1) * (2LL * 64 * KW);
+                                : (g.n - 1 - col0) * g.ldb + (k_end - k0)) * kSize + kRound) & ~kRound;
+    const long long a_step = (A_KSTR ? g.lda : 1) * ((long long)kSize * KT * KW);
+    const long long b_step = (B_KSTR ? g.ldb : 1) * ((long long)kSize * KT * KW);
     int k_left = k_end - k0;
     unsigned a_off[TA::kInstr], b_off[TB::kInstr];
 #pragma unroll
@@ -143,16 +187,16 @@ __global__ __launch_bounds__(KW * 64) void gemm_flex_kernel(GemmArgs g) {
         const buffer_rsrc ra = buffer_from(a_src, a_left), rb = buffer_from(b_src, b_left);
         const unsigned dst = mem0 + (unsigned)stage * kStageBytes;
         // a k-contiguous operand's last step: chunks past K are fetched from past the end of the operand
-        const bool tail = k_left < 64;
+        const bool tail = k_left < KT;
 #pragma unroll
         for (int q = 0; q < TA::kInstr; q++)
-            buffer_dtl_load(dst + q * 1024, !A_KSTR && tail && TA::k_of(q, lane) >= k_left ? kPastEnd : a_off[q], ra);
+            TA::load(dst, q, !A_KSTR && tail && TA::k_of(q, lane) >= k_left ? kPastEnd : a_off[q], ra);
 #pragma unroll
         for (int q = 0; q < TB::kInstr; q++)
-            buffer_dtl_load(dst + TA::kBytes + q * 1024, !B_KSTR && tail && TB::k_of(q, lane) >= k_left ? kPastEnd : b_off[q], rb);
+            TB::load(dst + TA::kBytes, q, !B_KSTR && tail && TB::k_of(q, lane) >= k_left ? kPastEnd : b_off[q], rb);
         a_src += a_step; a_left -= a_step;
         b_src += b_step; b_left -= b_step;
-        k_left -= 64 * KW;
+        k_left -= KT * KW;
     };
 
     f32x16 acc[FM][FN];
@@ -187,13 +231,22 @@ __global__ __launch_bounds__(KW * 64) void gemm_flex_kernel(GemmArgs g) {
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         if (t + ST < mine) issue(stage);
         stage = stage + 1 == ST ? 0 : stage + 1;
-        // operands swapped: a lane then holds four consecutive columns of one row of C
+        // Operands swapped: a lane then holds four consecutive columns of one row of C.  fp32: product s of a sub-step
+        // multiplies slot s of both halves of the wave, two k-values; the blocks take turns, so that no product waits
+        // for the one before it.
 #pragma unroll
         for (int ks = 0; ks < 4; ks++)
 #pragma unroll
-            for (int i = 0; i < FM; i++)
+            for (int s = 0; s < (CT == BR_GEMM_F32 ? 4 : 1); s++)
 #pragma unroll
-                for (int j = 0; j < FN; j++) acc[i][j] = Cvt<CT>::mfma(fb[ks][j], fa[ks][i], acc[i][j]);
+                for (int i = 0; i < FM; i++)
+#pragma unroll
+                    for (int j = 0; j < FN; j++) {
+                        if constexpr (CT == BR_GEMM_F32)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fb[ks][j][s]), __uint_as_float(fa[ks][i][s]), acc[i][j], 0, 0, 0);
+                        else
+                            acc[i][j] = Cvt<CT>::mfma(fb[ks][j], fa[ks][i], acc[i][j]);
+                    }
     }
 
     // acc[i][j][v] is C[row, col] with row = i*32 + lane%32, col = j*32 + (v/4)*8 + (lane/32)*4 + v%4.  Each wave
@@ -301,6 +354,29 @@ int launch_flex(const GemmArgs& g, const Problem& p, int kernel, long long batch
     if (kernel == kFlex64Short) return launch_flex_config<CT, 64, 64, 2, 1>(g, p, batch, st);
     if (kernel == kFlex32x64) return launch_flex_config<CT, 32, 64, 4, 1>(g, p, batch, st);
     return launch_flex_config<CT, 32, 32, 4, 2>(g, p, batch, st);
+}
+
+// fp32 operands and C.  `words`: an operand's rows are not aligned to 16 bytes (or a k-contiguous one's do not end on
+// such a boundary), so it is loaded value by value.
+template <int BM, int BN, bool WORDS>
+int launch_flex_fp32(GemmArgs g, const Problem& p, long long batch, hipStream_t st) {
+    constexpr int KW = 4;
+    g.tiles_m = (int)((g.m + BM - 1) / BM);
+    g.tiles_n = (int)((g.n + BN - 1) / BN);
+    const long long blocks = (long long)g.tiles_m * g.tiles_n * batch;
+    if (blocks > 0x7fffffffLL) return BR_ERR_ATTR;
+    const unsigned grid = (unsigned)blocks;
+    g.vec_c = g.ldc % 4 == 0 && g.sc % 4 == 0 && aligned16(g.c);
+    if (p.a_kstr && p.b_kstr)
+        gemm_flex_kernel<BR_GEMM_F32, BM, BN, KW, 1, true, true, float, false, WORDS><<<grid, KW * 64, 0, st>>>(g);
+    else if (p.a_kstr)
+        gemm_flex_kernel<BR_GEMM_F32, BM, BN, KW, 1, true, false, float, false, WORDS><<<grid, KW * 64, 0, st>>>(g);
+    else if (p.b_kstr)
+        gemm_flex_kernel<BR_GEMM_F32, BM, BN, KW, 1, false, true, float, false, WORDS><<<grid, KW * 64, 0, st>>>(g);
+    else
+        gemm_flex_kernel<BR_GEMM_F32, BM, BN, KW, 1, false, false, float, false, WORDS><<<grid, KW * 64, 0, st>>>(g);
+    BR_HIP_LAUNCH_CHECK();
+    return BR_OK;
 }
 
 }  // namespace gemm16

@@ -76,8 +76,8 @@ struct GemmArgs {
     int splits = 1;
     float* partials = nullptr;
     size_t partial_bytes = 0;
-    int k_slice = 0;      // gemm_flex16.hpp: with splits > 1, the k-values of one slice (a multiple of 64)
-    int vec_c = 0;        // gemm_flex16.hpp: rows of C (and of c2) can be written four elements at a time
+    int k_slice = 0;      // gemm_flex.hpp: with splits > 1, the k-values of one slice (a multiple of 64)
+    int vec_c = 0;        // gemm_flex.hpp: rows of C (and of c2) can be written four elements at a time
     int split_slot = 0;   // which set of the library's arrival counters the two slices of a tile meet through (one per stream)
 };
 

@@ -35,7 +35,7 @@ constexpr KernelCost kCost[kKernels] = {
     {256, 128, 1, 256, 3.07, 0.840, 1.048, 0.89},    // 8 waves of 64 x 64
     {256, 128, 1, 256, 3.09, 0.789, 0.993, 2.48},    // two groups of four 64 x 128 waves
     {128, 128, 1, 512, 2.80, 0.737, 0.606, 0.00},    // 4 waves of 64 x 64
-    {64, 64, 4, 512, 2.71, 0.856, 0.970, 1.44},      // gemm_flex16.hpp, K dealt to 4 waves
+    {64, 64, 4, 512, 2.71, 0.856, 0.970, 1.44},      // gemm_flex.hpp, K dealt to 4 waves
     {64, 64, 2, 1024, 2.84, 0.745, 0.449, 1.99},     // ... to 2 waves, for many tiles or a short K
     {32, 64, 4, 768, 2.95, 0.681, 0.637, 0.44},
     {32, 32, 4, 512, 1.67, 0.472, 0.435, 1.15},
@@ -133,6 +133,22 @@ inline int flex_kernel(long long m, long long n, long long k, long long batch) {
     int best = kFlex64;
     for (int c = kFlex64; c < kKernels; c++)
         if (kernel_us(c, m, n, k, batch) < kernel_us(best, m, n, k, batch)) best = c;
+    return best;
+}
+
+// fp32 products (gemm_flex.hpp): the tile whose matrix instructions finish first.  A step of 32 k-values takes a wave
+// 64 / 32 / 16 instructions of 64 clocks; measured with everything around them 2.45 / 1.4 / 0.78 us per step and
+// workgroup of a CU, and 2.7 us besides.  A CU that holds one workgroup more than the others sets the time.
+inline int fp32_kernel(long long m, long long n, long long k, long long batch) {
+    auto us = [&](int kernel, double per_step) {
+        const KernelCost& c = kCost[kernel];
+        const double load = (double)(ceil_div(m, c.bm) * ceil_div(n, c.bn) * batch) / 256.0;
+        return 2.7 + (load >= 4.0 ? load : ceil(load)) * (double)ceil_div(ceil_div(k, 32), 4) * per_step;
+    };
+    int best = kFlex64;
+    double t = us(kFlex64, 2.45);
+    if (us(kFlex32x64, 1.4) < 0.98 * t) best = kFlex32x64, t = us(kFlex32x64, 1.4);
+    if (us(kFlex32, 0.78) < 0.98 * t) best = kFlex32;
     return best;
 }
 

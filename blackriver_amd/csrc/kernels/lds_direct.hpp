@@ -43,6 +43,17 @@ __device__ __forceinline__ void buffer_dtl_load(unsigned lds_dst, unsigned voff,
         : "memory");
 }
 
+// The 32-bit form: 4 bytes a lane, to LDS byte lds_dst + 4*l.
+__device__ __forceinline__ void buffer_dtl_load_dword(unsigned lds_dst, unsigned voff, const buffer_rsrc& rsrc) {
+    asm volatile(
+        "s_mov_b32 m0, %0\n\t"
+        "s_nop 0\n\t"
+        "buffer_load_dword %1, %2, 0 offen lds"
+        :
+        : "s"(lds_dst), "v"(voff), "s"(rsrc)
+        : "memory");
+}
+
 // A raw buffer of `left` bytes (none if negative) at p; kPastEnd lies beyond the end of any.
 constexpr unsigned kPastEnd = 0x7ffffff0u;
 __device__ __forceinline__ buffer_rsrc buffer_from(const unsigned char* p, long long left) {

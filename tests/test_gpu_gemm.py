@@ -459,3 +459,27 @@ def test_gemm_small_and_ragged_products_are_exact_on_integers(ta, tb, c_dt, m, n
     if c_dt == F16:
         ref = ref.astype(np.float16).astype(np.float64)
     assert np.array_equal(to_host64(c).reshape(batch, m, n), ref)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k,batch", [
+    (1, 4, 4, 1),
+    (33, 36, 40, 2),         # 32 x 32 tiles, rows in 16-byte granules
+    (64, 1024, 260, 1),      # K dealt unevenly to the four waves
+    (512, 1028, 1024, 1),    # 32 x 64 tiles
+    (1000, 1028, 36, 4),     # 64 x 64 tiles
+    (31, 65, 7, 2),          # value by value: everything odd
+    (333, 64, 333, 3),       # attention products of 333 tokens
+    (1001, 2050, 70, 2),     # 64 x 64 tiles, value by value
+])
+def test_gemm_fp32_small_tiles_are_exact_on_integers(ta, tb, m, n, k, batch):
+    """The fp32 kernel's tiles and both ways it loads its operands, on small integers: every partial sum is exact."""
+    print("case ta=%d tb=%d m=%d n=%d k=%d batch=%d" % (ta, tb, m, n, k, batch), flush=True)
+    rng = np.random.default_rng(m + n + k)
+    a, b = operands(rng, ta, tb, m, n, k, batch)
+    a = rng.integers(-3, 4, a.shape).astype(np.float32)
+    b = rng.integers(-2, 3, b.shape).astype(np.float32)
+    bias = rng.integers(-5, 6, n).astype(np.float32)
+    c0 = rng.integers(-9, 10, (batch, m, n)).astype(np.float32)
+    got, ref = run_gemm(ta, tb, m, n, k, a, b, F32, F32, F32, hip.GEMM_F32, batch=batch, bias=bias, c0=c0)
+    assert np.array_equal(got, ref)
