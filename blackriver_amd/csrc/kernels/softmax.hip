@@ -12,6 +12,8 @@
 
 #include <float.h>
 
+#include <initializer_list>
+
 using namespace brk;
 
 namespace {
@@ -32,38 +34,87 @@ struct RowBias {
 // Scores, probabilities and their gradients are read once and written once: streaming (non-temporal) accesses,
 // measured at [4,32,512,512] fp32 on one box: forward 55.4 us plain, 54.5 with streaming loads, 51.0 with streaming
 // stores too; backward 71 / 66.6 / 62.4.
-#ifndef BR_SM_STREAM
-#define BR_SM_STREAM 7   // one-wave-per-row kernels: bit 0 streaming loads, bit 1 streaming stores (forward), bit 2 (backward)
-#endif
-__device__ __forceinline__ float4 sm_load(const float4* p) {
-#if BR_SM_STREAM & 1
-    return load_stream(p);
-#else
-    return *p;
-#endif
-}
-template <int BIT>
-__device__ __forceinline__ void sm_store(float4* p, const float4& v) {
-    if (BR_SM_STREAM & BIT) store_stream(p, v);
-    else *p = v;
-}
+// Rows are held in granules of G floats: four where rows are 16-byte aligned, two or one where an odd number of
+// tokens leaves them on 8- or 4-byte boundaries (three sweeps over such a row by a workgroup took 30 us forward and
+// 18 backward for the scores of 4 x 16 heads of 250 tokens; a row in one wave's registers takes 7 and 8).
+template <int G>
+struct Granule;
+template <>
+struct Granule<4> {
+    static __device__ __forceinline__ void load(const float* p, float (&v)[4]) {
+        const float4 t = load_stream(reinterpret_cast<const float4*>(p));
+        v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+    }
+    static __device__ __forceinline__ void load_cached(const float* p, float (&v)[4]) {
+        const float4 t = *reinterpret_cast<const float4*>(p);
+        v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+    }
+    static __device__ __forceinline__ void store(float* p, const float (&v)[4]) {
+        store_stream(reinterpret_cast<float4*>(p), make_float4(v[0], v[1], v[2], v[3]));
+    }
+    static __device__ __forceinline__ float sum(const float (&v)[4]) { return (v[0] + v[1]) + (v[2] + v[3]); }
+    static __device__ __forceinline__ float max(const float (&v)[4]) { return fmaxf(fmaxf(v[0], v[1]), fmaxf(v[2], v[3])); }
+    // also pins v to the values that are stored (see store4_as16)
+    static __device__ __forceinline__ void store16(const Copy16& c, int64_t at, float (&v)[4]) {
+        float4 t = make_float4(v[0], v[1], v[2], v[3]);
+        store4_as16(c, at / 4, t);
+        v[0] = t.x; v[1] = t.y; v[2] = t.z; v[3] = t.w;
+    }
+};
+template <>
+struct Granule<2> {
+    static __device__ __forceinline__ void load(const float* p, float (&v)[2]) {
+        const float2 t = *reinterpret_cast<const float2*>(p);
+        v[0] = t.x; v[1] = t.y;
+    }
+    static __device__ __forceinline__ void load_cached(const float* p, float (&v)[2]) { load(p, v); }
+    static __device__ __forceinline__ void store(float* p, const float (&v)[2]) {
+        *reinterpret_cast<float2*>(p) = make_float2(v[0], v[1]);
+    }
+    static __device__ __forceinline__ float sum(const float (&v)[2]) { return v[0] + v[1]; }
+    static __device__ __forceinline__ float max(const float (&v)[2]) { return fmaxf(v[0], v[1]); }
+    static __device__ __forceinline__ void store16(const Copy16& c, int64_t at, float (&v)[2]) {
+        asm volatile("" : "+v"(v[0]), "+v"(v[1]));
+        if (!c.base) return;
+        auto bits = [&](float f) {
+            return (unsigned)(c.bf16 ? __builtin_bit_cast(unsigned short, __float2bfloat16(f))
+                                     : __builtin_bit_cast(unsigned short, __float2half_rn(f)));
+        };
+        static_cast<unsigned*>(c.base)[at / 2] = bits(v[0]) | (bits(v[1]) << 16);
+    }
+};
+template <>
+struct Granule<1> {
+    static __device__ __forceinline__ void load(const float* p, float (&v)[1]) { v[0] = *p; }
+    static __device__ __forceinline__ void load_cached(const float* p, float (&v)[1]) { v[0] = *p; }
+    static __device__ __forceinline__ void store(float* p, const float (&v)[1]) { *p = v[0]; }
+    static __device__ __forceinline__ float sum(const float (&v)[1]) { return v[0]; }
+    static __device__ __forceinline__ float max(const float (&v)[1]) { return v[0]; }
+    static __device__ __forceinline__ void store16(const Copy16&, int64_t, float (&)[1]) {}   // not offered at odd widths
+};
 
 // exp(x - m) for x <= m, via the hardware exp2
 __device__ __forceinline__ float exp_sub(float x, float m) { return __expf(x - m); }
 
-// VPL = float4 vectors per lane; cols = 4 * cols4 <= 256 * VPL.
-template <int VPL, int MODE>
+// VPL granules of G floats per lane; cols = G * granules <= 64 * G * VPL.
+template <int VPL, int MODE, int G>
 __global__ __launch_bounds__(kBlock) void softmax_fwd_wave(const float* __restrict__ x, float* __restrict__ y,
-                                                            int64_t rows, int cols4, RowBias rb, Copy16 y16) {
+                                                            int64_t rows, int granules, RowBias rb, Copy16 y16) {
+    using Gr = Granule<G>;
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
     if (row >= rows) return;
-    const float4* xr = reinterpret_cast<const float4*>(x) + row * cols4;
-    float4 v[VPL];
+    const float* xr = x + row * granules * G;
+    float v[VPL][G];
 #pragma unroll
     for (int i = 0; i < VPL; i++) {
         const int idx = lane + i * kWave;
-        v[i] = idx < cols4 ? sm_load(xr + idx) : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+        if (idx < granules) {
+            Gr::load(xr + idx * G, v[i]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < G; j++) v[i][j] = -INFINITY;
+        }
     }
     if (MODE != kPlain) {
         // row = (b * heads + h) * tq + q
@@ -72,20 +123,22 @@ __global__ __launch_bounds__(kBlock) void softmax_fwd_wave(const float* __restri
         const int h = (int)(bh % rb.heads);
         const int64_t b = bh / rb.heads;
         if (MODE == kTables) {
-            const float4* ar = rb.alibi ? reinterpret_cast<const float4*>(rb.alibi) + (int64_t)h * cols4 : nullptr;
-            const float4* mr =
-                rb.xmask ? reinterpret_cast<const float4*>(rb.xmask) + (b * rb.tq + q) * cols4 : nullptr;
+            const float* ar = rb.alibi ? rb.alibi + (int64_t)h * granules * G : nullptr;
+            const float* mr = rb.xmask ? rb.xmask + (b * rb.tq + q) * granules * G : nullptr;
 #pragma unroll
             for (int i = 0; i < VPL; i++) {
                 const int idx = lane + i * kWave;
-                if (idx < cols4) {
+                if (idx < granules) {
+                    float t[G];
                     if (ar) {
-                        const float4 a = ar[idx];
-                        v[i].x += a.x; v[i].y += a.y; v[i].z += a.z; v[i].w += a.w;
+                        Gr::load_cached(ar + idx * G, t);
+#pragma unroll
+                        for (int j = 0; j < G; j++) v[i][j] += t[j];
                     }
                     if (mr) {
-                        const float4 m = mr[idx];
-                        v[i].x += m.x; v[i].y += m.y; v[i].z += m.z; v[i].w += m.w;
+                        Gr::load_cached(mr + idx * G, t);
+#pragma unroll
+                        for (int j = 0; j < G; j++) v[i][j] += t[j];
                     }
                 }
             }
@@ -95,14 +148,13 @@ __global__ __launch_bounds__(kBlock) void softmax_fwd_wave(const float* __restri
 #pragma unroll
             for (int i = 0; i < VPL; i++) {
                 const int idx = lane + i * kWave;
-                if (idx < cols4) {
-                    float* e = reinterpret_cast<float*>(&v[i]);
+                if (idx < granules) {
 #pragma unroll
-                    for (int j = 0; j < 4; j++) {
-                        const int k = idx * 4 + j;
+                    for (int j = 0; j < G; j++) {
+                        const int k = idx * G + j;
                         // same two additions, in the same order, as the table form
-                        e[j] += (float)((double)k * 1.0 * slope);
-                        e[j] += (k <= q && k < valid) ? 0.0f : -FLT_MAX;
+                        v[i][j] += (float)((double)k * 1.0 * slope);
+                        v[i][j] += (k <= q && k < valid) ? 0.0f : -FLT_MAX;
                     }
                 }
             }
@@ -110,58 +162,67 @@ __global__ __launch_bounds__(kBlock) void softmax_fwd_wave(const float* __restri
     }
     float m = -INFINITY;
 #pragma unroll
-    for (int i = 0; i < VPL; i++) m = fmaxf(m, fmaxf(fmaxf(v[i].x, v[i].y), fmaxf(v[i].z, v[i].w)));
+    for (int i = 0; i < VPL; i++) m = fmaxf(m, Gr::max(v[i]));
     m = wave_max(m);
     float s = 0.f;
 #pragma unroll
     for (int i = 0; i < VPL; i++) {
-        v[i].x = exp_sub(v[i].x, m); v[i].y = exp_sub(v[i].y, m);
-        v[i].z = exp_sub(v[i].z, m); v[i].w = exp_sub(v[i].w, m);
-        s += (v[i].x + v[i].y) + (v[i].z + v[i].w);
+#pragma unroll
+        for (int j = 0; j < G; j++) v[i][j] = exp_sub(v[i][j], m);
+        s += Gr::sum(v[i]);
     }
     s = wave_sum(s);
     const float inv = 1.0f / s;
-    float4* yr = reinterpret_cast<float4*>(y) + row * cols4;
+    float* yr = y + row * granules * G;
 #pragma unroll
     for (int i = 0; i < VPL; i++) {
         const int idx = lane + i * kWave;
-        if (idx < cols4) {
-            float4 o = make_float4(v[i].x * inv, v[i].y * inv, v[i].z * inv, v[i].w * inv);
-            store4_as16(y16, row * cols4 + idx, o);
-            sm_store<2>(yr + idx, o);
+        if (idx < granules) {
+#pragma unroll
+            for (int j = 0; j < G; j++) v[i][j] *= inv;
+            Gr::store16(y16, (row * granules + idx) * G, v[i]);
+            Gr::store(yr + idx * G, v[i]);
         }
     }
 }
 
-template <int VPL>
+template <int VPL, int G>
 __global__ __launch_bounds__(kBlock) void softmax_bwd_wave(const float* __restrict__ dy, const float* __restrict__ y,
-                                                            float* __restrict__ dx, int64_t rows, int cols4,
+                                                            float* __restrict__ dx, int64_t rows, int granules,
                                                             Copy16 dx16) {
+    using Gr = Granule<G>;
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * kRowsPerBlock + (threadIdx.x >> 6);
     if (row >= rows) return;
-    const float4* gr = reinterpret_cast<const float4*>(dy) + row * cols4;
-    const float4* yr = reinterpret_cast<const float4*>(y) + row * cols4;
-    float4 g[VPL], p[VPL];
+    const float* gr = dy + row * granules * G;
+    const float* yr = y + row * granules * G;
+    float g[VPL][G], p[VPL][G];
     float dot = 0.f;
 #pragma unroll
     for (int i = 0; i < VPL; i++) {
         const int idx = lane + i * kWave;
-        const bool ok = idx < cols4;
-        g[i] = ok ? sm_load(gr + idx) : make_float4(0.f, 0.f, 0.f, 0.f);
-        p[i] = ok ? sm_load(yr + idx) : make_float4(0.f, 0.f, 0.f, 0.f);
-        dot += (g[i].x * p[i].x + g[i].y * p[i].y) + (g[i].z * p[i].z + g[i].w * p[i].w);
+        float t[G];
+        if (idx < granules) {
+            Gr::load(gr + idx * G, g[i]);
+            Gr::load(yr + idx * G, p[i]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < G; j++) g[i][j] = p[i][j] = 0.f;
+        }
+#pragma unroll
+        for (int j = 0; j < G; j++) t[j] = g[i][j] * p[i][j];
+        dot += Gr::sum(t);
     }
     dot = wave_sum(dot);
-    float4* dr = dx ? reinterpret_cast<float4*>(dx) + row * cols4 : nullptr;
 #pragma unroll
     for (int i = 0; i < VPL; i++) {
         const int idx = lane + i * kWave;
-        if (idx < cols4) {
-            float4 o = make_float4(p[i].x * (g[i].x - dot), p[i].y * (g[i].y - dot), p[i].z * (g[i].z - dot),
-                                   p[i].w * (g[i].w - dot));
-            store4_as16(dx16, row * cols4 + idx, o);
-            if (dx) sm_store<4>(dr + idx, o);  // dx == nullptr: only the 16-bit gradient is wanted
+        if (idx < granules) {
+            float o[G];
+#pragma unroll
+            for (int j = 0; j < G; j++) o[j] = p[i][j] * (g[i][j] - dot);
+            Gr::store16(dx16, (row * granules + idx) * G, o);
+            if (dx) Gr::store(dx + (row * granules + idx) * G, o);  // dx == nullptr: only the 16-bit gradient is wanted
         }
     }
 }
@@ -214,51 +275,72 @@ __global__ __launch_bounds__(kBlock) void softmax_bwd_generic(const float* dy, c
         dx[row * cols + c] = y[row * cols + c] * (dy[row * cols + c] - s[0]);
 }
 
+// Floats per granule for rows of `cols` floats at these addresses (null ones do not count).
+int granule_of(int64_t cols, std::initializer_list<const void*> at) {
+    int g = cols % 4 == 0 ? 4 : cols % 2 == 0 ? 2 : 1;
+    for (const void* p : at)
+        while (reinterpret_cast<uintptr_t>(p) % (4 * g) != 0) g /= 2;
+    return g;
+}
+constexpr int64_t kMaxRegisterRow = 2048;   // floats of a row in granules of fewer than four (32 registers of a lane)
+
+template <int MODE, int G>
+void launch_softmax_fwd_wave(const float* x, float* y, int64_t rows, int64_t cols, const RowBias& rb, hipStream_t st,
+                             Copy16 y16) {
+    const int granules = (int)(cols / G);
+    const unsigned grid = (unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock);
+    const int vpl = (granules + kWave - 1) / kWave;
+    if (vpl <= 1) softmax_fwd_wave<1, MODE, G><<<grid, kBlock, 0, st>>>(x, y, rows, granules, rb, y16);
+    else if (vpl <= 2) softmax_fwd_wave<2, MODE, G><<<grid, kBlock, 0, st>>>(x, y, rows, granules, rb, y16);
+    else if (vpl <= 4) softmax_fwd_wave<4, MODE, G><<<grid, kBlock, 0, st>>>(x, y, rows, granules, rb, y16);
+    else if (vpl <= 8) softmax_fwd_wave<8, MODE, G><<<grid, kBlock, 0, st>>>(x, y, rows, granules, rb, y16);
+    else if (vpl <= 16) softmax_fwd_wave<16, MODE, G><<<grid, kBlock, 0, st>>>(x, y, rows, granules, rb, y16);
+    else if constexpr (G == 1) softmax_fwd_wave<32, MODE, G><<<grid, kBlock, 0, st>>>(x, y, rows, granules, rb, y16);
+}
+
 template <int MODE>
 int launch_softmax_fwd(const float* x, float* y, int64_t rows, int64_t cols, const RowBias& rb, hipStream_t st,
                        Copy16 y16 = Copy16{nullptr, 0}) {
-    bool vec = cols % 4 == 0 && cols <= 256 * 16 && aligned16(x) && aligned16(y);
-    if (MODE == kTables)
-        vec = vec && (!rb.alibi || aligned16(rb.alibi)) && (!rb.xmask || aligned16(rb.xmask));
-    if (vec) {
-        const int cols4 = (int)(cols / 4);
-        const unsigned grid = (unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock);
-        const int vpl = (cols4 + kWave - 1) / kWave;
-        if (vpl <= 1)
-            softmax_fwd_wave<1, MODE><<<grid, kBlock, 0, st>>>(x, y, rows, cols4, rb, y16);
-        else if (vpl <= 2)
-            softmax_fwd_wave<2, MODE><<<grid, kBlock, 0, st>>>(x, y, rows, cols4, rb, y16);
-        else if (vpl <= 4)
-            softmax_fwd_wave<4, MODE><<<grid, kBlock, 0, st>>>(x, y, rows, cols4, rb, y16);
-        else if (vpl <= 8)
-            softmax_fwd_wave<8, MODE><<<grid, kBlock, 0, st>>>(x, y, rows, cols4, rb, y16);
-        else
-            softmax_fwd_wave<16, MODE><<<grid, kBlock, 0, st>>>(x, y, rows, cols4, rb, y16);
+    const int g = MODE == kTables ? granule_of(cols, {x, y, rb.alibi, rb.xmask}) : granule_of(cols, {x, y});
+    if (g == 4 && cols <= 256 * 16) {
+        launch_softmax_fwd_wave<MODE, 4>(x, y, rows, cols, rb, st, y16);
+    } else if (g == 2 && cols <= kMaxRegisterRow) {
+        launch_softmax_fwd_wave<MODE, 2>(x, y, rows, cols, rb, st, y16);
     } else {
-        if (y16.base) return BR_ERR_TODO;  // the copy is only produced by the one-wave-per-row path
-        softmax_fwd_generic<MODE><<<(unsigned)rows, kBlock, 0, st>>>(x, y, cols, rb);
+        if (y16.base) return BR_ERR_TODO;  // the copy is written two or four values at a time
+        if (cols <= kMaxRegisterRow) launch_softmax_fwd_wave<MODE, 1>(x, y, rows, cols, rb, st, y16);
+        else softmax_fwd_generic<MODE><<<(unsigned)rows, kBlock, 0, st>>>(x, y, cols, rb);
     }
     BR_HIP_LAUNCH_CHECK();
     return BR_OK;
 }
 
-bool softmax_bwd_wave_ok(int64_t cols, const void* dy, const void* y, const void* dx) {
-    return cols % 4 == 0 && cols <= 256 * 8 && aligned16(dy) && aligned16(y) && aligned16(dx);
+// Granule of the one-wave-per-row backward, 0 where rows do not fit it.
+int softmax_bwd_granule(int64_t cols, const void* dy, const void* y, const void* dx) {
+    const int g = granule_of(cols, {dy, y, dx});
+    return cols <= kMaxRegisterRow ? g : 0;
 }
 
-int launch_softmax_bwd_wave(const float* dy, const float* y, float* dx, Copy16 dx16, int64_t rows, int64_t cols,
-                            hipStream_t st) {
-    const int cols4 = (int)(cols / 4);
+template <int G>
+void launch_softmax_bwd_granules(const float* dy, const float* y, float* dx, Copy16 dx16, int64_t rows, int64_t cols,
+                                 hipStream_t st) {
+    const int granules = (int)(cols / G);
     const unsigned grid = (unsigned)((rows + kRowsPerBlock - 1) / kRowsPerBlock);
-    const int vpl = (cols4 + kWave - 1) / kWave;
-    if (vpl <= 1)
-        softmax_bwd_wave<1><<<grid, kBlock, 0, st>>>(dy, y, dx, rows, cols4, dx16);
-    else if (vpl <= 2)
-        softmax_bwd_wave<2><<<grid, kBlock, 0, st>>>(dy, y, dx, rows, cols4, dx16);
-    else if (vpl <= 4)
-        softmax_bwd_wave<4><<<grid, kBlock, 0, st>>>(dy, y, dx, rows, cols4, dx16);
-    else
-        softmax_bwd_wave<8><<<grid, kBlock, 0, st>>>(dy, y, dx, rows, cols4, dx16);
+    const int vpl = (granules + kWave - 1) / kWave;
+    if (vpl <= 1) softmax_bwd_wave<1, G><<<grid, kBlock, 0, st>>>(dy, y, dx, rows, granules, dx16);
+    else if (vpl <= 2) softmax_bwd_wave<2, G><<<grid, kBlock, 0, st>>>(dy, y, dx, rows, granules, dx16);
+    else if (vpl <= 4) softmax_bwd_wave<4, G><<<grid, kBlock, 0, st>>>(dy, y, dx, rows, granules, dx16);
+    else if (vpl <= 8) softmax_bwd_wave<8, G><<<grid, kBlock, 0, st>>>(dy, y, dx, rows, granules, dx16);
+    else if constexpr (G <= 2) {
+        if (vpl <= 16) softmax_bwd_wave<16, G><<<grid, kBlock, 0, st>>>(dy, y, dx, rows, granules, dx16);
+        else if constexpr (G == 1) softmax_bwd_wave<32, G><<<grid, kBlock, 0, st>>>(dy, y, dx, rows, granules, dx16);
+    }
+}
+int launch_softmax_bwd_wave(int g, const float* dy, const float* y, float* dx, Copy16 dx16, int64_t rows, int64_t cols,
+                            hipStream_t st) {
+    if (g == 4) launch_softmax_bwd_granules<4>(dy, y, dx, dx16, rows, cols, st);
+    else if (g == 2) launch_softmax_bwd_granules<2>(dy, y, dx, dx16, rows, cols, st);
+    else launch_softmax_bwd_granules<1>(dy, y, dx, dx16, rows, cols, st);
     BR_HIP_LAUNCH_CHECK();
     return BR_OK;
 }
@@ -483,7 +565,8 @@ int br_hip_softmax_bwd(const float* dy, const float* y, float* dx, int64_t rows,
     if (!dy || !y) return BR_ERR_INPUT;
     if (!dx) return BR_ERR_OUTPUT;
     hipStream_t st = as_stream(stream);
-    if (softmax_bwd_wave_ok(cols, dy, y, dx)) return launch_softmax_bwd_wave(dy, y, dx, Copy16{nullptr, 0}, rows, cols, st);
+    const int g = softmax_bwd_granule(cols, dy, y, dx);
+    if (g > 0) return launch_softmax_bwd_wave(g, dy, y, dx, Copy16{nullptr, 0}, rows, cols, st);
     softmax_bwd_generic<<<(unsigned)rows, kBlock, 0, st>>>(dy, y, dx, cols);
     BR_HIP_LAUNCH_CHECK();
     return BR_OK;
@@ -495,8 +578,9 @@ int br_hip_softmax_bwd_to16(const float* dy, const float* y, void* dx16, int dx1
     if (rows == 0) return BR_OK;
     if (!dy || !y) return BR_ERR_INPUT;
     if (!dx16 || dx16 == (const void*)dy || dx16 == (const void*)y) return BR_ERR_OUTPUT;
-    if (!copy16_ok(dx16, dx16_dtype) || !softmax_bwd_wave_ok(cols, dy, y, dy)) return BR_ERR_TODO;
-    return launch_softmax_bwd_wave(dy, y, nullptr, Copy16{dx16, dx16_dtype == BR_BF16}, rows, cols, as_stream(stream));
+    const int g = softmax_bwd_granule(cols, dy, y, dy);
+    if (!copy16_ok(dx16, dx16_dtype) || g < 2) return BR_ERR_TODO;
+    return launch_softmax_bwd_wave(g, dy, y, nullptr, Copy16{dx16, dx16_dtype == BR_BF16}, rows, cols, as_stream(stream));
 }
 
 int br_hip_alibi_masked_softmax_fwd(const float* s, const float* alibi, const float* xmask, float* p,

@@ -257,6 +257,36 @@ def test_softmax_16_bit_outputs_are_the_cast_of_the_fp32_outputs(b, h, t, dtype,
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("b,h,t", [(2, 3, 250), (1, 2, 66), (1, 2, 333), (1, 1, 1), (1, 2, 65), (1, 1, 2046), (1, 1, 2047)])
+def test_softmax_of_rows_on_8_and_4_byte_boundaries(b, h, t):
+    """Token counts that leave the rows of [B, heads, T, T] unaligned: the fused score softmax and the backward
+    against the oracle's operators (32-bit sums: 1e-5), and for even counts the 16-bit outputs against the cast of
+    the fp32 ones, bit for bit."""
+    print("case b=%d h=%d t=%d" % (b, h, t), flush=True)
+    rng = np.random.default_rng(t)
+    s = rng.standard_normal((b, h, t, t)).astype(np.float32)
+    alibi = orc.alibi(h, t)
+    mask = np.ones((b, t), np.int32)
+    mask[0, t - t // 5:] = 0
+    xmask = orc.xmask(mask)
+    ds, da, dm = dev(s), dev(alibi), dev(xmask)
+    p = empty(s.shape)
+    call("br_hip_alibi_masked_softmax_fwd", ptr(ds), ptr(da), ptr(dm), ptr(p), b, h, t, t, stream())
+    ref = orc.softmax_fwd(orc.add_bcast(orc.add_bcast(s, alibi.reshape(1, h, 1, t)), xmask.reshape(b, 1, t, t)))
+    assert_close(host(p), ref, 1e-5, "forward")
+    dp = rng.standard_normal(s.shape).astype(np.float32)
+    g = empty(s.shape)
+    call("br_hip_softmax_bwd", ptr(dev(dp)), ptr(p), ptr(g), b * h * t, t, stream())
+    assert_close(host(g), orc.softmax_bwd(dp, host(p)), 1e-5, "backward")
+    if t % 2 == 0:
+        p2, p16, g16 = empty(s.shape), empty(s.shape, torch.float16), empty(s.shape, torch.float16)
+        call("br_hip_alibi_masked_softmax_fwd_copy16", ptr(ds), ptr(da), ptr(dm), ptr(p2), ptr(p16), F16, b, h, t, t, stream())
+        assert torch.equal(p2, p) and torch.equal(p16, p.half())
+        call("br_hip_softmax_bwd_to16", ptr(dev(dp)), ptr(p), ptr(g16), F16, b * h * t, t, stream())
+        assert torch.equal(g16, g.half())
+    torch.cuda.synchronize()
+
+
 def test_softmax_16_bit_outputs_decline_rows_the_wave_kernel_cannot_hold():
     lib = hip.load()
     rows, cols = 3, 1001
