@@ -252,9 +252,10 @@ __global__ __launch_bounds__(64 * G * KH, 2) void flash_fwd_kernel(FlashArgs a) 
         kv_fill.fill(st + kTileBytes, a.v + base, a.row, t * kBK, a.tokens, wave);
         fill_row(st + 2 * kTileBytes, alibi_row, t * kBK, a.tokens, lane);
     };
+    // the first tile travels together with the query fragments: one memory latency, not two
+    issue(0, 0);
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) landed(qf[ks]);
-    issue(0, 0);
     wait_vmem<0>();
     __syncthreads();
     // one key tile; the stage is a compile-time constant so that every LDS
@@ -422,7 +423,7 @@ __global__ __launch_bounds__(64 * G * QH) void flash_bwd_dkv_kernel(FlashArgs a)
     constexpr int NQB = 2 / QH;        // 32-query blocks of a tile per wave
     constexpr int kSpan = kBK / QH;    // queries of a tile per wave
     __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kQStageBytes];
-    static_assert(2 * kQStageBytes >= G * 64 * 64 * 4, "the merge puts G blocks of 64 x 64 floats into the stages");
+    static_assert(QH == 1 || 2 * kQStageBytes >= G * 2 * 64 * 64 * 4, "the merge puts 2 G blocks of 64 x 64 floats into the stages");
     const int lane = threadIdx.x & 63, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: branches on it are scalar
     const int kg = QH == 1 ? wave : wave % G, qh = QH == 1 ? 0 : wave / G;
@@ -471,13 +472,13 @@ __global__ __launch_bounds__(64 * G * QH) void flash_bwd_dkv_kernel(FlashArgs a)
         fill_row(st + 2 * kTileBytes, a.lse + (long long)bh * a.tokens, r0, a.tokens, lane);
         fill_row(st + 2 * kTileBytes + kBK * 4, a.delta + (long long)bh * a.tokens, r0, a.tokens, lane);
     };
+    if (ntiles > 0) issue(0, 0);
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) {
         landed(kf[ks]);
         landed(vf[ks]);
     }
     landed(bias);
-    if (ntiles > 0) issue(0, 0);
     wait_vmem<0>();
     __syncthreads();
     auto tile_step = [&](auto stage_c, int t) {
@@ -557,35 +558,39 @@ __global__ __launch_bounds__(64 * G * QH) void flash_bwd_dkv_kernel(FlashArgs a)
     }
 
     if (QH == 2) {
-        // the waves with the odd query halves hand their sums over, dK first, then dV (every wave is past the loop's
-        // last barrier: the stages are free)
-        float* const x = reinterpret_cast<float*>(lds) + kg * (64 * 64);
-        if (qh == 1) {
-#pragma unroll
-            for (int db = 0; db < 4; db++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) x[(db * 16 + v) * 64 + lane] = dk[db][v];
-        }
-        __syncthreads();
-        if (qh == 0) {
-#pragma unroll
-            for (int db = 0; db < 4; db++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) dk[db][v] += x[(db * 16 + v) * 64 + lane];
-        }
-        __syncthreads();
-        if (qh == 1) {
-#pragma unroll
-            for (int db = 0; db < 4; db++)
-#pragma unroll
-                for (int v = 0; v < 16; v++) x[(db * 16 + v) * 64 + lane] = dv[db][v];
-        }
-        __syncthreads();
-        if (qh == 1) return;
+        // Every wave is past the loop's last barrier: the stages are free.  The two waves of a key group trade sums,
+        // one takes dK and the other dV, so that adding and storing is shared (8 heads x 78 tokens: 14.1 -> 13.2 us
+        // with the first tile's loads issued ahead of the wait for the key fragments).
+        float* const give = reinterpret_cast<float*>(lds) + (kg * 2 + (1 - qh)) * (64 * 64);
+        const float* const take = reinterpret_cast<float*>(lds) + (kg * 2 + qh) * (64 * 64);
 #pragma unroll
         for (int db = 0; db < 4; db++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) dv[db][v] += x[(db * 16 + v) * 64 + lane];
+            for (int v = 0; v < 16; v++) give[(db * 16 + v) * 64 + lane] = qh == 0 ? dv[db][v] : dk[db][v];
+        __syncthreads();
+#pragma unroll
+        for (int db = 0; db < 4; db++)
+#pragma unroll
+            for (int v = 0; v < 16; v++) {
+                // the half with the smaller queries first, whichever wave adds
+                const float t = take[(db * 16 + v) * 64 + lane];
+                dk[db][v] = qh == 0 ? dk[db][v] + t : t + dv[db][v];
+            }
+        const float scale = qh == 0 ? a.scale : 1.0f;
+        void* const out = qh == 0 ? a.dk : a.dv;
+#pragma unroll
+        for (int v = 0; v < 16; v++) {
+            const int kk = key0 + acc_row(v, lane);
+            if (kk < a.tokens) {
+                const long long off = base + (long long)kk * a.row + (lane & 31);
+#pragma unroll
+                for (int db = 0; db < 4; db++) {
+                    if (a.grad16) static_cast<u16*>(out)[off + db * 32] = Cvt<CT>::from_f32(dk[db][v] * scale);
+                    else static_cast<float*>(out)[off + db * 32] = dk[db][v] * scale;
+                }
+            }
+        }
+        return;
     }
 
     // accumulator element v of block db: key key0 + acc_row(v), d = 32 * db + lane % 32
@@ -680,13 +685,13 @@ __global__ __launch_bounds__(64 * G * KH, 2) void flash_bwd_dq_kernel(FlashArgs 
         kv_fill.fill(st + kTileBytes, a.v + base, a.row, t * kBK, a.tokens, wave);
         fill_row(st + 2 * kTileBytes, alibi_row, t * kBK, a.tokens, lane);
     };
+    issue(0, 0);
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) {
         landed(qf[ks]);
         landed(gf[ks]);
     }
     landed(lse);
-    issue(0, 0);
     wait_vmem<0>();
     __syncthreads();
     auto tile_step = [&](auto stage_c, int t) {
