@@ -492,12 +492,12 @@ __global__ __launch_bounds__(kBlock) void colsum_final(const float* partial, flo
     out[col] = acc * scale;
 }
 
-// Vector forms of the two stages (cols % VEC == 0, 16-byte aligned rows).
-// Stage 1: a thread owns VEC adjacent columns and sums a strip of rows, four
+// Vector forms of the two stages for fp32 (cols % 4 == 0, 16-byte aligned rows).
+// Stage 1: a thread owns four adjacent columns and sums a strip of rows, four
 // rows of loads in flight at a time.
-template <typename T, int VEC>
-__global__ __launch_bounds__(kBlock) void colsum_partial_vec(const T* __restrict__ x, float* __restrict__ partial,
+__global__ __launch_bounds__(kBlock) void colsum_partial_vec(const float* __restrict__ x, float* __restrict__ partial,
                                                               int64_t rows, int64_t cols, int rows_per_block) {
+    constexpr int VEC = 4;
     const int64_t col = ((int64_t)blockIdx.x * kBlock + threadIdx.x) * VEC;
     if (col >= cols) return;
     const StripWalk w = strip_walk(rows, rows_per_block);
@@ -509,7 +509,7 @@ __global__ __launch_bounds__(kBlock) void colsum_partial_vec(const T* __restrict
     for (; r + 3 * step < r1; r += 4 * step) {
         float v[4][VEC];
 #pragma unroll
-        for (int u = 0; u < 4; u++) VecIO<T, VEC>::load(x + (r + u * step) * cols + col, v[u]);
+        for (int u = 0; u < 4; u++) VecIO<float, VEC>::load(x + (r + u * step) * cols + col, v[u]);
 #pragma unroll
         for (int u = 0; u < 4; u++)
 #pragma unroll
@@ -517,7 +517,7 @@ __global__ __launch_bounds__(kBlock) void colsum_partial_vec(const T* __restrict
     }
     for (; r < r1; r += step) {
         float v[VEC];
-        VecIO<T, VEC>::load(x + r * cols + col, v);
+        VecIO<float, VEC>::load(x + r * cols + col, v);
 #pragma unroll
         for (int j = 0; j < VEC; j++) acc[j] += v[j];
     }
@@ -678,14 +678,12 @@ int colsum_vec_rows_per_block(int64_t rows, int64_t blocks_x) {
 }
 
 // ------------------------------------------------ column sums in one launch
-// A workgroup of 1024 threads owns 8 * VEC columns (128 bytes of a 16-bit row, 128 bytes of an fp32 row) and walks
-// ALL rows: 8 lanes per row, 128 rows per pass, UNROLL passes in flight.  No partial sums leave the workgroup and
-// there is no second launch; the 128 row slots are combined in LDS in a fixed order, so the result depends on the
-// shape alone.  Measured against the two launches: 16-bit [2048,12288] 11.4 against 15.5 us, [2048,16384] 14.3
-// against 18.9, [512,16384] 4.6 against 11.0; fp32 [512,4096] with a 16-bit copy 3.9 against 6.6 -- but fp32
-// [2048,4096] 17 against 13.4 (128 workgroups are too few for 50 MB) and the fp16 bias-GELU backward at [2048,16384]
-// 44.5 against 43.0 (its arithmetic wants more waves than 1024 threads per CU give), which therefore keep the two
-// launches above 1024 rows (colsum_owner_applies).  Whole BLOOM-7B1 step at 512 tokens: -0.9 %.  What is summed, and what else is written on the way, is the Source's business:
+// A workgroup of 1024 threads owns LPR * VEC columns (LPR = 8: 128 bytes of a row) and walks ALL rows: LPR lanes per
+// row, 1024 / LPR rows per pass, UNROLL passes in flight.  No partial sums leave the workgroup and there is no second
+// launch; the row slots of a wave are combined by lane exchanges, the waves in LDS, in a fixed order, so the result
+// depends on the shape alone.  What bounds it on few rows is latency -- launch, one pass of loads, the combination --
+// and on wide ones the CU's load rate; fewer lanes per row make more, shorter workgroups (owner_lanes has the
+// measurements).  What is summed, and what else is written on the way, is the Source's business:
 //   load(at, in)      the loads of one row position (all of a pass's loads are issued before any is used)
 //   finish(at, in)    leaves the values to be summed in in[0]; may store
 template <typename T, int V>
@@ -761,80 +759,96 @@ struct OwnBiasGeluBwd {
     }
 };
 
-constexpr int kOwnThreads = 1024, kOwnLanesPerRow = 8, kOwnRowsPerPass = kOwnThreads / kOwnLanesPerRow;
+constexpr int kOwnThreads = 1024;
 
-template <int UNROLL, typename Src>
+// Workgroup ids are dealt to the 8 XCDs in turn: the b-th of n takes a position such that an XCD's workgroups are
+// neighbours (strips narrower than a cache line share their lines in one L2).
+__device__ __forceinline__ unsigned xcd_contiguous(unsigned b, unsigned n) {
+    const unsigned per = n / 8, rem = n % 8, x = b % 8;
+    return x * per + (x < rem ? x : rem) + b / 8;
+}
+
+template <int LPR, int UNROLL, typename Src>
 __global__ __launch_bounds__(kOwnThreads) void colsum_owner_kernel(Src src_arg, float* __restrict__ out, int64_t rows,
                                                                    int64_t cols, float scale) {
-    constexpr int VEC = Src::VEC, NIN = Src::NIN, RPP = kOwnRowsPerPass, CW = kOwnLanesPerRow * VEC;
-    __shared__ float slots[RPP][CW + 1];
+    constexpr int VEC = Src::VEC, NIN = Src::NIN, RPP = kOwnThreads / LPR, CW = LPR * VEC, WAVES = kOwnThreads / 64;
+    __shared__ float slots[WAVES][CW];
     Src src = src_arg;
-    const int lr = threadIdx.x % kOwnLanesPerRow, rr = threadIdx.x / kOwnLanesPerRow;
-    const int64_t col = (int64_t)blockIdx.x * CW + lr * VEC;
+    const int lr = threadIdx.x % LPR, rr = threadIdx.x / LPR;
+    const int64_t strip = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int64_t col = strip * CW + lr * VEC;
     float acc[VEC];
 #pragma unroll
     for (int j = 0; j < VEC; j++) acc[j] = 0.f;
     if (col < cols) {
         src.init(col);
-        int64_t r = rr;
-        for (; r + (UNROLL - 1) * RPP < rows; r += UNROLL * RPP) {
+        for (int64_t r = rr; r < rows; r += UNROLL * RPP) {
             float in[UNROLL][NIN][VEC];
-#pragma unroll
-            for (int u = 0; u < UNROLL; u++) src.load((r + u * RPP) * cols + col, in[u]);
+            // positions past the last row read that row (every load of a pass leaves before the first is used)
 #pragma unroll
             for (int u = 0; u < UNROLL; u++) {
-                src.finish((r + u * RPP) * cols + col, in[u]);
+                const int64_t at = r + u * RPP;
+                src.load((at < rows ? at : rows - 1) * cols + col, in[u]);
+            }
 #pragma unroll
-                for (int j = 0; j < VEC; j++) acc[j] += in[u][0][j];
+            for (int u = 0; u < UNROLL; u++) {
+                if (r + u * RPP < rows) {
+                    src.finish((r + u * RPP) * cols + col, in[u]);
+#pragma unroll
+                    for (int j = 0; j < VEC; j++) acc[j] += in[u][0][j];
+                }
             }
         }
-        for (; r < rows; r += RPP) {
-            float in[NIN][VEC];
-            src.load(r * cols + col, in);
-            src.finish(r * cols + col, in);
-#pragma unroll
-            for (int j = 0; j < VEC; j++) acc[j] += in[0][j];
-        }
     }
+    // the 64 / LPR row slots of a wave meet by lane exchanges, the waves through LDS
 #pragma unroll
-    for (int j = 0; j < VEC; j++) slots[rr][lr * VEC + j] = acc[j];
+    for (int d = LPR; d < 64; d *= 2)
+#pragma unroll
+        for (int j = 0; j < VEC; j++) acc[j] += __shfl_xor(acc[j], d);
+    if ((threadIdx.x & 63) < LPR) {
+#pragma unroll
+        for (int j = 0; j < VEC; j++) slots[threadIdx.x >> 6][lr * VEC + j] = acc[j];
+    }
     __syncthreads();
-    // 1024 / CW threads per column take every (1024 / CW)-th slot, then one thread per column takes those
-    constexpr int SLICES = kOwnThreads / CW;
-    static_assert(SLICES <= RPP, "the second stage reuses the slots");
-    const int c = threadIdx.x % CW, s = threadIdx.x / CW;
-    float t = 0.f;
-    for (int k = s; k < RPP; k += SLICES) t += slots[k][c];
-    __syncthreads();
-    slots[s][c] = t;
-    __syncthreads();
-    if (s == 0) {
+    if (threadIdx.x < CW) {
         float z = 0.f;
-        for (int k = 0; k < SLICES; k++) z += slots[k][c];
-        const int64_t oc = (int64_t)blockIdx.x * CW + c;
+#pragma unroll
+        for (int k = 0; k < WAVES; k++) z += slots[k][threadIdx.x];
+        const int64_t oc = strip * CW + threadIdx.x;
         if (oc < cols) out[oc] = z * scale;
     }
 }
 
-// Where one launch beats two (measured, see above): enough column blocks to occupy the chip, and for 4-byte elements
-// (32 columns per workgroup, half as many workgroups) and the bias-GELU backward only up to 1024 rows.  Depends on the shape and the element
-// size alone, so entries that promise each other's bits (br_hip_colsum / br_hip_colsum_cast /
-// br_hip_gelu_bwd_colsum_cast on fp32) always agree on the path.
-#ifndef BR_COLSUM_OWNER
-#define BR_COLSUM_OWNER 3   // bit 0: plain sums and sums with a copy; bit 1: the bias-GELU backward
-#endif
-bool colsum_owner_applies(int64_t rows, int64_t cols, int elem_bytes, int kind = 1) {
-    if (!(BR_COLSUM_OWNER & kind)) return false;
-    const int64_t cw = kOwnLanesPerRow * (elem_bytes == 4 ? 4 : 8);
-    const int64_t blocks = (cols + cw - 1) / cw;
-    if (cols % (elem_bytes == 4 ? 4 : 8) != 0 || blocks < 96 || blocks > 0x7fffffffLL) return false;
-    return (elem_bytes == 2 && kind == 1) || rows <= 1024;
+// Lanes per row of the one-launch column sum, or 0 where two launches are faster.  Depends on the shape, the element
+// size and the kind of source alone, so entries that promise each other's bits (br_hip_colsum / br_hip_colsum_cast /
+// br_hip_gelu_bwd_colsum_cast on fp32) always agree on the path.  Measured, us, two launches / one with 8, 4, 2 lanes:
+//   16-bit sums         [78,1024] 4.5 / 2.9 3.2 3.6   [512,1024] 5.1 / 3.5 3.8 4.0   [2048,4096] 8.6 / 8.6 7.4 7.7
+//                       [2048,12288] 15.9 / 11.9 18.2 19.8: 8 lanes, 4 for many rows of few columns
+//   fp32 sum and copy   [78,1024] 4.6 / 2.6 2.6 2.8   [512,1024] 5.2 / 3.3 3.2 3.4   [1000,4096] 10.8 / 8.2 7.6 11.2
+//                       [1000,8192] 15.4 / 11.2 14.4 22.8   [2048,2048] 8.9 / 13.5 11.7 10.4: 4 lanes while they
+//                       make at most 256 workgroups, one launch up to 1024 rows.  With the GELU backward in front the
+//                       arithmetic wants every CU: [250,1024] 5.7 / 3.4 3.2 3.2, [512,4096] 10.2 / 9.6 9.4 13.7,
+//                       [1000,4096] 17.0 / 18.0 17.4 27.7
+//   bias-GELU backward  [78,4096] 7.9 / 4.0 4.0 4.3   [200,2048] 7.9 / 5.1 4.6 4.4   [1000,4096] 13.5 / 16.4 12.4 12.2
+//   (fp16)              [1000,8192] 15.6 / 18.0 15.5 26.0   [2048,16384] 41.5 / 41.4 65.9 -: as narrow as makes at
+//                       most 256 workgroups, one launch up to 1024 rows
+enum OwnerKind { kOwnSum, kOwnBiasGelu };
+int owner_lanes(int64_t rows, int64_t cols, int elem_bytes, OwnerKind kind) {
+    const int64_t vec = elem_bytes == 4 ? 4 : 8;
+    if (cols % vec != 0) return 0;
+    if (kind == kOwnSum && elem_bytes == 2) return rows > 1024 && cols <= 64 * 64 ? 4 : 8;
+    if (rows > 1024) return 0;
+    if (kind == kOwnBiasGelu && cols <= 256 * 2 * vec) return 2;
+    return cols <= 256 * 4 * vec ? 4 : 8;
 }
 
 template <int UNROLL, typename Src>
-int colsum_owner_launch(const Src& src, float* out, int64_t rows, int64_t cols, float scale, hipStream_t st) {
-    const int64_t cw = kOwnLanesPerRow * Src::VEC;
-    colsum_owner_kernel<UNROLL, Src><<<(unsigned)((cols + cw - 1) / cw), kOwnThreads, 0, st>>>(src, out, rows, cols, scale);
+int colsum_owner_launch(int lanes, const Src& src, float* out, int64_t rows, int64_t cols, float scale, hipStream_t st) {
+    const int64_t cw = lanes * Src::VEC;
+    const unsigned grid = (unsigned)((cols + cw - 1) / cw);
+    if (lanes == 8) colsum_owner_kernel<8, UNROLL, Src><<<grid, kOwnThreads, 0, st>>>(src, out, rows, cols, scale);
+    else if (lanes == 4) colsum_owner_kernel<4, UNROLL, Src><<<grid, kOwnThreads, 0, st>>>(src, out, rows, cols, scale);
+    else colsum_owner_kernel<2, UNROLL, Src><<<grid, kOwnThreads, 0, st>>>(src, out, rows, cols, scale);
     BR_HIP_LAUNCH_CHECK();
     return BR_OK;
 }
@@ -1274,15 +1288,15 @@ int br_hip_bias_gelu_bwd(const void* dy, const void* x, const float* bias, void*
         partial = (float*)workspace;
     }
     const bool al = aligned16(dy) && aligned16(x) && aligned16(dx);
-    if (dbias && al && colsum_owner_applies(rows, cols, dtype == BR_F32 ? 4 : 2, 2)) {
+    if (const int lanes = dbias && al ? owner_lanes(rows, cols, dtype == BR_F32 ? 4 : 2, kOwnBiasGelu) : 0) {
         // gradient and bias gradient from one launch
         if (dtype == BR_F32)
-            return colsum_owner_launch<2>(OwnBiasGeluBwd<float, 4>{(const float*)dy, (const float*)x, bias, (float*)dx},
+            return colsum_owner_launch<2>(lanes, OwnBiasGeluBwd<float, 4>{(const float*)dy, (const float*)x, bias, (float*)dx},
                                           dbias, rows, cols, dbias_scale, st);
         if (dtype == BR_F16)
-            return colsum_owner_launch<2>(OwnBiasGeluBwd<__half, 8>{(const __half*)dy, (const __half*)x, bias, (__half*)dx},
+            return colsum_owner_launch<2>(lanes, OwnBiasGeluBwd<__half, 8>{(const __half*)dy, (const __half*)x, bias, (__half*)dx},
                                           dbias, rows, cols, dbias_scale, st);
-        return colsum_owner_launch<2>(OwnBiasGeluBwd<__hip_bfloat16, 8>{(const __hip_bfloat16*)dy, (const __hip_bfloat16*)x,
+        return colsum_owner_launch<2>(lanes, OwnBiasGeluBwd<__hip_bfloat16, 8>{(const __hip_bfloat16*)dy, (const __hip_bfloat16*)x,
                                                                         bias, (__hip_bfloat16*)dx},
                                       dbias, rows, cols, dbias_scale, st);
     }
@@ -1339,22 +1353,16 @@ int br_hip_colsum(const void* x, int dtype, float* out, int64_t rows, int64_t co
     float* partial = (float*)workspace;
     const int vec = dtype == BR_F32 ? 4 : 8;
     if (cols % vec == 0 && aligned16(x) && (cols * (dtype == BR_F32 ? 4 : 2)) % 16 == 0) {
-        if (colsum_owner_applies(rows, cols, dtype == BR_F32 ? 4 : 2)) {
-            if (dtype == BR_F32) return colsum_owner_launch<4>(OwnPlain<float, 4>{(const float*)x}, out, rows, cols, out_scale, st);
-            if (dtype == BR_F16) return colsum_owner_launch<4>(OwnPlain<__half, 8>{(const __half*)x}, out, rows, cols, out_scale, st);
-            return colsum_owner_launch<4>(OwnPlain<__hip_bfloat16, 8>{(const __hip_bfloat16*)x}, out, rows, cols, out_scale, st);
+        if (const int lanes = owner_lanes(rows, cols, dtype == BR_F32 ? 4 : 2, kOwnSum)) {
+            if (dtype == BR_F32) return colsum_owner_launch<4>(lanes, OwnPlain<float, 4>{(const float*)x}, out, rows, cols, out_scale, st);
+            if (dtype == BR_F16) return colsum_owner_launch<4>(lanes, OwnPlain<__half, 8>{(const __half*)x}, out, rows, cols, out_scale, st);
+            return colsum_owner_launch<4>(lanes, OwnPlain<__hip_bfloat16, 8>{(const __hip_bfloat16*)x}, out, rows, cols, out_scale, st);
         }
+        // two launches: fp32 only (16-bit sums of such columns always take the one)
         const int64_t blocks_x = (cols / vec + kBlock - 1) / kBlock;
         const int rpb = colsum_vec_rows_per_block(rows, blocks_x);
         const int groups = (int)((rows + rpb - 1) / rpb);
-        dim3 grid((unsigned)blocks_x, (unsigned)groups);
-        if (dtype == BR_F32)
-            colsum_partial_vec<float, 4><<<grid, kBlock, 0, st>>>((const float*)x, partial, rows, cols, rpb);
-        else if (dtype == BR_F16)
-            colsum_partial_vec<__half, 8><<<grid, kBlock, 0, st>>>((const __half*)x, partial, rows, cols, rpb);
-        else
-            colsum_partial_vec<__hip_bfloat16, 8><<<grid, kBlock, 0, st>>>((const __hip_bfloat16*)x, partial, rows, cols,
-                                                                          rpb);
+        colsum_partial_vec<<<dim3((unsigned)blocks_x, (unsigned)groups), kBlock, 0, st>>>((const float*)x, partial, rows, cols, rpb);
         BR_HIP_LAUNCH_CHECK();
         return colsum_finish(partial, out, groups, cols, out_scale, st);
     }
@@ -1380,9 +1388,9 @@ int br_hip_colsum_cast(const float* x, float* out, void* x16, int x16_dtype, int
     if (cols % 4 != 0 || !aligned16(x) || (reinterpret_cast<uintptr_t>(x16) & 7u) != 0) return BR_ERR_TODO;
     if (!workspace || workspace_bytes < br_hip_colsum_workspace(rows, cols)) return BR_ERR_ATTR;
     hipStream_t st = as_stream(stream);
-    if (colsum_owner_applies(rows, cols, 4)) {
-        if (x16_dtype == BR_F16) return colsum_owner_launch<4>(OwnCast<__half>{x, (__half*)x16}, out, rows, cols, out_scale, st);
-        return colsum_owner_launch<4>(OwnCast<__hip_bfloat16>{x, (__hip_bfloat16*)x16}, out, rows, cols, out_scale, st);
+    if (const int lanes = owner_lanes(rows, cols, 4, kOwnSum)) {
+        if (x16_dtype == BR_F16) return colsum_owner_launch<4>(lanes, OwnCast<__half>{x, (__half*)x16}, out, rows, cols, out_scale, st);
+        return colsum_owner_launch<4>(lanes, OwnCast<__hip_bfloat16>{x, (__hip_bfloat16*)x16}, out, rows, cols, out_scale, st);
     }
     float* partial = (float*)workspace;
     const int64_t blocks_x = (cols / 4 + kBlock - 1) / kBlock;
@@ -1409,10 +1417,10 @@ int br_hip_gelu_bwd_colsum_cast(const float* dy, const float* x, float* dx, floa
         return BR_ERR_TODO;
     if (!workspace || workspace_bytes < br_hip_colsum_workspace(rows, cols)) return BR_ERR_ATTR;
     hipStream_t st = as_stream(stream);
-    if (colsum_owner_applies(rows, cols, 4)) {
+    if (const int lanes = owner_lanes(rows, cols, 4, kOwnSum)) {
         if (dx16_dtype == BR_F16)
-            return colsum_owner_launch<2>(OwnGeluBwdCast<__half>{dy, x, dx, (__half*)dx16}, out, rows, cols, out_scale, st);
-        return colsum_owner_launch<2>(OwnGeluBwdCast<__hip_bfloat16>{dy, x, dx, (__hip_bfloat16*)dx16}, out, rows, cols,
+            return colsum_owner_launch<2>(lanes, OwnGeluBwdCast<__half>{dy, x, dx, (__half*)dx16}, out, rows, cols, out_scale, st);
+        return colsum_owner_launch<2>(lanes, OwnGeluBwdCast<__hip_bfloat16>{dy, x, dx, (__hip_bfloat16*)dx16}, out, rows, cols,
                                       out_scale, st);
     }
     float* partial = (float*)workspace;

@@ -367,3 +367,31 @@ def test_gelu_bwd_colsum_cast_equals_the_separate_kernels(rows, cols, dtype, tdt
     assert hip.load().br_hip_gelu_bwd_colsum_cast(ptr(d_dy), ptr(d_x), ptr(dx_sep), ptr(sums_sep), ptr(x16_sep), dtype,
                                                   4, 1001, 1.0, ptr(ws), ws.numel(), stream()) == -1
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("rows,cols", [(1, 8), (17, 264), (127, 72), (128, 1032), (300, 8200), (1000, 4096), (1024, 4104),
+                                       (1025, 4096), (1025, 4104)])
+def test_column_sums_in_one_launch(rows, cols):
+    """The one-launch column sums at the edges of their rules: strips of 2, 4 and 8 lanes, a last strip that sticks
+    out, rows that fill no pass, the row count beyond which some sources take two launches.  Bound: every order of
+    `rows` fp32 additions is within rows * 2^-24 * sum |x| of the exact sum."""
+    from gpu_util import BF16
+    print("case rows=%d cols=%d" % (rows, cols), flush=True)
+    g = torch.Generator(device="cuda").manual_seed(71)
+    x = torch.randn(rows, cols, device="cuda", generator=g)
+    bias = torch.randn(cols, device="cuda", generator=g)
+    ws = workspace(hip.load().br_hip_colsum_workspace(rows, cols))
+
+    def check(got, terms):
+        terms = terms.double()
+        assert bool(((got.double() - terms.sum(0)).abs() <= rows * 2.0 ** -24 * terms.abs().sum(0)).all())
+
+    for t, code in ((torch.float32, F32), (torch.float16, F16), (torch.bfloat16, BF16)):
+        h, out = x.to(t), empty(cols)
+        call("br_hip_colsum", ptr(h), code, ptr(out), rows, cols, 1.0, ptr(ws), ws.numel(), stream())
+        check(out, h)
+        # the sums are of the values that were stored
+        dx, dbias = empty((rows, cols), t), empty(cols)
+        call("br_hip_bias_gelu_bwd", ptr(h), ptr(h), ptr(bias), ptr(dx), ptr(dbias), code, rows, cols, 1.0, ptr(ws),
+             ws.numel(), stream())
+        check(dbias, dx)
