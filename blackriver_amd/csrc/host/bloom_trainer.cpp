@@ -136,6 +136,13 @@ void BloomTrainer::create_optimizer(float lr, float beta1, float beta2, float ep
     }
     s << "0 # op.sync\n";
     env_.execute(s.str());
+    // a step is one launch per block and one for the model's own parameters
+    std::ostringstream step;
+    const char* sfx = masters() ? "16" : "";
+    step << "0 # model_adamw" << sfx << "\n";
+    for (int i = 1; i <= cfg_.layers; i++) step << i << " # layer_adamw" << sfx << "\n";
+    step << "0 # op.sync\n";
+    adamw_.reset(env_.build(step.str()));
     has_optimizer_ = true;
     adam_step_ = 0;
 }
@@ -143,14 +150,11 @@ void BloomTrainer::create_optimizer(float lr, float beta1, float beta2, float ep
 void BloomTrainer::optimizer_step() {
     br_assert(has_optimizer_, "BloomTrainer::create_optimizer has not run");
     adam_step_++;
-    // the step count changes every call, so the (short) program is compiled per call
-    std::ostringstream s;
-    const char* sfx = masters() ? "16" : "";
-    s << "0 #  " << adam_step_ << " $adam_step !  model_adamw" << sfx << "\n";
-    for (int i = 1; i <= cfg_.layers; i++)
-        s << i << " #  " << adam_step_ << " $adam_step !  layer_adamw" << sfx << "\n";
-    s << "0 # op.sync\n";
-    env_.execute(s.str());
+    for (int i = cfg_.layers; i >= 0; i--) {
+        env_.change((size_t)i);
+        env_.hash().set("$adam_step", Hash::Item((double)adam_step_));
+    }
+    env_.run(adamw_.get());
 }
 
 float BloomTrainer::step(const int32_t* ids, const int32_t* mask) {

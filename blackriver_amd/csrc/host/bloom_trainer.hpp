@@ -69,6 +69,7 @@ private:
     Enviroment& env_;
     BloomModelConfig cfg_;
     std::unique_ptr<DaG> step_;
+    std::unique_ptr<DaG> adamw_;
     bool masters() const { return cfg_.weight_dtype != "float"; }
     bool has_optimizer_ = false;
     int64_t adam_step_ = 0;

@@ -425,16 +425,27 @@ BR_WORD(LayernormBackwardAddLinearBackward,
     }
 )
 
-// AdamW on one parameter tensor.  The reference stops at the gradients; these
-// two words are what a training loop runs after them.
-// ( param [master] grad m v lr beta1 beta2 eps weight_decay step -- )
-void adamw(Stack& stack, bool with_master) {
+// AdamW.  The reference stops at the gradients; these words are what a training
+// loop runs after them.
+struct AdamWHyper {
+    float lr, beta1, beta2, eps, wd;
+    int64_t step;
+};
+// ( lr beta1 beta2 eps weight_decay step -- )
+AdamWHyper pop_adamw_hyper(Stack& stack) {
+    AdamWHyper h;
     const double step = stack.pop_number();
-    const float wd = (float)stack.pop_number();
-    const float eps = (float)stack.pop_number();
-    const float beta2 = (float)stack.pop_number();
-    const float beta1 = (float)stack.pop_number();
-    const float lr = (float)stack.pop_number();
+    br_assert(step >= 1, "op.adamw: steps count from 1");
+    h.step = (int64_t)step;
+    h.wd = (float)stack.pop_number();
+    h.eps = (float)stack.pop_number();
+    h.beta2 = (float)stack.pop_number();
+    h.beta1 = (float)stack.pop_number();
+    h.lr = (float)stack.pop_number();
+    return h;
+}
+// ( param [master] grad m v -- )
+br_adamw_tensor pop_adamw_tensor(Stack& stack, bool with_master) {
     tensor_t v = stack.pop_tensor();
     tensor_t m = stack.pop_tensor();
     tensor_t grad = stack.pop_tensor();
@@ -444,19 +455,34 @@ void adamw(Stack& stack, bool with_master) {
     br_assert(param->is_cuda() && f32dev(grad) && f32dev(m) && f32dev(v), "op.adamw: device tensors, fp32 state");
     br_assert(grad->items() == param->items() && m->items() == param->items() && v->items() == param->items(),
               "op.adamw: parameter, gradient and moments differ in size");
-    br_assert(step >= 1, "op.adamw: steps count from 1");
     float* master_ptr = nullptr;
     if (with_master) {
         br_assert(f32dev(master) && master->items() == param->items() && param->dtype() != DataType::Float,
                   "op.adamw_master: an fp32 master copy of a 16-bit parameter");
         master_ptr = static_cast<float*>(master->data());
     }
-    BR_HIP_CHECK(br_hip_adamw(param->data(), (int)param->dtype(), master_ptr, static_cast<const float*>(grad->data()),
-                              static_cast<float*>(m->data()), static_cast<float*>(v->data()), (int64_t)param->items(),
-                              lr, beta1, beta2, eps, wd, (int64_t)step, ComputingContext::stream));
+    return {param->data(), master_ptr, static_cast<const float*>(grad->data()), static_cast<float*>(m->data()),
+            static_cast<float*>(v->data()), (int64_t)param->items(), (int)param->dtype()};
 }
-BR_WORD(AdamW, adamw(stack, false);)
-BR_WORD(AdamWMaster, adamw(stack, true);)
+void adamw(const std::vector<br_adamw_tensor>& tensors, const AdamWHyper& h) {
+    BR_HIP_CHECK(br_hip_adamw_group(tensors.data(), (int64_t)tensors.size(), h.lr, h.beta1, h.beta2, h.eps, h.wd, h.step,
+                                    ComputingContext::stream));
+}
+// ( param grad m v hyper.. step -- )    ( param master grad m v hyper.. step -- )
+BR_WORD(AdamW, const AdamWHyper h = pop_adamw_hyper(stack); adamw({pop_adamw_tensor(stack, false)}, h);)
+BR_WORD(AdamWMaster, const AdamWHyper h = pop_adamw_hyper(stack); adamw({pop_adamw_tensor(stack, true)}, h);)
+// ( {param grad m v}*s s {param master grad m v}*k k hyper.. step -- )  s tensors that are their own state and k with a
+// master copy, all in one launch
+BR_WORD(AdamWGroup,
+    const AdamWHyper h = pop_adamw_hyper(stack);
+    std::vector<br_adamw_tensor> tensors;
+    for (const bool with_master : {true, false}) {
+        const double n = stack.pop_number();
+        br_assert(n >= 0 && n == (double)(int64_t)n, "op.adamw_group: a count of tensors");
+        for (int64_t i = 0; i < (int64_t)n; i++) tensors.push_back(pop_adamw_tensor(stack, with_master));
+    }
+    adamw(tensors, h);
+)
 
 BR_WORD(Dump, tensor_t t = stack.pop_tensor(); t->io_dump(t);)
 // ( tensor filename -- )
@@ -523,6 +549,7 @@ void load_nn_words(Enviroment& env) {
         {"op.flash_attn_qkv_backward", FlashAttnQkvBackward::creator},
         {"op.adamw", AdamW::creator},
         {"op.adamw_master", AdamWMaster::creator},
+        {"op.adamw_group", AdamWGroup::creator},
     };
     for (const auto& e : table) env.insert_native_word(e.name, e.creator);
     // longer patterns first: a pass only sees what earlier passes left unfused

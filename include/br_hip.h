@@ -434,6 +434,21 @@ int br_hip_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
 int br_hip_adamw(void* param, int param_dtype, float* master, const float* grad, float* m, float* v,
                  int64_t n, float lr, float beta1, float beta2, float eps, float weight_decay,
                  int64_t step, br_stream_t stream);
+/* The same over `count` tensors that share their hyper-parameters, in as few
+ * launches as they fit (32 tensors each; tensors that share memory are updated
+ * one after the other).  Nothing is updated unless every tensor's description
+ * is valid. */
+typedef struct {
+    void* param;
+    float* master;
+    const float* grad;
+    float* m;
+    float* v;
+    int64_t n;
+    int param_dtype;
+} br_adamw_tensor;
+int br_hip_adamw_group(const br_adamw_tensor* tensors, int64_t count, float lr, float beta1, float beta2,
+                       float eps, float weight_decay, int64_t step, br_stream_t stream);
 
 /* ---- data preparation (bit-exact integer / gather work) ---------------- */
 /* The embedding row gather of blackriver/train_bloom.cpp:50-56. */

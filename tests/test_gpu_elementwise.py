@@ -315,6 +315,44 @@ def test_adamw_against_oracle(n, dtype, master):
             p = got
 
 
+class AdamWTensor(ctypes.Structure):
+    _fields_ = [("param", ctypes.c_void_p), ("master", ctypes.c_void_p), ("grad", ctypes.c_void_p), ("m", ctypes.c_void_p),
+                ("v", ctypes.c_void_p), ("n", ctypes.c_int64), ("dtype", ctypes.c_int)]
+
+
+@pytest.mark.parametrize("sizes", [[1], [1024, 3], [7, 0, 1023, 1024, 1025, 4096, 256, 260] * 5])
+def test_adamw_group_against_oracle(sizes):
+    """Tensors of every storage in shared launches (more than one launch holds in the last case), one on a 4-byte
+    boundary, and the first one listed twice: updated one after the other.  Bounds as for a tensor by itself."""
+    print("case", len(sizes), flush=True)
+    rng = np.random.default_rng(5)
+    hyper = (1e-2, 0.9, 0.95, 1e-8, 0.1)
+    kinds = [(F32, torch.float32), (F16, torch.float16), (BF16, torch.bfloat16)]
+    rows, entries = [], []
+    for i, n in enumerate(sizes):
+        code, tdt = kinds[i % 3]
+        off = 1 if i == 3 else 0
+        g, m, v = (np.abs(rng.standard_normal(n)).astype(np.float32) for _ in range(3))
+        p0 = torch.from_numpy(rng.standard_normal(n).astype(np.float32)).to(tdt)
+        d = [torch.zeros(n + 1, device="cuda")[off:off + n] for _ in range(4)]
+        for t, x in zip(d, (p0.float(), torch.from_numpy(g), torch.from_numpy(m), torch.from_numpy(v))):
+            t.copy_(x)
+        param = d[0] if code == F32 else p0.cuda()
+        rows.append((code, tdt, param, d, orc.adamw_step(p0.float().numpy(), g, m, v, *hyper, 3), g))
+        entries.append(AdamWTensor(param.data_ptr(), None if code == F32 else d[0].data_ptr(), d[1].data_ptr(),
+                                   d[2].data_ptr(), d[3].data_ptr(), n, code))
+    array = (AdamWTensor * (len(entries) + 1))(*entries, entries[0])
+    call("br_hip_adamw_group", ctypes.cast(array, ctypes.c_void_p), len(array), *hyper, 3, stream())
+    for i, (code, tdt, param, d, want, g) in enumerate(rows):
+        if i == 0:
+            want = orc.adamw_step(*want[:1], g, *want[1:], *hyper, 3)
+        for got, ref, what in zip((d[0], d[2], d[3]), want, ("parameter", "first moment", "second moment")):
+            if sizes[i]:
+                assert_close(host(got), ref, 1e-5, "%s of tensor %d" % (what, i))
+        if code != F32:
+            assert torch.equal(param, d[0].to(tdt))
+
+
 def test_adamw_rejects_bad_arguments():
     lib = hip.load()
     t = empty(16)
