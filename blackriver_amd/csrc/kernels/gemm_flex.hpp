@@ -4,7 +4,7 @@
 //
 //   C[b][i,j] = alpha * sum_p opA[b][i,p] * opB[b][p,j] (+ C) (+ bias[j])
 //
-// A workgroup owns a BM x BN tile of C (64 x 64 or 32 x 32) and EVERY of its
+// gemm_flex_kernel: a workgroup owns a BM x BN tile of C (64 x 64 or 32 x 32) and EVERY of its
 // KW waves computes the whole tile over its own share of K: wave w takes the
 // 128-byte K steps w, w + KW, w + 2 KW, ...  Each wave loads its steps into LDS
 // buffers of its own and reads them back itself, so the K loop has no barrier:
@@ -131,6 +131,76 @@ struct FlexTile {
 
 typedef float flex_f32x4 __attribute__((ext_vector_type(4)));
 
+typedef __attribute__((address_space(3))) flex_f32x4 lds_f32x4;
+
+// The end of a tile, in two parts with a barrier between them.  First every wave leaves its accumulators in BM x BN
+// floats of LDS of its own at `mem`:
+// acc[i][j][v] is C[row, col] with row = i*32 + lane%32, col = j*32 + (v/4)*8 + (lane/32)*4 + v%4; quad c of row r goes
+// to slot c ^ (r % 8) of the row (writes of 16 rows and reads along a row both touch every bank once).
+template <int BM, int BN>
+__device__ __forceinline__ void flex_park(const f32x16 (&acc)[BM / 32][BN / 32], lds_byte* mem, int lane) {
+    constexpr int FM = BM / 32, FN = BN / 32, QN = BN / 4;
+    lds_f32x4* const sums = (lds_f32x4*)mem;
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++)
+#pragma unroll
+            for (int q = 0; q < 4; q++) {
+                const int r = i * 32 + (lane & 31), c = j * 8 + q * 2 + (lane >> 5);
+                flex_f32x4 v;
+                v.x = acc[i][j][4 * q]; v.y = acc[i][j][4 * q + 1]; v.z = acc[i][j][4 * q + 2]; v.w = acc[i][j][4 * q + 3];
+                sums[r * QN + (c ^ (r & 7))] = v;
+            }
+}
+
+// Then THREADS threads add up the KW accumulators, `wave_bytes` apart from lds_all on, in wave order, and store C.
+template <int BM, int BN, int KW, int THREADS, typename TC, bool GELU>
+__device__ __forceinline__ void flex_emit(const GemmArgs& g, const lds_byte* lds_all, int wave_bytes, int row0, int col0, int b) {
+    constexpr int QN = BN / 4;
+    TC* c_base = static_cast<TC*>(g.c) + b * g.sc;
+    TC* c2_base = GELU ? static_cast<TC*>(g.c2) + b * g.sc : nullptr;
+    const TC* old_base = g.addend ? static_cast<const TC*>(g.addend) + b * g.sc : c_base;
+    const lds_f32x4* const all = (const lds_f32x4*)lds_all;
+    constexpr int kQuads = BM * QN, kThreads = THREADS;
+#pragma unroll
+    for (int it = 0; it < (kQuads + kThreads - 1) / kThreads; it++) {
+        const int e = it * kThreads + threadIdx.x;
+        if (kQuads % kThreads != 0 && e >= kQuads) break;
+        const int r = e / QN, c = e % QN;
+        const int at = r * QN + (c ^ (r & 7));
+        flex_f32x4 s = all[at];
+#pragma unroll
+        for (int w = 1; w < KW; w++) s += all[w * (wave_bytes / 16) + at];
+        const int row = row0 + r, col = col0 + c * 4;
+        if (row >= g.m) continue;
+        const long long off = row * g.ldc + col;
+        const int left = (int)(g.n - col);   // columns of C this quad covers
+        float o[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            o[u] = g.alpha * s[u] + (g.bias && u < left ? g.bias[col + u] : 0.f);
+            if (g.accumulate && u < left) o[u] += c_load<TC>(old_base + off + u);
+            if (sizeof(TC) == 2) asm volatile("" : "+v"(o[u]));   // one fp32 value, then one rounding
+        }
+        if (left >= 4 && g.vec_c) {
+            c_store4<TC>(c_base + off, o);
+            if (GELU) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) o[u] = gelu_one(o[u]);
+                c_store4<TC>(c2_base + off, o);
+            }
+        } else {
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+                if (u < left) {
+                    c_store<TC>(c_base + off + u, o[u]);
+                    if (GELU) c_store<TC>(c2_base + off + u, gelu_one(o[u]));
+                }
+        }
+    }
+}
+
 template <int CT, int BM, int BN, int KW, int ST, bool A_KSTR, bool B_KSTR, typename TC, bool GELU = false, bool WORDS = false>
 __global__ __launch_bounds__(KW * 64) void gemm_flex_kernel(GemmArgs g) {
     using TA = FlexTile<CT, BM, A_KSTR, WORDS>;
@@ -249,65 +319,165 @@ __global__ __launch_bounds__(KW * 64) void gemm_flex_kernel(GemmArgs g) {
                     }
     }
 
-    // acc[i][j][v] is C[row, col] with row = i*32 + lane%32, col = j*32 + (v/4)*8 + (lane/32)*4 + v%4.  Each wave
-    // leaves its tile in its own buffers, quad c of row r in slot c ^ (r % 8) of the row (writes of 16 rows and
-    // reads along a row both touch every bank once).
-    typedef __attribute__((address_space(3))) flex_f32x4 lds_f32x4;
-    constexpr int QN = BN / 4;
-    lds_f32x4* const sums = (lds_f32x4*)mem;
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++)
-#pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int r = i * 32 + (lane & 31), c = j * 8 + q * 2 + (lane >> 5);
-                flex_f32x4 v;
-                v.x = acc[i][j][4 * q]; v.y = acc[i][j][4 * q + 1]; v.z = acc[i][j][4 * q + 2]; v.w = acc[i][j][4 * q + 3];
-                sums[r * QN + (c ^ (r & 7))] = v;
-            }
+    flex_park<BM, BN>(acc, mem, lane);
     __syncthreads();
-    TC* c_base = static_cast<TC*>(g.c) + b * g.sc;
-    TC* c2_base = GELU ? static_cast<TC*>(g.c2) + b * g.sc : nullptr;
-    const TC* old_base = g.addend ? static_cast<const TC*>(g.addend) + b * g.sc : c_base;
-    const lds_f32x4* const all = (const lds_f32x4*)(lds_byte*)lds_raw;
-    constexpr int kQuads = BM * QN, kThreads = KW * 64;
+    flex_emit<BM, BN, KW, KW * 64, TC, GELU>(g, (lds_byte*)lds_raw, kWaveBytes, row0, col0, b);
+}
+
+// 64 x 128 tiles, a ring of six K steps, waves that load beside waves that multiply.  The kernel above gives a wave
+// whole K steps and buffers of its own; a tile of this size leaves no room for two such buffers a wave.  Here four
+// waves share a ring of 24 KB steps: wave w multiplies k-values 16 w .. 16 w + 15 of every step by itself, so a fragment
+// is still read from LDS exactly once, and four more waves do nothing but keep five steps of loads in flight.  With the
+// same waves doing both, a wave that waits for room in the load path holds up its own products: 52 us instead of 31 for
+// the first product below.  One barrier a step.
+//
+// Why: outputs of some 256 such tiles ([512 x 4096], [1024 x 2048]) are bound by the rate at which a CU fills LDS, about
+// 30 B per clock whatever the tile; 64 x 128 tiles ask for three quarters of the bytes of 64 x 64 ones, and 128 x 128
+// tiles would leave half of the CUs without one.  Inside model steps, 64 x 64 tiles of two waves / this (us, under the
+// profiler): [512 x 4096] K = 4096 50 / 39 and, with the weight the other way round, 40 / 35; [1002 x 2048] K = 2048
+// in bf16 35.5 / 27 and 24.8 / 22.7; [1024 x 2048] K = 2048 22 / 19.6.
+template <int CT, bool A_KSTR, bool B_KSTR, typename TC, bool GELU = false>
+__global__ __launch_bounds__(512) void gemm_ring_kernel(GemmArgs g) {
+    constexpr int BM = 64, BN = 128, KW = 4, ST = 6, KT = 64;
+    using TA = FlexTile<CT, BM, A_KSTR, false>;
+    using TB = FlexTile<CT, BN, B_KSTR, false>;
+    constexpr int FM = BM / 32, FN = BN / 32;
+    constexpr int kStageBytes = TA::kBytes + TB::kBytes;
+    constexpr int kA = TA::kInstr / KW, kB = TB::kInstr / KW, kLoads = kA + kB;   // a wave's share of a step's loads
+    static_assert(TA::kStep == KT && TA::kInstr % KW == 0 && TB::kInstr % KW == 0, "16-bit operands");
+    static_assert(ST * kStageBytes >= KW * BM * BN * 4 && ST * kStageBytes <= 160 * 1024, "LDS");
+    static_assert((ST - 1) * kLoads <= 63, "loads a partial wait can leave outstanding");
+    __shared__ __attribute__((aligned(1024))) unsigned char lds_raw[ST * kStageBytes];
+    const int lane = threadIdx.x & 63;
+    const bool loader = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= KW;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) % KW;   // among the loaders / the multipliers
+    long long batch;
+    int tm, tn;
+    tile_coords(g, batch, tm, tn);
+    tm = __builtin_amdgcn_readfirstlane(tm);
+    tn = __builtin_amdgcn_readfirstlane(tn);
+    const int b = __builtin_amdgcn_readfirstlane((int)batch);
+    const int row0 = tm * BM, col0 = tn * BN;
+    // slices of K take the place of the batch index
+    const bool sliced = g.splits > 1;
+    const int k_begin = sliced ? b * g.k_slice : 0;
+    const int k_end = sliced && k_begin + g.k_slice < g.k ? k_begin + g.k_slice : (int)g.k;
+    const int steps = (k_end - k_begin + KT - 1) / KT;
+    const int padded = steps + (steps & 1);   // the multipliers take steps in pairs
+    // step t of the loop covers K step (t + first) mod steps of the slice (see k_walk_start)
+    const int first = (int)(k_walk_start(row0, col0, g.k) / KT) % steps;
+    const int k0 = k_begin + first * KT;
+    const long long a_at = (sliced ? 0 : b * g.sa) + (A_KSTR ? (long long)k0 * g.lda + row0 : (long long)row0 * g.lda + k0);
+    const long long b_at = (sliced ? 0 : b * g.sb) + (B_KSTR ? (long long)k0 * g.ldb + col0 : (long long)col0 * g.ldb + k0);
+    const unsigned char* a_src = static_cast<const unsigned char*>(g.a) + 2 * a_at;
+    const unsigned char* b_src = static_cast<const unsigned char*>(g.b) + 2 * b_at;
+    // where each operand ends as seen from the current step, rounded up to the granule the last element lies in
+    long long a_left = ((A_KSTR ? (long long)(k_end - 1 - k0) * g.lda + g.m - row0
+                                : (g.m - 1 - row0) * g.lda + (k_end - k0)) * 2 + 15) & ~15LL;
+    long long b_left = ((B_KSTR ? (long long)(k_end - 1 - k0) * g.ldb + g.n - col0
+                                : (g.n - 1 - col0) * g.ldb + (k_end - k0)) * 2 + 15) & ~15LL;
+    const long long a_step = (A_KSTR ? g.lda : 1) * (2LL * KT);
+    const long long b_step = (B_KSTR ? g.ldb : 1) * (2LL * KT);
+    int k_left = k_end - k0;
+    int until_wrap = steps - first;
+    unsigned a_off[kA], b_off[kB];
 #pragma unroll
-    for (int it = 0; it < (kQuads + kThreads - 1) / kThreads; it++) {
-        const int e = it * kThreads + threadIdx.x;
-        if (kQuads % kThreads != 0 && e >= kQuads) break;
-        const int r = e / QN, c = e % QN;
-        const int at = r * QN + (c ^ (r & 7));
-        flex_f32x4 s = all[at];
+    for (int q = 0; q < kA; q++) a_off[q] = TA::source_offset(wave * kA + q, lane, g.lda);
 #pragma unroll
-        for (int w = 1; w < KW; w++) s += all[w * (kWaveBytes / 16) + at];
-        const int row = row0 + r, col = col0 + c * 4;
-        if (row >= g.m) continue;
-        const long long off = row * g.ldc + col;
-        const int left = (int)(g.n - col);   // columns of C this quad covers
-        float o[4];
+    for (int q = 0; q < kB; q++) b_off[q] = TB::source_offset(wave * kB + q, lane, g.ldb);
+    lds_byte* const lds = (lds_byte*)lds_raw;
+    const unsigned lds0 = (unsigned)(unsigned long long)lds;
+
+    auto issue = [&](int stage, int t) {
+        // an odd number of steps is filled up with one of zeros, loaded from past the end
+        const buffer_rsrc ra = buffer_from(a_src, t < steps ? a_left : 0), rb = buffer_from(b_src, t < steps ? b_left : 0);
+        const unsigned dst = lds0 + (unsigned)stage * kStageBytes;
+        // a k-contiguous operand's last step: chunks past K are fetched from past the end of the operand
+        const bool tail = k_left < KT;
 #pragma unroll
-        for (int u = 0; u < 4; u++) {
-            o[u] = g.alpha * s[u] + (g.bias && u < left ? g.bias[col + u] : 0.f);
-            if (g.accumulate && u < left) o[u] += c_load<TC>(old_base + off + u);
-            if (sizeof(TC) == 2) asm volatile("" : "+v"(o[u]));   // one fp32 value, then one rounding
+        for (int q = 0; q < kA; q++)
+            TA::load(dst, wave * kA + q, !A_KSTR && tail && TA::k_of(wave * kA + q, lane) >= k_left ? kPastEnd : a_off[q], ra);
+#pragma unroll
+        for (int q = 0; q < kB; q++)
+            TB::load(dst + TA::kBytes, wave * kB + q, !B_KSTR && tail && TB::k_of(wave * kB + q, lane) >= k_left ? kPastEnd : b_off[q], rb);
+        const bool wraps = --until_wrap == 0;
+        const long long da = wraps ? a_step - steps * a_step : a_step, db = wraps ? b_step - steps * b_step : b_step;
+        a_src += da; a_left -= da;
+        b_src += db; b_left -= db;
+        k_left -= wraps ? KT - steps * KT : KT;
+    };
+
+    // Barrier t, t = 0 .. padded - 1: step t is in LDS, and the fragments of step t - 1 are in registers.
+    if (loader) {
+#pragma unroll
+        for (int s = 0; s < ST; s++)
+            if (s < padded) issue(s, s);
+        if (padded >= ST) wait_vmem<(ST - 1) * kLoads>();
+        else wait_vmem<0>();
+        __builtin_amdgcn_s_barrier();
+        int stage = 0;
+        for (int t = 1; t < padded; t++) {
+            // step t is in once at most the ST - 2 steps after it are outstanding
+            if (t + ST <= padded + 1) wait_vmem<(ST - 2) * kLoads>();
+            else wait_vmem<0>();
+            __builtin_amdgcn_s_barrier();
+            if (t - 1 + ST < padded) issue(stage, t - 1 + ST);   // where step t - 1 was
+            stage = stage + 1 == ST ? 0 : stage + 1;
         }
-        if (left >= 4 && g.vec_c) {
-            c_store4<TC>(c_base + off, o);
-            if (GELU) {
+        __builtin_amdgcn_s_barrier();
+    } else {
+        unsigned fa_off[FM], fb_off[FN];
 #pragma unroll
-                for (int u = 0; u < 4; u++) o[u] = gelu_one(o[u]);
-                c_store4<TC>(c2_base + off, o);
-            }
-        } else {
+        for (int i = 0; i < FM; i++) fa_off[i] = TA::frag_offset(i * 32, wave, lane);
 #pragma unroll
-            for (int u = 0; u < 4; u++)
-                if (u < left) {
-                    c_store<TC>(c_base + off + u, o[u]);
-                    if (GELU) c_store<TC>(c2_base + off + u, gelu_one(o[u]));
-                }
+        for (int j = 0; j < FN; j++) fb_off[j] = TA::kBytes + TB::frag_offset(j * 32, wave, lane);
+        f32x16 acc[FM][FN];
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+        u32x4 fa0[FM], fb0[FN], fa1[FM], fb1[FN];
+        int stage = 0;
+        auto read = [&](u32x4 (&fa)[FM], u32x4 (&fb)[FN]) {
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            __builtin_amdgcn_s_barrier();
+            asm volatile("" ::: "memory");
+            const lds_byte* tile = lds + stage * kStageBytes;
+#pragma unroll
+            for (int i = 0; i < FM; i++) fa[i] = TA::fragment(tile, fa_off[i]);
+#pragma unroll
+            for (int j = 0; j < FN; j++) fb[j] = TB::fragment(tile, fb_off[j]);
+            stage = stage + 1 == ST ? 0 : stage + 1;
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        auto multiply = [&](const u32x4 (&fa)[FM], const u32x4 (&fb)[FN]) {
+            // operands swapped: a lane then holds four consecutive columns of one row of C
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+#pragma unroll
+                for (int j = 0; j < FN; j++) acc[i][j] = Cvt<CT>::mfma(fb[j], fa[i], acc[i][j]);
+            __builtin_amdgcn_sched_barrier(0);
+        };
+        read(fa0, fb0);
+        for (int t = 2; t < padded; t += 2) {
+            read(fa1, fb1);
+            multiply(fa0, fb0);
+            read(fa0, fb0);
+            multiply(fa1, fb1);
         }
+        read(fa1, fb1);
+        multiply(fa0, fb0);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        multiply(fa1, fb1);
+        // every load has landed and every fragment has been read once all waves are here
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        flex_park<BM, BN>(acc, lds + wave * (BM * BN * 4), lane);
     }
+    __syncthreads();
+    flex_emit<BM, BN, KW, 512, TC, GELU>(g, lds, BM * BN * 4, row0, col0, b);
 }
 
 // ---- host-side dispatch -------------------------------------------------------
@@ -334,17 +504,54 @@ int launch_flex_c(const GemmArgs& g, const Problem& p, unsigned grid, hipStream_
     return BR_OK;
 }
 
-template <int CT, int BM, int BN, int KW, int ST>
-int launch_flex_config(GemmArgs g, const Problem& p, long long batch, hipStream_t st) {
+template <int CT, typename TC>
+int launch_ring_c(const GemmArgs& g, const Problem& p, unsigned grid, hipStream_t st) {
+    if (g.c2) {
+        if constexpr (sizeof(TC) == 2) {
+            if (p.a_kstr || p.b_kstr) return BR_ERR_TODO;
+            gemm_ring_kernel<CT, false, false, TC, true><<<grid, 512, 0, st>>>(g);
+        } else {
+            return BR_ERR_TODO;
+        }
+    } else if (p.a_kstr && p.b_kstr) {
+        gemm_ring_kernel<CT, true, true, TC><<<grid, 512, 0, st>>>(g);
+    } else if (p.a_kstr) {
+        gemm_ring_kernel<CT, true, false, TC><<<grid, 512, 0, st>>>(g);
+    } else if (p.b_kstr) {
+        gemm_ring_kernel<CT, false, true, TC><<<grid, 512, 0, st>>>(g);
+    } else {
+        gemm_ring_kernel<CT, false, false, TC><<<grid, 512, 0, st>>>(g);
+    }
+    BR_HIP_LAUNCH_CHECK();
+    return BR_OK;
+}
+
+// The tiling of a product and whether four columns of C can be stored at once; the number of workgroups, or -1.
+template <int BM, int BN>
+long long flex_tiles(GemmArgs& g, const Problem& p, long long batch) {
     g.tiles_m = (int)((g.m + BM - 1) / BM);
     g.tiles_n = (int)((g.n + BN - 1) / BN);
     const long long blocks = (long long)g.tiles_m * g.tiles_n * (g.splits > 1 ? g.splits : batch);
-    if (blocks > 0x7fffffffLL) return BR_ERR_ATTR;
     const long long es = p.c_dtype == BR_F32 ? 4 : 2;
     auto quads = [&](const void* q) { return (reinterpret_cast<uintptr_t>(q) & (4 * es - 1)) == 0; };
     g.vec_c = g.ldc % 4 == 0 && g.sc % 4 == 0 && quads(g.c) && (!g.c2 || quads(g.c2));
+    return blocks > 0x7fffffffLL ? -1 : blocks;
+}
+
+template <int CT, int BM, int BN, int KW, int ST>
+int launch_flex_config(GemmArgs g, const Problem& p, long long batch, hipStream_t st) {
+    const long long blocks = flex_tiles<BM, BN>(g, p, batch);
+    if (blocks < 0) return BR_ERR_ATTR;
     if (p.c_dtype == BR_F32) return launch_flex_c<CT, BM, BN, KW, ST, float>(g, p, (unsigned)blocks, st);
     return launch_flex_c<CT, BM, BN, KW, ST, std::conditional_t<CT == BR_GEMM_F16, __half, __hip_bfloat16>>(g, p, (unsigned)blocks, st);
+}
+
+template <int CT>
+int launch_ring(GemmArgs g, const Problem& p, long long batch, hipStream_t st) {
+    const long long blocks = flex_tiles<64, 128>(g, p, batch);
+    if (blocks < 0) return BR_ERR_ATTR;
+    if (p.c_dtype == BR_F32) return launch_ring_c<CT, float>(g, p, (unsigned)blocks, st);
+    return launch_ring_c<CT, std::conditional_t<CT == BR_GEMM_F16, __half, __hip_bfloat16>>(g, p, (unsigned)blocks, st);
 }
 
 // Any K; slices of K as batch entries when g.splits > 1.
@@ -353,6 +560,7 @@ int launch_flex(const GemmArgs& g, const Problem& p, int kernel, long long batch
     if (kernel == kFlex64) return launch_flex_config<CT, 64, 64, 4, 1>(g, p, batch, st);
     if (kernel == kFlex64Short) return launch_flex_config<CT, 64, 64, 2, 1>(g, p, batch, st);
     if (kernel == kFlex32x64) return launch_flex_config<CT, 32, 64, 4, 1>(g, p, batch, st);
+    if (kernel == kRing64x128) return launch_ring<CT>(g, p, batch, st);
     return launch_flex_config<CT, 32, 32, 4, 2>(g, p, batch, st);
 }
 

@@ -22,7 +22,7 @@
 namespace brk {
 namespace gemm16 {
 
-enum Kernel { kTile256, kTile256x128, kTile256x128Groups, kTile128, kFlex64, kFlex64Short, kFlex32x64, kFlex32, kKernels };
+enum Kernel { kTile256, kTile256x128, kTile256x128Groups, kTile128, kFlex64, kFlex64Short, kFlex32x64, kFlex32, kRing64x128, kKernels };
 
 struct KernelCost {
     int bm, bn;
@@ -35,10 +35,14 @@ constexpr KernelCost kCost[kKernels] = {
     {256, 128, 1, 256, 3.07, 0.840, 1.048, 0.89},    // 8 waves of 64 x 64
     {256, 128, 1, 256, 3.09, 0.789, 0.993, 2.48},    // two groups of four 64 x 128 waves
     {128, 128, 1, 512, 2.80, 0.737, 0.606, 0.00},    // 4 waves of 64 x 64
-    {64, 64, 4, 512, 2.71, 0.856, 0.970, 1.44},      // gemm_flex.hpp, K dealt to 4 waves
+    {64, 64, 4, 512, 2.71, 0.856, 0.900, 1.44},      // gemm_flex.hpp, K dealt to 4 waves
     {64, 64, 2, 1024, 2.84, 0.745, 0.449, 1.99},     // ... to 2 waves, for many tiles or a short K
     {32, 64, 4, 768, 2.95, 0.681, 0.637, 0.44},
     {32, 32, 4, 512, 1.67, 0.472, 0.435, 1.15},
+    // gemm_flex.hpp, ring of K steps.  From timings inside whole steps, where weights come from memory: K = 512 (32
+    // products of [512 x 128]) 10-12 us against 8-10 on 64 x 64 tiles, K = 2048 20 against 22, K = 4096 35-39 against
+    // 40-50, K = 6144 51 against 49 and K = 8192 54-60 against 52-59 on 256 x 128 tiles with K in four slices.
+    {64, 128, 1, 256, 2.40, 0.380, 0.430, 2.20},
 };
 
 inline bool is_flex(int kernel) { return kernel >= kFlex64; }

@@ -483,3 +483,21 @@ def test_gemm_fp32_small_tiles_are_exact_on_integers(ta, tb, m, n, k, batch):
     c0 = rng.integers(-9, 10, (batch, m, n)).astype(np.float32)
     got, ref = run_gemm(ta, tb, m, n, k, a, b, F32, F32, F32, hip.GEMM_F32, batch=batch, bias=bias, c0=c0)
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("c_dt", [F32, F16])
+@pytest.mark.parametrize("m,n,k,batch", [
+    (1024, 2048, 328, 1),    # whole tiles, exactly as many K steps as the ring holds, the last one ragged
+    (960, 1800, 2056, 1),    # an odd number of steps, ragged columns
+    (1002, 2040, 1096, 1),   # ragged in every direction
+    (512, 1000, 1032, 4),    # batch entries
+])
+def test_gemm_tiles_on_a_ring_of_k_steps_are_exact_on_integers(ta, tb, c_dt, m, n, k, batch):
+    """64 x 128 tiles, one workgroup per CU: waves that load beside waves that multiply."""
+    test_gemm_small_and_ragged_products_are_exact_on_integers(ta, tb, c_dt, m, n, k, batch)
+
+
+@pytest.mark.parametrize("dtype", [F16, BF16])
+def test_linear_gelu_epilogue_on_a_ring_of_k_steps(dtype):
+    test_linear_gelu_epilogue_writes_both_tensors(dtype, 1024, 2048, 2048)
