@@ -2,6 +2,7 @@
 
 #include <cmath>
 #include <cstring>
+#include <vector>
 
 #include "br_hip.h"
 #include "host_tensor.hpp"
@@ -380,8 +381,9 @@ ComputingReturn HIPTensor<DT>::op_last_logits(tensor_t self, tensor_t mask_, ten
     const int64_t hidden = (int64_t)self->shape()[2], vocab = (int64_t)lm_head->shape()[0];
     if (!dev_f32(output) || (int64_t)output->items() < batch * vocab) return OP_OUTPUT_ERROR;
     const int* mask = static_cast<const int*>(mask_->data());
-    float* rows = static_cast<float*>(ComputingContext::workspace);
+    void* rows = ComputingContext::workspace;
     br_assert((size_t)(batch * hidden) * sizeof(float) <= head_bytes(), "workspace too small for last_logits");
+    std::vector<int64_t> targets((size_t)batch);
     for (int64_t b = 0; b < batch; b++) {
         const int* m = mask + b * tokens;
         int64_t target = 0;
@@ -391,11 +393,14 @@ ComputingReturn HIPTensor<DT>::op_last_logits(tensor_t self, tensor_t mask_, ten
                 break;
             }
         }
-        BR_OP(br_hip_memcpy_d2d(rows + b * hidden, static_cast<const float*>(mem_) + (b * tokens + target) * hidden,
-                                hidden * sizeof(float), stream()));
+        targets[b] = b * tokens + target;
     }
-    BR_OP(product(0, 1, batch, vocab, hidden, 1.0f, rows, BR_F32, hidden, 0, lm_head->data(), code(lm_head),
-                      hidden, 0, 0, output->data(), BR_F32, vocab, 0, nullptr, 1, pick_compute({self, lm_head})));
+    // the rows arrive in the type the product multiplies in (the rounding it would apply itself)
+    const int compute = pick_compute({self, lm_head});
+    const int type = compute == BR_GEMM_F16 ? BR_F16 : compute == BR_GEMM_BF16 ? BR_BF16 : BR_F32;
+    BR_OP(br_hip_pick_rows(static_cast<const float*>(mem_), targets.data(), rows, type, batch, hidden, stream()));
+    BR_OP(product(0, 1, batch, vocab, hidden, 1.0f, rows, type, hidden, 0, lm_head->data(), code(lm_head), hidden, 0, 0,
+                  output->data(), BR_F32, vocab, 0, nullptr, 1, compute));
     return OP_OK;
 }
 

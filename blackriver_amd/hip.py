@@ -87,6 +87,7 @@ SIGNATURES = {
     "br_hip_adamw": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _i64, _f32, _f32, _f32, _f32, _f32, _i64, _vp]),
     "br_hip_adamw_group": (_int, [_vp, _i64, _f32, _f32, _f32, _f32, _f32, _i64, _vp]),
     "br_hip_embedding_gather": (_int, [_vp, _vp, _vp, _int, _i64, _i64, _i64, _vp]),
+    "br_hip_pick_rows": (_int, [_vp, _vp, _vp, _int, _i64, _i64, _vp]),
     "br_hip_embedding_scatter_add": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _f32, _vp]),
     "br_hip_alibi_table": (_int, [_vp, _i64, _i64, _vp]),
     "br_hip_xmask_table": (_int, [_vp, _vp, _i64, _i64, _vp]),

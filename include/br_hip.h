@@ -454,6 +454,10 @@ int br_hip_adamw_group(const br_adamw_tensor* tensors, int64_t count, float lr, 
 /* The embedding row gather of blackriver/train_bloom.cpp:50-56. */
 int br_hip_embedding_gather(const void* table, const int32_t* ids, void* out, int elem_bytes,
                             int64_t n, int64_t hidden, int64_t vocab, br_stream_t stream);
+/* out[i, :] = x[rows[i], :] as out_dtype, rows being a host array that is read
+ * before the call returns: the last-token rows of cuda_tensor.cpp:424-432. */
+int br_hip_pick_rows(const float* x, const int64_t* rows, void* out, int out_dtype, int64_t n, int64_t cols,
+                     br_stream_t stream);
 /* Backward of that gather: grad[ids[i], :] += dx_scale * dx[i, :] for i = 0 .. n-1 in
  * ascending i (fp32; repeated ids are summed in position order, so the result
  * is deterministic); ids outside [0, vocab) are skipped.  The reference has no

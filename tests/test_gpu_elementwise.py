@@ -433,3 +433,21 @@ def test_column_sums_in_one_launch(rows, cols):
         call("br_hip_bias_gelu_bwd", ptr(h), ptr(h), ptr(bias), ptr(dx), ptr(dbias), code, rows, cols, 1.0, ptr(ws),
              ws.numel(), stream())
         check(dbias, dx)
+
+
+@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+@pytest.mark.parametrize("n,cols,offset", [(1, 1, 0), (3, 1028, 0), (5, 1030, 0), (257, 64, 0), (2, 64, 1)])
+def test_pick_rows_copies_and_rounds(dtype, n, cols, offset):
+    """Row pieces of 4 columns and of one (odd widths, an unaligned source), one row past a launch's 256."""
+    rng = np.random.default_rng(n + cols)
+    total = 300
+    flat = dev(rng.standard_normal(total * cols + offset).astype(np.float32))
+    x = flat[offset:].view(total, cols)
+    rows = rng.integers(0, total, n).astype(np.int64)
+    t = {F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16}[dtype]
+    out = torch.full((n + 1, cols), 7.0, dtype=t, device="cuda")
+    call("br_hip_pick_rows", ptr(x), rows.ctypes.data, ptr(out), dtype, n, cols, stream())
+    torch.cuda.synchronize()
+    assert torch.equal(out[:n], x[torch.from_numpy(rows).cuda()].to(t))
+    assert bool((out[n:] == 7.0).all())
+    assert hip.load().br_hip_pick_rows(ptr(x), np.array([-1], np.int64).ctypes.data, ptr(out), dtype, 1, cols, stream()) < 0
