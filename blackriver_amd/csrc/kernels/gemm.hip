@@ -558,8 +558,10 @@ int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
         ws += staged_bytes(b_rows, b_cols, batch);
     }
     const gemm16::Plan plan = gemm16::gemm_plan(m, n, k, batch, true);
-    const bool aligned = aligned16(a) && aligned16(b) && lda % 8 == 0 && ldb % 8 == 0;
-    if (plan.slices > 1 && aligned) {
+    // only the direct-to-LDS kernels know slices: the register-staged one would sum all of K once per slice
+    const bool sliceable = aligned16(a) && aligned16(b) && lda % 8 == 0 && ldb % 8 == 0 &&
+                           gemm16::dtl_spans(trans_a != 0, lda, trans_b == 0, ldb, n, m, n, k);
+    if (plan.slices > 1 && sliceable) {
         float* part = reinterpret_cast<float*>(ws);
         const int rc = gemm_impl(trans_a, trans_b, m, n, k, 1.0f, a, a_dtype, lda, 0, b, b_dtype, ldb, 0, 0, nullptr,
                                  part, BR_F32, n, m * n, nullptr, plan.slices, compute, stream, &plan, true);

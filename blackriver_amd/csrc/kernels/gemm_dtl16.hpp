@@ -924,13 +924,16 @@ inline bool ragged_applies(const Problem& p) { return !p.a_kstr || (p.b_kstr && 
 // The direct-to-LDS kernels apply when both operands are 16-bit and 16-byte aligned, a k-contiguous operand's rows
 // end on a 16-byte granule of their own (K a multiple of 8, or zero-filled up to one), and every per-lane offset fits
 // 32 bits (of the operands, and of a tile of C, which spans up to 256 rows).
+inline bool dtl_spans(bool a_kstr, long long lda, bool b_kstr, long long ldb, long long ldc, long long m, long long n, long long k) {
+    const long long lim = 1LL << 31;
+    const long long a_span = a_kstr ? 2 * 64 * lda : 2 * 256 * lda;
+    const long long b_span = b_kstr ? 2 * 64 * ldb : 2 * 256 * ldb;
+    return a_span < lim && b_span < lim && ldc < (1LL << 21) && m < lim && n < lim && k < lim;
+}
 inline bool dtl_applies(const GemmArgs& g, const Problem& p) {
     if (p.a_f32 || p.b_f32 || !g.vec_a || !g.vec_b || g.k <= 0) return false;
     if (g.k % 8 != 0 && !p.padded && !(p.a_kstr && p.b_kstr)) return false;
-    const long long lim = 1LL << 31;
-    const long long a_span = p.a_kstr ? 2 * 64 * g.lda : 2 * 256 * g.lda;
-    const long long b_span = p.b_kstr ? 2 * 64 * g.ldb : 2 * 256 * g.ldb;
-    return a_span < lim && b_span < lim && g.ldc < (1LL << 21) && g.m < lim && g.n < lim && g.k < lim;
+    return dtl_spans(p.a_kstr, g.lda, p.b_kstr, g.ldb, g.ldc, g.m, g.n, g.k);
 }
 
 // bytes of partial tiles the two-slice split wants in the caller's workspace (one per output tile)

@@ -501,3 +501,25 @@ def test_gemm_tiles_on_a_ring_of_k_steps_are_exact_on_integers(ta, tb, c_dt, m, 
 @pytest.mark.parametrize("dtype", [F16, BF16])
 def test_linear_gelu_epilogue_on_a_ring_of_k_steps(dtype):
     test_linear_gelu_epilogue_writes_both_tensors(dtype, 1024, 2048, 2048)
+
+
+@pytest.mark.parametrize("a_wide", [True, False])
+def test_gemm_staged_rows_too_far_apart_for_slices(a_wide):
+    """An operand whose rows lie 2^22 elements apart is beyond the offsets of the kernels that know slices of K: the
+    product is not sliced (small integers: exact), also where its sizes alone would have it in slices."""
+    print("case a_wide=%s" % a_wide, flush=True)
+    m, n, k, ld = 4, 4, 8192, 1 << 22
+    rng = np.random.default_rng(3)
+    a = rng.integers(-3, 4, (m, k)).astype(np.float32)
+    b = rng.integers(-2, 3, (n, k)).astype(np.float32)
+    spread = torch.zeros((4, ld), dtype=torch.float16, device="cuda")
+    spread[:, :k] = torch.from_numpy(a if a_wide else b).cuda().half()
+    dense = to_dev(b if a_wide else a, F16)
+    pa, lda, pb, ldb = (spread, ld, dense, k) if a_wide else (dense, k, spread, ld)
+    c = torch.zeros((m, n), device="cuda")
+    need = hip.load().br_hip_gemm_staged_workspace(0, 1, m, n, k, F16, F16, 1)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda").fill_(255)
+    call("br_hip_gemm_staged", 0, 1, m, n, k, 1.0, ptr(pa), F16, lda, 0, ptr(pb), F16, ldb, 0, 0, ptr(c), F32, n, 0, None,
+         1, hip.GEMM_F16, ptr(ws), need, stream())
+    assert need > 0   # sliced by its sizes
+    assert np.array_equal(to_host64(c), a.astype(np.float64) @ b.astype(np.float64).T)
