@@ -327,17 +327,17 @@ int br_hip_gemm(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
                 const float* bias, int64_t batch, int compute, br_stream_t stream);
 
 /* The same product for callers that can lend scratch memory.  fp32 operands
- * are first converted to the 16-bit compute type into `workspace` (dense
- * copies, one pass each), so that the product runs on the direct-to-LDS
- * kernel that needs both operands in the MFMA type.  Replaces the same
+ * are first converted to the 16-bit compute type into `workspace`, and 16-bit
+ * ones whose rows do not start on 16-byte boundaries moved to rows that do
+ * (one pass each), so that the product runs on the direct-to-LDS kernels,
+ * which need both operands aligned and in the MFMA type.  Replaces the same
  * kernels::LtSgemm call (LtSgemm.cu:55-126); `workspace` plays the part of
  * the scratch the reference hands to cublasLtMatmul (context.cpp:31).  An
  * unbatched product with too few output tiles for the 256 CUs and a long K is
  * split along K into fp32 partials in the same workspace and summed in a fixed
  * order (deterministic).  Falls back to br_hip_gemm when `compute`
- * is BR_GEMM_F32, no operand is fp32, the shape is not 16-byte friendly
- * (k % 32, operand row lengths % 8) or the workspace is smaller than
- * br_hip_gemm_staged_workspace() bytes.  Results equal br_hip_gemm's for the
+ * is BR_GEMM_F32, an operand has the other 16-bit type, or the workspace is
+ * not 16-byte aligned or smaller than br_hip_gemm_staged_workspace() bytes.  Results equal br_hip_gemm's for the
  * same `compute` up to the order of the fp32 summation (same rounding of the
  * operands). */
 size_t br_hip_gemm_staged_workspace(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k,
@@ -356,7 +356,7 @@ int br_hip_gemm_staged(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k
  * x [rows, in], w [out, in], u and y [rows, out] are dense, all of `dtype`
  * (BR_F16 or BR_BF16); bias fp32 (may be NULL).  The activation is evaluated on
  * the fp32 sum, before u is rounded.  BR_ERR_TODO when the shape or alignment
- * rules out the direct-to-LDS kernel (in % 32, 16-byte aligned rows): the
+ * rules out the direct-to-LDS kernels (in % 32, 16-byte aligned rows): the
  * caller then runs the two operators. */
 int br_hip_linear_gelu(const void* x, const void* w, const float* bias, void* u, void* y, int dtype,
                        int64_t rows, int64_t out, int64_t in, br_stream_t stream);
