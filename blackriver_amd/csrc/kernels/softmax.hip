@@ -275,11 +275,12 @@ __global__ __launch_bounds__(kBlock) void softmax_bwd_generic(const float* dy, c
         dx[row * cols + c] = y[row * cols + c] * (dy[row * cols + c] - s[0]);
 }
 
-// Floats per granule for rows of `cols` floats at these addresses (null ones do not count).
+// Floats per granule for rows of `cols` floats at these addresses (null ones do not count).  Never less than one: an
+// address that is no multiple of four bytes is read float by float, as the workgroup-per-row kernel reads it.
 int granule_of(int64_t cols, std::initializer_list<const void*> at) {
     int g = cols % 4 == 0 ? 4 : cols % 2 == 0 ? 2 : 1;
     for (const void* p : at)
-        while (reinterpret_cast<uintptr_t>(p) % (4 * g) != 0) g /= 2;
+        while (g > 1 && reinterpret_cast<uintptr_t>(p) % (4 * g) != 0) g /= 2;
     return g;
 }
 constexpr int64_t kMaxRegisterRow = 2048;   // floats of a row in granules of fewer than four (32 registers of a lane)

@@ -1,0 +1,31 @@
+"""What the entry points of libbr_hip.so decide on the host, before a kernel runs.
+
+Calls are made by a child process that is shown no GPU, so that nothing can be
+launched wherever the tests run: an accepted call ends in the runtime's error
+for a missing device, a refused one in the library's own code (negative)."""
+import os
+import subprocess
+import sys
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+
+
+def answer(call):
+    """Return code of `L.<call>`, made without a GPU."""
+    env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES="-1")
+    text = "from blackriver_amd import hip; L = hip.load(); print('answer', L.%s)" % call
+    out = subprocess.run([sys.executable, "-c", text], cwd=ROOT, env=env, timeout=60, capture_output=True, text=True)
+    assert out.returncode == 0, out
+    return int(out.stdout.split("answer")[1])
+
+
+@pytest.mark.parametrize("call", [
+    "br_hip_softmax_fwd(4097, 8192, 4, 8, None)",
+    "br_hip_softmax_fwd(4096, 8194, 4, 7, None)",
+    "br_hip_softmax_bwd(4096, 8192, 16387, 4, 8, None)",
+    "br_hip_alibi_masked_softmax_fwd(4096, 8193, 16384, 32768, 1, 1, 4, 4, None)",
+])
+def test_softmax_takes_addresses_of_any_alignment(call):
+    assert answer(call) > 0
