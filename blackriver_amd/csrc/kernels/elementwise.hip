@@ -1030,8 +1030,8 @@ __global__ __launch_bounds__(kBlock) void normal_kernel(T* dst, float mean, floa
 
 // Backward of the row gather: grad[ids[i], :] += dx[i, :] for i = 0 .. n-1, in
 // that order, so that the result does not depend on scheduling when an id
-// occurs several times.  Workgroup (i, s) owns columns s * kBlock * VEC .. of the row of
-// id = ids[i] if i is that id's first position; it collects the later positions
+// occurs several times.  Workgroup (i, s) owns column blocks s, s + gridDim.y, .. (of kBlock * VEC columns) of the
+// row of id = ids[i] if i is that id's first position; it collects the later positions
 // of the same id, a block of positions at a time, into an ascending list in LDS
 // and folds their rows in, four loads in flight, starting from the row's current
 // value.  What bounds it is the longest run of one id (text repeats a few ids
@@ -1050,52 +1050,54 @@ __global__ __launch_bounds__(kBlock) void scatter_add_rows(const float* __restri
     int seen = 0;
     for (int j = t; j < i; j += kBlock) seen |= ids[j] == id;
     if (__syncthreads_or(seen)) return;
-    const int64_t c = ((int64_t)blockIdx.y * kBlock + t) * VEC;
-    const bool mine = c < hidden;
-    float* row = grad + (int64_t)id * hidden + c;
-    float acc[VEC];
     auto read = [](const float* p, float (&f)[VEC]) {
         if constexpr (VEC == 4) VecIO<float, 4>::load(p, f);
         else f[0] = *p;
     };
-    if (mine) read(row, acc);
-    for (int base = i; base < n; base += kBlock) {
-        const int j = base + t;
-        const bool hit = j < n && ids[j] == id;
-        const unsigned long long hits = __ballot(hit);
-        if ((t & 63) == 0) found[t >> 6] = __popcll(hits);
-        __syncthreads();
-        int at = __popcll(hits & ((1ull << (t & 63)) - 1)), count = 0;
+    for (int64_t first = (int64_t)blockIdx.y * kBlock * VEC; first < hidden; first += (int64_t)gridDim.y * kBlock * VEC) {
+        const int64_t c = first + t * VEC;
+        const bool mine = c < hidden;
+        float* row = grad + (int64_t)id * hidden + c;
+        float acc[VEC];
+        if (mine) read(row, acc);
+        for (int base = i; base < n; base += kBlock) {
+            const int j = base + t;
+            const bool hit = j < n && ids[j] == id;
+            const unsigned long long hits = __ballot(hit);
+            if ((t & 63) == 0) found[t >> 6] = __popcll(hits);
+            __syncthreads();
+            int at = __popcll(hits & ((1ull << (t & 63)) - 1)), count = 0;
 #pragma unroll
-        for (int w = 0; w < kBlock / kWave; w++) {
-            at += w < (t >> 6) ? found[w] : 0;
-            count += found[w];
+            for (int w = 0; w < kBlock / kWave; w++) {
+                at += w < (t >> 6) ? found[w] : 0;
+                count += found[w];
+            }
+            if (hit) list[at] = j;
+            __syncthreads();
+            if (mine) {
+                int p = 0;
+                for (; p + 4 <= count; p += 4) {
+                    float d[4][VEC];
+#pragma unroll
+                    for (int u = 0; u < 4; u++) read(dx + (int64_t)list[p + u] * hidden + c, d[u]);
+#pragma unroll
+                    for (int u = 0; u < 4; u++)
+#pragma unroll
+                        for (int e = 0; e < VEC; e++) acc[e] += d[u][e] * scale;
+                }
+                for (; p < count; p++) {
+                    float d[VEC];
+                    read(dx + (int64_t)list[p] * hidden + c, d);
+#pragma unroll
+                    for (int e = 0; e < VEC; e++) acc[e] += d[e] * scale;
+                }
+            }
+            __syncthreads();   // the list is used up
         }
-        if (hit) list[at] = j;
-        __syncthreads();
         if (mine) {
-            int p = 0;
-            for (; p + 4 <= count; p += 4) {
-                float d[4][VEC];
-#pragma unroll
-                for (int u = 0; u < 4; u++) read(dx + (int64_t)list[p + u] * hidden + c, d[u]);
-#pragma unroll
-                for (int u = 0; u < 4; u++)
-#pragma unroll
-                    for (int e = 0; e < VEC; e++) acc[e] += d[u][e] * scale;
-            }
-            for (; p < count; p++) {
-                float d[VEC];
-                read(dx + (int64_t)list[p] * hidden + c, d);
-#pragma unroll
-                for (int e = 0; e < VEC; e++) acc[e] += d[e] * scale;
-            }
+            if constexpr (VEC == 4) VecIO<float, 4>::store(row, acc);
+            else *row = acc[0];
         }
-        __syncthreads();   // the list is used up
-    }
-    if (mine) {
-        if constexpr (VEC == 4) VecIO<float, 4>::store(row, acc);
-        else *row = acc[0];
     }
 }
 
@@ -1554,8 +1556,7 @@ int br_hip_embedding_scatter_add(const float* dx, const int32_t* ids, float* gra
     if (!grad || (const float*)grad == dx) return BR_ERR_OUTPUT;
     const int vec = hidden % 4 == 0 && aligned16(dx) && aligned16(grad) ? 4 : 1;
     const int64_t blocks = (hidden + (int64_t)kBlock * vec - 1) / ((int64_t)kBlock * vec);
-    if (blocks > 65535) return BR_ERR_ATTR;
-    const dim3 grid((unsigned)n, (unsigned)blocks);
+    const dim3 grid((unsigned)n, (unsigned)(blocks < 65535 ? blocks : 65535));
     if (vec == 4)
         scatter_add_rows<4><<<grid, kBlock, 0, as_stream(stream)>>>(dx, ids, grad, (int)n, hidden, vocab, dx_scale);
     else

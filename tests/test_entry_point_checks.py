@@ -29,3 +29,8 @@ def answer(call):
 ])
 def test_softmax_takes_addresses_of_any_alignment(call):
     assert answer(call) > 0
+
+
+@pytest.mark.parametrize("hidden", [65535 * 256 + 1, 65535 * 1024 + 4])
+def test_embedding_backward_takes_rows_of_any_length(hidden):
+    assert answer("br_hip_embedding_scatter_add(4096, 8192, 16384, 2, %d, 4, 1.0, None)" % hidden) > 0

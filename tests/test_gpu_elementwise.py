@@ -279,6 +279,23 @@ def test_embedding_scatter_add_is_the_sequential_scatter(n, hidden, vocab):
     assert np.array_equal(host(d_grad), want)
 
 
+@pytest.mark.parametrize("hidden", [65535 * 256 + 301, 65535 * 1024 + 1028])
+def test_embedding_scatter_add_rows_of_more_blocks_than_a_grid_is_high(hidden):
+    """Rows longer than 65535 column blocks: workgroups take several blocks
+    each.  Small integers, so that every sum is exact."""
+    print("case hidden=%d" % hidden, flush=True)
+    torch.manual_seed(3)
+    dx = torch.randint(-8, 9, (3, hidden), device="cuda").float()
+    grad = torch.randint(-8, 9, (2, hidden), device="cuda").float()
+    want = grad.clone()
+    want[1] += dx[0] + dx[2]
+    want[0] += dx[1]
+    ids = torch.tensor([1, 0, 1], dtype=torch.int32, device="cuda")
+    call("br_hip_embedding_scatter_add", ptr(dx), ptr(ids), ptr(grad), 3, hidden, 2, 1.0, stream())
+    torch.cuda.synchronize()
+    assert torch.equal(grad, want)
+
+
 @pytest.mark.parametrize("dtype,master", [(F32, False), (F16, True), (F16, False), (BF16, True)])
 @pytest.mark.parametrize("n", [4096 * 1024, 1001])
 def test_adamw_against_oracle(n, dtype, master):
