@@ -492,12 +492,12 @@ __global__ __launch_bounds__(kBlock) void colsum_final(const float* partial, flo
     out[col] = acc * scale;
 }
 
-// Vector forms of the two stages for fp32 (cols % 4 == 0, 16-byte aligned rows).
-// Stage 1: a thread owns four adjacent columns and sums a strip of rows, four
+// Vector forms of the two stages (cols % VEC == 0, 16-byte aligned rows).
+// Stage 1: a thread owns VEC adjacent columns and sums a strip of rows, four
 // rows of loads in flight at a time.
-__global__ __launch_bounds__(kBlock) void colsum_partial_vec(const float* __restrict__ x, float* __restrict__ partial,
+template <typename T, int VEC>
+__global__ __launch_bounds__(kBlock) void colsum_partial_vec(const T* __restrict__ x, float* __restrict__ partial,
                                                               int64_t rows, int64_t cols, int rows_per_block) {
-    constexpr int VEC = 4;
     const int64_t col = ((int64_t)blockIdx.x * kBlock + threadIdx.x) * VEC;
     if (col >= cols) return;
     const StripWalk w = strip_walk(rows, rows_per_block);
@@ -509,7 +509,7 @@ __global__ __launch_bounds__(kBlock) void colsum_partial_vec(const float* __rest
     for (; r + 3 * step < r1; r += 4 * step) {
         float v[4][VEC];
 #pragma unroll
-        for (int u = 0; u < 4; u++) VecIO<float, VEC>::load(x + (r + u * step) * cols + col, v[u]);
+        for (int u = 0; u < 4; u++) VecIO<T, VEC>::load(x + (r + u * step) * cols + col, v[u]);
 #pragma unroll
         for (int u = 0; u < 4; u++)
 #pragma unroll
@@ -517,7 +517,7 @@ __global__ __launch_bounds__(kBlock) void colsum_partial_vec(const float* __rest
     }
     for (; r < r1; r += step) {
         float v[VEC];
-        VecIO<float, VEC>::load(x + r * cols + col, v);
+        VecIO<T, VEC>::load(x + r * cols + col, v);
 #pragma unroll
         for (int j = 0; j < VEC; j++) acc[j] += v[j];
     }
@@ -782,20 +782,36 @@ __global__ __launch_bounds__(kOwnThreads) void colsum_owner_kernel(Src src_arg, 
     for (int j = 0; j < VEC; j++) acc[j] = 0.f;
     if (col < cols) {
         src.init(col);
-        for (int64_t r = rr; r < rows; r += UNROLL * RPP) {
+        // One pass over rows that are all there: nothing conditional, so that the arithmetic of all positions overlaps
+        // ([512 x 8192] fp16 5.4 -> 4.8 us).  Several passes keep the test of every position: each position then waits for
+        // its own loads alone ([4096 x 16384] fp16 25.9 us, 28.8 without).
+        const bool whole = UNROLL > 1 && rows <= UNROLL * RPP && rr + (UNROLL - 1) * RPP < rows;
+        if (whole) {
             float in[UNROLL][NIN][VEC];
-            // positions past the last row read that row (every load of a pass leaves before the first is used)
+#pragma unroll
+            for (int u = 0; u < UNROLL; u++) src.load((int64_t)(rr + u * RPP) * cols + col, in[u]);
 #pragma unroll
             for (int u = 0; u < UNROLL; u++) {
-                const int64_t at = r + u * RPP;
-                src.load((at < rows ? at : rows - 1) * cols + col, in[u]);
+                src.finish((int64_t)(rr + u * RPP) * cols + col, in[u]);
+#pragma unroll
+                for (int j = 0; j < VEC; j++) acc[j] += in[u][0][j];
             }
+        } else {
+            for (int64_t r = rr; r < rows; r += UNROLL * RPP) {
+                float in[UNROLL][NIN][VEC];
+                // positions past the last row read that row (every load of a pass leaves before the first is used)
 #pragma unroll
-            for (int u = 0; u < UNROLL; u++) {
-                if (r + u * RPP < rows) {
-                    src.finish((r + u * RPP) * cols + col, in[u]);
+                for (int u = 0; u < UNROLL; u++) {
+                    const int64_t at = r + u * RPP;
+                    src.load((at < rows ? at : rows - 1) * cols + col, in[u]);
+                }
 #pragma unroll
-                    for (int j = 0; j < VEC; j++) acc[j] += in[u][0][j];
+                for (int u = 0; u < UNROLL; u++) {
+                    if (r + u * RPP < rows) {
+                        src.finish((r + u * RPP) * cols + col, in[u]);
+#pragma unroll
+                        for (int j = 0; j < VEC; j++) acc[j] += in[u][0][j];
+                    }
                 }
             }
         }
@@ -819,36 +835,58 @@ __global__ __launch_bounds__(kOwnThreads) void colsum_owner_kernel(Src src_arg, 
     }
 }
 
-// Lanes per row of the one-launch column sum, or 0 where two launches are faster.  Depends on the shape, the element
-// size and the kind of source alone, so entries that promise each other's bits (br_hip_colsum / br_hip_colsum_cast /
-// br_hip_gelu_bwd_colsum_cast on fp32) always agree on the path.  Measured, us, two launches / one with 8, 4, 2 lanes:
-//   16-bit sums         [78,1024] 4.5 / 2.9 3.2 3.6   [512,1024] 5.1 / 3.5 3.8 4.0   [2048,4096] 8.6 / 8.6 7.4 7.7
-//                       [2048,12288] 15.9 / 11.9 18.2 19.8: 8 lanes, 4 for many rows of few columns
-//   fp32 sum and copy   [78,1024] 4.6 / 2.6 2.6 2.8   [512,1024] 5.2 / 3.3 3.2 3.4   [1000,4096] 10.8 / 8.2 7.6 11.2
-//                       [1000,8192] 15.4 / 11.2 14.4 22.8   [2048,2048] 8.9 / 13.5 11.7 10.4: 4 lanes while they
-//                       make at most 256 workgroups, one launch up to 1024 rows.  With the GELU backward in front the
-//                       arithmetic wants every CU: [250,1024] 5.7 / 3.4 3.2 3.2, [512,4096] 10.2 / 9.6 9.4 13.7,
-//                       [1000,4096] 17.0 / 18.0 17.4 27.7
-//   bias-GELU backward  [78,4096] 7.9 / 4.0 4.0 4.3   [200,2048] 7.9 / 5.1 4.6 4.4   [1000,4096] 13.5 / 16.4 12.4 12.2
-//   (fp16)              [1000,8192] 15.6 / 18.0 15.5 26.0   [2048,16384] 41.5 / 41.4 65.9 -: as narrow as makes at
-//                       most 256 workgroups, one launch up to 1024 rows
+// Lanes per row of the one-launch column sum, or 0 where two launches are faster: on many rows, where a workgroup's walk
+// takes longer than the second launch.  Depends on the shape, the element size and the kind of source alone, so entries
+// that promise each other's bits (br_hip_colsum / br_hip_colsum_cast / br_hip_gelu_bwd_colsum_cast on fp32) always
+// agree on the path -- the rule for fp32 is therefore one that suits all three.  Measured, us, two launches / one with 2,
+// 4, 8 lanes:
+//   16-bit sums         [64,1024] 4.8 / 3.7 3.4 3.1   [256,4096] 5.5 / 3.9 4.2 4.3   [512,2048] 5.8 / 4.6 5.0 4.5
+//                       [1000,1024] 6.7 / 6.0 6.1 6.6   [1024,8192] 12.0 / 9.8 7.0 7.0   [2048,1024] 6.6 / 8.7 9.1 10.2
+//                       [2048,4096] 9.6 / 9.4 9.8 10.8   [2048,6144] 11.7 / 16.5 10.4 11.3   [4096,512] 7.3 / 14 15 17
+//                       [4096,6144] 14.8 / 30 18 20   [4096,16384] 29.7 / 54 37 25.9   [65536,512] 44 / - 204 -
+//   fp32 sum and copy   [64,1024] 4.8 / 3.0 2.9 2.9   [256,1024] 4.9 / 3.2 3.2 3.4   [512,1024] 5.7 / 4.1 4.6 5.0
+//                       [512,8192] 10.3 / 12 9.0 7.3   [1000,1024] 7.5 / 6.9 7.0 7.8   [1000,4096] 11.2 / 12 8.6 9.2
+//                       [1000,8192] 14.7 / 23 15 11.7
+//   with GELU backward  [64,1024] 5.8 / 3.1 3.0 3.1   [256,1024] 6.4 / 4.2 4.5 5.1   [512,1024] 7.0 / 6.8 7.8 8.8
+//   in front            [768,1024] 8.0 / 9.9 11 12   [1000,2048] 11.7 / 15 16 17   [1000,4096] 16.8 / 30 18.1 19.1
+//                       [1000,8192] 26.1 / 65 38 25.4
+//   bias-GELU backward  [64,4096] 8.2 / 4.5 4.3 4.2   [256,2048] 8.2 / 6.3 5.6 5.8   [512,4096] 9.3 / 8.7 8.6 9.3
+//   (fp16)              [1000,1024] 12.3 / 11.0 12.4 14   [1000,4096] 13.7 / 14.4 14.1 15   [1000,8192] 15.7 / 27 16.5 17.2
+//                       [1000,16384] 24.4 / 55 32 21.9;  (fp32) [512,2048] 8.2 / 7.6 8.1 8.6   [768,1024] 8.7 / 9.2 10 11
 enum OwnerKind { kOwnSum, kOwnBiasGelu };
 int owner_lanes(int64_t rows, int64_t cols, int elem_bytes, OwnerKind kind) {
-    const int64_t vec = elem_bytes == 4 ? 4 : 8;
-    if (cols % vec != 0) return 0;
-    if (kind == kOwnSum && elem_bytes == 2) return rows > 1024 && cols <= 64 * 64 ? 4 : 8;
+    const bool narrow_type = elem_bytes != 4;   // 16-bit elements
+    if (cols % (narrow_type ? 8 : 4) != 0) return 0;
+    if (rows <= 128) return 8;   // one row position a thread
+    if (rows <= 512) {
+        if (cols > 4096) return 8;
+        if (narrow_type) return kind == kOwnSum ? 2 : 4;
+        return cols <= 2048 ? 2 : 4;
+    }
+    if (kind == kOwnSum && narrow_type) {
+        if (rows <= 1024) return cols <= 8192 ? 4 : 8;
+        if (rows <= 2048 && cols >= 6144) return cols <= 8192 ? 4 : 8;
+        return cols >= 12288 ? 8 : 0;
+    }
     if (rows > 1024) return 0;
-    if (kind == kOwnBiasGelu && cols <= 256 * 2 * vec) return 2;
-    return cols <= 256 * 4 * vec ? 4 : 8;
+    if (kind == kOwnBiasGelu) return narrow_type ? (cols <= 2048 ? 2 : cols < 12288 ? 0 : 8) : (cols < 6144 ? 0 : 8);
+    return cols < 3072 ? 0 : cols <= 4096 ? 4 : 8;
 }
 
+template <int LPR, int UNROLL, typename Src>
+void colsum_owner_launch_lanes(const Src& src, float* out, int64_t rows, int64_t cols, float scale, hipStream_t st) {
+    const int64_t cw = LPR * Src::VEC;
+    const unsigned grid = (unsigned)((cols + cw - 1) / cw);
+    // rows of a single pass: no loads beside those of that pass (with two or four passes in flight their surplus costs
+    // 0.4 us, half as much again with the GELU gradient)
+    if (rows <= kOwnThreads / LPR) colsum_owner_kernel<LPR, 1, Src><<<grid, kOwnThreads, 0, st>>>(src, out, rows, cols, scale);
+    else colsum_owner_kernel<LPR, UNROLL, Src><<<grid, kOwnThreads, 0, st>>>(src, out, rows, cols, scale);
+}
 template <int UNROLL, typename Src>
 int colsum_owner_launch(int lanes, const Src& src, float* out, int64_t rows, int64_t cols, float scale, hipStream_t st) {
-    const int64_t cw = lanes * Src::VEC;
-    const unsigned grid = (unsigned)((cols + cw - 1) / cw);
-    if (lanes == 8) colsum_owner_kernel<8, UNROLL, Src><<<grid, kOwnThreads, 0, st>>>(src, out, rows, cols, scale);
-    else if (lanes == 4) colsum_owner_kernel<4, UNROLL, Src><<<grid, kOwnThreads, 0, st>>>(src, out, rows, cols, scale);
-    else colsum_owner_kernel<2, UNROLL, Src><<<grid, kOwnThreads, 0, st>>>(src, out, rows, cols, scale);
+    if (lanes == 8) colsum_owner_launch_lanes<8, UNROLL>(src, out, rows, cols, scale, st);
+    else if (lanes == 4) colsum_owner_launch_lanes<4, UNROLL>(src, out, rows, cols, scale, st);
+    else colsum_owner_launch_lanes<2, UNROLL>(src, out, rows, cols, scale, st);
     BR_HIP_LAUNCH_CHECK();
     return BR_OK;
 }
@@ -1407,11 +1445,16 @@ int br_hip_colsum(const void* x, int dtype, float* out, int64_t rows, int64_t co
             if (dtype == BR_F16) return colsum_owner_launch<4>(lanes, OwnPlain<__half, 8>{(const __half*)x}, out, rows, cols, out_scale, st);
             return colsum_owner_launch<4>(lanes, OwnPlain<__hip_bfloat16, 8>{(const __hip_bfloat16*)x}, out, rows, cols, out_scale, st);
         }
-        // two launches: fp32 only (16-bit sums of such columns always take the one)
         const int64_t blocks_x = (cols / vec + kBlock - 1) / kBlock;
         const int rpb = colsum_vec_rows_per_block(rows, blocks_x);
         const int groups = (int)((rows + rpb - 1) / rpb);
-        colsum_partial_vec<<<dim3((unsigned)blocks_x, (unsigned)groups), kBlock, 0, st>>>((const float*)x, partial, rows, cols, rpb);
+        const dim3 grid((unsigned)blocks_x, (unsigned)groups);
+        if (dtype == BR_F32)
+            colsum_partial_vec<float, 4><<<grid, kBlock, 0, st>>>((const float*)x, partial, rows, cols, rpb);
+        else if (dtype == BR_F16)
+            colsum_partial_vec<__half, 8><<<grid, kBlock, 0, st>>>((const __half*)x, partial, rows, cols, rpb);
+        else
+            colsum_partial_vec<__hip_bfloat16, 8><<<grid, kBlock, 0, st>>>((const __hip_bfloat16*)x, partial, rows, cols, rpb);
         BR_HIP_LAUNCH_CHECK();
         return colsum_finish(partial, out, groups, cols, out_scale, st);
     }

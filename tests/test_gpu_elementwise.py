@@ -142,9 +142,9 @@ def test_colsum(rows, cols):
                                              (77, 6144, "bf16"), (1, 6144, "f16"), (40, 1024, "f16")])
 def test_colsum_16_bit(rows, cols, dtype):
     """Column sums of 16-bit tensors (the bias gradient of a linear layer whose
-    output gradient is kept in 16 bits): shapes wide enough for the
-    single-launch form (a workgroup per 64 columns walking all rows; ragged
-    last block, rows that do not fill a pass) and one that takes two launches."""
+    output gradient is kept in 16 bits): single-launch shapes (workgroups that
+    own 16, 32 or 64 columns and walk all rows; ragged last block, rows that do
+    not fill a pass)."""
     from gpu_util import BF16
     rng = np.random.default_rng(61)
     t, code = (torch.float16, F16) if dtype == "f16" else (torch.bfloat16, BF16)
@@ -153,6 +153,26 @@ def test_colsum_16_bit(rows, cols, dtype):
     ws = workspace(hip.load().br_hip_colsum_workspace(rows, cols))
     call("br_hip_colsum", ptr(x), code, ptr(out), rows, cols, 0.5, ptr(ws), ws.numel(), stream())
     assert_close(host(out), 0.5 * x.float().cpu().numpy().astype(np.float64).sum(0), RTOL, "colsum " + dtype)
+
+
+@pytest.mark.parametrize("dtype,rows,cols,launches", [
+    (F16, 65536, 512, 2), (BF16, 4096, 6144, 2), (F16, 1025, 64, 2), (F16, 1024, 64, 1), (F16, 2048, 6152, 1),
+    (BF16, 2049, 6152, 2), (F16, 4099, 12296, 1), (F16, 128, 264, 1), (BF16, 129, 264, 1), (F16, 512, 4104, 1),
+    (F32, 512, 64, 1), (F32, 513, 64, 2), (F32, 1024, 3072, 1), (F32, 1024, 3068, 2), (F32, 1025, 4096, 2),
+    (F32, 128, 4100, 1), (F32, 129, 2052, 1), (F32, 700, 4100, 1)])
+def test_colsum_takes_one_launch_or_two(dtype, rows, cols, launches):
+    """Both sides of the lines between the one-launch form and the two-launch
+    one, which alone leaves partial sums in the workspace: tall narrow sums
+    need its workgroups along the rows."""
+    print("case dtype=%d rows=%d cols=%d" % (dtype, rows, cols), flush=True)
+    torch.manual_seed(5)
+    t = {F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16}[dtype]
+    x = torch.randn((rows, cols), device="cuda").to(t)
+    out = empty(cols)
+    ws = workspace(hip.load().br_hip_colsum_workspace(rows, cols)).fill_(0x7f)
+    call("br_hip_colsum", ptr(x), dtype, ptr(out), rows, cols, 0.5, ptr(ws), ws.numel(), stream())
+    assert_close(host(out), host(0.5 * x.double().sum(0)), RTOL, "colsum")
+    assert bool((ws != 0x7f).any()) == (launches == 2)
 
 
 @pytest.mark.parametrize("rows,cols", [(2048, 4096), (300, 1000), (5, 8), (1, 4), (512, 4096), (300, 3080), (1, 3072)])
