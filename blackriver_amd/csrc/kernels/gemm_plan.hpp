@@ -22,6 +22,7 @@
 namespace brk {
 namespace gemm16 {
 
+// in the order of the BR_GEMM_* constants
 enum Kernel { kTile256, kTile256x128, kTile256x128Groups, kTile128, kFlex64, kFlex64Short, kFlex32x64, kFlex32, kRing64x128, kKernels };
 
 struct KernelCost {

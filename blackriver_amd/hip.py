@@ -82,6 +82,7 @@ SIGNATURES = {
     "br_hip_gemm_staged_workspace": (ctypes.c_size_t, [_int, _int, _i64, _i64, _i64, _int, _int, _i64]),
     "br_hip_gemm_staged": (_int, [_int, _int, _i64, _i64, _i64, _f32, _vp, _int, _i64, _i64, _vp, _int, _i64, _i64,
                                   _int, _vp, _int, _i64, _i64, _vp, _i64, _int, _vp, ctypes.c_size_t, _vp]),
+    "br_hip_gemm_kernel": (_int, [_int, _int, _i64, _i64, _i64, _int, _i64, _int, ctypes.POINTER(_int)]),
     "br_hip_flash_attn_fwd": (_int, [_vp, _vp, _vp, _int, _vp, _vp, _vp, _vp] + [_i64] * 9 + [_vp]),
     "br_hip_flash_attn_bwd": (_int, [_vp] * 5 + [_int] + [_vp] * 7 + [_int] + [_i64] * 9 + [_vp]),
     "br_hip_adamw": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _i64, _f32, _f32, _f32, _f32, _f32, _i64, _vp]),
@@ -114,6 +115,18 @@ def load() -> ctypes.CDLL:
             fn.argtypes = args
         _lib = lib
     return _lib
+
+
+GEMM_KERNELS = ("256", "256x128", "256x128 groups", "128", "flex 64", "flex 64 short", "flex 32x64", "flex 32",
+                "ring 64x128")
+
+
+def gemm_kernel(trans_a, trans_b, m, n, k, c_dtype=F32, batch=1, staged=False):
+    """(kernel, slices of K) of a 16-bit product: see br_hip_gemm_kernel."""
+    slices = _int(0)
+    code = load().br_hip_gemm_kernel(trans_a, trans_b, m, n, k, c_dtype, batch, int(staged), ctypes.byref(slices))
+    check(min(code, 0), "br_hip_gemm_kernel")
+    return GEMM_KERNELS[code], slices.value
 
 
 def check(code: int, what: str = "") -> None:

@@ -349,6 +349,27 @@ int br_hip_gemm_staged(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k
                        const float* bias, int64_t batch, int compute,
                        void* workspace, size_t workspace_bytes, br_stream_t stream);
 
+/* The kernel a 16-bit product runs on, for callers (and tests) that want to
+ * know: of br_hip_gemm, or with `staged` of br_hip_gemm_staged and the workspace
+ * it asks for, for aligned operands of the compute type.  *slices receives the
+ * number of slices of K whose partial sums a second pass adds (1: none), or -2
+ * where two halves of K meet inside the kernel.  Some products run their last
+ * columns as a second launch on BR_GEMM_TILE_256X128_GROUPS.  Launches nothing;
+ * negative on invalid arguments. */
+enum {
+    BR_GEMM_TILE_256 = 0,              /* 256 x 256 tiles, direct-to-LDS */
+    BR_GEMM_TILE_256X128 = 1,
+    BR_GEMM_TILE_256X128_GROUPS = 2,   /* two groups of waves share every K step */
+    BR_GEMM_TILE_128 = 3,
+    BR_GEMM_FLEX_64 = 4,               /* small tiles, K dealt to the waves of a workgroup */
+    BR_GEMM_FLEX_64_SHORT = 5,
+    BR_GEMM_FLEX_32X64 = 6,
+    BR_GEMM_FLEX_32 = 7,
+    BR_GEMM_RING_64X128 = 8            /* loading waves beside multiplying ones */
+};
+int br_hip_gemm_kernel(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, int c_dtype, int64_t batch,
+                       int staged, int* slices);
+
 /* op_linear followed by op_gelu (cuda_tensor.cpp:146-193 and :400-412; the pair
  * of bloomz-7b/train.words:188-189) in one product whose epilogue writes both
  * tensors the backward pass needs, in the products' own 16-bit type:

@@ -34,3 +34,14 @@ def test_softmax_takes_addresses_of_any_alignment(call):
 @pytest.mark.parametrize("hidden", [65535 * 256 + 1, 65535 * 1024 + 4])
 def test_embedding_backward_takes_rows_of_any_length(hidden):
     assert answer("br_hip_embedding_scatter_add(4096, 8192, 16384, 2, %d, 4, 1.0, None)" % hidden) > 0
+
+
+def test_gemm_kernel_names_the_kernel_of_a_product():
+    from blackriver_amd import hip
+    assert hip.gemm_kernel(0, 1, 4096, 4096, 4096)[0] == "256"
+    assert hip.gemm_kernel(0, 1, 32, 32, 64) == ("flex 32", 1)
+    kernel, slices = hip.gemm_kernel(0, 1, 512, 4096, 16384, staged=True)
+    assert kernel in hip.GEMM_KERNELS and slices > 1
+    assert hip.gemm_kernel(0, 1, 512, 4096, 16384)[1] == 1   # nowhere to put partial sums
+    with pytest.raises(hip.BrHipError):
+        hip.gemm_kernel(0, 1, 0, 32, 64)
