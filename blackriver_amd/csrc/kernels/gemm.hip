@@ -202,17 +202,6 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma32_kernel(GemmArgs g) {
 
 long long elem_size(int dtype) { return dtype == BR_F32 ? 4 : 2; }
 
-// Whether the loads have to be checked against the end of K: K, or a slice of it, is no whole number of steps.
-bool is_ragged(long long k, int splits) { return k % 64 != 0 || splits > 1; }
-
-// The kernel a plan comes to for operands of these layouts and this type of C.
-int kernel_of(const gemm16::Plan& plan, const gemm16::Problem& p, long long m, long long n, long long k, long long batch, bool ragged) {
-    using namespace gemm16;
-    if (!ragged || is_flex(plan.kernel)) return plan.kernel;
-    if (!ragged_applies(p)) return flex_kernel(m, n, k, batch);
-    return plan.kernel == kTile256x128Groups ? kTile256x128 : plan.kernel;
-}
-
 // A 16-bit product by its plan, operands already checked by dtl_applies.  g.splits > 1: slices of K as batch entries.
 int run_plan(GemmArgs g, const gemm16::Problem& p, const gemm16::Plan& plan, long long batch, int compute, hipStream_t st) {
     using namespace gemm16;
@@ -236,8 +225,9 @@ int run_plan(GemmArgs g, const gemm16::Problem& p, const gemm16::Plan& plan, lon
         if (rc != BR_OK) return rc;
         return f16 ? gemm16_tiles_f16(tail, p, kTile256x128Groups, 1, st) : gemm16_tiles_bf16(tail, p, kTile256x128Groups, 1, st);
     }
-    const bool ragged = is_ragged(g.k, g.splits);
-    const int kernel = kernel_of(plan, p, g.m, g.n, g.k, batch, ragged);
+    // the loads have to be checked against the end of K: K, or a slice of it, is no whole number of steps
+    const bool ragged = g.k % 64 != 0 || g.splits > 1;
+    const int kernel = plan.kernel;
     if (ragged || is_flex(kernel))
         return f16 ? gemm16_ragged_f16(g, p, kernel, batch, st) : gemm16_ragged_bf16(g, p, kernel, batch, st);
     return f16 ? gemm16_tiles_f16(g, p, kernel, batch, st) : gemm16_tiles_bf16(g, p, kernel, batch, st);
@@ -334,15 +324,15 @@ extern "C" int br_hip_gemm(int trans_a, int trans_b, int64_t m, int64_t n, int64
 extern "C" int br_hip_gemm_kernel(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, int c_dtype, int64_t batch,
                                   int staged, int* slices) {
     using namespace gemm16;
+    // sizes alone decide
+    (void)trans_a;
+    (void)trans_b;
+    (void)c_dtype;
     if (m <= 0 || n <= 0 || k <= 0 || batch <= 0) return BR_ERR_ATTR;
     if (!slices) return BR_ERR_OUTPUT;
     const Plan plan = gemm_plan(m, n, k, batch, staged != 0);
-    Problem p{};
-    p.a_kstr = trans_a != 0;
-    p.b_kstr = trans_b == 0;
-    p.c_dtype = plan.slices > 1 ? BR_F32 : c_dtype;
     *slices = plan.pair ? -2 : plan.slices;
-    return kernel_of(plan, p, m, n, k, plan.slices > 1 ? plan.slices : batch, is_ragged(k, plan.slices));
+    return plan.kernel;
 }
 
 extern "C" int br_hip_linear_gelu(const void* x, const void* w, const float* bias, void* u, void* y, int dtype,

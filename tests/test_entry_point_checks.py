@@ -45,3 +45,10 @@ def test_gemm_kernel_names_the_kernel_of_a_product():
     assert hip.gemm_kernel(0, 1, 512, 4096, 16384)[1] == 1   # nowhere to put partial sums
     with pytest.raises(hip.BrHipError):
         hip.gemm_kernel(0, 1, 0, 32, 64)
+
+
+@pytest.mark.parametrize("m,n,k", [(4096, 4096, 1056), (8192, 2048, 1002), (16384, 4096, 96), (2048, 2048, 8160)])
+def test_ragged_products_run_on_large_tiles_in_every_layout(m, n, k):
+    from blackriver_amd import hip
+    kernels = {hip.gemm_kernel(ta, tb, m, n, k, c_dtype=c) for ta in (0, 1) for tb in (0, 1) for c in (hip.F32, hip.F16)}
+    assert len(kernels) == 1 and not {"flex", "ring"} & {name.split()[0] for name, _ in kernels}

@@ -436,6 +436,8 @@ def test_linear_gelu_epilogue_writes_both_tensors(dtype, rows, out, inn):
     (1000, 1032, 1000, 1),   # 64 x 64 tiles with ragged edges
     (1002, 4096, 1002, 1),   # large tiles with a ragged K
     (200, 512, 12345, 1),    # slices of a ragged K
+    (4000, 4104, 136, 1),    # large tiles in every layout, ragged in every direction
+    (8200, 2056, 1002, 1),
 ])
 def test_gemm_small_and_ragged_products_are_exact_on_integers(ta, tb, c_dt, m, n, k, batch):
     """The kernels for small and ragged sizes through the staged entry, on operands of small integers: every
