@@ -966,13 +966,14 @@ int launch_dtl_pair(GemmArgs g, const Problem& p, int kernel, int slot, hipStrea
     return launch_dtl_config<CT, 256, 128, 64, 64, 64, 3>(g, p, 1, st);
 }
 
-// K a multiple of 64, one workgroup per tile and batch entry.
+// K a multiple of 64 (kTile128Half: of 32), one workgroup per tile and batch entry.
 template <int CT>
 int launch_dtl(const GemmArgs& g, const Problem& p, int kernel, long long batch, hipStream_t st) {
     if (kernel == kTile256 && walk_applies(g, batch)) return launch_dtl_walk<CT>(g, p, st);
     if (kernel == kTile256) return launch_dtl_config<CT, 256, 256, 64, 128, 64, 2>(g, p, batch, st);
     if (kernel == kTile256x128Groups) return launch_dtl_config<CT, 256, 128, 64, 128, 64, 3, 2>(g, p, batch, st);
     if (kernel == kTile256x128) return launch_dtl_config<CT, 256, 128, 64, 64, 64, 3>(g, p, batch, st);
+    if (kernel == kTile128Half) return launch_dtl_config<CT, 128, 128, 64, 64, 32, 3>(g, p, batch, st);
     return launch_dtl_config<CT, 128, 128, 64, 64, 64, 2>(g, p, batch, st);
 }
 

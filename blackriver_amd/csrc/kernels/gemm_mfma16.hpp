@@ -331,9 +331,11 @@ __device__ __forceinline__ void tile_coords(const GemmArgs& g, long long& batch,
 // Workgroups that run side by side would otherwise all read the same 128-byte column of their operand rows at the
 // same time; with row pitches that are large powers of two those lines fall on a few memory channels and the
 // fetches queue behind one another (a [2048 x 4096] by [16384 x 4096] product, run back to back: 1105 TFLOP/s so,
-// 1175 with the starts spread; the other shapes of the BLOOM-7B1 block measure the same either way).  The start depends only on the 256 x 256 block of C the tile lies in and on K, so every kernel and
-// every tile shape in this library sums a given element of C in the same order and produces the same bits; the
-// spread is kept to seven neighbouring columns so that tiles sharing an operand panel still meet in L2.
+// 1175 with the starts spread; the other shapes of the BLOOM-7B1 block measure the same either way).  The start depends only on the 256 x 256 block of C the tile lies in and on K: the kernels that
+// give a wave all of its tile's K (the large tiles but for the two-group form, unsliced, and the register-staged kernel)
+// sum a given element of C in the same order and produce the same bits.  Kernels that deal K to waves or slices sum in
+// orders of their own, and which kernel runs follows from the sizes, so a row's bits may change with the number of rows
+// multiplied beside it; the same product always gives the same bits.  The spread is kept to seven neighbouring columns so that tiles sharing an operand panel still meet in L2.
 __device__ __forceinline__ long long k_walk_start(long long row0, long long col0, long long k) {
     const long long n64 = k >> 6;
     if (n64 < 2) return 0;

@@ -1,11 +1,19 @@
-// Which kernel a 16-bit product runs on, decided from its sizes alone: the
-// bits of a result do not depend on where its operands or workspace lie.
+// Which kernel a 16-bit product runs on, and whether K is cut into slices:
+// planned from its sizes alone.  Products of the same sizes, types, layouts and
+// alignment are summed in the same order at every call; operands that are not
+// 16-byte aligned take the register-staged kernel instead, a caller without a
+// workspace gets no slices, and a stream beyond the library's counter sets no
+// two-slice form (split_slot_of), each with an order of its own.
 //
 // Every kernel's time is estimated from constants fitted to measurements on
-// MI355X (fp16, 37 shapes from [64 x 256] to [50008 x 2048], each kernel
-// unsplit and with K in 2, 4 and 8 slices; the estimates are within 8-15 % of
-// the measured times, and choosing by them costs 1 % on average and 8 % at
-// worst over choosing by the measurements):
+// MI355X: fp16 operands read from memory, 668 sizes from [16 x 16] to
+// [16384 x 4096], K = 16 to 16384, in the layouts of a linear layer's three
+// products and of batched attention products, 871 products in all, each on
+// every kernel, unsplit and with K in up to 16 slices
+// (profiles/gemm_plan_measurements.txt).  Where a kernel is within a quarter of
+// the fastest the estimates are off by 5-10 % (median; 12-26 % for one in ten).
+// Choosing by them costs 1 % on average over choosing by the measurements, more
+// than 7 % for one product in twenty.
 //
 //   us = start + rounds * (steps * max(step, load * groups) + round) + C bytes / 6 TB/s
 //
@@ -23,7 +31,7 @@ namespace brk {
 namespace gemm16 {
 
 // in the order of the BR_GEMM_* constants
-enum Kernel { kTile256, kTile256x128, kTile256x128Groups, kTile128, kFlex64, kFlex64Short, kFlex32x64, kFlex32, kRing64x128, kKernels };
+enum Kernel { kTile256, kTile256x128, kTile256x128Groups, kTile128, kTile128Half, kFlex64, kFlex64Short, kFlex32x64, kFlex32, kRing64x128, kKernels };
 
 struct KernelCost {
     int bm, bn;
@@ -32,18 +40,16 @@ struct KernelCost {
     double start, step, load, round;
 };
 constexpr KernelCost kCost[kKernels] = {
-    {256, 256, 1, 256, 4.47, 1.310, 1.655, 0.00},    // gemm_dtl16.hpp, 8 waves of 64 x 128
-    {256, 128, 1, 256, 3.07, 0.840, 1.048, 0.89},    // 8 waves of 64 x 64
-    {256, 128, 1, 256, 3.09, 0.789, 0.993, 2.48},    // two groups of four 64 x 128 waves
-    {128, 128, 1, 512, 2.80, 0.737, 0.606, 0.00},    // 4 waves of 64 x 64
-    {64, 64, 4, 512, 2.71, 0.856, 0.900, 1.44},      // gemm_flex.hpp, K dealt to 4 waves
-    {64, 64, 2, 1024, 2.84, 0.745, 0.449, 1.99},     // ... to 2 waves, for many tiles or a short K
-    {32, 64, 4, 768, 2.95, 0.681, 0.637, 0.44},
-    {32, 32, 4, 512, 1.67, 0.472, 0.435, 1.15},
-    // gemm_flex.hpp, ring of K steps.  From timings inside whole steps, where weights come from memory: K = 512 (32
-    // products of [512 x 128]) 10-12 us against 8-10 on 64 x 64 tiles, K = 2048 20 against 22, K = 4096 35-39 against
-    // 40-50, K = 6144 51 against 49 and K = 8192 54-60 against 52-59 on 256 x 128 tiles with K in four slices.
-    {64, 128, 1, 256, 2.40, 0.380, 0.430, 2.20},
+    {256, 256, 1, 256, 4.63, 1.233, 1.724, 0.00},     // gemm_dtl16.hpp, 8 waves of 64 x 128
+    {256, 128, 1, 256, 2.23, 0.845, 1.052, 2.18},     // 8 waves of 64 x 64
+    {256, 128, 1, 256, 2.47, 0.753, 1.004, 3.44},     // two groups of four 64 x 128 waves
+    {128, 128, 1, 512, 4.30, 0.785, 0.545, 0.00},     // 4 waves of 64 x 64
+    {128, 128, 1, 512, 1.73, 0.864, 0.521, 0.00},     // the same with K steps of 32
+    {64, 64, 4, 512, 2.97, 1.088, 1.066, 1.67},       // gemm_flex.hpp, K dealt to 4 waves
+    {64, 64, 2, 1024, 1.12, 0.981, 0.459, 4.73},      // ... to 2 waves, for many tiles or a short K
+    {32, 64, 4, 768, 2.34, 0.697, 0.879, 0.79},
+    {32, 32, 4, 512, 0.65, 0.514, 0.663, 1.77},
+    {64, 128, 1, 256, 2.89, 0.284, 0.411, 3.70},      // ring of K steps
 };
 
 inline bool is_flex(int kernel) { return kernel >= kFlex64; }
@@ -73,7 +79,7 @@ inline double kernel_us(int kernel, long long m, long long n, long long k, long 
     return us > memory ? us : memory + 0.02 * us;   // between two that memory bounds, the one with less to do
 }
 // the pass that adds the partial sums of `slices` slices
-inline double reduce_us(long long m, long long n, int slices) { return 3.0 + (double)(slices + 1) * m * n * 4.0 / 5.5e6; }
+inline double reduce_us(long long m, long long n, int slices) { return 3.16 + (double)(slices + 1) * m * n * 4.0 / 8.00e6; }
 
 constexpr int kMaxSplitTiles = 8192;   // the two-slice form's arrival counters per stream
 // The two-slice form: one partial tile per output tile is written and read back through device-coherent accesses, by
@@ -109,25 +115,29 @@ inline long long column_tail(long long m, long long n, long long k, double best_
 
 // slices_allowed: the caller has a workspace for partial sums.
 inline Plan gemm_plan(long long m, long long n, long long k, long long batch, bool slices_allowed) {
-    Plan best;
+    Plan whole, split;   // the best without and with K in slices
     for (int c = 0; c < kKernels; c++) {
+        // steps of half the length are for a K they divide and whole steps do not ([2048 x 2048] from K = 2016 in
+        // 30-36 us, 35-42 with a bounds-checked last step); a K of one such step is left to the small tiles
+        if (c == kTile128Half && (k % 64 != 32 || k == 32)) continue;
         // two groups of waves share a 64-wide K step: no ragged form
         if (c == kTile256x128Groups && k % 64 != 0) continue;
-        for (int s = 1; s <= 16; s *= 2) {
-            if (s > 1 && (!slices_allowed || batch != 1 || n % 4 != 0 || k / s < 256)) break;
+        const double us = kernel_us(c, m, n, k, batch);
+        if (us < whole.us) whole = Plan{c, 1, false, 0, us};
+        if (!slices_allowed || batch != 1) continue;
+        for (int s = 2; s <= 16 && k / s >= 256 && n % 4 == 0 && c != kTile128Half; s *= 2) {
             const long long per = slice_length(k, s);
             const int slices = (int)ceil_div(k, per);
-            if (s > 1 && (slices < 2 || c == kTile256x128Groups)) break;
-            const double us = s == 1 ? kernel_us(c, m, n, k, batch) : kernel_us(c, m, n, per, slices) + reduce_us(m, n, slices);
-            // a split has to win clearly: it takes a second launch
-            if (us < (s == 1 ? 1.0 : 0.97) * best.us) best = Plan{c, slices, false, 0, us};
+            if (slices < 2 || (c == kTile256x128Groups && per * s != k)) break;
+            const double t = kernel_us(c, m, n, per, slices) + reduce_us(m, n, slices);
+            if (t < split.us) split = Plan{c, slices, false, 0, t};
         }
+        if (c > kTile256x128) continue;
+        const double t = pair_us(c, m, n, k);
+        if (t < split.us) split = Plan{c, 1, true, 0, t};
     }
-    if (slices_allowed && batch == 1)
-        for (int c = kTile256; c <= kTile256x128; c++) {
-            const double us = pair_us(c, m, n, k);
-            if (us < 0.97 * best.us) best = Plan{c, 1, true, 0, us};
-        }
+    // slices have to win clearly over none: they take a second launch or an exchange of partial tiles
+    Plan best = split.us < 0.97 * whole.us ? split : whole;
     const long long tail = batch == 1 ? column_tail(m, n, k, best.us) : 0;
     if (tail > 0) best = Plan{kTile256, 1, false, tail, best.us};
     return best;

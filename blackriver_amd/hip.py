@@ -117,8 +117,8 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
-GEMM_KERNELS = ("256", "256x128", "256x128 groups", "128", "flex 64", "flex 64 short", "flex 32x64", "flex 32",
-                "ring 64x128")
+GEMM_KERNELS = ("256", "256x128", "256x128 groups", "128", "128 half", "flex 64", "flex 64 short",
+                "flex 32x64", "flex 32", "ring 64x128")
 
 
 def gemm_kernel(trans_a, trans_b, m, n, k, c_dtype=F32, batch=1, staged=False):

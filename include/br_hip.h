@@ -361,11 +361,12 @@ enum {
     BR_GEMM_TILE_256X128 = 1,
     BR_GEMM_TILE_256X128_GROUPS = 2,   /* two groups of waves share every K step */
     BR_GEMM_TILE_128 = 3,
-    BR_GEMM_FLEX_64 = 4,               /* small tiles, K dealt to the waves of a workgroup */
-    BR_GEMM_FLEX_64_SHORT = 5,
-    BR_GEMM_FLEX_32X64 = 6,
-    BR_GEMM_FLEX_32 = 7,
-    BR_GEMM_RING_64X128 = 8            /* loading waves beside multiplying ones */
+    BR_GEMM_TILE_128_HALF = 4,         /* the same with K steps of 32 */
+    BR_GEMM_FLEX_64 = 5,               /* small tiles, K dealt to the waves of a workgroup */
+    BR_GEMM_FLEX_64_SHORT = 6,
+    BR_GEMM_FLEX_32X64 = 7,
+    BR_GEMM_FLEX_32 = 8,
+    BR_GEMM_RING_64X128 = 9            /* loading waves beside multiplying ones */
 };
 int br_hip_gemm_kernel(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, int c_dtype, int64_t batch,
                        int staged, int* slices);

@@ -12,6 +12,25 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
+# (kernel, slices, m, n, k, batch): products of the staged entry that reach every kernel in each of its forms -- whole
+# and partial tiles, K of whole and of partial steps, slices of one length and not
+PLANNED = [
+    ("256", 1, 2048, 8192, 64, 1), ("256", 1, 4000, 4096, 64, 1), ("256", 1, 4000, 4096, 72, 1),
+    ("256", 1, 1024, 1024, 256, 16), ("256", 4, 520, 4096, 8192, 1), ("256", 4, 4000, 520, 8200, 1),
+    ("256x128", 1, 1000, 8192, 256, 1), ("256x128", 1, 1000, 8192, 136, 1), ("256x128", 8, 488, 2048, 8192, 1),
+    ("256x128", 15, 488, 1000, 8200, 1), ("256x128", -2, 1024, 4096, 2048, 1), ("256x128", -2, 4000, 1000, 2048, 1),
+    ("256x128 groups", 1, 1000, 2056, 4160, 2), ("256x128 groups", 4, 488, 4096, 8192, 1),
+    ("128", 1, 2048, 520, 64, 1), ("128", 1, 488, 4096, 72, 1), ("128", 1, 488, 520, 192, 16),
+    ("128", 16, 488, 520, 8192, 1), ("128", 8, 1000, 520, 4104, 1),
+    ("128 half", 1, 488, 1000, 96, 1), ("128 half", 1, 2048, 2048, 2016, 1),
+    ("flex 64", 1, 488, 4096, 256, 1), ("flex 64", 1, 488, 4096, 200, 1), ("flex 64", 4, 488, 512, 8192, 1),
+    ("flex 64", 4, 488, 512, 8200, 1), ("flex 64 short", 1, 488, 4104, 2048, 1), ("flex 64 short", 1, 488, 4104, 520, 1),
+    ("flex 32x64", 1, 488, 2048, 64, 1), ("flex 32x64", 1, 488, 2048, 72, 1), ("flex 32", 1, 488, 512, 72, 1),
+    ("flex 32", 4, 64, 1024, 4096, 1), ("ring 64x128", 1, 488, 4096, 2048, 1), ("ring 64x128", 1, 488, 4096, 520, 1),
+    ("ring 64x128", 4, 64, 4096, 8200, 1),
+]
+
+
 def answer(call):
     """Return code of `L.<call>`, made without a GPU."""
     env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES="-1")
@@ -40,8 +59,7 @@ def test_gemm_kernel_names_the_kernel_of_a_product():
     from blackriver_amd import hip
     assert hip.gemm_kernel(0, 1, 4096, 4096, 4096)[0] == "256"
     assert hip.gemm_kernel(0, 1, 32, 32, 64) == ("flex 32", 1)
-    kernel, slices = hip.gemm_kernel(0, 1, 512, 4096, 16384, staged=True)
-    assert kernel in hip.GEMM_KERNELS and slices > 1
+    assert hip.gemm_kernel(0, 1, 512, 4096, 16384, staged=True)[1] > 1
     assert hip.gemm_kernel(0, 1, 512, 4096, 16384)[1] == 1   # nowhere to put partial sums
     with pytest.raises(hip.BrHipError):
         hip.gemm_kernel(0, 1, 0, 32, 64)
@@ -52,3 +70,10 @@ def test_ragged_products_run_on_large_tiles_in_every_layout(m, n, k):
     from blackriver_amd import hip
     kernels = {hip.gemm_kernel(ta, tb, m, n, k, c_dtype=c) for ta in (0, 1) for tb in (0, 1) for c in (hip.F32, hip.F16)}
     assert len(kernels) == 1 and not {"flex", "ring"} & {name.split()[0] for name, _ in kernels}
+
+
+@pytest.mark.parametrize("kernel,slices,m,n,k,batch", PLANNED)
+def test_gemm_plan_reaches_every_kernel(kernel, slices, m, n, k, batch):
+    from blackriver_amd import hip
+    assert hip.gemm_kernel(0, 1, m, n, k, batch=batch, staged=True) == (kernel, slices)
+    assert {kernel for kernel, *_ in PLANNED} == set(hip.GEMM_KERNELS)

@@ -11,6 +11,7 @@ import torch
 from conftest import assert_close
 from gpu_util import BF16, F16, F32, call, dev, empty, host, ptr, stream
 from blackriver_amd import hip
+from test_entry_point_checks import PLANNED
 
 pytestmark = pytest.mark.gpu
 
@@ -135,18 +136,19 @@ def test_gemm_fp32_kernel_is_fp32_faithful_at_block_sizes():
     assert_close(got, ref, 1e-5, "fp32 gemm, k=4096")
 
 
-# Shapes that make the dispatcher pick each direct-to-LDS tile configuration
-# (256x256, 256x128, 128x128 with 64-wide K steps; 128x128 with 32-wide steps
-# when K % 64 != 0), with rows / columns that do not fill the last tile.
+# Products of the plain entry that run on each direct-to-LDS tile (256x256, 256x128, 128x128 with K steps of 64 and of
+# 32), with rows / columns that do not fill the last tile, several batch entries and a single K step.  The kernel is
+# asserted: which sizes go where follows from a table of fitted costs.
 DTL_SHAPES = [
-    ("256x256", 512, 512, 128, 64),
-    ("256x256 ragged", 488, 520, 192, 64),
-    ("256x128", 256, 128, 512, 1),
-    ("256x128 ragged", 1000, 1048, 256, 1),
-    ("128x128", 128, 51200, 64, 1),
-    ("128x128 k32", 264, 392, 96, 3),
-    ("one k step", 256, 256, 64, 1),
-    ("one k step k32", 256, 256, 32, 1),
+    ("256", 1024, 1024, 128, 16),
+    ("256", 1000, 1024, 192, 16),
+    ("256x128", 1024, 1024, 256, 8),
+    ("256x128", 1000, 8192, 256, 1),
+    ("128", 128, 51200, 64, 1),
+    ("128", 488, 520, 192, 16),
+    ("128 half", 264, 392, 96, 24),
+    ("256", 2048, 4096, 64, 2),
+    ("128", 2048, 2056, 64, 1),
 ]
 
 
@@ -155,6 +157,7 @@ DTL_SHAPES = [
 def test_gemm_direct_to_lds_kernel(ta, tb, name, m, n, k, batch):
     rng = np.random.default_rng(5)
     print("case %s ta=%d tb=%d m=%d n=%d k=%d batch=%d" % (name, ta, tb, m, n, k, batch), flush=True)
+    assert hip.gemm_kernel(ta, tb, m, n, k, batch=batch) == (name, 1)
     a, b = operands(rng, ta, tb, m, n, k, batch)
     got, ref = run_gemm(ta, tb, m, n, k, a, b, F16, F16, F32, hip.GEMM_F16, batch=batch)
     assert_close(got, ref, 2e-2, "dtl gemm " + name)
@@ -200,7 +203,7 @@ def test_gemm_direct_to_lds_at_linear_layer_shape():
     (2048, 8192, 192, F32),     # 256 tiles: one per workgroup, three K steps
     (2048, 16384, 128, F16),    # 512 tiles: two per workgroup, 16-bit C
     (3072, 16384, 64, F32),     # 768 tiles of a single K step
-    (2816, 6144, 320, F32),     # 264 tiles: 33 per XCD for 32 workgroups, one of them walks twice
+    (2816, 10240, 192, F32),    # 440 tiles: 55 per XCD for 32 workgroups, 23 of them walk twice
 ])
 def test_gemm_workgroups_that_walk_the_tiles(ta, tb, m, n, k, c_dt):
     """Plain products (no bias, nothing accumulated) of 256 or more interior
@@ -211,6 +214,7 @@ def test_gemm_workgroups_that_walk_the_tiles(ta, tb, m, n, k, c_dt):
     rng = np.random.default_rng(31)
     print("case ta=%d tb=%d m=%d n=%d k=%d c_dt=%d" % (ta, tb, m, n, k, c_dt), flush=True)
     a, b = operands(rng, ta, tb, m, n, k)
+    assert hip.gemm_kernel(ta, tb, m, n, k, c_dt) == ("256", 1)
     got, ref = run_gemm(ta, tb, m, n, k, a, b, F16, F16, c_dt, hip.GEMM_F16, alpha=0.5)
     assert_close(got, ref, 2e-2, "walking workgroups")
     per_tile, _ = run_gemm(ta, tb, m, n, k, a, b, F16, F16, c_dt, hip.GEMM_F16, alpha=0.5, bias=np.zeros(n, np.float32))
@@ -271,6 +275,7 @@ def test_gemm_tile_on_two_groups_of_waves(ta, tb, c_dt):
     bit."""
     rng = np.random.default_rng(33)
     m, n, k = 1024, 8192, 2048
+    assert hip.gemm_kernel(ta, tb, m, n, k) == ("256x128 groups", 1)
     print("case ta=%d tb=%d c_dt=%d" % (ta, tb, c_dt), flush=True)
     a, b = operands(rng, ta, tb, m, n, k)
     bias = rng.standard_normal(n).astype(np.float32)
@@ -434,9 +439,9 @@ def test_linear_gelu_epilogue_writes_both_tensors(dtype, rows, out, inn):
     (250, 64, 250, 3),       # attention products of 250 tokens: rows that are not 16-byte aligned
     (31, 65, 7, 2),          # everything odd
     (1000, 1032, 1000, 1),   # 64 x 64 tiles with ragged edges
-    (1002, 4096, 1002, 1),   # large tiles with a ragged K
+    (1002, 4096, 1002, 1),   # 128 x 128 tiles with a ragged K
     (200, 512, 12345, 1),    # slices of a ragged K
-    (4000, 4104, 136, 1),    # large tiles in every layout, ragged in every direction
+    (4000, 4104, 136, 1),    # the same, ragged in every direction
     (8200, 2056, 1002, 1),
 ])
 def test_gemm_small_and_ragged_products_are_exact_on_integers(ta, tb, c_dt, m, n, k, batch):
@@ -461,6 +466,29 @@ def test_gemm_small_and_ragged_products_are_exact_on_integers(ta, tb, c_dt, m, n
     if c_dt == F16:
         ref = ref.astype(np.float16).astype(np.float64)
     assert np.array_equal(to_host64(c).reshape(batch, m, n), ref)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("kernel,slices,m,n,k,batch", PLANNED)
+def test_gemm_every_kernel_is_exact_on_integers(ta, tb, kernel, slices, m, n, k, batch):
+    """Every kernel the plan knows, in each of its forms, with both 16-bit types and both types of C: bias and an old C
+    added, the workspace full of NaNs.  Small integers: every partial sum is exact in fp32."""
+    assert hip.gemm_kernel(ta, tb, m, n, k, batch=batch, staged=True) == (kernel, slices)
+    torch.manual_seed(m + n + k)
+    a = torch.randint(-3, 4, (batch, k, m) if ta else (batch, m, k), device="cuda").float()
+    b = torch.randint(-2, 3, (batch, n, k) if tb else (batch, k, n), device="cuda").float()
+    bias = torch.randint(-5, 6, (n,), device="cuda").float()
+    c0 = torch.randint(-9, 10, (batch, m, n), device="cuda").float()
+    want = torch.stack([(x.t() if ta else x) @ (y.t() if tb else y) for x, y in zip(a, b)]) + bias + c0
+    for t, dt, compute, c_dt in ((torch.float16, F16, hip.GEMM_F16, F32), (torch.bfloat16, BF16, hip.GEMM_BF16, BF16)):
+        print("case %s/%d ta=%d tb=%d m=%d n=%d k=%d c=%d" % (kernel, slices, ta, tb, m, n, k, c_dt), flush=True)
+        da, db_, c = a.to(t), b.to(t), c0.clone().to(TORCH_T[c_dt])
+        need = hip.load().br_hip_gemm_staged_workspace(ta, tb, m, n, k, dt, dt, batch)
+        ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda").fill_(255)
+        call("br_hip_gemm_staged", ta, tb, m, n, k, 1.0, ptr(da), dt, m if ta else k, m * k, ptr(db_), dt, k if tb else n,
+             n * k, 1, ptr(c), c_dt, n, m * n, ptr(bias), batch, compute, ptr(ws), need, stream())
+        torch.cuda.synchronize()
+        assert torch.equal(c, want.to(c.dtype))
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
@@ -490,18 +518,20 @@ def test_gemm_fp32_small_tiles_are_exact_on_integers(ta, tb, m, n, k, batch):
 @pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
 @pytest.mark.parametrize("c_dt", [F32, F16])
 @pytest.mark.parametrize("m,n,k,batch", [
-    (1024, 2048, 328, 1),    # whole tiles, exactly as many K steps as the ring holds, the last one ragged
+    (488, 4096, 520, 1),     # about as few K steps as the plan gives it, the last one ragged
     (960, 1800, 2056, 1),    # an odd number of steps, ragged columns
     (1002, 2040, 1096, 1),   # ragged in every direction
     (512, 1000, 1032, 4),    # batch entries
 ])
 def test_gemm_tiles_on_a_ring_of_k_steps_are_exact_on_integers(ta, tb, c_dt, m, n, k, batch):
     """64 x 128 tiles, one workgroup per CU: waves that load beside waves that multiply."""
+    assert hip.gemm_kernel(ta, tb, m, n, k, c_dt, batch, staged=True) == ("ring 64x128", 1)
     test_gemm_small_and_ragged_products_are_exact_on_integers(ta, tb, c_dt, m, n, k, batch)
 
 
 @pytest.mark.parametrize("dtype", [F16, BF16])
 def test_linear_gelu_epilogue_on_a_ring_of_k_steps(dtype):
+    assert hip.gemm_kernel(0, 1, 1024, 2048, 2048) == ("ring 64x128", 1)
     test_linear_gelu_epilogue_writes_both_tensors(dtype, 1024, 2048, 2048)
 
 
