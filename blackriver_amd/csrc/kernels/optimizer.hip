@@ -113,6 +113,19 @@ __device__ __forceinline__ void adamw_granule(const Tensor& t, int64_t at, const
     }
 }
 
+// A launch of one tensor needs no search and no table in its arguments, and its type and width are compiled in: with
+// the general kernel below a tensor of 16 million values, fp16 with an fp32 master copy, took 90.9 us instead of 86.7,
+// and one of a million odd fp32 values 8.6 instead of 7.3.
+struct Single {
+    AdamW a;
+    Tensor t;
+};
+template <typename T, int VEC>
+__global__ __launch_bounds__(kBlock) void adamw_single_kernel(Single g) {
+    g.t.vec = VEC == 4;
+    adamw_granule<T>(g.t, (int64_t)blockIdx.x * kBlock + threadIdx.x, g.a);
+}
+
 // Which tensor is found by counting: 32 scalar compares against kernel arguments, no dependent loads.
 __global__ __launch_bounds__(kBlock) void adamw_kernel(Group g) {
     int which = 0;
@@ -187,6 +200,22 @@ int br_hip_adamw_group(const br_adamw_tensor* tensors, int64_t count, float lr, 
     int used = 0;
     int64_t blocks = 0;
     auto launch = [&]() {
+        if (used == 1) {
+            const Single one{g.a, g.t[0]};
+            const hipStream_t st = as_stream(stream);
+            const unsigned grid = (unsigned)blocks;
+#define BR_ADAMW_SINGLE(T)                                                            \
+    if (one.t.vec) adamw_single_kernel<T, 4><<<grid, kBlock, 0, st>>>(one);           \
+    else adamw_single_kernel<T, 1><<<grid, kBlock, 0, st>>>(one)
+            if (one.t.dtype == BR_F32) { BR_ADAMW_SINGLE(float); }
+            else if (one.t.dtype == BR_F16) { BR_ADAMW_SINGLE(__half); }
+            else { BR_ADAMW_SINGLE(__hip_bfloat16); }
+#undef BR_ADAMW_SINGLE
+            used = 0;
+            blocks = 0;
+            BR_HIP_LAUNCH_CHECK();
+            return (int)BR_OK;
+        }
         for (int k = used; k < kTensors; k++) g.first[k] = 0xffffffffu;
         adamw_kernel<<<(unsigned)blocks, kBlock, 0, as_stream(stream)>>>(g);
         used = 0;
