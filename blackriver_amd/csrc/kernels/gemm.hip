@@ -8,9 +8,10 @@
 // and gemm_mfma16.hpp (fp32 operands converted on load, unaligned rows).  This
 // file holds the argument checking, the staging of fp32 and of unaligned
 // operands into a caller's workspace so that they too can take the
-// direct-to-LDS kernels, and a kernel for fp32 products whose leading dimensions
-// are too long for the 32-bit offsets of the one in gemm_flex.hpp (128x128x16
-// tiles, 4 wave64s x 2x2 MFMA blocks, register prefetch + LDS double buffering).
+// direct-to-LDS kernels, and a kernel for fp32 products of many whole tiles from a
+// short K, and for those whose leading dimensions are too long for the 32-bit
+// offsets of the one in gemm_flex.hpp (128x128x16 tiles, 4 wave64s x 2x2 MFMA
+// blocks, register prefetch + LDS double buffering).
 #include "common.hpp"
 
 #include <hip/hip_bf16.h>
@@ -286,9 +287,10 @@ int gemm_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float a
     if (compute == BR_GEMM_F32) {
         // the small-tile kernel's per-lane offsets span 64 rows in 32 bits
         const long long lim = 1LL << 31;
-        if (256 * lda < lim && 256 * ldb < lim && m < lim && n < lim && k < lim && k > 0) {
+        const int kernel = gemm16::fp32_kernel(m, n, k, batch);
+        if (kernel != gemm16::kTile128 && 256 * lda < lim && 256 * ldb < lim && m < lim && n < lim && k < lim && k > 0) {
             const bool words = !g.vec_a || !g.vec_b || (k % 4 != 0 && !(ak && bk));
-            return gemm_fp32(g, p, gemm16::fp32_kernel(m, n, k, batch), words, batch, st);
+            return gemm_fp32(g, p, kernel, words, batch, st);
         }
         if (ak && bk) gemm_mfma32_kernel<true, true><<<(unsigned)blocks, kThreads, 0, st>>>(g);
         else if (ak) gemm_mfma32_kernel<true, false><<<(unsigned)blocks, kThreads, 0, st>>>(g);

@@ -156,6 +156,13 @@ inline int fp32_kernel(long long m, long long n, long long k, long long batch) {
     double t = us(kFlex64, 2.45);
     if (us(kFlex32x64, 1.4) < 0.98 * t) best = kFlex32x64, t = us(kFlex32x64, 1.4);
     if (us(kFlex32, 0.78) < 0.98 * t) best = kFlex32;
+    // kTile128: 128 x 128 tiles of four waves (gemm.hip), three to a CU.  A short K gives a wave of the small tiles one
+    // step and an accumulator to merge; many whole tiles then go faster by rounds of these: [512 x 512] K = 128, 128
+    // products 126 us against 142 (1024 tiles, a round and a third, 80 against 67; 512 tiles 37 against 41).
+    const long long tiles = m / 128 * (n / 128) * batch;
+    if (k > 64 && k <= 128 && m % 128 == 0 && n % 128 == 0 && tiles >= 512 &&
+        38.0 * (double)ceil_div(tiles, 768) * (double)k / 128.0 < 5.0 + 0.067 * (double)tiles)
+        return kTile128;
     return best;
 }
 

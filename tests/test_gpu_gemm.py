@@ -501,6 +501,8 @@ def test_gemm_every_kernel_is_exact_on_integers(ta, tb, kernel, slices, m, n, k,
     (31, 65, 7, 2),          # value by value: everything odd
     (333, 64, 333, 3),       # attention products of 333 tokens
     (1001, 2050, 70, 2),     # 64 x 64 tiles, value by value
+    (128, 128, 128, 512),    # 128 x 128 tiles: a short K and 512 whole tiles
+    (256, 384, 68, 90),
 ])
 def test_gemm_fp32_small_tiles_are_exact_on_integers(ta, tb, m, n, k, batch):
     """The fp32 kernel's tiles and both ways it loads its operands, on small integers: every partial sum is exact."""
@@ -513,6 +515,37 @@ def test_gemm_fp32_small_tiles_are_exact_on_integers(ta, tb, m, n, k, batch):
     c0 = rng.integers(-9, 10, (batch, m, n)).astype(np.float32)
     got, ref = run_gemm(ta, tb, m, n, k, a, b, F32, F32, F32, hip.GEMM_F32, batch=batch, bias=bias, c0=c0)
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("wide", ["a", "b"])
+@pytest.mark.parametrize("ta,tb", [(0, 1), (1, 0)])
+def test_gemm_fp32_rows_far_apart(ta, tb, wide):
+    """Rows of an fp32 operand 2^23 elements apart: past the 32-bit offsets of the small-tile kernel, on 128 x 128
+    tiles.  Ragged sizes, small integers: exact."""
+    m, n, k, ld = 130, 70, 36, 1 << 23
+    print("case wide=%s ta=%d tb=%d" % (wide, ta, tb), flush=True)
+    rng = np.random.default_rng(9)
+    a = torch.from_numpy(rng.integers(-3, 4, (k, m) if ta else (m, k)).astype(np.float32)).cuda()
+    b = torch.from_numpy(rng.integers(-2, 3, (n, k) if tb else (k, n)).astype(np.float32)).cuda()
+    bias = torch.from_numpy(rng.integers(-5, 6, n).astype(np.float32)).cuda()
+    want = (a.t() if ta else a) @ (b.t() if tb else b) + bias
+    narrow = a if wide == "a" else b
+    spread = torch.empty((narrow.shape[0], ld), device="cuda")
+    spread[:, :narrow.shape[1]] = narrow
+    pa, pb = (spread, b) if wide == "a" else (a, spread)
+    c = torch.full((m, n), float("nan"), device="cuda")
+    call("br_hip_gemm", ta, tb, m, n, k, 1.0, ptr(pa), F32, pa.shape[1], 0, ptr(pb), F32, pb.shape[1], 0, 0, ptr(c), F32, n,
+         0, ptr(bias), 1, hip.GEMM_F32, stream())
+    torch.cuda.synchronize()
+    assert torch.equal(c, want)
+
+
+def test_gemm_fp32_without_k_leaves_the_bias():
+    bias, a = dev(np.arange(7, dtype=np.float32)), empty((5, 8))
+    c = torch.full((5, 7), float("nan"), device="cuda")
+    call("br_hip_gemm", 0, 1, 5, 7, 0, 1.0, ptr(a), F32, 8, 0, ptr(a), F32, 8, 0, 0, ptr(c), F32, 7, 0, ptr(bias), 1,
+         hip.GEMM_F32, stream())
+    assert np.array_equal(host(c), np.tile(np.arange(7, dtype=np.float32), (5, 1)))
 
 
 @pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
