@@ -203,25 +203,47 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma32_kernel(GemmArgs g) {
 
 long long elem_size(int dtype) { return dtype == BR_F32 ? 4 : 2; }
 
+// The product of `rows` x `cols` elements of C from (row, col) on; multiples of 8, so that operands stay aligned.
+GemmArgs part_of(GemmArgs g, const gemm16::Problem& p, long long row, long long col, long long rows, long long cols) {
+    const long long at = elem_size(p.c_dtype) * (row * g.ldc + col);
+    g.m = rows;
+    g.n = cols;
+    g.a = static_cast<const unsigned char*>(g.a) + 2 * (p.a_kstr ? row : row * g.lda);
+    g.b = static_cast<const unsigned char*>(g.b) + 2 * (p.b_kstr ? col : col * g.ldb);
+    g.c = static_cast<unsigned char*>(g.c) + at;
+    if (g.c2) g.c2 = static_cast<unsigned char*>(g.c2) + at;
+    if (g.addend) g.addend = static_cast<const unsigned char*>(g.addend) + at;
+    if (g.bias) g.bias += col;
+    return g;
+}
+
 // A 16-bit product by its plan, operands already checked by dtl_applies.  g.splits > 1: slices of K as batch entries.
 int run_plan(GemmArgs g, const gemm16::Problem& p, const gemm16::Plan& plan, long long batch, int compute, hipStream_t st) {
     using namespace gemm16;
     const bool f16 = compute == BR_GEMM_F16;
+    const KernelCost& tile = kCost[plan.kernel];
+    if (!is_flex(plan.kernel) && g.ldc >= kEdgeColumns && (g.m % tile.bm != 0 || g.n % tile.bn != 0)) {
+        // Partial large tiles of a C this wide are beyond their epilogue's offsets: whole tiles as planned, the columns
+        // and the rows that are left on small tiles, which address C in 64 bits.
+        const long long m_in = g.m / tile.bm * tile.bm, n_in = g.n / tile.bn * tile.bn;
+        const Plan small{flex_kernel(g.m, g.n - n_in > 0 ? g.n - n_in : g.n, g.k, batch)};
+        Plan whole = plan;
+        whole.pair = false;
+        whole.tail_from = 0;
+        int rc = BR_OK;
+        if (m_in > 0 && n_in > 0) rc = run_plan(part_of(g, p, 0, 0, m_in, n_in), p, whole, batch, compute, st);
+        if (rc == BR_OK && n_in < g.n) rc = run_plan(part_of(g, p, 0, n_in, g.m, g.n - n_in), p, small, batch, compute, st);
+        if (rc == BR_OK && m_in < g.m && n_in > 0) rc = run_plan(part_of(g, p, m_in, 0, g.m - m_in, n_in), p, small, batch, compute, st);
+        return rc;
+    }
     if (plan.pair && g.partials) {
         const int slot = split_slot_of(st);
         if (slot >= 0) return f16 ? gemm16_pair_f16(g, p, plan.kernel, slot, st) : gemm16_pair_bf16(g, p, plan.kernel, slot, st);
     }
     if (plan.tail_from > 0) {
         // whole rounds of 256x256 tiles, then the columns left over on 256x128 tiles (see column_tail)
-        GemmArgs head = g, tail = g;
-        head.n = plan.tail_from;
-        const size_t c_size = (size_t)elem_size(p.c_dtype);
-        tail.n = g.n - plan.tail_from;
-        tail.b = static_cast<const unsigned char*>(g.b) + 2 * (p.b_kstr ? plan.tail_from : plan.tail_from * g.ldb);
-        tail.c = static_cast<unsigned char*>(g.c) + c_size * plan.tail_from;
-        if (g.c2) tail.c2 = static_cast<unsigned char*>(g.c2) + c_size * plan.tail_from;
-        if (g.addend) tail.addend = static_cast<const unsigned char*>(g.addend) + c_size * plan.tail_from;
-        if (g.bias) tail.bias = g.bias + plan.tail_from;
+        const GemmArgs head = part_of(g, p, 0, 0, g.m, plan.tail_from);
+        const GemmArgs tail = part_of(g, p, 0, plan.tail_from, g.m, g.n - plan.tail_from);
         const int rc = f16 ? gemm16_tiles_f16(head, p, kTile256, 1, st) : gemm16_tiles_bf16(head, p, kTile256, 1, st);
         if (rc != BR_OK) return rc;
         return f16 ? gemm16_tiles_f16(tail, p, kTile256x128Groups, 1, st) : gemm16_tiles_bf16(tail, p, kTile256x128Groups, 1, st);

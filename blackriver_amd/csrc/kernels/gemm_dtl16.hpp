@@ -586,7 +586,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64) void gemm_dtl_kern
         bias[j] = g.bias && col < g.n ? g.bias[col] : 0.f;
         lane_at[j] = col < g.n ? (unsigned)(((lane >> 5) * 4 * g.ldc + j * 32 + (lane & 31)) * (long long)sizeof(TC)) : kPastEnd;
     }
-    // a row offset added to kPastEnd stays past the end: the tile spans less than 2^31 bytes (dtl_applies)
+    // a row offset added to kPastEnd stays past the end: the tile spans less than 2^31 bytes (kEdgeColumns)
     auto at = [&](int blk, int v) {
         return lane_at[blk % FN] + (unsigned)((blk / FN * 32 + (v >> 2) * 8 + (v & 3)) * (int)g.ldc * (int)sizeof(TC));
     };
@@ -924,12 +924,14 @@ int launch_dtl_ragged(GemmArgs g, const Problem& p, long long batch, hipStream_t
 
 // The direct-to-LDS kernels apply when both operands are 16-bit and 16-byte aligned, a k-contiguous operand's rows
 // end on a 16-byte granule of their own (K a multiple of 8, or zero-filled up to one), and every per-lane offset fits
-// 32 bits (of the operands, and of a tile of C, which spans up to 256 rows).
+// 32 bits: of the operands, and of the four rows of C a lane of a whole tile spans.  The edge epilogue's offsets span up
+// to 256 rows: partial tiles of a C of kEdgeColumns or more columns are left to other kernels (run_plan in gemm.hip).
+constexpr long long kEdgeColumns = 1LL << 21;
 inline bool dtl_spans(bool a_kstr, long long lda, bool b_kstr, long long ldb, long long ldc, long long m, long long n, long long k) {
     const long long lim = 1LL << 31;
     const long long a_span = a_kstr ? 2 * 64 * lda : 2 * 256 * lda;
     const long long b_span = b_kstr ? 2 * 64 * ldb : 2 * 256 * ldb;
-    return a_span < lim && b_span < lim && ldc < (1LL << 21) && m < lim && n < lim && k < lim;
+    return a_span < lim && b_span < lim && ldc < (1LL << 27) && m < lim && n < lim && k < lim;
 }
 inline bool dtl_applies(const GemmArgs& g, const Problem& p) {
     if (p.a_f32 || p.b_f32 || !g.vec_a || !g.vec_b || g.k <= 0) return false;

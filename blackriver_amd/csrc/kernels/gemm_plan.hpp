@@ -143,6 +143,14 @@ inline Plan gemm_plan(long long m, long long n, long long k, long long batch, bo
     return best;
 }
 
+// The fastest of the kernels that address C in 64 bits.
+inline int flex_kernel(long long m, long long n, long long k, long long batch) {
+    int best = kFlex64;
+    for (int c = kFlex64; c < kKernels; c++)
+        if (kernel_us(c, m, n, k, batch) < kernel_us(best, m, n, k, batch)) best = c;
+    return best;
+}
+
 // fp32 products (gemm_flex.hpp): the tile whose matrix instructions finish first.  A step of 32 k-values takes a wave
 // 64 / 32 / 16 instructions of 64 clocks; measured with everything around them 2.45 / 1.4 / 0.78 us per step and
 // workgroup of a CU, and 2.7 us besides.  A CU that holds one workgroup more than the others sets the time.

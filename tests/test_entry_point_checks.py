@@ -77,3 +77,8 @@ def test_gemm_plan_reaches_every_kernel(kernel, slices, m, n, k, batch):
     from blackriver_amd import hip
     assert hip.gemm_kernel(0, 1, m, n, k, batch=batch, staged=True) == (kernel, slices)
     assert {kernel for kernel, *_ in PLANNED} == set(hip.GEMM_KERNELS)
+
+
+@pytest.mark.parametrize("out", [(1 << 21) - 8, 1 << 21, (1 << 21) + 8, (1 << 26)])
+def test_linear_gelu_takes_wide_outputs(out):
+    assert answer("br_hip_linear_gelu(4096, 8192, None, 1 << 40, 1 << 41, 2, 300, %d, 32, None)" % out) > 0

@@ -588,3 +588,46 @@ def test_gemm_staged_rows_too_far_apart_for_slices(a_wide):
          1, hip.GEMM_F16, ptr(ws), need, stream())
     assert need > 0   # sliced by its sizes
     assert np.array_equal(to_host64(c), a.astype(np.float64) @ b.astype(np.float64).T)
+
+
+@pytest.mark.parametrize("c_dt", [F32, F16])
+@pytest.mark.parametrize("kernel,m,n,k", [("256", 4000, 4096, 72), ("256x128 groups", 1000, 4104, 4160), ("128", 500, 4100, 72),
+                                          ("flex 32", 40, 40, 72)])
+def test_gemm_into_a_slice_of_a_wide_tensor(kernel, m, n, k, c_dt):
+    """C is a block of columns of a tensor of 2^21 columns: whole large tiles as planned, the rest on small ones, and
+    nothing beside the block is written.  Alpha, bias and an old C; small integers: exact."""
+    ld = 1 << 21
+    print("case %s m=%d n=%d k=%d c=%d" % (kernel, m, n, k, c_dt), flush=True)
+    assert hip.gemm_kernel(0, 0, m, n, k)[0] == kernel
+    torch.manual_seed(k)
+    a = torch.randint(-3, 4, (m, k), device="cuda").float()
+    b = torch.randint(-2, 3, (k, n), device="cuda").float()
+    bias = torch.randint(-5, 6, (n,), device="cuda").float()
+    c0 = torch.randint(-9, 10, (m, n), device="cuda").float()
+    ah, bh = a.half(), b.half()
+    whole = torch.empty((m, ld), dtype=TORCH_T[c_dt], device="cuda")
+    at = 4096
+    whole[:, at - 300:at + n + 300] = 77
+    block = whole[:, at:at + n]
+    block.copy_(c0)
+    call("br_hip_gemm", 0, 0, m, n, k, 2.0, ptr(ah), F16, k, 0, ptr(bh), F16, n, 0, 1, ptr(block), c_dt, ld, 0,
+         ptr(bias), 1, hip.GEMM_F16, stream())
+    torch.cuda.synchronize()
+    assert torch.equal(block, (2 * (a @ b) + bias + c0).to(block.dtype))
+    assert bool((whole[:, at - 300:at] == 77).all()) and bool((whole[:, at + n:at + n + 300] == 77).all())
+
+
+def test_linear_gelu_epilogue_on_a_wide_output():
+    """More than 2^21 outputs, ragged in both directions; u is exact (small integers), y the GELU of it."""
+    rows, out, inn = 300, (1 << 21) + 8, 64
+    torch.manual_seed(2)
+    x = torch.randint(-2, 3, (rows, inn), device="cuda").half()
+    w = torch.randint(-1, 2, (out, inn), device="cuda").half()
+    u, y = (torch.full((rows, out), float("nan"), dtype=torch.float16, device="cuda") for _ in range(2))
+    call("br_hip_linear_gelu", ptr(x), ptr(w), None, ptr(u), ptr(y), F16, rows, out, inn, stream())
+    torch.cuda.synchronize()
+    for lo in range(0, out, 1 << 18):
+        want = x.float() @ w[lo:lo + (1 << 18)].float().t()
+        assert torch.equal(u[:, lo:lo + (1 << 18)].float(), want)
+        err = (y[:, lo:lo + (1 << 18)].float() - torch.nn.functional.gelu(want, approximate="tanh")).abs()
+        assert float((err / (1 + want.abs())).max()) < 1e-3   # half an fp16 ulp is 5e-4 of the value
