@@ -543,8 +543,8 @@ size_t staged_bytes(int64_t rows, int64_t cols, int64_t batch) {
     return (b + 255) & ~(size_t)255;
 }
 
-// Whether a dense operand is copied before the product: fp32 operands are converted, 16-bit ones whose rows do not
-// start on 16-byte boundaries are moved to rows that do.
+// Whether an operand is copied before the product, dense as it is: fp32 operands are converted, 16-bit ones whose rows
+// do not start on 16-byte boundaries are moved to rows that do.
 bool wants_staging(int dtype, int64_t cols) { return dtype == BR_F32 || cols % 8 != 0; }
 
 }  // namespace
@@ -582,8 +582,13 @@ int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
                          accumulate, addend, c, c_dtype, ldc, stride_c, bias, batch, compute, stream);
     hipStream_t st = as_stream(stream);
     char* ws = static_cast<char*>(workspace);
+    // 16-bit rows that start on 16-byte boundaries all the same (their pitch is padded) are taken where they are, unless
+    // they run along K and end inside a granule, whose rest would have to be zero
+    auto in_place = [&](const void* x, int dtype, bool along_k, int64_t ld, int64_t stride) {
+        return dtype != BR_F32 && !along_k && aligned16(x) && ld % 8 == 0 && (batch == 1 || stride % 8 == 0);
+    };
     // every row of a staged copy is zero-filled up to its pitch
-    if (wants_staging(a_dtype, a_cols)) {
+    if (wants_staging(a_dtype, a_cols) && !in_place(a, a_dtype, !trans_a, lda, stride_a)) {
         const int rc = stage_rows(a, a_dtype == BR_F32, lda, stride_a, a_rows, a_cols, batch, ws, compute, st);
         if (rc != BR_OK) return rc;
         a = ws;
@@ -592,7 +597,7 @@ int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
         stride_a = a_rows * lda;
         ws += staged_bytes(a_rows, a_cols, batch);
     }
-    if (wants_staging(b_dtype, b_cols)) {
+    if (wants_staging(b_dtype, b_cols) && !in_place(b, b_dtype, trans_b, ldb, stride_b)) {
         const int rc = stage_rows(b, b_dtype == BR_F32, ldb, stride_b, b_rows, b_cols, batch, ws, compute, st);
         if (rc != BR_OK) return rc;
         b = ws;

@@ -631,3 +631,30 @@ def test_linear_gelu_epilogue_on_a_wide_output():
         assert torch.equal(u[:, lo:lo + (1 << 18)].float(), want)
         err = (y[:, lo:lo + (1 << 18)].float() - torch.nn.functional.gelu(want, approximate="tanh")).abs()
         assert float((err / (1 + want.abs())).max()) < 1e-3   # half an fp16 ulp is 5e-4 of the value
+
+
+@pytest.mark.parametrize("batch", [1, 3])
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+def test_gemm_staged_takes_rows_of_a_padded_pitch_where_they_are(ta, tb, batch):
+    """16-bit operands of odd sizes whose rows start on 16-byte boundaries: only a row that runs along an odd K is
+    copied (its end has to be zero-filled).  NaNs in the padding, small integers: exact."""
+    m, n, k = 1001, 1003, 65
+    print("case ta=%d tb=%d batch=%d" % (ta, tb, batch), flush=True)
+    torch.manual_seed(4)
+
+    def padded(rows, cols, most):
+        t = torch.full((batch, rows, (cols + 7) // 8 * 8), float("nan"), dtype=torch.float16, device="cuda")
+        t[:, :, :cols] = torch.randint(-most, most + 1, (batch, rows, cols), device="cuda").half()
+        return t
+    a = padded(*((k, m) if ta else (m, k)), 3)
+    b = padded(*((n, k) if tb else (k, n)), 2)
+    c = torch.full((batch, m, n), float("nan"), device="cuda")
+    need = hip.load().br_hip_gemm_staged_workspace(ta, tb, m, n, k, F16, F16, batch)
+    ws = torch.full((need,), 0x7f, dtype=torch.uint8, device="cuda")
+    call("br_hip_gemm_staged", ta, tb, m, n, k, 1.0, ptr(a), F16, a.shape[2], a[0].numel(), ptr(b), F16, b.shape[2],
+         b[0].numel(), 0, ptr(c), F32, n, m * n, None, batch, hip.GEMM_F16, ptr(ws), need, stream())
+    torch.cuda.synchronize()
+    for i in range(batch):
+        x, y = a[i, :, :m if ta else k].float(), b[i, :, :k if tb else n].float()
+        assert torch.equal(c[i], (x.t() if ta else x) @ (y.t() if tb else y))
+    assert bool((ws != 0x7f).any()) == (not ta or tb)
