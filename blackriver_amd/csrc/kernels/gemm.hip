@@ -275,6 +275,25 @@ int gemm_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float a
     if (b_dtype != BR_F32 && b_dtype != native) return BR_ERR_TODO;
     if (c_dtype != BR_F32 && c_dtype != native) return BR_ERR_TODO;
 
+    // A launch of 2^32 or more work items runs without those beyond, and without an error: so many batch entries go in
+    // several launches, of as many as any kernel's tiles (of 32 x 32 elements or more, 512 threads or fewer) leave room for.
+    const double tiles = (double)((m + 31) / 32) * (double)((n + 31) / 32);
+    const int64_t fit = (int64_t)(4294967295.0 / 512.0 / tiles);
+    if (batch > 1 && batch > fit && fit >= 1 && !(planned && planned->slices > 1)) {
+        for (int64_t i = 0; i < batch; i += fit) {
+            auto entry = [&](const void* x, int64_t stride, int dtype) {
+                return static_cast<const char*>(x) + i * stride * elem_size(dtype);
+            };
+            const int rc = gemm_impl(trans_a, trans_b, m, n, k, alpha, entry(a, stride_a, a_dtype), a_dtype, lda, stride_a,
+                                     entry(b, stride_b, b_dtype), b_dtype, ldb, stride_b, accumulate,
+                                     addend ? entry(addend, stride_c, c_dtype) : nullptr,
+                                     const_cast<char*>(entry(c, stride_c, c_dtype)), c_dtype, ldc, stride_c, bias,
+                                     batch - i < fit ? batch - i : fit, compute, stream, planned, padded);
+            if (rc != BR_OK) return rc;
+        }
+        return BR_OK;
+    }
+
     GemmArgs g;
     g.a = a; g.b = b; g.c = c; g.bias = bias;
     g.m = m; g.n = n; g.k = k;

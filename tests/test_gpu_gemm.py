@@ -658,3 +658,16 @@ def test_gemm_staged_takes_rows_of_a_padded_pitch_where_they_are(ta, tb, batch):
         x, y = a[i, :, :m if ta else k].float(), b[i, :, :k if tb else n].float()
         assert torch.equal(c[i], (x.t() if ta else x) @ (y.t() if tb else y))
     assert bool((ws != 0x7f).any()) == (not ta or tb)
+
+
+def test_gemm_of_more_batch_entries_than_a_launch_has_work_items():
+    """1.9 million fp32 products of nine 32 x 32 tiles each are more than 2^32 work items, which a launch drops without
+    an error."""
+    m, k, batch = 65, 4, 1900000
+    print("case batch=%d" % batch, flush=True)
+    a, b = (torch.ones((batch, m * k), device="cuda") for _ in range(2))
+    c = torch.zeros((batch, m * m), device="cuda")
+    call("br_hip_gemm", 0, 1, m, m, k, 1.0, ptr(a), F32, k, m * k, ptr(b), F32, k, m * k, 0, ptr(c), F32, m, m * m, None,
+         batch, hip.GEMM_F32, stream())
+    torch.cuda.synchronize()
+    assert float(c.min()) == float(c.max()) == k
