@@ -177,8 +177,9 @@ __device__ __forceinline__ float gelu_one(float v) {
 // Measured with a plain copy of 134-537 MB: 6.0-6.5 TB/s one granule per thread, 4.4-5.5 TB/s for every persistent
 // or chunked form tried (and 5.4 for the runtime's own device-to-device copy); AdamW over 67 M parameters 396 -> 340 us.
 // The loops stay: they cover what the cap leaves over.
+// Past the cap (of 256-thread workgroups: a launch holds less than 2^32 work items) the kernel's loop takes the rest.
 #ifndef BR_GRID_CAP
-#define BR_GRID_CAP (1 << 24)
+#define BR_GRID_CAP ((1 << 24) - 1)
 #endif
 inline int grid_for(int64_t work_items, int block, int max_blocks = BR_GRID_CAP) {
     int64_t g = (work_items + block - 1) / block;

@@ -414,6 +414,20 @@ def test_memset_fills_exactly_the_requested_bytes(offset, nbytes):
     assert np.all(got[:offset] == 0x11) and np.all(got[offset + nbytes:] == 0x11)
 
 
+def test_memset_of_more_granules_than_a_launch_has_work_items():
+    """2^32 16-byte granules and some: a grid is capped below 2^32 work items and walks the rest."""
+    nbytes = (1 << 36) + (1 << 28) + 5
+    print("case nbytes=%d" % nbytes, flush=True)
+    buf = torch.empty(nbytes + 16, dtype=torch.uint8, device="cuda")
+    buf[-4096:] = 0x11
+    call("br_hip_memset", ptr(buf), 0xAB, nbytes, stream())
+    torch.cuda.synchronize()
+    for at in range(0, nbytes, 1 << 32):
+        part = buf[at:min(at + (1 << 32), nbytes)]
+        assert int(part.min()) == int(part.max()) == 0xAB
+    assert bool((buf[nbytes:] == 0x11).all())
+
+
 @pytest.mark.parametrize("dtype,tdtype", [(F16, torch.float16), (BF16, torch.bfloat16)])
 @pytest.mark.parametrize("rows,cols", [(2048, 16384), (37, 64), (5, 1000), (512, 16384), (300, 3080), (700, 1000),
                                        (700, 1404), (1000, 4100)])
