@@ -870,10 +870,10 @@ int owner_lanes(int64_t rows, int64_t cols, int elem_bytes, OwnerKind kind) {
     }
     if (rows > 1024) return 0;
     if (kind == kOwnBiasGelu) return narrow_type ? (cols <= 2048 ? 2 : cols < 12288 ? 0 : 8) : (cols < 6144 ? 0 : 8);
-    // About as many columns as rows: a block's sums over its hidden size, one launch fewer in a chain of short ones (a
-    // step over 1000 tokens at hidden 1024 450 us, 457 with two launches); the GELU backward comes at four times the
-    // columns there, and on fewer pays for it.
-    if (cols < 3072) return cols < 2 * rows ? 2 : 0;
+    // Fewer than four times as many columns as rows: a block's sums over its hidden size, one launch fewer in a chain of
+    // short ones (a step over 1000 tokens at hidden 1024 450 us, 457 with two launches).  The GELU backward, which comes
+    // at four times the hidden size in a block, pays for it where a caller has it on fewer columns.
+    if (cols < 3072) return cols < 4 * rows ? 2 : 0;
     return cols <= 4096 ? 4 : 8;
 }
 

@@ -158,8 +158,8 @@ def test_colsum_16_bit(rows, cols, dtype):
 @pytest.mark.parametrize("dtype,rows,cols,launches", [
     (F16, 65536, 512, 2), (BF16, 4096, 6144, 2), (F16, 1025, 64, 2), (F16, 1024, 64, 1), (F16, 2048, 6152, 1),
     (BF16, 2049, 6152, 2), (F16, 4099, 12296, 1), (F16, 128, 264, 1), (BF16, 129, 264, 1), (F16, 512, 4104, 1),
-    (F32, 512, 64, 1), (F32, 513, 64, 1), (F32, 1024, 2044, 1), (F32, 1024, 2048, 2), (F32, 1024, 3072, 1),
-    (F32, 1024, 3068, 2), (F32, 1025, 4096, 2),
+    (F32, 512, 64, 1), (F32, 513, 64, 1), (F32, 1024, 2048, 1), (F32, 513, 2048, 1), (F32, 513, 2052, 2),
+    (F32, 700, 2800, 2), (F32, 1024, 3072, 1), (F32, 1025, 4096, 2),
     (F32, 128, 4100, 1), (F32, 129, 2052, 1), (F32, 700, 4100, 1)])
 def test_colsum_takes_one_launch_or_two(dtype, rows, cols, launches):
     """Both sides of the lines between the one-launch form and the two-launch
