@@ -78,6 +78,13 @@ int product(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alp
                               accumulate, c, c_dtype, ldc, stride_c, bias, batch, compute, ws, need, stream);
 }
 
+// Column sums and the two products of a backward operator, in this order or, where they are small, as one launch.
+int two_products(const br_product& first, const br_product& second, const br_column_sums* sums, int compute) {
+    const size_t need = br_hip_gemm_pair_workspace(&first, &second, compute);
+    void* ws = need ? ComputingContext::gemm_staging(0, need) : nullptr;
+    return br_hip_gemm_pair(&first, &second, sums, compute, ws, need, ComputingContext::stream);
+}
+
 // An operand that several products of one operator read: with a 16-bit MFMA
 // type an fp32 operand is converted once here (same rounding as the staged
 // GEMM entry point applies), otherwise it is passed through.
@@ -100,12 +107,12 @@ Operand shared_operand(const void* p, int dtype, int64_t items, int compute) {
 // available in the products' type: weight_g[out,in] = dy^T . x, then
 // x_g[n,in] = dy . W (in that order: x_g may overwrite x).
 int linear_backward_products(const Operand& dy, const tensor_t& x, const tensor_t& weight, const tensor_t& x_g,
-                             const tensor_t& weight_g, int64_t n, int64_t in, int64_t out, int compute) {
-    int rc = product(1, 0, out, in, n, unlift(), dy.ptr, dy.dtype, out, 0, x->data(), code(x), in, 0, 0, weight_g->data(),
-                     code(weight_g), in, 0, nullptr, 1, compute);
-    if (rc != BR_OK) return rc;
-    return product(0, 0, n, in, out, 1.0f, dy.ptr, dy.dtype, out, 0, weight->data(), code(weight), in, 0, 0,
-                   x_g->data(), code(x_g), in, 0, nullptr, 1, compute);
+                             const tensor_t& weight_g, int64_t n, int64_t in, int64_t out, int compute,
+                             const br_column_sums* sums = nullptr) {
+    return two_products(
+        {1, 0, out, in, n, unlift(), dy.ptr, dy.dtype, out, 0, x->data(), code(x), in, 0, weight_g->data(), code(weight_g), in, 0, 1},
+        {0, 0, n, in, out, 1.0f, dy.ptr, dy.dtype, out, 0, weight->data(), code(weight), in, 0, x_g->data(), code(x_g), in, 0, 1},
+        sums, compute);
 }
 
 // fp32 device pointer to a bias vector, converting 16-bit storage on the fly
@@ -611,19 +618,18 @@ ComputingReturn HIPTensor<DT>::op_linear_backward(tensor_t self, tensor_t x, ten
     // bias_g[o] = sum_n dy[n,o]
     const size_t need = br_hip_colsum_workspace(n, out);
     void* ws = need <= head_bytes() ? ComputingContext::workspace : ComputingContext::scratch(need);
-    Operand dy{mem_, (int)DT};
     if (DT == DataType::Float && compute != BR_GEMM_F32 && out % 8 == 0) {
         // one pass over dy: its column sums and the 16-bit copy both products read
         const int native = compute == BR_GEMM_F16 ? BR_F16 : BR_BF16;
         void* dy16 = ComputingContext::gemm_staging(1, (size_t)(n * out) * 2);
         BR_OP(br_hip_colsum_cast(static_cast<const float*>(mem_), static_cast<float*>(bias_g->data()), dy16, native, n,
                                  out, unlift(), ws, need, stream()));
-        dy = Operand{dy16, native};
+        BR_OP(linear_backward_products(Operand{dy16, native}, x, weight, x_g, weight_g, n, in, out, compute));
     } else {
-        BR_OP(br_hip_colsum(mem_, (int)DT, static_cast<float*>(bias_g->data()), n, out, unlift(), ws, need, stream()));
-        dy = shared_operand(mem_, (int)DT, n * out, compute);
+        const br_column_sums sums{mem_, (int)DT, static_cast<float*>(bias_g->data()), n, out, unlift(), ws, need};
+        BR_OP(linear_backward_products(shared_operand(mem_, (int)DT, n * out, compute), x, weight, x_g, weight_g, n, in, out,
+                                       compute, &sums));
     }
-    BR_OP(linear_backward_products(dy, x, weight, x_g, weight_g, n, in, out, compute));
     return OP_OK;
 }
 
@@ -648,6 +654,15 @@ bool attn_dims(const tensor_t& d_o, const tensor_t& attn, const tensor_t& v, Att
     d.hd = (int64_t)s[3];
     return (int64_t)attn->items() == d.bh * d.t * d.t && (int64_t)v->items() == d.bh * d.t * d.hd;
 }
+// v_g = P^T . dO, then dP = dO . V^T
+int attn_products(const Operand& d_o, const tensor_t& attn, const tensor_t& v, void* dp, int dp_dtype, const tensor_t& v_g,
+                  const AttnDims& d, int compute) {
+    return two_products({1, 0, d.t, d.hd, d.t, 1.0f, attn->data(), code(attn), d.t, d.t * d.t, d_o.ptr, d_o.dtype, d.hd,
+                         d.t * d.hd, v_g->data(), code(v_g), d.hd, d.t * d.hd, d.bh},
+                        {0, 1, d.t, d.t, d.hd, 1.0f, d_o.ptr, d_o.dtype, d.hd, d.t * d.hd, v->data(), code(v), d.hd,
+                         d.t * d.hd, dp, dp_dtype, d.t, d.t * d.t, d.bh},
+                        nullptr, compute);
+}
 }  // namespace
 
 // self = dO[B,NH,T,HD]:  v_g = P^T . dO,  attn_g = dO . V^T
@@ -660,10 +675,7 @@ ComputingReturn HIPTensor<DT>::op_attn_backward(tensor_t self, tensor_t attn, te
         return OP_OUTPUT_ERROR;
     const int compute = pick_compute({self, attn, v});
     const Operand d_o = shared_operand(mem_, (int)DT, d.bh * d.t * d.hd, compute);
-    BR_OP(product(1, 0, d.t, d.hd, d.t, 1.0f, attn->data(), code(attn), d.t, d.t * d.t, d_o.ptr, d_o.dtype, d.hd,
-                  d.t * d.hd, 0, v_g->data(), code(v_g), d.hd, d.t * d.hd, nullptr, d.bh, compute));
-    BR_OP(product(0, 1, d.t, d.t, d.hd, 1.0f, d_o.ptr, d_o.dtype, d.hd, d.t * d.hd, v->data(), code(v), d.hd,
-                  d.t * d.hd, 0, attn_g->data(), code(attn_g), d.t, d.t * d.t, nullptr, d.bh, compute));
+    BR_OP(attn_products(d_o, attn, v, attn_g->data(), code(attn_g), v_g, d, compute));
     return OP_OK;
 }
 
@@ -705,11 +717,8 @@ ComputingReturn HIPTensor<DT>::op_softmax_attn_backward(tensor_t self, tensor_t 
         return OP_OUTPUT_ERROR;
     const int compute = pick_compute({self, attn, v});
     const Operand d_o = shared_operand(mem_, (int)DT, d.bh * d.t * d.hd, compute);
-    BR_OP(product(1, 0, d.t, d.hd, d.t, 1.0f, attn->data(), code(attn), d.t, d.t * d.t, d_o.ptr, d_o.dtype, d.hd,
-                  d.t * d.hd, 0, v_g->data(), code(v_g), d.hd, d.t * d.hd, nullptr, d.bh, compute));
     float* dp = static_cast<float*>(ComputingContext::scratch((size_t)(d.bh * d.t * d.t) * sizeof(float)));
-    BR_OP(product(0, 1, d.t, d.t, d.hd, 1.0f, d_o.ptr, d_o.dtype, d.hd, d.t * d.hd, v->data(), code(v), d.hd,
-                  d.t * d.hd, 0, dp, BR_F32, d.t, d.t * d.t, nullptr, d.bh, compute));
+    BR_OP(attn_products(d_o, attn, v, dp, BR_F32, v_g, d, compute));
     BR_OP(br_hip_softmax_bwd(dp, static_cast<const float*>(attn->data()), static_cast<float*>(attn_g->data()),
                              d.bh * d.t, d.t, stream()));
     return OP_OK;
@@ -726,10 +735,11 @@ ComputingReturn HIPTensor<DT>::op_qk_backward(tensor_t self, tensor_t q, tensor_
     const float alpha = (float)(1.0 / sqrt((double)hd));
     const int compute = pick_compute({self, q, k});
     const Operand ds = shared_operand(mem_, (int)DT, bh * t * t, compute);
-    BR_OP(product(0, 0, t, hd, t, alpha, ds.ptr, ds.dtype, t, t * t, k->data(), code(k), hd, t * hd, 0, q_g->data(),
-                  code(q_g), hd, t * hd, nullptr, bh, compute));
-    BR_OP(product(1, 0, t, hd, t, alpha, ds.ptr, ds.dtype, t, t * t, q->data(), code(q), hd, t * hd, 0, k_g->data(),
-                  code(k_g), hd, t * hd, nullptr, bh, compute));
+    BR_OP(two_products({0, 0, t, hd, t, alpha, ds.ptr, ds.dtype, t, t * t, k->data(), code(k), hd, t * hd, q_g->data(), code(q_g),
+                        hd, t * hd, bh},
+                       {1, 0, t, hd, t, alpha, ds.ptr, ds.dtype, t, t * t, q->data(), code(q), hd, t * hd, k_g->data(), code(k_g),
+                        hd, t * hd, bh},
+                       nullptr, compute));
     return OP_OK;
 }
 

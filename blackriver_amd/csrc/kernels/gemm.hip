@@ -20,6 +20,7 @@
 #include <string.h>
 
 #include "gemm_dtl16.hpp"
+#include "gemm_pair.hpp"
 
 using namespace brk;
 
@@ -33,6 +34,13 @@ BR_GEMM16_ENTRIES(f16)
 BR_GEMM16_ENTRIES(bf16)
 #undef BR_GEMM16_ENTRIES
 int gemm_fp32(const gemm16::GemmArgs& g, const gemm16::Problem& p, int kernel, bool words, long long batch, hipStream_t st);
+#define BR_GEMM_PAIR_ENTRY(T)                                                                                            \
+    int gemm_pair_##T(const gemm16::GemmArgs& w, const gemm16::Problem& pw, long long batch_w, const gemm16::GemmArgs& x,    \
+                      const gemm16::Problem& px, long long batch_x, int kernel, const gemm16::ColumnSums& sums, hipStream_t st);
+BR_GEMM_PAIR_ENTRY(f16)
+BR_GEMM_PAIR_ENTRY(bf16)
+BR_GEMM_PAIR_ENTRY(f32)
+#undef BR_GEMM_PAIR_ENTRY
 }  // namespace brk
 
 namespace {
@@ -669,4 +677,197 @@ extern "C" int br_hip_linear_residual(const void* x, int x_dtype, const void* w,
     if (!y) return BR_ERR_OUTPUT;
     return staged_impl(0, 1, rows, out, in, 1.0f, x, x_dtype, in, 0, w, w_dtype, in, 0, 1, r, y, y_dtype, out, 0, bias, 1,
                        compute, workspace, workspace_bytes, stream);
+}
+
+// ---- two products in one launch -------------------------------------------------
+namespace {
+
+// A stored operand: rows x cols of a batch entry, rows `ld` apart, entries `stride`.
+struct Stored {
+    const void* at;
+    int dtype;
+    int64_t rows, cols, ld, stride, batch;
+    bool along_k;   // rows run along K
+};
+Stored stored_a(const br_product& p) {
+    return {p.a, p.a_dtype, p.trans_a ? p.k : p.m, p.trans_a ? p.m : p.k, p.lda, p.stride_a, p.batch, p.trans_a == 0};
+}
+Stored stored_b(const br_product& p) {
+    return {p.b, p.b_dtype, p.trans_b ? p.n : p.k, p.trans_b ? p.k : p.n, p.ldb, p.stride_b, p.batch, p.trans_b != 0};
+}
+Stored stored_c(const br_product& p) { return {p.c, p.c_dtype, p.m, p.n, p.ldc, p.stride_c, p.batch, false}; }
+
+bool same_memory(const Stored& x, const Stored& y) {
+    return x.at == y.at && x.dtype == y.dtype && x.rows == y.rows && x.cols == y.cols && x.ld == y.ld &&
+           (x.batch == 1 || x.stride == y.stride) && x.batch == y.batch;
+}
+
+bool overlap(const Stored& x, const Stored& y) {
+    auto bytes = [](const Stored& s) { return (uintptr_t)((s.batch - 1) * s.stride + (s.rows - 1) * s.ld + s.cols) * elem_size(s.dtype); };
+    const uintptr_t x0 = reinterpret_cast<uintptr_t>(x.at), y0 = reinterpret_cast<uintptr_t>(y.at);
+    return x0 < y0 + bytes(y) && y0 < x0 + bytes(x);
+}
+
+size_t staged_size(const Stored& s) { return wants_staging(s.dtype, s.cols) ? staged_bytes(s.rows, s.cols, s.batch) : 0; }
+
+bool sizes_ok(const br_product& p) {
+    return p.m > 0 && p.n > 0 && p.k > 0 && p.batch > 0 && p.a && p.b && p.c && p.lda >= (p.trans_a ? p.m : p.k) &&
+           p.ldb >= (p.trans_b ? p.k : p.n) && p.ldc >= p.n && (p.batch == 1 || (p.stride_a >= 0 && p.stride_b >= 0 && p.stride_c >= 0));
+}
+
+// Both products (and the column sums) as one launch; BR_ERR_TODO where they have to run one after the other.
+int pair_impl(const br_product& first, const br_product& second, const br_column_sums* sums, int compute, void* workspace,
+              size_t workspace_bytes, hipStream_t st) {
+    using namespace gemm16;
+    const bool fp32 = compute == BR_GEMM_F32;
+    const int native = compute == BR_GEMM_F16 ? BR_F16 : fp32 ? BR_F32 : BR_BF16;
+    // the one with both operands row-contiguous
+    auto wide = [](const br_product& p) { return p.trans_a && !p.trans_b && p.c_dtype == BR_F32; };
+    const int w = wide(first) ? 0 : 1, x = 1 - w;
+    if (!sizes_ok(first) || !sizes_ok(second) || !wide(w ? second : first) || (w ? first : second).trans_a) return BR_ERR_TODO;
+    const int kernel = pair_kernel({first.m, first.n, first.k, first.batch}, {second.m, second.n, second.k, second.batch}, fp32);
+    if (kernel < 0) return BR_ERR_TODO;
+    const br_product* const products[2] = {&first, &second};
+    Stored in[4] = {stored_a(first), stored_b(first), stored_a(second), stored_b(second)};
+    const Stored out[2] = {stored_c(first), stored_c(second)};
+    for (const Stored& s : in)
+        if (s.dtype != native && s.dtype != BR_F32) return BR_ERR_TODO;
+    if (out[x].dtype != native && out[x].dtype != BR_F32) return BR_ERR_TODO;
+    // nothing is written that another part reads or writes (before staging: what is staged is read ahead of all writes)
+    if (overlap(out[0], out[1]) || overlap(out[0], in[2]) || overlap(out[0], in[3])) return BR_ERR_TODO;
+    ColumnSums cs;
+    if (sums) {
+        const Stored sx{sums->x, sums->dtype, sums->rows, sums->cols, sums->cols, 0, 1, false};
+        const Stored so{sums->out, BR_F32, 1, sums->cols, sums->cols, 0, 1, false};
+        const long long vec = fp32 ? 4 : 8;
+        if (!sums->x || !sums->out || sums->dtype != native || sums->rows <= 0 || sums->cols <= 0 || sums->cols % vec != 0 ||
+            sums->rows > 0x3fffffffLL || sums->cols > 0x3fffffffLL || !aligned16(sums->x))
+            return BR_ERR_TODO;
+        for (const Stored& s : in)
+            if (overlap(so, s)) return BR_ERR_TODO;
+        for (const Stored& s : out)
+            if (overlap(so, s) || overlap(sx, s)) return BR_ERR_TODO;
+        cs.x = sums->x;
+        cs.out = sums->out;
+        cs.rows = (int)sums->rows;
+        cs.cols = (int)sums->cols;
+        cs.scale = sums->scale;
+    }
+    // which operands are copied, and where to; one that both products read is copied once
+    const Stored before[4] = {in[0], in[1], in[2], in[3]};
+    char* ws = static_cast<char*>(workspace);
+    size_t used = 0;
+    int copy_of[4] = {-1, -1, -1, -1};
+    for (int i = 0; i < 4 && !fp32; i++) {
+        const bool in_place = in[i].dtype != BR_F32 && !in[i].along_k && aligned16(in[i].at) && in[i].ld % 8 == 0 &&
+                              (in[i].batch == 1 || in[i].stride % 8 == 0);
+        if (!wants_staging(in[i].dtype, in[i].cols) || in_place) continue;
+        copy_of[i] = i;
+        for (int j = 0; j < i; j++)
+            if (copy_of[j] == j && same_memory(before[i], before[j])) copy_of[i] = j;
+        if (copy_of[i] == i) {
+            in[i].at = ws + used;
+            used += staged_bytes(in[i].rows, in[i].cols, in[i].batch);
+            in[i].dtype = native;
+            in[i].ld = staged_pitch(in[i].cols);
+            in[i].stride = in[i].rows * in[i].ld;
+        } else {
+            const Stored& from = in[copy_of[i]];
+            in[i].at = from.at;
+            in[i].dtype = native;
+            in[i].ld = from.ld;
+            in[i].stride = from.stride;
+        }
+    }
+    if (used > 0 && (!ws || !aligned16(ws) || used > workspace_bytes)) return BR_ERR_TODO;
+    for (int i = 0; i < 2; i++)
+        if (overlap(out[1], in[i])) return BR_ERR_TODO;
+    GemmArgs g[2];
+    Problem p[2];
+    for (int i = 0; i < 2; i++) {
+        const Stored &a = in[2 * i], &b = in[2 * i + 1];
+        const br_product& d = *products[i];
+        GemmArgs& q = g[i];
+        q.a = a.at; q.b = b.at; q.c = d.c; q.bias = nullptr;
+        q.m = d.m; q.n = d.n; q.k = d.k;
+        q.lda = a.ld; q.ldb = b.ld; q.ldc = d.ldc;
+        q.sa = a.stride; q.sb = b.stride; q.sc = d.stride_c;
+        q.alpha = d.alpha;
+        q.accumulate = 0;
+        q.tiles_m = q.tiles_n = 0;   // set by the launcher
+        auto aligned = [&](const Stored& s) {
+            const long long es = elem_size(s.dtype);
+            return aligned16(s.at) && s.ld * es % 16 == 0 && (s.batch == 1 || s.stride * es % 16 == 0);
+        };
+        q.vec_a = aligned(a);
+        q.vec_b = aligned(b);
+        p[i].a_f32 = a.dtype == BR_F32;
+        p[i].b_f32 = b.dtype == BR_F32;
+        p[i].a_kstr = d.trans_a != 0;
+        p[i].b_kstr = d.trans_b == 0;
+        p[i].c_dtype = d.c_dtype;
+        p[i].guarded = false;
+        p[i].padded = true;
+        if (fp32) {
+            const long long lim = 1LL << 31;
+            if (256 * q.lda >= lim || 256 * q.ldb >= lim || q.m >= lim || q.n >= lim || q.k >= lim || !q.vec_a || !q.vec_b ||
+                (q.k % 4 != 0 && !(p[i].a_kstr && p[i].b_kstr)))
+                return BR_ERR_TODO;
+        } else if (!dtl_applies(q, p[i])) {
+            return BR_ERR_TODO;
+        }
+    }
+    for (int i = 0; i < 4; i++) {
+        if (copy_of[i] != i) continue;
+        const int rc = stage_rows(before[i].at, before[i].dtype == BR_F32, before[i].ld, before[i].stride, before[i].rows, before[i].cols,
+                                  before[i].batch, const_cast<void*>(in[i].at), compute, st);
+        if (rc != BR_OK) return rc;
+    }
+    auto* const launch = fp32 ? gemm_pair_f32 : compute == BR_GEMM_F16 ? gemm_pair_f16 : gemm_pair_bf16;
+    return launch(g[w], p[w], products[w]->batch, g[x], p[x], products[x]->batch, kernel, cs, st);
+}
+
+}  // namespace
+
+extern "C" size_t br_hip_gemm_pair_workspace(const br_product* first, const br_product* second, int compute) {
+    if (!first || !second || compute == BR_GEMM_F32) return 0;
+    const bool one_launch = br_hip_gemm_pair_kernel(first->m, first->n, first->k, first->batch, second->m, second->n, second->k,
+                                                    second->batch, compute) >= 0;
+    size_t both = 0, most = 0;
+    for (const br_product* p : {first, second}) {
+        if (p->m <= 0 || p->n <= 0 || p->k <= 0 || p->batch <= 0) continue;
+        if (one_launch) both += staged_size(stored_a(*p)) + staged_size(stored_b(*p));
+        const size_t one = br_hip_gemm_staged_workspace(p->trans_a, p->trans_b, p->m, p->n, p->k, p->a_dtype, p->b_dtype, p->batch);
+        if (one > most) most = one;
+    }
+    return both > most ? both : most;
+}
+
+extern "C" int br_hip_gemm_pair_kernel(int64_t m1, int64_t n1, int64_t k1, int64_t batch1, int64_t m2, int64_t n2, int64_t k2,
+                                       int64_t batch2, int compute) {
+    if (m1 <= 0 || n1 <= 0 || k1 <= 0 || batch1 <= 0 || m2 <= 0 || n2 <= 0 || k2 <= 0 || batch2 <= 0) return BR_ERR_ATTR;
+    return gemm16::pair_kernel({m1, n1, k1, batch1}, {m2, n2, k2, batch2}, compute == BR_GEMM_F32);
+}
+
+extern "C" int br_hip_gemm_pair(const br_product* first, const br_product* second, const br_column_sums* sums, int compute,
+                                void* workspace, size_t workspace_bytes, br_stream_t stream) {
+    if (!first || !second) return BR_ERR_INPUT;
+    if (compute != BR_GEMM_F16 && compute != BR_GEMM_BF16 && compute != BR_GEMM_F32) return BR_ERR_ATTR;
+    const int rc = pair_impl(*first, *second, sums, compute, workspace, workspace_bytes, as_stream(stream));
+    if (rc != BR_ERR_TODO) return rc;
+    if (sums) {
+        const int rs = br_hip_colsum(sums->x, sums->dtype, sums->out, sums->rows, sums->cols, sums->scale, sums->workspace,
+                                     sums->workspace_bytes, stream);
+        if (rs != BR_OK) return rs;
+    }
+    for (const br_product* p : {first, second}) {
+        const int rp = compute == BR_GEMM_F32
+            ? gemm_impl(p->trans_a, p->trans_b, p->m, p->n, p->k, p->alpha, p->a, p->a_dtype, p->lda, p->stride_a, p->b, p->b_dtype,
+                        p->ldb, p->stride_b, 0, nullptr, p->c, p->c_dtype, p->ldc, p->stride_c, nullptr, p->batch, compute, stream)
+            : staged_impl(p->trans_a, p->trans_b, p->m, p->n, p->k, p->alpha, p->a, p->a_dtype, p->lda, p->stride_a, p->b, p->b_dtype,
+                          p->ldb, p->stride_b, 0, nullptr, p->c, p->c_dtype, p->ldc, p->stride_c, nullptr, p->batch, compute,
+                          workspace, workspace_bytes, stream);
+        if (rp != BR_OK) return rp;
+    }
+    return BR_OK;
 }

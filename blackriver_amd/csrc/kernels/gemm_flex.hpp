@@ -201,8 +201,13 @@ __device__ __forceinline__ void flex_emit(const GemmArgs& g, const lds_byte* lds
     }
 }
 
-template <int CT, int BM, int BN, int KW, int ST, bool A_KSTR, bool B_KSTR, typename TC, bool GELU = false, bool WORDS = false>
-__global__ __launch_bounds__(KW * 64) void gemm_flex_kernel(GemmArgs g) {
+// LDS of a workgroup of such tiles
+template <int BM, int BN, int KW, int ST>
+constexpr int flex_lds_bytes() { return KW * ST * (BM + BN) * 128; }
+
+// Workgroup `id` of the `groups` a product has.  SLICES: it may be one of several slices of K (g.splits).
+template <int CT, int BM, int BN, int KW, int ST, bool A_KSTR, bool B_KSTR, typename TC, bool GELU, bool WORDS, bool SLICES>
+__device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, unsigned groups, unsigned char* lds_raw) {
     using TA = FlexTile<CT, BM, A_KSTR, WORDS>;
     using TB = FlexTile<CT, BN, B_KSTR, WORDS>;
     constexpr int kSize = TA::kSize, KT = TA::kStep;
@@ -211,22 +216,22 @@ __global__ __launch_bounds__(KW * 64) void gemm_flex_kernel(GemmArgs g) {
     constexpr int kLoads = TA::kInstr + TB::kInstr;
     constexpr int kWaveBytes = ST * kStageBytes;
     static_assert(kWaveBytes >= BM * BN * 4, "a wave's buffers hold its accumulators at the end");
-    static_assert(KW * kWaveBytes <= 160 * 1024, "LDS");
+    static_assert(KW * kWaveBytes <= 160 * 1024 && KW * kWaveBytes == flex_lds_bytes<BM, BN, KW, ST>(), "LDS");
     static_assert((ST - 1) * kLoads <= 63, "loads a partial wait can leave outstanding");
-    __shared__ __attribute__((aligned(1024))) unsigned char lds_raw[KW * kWaveBytes];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     long long batch;
     int tm, tn;
-    tile_coords(g, batch, tm, tn);
+    tile_coords(g, id, groups, batch, tm, tn);
     tm = __builtin_amdgcn_readfirstlane(tm);
     tn = __builtin_amdgcn_readfirstlane(tn);
     const int b = __builtin_amdgcn_readfirstlane((int)batch);
     const int row0 = tm * BM, col0 = tn * BN;
     // slices of K take the place of the batch index
-    const bool sliced = g.splits > 1;
+    const bool sliced = SLICES && g.splits > 1;
     const int k_begin = sliced ? b * g.k_slice : 0;
-    const int k_end = sliced && k_begin + g.k_slice < g.k ? k_begin + g.k_slice : (int)g.k;
+    const int k_rest = (int)g.k - k_begin;
+    const int k_end = k_begin + (sliced && g.k_slice < k_rest ? g.k_slice : k_rest);
 
     // this wave's first K step, and where each operand ends as seen from it
     const int k0 = k_begin + wave * KT;
@@ -324,6 +329,12 @@ __global__ __launch_bounds__(KW * 64) void gemm_flex_kernel(GemmArgs g) {
     flex_emit<BM, BN, KW, KW * 64, TC, GELU>(g, (lds_byte*)lds_raw, kWaveBytes, row0, col0, b);
 }
 
+template <int CT, int BM, int BN, int KW, int ST, bool A_KSTR, bool B_KSTR, typename TC, bool GELU = false, bool WORDS = false>
+__global__ __launch_bounds__(KW * 64) void gemm_flex_kernel(GemmArgs g) {
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[flex_lds_bytes<BM, BN, KW, ST>()];
+    flex_product<CT, BM, BN, KW, ST, A_KSTR, B_KSTR, TC, GELU, WORDS, true>(g, blockIdx.x, gridDim.x, lds);
+}
+
 // 64 x 128 tiles, a ring of six K steps, waves that load beside waves that multiply.  The kernel above gives a wave
 // whole K steps and buffers of its own; a tile of this size leaves no room for two such buffers a wave.  Here four
 // waves share a ring of 24 KB steps: wave w multiplies k-values 16 w .. 16 w + 15 of every step by itself, so a fragment
@@ -361,7 +372,8 @@ __global__ __launch_bounds__(512) void gemm_ring_kernel(GemmArgs g) {
     // slices of K take the place of the batch index
     const bool sliced = g.splits > 1;
     const int k_begin = sliced ? b * g.k_slice : 0;
-    const int k_end = sliced && k_begin + g.k_slice < g.k ? k_begin + g.k_slice : (int)g.k;
+    const int k_rest = (int)g.k - k_begin;
+    const int k_end = k_begin + (sliced && g.k_slice < k_rest ? g.k_slice : k_rest);
     const int steps = (k_end - k_begin + KT - 1) / KT;
     const int padded = steps + (steps & 1);   // the multipliers take steps in pairs
     // step t of the loop covers K step (t + first) mod steps of the slice (see k_walk_start)

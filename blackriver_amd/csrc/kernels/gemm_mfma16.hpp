@@ -314,10 +314,8 @@ __device__ __forceinline__ void tile_in_order(const GemmArgs& g, int rem, int& t
     tn = first_n + within / gm;
 }
 
-// Workgroup id -> (batch, tile_m, tile_n).
-__device__ __forceinline__ void tile_coords(const GemmArgs& g, long long& batch, int& tm, int& tn) {
-    const long long nb = gridDim.x;
-    long long id = blockIdx.x;
+// Workgroup `id` of the `nb` a product has -> (batch, tile_m, tile_n).
+__device__ __forceinline__ void tile_coords(const GemmArgs& g, long long id, long long nb, long long& batch, int& tm, int& tn) {
     // ids are dealt to the 8 XCDs round-robin; make each XCD's share contiguous
     const long long per_xcd = nb / 8;
     if (per_xcd > 0 && id < per_xcd * 8) id = (id % 8) * per_xcd + id / 8;
@@ -325,6 +323,9 @@ __device__ __forceinline__ void tile_coords(const GemmArgs& g, long long& batch,
     batch = id / per_batch;
     const int rem = (int)(id % per_batch);
     tile_in_order(g, rem, tm, tn);
+}
+__device__ __forceinline__ void tile_coords(const GemmArgs& g, long long& batch, int& tm, int& tn) {
+    tile_coords(g, blockIdx.x, gridDim.x, batch, tm, tn);
 }
 
 // Where a tile starts its walk over K (an element index, a multiple of 64; the walk wraps round at the end of K).

@@ -174,5 +174,62 @@ inline int fp32_kernel(long long m, long long n, long long k, long long batch) {
     return best;
 }
 
+// Two products as one launch of small tiles (gemm_pair.hpp): the tile, or -1 where they run one after the other.
+//
+//   us = start + max(longest walk * step, sum over both of workgroups * (steps + merge) * load / 256)
+//
+// fitted to 124 pairs (linear layers of 256 .. 3072 features and 19 .. 953 tokens, attention heads of 16 .. 512 tokens),
+// each on every tile and as two launches; median error 3-7 %.  By the rule all of them together take 0.74 of the time of
+// two launches, by the best of the measurements too; the longest that gained was one of 27 us in two launches (18.3 in
+// one: 885 tokens, 640 -> 2560 in fp16), from 30 us on large tiles win ([1024 x 4096] from 622 tokens 28.3 in two, 29.7).
+struct PairCost {
+    double start, step, load, merge;
+};
+constexpr int kPairKernels[3] = {kFlex64, kFlex32x64, kFlex32};
+constexpr PairCost kPairCost16[3] = {{4.29, 0.884, 0.757, 1.80}, {3.47, 0.722, 0.596, 0.79}, {3.02, 0.542, 0.433, 1.47}};
+constexpr PairCost kPairCost32[3] = {{4.55, 2.392, 2.434, 0.54}, {3.72, 1.365, 0.962, 1.72}, {3.31, 0.807, 0.650, 0.65}};
+struct PairSizes {
+    long long m, n, k, batch;
+};
+inline double fp32_us(int kernel, const PairSizes& s) {
+    const KernelCost& c = kCost[kernel];
+    const double load = (double)(ceil_div(s.m, c.bm) * ceil_div(s.n, c.bn) * s.batch) / 256.0;
+    const double step = kernel == kFlex64 ? 2.45 : kernel == kFlex32x64 ? 1.4 : 0.78;
+    return 2.7 + (load >= 4.0 ? load : ceil(load)) * (double)ceil_div(ceil_div(s.k, 32), 4) * step;
+}
+#ifndef BR_PAIR_FORCE
+#define BR_PAIR_FORCE -1   // a kernel: every pair of products on it, for measuring
+#endif
+inline int pair_kernel(const PairSizes& a, const PairSizes& b, bool fp32) {
+    if (BR_PAIR_FORCE >= 0) return BR_PAIR_FORCE;
+    double us = 0.0;   // one after the other
+    for (const PairSizes* s : {&a, &b}) {
+        if (fp32) {
+            const int kernel = fp32_kernel(s->m, s->n, s->k, s->batch);
+            if (kernel == kTile128) return -1;
+            us += fp32_us(kernel, *s);
+        } else {
+            us += gemm_plan(s->m, s->n, s->k, s->batch, true).us;
+        }
+    }
+    int best = -1;
+    double best_us = 1e30;
+    for (int i = 0; i < 3; i++) {
+        const KernelCost& tile = kCost[kPairKernels[i]];
+        const PairCost& c = fp32 ? kPairCost32[i] : kPairCost16[i];
+        double longest = 0.0, all = 0.0;
+        for (const PairSizes* s : {&a, &b}) {
+            const double groups = (double)(ceil_div(s->m, tile.bm) * ceil_div(s->n, tile.bn) * s->batch);
+            const double steps = (double)ceil_div(ceil_div(s->k, fp32 ? 32 : 64), tile.k_waves);
+            if (steps * c.step > longest) longest = steps * c.step;
+            all += groups * (steps + c.merge) * c.load / 256.0;
+        }
+        const double t = c.start + (all > longest ? all : longest);
+        // (a hurdle for the close ones: [1024 x 4096] from 74 tokens 14.3 in two launches, 14.8 in one)
+        if (t < 0.97 * us && t < best_us) best = kPairKernels[i], best_us = t;
+    }
+    return best;
+}
+
 }  // namespace gemm16
 }  // namespace brk

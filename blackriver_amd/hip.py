@@ -22,6 +22,20 @@ _int = ctypes.c_int
 _f32 = ctypes.c_float
 _sz = ctypes.c_size_t
 
+
+class Product(ctypes.Structure):
+    """br_product: one of the two products of br_hip_gemm_pair."""
+    _fields_ = [("trans_a", _int), ("trans_b", _int), ("m", _i64), ("n", _i64), ("k", _i64), ("alpha", _f32), ("a", _vp),
+                ("a_dtype", _int), ("lda", _i64), ("stride_a", _i64), ("b", _vp), ("b_dtype", _int), ("ldb", _i64),
+                ("stride_b", _i64), ("c", _vp), ("c_dtype", _int), ("ldc", _i64), ("stride_c", _i64), ("batch", _i64)]
+
+
+class ColumnSums(ctypes.Structure):
+    """br_column_sums: the column sums beside them."""
+    _fields_ = [("x", _vp), ("dtype", _int), ("out", _vp), ("rows", _i64), ("cols", _i64), ("scale", _f32),
+                ("workspace", _vp), ("workspace_bytes", _sz)]
+
+
 # name -> (restype, argtypes); mirrors include/br_hip.h one to one
 SIGNATURES = {
     "br_hip_device_count": (_int, [ctypes.POINTER(_int)]),
@@ -82,6 +96,9 @@ SIGNATURES = {
     "br_hip_gemm_staged_workspace": (ctypes.c_size_t, [_int, _int, _i64, _i64, _i64, _int, _int, _i64]),
     "br_hip_gemm_staged": (_int, [_int, _int, _i64, _i64, _i64, _f32, _vp, _int, _i64, _i64, _vp, _int, _i64, _i64,
                                   _int, _vp, _int, _i64, _i64, _vp, _i64, _int, _vp, ctypes.c_size_t, _vp]),
+    "br_hip_gemm_pair_workspace": (ctypes.c_size_t, [_vp, _vp, _int]),
+    "br_hip_gemm_pair": (_int, [_vp, _vp, _vp, _int, _vp, ctypes.c_size_t, _vp]),
+    "br_hip_gemm_pair_kernel": (_int, [_i64] * 8 + [_int]),
     "br_hip_gemm_kernel": (_int, [_int, _int, _i64, _i64, _i64, _int, _i64, _int, ctypes.POINTER(_int)]),
     "br_hip_flash_attn_fwd": (_int, [_vp, _vp, _vp, _int, _vp, _vp, _vp, _vp] + [_i64] * 9 + [_vp]),
     "br_hip_flash_attn_bwd": (_int, [_vp] * 5 + [_int] + [_vp] * 7 + [_int] + [_i64] * 9 + [_vp]),

@@ -349,6 +349,48 @@ int br_hip_gemm_staged(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k
                        const float* bias, int64_t batch, int compute,
                        void* workspace, size_t workspace_bytes, br_stream_t stream);
 
+/* Two products, with the column sums of a matrix before them (sums may be
+ * null): what br_hip_colsum(sums), br_hip_gemm_staged(first) and
+ * br_hip_gemm_staged(second) do one after the other (br_hip_gemm in place of the
+ * latter with BR_GEMM_F32), for the operators that multiply one gradient twice:
+ * op_linear_backward (cuda_tensor.cpp:565-622), op_attn_backward and
+ * op_qk_backward (:670-800).  Nothing accumulates and there is no bias.  Where
+ * the sizes are small, one of them has both operands row-contiguous and an fp32
+ * C (trans_a = 1, trans_b = 0), the other has trans_a = 0, and none writes what
+ * another reads or writes, all of it is ONE launch; results then differ from the
+ * separate calls' in the order of the fp32 sums alone.  The same arguments
+ * always take the same way.  br_hip_gemm_pair_kernel tells which kernel the one
+ * launch runs on (BR_GEMM_FLEX_*), or -1 where there are several; sizes decide. */
+typedef struct br_product {
+    int trans_a, trans_b;
+    int64_t m, n, k;
+    float alpha;
+    const void* a;
+    int a_dtype;
+    int64_t lda, stride_a;
+    const void* b;
+    int b_dtype;
+    int64_t ldb, stride_b;
+    void* c;
+    int c_dtype;
+    int64_t ldc, stride_c;
+    int64_t batch;
+} br_product;
+typedef struct br_column_sums {
+    const void* x;       /* [rows, cols], dense */
+    int dtype;
+    float* out;          /* out[c] = scale * sum_r x[r, c] */
+    int64_t rows, cols;
+    float scale;
+    void* workspace;     /* br_hip_colsum_workspace(rows, cols) bytes */
+    size_t workspace_bytes;
+} br_column_sums;
+size_t br_hip_gemm_pair_workspace(const br_product* first, const br_product* second, int compute);
+int br_hip_gemm_pair(const br_product* first, const br_product* second, const br_column_sums* sums, int compute,
+                     void* workspace, size_t workspace_bytes, br_stream_t stream);
+int br_hip_gemm_pair_kernel(int64_t m1, int64_t n1, int64_t k1, int64_t batch1, int64_t m2, int64_t n2, int64_t k2,
+                            int64_t batch2, int compute);
+
 /* The kernel a 16-bit product runs on, for callers (and tests) that want to
  * know: of br_hip_gemm, or with `staged` of br_hip_gemm_staged and the workspace
  * it asks for, for aligned operands of the compute type.  *slices receives the

@@ -27,7 +27,7 @@ PLANNED = [
     ("flex 64", 4, 488, 512, 8200, 1), ("flex 64 short", 1, 488, 4104, 2048, 1), ("flex 64 short", 1, 488, 4104, 520, 1),
     ("flex 32x64", 1, 488, 2048, 64, 1), ("flex 32x64", 1, 488, 2048, 72, 1), ("flex 32", 1, 488, 512, 72, 1),
     ("flex 32", 4, 64, 1024, 4096, 1), ("ring 64x128", 1, 488, 4096, 2048, 1), ("ring 64x128", 1, 488, 4096, 520, 1),
-    ("ring 64x128", 4, 64, 4096, 8200, 1),
+    ("ring 64x128", 4, 64, 4096, 8200, 1), ("flex 32", 4, 47, 896, 2688, 1), ("flex 32x64", 8, 41, 1152, 3456, 1),
 ]
 
 

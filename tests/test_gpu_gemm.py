@@ -671,3 +671,87 @@ def test_gemm_of_more_batch_entries_than_a_launch_has_work_items():
          batch, hip.GEMM_F32, stream())
     torch.cuda.synchronize()
     assert float(c.min()) == float(c.max()) == k
+
+
+def whole_numbers(shape, most, dtype):
+    return torch.randint(-most, most + 1, shape, device="cuda").to(TORCH_T[dtype])
+
+
+def run_pair(products, compute, sums=None):
+    """br_hip_gemm_pair on (trans_a, trans_b, a, b, c) with [batch, rows, cols] tensors; whether it was one launch."""
+    code = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
+    descs, sizes = [], []
+    for ta, tb, a, b, c in products:
+        m, n, k = c.shape[1], c.shape[2], a.shape[1] if ta else a.shape[2]
+        descs.append(hip.Product(ta, tb, m, n, k, 2.0, ptr(a), code[a.dtype], a.shape[2], a[0].numel(), ptr(b), code[b.dtype],
+                                 b.shape[2], b[0].numel(), ptr(c), code[c.dtype], n, m * n, c.shape[0]))
+        sizes += [m, n, k, c.shape[0]]
+    first, second = (ctypes.byref(d) for d in descs)
+    need = hip.load().br_hip_gemm_pair_workspace(first, second, compute)
+    ws = torch.full((max(need, 16),), 0x7f, dtype=torch.uint8, device="cuda")
+    call("br_hip_gemm_pair", first, second, ctypes.byref(sums) if sums else None, compute, ptr(ws), need, stream())
+    torch.cuda.synchronize()
+    return hip.load().br_hip_gemm_pair_kernel(*sizes, compute) >= 0
+
+
+def pair_reference(ta, tb, a, b):
+    a, b = a.double(), b.double()
+    return 2 * torch.bmm(a.transpose(1, 2).contiguous() if ta else a, b.transpose(1, 2).contiguous() if tb else b)
+
+
+COMPUTE_T = {hip.GEMM_F16: F16, hip.GEMM_BF16: BF16, hip.GEMM_F32: F32}
+
+
+@pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16, hip.GEMM_F32])
+@pytest.mark.parametrize("n,inn,out,x_dt", [
+    (1, 8, 8, None), (64, 256, 1024, None), (65, 1032, 264, None), (333, 136, 520, F32), (40, 2560, 640, F32), (516, 640, 640, None),
+    (830, 640, 2560, F32), (700, 4096, 4096, None)])
+def test_two_products_of_a_linear_layer_in_one_launch_are_exact_on_integers(n, inn, out, x_dt, compute):
+    """dW = dy^T x, dx = dy W and the column sums of dy, every tile the rule picks and its remainders; the largest is two
+    launches.  x and W in the products' type or as fp32 that is converted first; dx in either type."""
+    dt = COMPUTE_T[compute]
+    print("case n=%d in=%d out=%d compute=%d" % (n, inn, out, compute), flush=True)
+    torch.manual_seed(n)
+    for dx_dt in {dt, F32}:
+        dy, x, w = whole_numbers((1, n, out), 1, dt), whole_numbers((1, n, inn), 1, x_dt or dt), whole_numbers((1, out, inn), 1, x_dt or dt)
+        dw = torch.full((1, out, inn), float("nan"), device="cuda")
+        dx = torch.full((1, n, inn), float("nan"), device="cuda", dtype=TORCH_T[dx_dt])
+        db = torch.full((out,), float("nan"), device="cuda")
+        need = hip.load().br_hip_colsum_workspace(n, out)
+        ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+        sums = hip.ColumnSums(ptr(dy), dt, ptr(db), n, out, 0.5, ptr(ws), need)
+        assert run_pair([(1, 0, dy, x, dw), (0, 0, dy, w, dx)], compute, sums) == (n != 700) or compute == hip.GEMM_F32
+        assert torch.equal(dw, pair_reference(1, 0, dy, x).float())
+        assert torch.equal(dx, pair_reference(0, 0, dy, w).to(dx.dtype))
+        assert torch.equal(db, 0.5 * dy[0].float().sum(0))
+
+
+@pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16, hip.GEMM_F32])
+@pytest.mark.parametrize("bh,t,hd,p_dt", [(2, 4, 64, None), (6, 40, 64, F32), (5, 50, 96, None), (3, 250, 128, None), (40, 120, 128, F32)])
+def test_two_products_of_attention_in_one_launch_are_exact_on_integers(bh, t, hd, p_dt, compute):
+    """dV = P^T dO with dP = dO V^T, and dQ = dS K with dK = dS^T Q in that order; rows of T values that are no multiple of a
+    granule are copied once for both."""
+    dt = COMPUTE_T[compute]
+    print("case bh=%d t=%d hd=%d compute=%d" % (bh, t, hd, compute), flush=True)
+    torch.manual_seed(t)
+    p, d_o, v = whole_numbers((bh, t, t), 1, p_dt or dt), whole_numbers((bh, t, hd), 1, dt), whole_numbers((bh, t, hd), 1, p_dt or dt)
+    dv, dq = (torch.full((bh, t, hd), float("nan"), device="cuda") for _ in range(2))
+    dp = torch.full((bh, t, t), float("nan"), device="cuda")
+    assert run_pair([(1, 0, p, d_o, dv), (0, 1, d_o, v, dp)], compute)
+    assert torch.equal(dv, pair_reference(1, 0, p, d_o).float()) and torch.equal(dp, pair_reference(0, 1, d_o, v).float())
+    dv.fill_(float("nan"))
+    assert run_pair([(0, 0, p, v, dq), (1, 0, p, d_o, dv)], compute)
+    assert torch.equal(dq, pair_reference(0, 0, p, v).float()) and torch.equal(dv, pair_reference(1, 0, p, d_o).float())
+
+
+@pytest.mark.parametrize("staged", [False, True])
+def test_two_products_keep_their_order_where_one_overwrites_the_others_operand(staged):
+    """dx over x, as the model's scripts have it: the weight gradient is formed from x as it was."""
+    torch.manual_seed(7)
+    n, inn, out = 72, 256, 512
+    dy, w = whole_numbers((1, n, out), 1, F16), whole_numbers((1, out, inn), 1, F16)
+    x = whole_numbers((1, n, inn), 1, F32 if staged else F16)
+    dw = torch.empty((1, out, inn), device="cuda")
+    want = pair_reference(1, 0, dy, x).float()
+    assert run_pair([(1, 0, dy, x, dw), (0, 0, dy, w, x)], hip.GEMM_F16)   # one launch by its sizes
+    assert torch.equal(dw, want) and torch.equal(x, pair_reference(0, 0, dy, w).to(x.dtype))
