@@ -402,6 +402,17 @@ __device__ __forceinline__ float to_f32<BR_GEMM_F16>(u16 x) { return (float)__bu
 template <>
 __device__ __forceinline__ float to_f32<BR_GEMM_BF16>(u16 x) { return __uint_as_float((unsigned)x << 16); }
 
+// sum + the products of eight pairs of 16-bit values
+template <int CT>
+__device__ __forceinline__ float dot8(const u32x4& x, const u32x4& y, float sum = 0.f) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        sum += to_f32<CT>((u16)(x[j] & 0xffffu)) * to_f32<CT>((u16)(y[j] & 0xffffu));
+        sum += to_f32<CT>((u16)(x[j] >> 16)) * to_f32<CT>((u16)(y[j] >> 16));
+    }
+    return sum;
+}
+
 // One LDS stage of the query loop of the dK / dV pass: a Q tile, a dO tile and
 // the tile's lse and delta values.
 constexpr int kQStageBytes = 2 * kTileBytes + 2 * kBK * 4;
@@ -416,19 +427,20 @@ constexpr int kQStageBytes = 2 * kTileBytes + 2 * kBK * 4;
 // (G, QH) = (4, 1): 128 keys per workgroup, 32 per wave, every query of a tile.  (2, 2): 64 keys per workgroup; wave
 // (kg, qh) has the keys of group kg = wave % 2 and queries 32 * qh .. + 31 of every query tile; the two partial dK
 // and dV of a key group are added through LDS at the end.
-template <int CT, int G, int QH>
-__global__ __launch_bounds__(64 * G * QH) void flash_bwd_dkv_kernel(FlashArgs a) {
+// OWN_DELTA: delta is formed here, tile by tile, instead of read from the dQ pass's, so that the passes can run side by
+// side: four threads take a query's dO and O, 64 bytes of each a thread, ahead of the tile before it.
+template <int CT, int G, int QH, bool OWN_DELTA>
+__device__ __forceinline__ void flash_bwd_dkv(const FlashArgs& a, int id, unsigned char* lds) {
     static_assert(G * QH == 4, "TileFill deals a tile to four waves");
     constexpr int BKEYS = 32 * G;      // keys per workgroup
     constexpr int NQB = 2 / QH;        // 32-query blocks of a tile per wave
     constexpr int kSpan = kBK / QH;    // queries of a tile per wave
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kQStageBytes];
     static_assert(QH == 1 || 2 * kQStageBytes >= G * 2 * 64 * 64 * 4, "the merge puts 2 G blocks of 64 x 64 floats into the stages");
     const int lane = threadIdx.x & 63, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: branches on it are scalar
     const int kg = QH == 1 ? wave : wave % G, qh = QH == 1 ? 0 : wave / G;
-    const int bh = (int)(blockIdx.x % a.batch_heads), b = bh / a.heads, h = bh % a.heads;
-    const int kt = (int)(blockIdx.x / a.batch_heads);  // key tile 0 meets the most queries: longest first
+    const int bh = id % a.batch_heads, b = bh / a.heads, h = bh % a.heads;
+    const int kt = id / a.batch_heads;  // key tile 0 meets the most queries: longest first
     const long long base = (long long)b * a.batch_stride + (long long)h * a.head;
     const long long obase = (long long)b * a.obatch + (long long)h * a.head;
     const int valid = a.valid[b] < a.tokens ? a.valid[b] : a.tokens;
@@ -470,21 +482,47 @@ __global__ __launch_bounds__(64 * G * QH) void flash_bwd_dkv_kernel(FlashArgs a)
         q_fill.fill(st, a.q + base, a.row, r0, a.tokens, wave);
         g_fill.fill(st + kTileBytes, a.d_o + obase, a.orow, r0, a.tokens, wave);
         fill_row(st + 2 * kTileBytes, a.lse + (long long)bh * a.tokens, r0, a.tokens, lane);
-        fill_row(st + 2 * kTileBytes + kBK * 4, a.delta + (long long)bh * a.tokens, r0, a.tokens, lane);
+        if (!OWN_DELTA) fill_row(st + 2 * kTileBytes + kBK * 4, a.delta + (long long)bh * a.tokens, r0, a.tokens, lane);
     };
-    if (ntiles > 0) issue(0, 0);
+    u32x4 own_g[4], own_o[4];
+    auto take_rows = [&](int t) {
+        const int r0 = q_begin + t * kBK, r = r0 + (int)(threadIdx.x >> 2);
+        const long long at = obase + (long long)(r < a.tokens ? r : a.tokens - 1) * a.orow + (threadIdx.x & 3) * 32;
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            own_g[c] = *reinterpret_cast<const u32x4*>(a.d_o + at + c * 8);
+            own_o[c] = *reinterpret_cast<const u32x4*>(a.o + at + c * 8);
+        }
+    };
+    auto leave_delta = [&](unsigned stage_bytes) {
+        float d = 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; c++) d += dot8<CT>(own_g[c], own_o[c]);
+        d += __shfl_xor(d, 1, kWave);
+        d += __shfl_xor(d, 2, kWave);
+        if ((threadIdx.x & 3) == 0)
+            reinterpret_cast<float*>(lds + stage_bytes + 2 * kTileBytes)[kBK + (threadIdx.x >> 2)] = d;
+    };
+    if (ntiles > 0) {
+        if (OWN_DELTA) take_rows(0);
+        issue(0, 0);
+    }
 #pragma unroll
     for (int ks = 0; ks < 8; ks++) {
         landed(kf[ks]);
         landed(vf[ks]);
     }
     landed(bias);
+    if (OWN_DELTA && ntiles > 0) leave_delta(0);
     wait_vmem<0>();
     __syncthreads();
     auto tile_step = [&](auto stage_c, int t) {
         constexpr int kStage = decltype(stage_c)::value * kQStageBytes;
         const int q0 = q_begin + t * kBK + qh * 32;   // this wave's first query of the tile
-        if (t + 1 < ntiles) issue(t + 1, kQStageBytes - kStage);
+        if (t + 1 < ntiles) {
+            if (OWN_DELTA) take_rows(t + 1);
+            issue(t + 1, kQStageBytes - kStage);
+        }
         const float* tl = reinterpret_cast<const float*>(lds + kStage + 2 * kTileBytes) + qh * 32 + half * 4;
         const float* td = tl + kBK;
         // queries that all precede this wave's keys see none of them
@@ -549,6 +587,7 @@ __global__ __launch_bounds__(64 * G * QH) void flash_bwd_dkv_kernel(FlashArgs a)
                 }
             }
         }
+        if (OWN_DELTA && t + 1 < ntiles) leave_delta(kQStageBytes - kStage);
         wait_vmem<0>();   // this wave's part of tile t + 1 is in
         __syncthreads();
     };
@@ -613,25 +652,30 @@ __global__ __launch_bounds__(64 * G * QH) void flash_bwd_dkv_kernel(FlashArgs a)
     }
 }
 
+template <int CT, int G, int QH>
+__global__ __launch_bounds__(64 * G * QH) void flash_bwd_dkv_kernel(FlashArgs a) {
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kQStageBytes];
+    flash_bwd_dkv<CT, G, QH, false>(a, (int)blockIdx.x, lds);
+}
+
 // dQ of 128 queries (32 per wave) of one (batch, head): the forward's loop over
 // key tiles, with  S^T = K . Q^T,  dP^T = V . dO^T  and
 // dQ^T[d, query] += K^T . dS^T  (K^T by transposing reads of the K tile).
 // (G, KH) = (2, 2): 64 queries per workgroup, the keys of every tile split between two waves as in the forward
 // kernel; the two partial dQ of a query group are added through LDS at the end.
 template <int CT, int G, int KH>
-__global__ __launch_bounds__(64 * G * KH, 2) void flash_bwd_dq_kernel(FlashArgs a) {
+__device__ __forceinline__ void flash_bwd_dq(const FlashArgs& a, int id, unsigned char* lds) {
     static_assert(G * KH == 4, "TileFill deals a tile to four waves");
     constexpr int BQ = 32 * G;
     constexpr int NKB = 2 / KH;
     constexpr int kSpan = kBK / KH;
-    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kStageBytes];
     static_assert(2 * kStageBytes >= G * 64 * 64 * 4, "the merge puts G blocks of 64 x 64 floats into the stages");
     const int lane = threadIdx.x & 63, half = lane >> 5;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform: branches on it are scalar
     const int qg = KH == 1 ? wave : wave % G, kh = KH == 1 ? 0 : wave / G;
     const int tiles_q = (a.tokens + BQ - 1) / BQ;
-    const int bh = (int)(blockIdx.x % a.batch_heads), b = bh / a.heads, h = bh % a.heads;
-    const int qt = tiles_q - 1 - (int)(blockIdx.x / a.batch_heads);
+    const int bh = id % a.batch_heads, b = bh / a.heads, h = bh % a.heads;
+    const int qt = tiles_q - 1 - id / a.batch_heads;
     const long long base = (long long)b * a.batch_stride + (long long)h * a.head;
     const int valid = a.valid[b] < a.tokens ? a.valid[b] : a.tokens;
     const int q0 = qt * BQ + qg * 32;
@@ -651,11 +695,7 @@ __global__ __launch_bounds__(64 * G * KH, 2) void flash_bwd_dq_kernel(FlashArgs 
     for (int ks = 0; ks < 8; ks++) {
         gf[ks] = *reinterpret_cast<const u32x4*>(a.d_o + orow + ks * 16 + half * 8);
         const u32x4 y = *reinterpret_cast<const u32x4*>(a.o + orow + ks * 16 + half * 8);
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            delta += to_f32<CT>((u16)(gf[ks][j] & 0xffffu)) * to_f32<CT>((u16)(y[j] & 0xffffu));
-            delta += to_f32<CT>((u16)(gf[ks][j] >> 16)) * to_f32<CT>((u16)(y[j] >> 16));
-        }
+        delta = dot8<CT>(gf[ks], y, delta);
     }
     delta += __shfl_xor(delta, 32, kWave);
     if (half == 0 && kh == 0 && query < a.tokens) a.delta[(long long)bh * a.tokens + query] = delta;
@@ -798,6 +838,21 @@ __global__ __launch_bounds__(64 * G * KH, 2) void flash_bwd_dq_kernel(FlashArgs 
     }
 }
 
+template <int CT, int G, int KH>
+__global__ __launch_bounds__(64 * G * KH, 2) void flash_bwd_dq_kernel(FlashArgs a) {
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[2 * kStageBytes];
+    flash_bwd_dq<CT, G, KH>(a, (int)blockIdx.x, lds);
+}
+
+// Both passes of a small launch side by side: workgroups [0, n) sum dK and dV of 64 keys each, as many more dQ of 64 queries.
+template <int CT>
+__global__ __launch_bounds__(kThreads) void flash_bwd_both_kernel(FlashArgs a, unsigned n) {
+    constexpr int kBytes = 2 * (kQStageBytes > kStageBytes ? kQStageBytes : kStageBytes);
+    __shared__ __attribute__((aligned(1024))) unsigned char lds[kBytes];
+    if (blockIdx.x < n) flash_bwd_dkv<CT, 2, 2, true>(a, (int)blockIdx.x, lds);
+    else flash_bwd_dq<CT, 2, 2>(a, (int)(blockIdx.x - n), lds);
+}
+
 // Whether a launch that would take `workgroups` workgroups of 128 queries (or keys) runs on twice as many of 64
 // instead, each tile's work split between two waves: where the wider ones would leave compute units empty or with
 // one workgroup each.  Measured at 32 heads x 512 tokens, batch 1 / 2 / 4 (128 / 256 / 512 wide workgroups), wide
@@ -812,6 +867,19 @@ __global__ __launch_bounds__(64 * G * KH, 2) void flash_bwd_dq_kernel(FlashArgs 
 #endif
 inline bool narrow_split(unsigned workgroups) { return workgroups <= (unsigned)BR_FA_SPLIT_UP_TO; }
 inline bool narrow_split_dkv(unsigned workgroups) { return workgroups < (unsigned)BR_FA_DKV_SPLIT_BELOW; }
+// Long sequences in a little over a round of wide workgroups: the first key tile's walk is the whole pass, so both
+// backward passes run narrow (wide / narrow, us: 32 heads x 1024 78.2 / 74.3, 16 x 2048 133.5 / 112.0, 24 x 1536 124.7 /
+// 105.7, 20 x 2000 160.1 / 140.4; 64 x 600 68.2 / 73.9, 64 x 1024 113 / 130, 32 x 2048 185 / 198).
+inline bool long_walk(unsigned workgroups, int64_t tokens) { return workgroups <= 320 && tokens >= 896; }
+
+// Both passes in one launch (of narrow workgroups, one to a CU): up to three rounds of them.  us as two launches / as one:
+// 2 heads x 32 tokens 16.1 / 9.8, 8 x 78 20.6 / 12.9, 32 x 256 26.5 / 17.1 (256 workgroups), 48 x 192 24.1 / 18.5 (288),
+// 32 x 512 37.1 / 32.1 (512), 48 x 334 34.5 / 32.7 (576), 320 x 64 32.4 / 27.1 (640), 96 x 200 37.8 / 34.8 (768), 48 x 550
+// 51.3 / 56.7 (864), 224 x 128 35.5 / 39.5 (896), 96 x 300 43.9 / 47.8 (960).
+#ifndef BR_FA_BOTH_UP_TO
+#define BR_FA_BOTH_UP_TO 768
+#endif
+inline bool both_at_once(unsigned workgroups) { return workgroups <= (unsigned)BR_FA_BOTH_UP_TO; }
 
 bool flash_shape_ok(int64_t batch, int64_t heads, int64_t tokens, int64_t head_dim, int64_t row, int64_t head,
                     int64_t batch_stride, int64_t orow, int64_t obatch) {
@@ -918,7 +986,14 @@ int br_hip_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
     const unsigned tiles = (unsigned)(((tokens + kBQ - 1) / kBQ) * batch * heads);
     // the dQ pass first: it leaves delta behind for the dK / dV pass
     const unsigned tiles2 = (unsigned)(((tokens + 63) / 64) * batch * heads);
-    const bool split_q = narrow_split(tiles), split_kv = narrow_split_dkv(tiles);
+    const bool walk = long_walk(tiles, tokens);
+    const bool split_q = walk || narrow_split(tiles), split_kv = walk || narrow_split_dkv(tiles);
+    if (both_at_once(2 * tiles2)) {
+        if (dtype == BR_F16) flash_bwd_both_kernel<BR_GEMM_F16><<<2 * tiles2, kThreads, 0, st>>>(a, tiles2);
+        else flash_bwd_both_kernel<BR_GEMM_BF16><<<2 * tiles2, kThreads, 0, st>>>(a, tiles2);
+        BR_HIP_LAUNCH_CHECK();
+        return BR_OK;
+    }
     if (dtype == BR_F16) {
         if (split_q) flash_bwd_dq_kernel<BR_GEMM_F16, 2, 2><<<tiles2, kThreads, 0, st>>>(a);
         else flash_bwd_dq_kernel<BR_GEMM_F16, 4, 1><<<tiles, kThreads, 0, st>>>(a);
