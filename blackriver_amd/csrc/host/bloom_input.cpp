@@ -42,22 +42,34 @@ void BloomInput::build_xmask(const int32_t* mask, int64_t batch, int64_t tokens,
 
 namespace {
 
+// Host words to the device: as kernel arguments, which waits for nothing, or where that would be many launches as a copy.
+int upload(int32_t* dst, const int32_t* src, int64_t n) {
+    if (n <= 4096) return br_hip_upload_words(dst, src, n, ComputingContext::stream);
+    return br_hip_memcpy_h2d(dst, src, (size_t)n * sizeof(int32_t), ComputingContext::stream);
+}
+
 struct Embed : public NativeWord {
     void run(Stack& stack) override {
         tensor_t out = stack.pop_tensor();
         tensor_t table = stack.pop_tensor();
         tensor_t ids = stack.pop_tensor();
         br_assert(ids->is_cpu() && ids->dtype() == DataType::Int, "bloom.embed: ids must be a cpu int tensor");
-        br_assert(table->is_cuda() && out->is_cuda() && table->dtype() == out->dtype(),
-                  "bloom.embed: table and out must be device tensors of one type");
+        const bool widens = out->dtype() == DataType::Float &&
+                            (table->dtype() == DataType::F16 || table->dtype() == DataType::BF16);
+        br_assert(table->is_cuda() && out->is_cuda() && (table->dtype() == out->dtype() || widens),
+                  "bloom.embed: table and out must be device tensors of one type, or out fp32 and the table 16 bit");
         const int64_t hidden = (int64_t)table->shape().vec().back();
         const int64_t vocab = (int64_t)table->items() / hidden;
         const int64_t n = (int64_t)out->items() / hidden;
         br_assert((int64_t)ids->items() >= n, "bloom.embed: not enough ids");
         int32_t* d_ids = static_cast<int32_t*>(ComputingContext::scratch((size_t)n * sizeof(int32_t)));
-        BR_HIP_CHECK(br_hip_memcpy_h2d(d_ids, ids->data(), (size_t)n * sizeof(int32_t), ComputingContext::stream));
-        BR_HIP_CHECK(br_hip_embedding_gather(table->data(), d_ids, out->data(), (int)DataType_size(table->dtype()), n,
-                                             hidden, vocab, ComputingContext::stream));
+        BR_HIP_CHECK(upload(d_ids, static_cast<const int32_t*>(ids->data()), n));
+        if (widens)
+            BR_HIP_CHECK(br_hip_embedding_gather_f32(table->data(), (int)table->dtype(), d_ids, static_cast<float*>(out->data()),
+                                                     n, hidden, vocab, ComputingContext::stream));
+        else
+            BR_HIP_CHECK(br_hip_embedding_gather(table->data(), d_ids, out->data(), (int)DataType_size(table->dtype()), n,
+                                                 hidden, vocab, ComputingContext::stream));
     }
     NWORD_CREATOR_DEFINE_LR(Embed)
 };
@@ -79,7 +91,7 @@ struct EmbedBackward : public NativeWord {
         const int64_t n = (int64_t)dx->items() / hidden;
         br_assert((int64_t)ids->items() >= n, "bloom.embed_backward: not enough ids");
         int32_t* d_ids = static_cast<int32_t*>(ComputingContext::scratch((size_t)n * sizeof(int32_t)));
-        BR_HIP_CHECK(br_hip_memcpy_h2d(d_ids, ids->data(), (size_t)n * sizeof(int32_t), ComputingContext::stream));
+        BR_HIP_CHECK(upload(d_ids, static_cast<const int32_t*>(ids->data()), n));
         BR_HIP_CHECK(br_hip_embedding_scatter_add(static_cast<const float*>(dx->data()), d_ids,
                                                   static_cast<float*>(grad->data()), n, hidden, vocab,
                                                   1.0f / ComputingContext::grad_lift, ComputingContext::stream));
@@ -108,8 +120,7 @@ struct XMask : public NativeWord {
         const int64_t batch = (int64_t)xmask->shape()[0], tokens = (int64_t)xmask->shape()[3];
         br_assert((int64_t)mask->items() >= batch * tokens, "bloom.xmask: mask too small");
         int32_t* d_mask = static_cast<int32_t*>(ComputingContext::scratch((size_t)(batch * tokens) * sizeof(int32_t)));
-        BR_HIP_CHECK(br_hip_memcpy_h2d(d_mask, mask->data(), (size_t)(batch * tokens) * sizeof(int32_t),
-                                       ComputingContext::stream));
+        BR_HIP_CHECK(upload(d_mask, static_cast<const int32_t*>(mask->data()), batch * tokens));
         BR_HIP_CHECK(br_hip_xmask_table(d_mask, static_cast<float*>(xmask->data()), batch, tokens,
                                         ComputingContext::stream));
     }
@@ -136,9 +147,7 @@ struct Valid : public NativeWord {
             while (n < tokens && m[b * tokens + n] != 0) n++;
             count[(size_t)b] = (int32_t)n;
         }
-        BR_HIP_CHECK(br_hip_memcpy_h2d(valid->data(), count.data(), (size_t)batch * sizeof(int32_t),
-                                       ComputingContext::stream));
-        ComputingContext::sync();  // `count` leaves scope; once per batch
+        BR_HIP_CHECK(br_hip_upload_words(valid->data(), count.data(), batch, ComputingContext::stream));
     }
     NWORD_CREATOR_DEFINE_LR(Valid)
 };

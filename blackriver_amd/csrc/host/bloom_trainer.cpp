@@ -7,10 +7,19 @@
 
 #include "br_hip.h"
 #include "common.hpp"
+#include "hip_tensor.hpp"
 #include "runtime.hpp"
 #include "tensor.hpp"
 
 namespace br {
+
+namespace {
+// op.loss_backward leaves its value to hip_finish_loss while one of these lives.
+struct LaterLoss {
+    LaterLoss() { ComputingContext::loss_later = true; }
+    ~LaterLoss() { ComputingContext::loss_later = false; }
+};
+}  // namespace
 
 BloomTrainer::BloomTrainer(Enviroment& env, const BloomModelConfig& cfg) : env_(env), cfg_(cfg) {
     br_assert(cfg.layers >= 1, "a model needs at least one block");
@@ -72,6 +81,11 @@ std::string BloomTrainer::setup_script() const {
     // for the gradient once every later block has finished, forward and backward).
     for (int i = 2; i <= cfg_.layers; i++) s << i - 1 << " # 'xa' @  " << i << " # 'xinput' !\n";
     for (int i = 1; i < cfg_.layers; i++) s << i + 1 << " # 'xa' @  " << i << " # 'yout_g' !\n";
+    // likewise between hash 0 and the first and the last block: the embedding LayerNorm writes the first block's xinput,
+    // the head reads the last block's xa and writes its yout_g
+    s << "0 # 'xinput' @  1 # 'xinput' !\n";
+    s << cfg_.layers << " # 'xa' @  0 # 'xa' !\n";
+    s << "0 # 'xc' @  " << cfg_.layers << " # 'yout_g' !\n";
     s << "0 #\n";
     return s.str();
 }
@@ -82,13 +96,10 @@ std::string BloomTrainer::step_script() const {
     const char* forward = flash() ? "layer_forward_flash" : mixed() ? "layer_forward_mixed" : "layer_forward";
     const char* backward = flash() ? "layer_backward_flash" : mixed() ? "layer_backward_mixed" : "layer_backward_core";
     s << "0 # model_input\n";
-    s << "1 # 'xinput' @  0 # 'xinput' @  op.copy   1 # " << forward << "\n";
-    for (int i = 2; i <= n; i++) s << i << " # " << forward << "\n";  // xinput is block i-1's xa
-    s << "0 # 'xa' @  " << n << " # 'xa' @  op.copy   0 # model_head\n";
-    s << n << " # 'yout_g' @  0 # 'xc' @  op.copy   " << n << " # " << backward << "\n";
-    for (int i = n - 1; i >= 1; i--) s << i << " # " << backward << "\n";  // yout_g is block i+1's xa
-    s << "0 # 'xb' @  1 # 'xa' @  op.copy   0 # model_input_backward\n";
-    s << "op.sync\n";
+    for (int i = 1; i <= n; i++) s << i << " # " << forward << "\n";  // xinput is block i-1's xa, or the model's xinput
+    s << "0 # model_head\n";
+    for (int i = n; i >= 1; i--) s << i << " # " << backward << "\n";  // yout_g is block i+1's xa, or the model's xc
+    s << "1 # 'xa' @  0 # model_input_backward_of\n";
     return s.str();
 }
 
@@ -169,7 +180,11 @@ float BloomTrainer::step(const int32_t* ids, const int32_t* mask) {
     // backward pass; the setting is this step's only (the context is global)
     ComputingContext::grad_lift_auto = cfg_.gemm_precision != "f32" && cfg_.gemm_precision != "float";
     ComputingContext::grad_lift = 1.0f;
-    env_.run(step_.get());
+    {
+        // the loss is read with the rest of what the step reads back, in its one wait for the device
+        LaterLoss later;
+        env_.run(step_.get());
+    }
     grad_lift_ = ComputingContext::grad_lift;
     ComputingContext::grad_lift_auto = false;
     ComputingContext::grad_lift = 1.0f;
@@ -177,15 +192,16 @@ float BloomTrainer::step(const int32_t* ids, const int32_t* mask) {
     // 65504 / lift, and every gradient further down the backward chain inherits it.  The embedding LayerNorm sits at
     // the bottom of that chain: its weight gradient (hidden floats) and the loss being finite means no activation
     // gradient of this step overflowed.
-    const float loss = ComputingContext::last_loss;
     tensor_t probe = env_.hash().find_tensor("word_embeddings_layernorm.weight_g");
-    std::vector<float> g((size_t)cfg_.hidden);
-    br_assert(probe->items() == g.size(), "embedding LayerNorm gradient has an unexpected size");
-    if (br_hip_memcpy_d2h(g.data(), probe->data(), g.size() * sizeof(float), ComputingContext::stream) != 0)
+    const size_t h = (size_t)cfg_.hidden;
+    br_assert(probe->items() == h, "embedding LayerNorm gradient has an unexpected size");
+    float* g = static_cast<float*>(ComputingContext::pinned(1, h * sizeof(float)));
+    if (br_hip_memcpy_d2h(g, probe->data(), h * sizeof(float), ComputingContext::stream) != 0)
         br_panic("BloomTrainer::step: reading back the embedding LayerNorm gradient failed");
     ComputingContext::sync();
+    const float loss = hip_finish_loss();
     bool finite = std::isfinite(loss);
-    for (float v : g) finite = finite && std::isfinite(v);
+    for (size_t i = 0; i < h; i++) finite = finite && std::isfinite(g[i]);
     if (!finite) {
         std::ostringstream why;
         why << "BloomTrainer::step: non-finite loss or gradient (loss " << loss << ", gradient lift " << grad_lift_

@@ -411,6 +411,27 @@ ComputingReturn HIPTensor<DT>::op_last_logits(tensor_t self, tensor_t mask_, ten
     return OP_OK;
 }
 
+namespace {
+// What the newest op_loss_backward has its value from: log p(label) of every position in pinned memory (the context's
+// slot 0, there once the stream has been waited for) and which of them count.
+struct LossRecord {
+    const float* logp = nullptr;
+    int64_t count = 0;
+    std::vector<int32_t> keep;
+} g_loss;
+}  // namespace
+
+float hip_finish_loss() {
+    double total = 0.0;
+    if (g_loss.count > 0)
+        for (size_t i = 0; i < g_loss.keep.size(); i++)
+            if (g_loss.keep[i]) total += (double)g_loss.logp[i];
+    const float ret = g_loss.count > 0 ? (float)(total / (double)g_loss.count) : 0.0f;
+    ComputingContext::last_loss = ret;
+    if (ComputingContext::echo_loss) std::cout << "#################  " << g_loss.count << " " << ret << std::endl;
+    return ret;
+}
+
 // ------------------------------------------------------------- backward
 // Shift-by-one masked cross entropy through the LM head, all on the device.
 // Integer part (on the host, from the CPU ids / mask tensors, bit-exact):
@@ -418,7 +439,7 @@ ComputingReturn HIPTensor<DT>::op_last_logits(tensor_t self, tensor_t mask_, ten
 //   its label is ids[t+1]; count = number of such positions.
 // Float part, per chunk of rows that fits `all_logits`:
 //   logits = x . W^T  ->  lse, log p(label)  ->  dlogits in place
-//   x_g = dlogits . W          (x_g is zeroed first)
+//   x_g = dlogits . W          (zero in chunks without a label)
 //   lm_head_g += dlogits^T . x
 // Returns +mean log-prob of the labels (the reference's sign convention).
 template <DataType DT>
@@ -441,7 +462,9 @@ TransformerComputing::loss_result_t HIPTensor<DT>::op_loss_backward(tensor_t sel
 
     const int* ids = static_cast<const int*>(ids_->data());
     const int* mask = static_cast<const int*>(mask_->data());
-    std::vector<int32_t> labels(n, -100), keep(n, 0);
+    std::vector<int32_t> labels(2 * n, -100);
+    int32_t* const keep = labels.data() + n;
+    std::fill(keep, keep + n, 0);
     int64_t count = 0;
     for (int64_t b = 0; b < batch; b++) {
         for (int64_t t = 0; t + 1 < tokens; t++) {
@@ -475,8 +498,12 @@ TransformerComputing::loss_result_t HIPTensor<DT>::op_loss_backward(tensor_t sel
     float* d_lse = reinterpret_cast<float*>(d_keep + n);
     float* d_logp = d_lse + n;
     float* d_result = d_logp + n;
-    BR_OP(br_hip_memcpy_h2d(d_labels, labels.data(), n * sizeof(int32_t), stream()));
-    BR_OP(br_hip_memcpy_h2d(d_keep, keep.data(), n * sizeof(int32_t), stream()));
+    // labels and keep lie next to each other, here and on the device
+    if (n <= 2048) {
+        BR_OP(br_hip_upload_words(d_labels, labels.data(), 2 * n, stream()));
+    } else {
+        BR_OP(br_hip_memcpy_h2d(d_labels, labels.data(), 2 * n * sizeof(int32_t), stream()));
+    }
 
     // weight gradient target: the tensor itself when it lives on the device,
     // otherwise a zeroed device staging buffer that is added into the CPU
@@ -491,7 +518,6 @@ TransformerComputing::loss_result_t HIPTensor<DT>::op_loss_backward(tensor_t sel
         BR_OP(br_hip_fill(d_wg, BR_F32, 0.f, vocab * hidden, stream()));
     }
 
-    BR_OP(br_hip_fill(x_g->data(), BR_F32, 0.f, n * hidden, stream()));
     const float* x = static_cast<const float*>(mem_);
     float* dx = static_cast<float*>(x_g->data());
     float* logits = static_cast<float*>(all_logits->data());
@@ -504,11 +530,16 @@ TransformerComputing::loss_result_t HIPTensor<DT>::op_loss_backward(tensor_t sel
     const bool overwrite_host = ComputingContext::loss_head_overwrite && !lm_head_g->is_cuda();
     bool overwrite = ComputingContext::loss_head_overwrite && lm_head_g->is_cuda();
     if (overwrite && count == 0) BR_OP(br_hip_fill(d_wg, BR_F32, 0.f, vocab * hidden, stream()));
+    // x_g is zero where no position carries a loss; the others' rows are written by their product
+    if (count == 0) BR_OP(br_hip_fill(dx, BR_F32, 0.f, n * hidden, stream()));
     for (int64_t r0 = 0; r0 < n && count > 0; r0 += cap) {
         const int64_t rows = std::min(cap, n - r0);
         bool any = false;
         for (int64_t r = r0; r < r0 + rows; r++) any = any || keep[r] != 0;
-        if (!any) continue;  // nothing but zero gradients in this chunk
+        if (!any) {  // nothing but zero gradients in this chunk
+            BR_OP(br_hip_fill(dx + r0 * hidden, BR_F32, 0.f, rows * hidden, stream()));
+            continue;
+        }
         BR_OP(product(0, 1, rows, vocab, hidden, 1.0f, x + r0 * hidden, BR_F32, hidden, 0, lm_head->data(),
                           code(lm_head), hidden, 0, 0, logits, BR_F32, vocab, 0, nullptr, 1, compute));
         BR_OP(br_hip_logsoftmax_nll_fwd(logits, d_labels + r0, d_keep + r0, d_lse + r0, d_logp + r0, d_result, rows,
@@ -549,12 +580,13 @@ TransformerComputing::loss_result_t HIPTensor<DT>::op_loss_backward(tensor_t sel
     if (overwrite && count > 0) BR_OP(br_hip_fill(d_wg, BR_F32, 0.f, vocab * hidden, stream()));
 
     // sum of log p(label) in fp64 on the host, as the reference accumulates it
-    std::vector<float> logp(n, 0.f);
-    if (count > 0) BR_OP(br_hip_memcpy_d2h(logp.data(), d_logp, n * sizeof(float), stream()));
-    ComputingContext::sync();
-    double total = 0.0;
-    for (int64_t i = 0; i < n; i++)
-        if (keep[i]) total += (double)logp[i];
+    float* logp = static_cast<float*>(ComputingContext::pinned(0, n * sizeof(float)));
+    if (count > 0) BR_OP(br_hip_memcpy_d2h(logp, d_logp, n * sizeof(float), stream()));
+    g_loss.logp = logp;
+    g_loss.count = count;
+    g_loss.keep.assign(keep, keep + n);
+    const bool later = ComputingContext::loss_later && !staging;
+    if (!later) ComputingContext::sync();
 
     if (staging) {
         float* host_g = static_cast<float*>(lm_head_g->data());
@@ -574,10 +606,7 @@ TransformerComputing::loss_result_t HIPTensor<DT>::op_loss_backward(tensor_t sel
         hip_tensor_free(staging);
     }
 
-    const float ret = count > 0 ? (float)(total / (double)count) : 0.0f;
-    ComputingContext::last_loss = ret;
-    if (ComputingContext::echo_loss) std::cout << "#################  " << count << " " << ret << std::endl;
-    return ret;
+    return later ? 0.0f : hip_finish_loss();
 }
 
 template <DataType DT>

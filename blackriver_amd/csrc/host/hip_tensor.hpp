@@ -71,6 +71,10 @@ private:
     const bool owner_;
 };
 
+// The value of the newest op_loss_backward (also left in ComputingContext::last_loss, and printed where losses are).  With
+// ComputingContext::loss_later the caller has waited for the stream first.
+float hip_finish_loss();
+
 // op_gelu_backward(dy, u, du) followed by op_linear_backward(du, x, ...): with a
 // 16-bit MFMA type one pass produces du, its 16-bit copy and the bias gradient
 // (same bits as the two operators), then the two products run.

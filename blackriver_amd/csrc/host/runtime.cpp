@@ -57,10 +57,13 @@ bool ComputingContext::echo_loss = true;
 float ComputingContext::grad_lift = 1.0f;
 bool ComputingContext::grad_lift_auto = false;
 bool ComputingContext::loss_head_overwrite = false;
+bool ComputingContext::loss_later = false;
 void* ComputingContext::scratch_ptr_ = nullptr;
 size_t ComputingContext::scratch_size_ = 0;
 void* ComputingContext::staging_ptr_[2] = {nullptr, nullptr};
 size_t ComputingContext::staging_size_[2] = {0, 0};
+void* ComputingContext::pinned_ptr_[2] = {nullptr, nullptr};
+size_t ComputingContext::pinned_size_[2] = {0, 0};
 
 void ComputingContext::boot(int dev) {
     br_assert(device < 0, "ComputingContext is already booted");
@@ -82,6 +85,9 @@ void ComputingContext::shutdown() {
         if (staging_ptr_[i]) BR_HIP_CHECK(br_hip_free(staging_ptr_[i]));
         staging_ptr_[i] = nullptr;
         staging_size_[i] = 0;
+        if (pinned_ptr_[i]) BR_HIP_CHECK(br_hip_host_free(pinned_ptr_[i]));
+        pinned_ptr_[i] = nullptr;
+        pinned_size_[i] = 0;
     }
     BR_HIP_CHECK(br_hip_free(workspace));
     BR_HIP_CHECK(br_hip_stream_destroy(stream));
@@ -121,6 +127,20 @@ void* ComputingContext::gemm_staging(int slot, size_t bytes) {
         staging_size_[slot] = bytes;
     }
     return staging_ptr_[slot];
+}
+
+void* ComputingContext::pinned(int slot, size_t bytes) {
+    br_assert(device >= 0, "ComputingContext is not booted");
+    br_assert(slot == 0 || slot == 1, "pinned slot");
+    if (bytes > pinned_size_[slot]) {
+        sync();   // a copy into the old block may be in flight
+        if (pinned_ptr_[slot]) BR_HIP_CHECK(br_hip_host_free(pinned_ptr_[slot]));
+        pinned_ptr_[slot] = nullptr;
+        pinned_size_[slot] = 0;
+        BR_HIP_CHECK(br_hip_host_malloc(&pinned_ptr_[slot], bytes));
+        pinned_size_[slot] = bytes;
+    }
+    return pinned_ptr_[slot];
 }
 
 // ----------------------------------------------------- CollectiveContext

@@ -950,6 +950,16 @@ __global__ __launch_bounds__(kBlock) void gather_rows_bytes(const unsigned char*
         out[row * row_bytes + i] = ok ? table[id * row_bytes + i] : (unsigned char)0;
 }
 
+// The same with 16-bit rows converted to fp32 on the way; one launch and one pass over the rows fewer than gathering and
+// then converting them.
+template <typename T>
+__global__ __launch_bounds__(kBlock) void gather_rows_f32(const T* table, const int32_t* ids, float* out, int64_t hidden, int64_t vocab) {
+    const int64_t row = blockIdx.x;
+    const int64_t id = ids[row];
+    const bool ok = id >= 0 && id < vocab;
+    for (int64_t i = threadIdx.x; i < hidden; i += kBlock) out[row * hidden + i] = ok ? (float)table[id * hidden + i] : 0.f;
+}
+
 // Rows picked by the host, named in the kernel's arguments: row i of out is x[at[i], :] as type D.  Grid (rows, pieces
 // of a row), VEC columns a thread.
 //
@@ -1576,6 +1586,23 @@ int br_hip_embedding_gather(const void* table, const int32_t* ids, void* out, in
     else
         gather_rows_bytes<<<(unsigned)n, kBlock, 0, st>>>((const unsigned char*)table, ids, (unsigned char*)out,
                                                           row_bytes, vocab);
+    BR_HIP_LAUNCH_CHECK();
+    return BR_OK;
+}
+
+int br_hip_embedding_gather_f32(const void* table, int table_dtype, const int32_t* ids, float* out, int64_t n,
+                                int64_t hidden, int64_t vocab, br_stream_t stream) {
+    if (n < 0 || hidden <= 0 || vocab <= 0) return BR_ERR_ATTR;
+    if (table_dtype != BR_F16 && table_dtype != BR_BF16) return BR_ERR_TODO;
+    if (n == 0) return BR_OK;
+    if (!table || !ids) return BR_ERR_INPUT;
+    if (!out) return BR_ERR_OUTPUT;
+    if (n > 0xffffff) return BR_ERR_ATTR;
+    hipStream_t st = as_stream(stream);
+    if (table_dtype == BR_F16)
+        gather_rows_f32<__half><<<(unsigned)n, kBlock, 0, st>>>((const __half*)table, ids, out, hidden, vocab);
+    else
+        gather_rows_f32<__hip_bfloat16><<<(unsigned)n, kBlock, 0, st>>>((const __hip_bfloat16*)table, ids, out, hidden, vocab);
     BR_HIP_LAUNCH_CHECK();
     return BR_OK;
 }

@@ -4,6 +4,7 @@
 #include "common.hpp"
 
 #include <math.h>
+#include <string.h>
 
 using namespace brk;
 
@@ -23,6 +24,17 @@ __global__ __launch_bounds__(256) void memset_kernel(unsigned char* dst, unsigne
     const size_t tail0 = lead + vecs * 16;
     for (size_t i = tid; i < lead; i += stride) dst[i] = value;
     for (size_t i = tail0 + tid; i < bytes; i += stride) dst[i] = value;
+}
+
+// Host words that travel in the kernel's arguments.  A copy of pageable memory holds the caller up until the device has
+// caught up with it; the arguments of a launch are taken over when it is enqueued.
+constexpr int kUploadWords = 960;   // with the other arguments less than the 4 KB a launch takes
+struct UploadWords {
+    uint32_t w[kUploadWords];
+};
+__global__ __launch_bounds__(256) void upload_kernel(UploadWords words, int count, uint32_t* __restrict__ dst) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < count) dst[i] = words.w[i];
 }
 
 }  // namespace
@@ -126,6 +138,21 @@ int br_hip_event_elapsed_ms(br_event_t start, br_event_t stop, float* ms) {
 int br_hip_memcpy_h2d(void* dst, const void* src, size_t bytes, br_stream_t stream) {
     if (bytes == 0) return BR_OK;
     BR_HIP_TRY(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, as_stream(stream)));
+    return BR_OK;
+}
+
+int br_hip_upload_words(void* dst, const void* src, int64_t count, br_stream_t stream) {
+    if (count < 0) return BR_ERR_ATTR;
+    if (count == 0) return BR_OK;
+    if (!src) return BR_ERR_INPUT;
+    if (!dst || (reinterpret_cast<uintptr_t>(dst) & 3u) != 0) return BR_ERR_OUTPUT;
+    UploadWords words;
+    for (int64_t at = 0; at < count; at += kUploadWords) {
+        const int n = (int)(count - at < kUploadWords ? count - at : kUploadWords);
+        memcpy(words.w, static_cast<const char*>(src) + at * 4, (size_t)n * 4);
+        upload_kernel<<<(n + 255) / 256, 256, 0, as_stream(stream)>>>(words, n, static_cast<uint32_t*>(dst) + at);
+        BR_HIP_LAUNCH_CHECK();
+    }
     return BR_OK;
 }
 

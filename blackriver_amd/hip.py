@@ -54,6 +54,7 @@ SIGNATURES = {
     "br_hip_event_sync": (_int, [_vp]),
     "br_hip_event_elapsed_ms": (_int, [_vp, _vp, ctypes.POINTER(_f32)]),
     "br_hip_memcpy_h2d": (_int, [_vp, _vp, _sz, _vp]),
+    "br_hip_upload_words": (_int, [_vp, _vp, _i64, _vp]),
     "br_hip_memcpy_d2h": (_int, [_vp, _vp, _sz, _vp]),
     "br_hip_memcpy_d2d": (_int, [_vp, _vp, _sz, _vp]),
     "br_hip_memset": (_int, [_vp, _int, _sz, _vp]),
@@ -105,6 +106,7 @@ SIGNATURES = {
     "br_hip_adamw": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _i64, _f32, _f32, _f32, _f32, _f32, _i64, _vp]),
     "br_hip_adamw_group": (_int, [_vp, _i64, _f32, _f32, _f32, _f32, _f32, _i64, _vp]),
     "br_hip_embedding_gather": (_int, [_vp, _vp, _vp, _int, _i64, _i64, _i64, _vp]),
+    "br_hip_embedding_gather_f32": (_int, [_vp, _int, _vp, _vp, _i64, _i64, _i64, _vp]),
     "br_hip_pick_rows": (_int, [_vp, _vp, _vp, _int, _i64, _i64, _vp]),
     "br_hip_embedding_scatter_add": (_int, [_vp, _vp, _vp, _i64, _i64, _i64, _f32, _vp]),
     "br_hip_alibi_table": (_int, [_vp, _i64, _i64, _vp]),

@@ -70,6 +70,10 @@ int br_hip_event_elapsed_ms(br_event_t start, br_event_t stop, float* ms);
 /* cudaMemcpyAsync in cuda_tensor.cpp:135,139 and cpu_tensor.cpp:31, and
  * cudaMemset in cuda_tensor.cpp:104.  Asynchronous on `stream`. */
 int br_hip_memcpy_h2d(void* dst, const void* src, size_t bytes, br_stream_t stream);
+/* `count` 32-bit words of host memory to the device, read before the call
+ * returns and without waiting for the stream (they travel as kernel arguments,
+ * 960 a launch: for the ids and masks of a batch). */
+int br_hip_upload_words(void* dst, const void* src, int64_t count, br_stream_t stream);
 int br_hip_memcpy_d2h(void* dst, const void* src, size_t bytes, br_stream_t stream);
 int br_hip_memcpy_d2d(void* dst, const void* src, size_t bytes, br_stream_t stream);
 int br_hip_memset(void* dst, int byte_value, size_t bytes, br_stream_t stream);
@@ -518,6 +522,9 @@ int br_hip_adamw_group(const br_adamw_tensor* tensors, int64_t count, float lr, 
 /* The embedding row gather of blackriver/train_bloom.cpp:50-56. */
 int br_hip_embedding_gather(const void* table, const int32_t* ids, void* out, int elem_bytes,
                             int64_t n, int64_t hidden, int64_t vocab, br_stream_t stream);
+/* The same with the rows converted on the way (16-bit table, fp32 out). */
+int br_hip_embedding_gather_f32(const void* table, int table_dtype, const int32_t* ids, float* out, int64_t n,
+                                int64_t hidden, int64_t vocab, br_stream_t stream);
 /* out[i, :] = x[rows[i], :] as out_dtype, rows being a host array that is read
  * before the call returns: the last-token rows of cuda_tensor.cpp:424-432. */
 int br_hip_pick_rows(const float* x, const int64_t* rows, void* out, int out_dtype, int64_t n, int64_t cols,
