@@ -79,6 +79,7 @@ int product(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alp
 }
 
 // Column sums and the two products of a backward operator, in this order or, where they are small, as one launch.
+// Operands that have to be converted are, in one launch, and once where both products read them.
 int two_products(const br_product& first, const br_product& second, const br_column_sums* sums, int compute) {
     const size_t need = br_hip_gemm_pair_workspace(&first, &second, compute);
     void* ws = need ? ComputingContext::gemm_staging(0, need) : nullptr;
@@ -703,8 +704,7 @@ ComputingReturn HIPTensor<DT>::op_attn_backward(tensor_t self, tensor_t attn, te
     if (!dev(attn_g) || !dev(v_g) || attn_g->items() != attn->items() || v_g->items() != v->items())
         return OP_OUTPUT_ERROR;
     const int compute = pick_compute({self, attn, v});
-    const Operand d_o = shared_operand(mem_, (int)DT, d.bh * d.t * d.hd, compute);
-    BR_OP(attn_products(d_o, attn, v, attn_g->data(), code(attn_g), v_g, d, compute));
+    BR_OP(attn_products(Operand{mem_, (int)DT}, attn, v, attn_g->data(), code(attn_g), v_g, d, compute));
     return OP_OK;
 }
 
@@ -745,9 +745,8 @@ ComputingReturn HIPTensor<DT>::op_softmax_attn_backward(tensor_t self, tensor_t 
     if (!dev_f32(attn_g) || !dev(v_g) || attn_g->items() != attn->items() || v_g->items() != v->items())
         return OP_OUTPUT_ERROR;
     const int compute = pick_compute({self, attn, v});
-    const Operand d_o = shared_operand(mem_, (int)DT, d.bh * d.t * d.hd, compute);
     float* dp = static_cast<float*>(ComputingContext::scratch((size_t)(d.bh * d.t * d.t) * sizeof(float)));
-    BR_OP(attn_products(d_o, attn, v, dp, BR_F32, v_g, d, compute));
+    BR_OP(attn_products(Operand{mem_, (int)DT}, attn, v, dp, BR_F32, v_g, d, compute));
     BR_OP(br_hip_softmax_bwd(dp, static_cast<const float*>(attn->data()), static_cast<float*>(attn_g->data()),
                              d.bh * d.t, d.t, stream()));
     return OP_OK;
@@ -763,10 +762,9 @@ ComputingReturn HIPTensor<DT>::op_qk_backward(tensor_t self, tensor_t q, tensor_
     if (!dev(q_g) || !dev(k_g) || q_g->items() != q->items() || k_g->items() != q->items()) return OP_OUTPUT_ERROR;
     const float alpha = (float)(1.0 / sqrt((double)hd));
     const int compute = pick_compute({self, q, k});
-    const Operand ds = shared_operand(mem_, (int)DT, bh * t * t, compute);
-    BR_OP(two_products({0, 0, t, hd, t, alpha, ds.ptr, ds.dtype, t, t * t, k->data(), code(k), hd, t * hd, q_g->data(), code(q_g),
+    BR_OP(two_products({0, 0, t, hd, t, alpha, mem_, (int)DT, t, t * t, k->data(), code(k), hd, t * hd, q_g->data(), code(q_g),
                         hd, t * hd, bh},
-                       {1, 0, t, hd, t, alpha, ds.ptr, ds.dtype, t, t * t, q->data(), code(q), hd, t * hd, k_g->data(), code(k_g),
+                       {1, 0, t, hd, t, alpha, mem_, (int)DT, t, t * t, q->data(), code(q), hd, t * hd, k_g->data(), code(k_g),
                         hd, t * hd, bh},
                        nullptr, compute));
     return OP_OK;

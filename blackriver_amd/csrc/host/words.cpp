@@ -121,6 +121,26 @@ BR_WORD(Layernorm,
 )
 // ( x y -- )
 BR_WORD(Transpos0213, Tensors<2> a(stack); a[0]->op_transpos_0213(a[0], a[1]);)
+// ( x y  x y  x y -- )  three in a row, q, k and v: one launch where they are of one shape and do not meet
+BR_WORD(Transpos0213x3,
+    Tensors<6> a(stack);
+    bool fast = true;
+    for (size_t i = 0; i < 6; i++)
+        fast = fast && a[i]->is_cuda() && a[i]->dtype() == a[0]->dtype() && a[i]->items() == a[0]->items();
+    for (size_t i = 0; fast && i < 6; i += 2) {
+        fast = a[i]->shape().dim() == 4 && a[i]->data() != a[i + 1]->data() && a[i]->dtype() != DataType::Int;
+        for (size_t d = 0; fast && d < 4; d++) fast = a[i]->shape()[d] == a[0]->shape()[d];
+    }
+    if (fast) {
+        const void* x[3] = {a[0]->data(), a[2]->data(), a[4]->data()};
+        void* y[3] = {a[1]->data(), a[3]->data(), a[5]->data()};
+        const auto& s = a[0]->shape();
+        BR_HIP_CHECK(br_hip_transpose_0213_group(x, y, 3, (int)DataType_size(a[0]->dtype()), (int64_t)s[0], (int64_t)s[1],
+                                                 (int64_t)s[2], (int64_t)s[3], ComputingContext::stream));
+    } else {
+        for (size_t i = 0; i < 6; i += 2) a[i]->op_transpos_0213(a[i], a[i + 1]);
+    }
+)
 // ( q k qk -- )
 BR_WORD(QueryKey, Tensors<3> a(stack); a[0]->op_qk(a[0], a[1], a[2]);)
 // ( a b c -- )
@@ -537,6 +557,7 @@ void load_nn_words(Enviroment& env) {
         {"op.softmax_backward", SoftmaxBackward::creator},
         {"op.softmax_attn_backward", SoftmaxAttnBackward::creator},
         {"op.qk_backward", QueryKeyBackward::creator},
+        {"op.transpos_0213_x3", Transpos0213x3::creator},
         {"op.gelu_linear_backward", GeluLinearBackward::creator},
         {"op.linear_add", LinearAdd::creator},
         {"op.linear_gelu", LinearGelu::creator},
@@ -557,6 +578,7 @@ void load_nn_words(Enviroment& env) {
     env.insert_fusion({"op.add", "op.add", "op.softmax"}, "op.add_add_softmax");
     env.insert_fusion({"op.layernorm", "op.copy"}, "op.layernorm_copy");
     env.insert_fusion({"op.gelu_backward", "op.linear_backward"}, "op.gelu_linear_backward");
+    env.insert_fusion({"op.transpos_0213", "op.transpos_0213", "op.transpos_0213"}, "op.transpos_0213_x3");
     // the pair also stands across a block boundary of a model program
     env.insert_fusion({"op.layernorm_backward_add", "op.linear_backward"}, "op.layernorm_backward_add_linear_backward", true);
 }

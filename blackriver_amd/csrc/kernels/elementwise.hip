@@ -898,8 +898,21 @@ int colsum_owner_launch(int lanes, const Src& src, float* out, int64_t rows, int
 // ------------------------------------------------------- transpose 0213
 // One 16-byte granule per thread, indexed by OUTPUT position so stores are
 // fully coalesced; loads are contiguous runs of s3 elements.
-__global__ __launch_bounds__(kBlock) void transpose_0213_x16(const uint4* x, uint4* y, long long n16,
+//
+// blockIdx.y picks one of several tensors of the same shape: the heads of q, k and v change places in one launch (a
+// launch of 2.5-5 us each, of which a block of a thousand tokens has two times three).
+constexpr int kTransposes = 4;
+struct TransposeSet {
+    const uint4* x[kTransposes];
+    uint4* y[kTransposes];
+};
+__global__ __launch_bounds__(kBlock) void transpose_0213_x16(TransposeSet set, long long n16,
                                                               unsigned s1, unsigned s2, unsigned s3g) {
+    const uint4* x = set.x[0];
+    uint4* y = set.y[0];
+#pragma unroll
+    for (int i = 1; i < kTransposes; i++)
+        if (blockIdx.y == (unsigned)i) x = set.x[i], y = set.y[i];
     const long long stride = (long long)gridDim.x * kBlock;
     for (long long o = (long long)blockIdx.x * kBlock + threadIdx.x; o < n16; o += stride) {
         unsigned long long r = (unsigned long long)o;
@@ -1544,6 +1557,43 @@ int br_hip_gelu_bwd_colsum_cast(const float* dy, const float* x, float* dx, floa
     return colsum_finish(partial, out, groups, cols, out_scale, st);
 }
 
+int br_hip_transpose_0213_group(const void* const* x, void* const* y, int count, int elem_bytes, int64_t s0, int64_t s1,
+                                int64_t s2, int64_t s3, br_stream_t stream) {
+    if (count < 0) return BR_ERR_ATTR;
+    if (count == 0) return BR_OK;
+    if (!x) return BR_ERR_INPUT;
+    if (!y) return BR_ERR_OUTPUT;
+    bool together = count > 1 && count <= kTransposes && (elem_bytes == 2 || elem_bytes == 4) && s0 > 0 && s1 > 0 && s2 > 0 &&
+                    s3 > 0 && fits_u32(s1) && fits_u32(s2) && fits_u32(s3) && s3 % (16 / elem_bytes) == 0;
+    const uintptr_t bytes = together ? (uintptr_t)(s0 * s1 * s2 * s3) * (uintptr_t)elem_bytes : 0;
+    const int64_t n16 = (int64_t)(bytes / 16);
+    together = together && n16 <= (int64_t)1 << 28;   // each within a grid of its own size
+    for (int i = 0; together && i < count; i++) {
+        together = x[i] && y[i] && aligned16(x[i]) && aligned16(y[i]);
+        // no tensor written is one that another of them reads or writes
+        for (int j = 0; together && j < count; j++) {
+            auto apart = [&](const void* a, const void* b) {
+                const uintptr_t p = reinterpret_cast<uintptr_t>(a), q = reinterpret_cast<uintptr_t>(b);
+                return p + bytes <= q || q + bytes <= p;
+            };
+            together = apart(y[i], x[j]) && (i == j || apart(y[i], y[j]));
+        }
+    }
+    if (together) {
+        TransposeSet set = {};
+        for (int i = 0; i < count; i++) set.x[i] = (const uint4*)x[i], set.y[i] = (uint4*)y[i];
+        transpose_0213_x16<<<dim3((unsigned)grid_for(n16, kBlock), (unsigned)count), kBlock, 0, as_stream(stream)>>>(
+            set, n16, (unsigned)s1, (unsigned)s2, (unsigned)(s3 / (16 / elem_bytes)));
+        BR_HIP_LAUNCH_CHECK();
+        return BR_OK;
+    }
+    for (int i = 0; i < count; i++) {
+        const int rc = br_hip_transpose_0213(x[i], y[i], elem_bytes, s0, s1, s2, s3, stream);
+        if (rc != BR_OK) return rc;
+    }
+    return BR_OK;
+}
+
 int br_hip_transpose_0213(const void* x, void* y, int elem_bytes, int64_t s0, int64_t s1, int64_t s2,
                           int64_t s3, br_stream_t stream) {
     if (s0 < 0 || s1 <= 0 || s2 <= 0 || s3 <= 0) return BR_ERR_ATTR;
@@ -1557,8 +1607,10 @@ int br_hip_transpose_0213(const void* x, void* y, int elem_bytes, int64_t s0, in
     const int per16 = 16 / elem_bytes;
     if (s3 % per16 == 0 && aligned16(x) && aligned16(y)) {
         const int64_t n16 = n / per16;
-        transpose_0213_x16<<<grid_for(n16, kBlock), kBlock, 0, st>>>((const uint4*)x, (uint4*)y, n16,
-                                                                    (unsigned)s1, (unsigned)s2,
+        TransposeSet one = {};
+        one.x[0] = (const uint4*)x;
+        one.y[0] = (uint4*)y;
+        transpose_0213_x16<<<grid_for(n16, kBlock), kBlock, 0, st>>>(one, n16, (unsigned)s1, (unsigned)s2,
                                                                     (unsigned)(s3 / per16));
     } else if (elem_bytes == 4) {
         transpose_0213_scalar<uint32_t><<<grid_for(n, kBlock), kBlock, 0, st>>>(

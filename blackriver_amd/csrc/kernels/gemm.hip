@@ -427,95 +427,147 @@ extern "C" int br_hip_linear_gelu(const void* x, const void* w, const float* bia
 // ---- operands staged as dense, aligned 16-bit copies ------------------------
 namespace {
 
-// dst[b][r][0 .. pitch) = convert(src[b*stride + r*ld + c]) for c < cols, zero from there to the pitch (a multiple
-// of 8): fp32 rows, or 16-bit rows that do not start on 16-byte boundaries.  One 16-byte granule per thread.
-template <bool F32SRC, bool BF>
-__global__ __launch_bounds__(256) void stage_rows_kernel(const void* __restrict__ src, long long ld, long long stride,
-                                                         unsigned rows, unsigned cols, unsigned granules,
-                                                         long long total, gemm16::u32x4* __restrict__ dst) {
-    constexpr int CT = BF ? BR_GEMM_BF16 : BR_GEMM_F16;
-    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < total;
-         i += (long long)gridDim.x * blockDim.x) {
-        const unsigned c = (unsigned)(i % granules) * 8;
-        const long long row = i / granules;
-        const long long at = row / rows * stride + row % rows * ld + c;
-        gemm16::u32x4 o;
-        if (F32SRC) {
-            const float* s = static_cast<const float*>(src) + at;
-            float v[8];
-            if (c + 8 <= cols) {
-                __builtin_memcpy(v, s, sizeof(v));
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; e++) v[e] = c + e < cols ? s[e] : 0.f;
-            }
-            o = gemm16::mk4(gemm16::pack2(gemm16::Cvt<CT>::from_f32(v[0]), gemm16::Cvt<CT>::from_f32(v[1])),
-                            gemm16::pack2(gemm16::Cvt<CT>::from_f32(v[2]), gemm16::Cvt<CT>::from_f32(v[3])),
-                            gemm16::pack2(gemm16::Cvt<CT>::from_f32(v[4]), gemm16::Cvt<CT>::from_f32(v[5])),
-                            gemm16::pack2(gemm16::Cvt<CT>::from_f32(v[6]), gemm16::Cvt<CT>::from_f32(v[7])));
-        } else {
-            const gemm16::u16* s = static_cast<const gemm16::u16*>(src) + at;
-            if (c + 8 <= cols) {
-                __builtin_memcpy(&o, s, sizeof(o));
-            } else {
-                gemm16::u16 h[8];
-#pragma unroll
-                for (int e = 0; e < 8; e++) h[e] = c + e < cols ? s[e] : (gemm16::u16)0;
-                o = gemm16::mk4(gemm16::pack2(h[0], h[1]), gemm16::pack2(h[2], h[3]), gemm16::pack2(h[4], h[5]),
-                                gemm16::pack2(h[6], h[7]));
-            }
-        }
-        dst[i] = o;
-    }
+// What is copied: dst[b][r][0 .. pitch) = convert(src[b*stride + r*ld + c]) for c < cols, zero from there to the pitch
+// (a multiple of 8); fp32 values, or 16-bit ones whose rows do not start on 16-byte boundaries.
+struct StageJob {
+    const void* src;
+    gemm16::u32x4* dst;
+    long long ld, stride, total;   // total: 16-byte granules written
+    unsigned rows, cols, granules; // granules: of a row
+    unsigned first;                // the first workgroup of this operand
+    bool f32, flat;                // flat: rows follow each other without gaps, fp32 and aligned
+};
+constexpr int kStageJobs = 4;
+struct StageJobs {
+    StageJob job[kStageJobs];
+    int count;
+};
+
+__device__ __forceinline__ gemm16::u32x4 pack16(const float (&v)[8], bool bf) {
+    using namespace gemm16;
+    if (bf)
+        return mk4(pack2(Cvt<BR_GEMM_BF16>::from_f32(v[0]), Cvt<BR_GEMM_BF16>::from_f32(v[1])),
+                   pack2(Cvt<BR_GEMM_BF16>::from_f32(v[2]), Cvt<BR_GEMM_BF16>::from_f32(v[3])),
+                   pack2(Cvt<BR_GEMM_BF16>::from_f32(v[4]), Cvt<BR_GEMM_BF16>::from_f32(v[5])),
+                   pack2(Cvt<BR_GEMM_BF16>::from_f32(v[6]), Cvt<BR_GEMM_BF16>::from_f32(v[7])));
+    return mk4(pack2(Cvt<BR_GEMM_F16>::from_f32(v[0]), Cvt<BR_GEMM_F16>::from_f32(v[1])),
+               pack2(Cvt<BR_GEMM_F16>::from_f32(v[2]), Cvt<BR_GEMM_F16>::from_f32(v[3])),
+               pack2(Cvt<BR_GEMM_F16>::from_f32(v[4]), Cvt<BR_GEMM_F16>::from_f32(v[5])),
+               pack2(Cvt<BR_GEMM_F16>::from_f32(v[6]), Cvt<BR_GEMM_F16>::from_f32(v[7])));
 }
 
-// Dense operand (rows follow each other without gaps): a flat conversion, 8
-// elements per thread, no index arithmetic.
+// One 16-byte granule per thread; the operands of a product (or of two) one after the other in one launch.  What it costs
+// is bytes on large operands and the launch on small ones: [1024 x 2048] fp32 4-6 us, as does [64 x 256].  The operands
+// of attention's backward products over 32 heads x 512 tokens, scores among them, one by one / at once (us):
+// dO, P, V 5.3 + 11.2 + 6.2 / 13.5, dS, K, Q 10.5 + 5.2 + 5.4 / 12.
 template <bool BF>
-__global__ __launch_bounds__(256) void stage_flat_kernel(const float4* __restrict__ src, gemm16::u32x4* __restrict__ dst,
-                                                         long long n8) {
-    for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < n8;
-         i += (long long)gridDim.x * blockDim.x) {
-        const float4 a = src[2 * i], b = src[2 * i + 1];
-        constexpr int CT = BF ? BR_GEMM_BF16 : BR_GEMM_F16;
-        gemm16::u32x4 o;
-        o.x = gemm16::pack2(gemm16::Cvt<CT>::from_f32(a.x), gemm16::Cvt<CT>::from_f32(a.y));
-        o.y = gemm16::pack2(gemm16::Cvt<CT>::from_f32(a.z), gemm16::Cvt<CT>::from_f32(a.w));
-        o.z = gemm16::pack2(gemm16::Cvt<CT>::from_f32(b.x), gemm16::Cvt<CT>::from_f32(b.y));
-        o.w = gemm16::pack2(gemm16::Cvt<CT>::from_f32(b.z), gemm16::Cvt<CT>::from_f32(b.w));
-        dst[i] = o;
+__global__ __launch_bounds__(256) void stage_kernel(StageJobs jobs) {
+    int which = 0;
+#pragma unroll
+    for (int i = 1; i < kStageJobs; i++)
+        if (i < jobs.count && blockIdx.x >= jobs.job[i].first) which = i;
+    which = __builtin_amdgcn_readfirstlane(which);
+    // picked field by field: the arguments stay where they are
+    auto pick = [&](auto field) {
+        auto v = field(jobs.job[0]);
+#pragma unroll
+        for (int i = 1; i < kStageJobs; i++) v = which == i ? field(jobs.job[i]) : v;
+        return v;
+    };
+    const void* const src = pick([](const StageJob& j) { return j.src; });
+    gemm16::u32x4* const dst = pick([](const StageJob& j) { return j.dst; });
+    const long long total = pick([](const StageJob& j) { return j.total; });
+    const unsigned first = pick([](const StageJob& j) { return j.first; });
+    const bool f32 = pick([](const StageJob& j) { return j.f32; }), flat = pick([](const StageJob& j) { return j.flat; });
+    const long long i = (long long)(blockIdx.x - first) * 256 + threadIdx.x;
+    if (i >= total) return;
+    if (flat) {
+        const float4 a = static_cast<const float4*>(src)[2 * i], b = static_cast<const float4*>(src)[2 * i + 1];
+        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        dst[i] = pack16(v, BF);
+        return;
     }
+    const unsigned rows = pick([](const StageJob& j) { return j.rows; }), cols = pick([](const StageJob& j) { return j.cols; });
+    const unsigned granules = pick([](const StageJob& j) { return j.granules; });
+    const long long ld = pick([](const StageJob& j) { return j.ld; }), stride = pick([](const StageJob& j) { return j.stride; });
+    const unsigned c = (unsigned)(i % granules) * 8;
+    const long long row = i / granules;
+    const long long at = row / rows * stride + row % rows * ld + c;
+    gemm16::u32x4 o;
+    if (f32) {
+        const float* s = static_cast<const float*>(src) + at;
+        float v[8];
+        if (c + 8 <= cols) {
+            __builtin_memcpy(v, s, sizeof(v));
+        } else {
+#pragma unroll
+            for (int e = 0; e < 8; e++) v[e] = c + e < cols ? s[e] : 0.f;
+        }
+        o = pack16(v, BF);
+    } else {   // bits are moved as they are
+        const gemm16::u16* s = static_cast<const gemm16::u16*>(src) + at;
+        if (c + 8 <= cols) {
+            __builtin_memcpy(&o, s, sizeof(o));
+        } else {
+            gemm16::u16 h[8];
+#pragma unroll
+            for (int e = 0; e < 8; e++) h[e] = c + e < cols ? s[e] : (gemm16::u16)0;
+            o = gemm16::mk4(gemm16::pack2(h[0], h[1]), gemm16::pack2(h[2], h[3]), gemm16::pack2(h[4], h[5]),
+                            gemm16::pack2(h[6], h[7]));
+        }
+    }
+    dst[i] = o;
 }
 
 // Row length of a staged copy of `cols` columns.
 int64_t staged_pitch(int64_t cols) { return (cols + 7) & ~(int64_t)7; }
 
-int stage_rows(const void* src, bool f32, long long ld, long long stride, long long rows, long long cols,
-               long long batch, void* dst, int compute, hipStream_t st) {
-    const bool bf = compute == BR_GEMM_BF16;
-    if (f32 && ld == cols && cols % 8 == 0 && (batch == 1 || stride == rows * cols) && aligned16(src)) {
-        const long long n8 = batch * rows * cols / 8;
-        const unsigned grid = grid_for(n8, 256);
-        if (bf)
-            stage_flat_kernel<true><<<grid, 256, 0, st>>>(static_cast<const float4*>(src), static_cast<gemm16::u32x4*>(dst), n8);
-        else
-            stage_flat_kernel<false><<<grid, 256, 0, st>>>(static_cast<const float4*>(src), static_cast<gemm16::u32x4*>(dst), n8);
+// Operands gathered for one launch.
+struct Stager {
+    StageJobs jobs;
+    long long blocks = 0;
+    int compute;
+    hipStream_t st;
+    Stager(int compute_, hipStream_t st_) : compute(compute_), st(st_) { jobs.count = 0; }
+    int add(const void* src, bool f32, long long ld, long long stride, long long rows, long long cols, long long batch, void* dst) {
+        const bool flat = f32 && ld == cols && cols % 8 == 0 && (batch == 1 || stride == rows * cols) && aligned16(src);
+        const long long granules = staged_pitch(cols) / 8, total = batch * rows * granules;
+        if (rows > 0xffffffffLL || cols > 0xfffffff0LL) return BR_ERR_ATTR;
+        const long long need = (total + 255) / 256;
+        // a launch holds less than 2^32 work items: what does not fit into this one starts another
+        constexpr long long most = (1 << 24) - 1;
+        if (need > most) {
+            // so much in one operand goes in pieces of whole batch entries and rows
+            const long long piece = most * 256 / granules;
+            if (piece < 1) return BR_ERR_ATTR;
+            for (long long b = 0; b < batch; b++)
+                for (long long r = 0; r < rows; r += piece) {
+                    const long long some = rows - r < piece ? rows - r : piece;
+                    const char* from = static_cast<const char*>(src) + (b * stride + r * ld) * (f32 ? 4 : 2);
+                    const int rc = add(from, f32, ld, some * ld, some, cols, 1, static_cast<char*>(dst) + (b * rows + r) * granules * 16);
+                    if (rc != BR_OK) return rc;
+                }
+            return BR_OK;
+        }
+        if (jobs.count == kStageJobs || blocks + need > most) {
+            const int rc = run();
+            if (rc != BR_OK) return rc;
+        }
+        jobs.job[jobs.count++] = StageJob{src, static_cast<gemm16::u32x4*>(dst), ld, stride, total, (unsigned)rows, (unsigned)cols,
+                                          (unsigned)granules, (unsigned)blocks, f32, flat};
+        blocks += need;
+        return BR_OK;
+    }
+    int run() {
+        if (jobs.count == 0) return BR_OK;
+        if (compute == BR_GEMM_BF16) stage_kernel<true><<<(unsigned)blocks, 256, 0, st>>>(jobs);
+        else stage_kernel<false><<<(unsigned)blocks, 256, 0, st>>>(jobs);
+        jobs.count = 0;
+        blocks = 0;
         BR_HIP_LAUNCH_CHECK();
         return BR_OK;
     }
-    const long long granules = staged_pitch(cols) / 8, total = batch * rows * granules;
-    if (rows > 0xffffffffLL || cols > 0xfffffff0LL) return BR_ERR_ATTR;
-    const unsigned grid = grid_for(total, 256);
-    gemm16::u32x4* d = static_cast<gemm16::u32x4*>(dst);
-#define BR_STAGE(F32, BF) \
-    stage_rows_kernel<F32, BF><<<grid, 256, 0, st>>>(src, ld, stride, (unsigned)rows, (unsigned)cols, (unsigned)granules, total, d)
-    if (!f32) BR_STAGE(false, false);   // bits are moved as they are
-    else if (bf) BR_STAGE(true, true);
-    else BR_STAGE(true, false);
-#undef BR_STAGE
-    BR_HIP_LAUNCH_CHECK();
-    return BR_OK;
-}
+};
 
 // ---- split-K ------------------------------------------------------------------
 // A product with few output tiles and a long K leaves most CUs idle.  Two forms,
@@ -574,6 +626,12 @@ size_t staged_bytes(int64_t rows, int64_t cols, int64_t batch) {
 // do not start on 16-byte boundaries are moved to rows that do.
 bool wants_staging(int dtype, int64_t cols) { return dtype == BR_F32 || cols % 8 != 0; }
 
+// Room for the partial sums of a product whose K is cut.
+size_t sums_bytes(int64_t m, int64_t n, int64_t k, int64_t batch) {
+    const gemm16::Plan plan = gemm16::gemm_plan(m, n, k, batch, true);
+    return (plan.slices > 1 ? (size_t)plan.slices * (size_t)m * (size_t)n * sizeof(float) : 0) + gemm16::pair_bytes(plan, m, n);
+}
+
 }  // namespace
 
 extern "C" size_t br_hip_gemm_staged_workspace(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, int a_dtype,
@@ -582,17 +640,17 @@ extern "C" size_t br_hip_gemm_staged_workspace(int trans_a, int trans_b, int64_t
     size_t need = 0;
     if (wants_staging(a_dtype, trans_a ? m : k)) need += staged_bytes(trans_a ? k : m, trans_a ? m : k, batch);
     if (wants_staging(b_dtype, trans_b ? k : n)) need += staged_bytes(trans_b ? n : k, trans_b ? k : n, batch);
-    const gemm16::Plan plan = gemm16::gemm_plan(m, n, k, batch, true);
-    if (plan.slices > 1) need += (size_t)plan.slices * (size_t)m * (size_t)n * sizeof(float);
-    return need + gemm16::pair_bytes(plan, m, n);
+    return need + sums_bytes(m, n, k, batch);
 }
 
 namespace {
-// br_hip_gemm_staged with the tensor an accumulating product adds to named separately (null = c itself).
+// br_hip_gemm_staged with the tensor an accumulating product adds to named separately (null = c itself).  zero_filled: the
+// operands are in the products' type already, their rows aligned and zero-filled to whole granules.
 int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alpha, const void* a, int a_dtype,
                 int64_t lda, int64_t stride_a, const void* b, int b_dtype, int64_t ldb, int64_t stride_b, int accumulate,
                 const void* addend, void* c, int c_dtype, int64_t ldc, int64_t stride_c, const float* bias,
-                int64_t batch, int compute, void* workspace, size_t workspace_bytes, br_stream_t stream) {
+                int64_t batch, int compute, void* workspace, size_t workspace_bytes, br_stream_t stream,
+                bool zero_filled = false) {
     const int native = compute == BR_GEMM_F16 ? BR_F16 : BR_BF16;
     const bool sixteen = compute == BR_GEMM_F16 || compute == BR_GEMM_BF16;
     const int64_t a_rows = trans_a ? k : m, a_cols = trans_a ? m : k;
@@ -603,7 +661,9 @@ int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
                        c && lda >= a_cols && ldb >= b_cols && ldc >= n &&
                        (a_dtype == BR_F32 || a_dtype == native) && (b_dtype == BR_F32 || b_dtype == native) &&
                        (c_dtype == BR_F32 || c_dtype == native) &&
-                       br_hip_gemm_staged_workspace(trans_a, trans_b, m, n, k, a_dtype, b_dtype, batch) <= workspace_bytes;
+                       (zero_filled ? sums_bytes(m, n, k, batch)
+                                    : br_hip_gemm_staged_workspace(trans_a, trans_b, m, n, k, a_dtype, b_dtype, batch)) <=
+                           workspace_bytes;
     if (!stage)
         return gemm_impl(trans_a, trans_b, m, n, k, alpha, a, a_dtype, lda, stride_a, b, b_dtype, ldb, stride_b,
                          accumulate, addend, c, c_dtype, ldc, stride_c, bias, batch, compute, stream);
@@ -615,8 +675,9 @@ int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
         return dtype != BR_F32 && !along_k && aligned16(x) && ld % 8 == 0 && (batch == 1 || stride % 8 == 0);
     };
     // every row of a staged copy is zero-filled up to its pitch
-    if (wants_staging(a_dtype, a_cols) && !in_place(a, a_dtype, !trans_a, lda, stride_a)) {
-        const int rc = stage_rows(a, a_dtype == BR_F32, lda, stride_a, a_rows, a_cols, batch, ws, compute, st);
+    Stager stager(compute, st);
+    if (wants_staging(a_dtype, a_cols) && !zero_filled && !in_place(a, a_dtype, !trans_a, lda, stride_a)) {
+        const int rc = stager.add(a, a_dtype == BR_F32, lda, stride_a, a_rows, a_cols, batch, ws);
         if (rc != BR_OK) return rc;
         a = ws;
         a_dtype = native;
@@ -624,8 +685,8 @@ int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
         stride_a = a_rows * lda;
         ws += staged_bytes(a_rows, a_cols, batch);
     }
-    if (wants_staging(b_dtype, b_cols) && !in_place(b, b_dtype, trans_b, ldb, stride_b)) {
-        const int rc = stage_rows(b, b_dtype == BR_F32, ldb, stride_b, b_rows, b_cols, batch, ws, compute, st);
+    if (wants_staging(b_dtype, b_cols) && !zero_filled && !in_place(b, b_dtype, trans_b, ldb, stride_b)) {
+        const int rc = stager.add(b, b_dtype == BR_F32, ldb, stride_b, b_rows, b_cols, batch, ws);
         if (rc != BR_OK) return rc;
         b = ws;
         b_dtype = native;
@@ -633,6 +694,8 @@ int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
         stride_b = b_rows * ldb;
         ws += staged_bytes(b_rows, b_cols, batch);
     }
+    const int staged = stager.run();
+    if (staged != BR_OK) return staged;
     const gemm16::Plan plan = gemm16::gemm_plan(m, n, k, batch, true);
     // only the direct-to-LDS kernels know slices: the register-staged one would sum all of K once per slice
     const bool sliceable = aligned16(a) && aligned16(b) && lda % 8 == 0 && ldb % 8 == 0 &&
@@ -715,26 +778,62 @@ bool sizes_ok(const br_product& p) {
            p.ldb >= (p.trans_b ? p.k : p.n) && p.ldc >= p.n && (p.batch == 1 || (p.stride_a >= 0 && p.stride_b >= 0 && p.stride_c >= 0));
 }
 
+// What two products read, with the operands that have to be copied first in `copies`: one that both read is copied once.
+struct PairOperands {
+    Stored before[4], now[4];   // a and b of the first, a and b of the second
+    int copy_of[4] = {-1, -1, -1, -1};
+    size_t bytes = 0;           // of all copies
+    PairOperands(const br_product& first, const br_product& second, int compute, char* ws)
+        : before{stored_a(first), stored_b(first), stored_a(second), stored_b(second)}, now{before[0], before[1], before[2], before[3]} {
+        if (compute == BR_GEMM_F32) return;
+        for (int i = 0; i < 4; i++) {
+            const Stored& s = before[i];
+            // as in staged_impl
+            const bool in_place = s.dtype != BR_F32 && !s.along_k && aligned16(s.at) && s.ld % 8 == 0 && (s.batch == 1 || s.stride % 8 == 0);
+            if (!wants_staging(s.dtype, s.cols) || in_place) continue;
+            copy_of[i] = i;
+            for (int j = 0; j < i; j++)
+                if (copy_of[j] == j && same_memory(s, before[j])) copy_of[i] = j;
+            if (copy_of[i] == i) {
+                now[i].at = ws + bytes;
+                bytes += staged_bytes(s.rows, s.cols, s.batch);
+            } else {
+                now[i].at = now[copy_of[i]].at;
+            }
+            now[i].dtype = compute == BR_GEMM_F16 ? BR_F16 : BR_BF16;
+            now[i].ld = staged_pitch(s.cols);
+            now[i].stride = s.rows * now[i].ld;
+        }
+    }
+    int run(int compute, hipStream_t st) const {
+        Stager stager(compute, st);
+        for (int i = 0; i < 4; i++) {
+            if (copy_of[i] != i) continue;
+            const Stored& s = before[i];
+            const int rc = stager.add(s.at, s.dtype == BR_F32, s.ld, s.stride, s.rows, s.cols, s.batch, const_cast<void*>(now[i].at));
+            if (rc != BR_OK) return rc;
+        }
+        return stager.run();
+    }
+};
+
 // Both products (and the column sums) as one launch; BR_ERR_TODO where they have to run one after the other.
-int pair_impl(const br_product& first, const br_product& second, const br_column_sums* sums, int compute, void* workspace,
-              size_t workspace_bytes, hipStream_t st) {
+int pair_impl(const br_product& first, const br_product& second, const PairOperands& ops, const br_column_sums* sums, int compute,
+              hipStream_t st) {
     using namespace gemm16;
     const bool fp32 = compute == BR_GEMM_F32;
     const int native = compute == BR_GEMM_F16 ? BR_F16 : fp32 ? BR_F32 : BR_BF16;
     // the one with both operands row-contiguous
     auto wide = [](const br_product& p) { return p.trans_a && !p.trans_b && p.c_dtype == BR_F32; };
     const int w = wide(first) ? 0 : 1, x = 1 - w;
-    if (!sizes_ok(first) || !sizes_ok(second) || !wide(w ? second : first) || (w ? first : second).trans_a) return BR_ERR_TODO;
+    if (!wide(w ? second : first) || (w ? first : second).trans_a) return BR_ERR_TODO;
     const int kernel = pair_kernel({first.m, first.n, first.k, first.batch}, {second.m, second.n, second.k, second.batch}, fp32);
     if (kernel < 0) return BR_ERR_TODO;
     const br_product* const products[2] = {&first, &second};
-    Stored in[4] = {stored_a(first), stored_b(first), stored_a(second), stored_b(second)};
     const Stored out[2] = {stored_c(first), stored_c(second)};
-    for (const Stored& s : in)
-        if (s.dtype != native && s.dtype != BR_F32) return BR_ERR_TODO;
     if (out[x].dtype != native && out[x].dtype != BR_F32) return BR_ERR_TODO;
-    // nothing is written that another part reads or writes (before staging: what is staged is read ahead of all writes)
-    if (overlap(out[0], out[1]) || overlap(out[0], in[2]) || overlap(out[0], in[3])) return BR_ERR_TODO;
+    // nothing is written that another part reads or writes (what is copied first is read ahead of all writes)
+    if (overlap(out[0], out[1]) || overlap(out[1], ops.now[0]) || overlap(out[1], ops.now[1])) return BR_ERR_TODO;
     ColumnSums cs;
     if (sums) {
         const Stored sx{sums->x, sums->dtype, sums->rows, sums->cols, sums->cols, 0, 1, false};
@@ -743,7 +842,7 @@ int pair_impl(const br_product& first, const br_product& second, const br_column
         if (!sums->x || !sums->out || sums->dtype != native || sums->rows <= 0 || sums->cols <= 0 || sums->cols % vec != 0 ||
             sums->rows > 0x3fffffffLL || sums->cols > 0x3fffffffLL || !aligned16(sums->x))
             return BR_ERR_TODO;
-        for (const Stored& s : in)
+        for (const Stored& s : ops.before)
             if (overlap(so, s)) return BR_ERR_TODO;
         for (const Stored& s : out)
             if (overlap(so, s) || overlap(sx, s)) return BR_ERR_TODO;
@@ -753,39 +852,10 @@ int pair_impl(const br_product& first, const br_product& second, const br_column
         cs.cols = (int)sums->cols;
         cs.scale = sums->scale;
     }
-    // which operands are copied, and where to; one that both products read is copied once
-    const Stored before[4] = {in[0], in[1], in[2], in[3]};
-    char* ws = static_cast<char*>(workspace);
-    size_t used = 0;
-    int copy_of[4] = {-1, -1, -1, -1};
-    for (int i = 0; i < 4 && !fp32; i++) {
-        const bool in_place = in[i].dtype != BR_F32 && !in[i].along_k && aligned16(in[i].at) && in[i].ld % 8 == 0 &&
-                              (in[i].batch == 1 || in[i].stride % 8 == 0);
-        if (!wants_staging(in[i].dtype, in[i].cols) || in_place) continue;
-        copy_of[i] = i;
-        for (int j = 0; j < i; j++)
-            if (copy_of[j] == j && same_memory(before[i], before[j])) copy_of[i] = j;
-        if (copy_of[i] == i) {
-            in[i].at = ws + used;
-            used += staged_bytes(in[i].rows, in[i].cols, in[i].batch);
-            in[i].dtype = native;
-            in[i].ld = staged_pitch(in[i].cols);
-            in[i].stride = in[i].rows * in[i].ld;
-        } else {
-            const Stored& from = in[copy_of[i]];
-            in[i].at = from.at;
-            in[i].dtype = native;
-            in[i].ld = from.ld;
-            in[i].stride = from.stride;
-        }
-    }
-    if (used > 0 && (!ws || !aligned16(ws) || used > workspace_bytes)) return BR_ERR_TODO;
-    for (int i = 0; i < 2; i++)
-        if (overlap(out[1], in[i])) return BR_ERR_TODO;
     GemmArgs g[2];
     Problem p[2];
     for (int i = 0; i < 2; i++) {
-        const Stored &a = in[2 * i], &b = in[2 * i + 1];
+        const Stored &a = ops.now[2 * i], &b = ops.now[2 * i + 1];
         const br_product& d = *products[i];
         GemmArgs& q = g[i];
         q.a = a.at; q.b = b.at; q.c = d.c; q.bias = nullptr;
@@ -817,12 +887,8 @@ int pair_impl(const br_product& first, const br_product& second, const br_column
             return BR_ERR_TODO;
         }
     }
-    for (int i = 0; i < 4; i++) {
-        if (copy_of[i] != i) continue;
-        const int rc = stage_rows(before[i].at, before[i].dtype == BR_F32, before[i].ld, before[i].stride, before[i].rows, before[i].cols,
-                                  before[i].batch, const_cast<void*>(in[i].at), compute, st);
-        if (rc != BR_OK) return rc;
-    }
+    const int rc = ops.run(compute, st);
+    if (rc != BR_OK) return rc;
     auto* const launch = fp32 ? gemm_pair_f32 : compute == BR_GEMM_F16 ? gemm_pair_f16 : gemm_pair_bf16;
     return launch(g[w], p[w], products[w]->batch, g[x], p[x], products[x]->batch, kernel, cs, st);
 }
@@ -831,16 +897,16 @@ int pair_impl(const br_product& first, const br_product& second, const br_column
 
 extern "C" size_t br_hip_gemm_pair_workspace(const br_product* first, const br_product* second, int compute) {
     if (!first || !second || compute == BR_GEMM_F32) return 0;
-    const bool one_launch = br_hip_gemm_pair_kernel(first->m, first->n, first->k, first->batch, second->m, second->n, second->k,
-                                                    second->batch, compute) >= 0;
-    size_t both = 0, most = 0;
+    size_t copies = 0, sums = 0, most = 0;
     for (const br_product* p : {first, second}) {
         if (p->m <= 0 || p->n <= 0 || p->k <= 0 || p->batch <= 0) continue;
-        if (one_launch) both += staged_size(stored_a(*p)) + staged_size(stored_b(*p));
+        copies += staged_size(stored_a(*p)) + staged_size(stored_b(*p));
+        const size_t partial = sums_bytes(p->m, p->n, p->k, p->batch);
         const size_t one = br_hip_gemm_staged_workspace(p->trans_a, p->trans_b, p->m, p->n, p->k, p->a_dtype, p->b_dtype, p->batch);
+        if (partial > sums) sums = partial;
         if (one > most) most = one;
     }
-    return both > most ? both : most;
+    return copies + sums > most ? copies + sums : most;
 }
 
 extern "C" int br_hip_gemm_pair_kernel(int64_t m1, int64_t n1, int64_t k1, int64_t batch1, int64_t m2, int64_t n2, int64_t k2,
@@ -853,13 +919,47 @@ extern "C" int br_hip_gemm_pair(const br_product* first, const br_product* secon
                                 void* workspace, size_t workspace_bytes, br_stream_t stream) {
     if (!first || !second) return BR_ERR_INPUT;
     if (compute != BR_GEMM_F16 && compute != BR_GEMM_BF16 && compute != BR_GEMM_F32) return BR_ERR_ATTR;
-    const int rc = pair_impl(*first, *second, sums, compute, workspace, workspace_bytes, as_stream(stream));
-    if (rc != BR_ERR_TODO) return rc;
-    if (sums) {
-        const int rs = br_hip_colsum(sums->x, sums->dtype, sums->out, sums->rows, sums->cols, sums->scale, sums->workspace,
-                                     sums->workspace_bytes, stream);
-        if (rs != BR_OK) return rs;
+    hipStream_t st = as_stream(stream);
+    auto before_them = [&]() {
+        if (!sums) return (int)BR_OK;
+        return br_hip_colsum(sums->x, sums->dtype, sums->out, sums->rows, sums->cols, sums->scale, sums->workspace,
+                             sums->workspace_bytes, stream);
+    };
+    const int native = compute == BR_GEMM_F16 ? BR_F16 : compute == BR_GEMM_BF16 ? BR_BF16 : BR_F32;
+    auto types_ok = [&](const br_product& p) {
+        return (p.a_dtype == BR_F32 || p.a_dtype == native) && (p.b_dtype == BR_F32 || p.b_dtype == native) &&
+               (p.c_dtype == BR_F32 || p.c_dtype == native);
+    };
+    if (sizes_ok(*first) && sizes_ok(*second) && types_ok(*first) && types_ok(*second)) {
+        char* ws = static_cast<char*>(workspace);
+        const PairOperands ops(*first, *second, compute, ws);
+        const bool room = ops.bytes == 0 || (ws && aligned16(ws) && ops.bytes <= workspace_bytes);
+        // copies are made ahead of both products: the first must not write what the second's are made of
+        const bool apart = !overlap(stored_c(*first), ops.before[2]) && !overlap(stored_c(*first), ops.before[3]);
+        if (room && apart) {
+            const int rc = pair_impl(*first, *second, ops, sums, compute, st);
+            if (rc != BR_ERR_TODO) return rc;
+            if (ops.bytes > 0 && workspace_bytes >= ops.bytes) {
+                // one after the other, on copies made in one launch
+                const int rs = before_them();
+                if (rs != BR_OK) return rs;
+                const int rt = ops.run(compute, st);
+                if (rt != BR_OK) return rt;
+                const size_t left = workspace_bytes - ops.bytes;
+                for (int i = 0; i < 2; i++) {
+                    const br_product& p = i ? *second : *first;
+                    const Stored &a = ops.now[2 * i], &b = ops.now[2 * i + 1];
+                    const int rp = staged_impl(p.trans_a, p.trans_b, p.m, p.n, p.k, p.alpha, a.at, a.dtype, a.ld, a.stride, b.at,
+                                               b.dtype, b.ld, b.stride, 0, nullptr, p.c, p.c_dtype, p.ldc, p.stride_c, nullptr,
+                                               p.batch, compute, ws + ops.bytes, left, stream, true);
+                    if (rp != BR_OK) return rp;
+                }
+                return BR_OK;
+            }
+        }
     }
+    const int rs = before_them();
+    if (rs != BR_OK) return rs;
     for (const br_product* p : {first, second}) {
         const int rp = compute == BR_GEMM_F32
             ? gemm_impl(p->trans_a, p->trans_b, p->m, p->n, p->k, p->alpha, p->a, p->a_dtype, p->lda, p->stride_a, p->b, p->b_dtype,

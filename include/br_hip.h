@@ -129,6 +129,10 @@ int br_hip_bias_gelu_bwd(const void* dy, const void* x, const float* bias, void*
 /* kernels::launch_transform_0213<float>, kernels/transform_kernels.cu:56-65
  * (declared kernels/kernels.h:35), called at cuda_tensor.cpp:257-275: [s0,s1,s2,s3] -> [s0,s2,s1,s3].
  * elem_bytes is 2 or 4. */
+/* `count` of them, one after the other or, where none writes what another
+ * reads, in one launch (up to 4 of one shape). */
+int br_hip_transpose_0213_group(const void* const* x, void* const* y, int count, int elem_bytes, int64_t s0,
+                                int64_t s1, int64_t s2, int64_t s3, br_stream_t stream);
 int br_hip_transpose_0213(const void* x, void* y, int elem_bytes, int64_t s0, int64_t s1,
                           int64_t s2, int64_t s3, br_stream_t stream);
 

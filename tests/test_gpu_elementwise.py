@@ -128,6 +128,23 @@ def test_transpose_0213_bit_exact(shape, eb):
     assert np.array_equal(host(y), np.ascontiguousarray(x.transpose(0, 2, 1, 3)))
 
 
+@pytest.mark.parametrize("shape,eb", [((2, 25, 3, 64), 4), ((1, 7, 5, 96), 2), ((2, 7, 3, 5), 4)])
+@pytest.mark.parametrize("chained", [False, True])
+def test_transpose_0213_of_several_tensors(shape, eb, chained):
+    """Three in one call; `chained`: the second reads what the first wrote, so they cannot run side by side."""
+    rng = np.random.default_rng(7)
+    dtype = torch.float32 if eb == 4 else torch.float16
+    x = [torch.from_numpy(rng.standard_normal(shape)).to(dtype).cuda() for _ in range(3)]
+    y = [torch.empty(x[0].numel(), dtype=dtype, device="cuda") for _ in range(3)]
+    if chained:
+        x[1] = y[0]
+    a, b = ((ctypes.c_void_p * 3)(*(t.data_ptr() for t in ts)) for ts in (x, y))
+    call("br_hip_transpose_0213_group", a, b, 3, eb, *shape, stream())
+    torch.cuda.synchronize()
+    for s, d in zip(x, y):
+        assert torch.equal(d, s.reshape(shape).permute(0, 2, 1, 3).reshape(-1))
+
+
 @pytest.mark.parametrize("rows,cols", [(2048, 4096), (77, 130), (1, 8), (512, 4096), (1000, 3080)])
 def test_colsum(rows, cols):
     rng = np.random.default_rng(6)
