@@ -107,6 +107,7 @@ Operand shared_operand(const void* p, int dtype, int64_t items, int compute) {
 // The two products of a linear layer's backward once the gradient dy[n,out] is
 // available in the products' type: weight_g[out,in] = dy^T . x, then
 // x_g[n,in] = dy . W (in that order: x_g may overwrite x).
+// (weight and weight_g may be the first rows of the `out` rows meant)
 int linear_backward_products(const Operand& dy, const tensor_t& x, const tensor_t& weight, const tensor_t& x_g,
                              const tensor_t& weight_g, int64_t n, int64_t in, int64_t out, int compute,
                              const br_column_sums* sums = nullptr) {
@@ -910,6 +911,142 @@ ComputingReturn hip_layernorm_backward_add(const tensor_t& dy, const tensor_t& s
     ComputingReturn r = dy->op_layernorm_backward(dy, scale, bias, var, y, dscale, dbias, din, eps);
     if (r != OP_OK) return r;
     return din->op_add(din, residual, din);
+}
+
+namespace {
+bool apart(const tensor_t& x, const tensor_t& y) {
+    auto begin = [](const tensor_t& t) { return reinterpret_cast<uintptr_t>(t->data()); };
+    auto end = [&](const tensor_t& t) { return begin(t) + t->items() * DataType_size(t->dtype()); };
+    return end(x) <= begin(y) || end(y) <= begin(x);
+}
+bool same_tensor(const tensor_t& x, const tensor_t& y) {
+    return x->data() == y->data() && x->items() == y->items() && x->dtype() == y->dtype();
+}
+bool same_shape(const tensor_t& x, const tensor_t& y) {
+    bool same = x->shape().dim() == y->shape().dim();
+    for (size_t i = 0; same && i < x->shape().dim(); i++) same = x->shape()[i] == y->shape()[i];
+    return same;
+}
+// `next` starts where `t` ends
+bool adjacent(const tensor_t& t, const tensor_t& next) {
+    return t->dtype() == next->dtype() && t->items() == next->items() &&
+           static_cast<const char*>(t->data()) + t->items() * DataType_size(t->dtype()) == static_cast<const char*>(next->data());
+}
+}  // namespace
+
+// op_layernorm_backward(ln[0..7], eps) followed by op_add(add[0], add[1], add[2]) of its din and a residual, and, unless
+// lin is null, by op_linear_backward(lin[0..6]) of that sum.  One pass of the LayerNorm kernel leaves din, the sum, and for
+// the linear layer the sum's 16-bit image and its bias gradient; anything else runs as the operators.
+ComputingReturn hip_layernorm_backward_then_add(const tensor_t* ln, float eps, const tensor_t* add, const tensor_t* lin) {
+    const tensor_t &dy = ln[0], &scale = ln[1], &bias = ln[2], &var = ln[3], &y = ln[4], &dscale = ln[5], &dbias = ln[6], &din = ln[7];
+    const bool first = same_tensor(add[0], din);
+    const tensor_t &residual = first ? add[1] : add[0], &sum = add[2];
+    bool fast = first != same_tensor(add[1], din) && (dev_f32(dy) && dy->shape().dim() == 3) && dev_f32(residual) && dev_f32(sum) &&
+                same_shape(residual, din) && same_shape(add[first ? 0 : 1], dy) && sum->items() == dy->items() &&
+                residual->items() == dy->items() && din->items() == dy->items();
+    for (int i = 1; fast && i < 8; i++) fast = dev_f32(ln[i]);
+    bool linear = false;
+    if (fast) {
+        const int64_t rows = (int64_t)(dy->shape()[0] * dy->shape()[1]), cols = (int64_t)dy->shape()[2];
+        fast = y->items() == dy->items() && (int64_t)var->items() >= rows && (int64_t)dscale->items() == cols &&
+               (int64_t)dbias->items() == cols && (int64_t)scale->items() == cols && (int64_t)bias->items() == cols &&
+               // the sum is written row by row, beside din: over the rows of dy or of the residual, or apart from all
+               apart(sum, din) && apart(sum, y) && apart(din, residual) && apart(din, y) && apart(din, dy) &&
+               (same_tensor(sum, residual) || apart(sum, residual)) && (same_tensor(sum, dy) || apart(sum, dy));
+        for (const tensor_t* t : {&scale, &bias, &var, &dscale, &dbias}) fast = fast && apart(sum, *t) && apart(din, *t);
+        if (fast) {
+            int compute = BR_GEMM_F32;
+            int64_t in = 0;
+            void* sum16 = nullptr;
+            float* sums = nullptr;
+            if (lin && same_tensor(lin[0], sum) && lin[0]->shape().dim() == 3 && dev(lin[1]) && lin[1]->shape().dim() == 3 &&
+                dev(lin[2]) && dev(lin[4]) && dev(lin[5]) && dev_f32(lin[6]) && (int64_t)lin[0]->shape()[2] == cols) {
+                compute = pick_compute({lin[0], lin[1], lin[2]});
+                in = (int64_t)lin[1]->shape()[2];
+                linear = compute != BR_GEMM_F32 && cols % 8 == 0 && (int64_t)lin[1]->items() == rows * in &&
+                         (int64_t)lin[2]->items() == cols * in && (int64_t)lin[4]->items() == rows * in &&
+                         (int64_t)lin[5]->items() == cols * in && (int64_t)lin[6]->items() == cols;
+                // the bias gradient is written before the LayerNorm's operands have all been read
+                for (int i = 0; i < 8; i++) linear = linear && apart(lin[6], ln[i]);
+                linear = linear && apart(lin[6], residual) && apart(lin[6], sum) && apart(lin[6], lin[1]) && apart(lin[6], lin[2]);
+            }
+            const int native = compute == BR_GEMM_F16 ? BR_F16 : BR_BF16;
+            if (linear) {
+                sum16 = ComputingContext::gemm_staging(1, (size_t)(rows * cols) * 2);
+                sums = static_cast<float*>(lin[6]->data());
+            }
+            const size_t need = br_hip_layernorm_bwd_sums_workspace(rows, cols);
+            void* ws = need <= head_bytes() ? ComputingContext::workspace : ComputingContext::scratch(need);
+            auto run = [&]() {
+                return br_hip_layernorm_bwd_add(
+                    static_cast<const float*>(dy->data()), static_cast<const float*>(y->data()),
+                    static_cast<const float*>(scale->data()), static_cast<const float*>(bias->data()),
+                    static_cast<const float*>(var->data()), static_cast<const float*>(residual->data()),
+                    static_cast<float*>(dscale->data()), static_cast<float*>(dbias->data()), static_cast<float*>(din->data()),
+                    static_cast<float*>(sum->data()), sum16, native, sums, rows, cols, eps, unlift(), ws, need, stream());
+            };
+            int rc = run();
+            if (rc == BR_ERR_TODO && linear) {
+                linear = false;
+                sum16 = nullptr;
+                sums = nullptr;
+                rc = run();
+            }
+            fast = rc != BR_ERR_TODO;
+            if (fast) BR_OP(rc);
+            if (fast && linear)
+                BR_OP(linear_backward_products(Operand{sum16, native}, lin[1], lin[2], lin[4], lin[5], rows, in, cols, compute));
+        }
+    }
+    if (!fast) {
+        ComputingReturn r = dy->op_layernorm_backward(dy, scale, bias, var, y, dscale, dbias, din, eps);
+        if (r != OP_OK) return r;
+        r = add[0]->op_add(add[0], add[1], add[2]);
+        if (r != OP_OK) return r;
+    }
+    if (lin && !(fast && linear)) return lin[0]->op_linear_backward(lin[0], lin[1], lin[2], lin[3], lin[4], lin[5], lin[6]);
+    return OP_OK;
+}
+
+// The backward pass of the query, key and value layers as the model scripts have it: acc = 0, then for each layer
+// op_linear_backward into `tmp` and acc += tmp.  lin: 3 x (dy x w b x_g w_g b_g).  Where the three read one x, their
+// weights and gradients lie one behind the other and tmp is not read afterwards (the caller's word), it is the backward
+// pass of ONE layer of three times the outputs: the gradients are packed side by side in the products' type, summed over
+// rows on the way, and two products are left of six.  BR_ERR_TODO: not of that form, nothing has been done.
+int hip_qkv_backward(const tensor_t& acc, const tensor_t* lin) {
+    const tensor_t &x = lin[1], &tmp = lin[4];
+    if (!dev_f32(acc) || !dev(x) || x->shape().dim() != 3 || !dev_f32(tmp) || tmp->items() != x->items() || acc->items() != x->items())
+        return BR_ERR_TODO;
+    const int64_t n = (int64_t)(x->shape()[0] * x->shape()[1]), in = (int64_t)x->shape()[2];
+    const int64_t out = (int64_t)(lin[6]->items());
+    for (int i = 0; i < 3; i++) {
+        const tensor_t* l = lin + 7 * i;
+        if (!dev_f32(l[0]) || l[0]->shape().dim() != 3 || (int64_t)(l[0]->shape()[0] * l[0]->shape()[1]) != n ||
+            (int64_t)l[0]->shape()[2] != out || !same_tensor(l[1], x) || !dev(l[2]) || !same_tensor(l[4], tmp) || !dev_f32(l[5]) ||
+            !dev_f32(l[6]) || (int64_t)l[2]->items() != out * in || (int64_t)l[5]->items() != out * in || (int64_t)l[6]->items() != out)
+            return BR_ERR_TODO;
+        if (i > 0 && !(adjacent(lin[7 * i - 5], l[2]) && adjacent(lin[7 * i - 2], l[5]) && adjacent(lin[7 * i - 1], l[6])))
+            return BR_ERR_TODO;
+        // what is written is neither read nor written by another part
+        for (const tensor_t* t : {&l[0], &l[1], &l[2]}) {
+            if (!apart(acc, *t) || !apart(tmp, *t)) return BR_ERR_TODO;
+            for (int j = 0; j < 3; j++)
+                if (!apart(lin[7 * j + 5], *t) || !apart(lin[7 * j + 6], *t)) return BR_ERR_TODO;
+        }
+        for (const tensor_t* t : {&l[5], &l[6]})
+            if (!apart(acc, *t) || !apart(tmp, *t) || !apart(l[5], lin[6]) || !apart(lin[5], l[6])) return BR_ERR_TODO;
+    }
+    if (!apart(acc, tmp)) return BR_ERR_TODO;
+    const int compute = pick_compute({lin[0], x, lin[2]});
+    const int native = compute == BR_GEMM_F16 ? BR_F16 : compute == BR_GEMM_BF16 ? BR_BF16 : BR_F32;
+    // one workgroup walks all rows of its columns
+    if (out % 8 != 0 || n > 4096) return BR_ERR_TODO;
+    void* packed = ComputingContext::gemm_staging(1, (size_t)(n * 3 * out) * (native == BR_F32 ? 4 : 2));
+    const float* dy[3] = {static_cast<const float*>(lin[0]->data()), static_cast<const float*>(lin[7]->data()),
+                          static_cast<const float*>(lin[14]->data())};
+    const int rc = br_hip_pack_colsum(dy, 3, static_cast<float*>(lin[6]->data()), packed, native, n, out, unlift(), stream());
+    if (rc != BR_OK) return rc;
+    return linear_backward_products(Operand{packed, native}, x, lin[2], acc, lin[5], n, in, 3 * out, compute);
 }
 
 // `op.layernorm_backward_add` followed by the `op.linear_backward` whose dy is the LayerNorm's din: the

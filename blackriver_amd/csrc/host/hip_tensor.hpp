@@ -98,6 +98,12 @@ ComputingReturn hip_layernorm_backward_add(const tensor_t& dy, const tensor_t& s
                                            const tensor_t& var, const tensor_t& y, const tensor_t& dscale,
                                            const tensor_t& dbias, const tensor_t& residual, const tensor_t& din,
                                            float eps);
+// op_layernorm_backward (ln: dy scale bias var y dscale dbias din) followed by op_add (add: a b c) of din and a residual
+// and, unless lin is null, by op_linear_backward (lin: dy x w b x_g w_g b_g) of the sum.
+ComputingReturn hip_layernorm_backward_then_add(const tensor_t* ln, float eps, const tensor_t* add, const tensor_t* lin);
+// acc = the sum of the input gradients of three linear layers over one x (lin: 3 x (dy x w b x_g w_g b_g)), their weight
+// and bias gradients; BR_ERR_TODO unless they can be taken as one layer, in which case x_g is left alone.
+int hip_qkv_backward(const tensor_t& acc, const tensor_t* lin);
 // The same followed by the linear backward whose output gradient is din (x, weight, bias of that layer and its
 // three gradients): din's 16-bit image and the bias gradient come out of the LayerNorm kernel.
 ComputingReturn hip_layernorm_backward_add_linear_backward(

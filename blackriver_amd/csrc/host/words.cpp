@@ -445,6 +445,70 @@ BR_WORD(LayernormBackwardAddLinearBackward,
     }
 )
 
+// ( dy scale bias var y dscale dbias din eps   a b c   dy' x w b x_g w_g b_g -- )  `op.layernorm_backward`, `op.add` and
+// `op.linear_backward` in a row: one pass where the sum is of din and the linear layer's dy is the sum
+BR_WORD(LayernormBackwardThenAddLinear,
+    Tensors<7> l(stack);
+    Tensors<3> c(stack);
+    const float eps = (float)stack.pop_number();
+    Tensors<8> a(stack);
+    op_check_word(hip_layernorm_backward_then_add(a.t, eps, c.t, l.t), "op.layernorm_backward + op.add + op.linear_backward");
+)
+// ( xa   3 x (dy x w b xb w_g b_g   xa xb xa)   dy scale bias var y dscale dbias din eps   a b c -- )
+// the backward pass of the query, key and value layers (`op.zero` and three times `op.linear_backward op.add`) and of the
+// LayerNorm ahead of them (`op.layernorm_backward op.add`).  Where the LayerNorm writes its din over xb, nobody sees the
+// three layers' own input gradients: they are formed as one layer's.
+BR_WORD(QkvBackwardLayernorm,
+    Tensors<3> c(stack);
+    const float eps = (float)stack.pop_number();
+    Tensors<8> n(stack);
+    Tensors<3> add2(stack);
+    Tensors<7> l2(stack);
+    Tensors<3> add1(stack);
+    Tensors<7> l1(stack);
+    Tensors<3> add0(stack);
+    Tensors<7> l0(stack);
+    Tensors<1> z(stack);
+    Tensors<7>* const layer[3] = {&l0, &l1, &l2};
+    Tensors<3>* const add[3] = {&add0, &add1, &add2};
+    auto same = [](const tensor_t& x, const tensor_t& y) {
+        return x->data() == y->data() && x->items() == y->items() && x->dtype() == y->dtype();
+    };
+    auto apart = [](const tensor_t& x, const tensor_t& y) {
+        const char* p = static_cast<const char*>(x->data());
+        const char* q = static_cast<const char*>(y->data());
+        return p + x->items() * DataType_size(x->dtype()) <= q || q + y->items() * DataType_size(y->dtype()) <= p;
+    };
+    const tensor_t& xa = z[0];
+    const tensor_t& xb = l0[4];
+    bool one = xa->is_cuda() && xb->is_cuda();
+    for (int i = 0; one && i < 3; i++) {
+        for (int j = 0; one && j < 7; j++) one = (*layer[i])[j]->is_cuda();
+        for (int j = 0; one && j < 3; j++) one = (*add[i])[j]->is_cuda();
+        one = one && same((*add[i])[0], xa) && same((*add[i])[1], xb) && same((*add[i])[2], xa) && same((*layer[i])[4], xb);
+    }
+    // xb is written whole by the LayerNorm, which reads nothing of it
+    for (int j = 0; one && j < 8; j++) one = n[j]->is_cuda() && (j == 7 ? same(n[j], xb) : apart(n[j], xb));
+    if (one) {
+        tensor_t lin[21];
+        for (int i = 0; i < 3; i++)
+            for (int j = 0; j < 7; j++) lin[7 * i + j] = (*layer[i])[j];
+        const int rc = hip_qkv_backward(xa, lin);
+        one = rc != BR_ERR_TODO;
+        if (one) BR_HIP_CHECK(rc);
+    }
+    if (!one) {
+        xa->op_zero(xa);
+        for (int i = 0; i < 3; i++) {
+            Tensors<7>& l = *layer[i];
+            Tensors<3>& s = *add[i];
+            l[0]->op_linear_backward(l[0], l[1], l[2], l[3], l[4], l[5], l[6]);
+            s[0]->op_add(s[0], s[1], s[2]);
+        }
+    }
+    op_check_word(hip_layernorm_backward_then_add(n.t, eps, c.t, nullptr), "op.layernorm_backward + op.add");
+)
+
 // AdamW.  The reference stops at the gradients; these words are what a training
 // loop runs after them.
 struct AdamWHyper {
@@ -557,6 +621,8 @@ void load_nn_words(Enviroment& env) {
         {"op.softmax_backward", SoftmaxBackward::creator},
         {"op.softmax_attn_backward", SoftmaxAttnBackward::creator},
         {"op.qk_backward", QueryKeyBackward::creator},
+        {"op.layernorm_backward_then_add_linear_backward", LayernormBackwardThenAddLinear::creator},
+        {"op.qkv_backward_layernorm", QkvBackwardLayernorm::creator},
         {"op.transpos_0213_x3", Transpos0213x3::creator},
         {"op.gelu_linear_backward", GeluLinearBackward::creator},
         {"op.linear_add", LinearAdd::creator},
@@ -579,6 +645,9 @@ void load_nn_words(Enviroment& env) {
     env.insert_fusion({"op.layernorm", "op.copy"}, "op.layernorm_copy");
     env.insert_fusion({"op.gelu_backward", "op.linear_backward"}, "op.gelu_linear_backward");
     env.insert_fusion({"op.transpos_0213", "op.transpos_0213", "op.transpos_0213"}, "op.transpos_0213_x3");
+    env.insert_fusion({"op.zero", "op.linear_backward", "op.add", "op.linear_backward", "op.add", "op.linear_backward", "op.add",
+                       "op.layernorm_backward", "op.add"}, "op.qkv_backward_layernorm");
+    env.insert_fusion({"op.layernorm_backward", "op.add", "op.linear_backward"}, "op.layernorm_backward_then_add_linear_backward");
     // the pair also stands across a block boundary of a model program
     env.insert_fusion({"op.layernorm_backward_add", "op.linear_backward"}, "op.layernorm_backward_add_linear_backward", true);
 }

@@ -895,6 +895,77 @@ int colsum_owner_launch(int lanes, const Src& src, float* out, int64_t rows, int
     return BR_OK;
 }
 
+// Several fp32 matrices packed side by side, columns summed on the way: blockIdx.y is the matrix, a workgroup owns a
+// strip of LPR quads of its columns as in colsum_owner_kernel.
+constexpr int kPacked = 4;
+struct PackSet {
+    const float* x[kPacked];
+};
+template <int LPR, typename D>
+__global__ __launch_bounds__(kOwnThreads) void pack_colsum_kernel(PackSet set, float* __restrict__ out, D* __restrict__ packed,
+                                                                  int64_t rows, int64_t cols, int64_t pitch, float scale) {
+    constexpr int VEC = 4, UNROLL = 4, RPP = kOwnThreads / LPR, CW = LPR * VEC, WAVES = kOwnThreads / 64;
+    __shared__ float slots[WAVES][CW];
+    const float* x = set.x[0];
+#pragma unroll
+    for (int i = 1; i < kPacked; i++)
+        if (blockIdx.y == (unsigned)i) x = set.x[i];
+    out += blockIdx.y * cols;
+    packed += blockIdx.y * cols;
+    const int lr = threadIdx.x % LPR, rr = threadIdx.x / LPR;
+    const int64_t strip = xcd_contiguous(blockIdx.x, gridDim.x);
+    const int64_t col = strip * CW + lr * VEC;
+    float acc[VEC] = {0.f, 0.f, 0.f, 0.f};
+    if (col < cols) {
+        for (int64_t r = rr; r < rows; r += UNROLL * RPP) {
+            float in[UNROLL][VEC];
+            // positions past the last row read that row (every load of a pass leaves before the first is used)
+#pragma unroll
+            for (int u = 0; u < UNROLL; u++) {
+                const int64_t at = r + u * RPP;
+                VecIO<float, VEC>::load(x + (at < rows ? at : rows - 1) * cols + col, in[u]);
+            }
+#pragma unroll
+            for (int u = 0; u < UNROLL; u++) {
+                if (r + u * RPP >= rows) break;
+                D* const to = packed + (r + u * RPP) * pitch + col;
+                if constexpr (sizeof(D) == 4) VecIO<float, VEC>::store(to, in[u]);
+                else store4_as16<D>(to, in[u]);
+#pragma unroll
+                for (int j = 0; j < VEC; j++) acc[j] += in[u][j];
+            }
+        }
+    }
+#pragma unroll
+    for (int d = LPR; d < 64; d *= 2)
+#pragma unroll
+        for (int j = 0; j < VEC; j++) acc[j] += __shfl_xor(acc[j], d);
+    if ((threadIdx.x & 63) < LPR) {
+#pragma unroll
+        for (int j = 0; j < VEC; j++) slots[threadIdx.x >> 6][lr * VEC + j] = acc[j];
+    }
+    __syncthreads();
+    if (threadIdx.x < CW) {
+        float z = 0.f;
+#pragma unroll
+        for (int k = 0; k < WAVES; k++) z += slots[k][threadIdx.x];
+        const int64_t oc = strip * CW + threadIdx.x;
+        if (oc < cols) out[oc] = z * scale;
+    }
+}
+template <typename D>
+int pack_colsum(const PackSet& set, int count, float* out, void* packed, int64_t rows, int64_t cols, float scale, hipStream_t st) {
+    // lanes per row as in owner_lanes: the narrowest strips whose workgroups fit the chip
+    const int lanes = rows <= 128 ? 8 : count * cols / 8 <= 512 ? 2 : count * cols / 16 <= 512 ? 4 : 8;
+    const dim3 grid((unsigned)((cols + lanes * 4 - 1) / (lanes * 4)), (unsigned)count);
+    D* const p = (D*)packed;
+    if (lanes == 2) pack_colsum_kernel<2, D><<<grid, kOwnThreads, 0, st>>>(set, out, p, rows, cols, count * cols, scale);
+    else if (lanes == 4) pack_colsum_kernel<4, D><<<grid, kOwnThreads, 0, st>>>(set, out, p, rows, cols, count * cols, scale);
+    else pack_colsum_kernel<8, D><<<grid, kOwnThreads, 0, st>>>(set, out, p, rows, cols, count * cols, scale);
+    BR_HIP_LAUNCH_CHECK();
+    return BR_OK;
+}
+
 // ------------------------------------------------------- transpose 0213
 // One 16-byte granule per thread, indexed by OUTPUT position so stores are
 // fully coalesced; loads are contiguous runs of s3 elements.
@@ -1522,6 +1593,25 @@ int br_hip_colsum_cast(const float* x, float* out, void* x16, int x16_dtype, int
         colsum_cast_partial<__hip_bfloat16><<<grid, kBlock, 0, st>>>(x, partial, (__hip_bfloat16*)x16, rows, cols, rpb);
     BR_HIP_LAUNCH_CHECK();
     return colsum_finish(partial, out, groups, cols, out_scale, st);
+}
+
+int br_hip_pack_colsum(const float* const* x, int count, float* out, void* packed, int packed_dtype, int64_t rows,
+                       int64_t cols, float out_scale, br_stream_t stream) {
+    if (rows <= 0 || cols <= 0 || count <= 0) return BR_ERR_ATTR;
+    if (!x) return BR_ERR_INPUT;
+    if (!out || !packed) return BR_ERR_OUTPUT;
+    if (count > kPacked || cols % 8 != 0 || !aligned16(packed) || cols > (1 << 24)) return BR_ERR_TODO;
+    PackSet set = {};
+    for (int i = 0; i < count; i++) {
+        if (!x[i]) return BR_ERR_INPUT;
+        if (!aligned16(x[i])) return BR_ERR_TODO;
+        set.x[i] = x[i];
+    }
+    hipStream_t st = as_stream(stream);
+    if (packed_dtype == BR_F32) return pack_colsum<float>(set, count, out, packed, rows, cols, out_scale, st);
+    if (packed_dtype == BR_F16) return pack_colsum<__half>(set, count, out, packed, rows, cols, out_scale, st);
+    if (packed_dtype == BR_BF16) return pack_colsum<__hip_bfloat16>(set, count, out, packed, rows, cols, out_scale, st);
+    return BR_ERR_TODO;
 }
 
 int br_hip_gelu_bwd_colsum_cast(const float* dy, const float* x, float* dx, float* out, void* dx16, int dx16_dtype,

@@ -131,6 +131,7 @@ __global__ __launch_bounds__(kWalker * GROUPS) void ln_bwd_regs(const float* dy,
                                                                  float* __restrict__ part_dbeta, int64_t rows,
                                                                  int cols4, float eps, float inv_cols,
                                                                  const float* residual,
+                                                                 float* sum = nullptr,
                                                                  float* __restrict__ part_dx = nullptr,
                                                                  Copy16 dx16 = Copy16{nullptr, 0}) {
     __shared__ float lds[2][GROUPS][2 * kWaves];
@@ -223,6 +224,7 @@ __global__ __launch_bounds__(kWalker * GROUPS) void ln_bwd_regs(const float* dy,
         }
         const float m1 = s[0] * inv_cols, m2 = s[1] * inv_cols;
         float4* dxr = reinterpret_cast<float4*>(dx) + row * cols4;
+        float4* outr = sum ? reinterpret_cast<float4*>(sum) + row * cols4 : dxr;
 #pragma unroll
         for (int i = 0; i < VPT; i++) {
             const int idx = tid + i * kWalker;
@@ -235,9 +237,10 @@ __global__ __launch_bounds__(kWalker * GROUPS) void ln_bwd_regs(const float* dy,
                 if (residual) {
                     // dx is rounded to fp32 before the add, as a separate add kernel would see it
                     asm volatile("" : "+v"(o.x), "+v"(o.y), "+v"(o.z), "+v"(o.w));
+                    if (sum) dxr[idx] = o;
                     o.x += res[i].x; o.y += res[i].y; o.z += res[i].z; o.w += res[i].w;
                 }
-                dxr[idx] = o;  // an ordinary store: measured faster here than the streaming form
+                outr[idx] = o;  // an ordinary store: measured faster here than the streaming form
                 if (SUMS) {
                     store4_as16(dx16, row * cols4 + idx, o);   // o as stored, rounded once more
                     float4& ax = acc_x[SUMS ? i : 0];
@@ -520,12 +523,13 @@ size_t br_hip_layernorm_bwd_sums_workspace(int64_t rows, int64_t cols) {
     return br_hip_layernorm_bwd_workspace(rows, cols) / 2 * 3;   // a third partial array
 }
 
-// dx16 / dx_sum (both or neither): the 16-bit copy and the column sums of dx, register path only
+// dx16 / dx_sum (both or neither): the 16-bit copy and the column sums of dx, register path only.  sum: dx keeps what it
+// is without the residual, dx + residual goes there, and is what dx16 / dx_sum are of.
 static int layernorm_bwd_impl(const float* dy, const float* y, const float* gamma, const float* beta,
                               const float* var, const float* residual, float* dgamma, float* dbeta, float* dx,
                               int64_t rows, int64_t cols, float eps, float param_scale, void* workspace,
                               size_t workspace_bytes, br_stream_t stream, void* dx16 = nullptr, int dx16_dtype = 0,
-                              float* dx_sum = nullptr) {
+                              float* dx_sum = nullptr, float* sum = nullptr) {
     if (rows < 0 || cols <= 0 || rows > 0x7fffffff) return BR_ERR_ATTR;
     if (!dgamma || !dbeta) return BR_ERR_OUTPUT;
     const bool sums = dx_sum != nullptr;
@@ -542,7 +546,7 @@ static int layernorm_bwd_impl(const float* dy, const float* y, const float* gamm
     int parts;
     float* part_g = (float*)workspace;
     const bool regs = regs_path_ok(cols, dy, y, gamma, beta, dx) && aligned16(workspace) &&
-                      (!residual || aligned16(residual));
+                      (!residual || aligned16(residual)) && (!sum || aligned16(sum));
     if (residual && !regs) return BR_ERR_TODO;  // only the register path adds the residual
     const int cols4 = (int)(cols / 4);
     const int vpt = (cols4 + kBlock - 1) / kBlock;
@@ -562,10 +566,10 @@ static int layernorm_bwd_impl(const float* dy, const float* y, const float* gamm
     do {                                                                                                             \
         if (sums)                                                                                                    \
             ln_bwd_regs<V, W, true><<<parts, kWalker * W, 0, st>>>(dy, y, gamma, beta, var, dx, part_g, part_b, rows, \
-                                                                   cols4, eps, inv, residual, part_x, c16);          \
+                                                                   cols4, eps, inv, residual, sum, part_x, c16);     \
         else                                                                                                         \
             ln_bwd_regs<V, W><<<parts, kWalker * W, 0, st>>>(dy, y, gamma, beta, var, dx, part_g, part_b, rows,      \
-                                                             cols4, eps, inv, residual);                             \
+                                                             cols4, eps, inv, residual, sum);                        \
     } while (0)
         // Rows wider than 4096 floats keep 8 quads per thread in flight twice over; with two walkers (512
         // threads, 256 registers per wave) that spills, so they run one walker per workgroup.
@@ -573,7 +577,7 @@ static int layernorm_bwd_impl(const float* dy, const float* y, const float* gamm
         else if (vpt <= 2) BR_LN_BWD(2, G);
         else if (vpt <= 4) BR_LN_BWD(4, G);
         else ln_bwd_regs<8, 1><<<parts, kWalker, 0, st>>>(dy, y, gamma, beta, var, dx, part_g, part_b, rows, cols4, eps,
-                                                          inv, residual);
+                                                          inv, residual, sum);
 #undef BR_LN_BWD
         BR_HIP_LAUNCH_CHECK();
         if (aligned16(dgamma) && aligned16(dbeta)) {
@@ -635,6 +639,17 @@ int br_hip_layernorm_bwd_residual_sums(const float* dy, const float* y, const fl
     if (rows == 0) residual = nullptr;
     return layernorm_bwd_impl(dy, y, gamma, beta, var, residual, dgamma, dbeta, dx, rows, cols, eps, param_scale,
                               workspace, workspace_bytes, stream, dx16, dx16_dtype, dx_sum);
+}
+
+int br_hip_layernorm_bwd_add(const float* dy, const float* y, const float* gamma, const float* beta, const float* var,
+                             const float* residual, float* dgamma, float* dbeta, float* dx, float* sum, void* sum16,
+                             int sum16_dtype, float* column_sums, int64_t rows, int64_t cols, float eps, float param_scale,
+                             void* workspace, size_t workspace_bytes, br_stream_t stream) {
+    if (rows > 0 && !residual) return BR_ERR_INPUT;
+    if (!sum || sum == dx || (column_sums != nullptr) != (sum16 != nullptr)) return BR_ERR_OUTPUT;
+    if (rows == 0) residual = nullptr;
+    return layernorm_bwd_impl(dy, y, gamma, beta, var, residual, dgamma, dbeta, dx, rows, cols, eps, param_scale,
+                              workspace, workspace_bytes, stream, sum16, sum16_dtype, column_sums, sum);
 }
 
 int br_hip_layernorm_bwd_residual(const float* dy, const float* y, const float* gamma, const float* beta,

@@ -144,6 +144,13 @@ int br_hip_transpose_0213(const void* x, void* y, int elem_bytes, int64_t s0, in
 size_t br_hip_colsum_workspace(int64_t rows, int64_t cols);
 int br_hip_colsum(const void* x, int dtype, float* out, int64_t rows, int64_t cols, float out_scale,
                   void* workspace, size_t workspace_bytes, br_stream_t stream);
+/* `count` (up to 4) fp32 matrices [rows, cols] side by side: packed[r, i * cols + c]
+ * = x[i][r, c] in packed_dtype, and out[i * cols + c] = out_scale * sum_r x[i][r, c]:
+ * the bias gradients of the query, key and value layers and the operand of
+ * their products as one layer of 3 * cols outputs.  BR_ERR_TODO unless
+ * cols % 8 == 0 and everything is 16-byte aligned. */
+int br_hip_pack_colsum(const float* const* x, int count, float* out, void* packed, int packed_dtype, int64_t rows,
+                       int64_t cols, float out_scale, br_stream_t stream);
 /* The same column sums of an fp32 x together with a 16-bit copy of x (x16,
  * BR_F16 or BR_BF16, dense [rows, cols]) in one pass: op_linear_backward
  * (cuda_tensor.cpp:730-812) needs the sums as the bias gradient and, with a
@@ -221,6 +228,17 @@ int br_hip_layernorm_bwd_residual(const float* dy, const float* y, const float* 
                                   int64_t cols, float eps, float param_scale, void* workspace,
                                   size_t workspace_bytes, br_stream_t stream);
 
+/* op_layernorm_backward followed by op_add of a residual into a tensor of its
+ * own: dx is what op_layernorm_backward leaves, sum = dx + residual (residual's
+ * or dy's own buffer if need be), and, where asked for (both or neither), sum16 and
+ * column_sums are the 16-bit image and the scaled column sums of sum.  Bits as
+ * the separate entries'.  BR_ERR_TODO as for br_hip_layernorm_bwd_residual, or
+ * with sums as for br_hip_layernorm_bwd_residual_sums, whose workspace it takes. */
+int br_hip_layernorm_bwd_add(const float* dy, const float* y, const float* gamma, const float* beta,
+                             const float* var, const float* residual, float* dgamma, float* dbeta, float* dx,
+                             float* sum, void* sum16, int sum16_dtype, float* column_sums, int64_t rows,
+                             int64_t cols, float eps, float param_scale, void* workspace,
+                             size_t workspace_bytes, br_stream_t stream);
 /* The same followed by what the `op.linear_backward` of the layer below does to
  * dx first (cuda_tensor.cpp:738-760: its bias gradient, the column sums of dx;
  * and, for 16-bit products, the 16-bit image of dx both of its products read):

@@ -706,3 +706,46 @@ def test_block_at_the_full_headline_size_against_oracle(runtime):
     env.execute("create_operand_buffers create_flash_buffers prepare_batch_flash")
     check("block_step_flash", "layer_forward_flash", "fused-attention words")
     env.close()
+
+
+BACKWARD_SPLITS = {   # the words of a program, as they are and with each run by itself
+    "plain": ("layer_forward", "layer_backward_core"),
+    "mixed": ("layer_forward_mixed", "layer_backward_mixed"),
+}
+
+
+@pytest.mark.parametrize("mode,words", [("fp32", "plain"), ("f16", "plain"), ("f16", "mixed"), ("bf16", "mixed")])
+@pytest.mark.parametrize("hidden,heads,batch,tokens", [(256, 4, 2, 24), (512, 4, 1, 130)])
+def test_fused_block_words_against_the_words_one_by_one(runtime, mode, words, hidden, heads, batch, tokens):
+    """A whole step as one program, with what the word machine joins, against the same words with a `1 drop` between them,
+    which keeps them apart: every tensor a step leaves.  Joined query, key and value gradients are summed in another order."""
+    print("case", mode, words, hidden, tokens, flush=True)
+    left = ["xa", "xb", "xc", "yout_g", "xattn_in", "xattn_out", "x4a", "xquery", "xkey", "xvalue"] + GRADIENTS
+    if words == "mixed":
+        left = [n for n in left if n != "xattn_out"] + ["xattn_out.h", "xa.h", "xb.h", "xc.h", "zquery.h", "zkey.h", "zvalue.h", "x4b.h"]
+    out = {}
+    for joined in (True, False):
+        env, *_ = setup_block(runtime, hidden, heads, batch, tokens, mode)
+        if words == "mixed":
+            env.execute("create_operand_buffers")
+        for word in BACKWARD_SPLITS[words]:
+            env.execute(word if joined else apart_text(word))
+        env.execute("op.sync")
+        out[joined] = {n: env.read(n) for n in left}
+        env.close()
+    # one rounding of an fp32 sum (f32), of a 16-bit operand made from it
+    tol = {"fp32": 1e-5, "f16": 2e-3, "bf16": 1.6e-2}[mode]
+    for n in left:
+        assert_close(out[True][n], out[False][n], tol, n)
+
+
+GRADIENTS = ["input_layernorm.weight_g", "input_layernorm.bias_g", "post_attention_layernorm.weight_g",
+             "post_attention_layernorm.bias_g", "query_key_value.weight_g", "query_key_value.bias_g", "dense.weight_g",
+             "dense.bias_g", "dense_h_to_4h.weight_g", "dense_h_to_4h.bias_g", "dense_4h_to_h.weight_g", "dense_4h_to_h.bias_g"]
+
+
+def apart_text(word):
+    """The definition of `word` in the package's word file with `1 drop` after every line."""
+    text = host.words_text("bloom.words")
+    body = text.split("%def " + word + "\n")[1].split("%end")[0]
+    return "\n".join(line + "  1 drop" for line in body.splitlines() if line.strip() and not line.strip().startswith(";;"))

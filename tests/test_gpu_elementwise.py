@@ -145,6 +145,20 @@ def test_transpose_0213_of_several_tensors(shape, eb, chained):
         assert torch.equal(d, s.reshape(shape).permute(0, 2, 1, 3).reshape(-1))
 
 
+@pytest.mark.parametrize("dtype", [F32, F16, BF16])
+@pytest.mark.parametrize("rows,cols,count", [(1, 8, 3), (129, 264, 3), (1000, 1024, 3), (513, 1400, 2), (2049, 8, 4), (300, 2736, 3)])
+def test_pack_colsum_is_exact_on_integers(rows, cols, count, dtype):
+    torch.manual_seed(rows)
+    x = [torch.randint(-4, 5, (rows, cols), device="cuda").float() for _ in range(count)]
+    packed = torch.full((rows, count * cols), 77, dtype={F32: torch.float32, F16: torch.float16, BF16: torch.bfloat16}[dtype], device="cuda")
+    out = torch.full((count * cols,), float("nan"), device="cuda")
+    at = (ctypes.c_void_p * count)(*(t.data_ptr() for t in x))
+    call("br_hip_pack_colsum", at, count, ptr(out), ptr(packed), dtype, rows, cols, 0.5, stream())
+    torch.cuda.synchronize()
+    want = torch.cat(x, 1)
+    assert torch.equal(packed.float(), want) and torch.equal(out, 0.5 * want.sum(0))
+
+
 @pytest.mark.parametrize("rows,cols", [(2048, 4096), (77, 130), (1, 8), (512, 4096), (1000, 3080)])
 def test_colsum(rows, cols):
     rng = np.random.default_rng(6)

@@ -213,6 +213,38 @@ def test_layernorm_bwd_with_residual_sums_and_16_bit_copy(rows, cols, dtype, tdt
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("alias", ["none", "residual", "dy"])
+@pytest.mark.parametrize("rows,cols,dtype", [(1, 256, F16), (37, 1024, BF16), (513, 2048, F16), (250, 4096, None), (5, 8192, None)])
+def test_layernorm_bwd_with_the_sum_beside_it(rows, cols, dtype, alias):
+    """dx and dx + residual of one pass: dx, dgamma, dbeta bit for bit br_hip_layernorm_bwd's, the sum, its 16-bit image
+    and its column sums bit for bit br_hip_layernorm_bwd_residual_sums'; the sum may lie over the residual or over dy."""
+    print("case rows=%d cols=%d alias=%s" % (rows, cols, alias), flush=True)
+    x, g, b, dy = make(rows, cols, seed=9)
+    res = np.random.default_rng(10).standard_normal((rows, cols)).astype(np.float32)
+    y, _, var = orc.layernorm_fwd(x, g, b, 1e-5)
+    t_dy, t_y, t_g, t_b, t_var, t_res = (dev(a) for a in (dy, y, g, b, var, res))
+    ws = workspace(hip.load().br_hip_layernorm_bwd_sums_workspace(rows, cols))
+    args = (ptr(t_dy), ptr(t_y), ptr(t_g), ptr(t_b), ptr(t_var))
+    tail = (rows, cols, 1e-5, 0.25, ptr(ws), ws.numel(), stream())
+    dg, db, dx = empty(cols), empty(cols), empty((rows, cols))
+    call("br_hip_layernorm_bwd", *args, ptr(dg), ptr(db), ptr(dx), *tail)
+    want = {"sum": dx + t_res}
+    if dtype is not None:
+        d16 = torch.float16 if dtype == F16 else torch.bfloat16
+        want["sum16"], want["sums"] = torch.zeros((rows, cols), dtype=d16, device="cuda"), empty(cols)
+        call("br_hip_layernorm_bwd_residual_sums", *args, ptr(t_res), ptr(empty(cols)), ptr(empty(cols)), ptr(empty((rows, cols))),
+             ptr(want["sum16"]), dtype, ptr(want["sums"]), *tail)
+    got = {n: torch.full_like(t, 7) for n, t in want.items()}
+    got["sum"] = {"none": got["sum"], "residual": t_res, "dy": t_dy}[alias]
+    dg2, db2, dx2 = empty(cols), empty(cols), empty((rows, cols))
+    call("br_hip_layernorm_bwd_add", *args, ptr(t_res), ptr(dg2), ptr(db2), ptr(dx2), ptr(got["sum"]), ptr(got.get("sum16")),
+         dtype or 0, ptr(got.get("sums")), *tail)
+    torch.cuda.synchronize()
+    assert torch.equal(dx2, dx) and torch.equal(dg2, dg) and torch.equal(db2, db)
+    for name in want:
+        assert torch.equal(got[name], want[name]), name
+
+
 def test_layernorm_bwd_param_scale_is_an_exact_power_of_two_factor():
     """dy lifted by S = 1024 with param_scale = 1/S: dx comes out S times the
     plain one and dgamma / dbeta equal the plain ones, all bit for bit (scaling
