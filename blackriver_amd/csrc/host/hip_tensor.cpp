@@ -1041,6 +1041,9 @@ int hip_qkv_backward(const tensor_t& acc, const tensor_t* lin) {
     const int native = compute == BR_GEMM_F16 ? BR_F16 : compute == BR_GEMM_BF16 ? BR_BF16 : BR_F32;
     // one workgroup walks all rows of its columns
     if (out % 8 != 0 || n > 4096) return BR_ERR_TODO;
+    // fp32: one sum over three times the K is as exact as three sums on the kernel that adds up in pieces
+    auto aligned = [](const tensor_t& t) { return reinterpret_cast<uintptr_t>(t->data()) % 16 == 0; };
+    if (native == BR_F32 && (in % 4 != 0 || !aligned(x) || !aligned(lin[2]))) return BR_ERR_TODO;
     void* packed = ComputingContext::gemm_staging(1, (size_t)(n * 3 * out) * (native == BR_F32 ? 4 : 2));
     const float* dy[3] = {static_cast<const float*>(lin[0]->data()), static_cast<const float*>(lin[7]->data()),
                           static_cast<const float*>(lin[14]->data())};

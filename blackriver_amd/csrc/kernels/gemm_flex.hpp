@@ -275,12 +275,17 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
     };
 
     f32x16 acc[FM][FN];
+    constexpr bool kFold = CT == BR_GEMM_F32 && !WORDS;   // see below
+    f32x16 held[kFold ? FM : 1][kFold ? FN : 1];
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
         for (int j = 0; j < FN; j++)
 #pragma unroll
-            for (int v = 0; v < 16; v++) acc[i][j][v] = 0.f;
+            for (int v = 0; v < 16; v++) {
+                acc[i][j][v] = 0.f;
+                if (kFold) held[kFold ? i : 0][kFold ? j : 0][v] = 0.f;
+            }
 
 #pragma unroll
     for (int s = 0; s < ST; s++)
@@ -322,15 +327,33 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
                         else
                             acc[i][j] = Cvt<CT>::mfma(fb[ks][j], fa[ks][i], acc[i][j]);
                     }
+        // fp32 sums of 64 k-values go to a second set of registers, so that rounding errors grow with the number of such
+        // sums and not with K: against 64 bits, [512 x 1024] from K = 1024 2.9e-7 -> 1.6e-7, from 4096 5.7e-7 -> 1.7e-7.  An
+        // addition and a move per 128 clocks of products; it has to fit 256 registers, so that two waves share a SIMD (with
+        // one a block's step is 11 % slower), which it does not where values are loaded one by one (WORDS).
+        if constexpr (kFold) {
+            if ((t & 1) || t + 1 == mine) {
+#pragma unroll
+                for (int i = 0; i < FM; i++)
+#pragma unroll
+                    for (int j = 0; j < FN; j++)
+#pragma unroll
+                        for (int v = 0; v < 16; v++) {
+                            held[i][j][v] += acc[i][j][v];
+                            acc[i][j][v] = 0.f;
+                        }
+            }
+        }
     }
 
-    flex_park<BM, BN>(acc, mem, lane);
+    if constexpr (kFold) flex_park<BM, BN>(held, mem, lane);
+    else flex_park<BM, BN>(acc, mem, lane);
     __syncthreads();
     flex_emit<BM, BN, KW, KW * 64, TC, GELU>(g, (lds_byte*)lds_raw, kWaveBytes, row0, col0, b);
 }
 
 template <int CT, int BM, int BN, int KW, int ST, bool A_KSTR, bool B_KSTR, typename TC, bool GELU = false, bool WORDS = false>
-__global__ __launch_bounds__(KW * 64) void gemm_flex_kernel(GemmArgs g) {
+__global__ __launch_bounds__(KW * 64, CT == BR_GEMM_F32 && !WORDS ? 2 : 1) void gemm_flex_kernel(GemmArgs g) {
     __shared__ __attribute__((aligned(1024))) unsigned char lds[flex_lds_bytes<BM, BN, KW, ST>()];
     flex_product<CT, BM, BN, KW, ST, A_KSTR, B_KSTR, TC, GELU, WORDS, true>(g, blockIdx.x, gridDim.x, lds);
 }

@@ -79,7 +79,7 @@ __device__ __forceinline__ void sum_strip(const ColumnSums& s, int strip, float*
 // Workgroups [0, n1) run `a`, [n1, n1 + n2) run `b`, those after them the column sums.  AK1 .. BK2: which operands are
 // row-contiguous.
 template <int CT, int BM, int BN, int KW, int ST, bool AK1, bool BK1, typename TC1, bool AK2, bool BK2, typename TC2>
-__global__ __launch_bounds__(KW * 64) void gemm_flex_pair_kernel(GemmArgs a, GemmArgs b, unsigned n1, unsigned n2, ColumnSums sums) {
+__global__ __launch_bounds__(KW * 64, CT == BR_GEMM_F32 ? 2 : 1) void gemm_flex_pair_kernel(GemmArgs a, GemmArgs b, unsigned n1, unsigned n2, ColumnSums sums) {
     static_assert(KW == 4, "the column sums are four waves'");
     __shared__ __attribute__((aligned(1024))) unsigned char lds[flex_lds_bytes<BM, BN, KW, ST>()];
     const unsigned id = blockIdx.x;
