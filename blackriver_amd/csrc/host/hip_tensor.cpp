@@ -934,6 +934,137 @@ bool adjacent(const tensor_t& t, const tensor_t& next) {
 }
 }  // namespace
 
+namespace {
+// A linear layer's operands (lin: x w b y), checked as op_linear checks them.
+bool linear_ok(const tensor_t* lin) {
+    const tensor_t &x = lin[0], &w = lin[1], &b = lin[2], &y = lin[3];
+    if (!dev(x) || !dev(w) || !dev_f32(b) || !dev(y) || x->shape().dim() != 3 || w->shape().dim() != 2) return false;
+    const size_t n = x->shape()[0] * x->shape()[1], in = x->shape()[2], out = w->shape()[0];
+    return w->shape()[1] == in && b->items() == out && y->items() == n * out;
+}
+// `count` linear layers of one x (lin: count x (x w b y)) whose weights, biases and outputs lie one behind the other.
+bool linears_ok(const tensor_t* lin, int count) {
+    for (int i = 0; i < count; i++) {
+        const tensor_t* l = lin + 4 * i;
+        if (!linear_ok(l) || !same_tensor(l[0], lin[0])) return false;
+        // nothing that one of them writes is read or written by another
+        for (int j = 0; j < count; j++)
+            for (int k = 0; k < 3; k++)
+                if (!apart(l[3], lin[4 * j + k])) return false;
+        if (i > 0)
+            for (int k = 1; k < 4; k++)
+                if (!adjacent(lin[4 * i - 4 + k], l[k])) return false;
+    }
+    return true;
+}
+// Runs them with x as `x` says (the layers' own, or its image in the products' type).
+int linears(const Operand& x, const tensor_t* lin, int count, int compute) {
+    const int64_t n = (int64_t)(lin[0]->shape()[0] * lin[0]->shape()[1]), in = (int64_t)lin[0]->shape()[2];
+    const int64_t out = (int64_t)lin[1]->shape()[0];
+    const size_t need = compute == BR_GEMM_F32 ? 0 : br_hip_linear_group_workspace(count, n, out, in, x.dtype, code(lin[1]));
+    void* ws = need ? ComputingContext::gemm_staging(0, need) : nullptr;
+    return br_hip_linear_group(x.ptr, x.dtype, lin[1]->data(), code(lin[1]), static_cast<const float*>(lin[2]->data()),
+                               lin[3]->data(), code(lin[3]), count, n, out, in, compute, ws, need, stream());
+}
+// op_linear followed by op_add, one product where the sum is of its output and a residual.
+ComputingReturn linear_then_add(const Operand& x, const tensor_t* lin, const tensor_t* add) {
+    const tensor_t& y = lin[3];
+    bool fast = linear_ok(lin) && dev_f32(y) && dev_f32(add[0]) && dev_f32(add[1]) && dev_f32(add[2]);
+    if (fast) {
+        const bool first = same_tensor(add[0], y);
+        const tensor_t &r = first ? add[1] : add[0], &sum = add[2];
+        fast = first != same_tensor(add[1], y) && same_shape(add[0], add[1]) && r->items() == y->items() && sum->items() == y->items() &&
+               apart(y, r) && apart(y, sum) && (same_tensor(sum, r) || apart(sum, r)) && y->items() % 4 == 0;
+        for (int k = 0; fast && k < 3; k++) fast = apart(y, lin[k]) && apart(sum, lin[k]);
+        if (fast) {
+            const int compute = pick_compute({lin[0], lin[1], y});
+            const int64_t n = (int64_t)(lin[0]->shape()[0] * lin[0]->shape()[1]), in = (int64_t)lin[0]->shape()[2];
+            const int64_t out = (int64_t)lin[1]->shape()[0];
+            const size_t need = compute == BR_GEMM_F32 ? 0 : br_hip_gemm_staged_workspace(0, 1, n, out, in, x.dtype, code(lin[1]), 1);
+            void* ws = need ? ComputingContext::gemm_staging(0, need) : nullptr;
+            BR_OP(br_hip_linear_sum(x.ptr, x.dtype, lin[1]->data(), code(lin[1]), static_cast<const float*>(lin[2]->data()),
+                                    static_cast<const float*>(r->data()), static_cast<float*>(y->data()),
+                                    static_cast<float*>(sum->data()), n, out, in, compute, ws, need, stream()));
+            return OP_OK;
+        }
+    }
+    if (x.ptr != lin[0]->data()) {
+        // (x's image is what the product would have made of it)
+        const int64_t n = (int64_t)(lin[0]->shape()[0] * lin[0]->shape()[1]), in = (int64_t)lin[0]->shape()[2];
+        const int64_t out = (int64_t)lin[1]->shape()[0];
+        BR_OP(product(0, 1, n, out, in, 1.0f, x.ptr, x.dtype, in, 0, lin[1]->data(), code(lin[1]), in, 0, 0, y->data(), code(y), out,
+                      0, static_cast<const float*>(lin[2]->data()), 1, pick_compute({lin[0], lin[1], y})));
+    } else {
+        const ComputingReturn r = lin[0]->op_linear(lin[0], lin[1], lin[2], y);
+        if (r != OP_OK) return r;
+    }
+    return add[0]->op_add(add[0], add[1], add[2]);
+}
+}  // namespace
+
+ComputingReturn hip_linears(const tensor_t* lin, int count) {
+    if (linears_ok(lin, count)) {
+        BR_OP(linears(Operand{lin[0]->data(), code(lin[0])}, lin, count, pick_compute({lin[0], lin[1], lin[3]})));
+        return OP_OK;
+    }
+    for (int i = 0; i < count; i++) {
+        const tensor_t* l = lin + 4 * i;
+        const ComputingReturn r = l[0]->op_linear(l[0], l[1], l[2], l[3]);
+        if (r != OP_OK) return r;
+    }
+    return OP_OK;
+}
+
+// The LayerNorm kernel has every row of y in registers: with 16-bit products it writes y's image for the layers, too.
+ComputingReturn hip_layernorm_then_linears(const tensor_t* ln, float eps, const tensor_t* lin, int count) {
+    const tensor_t &x = ln[0], &mean = ln[1], &var = ln[2], &scale = ln[3], &bias = ln[4], &y = ln[5];
+    bool fast = linears_ok(lin, count) && same_tensor(lin[0], y) && x->shape().dim() == 3;
+    for (int i = 0; fast && i < 6; i++) fast = dev_f32(ln[i]);
+    const int compute = fast ? pick_compute({y, lin[1], lin[3]}) : BR_GEMM_F32;
+    if (fast && compute != BR_GEMM_F32) {
+        const int64_t rows = (int64_t)(x->shape()[0] * x->shape()[1]), cols = (int64_t)x->shape()[2];
+        if ((int64_t)mean->items() >= rows && (int64_t)var->items() >= rows && (int64_t)scale->items() == cols &&
+            (int64_t)bias->items() == cols && y->items() == x->items() && cols % 8 == 0) {
+            const int native = compute == BR_GEMM_F16 ? BR_F16 : BR_BF16;
+            void* y16 = ComputingContext::gemm_staging(1, y->items() * 2);
+            const int rc = br_hip_layernorm_fwd_copy16(
+                static_cast<const float*>(x->data()), static_cast<const float*>(scale->data()),
+                static_cast<const float*>(bias->data()), static_cast<float*>(y->data()), y16, native,
+                static_cast<float*>(mean->data()), static_cast<float*>(var->data()), rows, cols, eps, stream());
+            if (rc != BR_ERR_TODO) {
+                BR_OP(rc);
+                BR_OP(linears(Operand{y16, native}, lin, count, compute));
+                return OP_OK;
+            }
+        }
+    }
+    const ComputingReturn r = x->op_layernorm(x, mean, var, scale, bias, y, eps);
+    return r != OP_OK ? r : hip_linears(lin, count);
+}
+
+ComputingReturn hip_linear_then_add(const tensor_t* lin, const tensor_t* add) {
+    return linear_then_add(Operand{lin[0]->data(), code(lin[0])}, lin, add);
+}
+
+// op_gelu(u, v), op_linear(lin) and op_add(add): the GELU writes the image of an fp32 v that the product reads.
+ComputingReturn hip_gelu_linear_then_add(const tensor_t& u, const tensor_t& v, const tensor_t* lin, const tensor_t* add) {
+    if (dev_f32(u) && dev_f32(v) && u->items() == v->items() && linear_ok(lin) && same_tensor(lin[0], v)) {
+        const int compute = pick_compute({v, lin[1], lin[3]});
+        if (compute != BR_GEMM_F32 && lin[0]->shape()[2] % 8 == 0) {
+            const int native = compute == BR_GEMM_F16 ? BR_F16 : BR_BF16;
+            void* v16 = ComputingContext::gemm_staging(1, v->items() * 2);
+            const int rc = br_hip_gelu_fwd_copy16(static_cast<const float*>(u->data()), static_cast<float*>(v->data()), v16, native,
+                                                  (int64_t)v->items(), stream());
+            if (rc != BR_ERR_TODO) {
+                BR_OP(rc);
+                return linear_then_add(Operand{v16, native}, lin, add);
+            }
+        }
+    }
+    const ComputingReturn r = u->op_gelu(u, v);
+    return r != OP_OK ? r : hip_linear_then_add(lin, add);
+}
+
 // op_layernorm_backward(ln[0..7], eps) followed by op_add(add[0], add[1], add[2]) of its din and a residual, and, unless
 // lin is null, by op_linear_backward(lin[0..6]) of that sum.  One pass of the LayerNorm kernel leaves din, the sum, and for
 // the linear layer the sum's 16-bit image and its bias gradient; anything else runs as the operators.

@@ -98,6 +98,14 @@ ComputingReturn hip_layernorm_backward_add(const tensor_t& dy, const tensor_t& s
                                            const tensor_t& var, const tensor_t& y, const tensor_t& dscale,
                                            const tensor_t& dbias, const tensor_t& residual, const tensor_t& din,
                                            float eps);
+// `count` times op_linear (lin: count x (x w b y)); one batch where they read one x and the rest of each lies behind the
+// one before it.
+ComputingReturn hip_linears(const tensor_t* lin, int count);
+// op_layernorm (ln: x mean var scale bias y) followed by them.
+ComputingReturn hip_layernorm_then_linears(const tensor_t* ln, float eps, const tensor_t* lin, int count);
+// op_linear (lin: x w b y) followed by op_add (add: a b c), and the same behind op_gelu(u, v).
+ComputingReturn hip_linear_then_add(const tensor_t* lin, const tensor_t* add);
+ComputingReturn hip_gelu_linear_then_add(const tensor_t& u, const tensor_t& v, const tensor_t* lin, const tensor_t* add);
 // op_layernorm_backward (ln: dy scale bias var y dscale dbias din) followed by op_add (add: a b c) of din and a residual
 // and, unless lin is null, by op_linear_backward (lin: dy x w b x_g w_g b_g) of the sum.
 ComputingReturn hip_layernorm_backward_then_add(const tensor_t* ln, float eps, const tensor_t* add, const tensor_t* lin);

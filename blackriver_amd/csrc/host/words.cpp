@@ -121,6 +121,38 @@ BR_WORD(Layernorm,
 )
 // ( x y -- )
 BR_WORD(Transpos0213, Tensors<2> a(stack); a[0]->op_transpos_0213(a[0], a[1]);)
+// ( 3 x (x w b y) -- )  three linear layers in a row, query, key and value: one batch of products where they are alike
+BR_WORD(Linear3,
+    Tensors<12> l(stack);
+    op_check_word(hip_linears(l.t, 3), "op.linear op.linear op.linear");
+)
+// ( x mean var scale bias y eps   3 x (x w b y) -- )  the same behind the LayerNorm they read
+BR_WORD(LayernormLinear3,
+    Tensors<12> l(stack);
+    const float eps = (float)stack.pop_number();
+    Tensors<6> a(stack);
+    op_check_word(hip_layernorm_then_linears(a.t, eps, l.t, 3), "op.layernorm + three op.linear");
+)
+// ( x mean var scale bias y eps   x w b y -- )
+BR_WORD(LayernormLinear,
+    Tensors<4> l(stack);
+    const float eps = (float)stack.pop_number();
+    Tensors<6> a(stack);
+    op_check_word(hip_layernorm_then_linears(a.t, eps, l.t, 1), "op.layernorm + op.linear");
+)
+// ( x w b y   a b c -- )  a linear layer and the residual sum behind it
+BR_WORD(LinearThenAdd,
+    Tensors<3> c(stack);
+    Tensors<4> l(stack);
+    op_check_word(hip_linear_then_add(l.t, c.t), "op.linear + op.add");
+)
+// ( u v   v w b y   a b c -- )
+BR_WORD(GeluLinearThenAdd,
+    Tensors<3> c(stack);
+    Tensors<4> l(stack);
+    Tensors<2> a(stack);
+    op_check_word(hip_gelu_linear_then_add(a[0], a[1], l.t, c.t), "op.gelu + op.linear + op.add");
+)
 // ( x y  x y  x y -- )  three in a row, q, k and v: one launch where they are of one shape and do not meet
 BR_WORD(Transpos0213x3,
     Tensors<6> a(stack);
@@ -623,6 +655,11 @@ void load_nn_words(Enviroment& env) {
         {"op.qk_backward", QueryKeyBackward::creator},
         {"op.layernorm_backward_then_add_linear_backward", LayernormBackwardThenAddLinear::creator},
         {"op.qkv_backward_layernorm", QkvBackwardLayernorm::creator},
+        {"op.linear_x3", Linear3::creator},
+        {"op.layernorm_linear_x3", LayernormLinear3::creator},
+        {"op.layernorm_linear", LayernormLinear::creator},
+        {"op.linear_then_add", LinearThenAdd::creator},
+        {"op.gelu_linear_then_add", GeluLinearThenAdd::creator},
         {"op.transpos_0213_x3", Transpos0213x3::creator},
         {"op.gelu_linear_backward", GeluLinearBackward::creator},
         {"op.linear_add", LinearAdd::creator},
@@ -644,6 +681,11 @@ void load_nn_words(Enviroment& env) {
     env.insert_fusion({"op.add", "op.add", "op.softmax"}, "op.add_add_softmax");
     env.insert_fusion({"op.layernorm", "op.copy"}, "op.layernorm_copy");
     env.insert_fusion({"op.gelu_backward", "op.linear_backward"}, "op.gelu_linear_backward");
+    env.insert_fusion({"op.layernorm", "op.linear", "op.linear", "op.linear"}, "op.layernorm_linear_x3");
+    env.insert_fusion({"op.linear", "op.linear", "op.linear"}, "op.linear_x3");
+    env.insert_fusion({"op.gelu", "op.linear", "op.add"}, "op.gelu_linear_then_add");
+    env.insert_fusion({"op.layernorm", "op.linear"}, "op.layernorm_linear");
+    env.insert_fusion({"op.linear", "op.add"}, "op.linear_then_add");
     env.insert_fusion({"op.transpos_0213", "op.transpos_0213", "op.transpos_0213"}, "op.transpos_0213_x3");
     env.insert_fusion({"op.zero", "op.linear_backward", "op.add", "op.linear_backward", "op.add", "op.linear_backward", "op.add",
                        "op.layernorm_backward", "op.add"}, "op.qkv_backward_layernorm");

@@ -241,9 +241,11 @@ __global__ __launch_bounds__(kBlock) void gelu_fwd_f16(const half8* x, half8* y,
 }
 
 // fp32 in, 16-bit out: the output of the 4h activation when it only feeds the
-// next product (rounded once, exactly as that product would round an fp32 copy)
+// next product (rounded once, exactly as that product would round an fp32 copy);
+// y32: written as fp32 too ([1024 x 8192] 11 us, and 8.6 for the product's own
+// copy of it otherwise)
 template <typename D>
-__global__ __launch_bounds__(kBlock) void gelu_fwd_f32_to_16(const float4* x, uint4* y, int64_t n8) {
+__global__ __launch_bounds__(kBlock) void gelu_fwd_f32_to_16(const float4* x, uint4* y, int64_t n8, float4* y32 = nullptr) {
     const int64_t stride = (int64_t)gridDim.x * kBlock;
     for (int64_t i = (int64_t)blockIdx.x * kBlock + threadIdx.x; i < n8; i += stride) {
         const float4 a = x[2 * i], b = x[2 * i + 1];
@@ -256,6 +258,12 @@ __global__ __launch_bounds__(kBlock) void gelu_fwd_f32_to_16(const float4* x, ui
             asm volatile("" : "+v"(lo), "+v"(hi));
             w[j] = (unsigned)__builtin_bit_cast(unsigned short, from_f32<D>(lo)) |
                    ((unsigned)__builtin_bit_cast(unsigned short, from_f32<D>(hi)) << 16);
+            f[2 * j] = lo;
+            f[2 * j + 1] = hi;
+        }
+        if (y32) {
+            y32[2 * i] = make_float4(f[0], f[1], f[2], f[3]);
+            y32[2 * i + 1] = make_float4(f[4], f[5], f[6], f[7]);
         }
         y[i] = make_uint4(w[0], w[1], w[2], w[3]);
     }
@@ -1365,6 +1373,22 @@ int br_hip_gelu_fwd_f32_to_16(const float* x, void* y, int y_dtype, int64_t n, b
         gelu_fwd_f32_to_16<__half><<<grid, kBlock, 0, as_stream(stream)>>>((const float4*)x, (uint4*)y, n / 8);
     else
         gelu_fwd_f32_to_16<__hip_bfloat16><<<grid, kBlock, 0, as_stream(stream)>>>((const float4*)x, (uint4*)y, n / 8);
+    BR_HIP_LAUNCH_CHECK();
+    return BR_OK;
+}
+
+int br_hip_gelu_fwd_copy16(const float* x, float* y, void* y16, int y16_dtype, int64_t n, br_stream_t stream) {
+    if (n < 0) return BR_ERR_ATTR;
+    if (y16_dtype != BR_F16 && y16_dtype != BR_BF16) return BR_ERR_TODO;
+    if (n == 0) return BR_OK;
+    if (!x) return BR_ERR_INPUT;
+    if (!y || !y16) return BR_ERR_OUTPUT;
+    if (n % 8 != 0 || !aligned16(x) || !aligned16(y) || !aligned16(y16)) return BR_ERR_TODO;
+    const unsigned grid = (unsigned)grid_for(n / 8, kBlock);
+    if (y16_dtype == BR_F16)
+        gelu_fwd_f32_to_16<__half><<<grid, kBlock, 0, as_stream(stream)>>>((const float4*)x, (uint4*)y16, n / 8, (float4*)y);
+    else
+        gelu_fwd_f32_to_16<__hip_bfloat16><<<grid, kBlock, 0, as_stream(stream)>>>((const float4*)x, (uint4*)y16, n / 8, (float4*)y);
     BR_HIP_LAUNCH_CHECK();
     return BR_OK;
 }

@@ -192,7 +192,7 @@ __global__ __launch_bounds__(kThreads) void gemm_mfma32_kernel(GemmArgs g) {
     for (int j = 0; j < 2; j++) {
         const long long col = col0 + wn * 64 + j * 32 + lrow;
         if (col >= g.n) continue;
-        const float bias = g.bias ? g.bias[col] : 0.f;
+        const float bias = g.bias ? g.bias[batch * g.sbias + col] : 0.f;
 #pragma unroll
         for (int i = 0; i < 2; i++) {
 #pragma unroll
@@ -264,13 +264,21 @@ int run_plan(GemmArgs g, const gemm16::Problem& p, const gemm16::Plan& plan, lon
     return f16 ? gemm16_tiles_f16(g, p, kernel, batch, st) : gemm16_tiles_bf16(g, p, kernel, batch, st);
 }
 
+// What products have beyond br_hip_gemm's arguments.
+struct Extra {
+    long long bias_stride = 0;          // between batch entries
+    const float* addend = nullptr;      // with `sum`: sum = C + addend beside C (one batch entry, fp32)
+    float* sum = nullptr;
+    bool summed = false;                // out: the product's kernel has written `sum`
+};
+
 // br_hip_gemm with the tensor an accumulating product adds to named separately (null = c itself).  `planned`: what a
 // caller with a workspace has planned (null: plan here, nothing split); `padded`: see gemm16::Problem.
 int gemm_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alpha, const void* a, int a_dtype,
               int64_t lda, int64_t stride_a, const void* b, int b_dtype, int64_t ldb, int64_t stride_b, int accumulate,
               const void* addend, void* c, int c_dtype, int64_t ldc, int64_t stride_c, const float* bias, int64_t batch,
               int compute, br_stream_t stream, const gemm16::Plan* planned = nullptr, bool padded = false,
-              float* partials = nullptr, size_t partial_bytes = 0) {
+              float* partials = nullptr, size_t partial_bytes = 0, Extra* extra = nullptr) {
     if (m < 0 || n < 0 || k < 0 || batch < 0) return BR_ERR_ATTR;
     if (m == 0 || n == 0 || batch == 0) return BR_OK;
     if (!a || !b) return BR_ERR_INPUT;
@@ -295,8 +303,9 @@ int gemm_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float a
             const int rc = gemm_impl(trans_a, trans_b, m, n, k, alpha, entry(a, stride_a, a_dtype), a_dtype, lda, stride_a,
                                      entry(b, stride_b, b_dtype), b_dtype, ldb, stride_b, accumulate,
                                      addend ? entry(addend, stride_c, c_dtype) : nullptr,
-                                     const_cast<char*>(entry(c, stride_c, c_dtype)), c_dtype, ldc, stride_c, bias,
-                                     batch - i < fit ? batch - i : fit, compute, stream, planned, padded);
+                                     const_cast<char*>(entry(c, stride_c, c_dtype)), c_dtype, ldc, stride_c,
+                                     bias && extra ? bias + i * extra->bias_stride : bias,
+                                     batch - i < fit ? batch - i : fit, compute, stream, planned, padded, nullptr, 0, extra);
             if (rc != BR_OK) return rc;
         }
         return BR_OK;
@@ -310,6 +319,14 @@ int gemm_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float a
     g.alpha = alpha;
     g.accumulate = accumulate ? 1 : 0;
     g.addend = accumulate ? addend : nullptr;
+    if (extra) g.sbias = extra->bias_stride;
+    // taken by the small-tile kernels
+    auto sum_beside = [&]() {
+        if (!extra || !extra->sum || accumulate || batch != 1) return;
+        g.addend = extra->addend;
+        g.sum = extra->sum;
+        extra->summed = true;
+    };
     g.partials = partials;   // room for the partial tiles of a K split inside the kernel
     g.partial_bytes = partials ? partial_bytes : 0;
     g.tiles_m = (int)((m + BM - 1) / BM);
@@ -339,6 +356,7 @@ int gemm_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float a
         const int kernel = gemm16::fp32_kernel(m, n, k, batch);
         if (kernel != gemm16::kTile128 && 256 * lda < lim && 256 * ldb < lim && m < lim && n < lim && k < lim && k > 0) {
             const bool words = !g.vec_a || !g.vec_b || (k % 4 != 0 && !(ak && bk));
+            sum_beside();
             return gemm_fp32(g, p, kernel, words, batch, st);
         }
         if (ak && bk) gemm_mfma32_kernel<true, true><<<(unsigned)blocks, kThreads, 0, st>>>(g);
@@ -363,7 +381,9 @@ int gemm_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float a
                 g.k_slice = (int)per;
             }
         }
-        return run_plan(g, p, planned ? *planned : gemm16::gemm_plan(m, n, k, batch, false), batch, compute, st);
+        const gemm16::Plan plan = planned ? *planned : gemm16::gemm_plan(m, n, k, batch, false);
+        if (gemm16::is_flex(plan.kernel) && c_dtype == BR_F32) sum_beside();
+        return run_plan(g, p, plan, batch, compute, st);
     }
     // the register-staged kernel; its fast form loads 128 bits at a time and never checks k
     const long long va = p.a_f32 ? 4 : 8, vb = p.b_f32 ? 4 : 8;
@@ -583,7 +603,8 @@ struct Stager {
 __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float4* __restrict__ part, int splits,
                                                             long long mn4, long long n4, float alpha,
                                                             const float* __restrict__ bias, const void* old,
-                                                            void* c, int c_dtype, long long ldc) {
+                                                            void* c, int c_dtype, long long ldc, const float* addend,
+                                                            float* sum) {
     for (long long i = blockIdx.x * (long long)blockDim.x + threadIdx.x; i < mn4;
          i += (long long)gridDim.x * blockDim.x) {
         float4 s = part[i];
@@ -603,6 +624,10 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const float4* __rest
             const float* was = static_cast<const float*>(old) + row * ldc + col;
 #pragma unroll
             for (int j = 0; j < 4; j++) dst[j] = old ? o[j] + was[j] : o[j];
+            if (sum) {   // c plus the addend, beside c
+#pragma unroll
+                for (int j = 0; j < 4; j++) sum[row * ldc + col + j] = o[j] + addend[row * ldc + col + j];
+            }
         } else if (c_dtype == BR_F16) {
             __half* dst = static_cast<__half*>(c) + row * ldc + col;
             const __half* was = static_cast<const __half*>(old) + row * ldc + col;
@@ -650,7 +675,7 @@ int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
                 int64_t lda, int64_t stride_a, const void* b, int b_dtype, int64_t ldb, int64_t stride_b, int accumulate,
                 const void* addend, void* c, int c_dtype, int64_t ldc, int64_t stride_c, const float* bias,
                 int64_t batch, int compute, void* workspace, size_t workspace_bytes, br_stream_t stream,
-                bool zero_filled = false) {
+                bool zero_filled = false, Extra* extra = nullptr) {
     const int native = compute == BR_GEMM_F16 ? BR_F16 : BR_BF16;
     const bool sixteen = compute == BR_GEMM_F16 || compute == BR_GEMM_BF16;
     const int64_t a_rows = trans_a ? k : m, a_cols = trans_a ? m : k;
@@ -666,7 +691,8 @@ int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
                            workspace_bytes;
     if (!stage)
         return gemm_impl(trans_a, trans_b, m, n, k, alpha, a, a_dtype, lda, stride_a, b, b_dtype, ldb, stride_b,
-                         accumulate, addend, c, c_dtype, ldc, stride_c, bias, batch, compute, stream);
+                         accumulate, addend, c, c_dtype, ldc, stride_c, bias, batch, compute, stream, nullptr, false, nullptr, 0,
+                         extra);
     hipStream_t st = as_stream(stream);
     char* ws = static_cast<char*>(workspace);
     // 16-bit rows that start on 16-byte boundaries all the same (their pitch is padded) are taken where they are, unless
@@ -677,13 +703,14 @@ int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
     // every row of a staged copy is zero-filled up to its pitch
     Stager stager(compute, st);
     if (wants_staging(a_dtype, a_cols) && !zero_filled && !in_place(a, a_dtype, !trans_a, lda, stride_a)) {
-        const int rc = stager.add(a, a_dtype == BR_F32, lda, stride_a, a_rows, a_cols, batch, ws);
+        const int64_t copies = stride_a == 0 ? 1 : batch;   // one A for every batch entry
+        const int rc = stager.add(a, a_dtype == BR_F32, lda, stride_a, a_rows, a_cols, copies, ws);
         if (rc != BR_OK) return rc;
         a = ws;
         a_dtype = native;
         lda = staged_pitch(a_cols);
-        stride_a = a_rows * lda;
-        ws += staged_bytes(a_rows, a_cols, batch);
+        stride_a = stride_a == 0 ? 0 : a_rows * lda;
+        ws += staged_bytes(a_rows, a_cols, copies);
     }
     if (wants_staging(b_dtype, b_cols) && !zero_filled && !in_place(b, b_dtype, trans_b, ldb, stride_b)) {
         const int rc = stager.add(b, b_dtype == BR_F32, ldb, stride_b, b_rows, b_cols, batch, ws);
@@ -706,10 +733,13 @@ int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
                                  part, BR_F32, n, m * n, nullptr, plan.slices, compute, stream, &plan, true);
         if (rc != BR_OK) return rc;
         const long long mn4 = m * n / 4;
+        const bool summing = extra && extra->sum && !accumulate && c_dtype == BR_F32;
         splitk_reduce_kernel<<<grid_for(mn4, 256), 256, 0, st>>>(reinterpret_cast<const float4*>(part),
                                                                         plan.slices, mn4, n / 4, alpha, bias,
                                                                         accumulate ? (addend ? addend : c) : nullptr,
-                                                                        c, c_dtype, ldc);
+                                                                        c, c_dtype, ldc, summing ? extra->addend : nullptr,
+                                                                        summing ? extra->sum : nullptr);
+        if (summing) extra->summed = true;
         BR_HIP_LAUNCH_CHECK();
         return BR_OK;
     }
@@ -717,7 +747,7 @@ int staged_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float
     float* partials = plan.pair ? reinterpret_cast<float*>(ws) : nullptr;
     return gemm_impl(trans_a, trans_b, m, n, k, alpha, a, a_dtype, lda, stride_a, b, b_dtype, ldb, stride_b, accumulate,
                      addend, c, c_dtype, ldc, stride_c, bias, batch, compute, stream, plan.slices > 1 ? nullptr : &plan,
-                     true, partials, gemm16::pair_bytes(plan, m, n));
+                     true, partials, gemm16::pair_bytes(plan, m, n), extra);
 }
 }  // namespace
 
@@ -970,4 +1000,40 @@ extern "C" int br_hip_gemm_pair(const br_product* first, const br_product* secon
         if (rp != BR_OK) return rp;
     }
     return BR_OK;
+}
+
+// ---- linear layers of the operator stream ----------------------------------------
+extern "C" size_t br_hip_linear_group_workspace(int count, int64_t rows, int64_t out, int64_t in, int x_dtype, int w_dtype) {
+    if (count <= 0 || rows <= 0 || out <= 0 || in <= 0) return 0;
+    return br_hip_gemm_staged_workspace(0, 1, rows, out, in, x_dtype, w_dtype, count);
+}
+
+extern "C" int br_hip_linear_group(const void* x, int x_dtype, const void* w, int w_dtype, const float* bias, void* y, int y_dtype,
+                                   int count, int64_t rows, int64_t out, int64_t in, int compute, void* workspace,
+                                   size_t workspace_bytes, br_stream_t stream) {
+    if (count < 0 || rows < 0 || out <= 0 || in <= 0) return BR_ERR_ATTR;
+    if (rows == 0 || count == 0) return BR_OK;
+    if (!x || !w) return BR_ERR_INPUT;
+    if (!y) return BR_ERR_OUTPUT;
+    Extra extra;
+    extra.bias_stride = out;
+    return staged_impl(0, 1, rows, out, in, 1.0f, x, x_dtype, in, 0, w, w_dtype, in, out * in, 0, nullptr, y, y_dtype, out,
+                       rows * out, bias, count, compute, workspace, workspace_bytes, stream, false, &extra);
+}
+
+extern "C" int br_hip_linear_sum(const void* x, int x_dtype, const void* w, int w_dtype, const float* bias, const float* r,
+                                 float* y, float* sum, int64_t rows, int64_t out, int64_t in, int compute, void* workspace,
+                                 size_t workspace_bytes, br_stream_t stream) {
+    if (rows < 0 || out <= 0 || in <= 0) return BR_ERR_ATTR;
+    if (rows == 0) return BR_OK;
+    if (!x || !w || !r) return BR_ERR_INPUT;
+    if (!y || !sum || y == sum || y == r) return BR_ERR_OUTPUT;
+    Extra extra;
+    extra.addend = r;
+    extra.sum = sum;
+    const int rc = staged_impl(0, 1, rows, out, in, 1.0f, x, x_dtype, in, 0, w, w_dtype, in, 0, 0, nullptr, y, BR_F32, out, 0,
+                               bias, 1, compute, workspace, workspace_bytes, stream, false, &extra);
+    if (rc != BR_OK || extra.summed) return rc;
+    const int64_t shape[4] = {1, rows, 1, out};
+    return br_hip_add_bcast(y, r, sum, BR_F32, shape, shape, stream);
 }

@@ -504,6 +504,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64) void gemm_dtl_kern
     //   row = wm*WM + i*32 + (v/4)*8 + (lane/32)*4 + v%4,  col = wn*WN + j*32 + lane%32
     TC* c_base = static_cast<TC*>(g.c) + batch * g.sc;
     TC* c2_base = GELU ? static_cast<TC*>(g.c2) + batch * g.sc : nullptr;
+    const float* const bias_row = g.bias ? g.bias + operand_batch * g.sbias : nullptr;
     const TC* old_base = g.addend ? static_cast<const TC*>(g.addend) + batch * g.sc : c_base;  // read when accumulating
     if (row0 + BM <= g.m && col0 + BN <= g.n) {
         // Interior tile: straight-line code without guards, one 32x32 block of accumulators at a time.  A block's
@@ -527,7 +528,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64) void gemm_dtl_kern
         };
         float bias[FN];
 #pragma unroll
-        for (int j = 0; j < FN; j++) bias[j] = g.bias ? g.bias[col0 + wn * WN + j * 32 + (lane & 31)] : 0.f;
+        for (int j = 0; j < FN; j++) bias[j] = bias_row ? bias_row[col0 + wn * WN + j * 32 + (lane & 31)] : 0.f;
         auto interior = [&](auto adds) {
             constexpr bool ADDS = decltype(adds)::value;
             // alpha made opaque per form, or the compiler merges the scaling of all 128 elements of the two forms
@@ -583,7 +584,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64) void gemm_dtl_kern
 #pragma unroll
     for (int j = 0; j < FN; j++) {
         const long long col = col0 + wn * WN + j * 32 + (lane & 31);
-        bias[j] = g.bias && col < g.n ? g.bias[col] : 0.f;
+        bias[j] = bias_row && col < g.n ? bias_row[col] : 0.f;
         lane_at[j] = col < g.n ? (unsigned)(((lane >> 5) * 4 * g.ldc + j * 32 + (lane & 31)) * (long long)sizeof(TC)) : kPastEnd;
     }
     // a row offset added to kPastEnd stays past the end: the tile spans less than 2^31 bytes (kEdgeColumns)

@@ -161,6 +161,7 @@ __device__ __forceinline__ void flex_emit(const GemmArgs& g, const lds_byte* lds
     TC* c_base = static_cast<TC*>(g.c) + b * g.sc;
     TC* c2_base = GELU ? static_cast<TC*>(g.c2) + b * g.sc : nullptr;
     const TC* old_base = g.addend ? static_cast<const TC*>(g.addend) + b * g.sc : c_base;
+    const float* const bias = g.bias ? g.bias + b * g.sbias : nullptr;
     const lds_f32x4* const all = (const lds_f32x4*)lds_all;
     constexpr int kQuads = BM * QN, kThreads = THREADS;
 #pragma unroll
@@ -179,7 +180,7 @@ __device__ __forceinline__ void flex_emit(const GemmArgs& g, const lds_byte* lds
         float o[4];
 #pragma unroll
         for (int u = 0; u < 4; u++) {
-            o[u] = g.alpha * s[u] + (g.bias && u < left ? g.bias[col + u] : 0.f);
+            o[u] = g.alpha * s[u] + (bias && u < left ? bias[col + u] : 0.f);
             if (g.accumulate && u < left) o[u] += c_load<TC>(old_base + off + u);
             if (sizeof(TC) == 2) asm volatile("" : "+v"(o[u]));   // one fp32 value, then one rounding
         }
@@ -197,6 +198,19 @@ __device__ __forceinline__ void flex_emit(const GemmArgs& g, const lds_byte* lds
                     c_store<TC>(c_base + off + u, o[u]);
                     if (GELU) c_store<TC>(c2_base + off + u, gelu_one(o[u]));
                 }
+        }
+        if constexpr (!GELU && sizeof(TC) == 4) {
+            if (g.sum) {
+                float* const to = g.sum + b * g.sc + off;
+                if (left >= 4 && g.vec_c) {
+                    const float4 r = *reinterpret_cast<const float4*>(old_base + off);
+                    *reinterpret_cast<float4*>(to) = make_float4(o[0] + r.x, o[1] + r.y, o[2] + r.z, o[3] + r.w);
+                } else {
+#pragma unroll
+                    for (int u = 0; u < 4; u++)
+                        if (u < left) to[u] = o[u] + old_base[off + u];
+                }
+            }
         }
     }
 }
@@ -569,7 +583,7 @@ long long flex_tiles(GemmArgs& g, const Problem& p, long long batch) {
     const long long blocks = (long long)g.tiles_m * g.tiles_n * (g.splits > 1 ? g.splits : batch);
     const long long es = p.c_dtype == BR_F32 ? 4 : 2;
     auto quads = [&](const void* q) { return (reinterpret_cast<uintptr_t>(q) & (4 * es - 1)) == 0; };
-    g.vec_c = g.ldc % 4 == 0 && g.sc % 4 == 0 && quads(g.c) && (!g.c2 || quads(g.c2));
+    g.vec_c = g.ldc % 4 == 0 && g.sc % 4 == 0 && quads(g.c) && (!g.c2 || quads(g.c2)) && (!g.sum || (quads(g.sum) && quads(g.addend)));
     return blocks > 0x7fffffffLL ? -1 : blocks;
 }
 
@@ -609,7 +623,7 @@ int launch_flex_fp32(GemmArgs g, const Problem& p, long long batch, hipStream_t 
     const long long blocks = (long long)g.tiles_m * g.tiles_n * batch;
     if (blocks > 0x7fffffffLL) return BR_ERR_ATTR;
     const unsigned grid = (unsigned)blocks;
-    g.vec_c = g.ldc % 4 == 0 && g.sc % 4 == 0 && aligned16(g.c);
+    g.vec_c = g.ldc % 4 == 0 && g.sc % 4 == 0 && aligned16(g.c) && (!g.sum || (aligned16(g.sum) && aligned16(g.addend)));
     if (p.a_kstr && p.b_kstr)
         gemm_flex_kernel<BR_GEMM_F32, BM, BN, KW, 1, true, true, float, false, WORDS><<<grid, KW * 64, 0, st>>>(g);
     else if (p.a_kstr)

@@ -70,6 +70,10 @@ struct GemmArgs {
     // what an accumulating product adds to: a tensor laid out like c (same type, leading dimension and batch
     // stride), read where c is written; null = c itself
     const void* addend = nullptr;
+    long long sbias = 0;   // batch stride of bias
+    // second fp32 output of the small-tile kernels, laid out like c: what goes to c plus the addend (which then is no part
+    // of c; null = none)
+    float* sum = nullptr;
     // K split of the direct-to-LDS kernel: with splits == 2 two workgroups share an output tile, each summing one
     // half of K; the first to finish leaves its fp32 partial tile in `partials`, the second adds it to its own and
     // runs the epilogue (see gemm_dtl16.hpp).  splits == 1: no split, partials unused.
@@ -442,7 +446,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * 64) void gemm_kernel(GemmAr
     for (int j = 0; j < FN; j++) {
         const long long col = col0 + wn * WN + j * 32 + (lane & 31);
         if (col >= g.n) continue;
-        const float bias = g.bias ? g.bias[col] : 0.f;
+        const float bias = g.bias ? g.bias[batch * g.sbias + col] : 0.f;
 #pragma unroll
         for (int i = 0; i < FM; i++) {
 #pragma unroll

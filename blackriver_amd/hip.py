@@ -68,6 +68,10 @@ SIGNATURES = {
     "br_hip_bias_gelu_fwd": (_int, [_vp, _vp, _vp, _int, _i64, _i64, _vp]),
     "br_hip_bias_gelu_bwd_workspace": (_sz, [_i64, _i64]),
     "br_hip_linear_gelu": (_int, [_vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _vp]),
+    "br_hip_linear_group_workspace": (_sz, [_int, _i64, _i64, _i64, _int, _int]),
+    "br_hip_linear_group": (_int, [_vp, _int, _vp, _int, _vp, _vp, _int, _int, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
+    "br_hip_linear_sum": (_int, [_vp, _int, _vp, _int, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
+    "br_hip_gelu_fwd_copy16": (_int, [_vp, _vp, _vp, _int, _i64, _vp]),
     "br_hip_linear_residual": (_int, [_vp, _int, _vp, _int, _vp, _vp, _vp, _int, _i64, _i64, _i64, _int, _vp, _sz, _vp]),
     "br_hip_bias_gelu_bwd": (_int, [_vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _f32, _vp, _sz, _vp]),
     "br_hip_transpose_0213_group": (_int, [ctypes.POINTER(_vp), ctypes.POINTER(_vp), _int, _int, _i64, _i64, _i64, _i64, _vp]),

@@ -108,6 +108,7 @@ int br_hip_gelu_fwd(const void* x, void* y, int dtype, int64_t n, br_stream_t st
 /* The same forward with fp32 x and a 16-bit y (BR_F16 or BR_BF16; n % 8 == 0,
  * 16-byte aligned): for an activation that only feeds a 16-bit product, which
  * would round an fp32 y the same way. */
+int br_hip_gelu_fwd_copy16(const float* x, float* y, void* y16, int y16_dtype, int64_t n, br_stream_t stream);
 int br_hip_gelu_fwd_f32_to_16(const float* x, void* y, int y_dtype, int64_t n, br_stream_t stream);
 int br_hip_gelu_bwd(const void* dy, const void* x, void* dx, int dtype, int64_t n,
                     br_stream_t stream);
@@ -450,6 +451,23 @@ int br_hip_gemm_kernel(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k
  * caller then runs the two operators. */
 int br_hip_linear_gelu(const void* x, const void* w, const float* bias, void* u, void* y, int dtype,
                        int64_t rows, int64_t out, int64_t in, br_stream_t stream);
+
+/* `count` op_linear of one x (cuda_tensor.cpp:146-193; the query, key and value
+ * layers of bloomz-7b/train.words:139-145) whose weights [out, in], biases [out]
+ * and outputs [rows, out] lie one behind the other: one batch of products, x
+ * converted once.  workspace: br_hip_linear_group_workspace() bytes. */
+size_t br_hip_linear_group_workspace(int count, int64_t rows, int64_t out, int64_t in, int x_dtype, int w_dtype);
+int br_hip_linear_group(const void* x, int x_dtype, const void* w, int w_dtype, const float* bias, void* y, int y_dtype,
+                        int count, int64_t rows, int64_t out, int64_t in, int compute, void* workspace,
+                        size_t workspace_bytes, br_stream_t stream);
+
+/* op_linear followed by op_add into a tensor of its own: y = x . w^T + bias and
+ * sum = y + r, dense fp32 (r may be sum).  The sum is written by the product
+ * where its kernel can, else in a pass of its own; bits as the two operators'.
+ * workspace as for br_hip_linear_residual. */
+int br_hip_linear_sum(const void* x, int x_dtype, const void* w, int w_dtype, const float* bias, const float* r,
+                      float* y, float* sum, int64_t rows, int64_t out, int64_t in, int compute, void* workspace,
+                      size_t workspace_bytes, br_stream_t stream);
 
 /* op_linear followed by op_add of a residual (cuda_tensor.cpp:146-193 and
  * :206-232; the pair of bloomz-7b/train.words:172-173 and :191-192) in one

@@ -118,6 +118,18 @@ def test_add_f16_same_shape():
     assert np.array_equal(host(c), (a.astype(np.float32) + b.astype(np.float32)).astype(np.float16))
 
 
+@pytest.mark.parametrize("n,dtype,d16", [(8, F16, torch.float16), (1000 * 264, BF16, torch.bfloat16)])
+def test_gelu_with_its_16_bit_copy(n, dtype, d16):
+    """Bit for bit br_hip_gelu_fwd's result and that result rounded once; in place too."""
+    x = dev(np.random.default_rng(4).standard_normal(n).astype(np.float32) * 3)
+    want, y, y16 = empty(n), empty(n), torch.zeros(n, dtype=d16, device="cuda")
+    call("br_hip_gelu_fwd", ptr(x), ptr(want), F32, n, stream())
+    call("br_hip_gelu_fwd_copy16", ptr(x), ptr(y), ptr(y16), dtype, n, stream())
+    call("br_hip_gelu_fwd_copy16", ptr(x), ptr(x), ptr(y16), dtype, n, stream())
+    torch.cuda.synchronize()
+    assert torch.equal(y, want) and torch.equal(x, want) and torch.equal(y16, want.to(d16))
+
+
 # ----------------------------------------------------- transpose / colsum
 @pytest.mark.parametrize("shape,eb", [((4, 512, 32, 128), 4), ((2, 7, 3, 5), 4), ((2, 16, 4, 8), 2), ((1, 3, 5, 3), 2)])
 def test_transpose_0213_bit_exact(shape, eb):

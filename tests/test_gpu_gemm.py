@@ -755,3 +755,48 @@ def test_two_products_keep_their_order_where_one_overwrites_the_others_operand(s
     want = pair_reference(1, 0, dy, x).float()
     assert run_pair([(1, 0, dy, x, dw), (0, 0, dy, w, x)], hip.GEMM_F16)   # one launch by its sizes
     assert torch.equal(dw, want) and torch.equal(x, pair_reference(0, 0, dy, w).to(x.dtype))
+
+
+@pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16, hip.GEMM_F32])
+@pytest.mark.parametrize("rows,out,inn,x_dt,y_dt", [
+    (24, 256, 256, F32, F32), (65, 40, 72, None, None), (130, 1000, 136, None, F32), (1000, 1024, 64, F32, F32), (1000, 2048, 256, None, F32),
+    (2100, 1280, 128, F32, None), (33, 30, 20, F32, F32)])
+def test_linear_group_is_exact_on_integers(rows, out, inn, x_dt, y_dt, compute):
+    """Three layers of one x as a batch, each with a bias of its own; the kernels of small and of large tiles, sizes that
+    are no multiple of a granule among them."""
+    dt = COMPUTE_T[compute]
+    print("case rows=%d out=%d in=%d compute=%d" % (rows, out, inn, compute), flush=True)
+    torch.manual_seed(rows)
+    x, w = whole_numbers((rows, inn), 1, x_dt or dt), whole_numbers((3, out, inn), 1, dt)
+    bias = whole_numbers((3, out), 5, F32)
+    y = torch.full((3, rows, out), float("nan"), device="cuda", dtype=TORCH_T[y_dt or dt])
+    need = hip.load().br_hip_linear_group_workspace(3, rows, out, inn, x_dt or dt, dt)
+    ws = torch.full((max(need, 16),), 0x7f, dtype=torch.uint8, device="cuda")
+    call("br_hip_linear_group", ptr(x), x_dt or dt, ptr(w), dt, ptr(bias), ptr(y), y_dt or dt, 3, rows, out, inn, compute, ptr(ws),
+         need, stream())
+    torch.cuda.synchronize()
+    for i in range(3):
+        assert torch.equal(y[i], (x.double() @ w[i].double().t() + bias[i].double()).to(y.dtype))
+
+
+@pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_F32])
+@pytest.mark.parametrize("rows,out,inn", [(24, 256, 256), (65, 44, 72), (78, 1024, 4096), (1000, 1024, 1024), (1000, 2048, 2048), (2048, 4096, 64), (33, 30, 20)])
+@pytest.mark.parametrize("over", [False, True])
+def test_linear_with_the_sum_beside_it_is_exact_on_integers(rows, out, inn, over, compute):
+    """y and y + r, the sum over r or apart: small tiles, a ring of K steps, slices of K, and large tiles followed by an
+    addition."""
+    dt = COMPUTE_T[compute]
+    print("case rows=%d out=%d in=%d compute=%d" % (rows, out, inn, compute), flush=True)
+    torch.manual_seed(rows)
+    x, w = whole_numbers((rows, inn), 1, dt), whole_numbers((out, inn), 1, dt)
+    bias, r = whole_numbers((out,), 5, F32), whole_numbers((rows, out), 9, F32)
+    want = x.double() @ w.double().t() + bias.double()
+    want_sum = want + r.double()
+    y = torch.full((rows, out), float("nan"), device="cuda")
+    total = r if over else torch.full_like(y, float("nan"))
+    need = hip.load().br_hip_gemm_staged_workspace(0, 1, rows, out, inn, dt, dt, 1) if compute != hip.GEMM_F32 else 0
+    ws = torch.full((max(need, 16),), 0x7f, dtype=torch.uint8, device="cuda")
+    call("br_hip_linear_sum", ptr(x), dt, ptr(w), dt, ptr(bias), ptr(r), ptr(y), ptr(total), rows, out, inn, compute, ptr(ws), need,
+         stream())
+    torch.cuda.synchronize()
+    assert torch.equal(y, want.float()) and torch.equal(total, want_sum.float())
