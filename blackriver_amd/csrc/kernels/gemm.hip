@@ -256,7 +256,8 @@ int run_plan(GemmArgs g, const gemm16::Problem& p, const gemm16::Plan& plan, lon
         if (rc != BR_OK) return rc;
         return f16 ? gemm16_tiles_f16(tail, p, kTile256x128Groups, 1, st) : gemm16_tiles_bf16(tail, p, kTile256x128Groups, 1, st);
     }
-    const int kernel = plan.kernel;
+    // a bias of its own for every batch entry: not on two groups of waves (see gemm_dtl16.hpp)
+    const int kernel = plan.kernel == kTile256x128Groups && g.sbias != 0 && batch > 1 ? kTile256x128 : plan.kernel;
     // the loads have to be checked against the end of K: K, or a slice of it, is no whole number of steps
     const bool ragged = (g.k % 64 != 0 && kernel != kTile128Half) || g.splits > 1;
     if (ragged || is_flex(kernel))

@@ -504,7 +504,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64) void gemm_dtl_kern
     //   row = wm*WM + i*32 + (v/4)*8 + (lane/32)*4 + v%4,  col = wn*WN + j*32 + lane%32
     TC* c_base = static_cast<TC*>(g.c) + batch * g.sc;
     TC* c2_base = GELU ? static_cast<TC*>(g.c2) + batch * g.sc : nullptr;
-    const float* const bias_row = g.bias ? g.bias + operand_batch * g.sbias : nullptr;
+    // (two groups of waves: the batch index is eight registers too many; run_plan keeps such batches from them)
+    const float* const bias_row = g.bias && KW == 1 ? g.bias + batch * g.sbias : g.bias;
     const TC* old_base = g.addend ? static_cast<const TC*>(g.addend) + batch * g.sc : c_base;  // read when accumulating
     if (row0 + BM <= g.m && col0 + BN <= g.n) {
         // Interior tile: straight-line code without guards, one 32x32 block of accumulators at a time.  A block's
