@@ -80,10 +80,12 @@ int product(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float alp
 
 // Column sums and the two products of a backward operator, in this order or, where they are small, as one launch.
 // Operands that have to be converted are, in one launch, and once where both products read them.
-int two_products(const br_product& first, const br_product& second, const br_column_sums* sums, int compute) {
+int two_products(const br_product& first, const br_product& second, const br_column_sums* sums, int compute,
+                 const br_partial_sums* later = nullptr) {
     const size_t need = br_hip_gemm_pair_workspace(&first, &second, compute);
     void* ws = need ? ComputingContext::gemm_staging(0, need) : nullptr;
-    return br_hip_gemm_pair(&first, &second, sums, compute, ws, need, ComputingContext::stream);
+    return br_hip_gemm_pair(&first, &second, sums, later && later->partials ? later : nullptr, compute, ws, need,
+                            ComputingContext::stream);
 }
 
 // An operand that several products of one operator read: with a 16-bit MFMA
@@ -110,11 +112,11 @@ Operand shared_operand(const void* p, int dtype, int64_t items, int compute) {
 // (weight and weight_g may be the first rows of the `out` rows meant)
 int linear_backward_products(const Operand& dy, const tensor_t& x, const tensor_t& weight, const tensor_t& x_g,
                              const tensor_t& weight_g, int64_t n, int64_t in, int64_t out, int compute,
-                             const br_column_sums* sums = nullptr) {
+                             const br_column_sums* sums = nullptr, const br_partial_sums* later = nullptr) {
     return two_products(
         {1, 0, out, in, n, unlift(), dy.ptr, dy.dtype, out, 0, x->data(), code(x), in, 0, weight_g->data(), code(weight_g), in, 0, 1},
         {0, 0, n, in, out, 1.0f, dy.ptr, dy.dtype, out, 0, weight->data(), code(weight), in, 0, x_g->data(), code(x_g), in, 0, 1},
-        sums, compute);
+        sums, compute, later);
 }
 
 // fp32 device pointer to a bias vector, converting 16-bit storage on the fly
@@ -1108,13 +1110,15 @@ ComputingReturn hip_layernorm_backward_then_add(const tensor_t* ln, float eps, c
             }
             const size_t need = br_hip_layernorm_bwd_sums_workspace(rows, cols);
             void* ws = need <= head_bytes() ? ComputingContext::workspace : ComputingContext::scratch(need);
+            br_partial_sums later = {};
             auto run = [&]() {
                 return br_hip_layernorm_bwd_add(
                     static_cast<const float*>(dy->data()), static_cast<const float*>(y->data()),
                     static_cast<const float*>(scale->data()), static_cast<const float*>(bias->data()),
                     static_cast<const float*>(var->data()), static_cast<const float*>(residual->data()),
                     static_cast<float*>(dscale->data()), static_cast<float*>(dbias->data()), static_cast<float*>(din->data()),
-                    static_cast<float*>(sum->data()), sum16, native, sums, rows, cols, eps, unlift(), ws, need, stream());
+                    static_cast<float*>(sum->data()), sum16, native, sums, rows, cols, eps, unlift(), linear ? &later : nullptr, ws,
+                    need, stream());
             };
             int rc = run();
             if (rc == BR_ERR_TODO && linear) {
@@ -1126,7 +1130,8 @@ ComputingReturn hip_layernorm_backward_then_add(const tensor_t* ln, float eps, c
             fast = rc != BR_ERR_TODO;
             if (fast) BR_OP(rc);
             if (fast && linear)
-                BR_OP(linear_backward_products(Operand{sum16, native}, lin[1], lin[2], lin[4], lin[5], rows, in, cols, compute));
+                BR_OP(linear_backward_products(Operand{sum16, native}, lin[1], lin[2], lin[4], lin[5], rows, in, cols, compute, nullptr,
+                                               &later));
         }
     }
     if (!fast) {
@@ -1213,16 +1218,19 @@ ComputingReturn hip_layernorm_backward_add_linear_backward(
             const size_t need = br_hip_layernorm_bwd_sums_workspace(rows, cols);
             void* ws = need <= head_bytes() ? ComputingContext::workspace : ComputingContext::scratch(need);
             void* d16 = ComputingContext::gemm_staging(1, (size_t)(rows * cols) * 2);
-            const int rc = br_hip_layernorm_bwd_residual_sums(
+            // dgamma, dbeta and the bias gradient are added up beside the products
+            br_partial_sums later = {};
+            const int rc = br_hip_layernorm_bwd_add(
                 static_cast<const float*>(dy->data()), static_cast<const float*>(y->data()),
                 static_cast<const float*>(scale->data()), static_cast<const float*>(bias->data()),
                 static_cast<const float*>(var->data()), static_cast<const float*>(residual->data()),
-                static_cast<float*>(dscale->data()), static_cast<float*>(dbias->data()),
+                static_cast<float*>(dscale->data()), static_cast<float*>(dbias->data()), nullptr,
                 static_cast<float*>(din->data()), d16, native, static_cast<float*>(bias_g->data()), rows, cols, eps,
-                unlift(), ws, need, stream());
+                unlift(), &later, ws, need, stream());
             if (rc != BR_ERR_TODO) {
                 BR_OP(rc);
-                BR_OP(linear_backward_products(Operand{d16, native}, x, weight, x_g, weight_g, rows, in, cols, compute));
+                BR_OP(linear_backward_products(Operand{d16, native}, x, weight, x_g, weight_g, rows, in, cols, compute, nullptr,
+                                               &later));
                 return OP_OK;
             }
         }

@@ -36,7 +36,8 @@ BR_GEMM16_ENTRIES(bf16)
 int gemm_fp32(const gemm16::GemmArgs& g, const gemm16::Problem& p, int kernel, bool words, long long batch, hipStream_t st);
 #define BR_GEMM_PAIR_ENTRY(T)                                                                                            \
     int gemm_pair_##T(const gemm16::GemmArgs& w, const gemm16::Problem& pw, long long batch_w, const gemm16::GemmArgs& x,    \
-                      const gemm16::Problem& px, long long batch_x, int kernel, const gemm16::ColumnSums& sums, hipStream_t st);
+                      const gemm16::Problem& px, long long batch_x, int kernel, const gemm16::ColumnSums& sums,                   \
+                      const gemm16::PartialSums& later, hipStream_t st);
 BR_GEMM_PAIR_ENTRY(f16)
 BR_GEMM_PAIR_ENTRY(bf16)
 BR_GEMM_PAIR_ENTRY(f32)
@@ -849,8 +850,8 @@ struct PairOperands {
 };
 
 // Both products (and the column sums) as one launch; BR_ERR_TODO where they have to run one after the other.
-int pair_impl(const br_product& first, const br_product& second, const PairOperands& ops, const br_column_sums* sums, int compute,
-              hipStream_t st) {
+int pair_impl(const br_product& first, const br_product& second, const PairOperands& ops, const br_column_sums* sums,
+              const br_partial_sums* later, int compute, hipStream_t st) {
     using namespace gemm16;
     const bool fp32 = compute == BR_GEMM_F32;
     const int native = compute == BR_GEMM_F16 ? BR_F16 : fp32 ? BR_F32 : BR_BF16;
@@ -882,6 +883,28 @@ int pair_impl(const br_product& first, const br_product& second, const PairOpera
         cs.rows = (int)sums->rows;
         cs.cols = (int)sums->cols;
         cs.scale = sums->scale;
+    }
+    PartialSums ps;
+    if (later && later->partials) {
+        if (later->arrays < 1 || later->arrays > 3 || later->parts <= 0 || later->parts > 0x3fffffffLL || later->cols <= 0 ||
+            later->cols % 4 != 0 || later->cols > 0x3fffffffLL || !aligned16(later->partials))
+            return BR_ERR_TODO;
+        const Stored sp{later->partials, BR_F32, later->arrays * later->parts, later->cols, later->cols, 0, 1, false};
+        for (int i = 0; i < later->arrays; i++) {
+            if (!later->out[i] || !aligned16(later->out[i])) return BR_ERR_TODO;
+            const Stored so{later->out[i], BR_F32, 1, later->cols, later->cols, 0, 1, false};
+            if (sums && overlap(so, Stored{sums->out, BR_F32, 1, sums->cols, sums->cols, 0, 1, false})) return BR_ERR_TODO;
+            for (const Stored& s : ops.now)
+                if (overlap(so, s)) return BR_ERR_TODO;
+            for (const Stored& s : out)
+                if (overlap(so, s) || overlap(sp, s)) return BR_ERR_TODO;
+            ps.out[i] = reinterpret_cast<flex_f32x4*>(later->out[i]);
+        }
+        ps.partials = reinterpret_cast<const flex_f32x4*>(later->partials);
+        ps.arrays = later->arrays;
+        ps.parts = (int)later->parts;
+        ps.cols4 = (int)(later->cols / 4);
+        ps.scale = later->scale;
     }
     GemmArgs g[2];
     Problem p[2];
@@ -921,7 +944,7 @@ int pair_impl(const br_product& first, const br_product& second, const PairOpera
     const int rc = ops.run(compute, st);
     if (rc != BR_OK) return rc;
     auto* const launch = fp32 ? gemm_pair_f32 : compute == BR_GEMM_F16 ? gemm_pair_f16 : gemm_pair_bf16;
-    return launch(g[w], p[w], products[w]->batch, g[x], p[x], products[x]->batch, kernel, cs, st);
+    return launch(g[w], p[w], products[w]->batch, g[x], p[x], products[x]->batch, kernel, cs, ps, st);
 }
 
 }  // namespace
@@ -946,13 +969,15 @@ extern "C" int br_hip_gemm_pair_kernel(int64_t m1, int64_t n1, int64_t k1, int64
     return gemm16::pair_kernel({m1, n1, k1, batch1}, {m2, n2, k2, batch2}, compute == BR_GEMM_F32);
 }
 
-extern "C" int br_hip_gemm_pair(const br_product* first, const br_product* second, const br_column_sums* sums, int compute,
-                                void* workspace, size_t workspace_bytes, br_stream_t stream) {
+extern "C" int br_hip_gemm_pair(const br_product* first, const br_product* second, const br_column_sums* sums,
+                                const br_partial_sums* later, int compute, void* workspace, size_t workspace_bytes,
+                                br_stream_t stream) {
     if (!first || !second) return BR_ERR_INPUT;
     if (compute != BR_GEMM_F16 && compute != BR_GEMM_BF16 && compute != BR_GEMM_F32) return BR_ERR_ATTR;
     hipStream_t st = as_stream(stream);
     auto before_them = [&]() {
-        if (!sums) return (int)BR_OK;
+        const int rl = later ? br_hip_finish_sums(later, stream) : (int)BR_OK;
+        if (!sums || rl != BR_OK) return rl;
         return br_hip_colsum(sums->x, sums->dtype, sums->out, sums->rows, sums->cols, sums->scale, sums->workspace,
                              sums->workspace_bytes, stream);
     };
@@ -968,7 +993,7 @@ extern "C" int br_hip_gemm_pair(const br_product* first, const br_product* secon
         // copies are made ahead of both products: the first must not write what the second's are made of
         const bool apart = !overlap(stored_c(*first), ops.before[2]) && !overlap(stored_c(*first), ops.before[3]);
         if (room && apart) {
-            const int rc = pair_impl(*first, *second, ops, sums, compute, st);
+            const int rc = pair_impl(*first, *second, ops, sums, later, compute, st);
             if (rc != BR_ERR_TODO) return rc;
             if (ops.bytes > 0 && workspace_bytes >= ops.bytes) {
                 // one after the other, on copies made in one launch

@@ -76,57 +76,101 @@ __device__ __forceinline__ void sum_strip(const ColumnSums& s, int strip, float*
         s.out[at] = (lds[threadIdx.x] + lds[kWidth + threadIdx.x] + lds[2 * kWidth + threadIdx.x] + lds[3 * kWidth + threadIdx.x]) * s.scale;
 }
 
-// Workgroups [0, n1) run `a`, [n1, n1 + n2) run `b`, those after them the column sums.  AK1 .. BK2: which operands are
-// row-contiguous.
+// What a LayerNorm backward has left to add up: `arrays` of `parts` partial rows of cols4 quads, one behind the other.
+// In a launch of their own these sums take 4 us, nearly all of it the launch; beside the products next to nothing: the
+// forward and backward pass of a block 82.7 -> 79.3 us on [64 x 256] and 135.1 -> 132.8 on [78 x 1024]; no difference on
+// [1000 x 1024], where the products fill the chip (366.8 and 366.5).
+struct PartialSums {
+    const flex_f32x4* partials = nullptr;   // null: none
+    flex_f32x4* out[3] = {nullptr, nullptr, nullptr};
+    int arrays = 0, parts = 0, cols4 = 0;
+    float scale = 1.0f;
+    int groups() const { return partials ? arrays * ((cols4 + 15) / 16) : 0; }
+};
+// 16 quads of columns of one array, in the order of ln_bwd_finalize_x4 (layernorm.hip): 64 slices of the parts, folded
+// 8 at a time.
+__device__ __forceinline__ void add_partials(const PartialSums& s, int group, flex_f32x4* lds) {
+    constexpr int kSlices = 64;
+    const int per = (s.cols4 + 15) / 16, array = group / per, q = threadIdx.x & 15, g = threadIdx.x >> 4;
+    const int c4 = (group - array * per) * 16 + q;
+    const flex_f32x4* part = s.partials + (long long)array * s.parts * s.cols4;
+    flex_f32x4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        v[k] = 0.f;
+        if (c4 < s.cols4)
+            for (int p = g + 16 * k; p < s.parts; p += kSlices) v[k] += part[(long long)p * s.cols4 + c4];
+        lds[(g + 16 * k) * 16 + q] = v[k];
+    }
+    __syncthreads();
+    if (g < 8) {
+        for (int k = g + 8; k < kSlices; k += 8) v[0] += lds[k * 16 + q];
+    }
+    __syncthreads();
+    if (g < 8) lds[g * 16 + q] = v[0];
+    __syncthreads();
+    if (g == 0 && c4 < s.cols4) {
+        for (int k = 1; k < 8; k++) v[0] += lds[k * 16 + q];
+        flex_f32x4* const out = array == 0 ? s.out[0] : array == 1 ? s.out[1] : s.out[2];
+        out[c4] = v[0] * s.scale;
+    }
+}
+
+// Workgroups [0, n1) run `a`, [n1, n1 + n2) run `b`, those after them the column sums and the partial sums.  AK1 .. BK2:
+// which operands are row-contiguous.
 template <int CT, int BM, int BN, int KW, int ST, bool AK1, bool BK1, typename TC1, bool AK2, bool BK2, typename TC2>
-__global__ __launch_bounds__(KW * 64, CT == BR_GEMM_F32 ? 2 : 1) void gemm_flex_pair_kernel(GemmArgs a, GemmArgs b, unsigned n1, unsigned n2, ColumnSums sums) {
+__global__ __launch_bounds__(KW * 64, CT == BR_GEMM_F32 ? 2 : 1) void gemm_flex_pair_kernel(GemmArgs a, GemmArgs b, unsigned n1, unsigned n2, unsigned n3, ColumnSums sums,
+                                                                                       PartialSums later) {
     static_assert(KW == 4, "the column sums are four waves'");
+    static_assert(flex_lds_bytes<BM, BN, KW, ST>() >= 64 * 16 * sizeof(flex_f32x4), "add_partials' slices");
     __shared__ __attribute__((aligned(1024))) unsigned char lds[flex_lds_bytes<BM, BN, KW, ST>()];
     const unsigned id = blockIdx.x;
     if (id < n1) flex_product<CT, BM, BN, KW, ST, AK1, BK1, TC1, false, false, false>(a, id, n1, lds);
     else if (id < n1 + n2) flex_product<CT, BM, BN, KW, ST, AK2, BK2, TC2, false, false, false>(b, id - n1, n2, lds);
-    else sum_strip<CT>(sums, (int)(id - n1 - n2), reinterpret_cast<float*>(lds));
+    else if (id < n1 + n2 + n3) sum_strip<CT>(sums, (int)(id - n1 - n2), reinterpret_cast<float*>(lds));
+    else add_partials(later, (int)(id - n1 - n2 - n3), reinterpret_cast<flex_f32x4*>(lds));
 }
 
 // `w`: C of fp32, both operands row-contiguous.  `x`: A k-contiguous.  The one whose workgroups walk further along K
 // starts first.
 template <int CT, int BM, int BN, int KW, int ST, bool BK2, typename TC2>
-int launch_pair_layout(const GemmArgs& w, const GemmArgs& x, unsigned nw, unsigned nx, const ColumnSums& sums, hipStream_t st) {
+int launch_pair_layout(const GemmArgs& w, const GemmArgs& x, unsigned nw, unsigned nx, const ColumnSums& sums,
+                       const PartialSums& later, hipStream_t st) {
     const unsigned strip = kSumLanes * (CT == BR_GEMM_F32 ? 4 : 8);
     const unsigned extra = sums.x ? ((unsigned)sums.cols + strip - 1) / strip : 0;
-    if ((long long)nw + nx + extra > 0x7fffffffLL / (KW * 64)) return BR_ERR_TODO;
-    const unsigned grid = nw + nx + extra;
+    if ((long long)nw + nx + extra + later.groups() > 0x7fffffffLL / (KW * 64)) return BR_ERR_TODO;
+    const unsigned grid = nw + nx + extra + (unsigned)later.groups();
     if (x.k >= w.k)
-        gemm_flex_pair_kernel<CT, BM, BN, KW, ST, false, BK2, TC2, true, true, float><<<grid, KW * 64, 0, st>>>(x, w, nx, nw, sums);
+        gemm_flex_pair_kernel<CT, BM, BN, KW, ST, false, BK2, TC2, true, true, float><<<grid, KW * 64, 0, st>>>(x, w, nx, nw, extra, sums, later);
     else
-        gemm_flex_pair_kernel<CT, BM, BN, KW, ST, true, true, float, false, BK2, TC2><<<grid, KW * 64, 0, st>>>(w, x, nw, nx, sums);
+        gemm_flex_pair_kernel<CT, BM, BN, KW, ST, true, true, float, false, BK2, TC2><<<grid, KW * 64, 0, st>>>(w, x, nw, nx, extra, sums, later);
     BR_HIP_LAUNCH_CHECK();
     return BR_OK;
 }
 
 template <int CT, int BM, int BN, int KW, int ST>
 int launch_pair_config(GemmArgs w, const Problem& pw, long long batch_w, GemmArgs x, const Problem& px, long long batch_x,
-                       const ColumnSums& sums, hipStream_t st) {
+                       const ColumnSums& sums, const PartialSums& later, hipStream_t st) {
     const long long nw = flex_tiles<BM, BN>(w, pw, batch_w), nx = flex_tiles<BM, BN>(x, px, batch_x);
     if (nw < 0 || nx < 0) return BR_ERR_TODO;
     if constexpr (CT != BR_GEMM_F32) {
         using T = std::conditional_t<CT == BR_GEMM_F16, __half, __hip_bfloat16>;
         if (px.c_dtype != BR_F32) {
-            if (px.b_kstr) return launch_pair_layout<CT, BM, BN, KW, ST, true, T>(w, x, (unsigned)nw, (unsigned)nx, sums, st);
-            return launch_pair_layout<CT, BM, BN, KW, ST, false, T>(w, x, (unsigned)nw, (unsigned)nx, sums, st);
+            if (px.b_kstr) return launch_pair_layout<CT, BM, BN, KW, ST, true, T>(w, x, (unsigned)nw, (unsigned)nx, sums, later, st);
+            return launch_pair_layout<CT, BM, BN, KW, ST, false, T>(w, x, (unsigned)nw, (unsigned)nx, sums, later, st);
         }
     }
-    if (px.b_kstr) return launch_pair_layout<CT, BM, BN, KW, ST, true, float>(w, x, (unsigned)nw, (unsigned)nx, sums, st);
-    return launch_pair_layout<CT, BM, BN, KW, ST, false, float>(w, x, (unsigned)nw, (unsigned)nx, sums, st);
+    if (px.b_kstr) return launch_pair_layout<CT, BM, BN, KW, ST, true, float>(w, x, (unsigned)nw, (unsigned)nx, sums, later, st);
+    return launch_pair_layout<CT, BM, BN, KW, ST, false, float>(w, x, (unsigned)nw, (unsigned)nx, sums, later, st);
 }
 
 template <int CT>
 int launch_pair(const GemmArgs& w, const Problem& pw, long long batch_w, const GemmArgs& x, const Problem& px,
-                long long batch_x, int kernel, const ColumnSums& sums, hipStream_t st) {
+                long long batch_x, int kernel, const ColumnSums& sums, const PartialSums& later, hipStream_t st) {
     constexpr int ST32 = CT == BR_GEMM_F32 ? 1 : 2;   // as each is launched by itself
-    if (kernel == kFlex64) return launch_pair_config<CT, 64, 64, 4, 1>(w, pw, batch_w, x, px, batch_x, sums, st);
-    if (kernel == kFlex32x64) return launch_pair_config<CT, 32, 64, 4, 1>(w, pw, batch_w, x, px, batch_x, sums, st);
-    return launch_pair_config<CT, 32, 32, 4, ST32>(w, pw, batch_w, x, px, batch_x, sums, st);
+    if (kernel == kFlex64) return launch_pair_config<CT, 64, 64, 4, 1>(w, pw, batch_w, x, px, batch_x, sums, later, st);
+    if (kernel == kFlex32x64) return launch_pair_config<CT, 32, 64, 4, 1>(w, pw, batch_w, x, px, batch_x, sums, later, st);
+    return launch_pair_config<CT, 32, 32, 4, ST32>(w, pw, batch_w, x, px, batch_x, sums, later, st);
 }
 
 }  // namespace gemm16

@@ -529,10 +529,11 @@ static int layernorm_bwd_impl(const float* dy, const float* y, const float* gamm
                               const float* var, const float* residual, float* dgamma, float* dbeta, float* dx,
                               int64_t rows, int64_t cols, float eps, float param_scale, void* workspace,
                               size_t workspace_bytes, br_stream_t stream, void* dx16 = nullptr, int dx16_dtype = 0,
-                              float* dx_sum = nullptr, float* sum = nullptr) {
+                              float* dx_sum = nullptr, float* sum = nullptr, br_partial_sums* later = nullptr) {
     if (rows < 0 || cols <= 0 || rows > 0x7fffffff) return BR_ERR_ATTR;
     if (!dgamma || !dbeta) return BR_ERR_OUTPUT;
     const bool sums = dx_sum != nullptr;
+    if (later) later->partials = nullptr;
     if (rows == 0) {
         int rc = br_hip_fill(dgamma, BR_F32, 0.f, cols, stream);
         if (!rc && sums) rc = br_hip_fill(dx_sum, BR_F32, 0.f, cols, stream);
@@ -581,13 +582,14 @@ static int layernorm_bwd_impl(const float* dy, const float* y, const float* gamm
 #undef BR_LN_BWD
         BR_HIP_LAUNCH_CHECK();
         if (aligned16(dgamma) && aligned16(dbeta)) {
-            const FinalSums out{{reinterpret_cast<float4*>(dgamma), reinterpret_cast<float4*>(dbeta),
-                                 reinterpret_cast<float4*>(dx_sum)}};
-            ln_bwd_finalize_x4<<<dim3((unsigned)((cols4 + 15) / 16), sums ? 3u : 2u), 1024, 0, st>>>(
-                reinterpret_cast<const float4*>(part_g), out, parts, cols4, param_scale);
-        } else {
-            ln_bwd_finalize<<<(unsigned)((cols + 63) / 64), kBlock, 0, st>>>(part_g, part_b, dgamma, dbeta, parts, cols, param_scale);
+            const br_partial_sums left{part_g, sums ? 3 : 2, parts, cols, {dgamma, dbeta, dx_sum}, param_scale};
+            if (later) {   // the caller's next launch adds them up
+                *later = left;
+                return BR_OK;
+            }
+            return br_hip_finish_sums(&left, stream);
         }
+        ln_bwd_finalize<<<(unsigned)((cols + 63) / 64), kBlock, 0, st>>>(part_g, part_b, dgamma, dbeta, parts, cols, param_scale);
     } else {
         const int rpb = strip_rows(rows);
         parts = (int)((rows + rpb - 1) / rpb);
@@ -644,12 +646,29 @@ int br_hip_layernorm_bwd_residual_sums(const float* dy, const float* y, const fl
 int br_hip_layernorm_bwd_add(const float* dy, const float* y, const float* gamma, const float* beta, const float* var,
                              const float* residual, float* dgamma, float* dbeta, float* dx, float* sum, void* sum16,
                              int sum16_dtype, float* column_sums, int64_t rows, int64_t cols, float eps, float param_scale,
-                             void* workspace, size_t workspace_bytes, br_stream_t stream) {
+                             br_partial_sums* later, void* workspace, size_t workspace_bytes, br_stream_t stream) {
     if (rows > 0 && !residual) return BR_ERR_INPUT;
     if (!sum || sum == dx || (column_sums != nullptr) != (sum16 != nullptr)) return BR_ERR_OUTPUT;
     if (rows == 0) residual = nullptr;
-    return layernorm_bwd_impl(dy, y, gamma, beta, var, residual, dgamma, dbeta, dx, rows, cols, eps, param_scale,
-                              workspace, workspace_bytes, stream, sum16, sum16_dtype, column_sums, sum);
+    return layernorm_bwd_impl(dy, y, gamma, beta, var, residual, dgamma, dbeta, dx ? dx : sum, rows, cols, eps, param_scale,
+                              workspace, workspace_bytes, stream, sum16, sum16_dtype, column_sums, dx ? sum : nullptr, later);
+}
+
+int br_hip_finish_sums(const br_partial_sums* sums, br_stream_t stream) {
+    if (!sums || !sums->partials) return BR_OK;
+    if (sums->arrays < 1 || sums->arrays > 3 || sums->parts <= 0 || sums->parts > 0x7fffffff || sums->cols <= 0 ||
+        sums->cols % 4 != 0 || sums->cols > 0x7fffffff || !aligned16(sums->partials))
+        return BR_ERR_ATTR;
+    FinalSums out = {};
+    for (int i = 0; i < sums->arrays; i++) {
+        if (!sums->out[i] || !aligned16(sums->out[i])) return BR_ERR_OUTPUT;
+        out.out[i] = reinterpret_cast<float4*>(sums->out[i]);
+    }
+    const int cols4 = (int)(sums->cols / 4);
+    ln_bwd_finalize_x4<<<dim3((unsigned)((cols4 + 15) / 16), (unsigned)sums->arrays), 1024, 0, as_stream(stream)>>>(
+        reinterpret_cast<const float4*>(sums->partials), out, (int)sums->parts, cols4, sums->scale);
+    BR_HIP_LAUNCH_CHECK();
+    return BR_OK;
 }
 
 int br_hip_layernorm_bwd_residual(const float* dy, const float* y, const float* gamma, const float* beta,

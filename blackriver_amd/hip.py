@@ -36,6 +36,11 @@ class ColumnSums(ctypes.Structure):
                 ("workspace", _vp), ("workspace_bytes", _sz)]
 
 
+class PartialSums(ctypes.Structure):
+    """br_partial_sums: what a LayerNorm backward leaves to be added up."""
+    _fields_ = [("partials", _vp), ("arrays", _int), ("parts", _i64), ("cols", _i64), ("out", _vp * 3), ("scale", _f32)]
+
+
 # name -> (restype, argtypes); mirrors include/br_hip.h one to one
 SIGNATURES = {
     "br_hip_device_count": (_int, [ctypes.POINTER(_int)]),
@@ -87,7 +92,8 @@ SIGNATURES = {
     "br_hip_layernorm_bwd_static": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _f32, _f32, _vp]),
     "br_hip_layernorm_bwd_static_limit": (_sz, []),
     "br_hip_layernorm_bwd_residual": (_int, [_vp] * 9 + [_i64, _i64, _f32, _f32, _vp, _sz, _vp]),
-    "br_hip_layernorm_bwd_add": (_int, [_vp] * 11 + [_int, _vp, _i64, _i64, _f32, _f32, _vp, _sz, _vp]),
+    "br_hip_layernorm_bwd_add": (_int, [_vp] * 11 + [_int, _vp, _i64, _i64, _f32, _f32, _vp, _vp, _sz, _vp]),
+    "br_hip_finish_sums": (_int, [_vp, _vp]),
     "br_hip_pack_colsum": (_int, [ctypes.POINTER(_vp), _int, _vp, _vp, _int, _i64, _i64, _f32, _vp]),
     "br_hip_layernorm_bwd_sums_workspace": (_sz, [_i64, _i64]),
     "br_hip_layernorm_bwd_residual_sums": (_int, [_vp] * 10 + [_int, _vp, _i64, _i64, _f32, _f32, _vp, _sz, _vp]),
@@ -105,7 +111,7 @@ SIGNATURES = {
     "br_hip_gemm_staged": (_int, [_int, _int, _i64, _i64, _i64, _f32, _vp, _int, _i64, _i64, _vp, _int, _i64, _i64,
                                   _int, _vp, _int, _i64, _i64, _vp, _i64, _int, _vp, ctypes.c_size_t, _vp]),
     "br_hip_gemm_pair_workspace": (ctypes.c_size_t, [_vp, _vp, _int]),
-    "br_hip_gemm_pair": (_int, [_vp, _vp, _vp, _int, _vp, ctypes.c_size_t, _vp]),
+    "br_hip_gemm_pair": (_int, [_vp, _vp, _vp, _vp, _int, _vp, ctypes.c_size_t, _vp]),
     "br_hip_gemm_pair_kernel": (_int, [_i64] * 8 + [_int]),
     "br_hip_gemm_kernel": (_int, [_int, _int, _i64, _i64, _i64, _int, _i64, _int, ctypes.POINTER(_int)]),
     "br_hip_flash_attn_fwd": (_int, [_vp, _vp, _vp, _int, _vp, _vp, _vp, _vp] + [_i64] * 9 + [_vp]),

@@ -234,12 +234,25 @@ int br_hip_layernorm_bwd_residual(const float* dy, const float* y, const float* 
  * or dy's own buffer if need be), and, where asked for (both or neither), sum16 and
  * column_sums are the 16-bit image and the scaled column sums of sum.  Bits as
  * the separate entries'.  BR_ERR_TODO as for br_hip_layernorm_bwd_residual, or
- * with sums as for br_hip_layernorm_bwd_residual_sums, whose workspace it takes. */
+ * with sums as for br_hip_layernorm_bwd_residual_sums, whose workspace it takes.
+ * dx null: the sum alone.  `later` (may be null): the partial sums behind dgamma,
+ * dbeta and column_sums are left in the workspace and described in *later, for
+ * br_hip_gemm_pair to add up in its launch or br_hip_finish_sums in one of its
+ * own (later->partials is null where there was nothing to leave). */
+typedef struct br_partial_sums {
+    const float* partials;   /* arrays x parts x cols, dense */
+    int arrays;              /* up to 3 */
+    int64_t parts, cols;
+    float* out[3];           /* out[i][c] = scale * sum_p partials[i][p][c] */
+    float scale;
+} br_partial_sums;
 int br_hip_layernorm_bwd_add(const float* dy, const float* y, const float* gamma, const float* beta,
                              const float* var, const float* residual, float* dgamma, float* dbeta, float* dx,
                              float* sum, void* sum16, int sum16_dtype, float* column_sums, int64_t rows,
-                             int64_t cols, float eps, float param_scale, void* workspace,
+                             int64_t cols, float eps, float param_scale, br_partial_sums* later, void* workspace,
                              size_t workspace_bytes, br_stream_t stream);
+/* Adds up what is described in *sums (nothing where its partials are null). */
+int br_hip_finish_sums(const br_partial_sums* sums, br_stream_t stream);
 /* The same followed by what the `op.linear_backward` of the layer below does to
  * dx first (cuda_tensor.cpp:738-760: its bias gradient, the column sums of dx;
  * and, for 16-bit products, the 16-bit image of dx both of its products read):
@@ -377,7 +390,7 @@ int br_hip_gemm_staged(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k
                        void* workspace, size_t workspace_bytes, br_stream_t stream);
 
 /* Two products, with the column sums of a matrix before them (sums may be
- * null): what br_hip_colsum(sums), br_hip_gemm_staged(first) and
+ * null, and so may later): what br_hip_finish_sums(later), br_hip_colsum(sums), br_hip_gemm_staged(first) and
  * br_hip_gemm_staged(second) do one after the other (br_hip_gemm in place of the
  * latter with BR_GEMM_F32), for the operators that multiply one gradient twice:
  * op_linear_backward (cuda_tensor.cpp:565-622), op_attn_backward and
@@ -413,8 +426,9 @@ typedef struct br_column_sums {
     size_t workspace_bytes;
 } br_column_sums;
 size_t br_hip_gemm_pair_workspace(const br_product* first, const br_product* second, int compute);
-int br_hip_gemm_pair(const br_product* first, const br_product* second, const br_column_sums* sums, int compute,
-                     void* workspace, size_t workspace_bytes, br_stream_t stream);
+int br_hip_gemm_pair(const br_product* first, const br_product* second, const br_column_sums* sums,
+                     const br_partial_sums* later, int compute, void* workspace, size_t workspace_bytes,
+                     br_stream_t stream);
 int br_hip_gemm_pair_kernel(int64_t m1, int64_t n1, int64_t k1, int64_t batch1, int64_t m2, int64_t n2, int64_t k2,
                             int64_t batch2, int compute);
 

@@ -677,7 +677,7 @@ def whole_numbers(shape, most, dtype):
     return torch.randint(-most, most + 1, shape, device="cuda").to(TORCH_T[dtype])
 
 
-def run_pair(products, compute, sums=None):
+def run_pair(products, compute, sums=None, later=None):
     """br_hip_gemm_pair on (trans_a, trans_b, a, b, c) with [batch, rows, cols] tensors; whether it was one launch."""
     code = {torch.float32: F32, torch.float16: F16, torch.bfloat16: BF16}
     descs, sizes = [], []
@@ -689,7 +689,8 @@ def run_pair(products, compute, sums=None):
     first, second = (ctypes.byref(d) for d in descs)
     need = hip.load().br_hip_gemm_pair_workspace(first, second, compute)
     ws = torch.full((max(need, 16),), 0x7f, dtype=torch.uint8, device="cuda")
-    call("br_hip_gemm_pair", first, second, ctypes.byref(sums) if sums else None, compute, ptr(ws), need, stream())
+    call("br_hip_gemm_pair", first, second, ctypes.byref(sums) if sums else None, ctypes.byref(later) if later else None, compute,
+         ptr(ws), need, stream())
     torch.cuda.synchronize()
     return hip.load().br_hip_gemm_pair_kernel(*sizes, compute) >= 0
 
@@ -724,6 +725,30 @@ def test_two_products_of_a_linear_layer_in_one_launch_are_exact_on_integers(n, i
         assert torch.equal(dw, pair_reference(1, 0, dy, x).float())
         assert torch.equal(dx, pair_reference(0, 0, dy, w).to(dx.dtype))
         assert torch.equal(db, 0.5 * dy[0].float().sum(0))
+
+
+@pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16, hip.GEMM_F32])
+@pytest.mark.parametrize("n", [64, 700])   # one launch, and (16-bit) two after the sums
+@pytest.mark.parametrize("arrays,parts,cols", [(2, 1, 4), (3, 7, 68), (3, 39, 256), (2, 64, 1000), (3, 65, 60), (3, 256, 4096)])
+def test_partial_sums_are_added_up_beside_two_products(arrays, parts, cols, n, compute):
+    """Whole numbers, so exact; a partial last group of columns, fewer parts than slices and more, and no room outside."""
+    torch.manual_seed(cols)
+    inn = out = 256 if n == 64 else 4096
+    dt = COMPUTE_T[compute]
+    print("case n=%d arrays=%d parts=%d cols=%d compute=%d" % (n, arrays, parts, cols, compute), flush=True)
+    dy, x, w = (whole_numbers(s, 1, dt) for s in ((1, n, out), (1, n, inn), (1, out, inn)))
+    dw, dx = torch.empty((1, out, inn), device="cuda"), torch.empty((1, n, inn), device="cuda", dtype=TORCH_T[dt])
+    partials = whole_numbers((arrays, parts, cols), 50, F32)
+    sums = torch.full((arrays, cols + 4), float("nan"), device="cuda")
+    outs = (ctypes.c_void_p * 3)(*[sums[i].data_ptr() for i in range(arrays)])
+    later = hip.PartialSums(ptr(partials), arrays, parts, cols, outs, 0.5)
+    assert run_pair([(1, 0, dy, x, dw), (0, 0, dy, w, dx)], compute, None, later) == (n == 64 or compute == hip.GEMM_F32)
+    assert torch.equal(sums[:, :cols], 0.5 * partials.sum(1)) and sums[:, cols:].isnan().all()
+    assert torch.equal(dw, pair_reference(1, 0, dy, x).float())
+    assert torch.equal(dx, pair_reference(0, 0, dy, w).to(dx.dtype))
+    sums.fill_(float("nan"))
+    call("br_hip_finish_sums", ctypes.byref(later), stream())   # a launch of their own
+    assert torch.equal(sums[:, :cols], 0.5 * partials.sum(1)) and sums[:, cols:].isnan().all()
 
 
 @pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16, hip.GEMM_F32])
