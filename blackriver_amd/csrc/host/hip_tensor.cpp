@@ -1067,6 +1067,80 @@ ComputingReturn hip_gelu_linear_then_add(const tensor_t& u, const tensor_t& v, c
     return r != OP_OK ? r : hip_linear_then_add(lin, add);
 }
 
+namespace {
+// The backward pass of a linear layer whose input is a GELU's output and whose input gradient is written over it, then of
+// that GELU and of the layer ahead (low: x w b x_g w_g b_g of the first, its dy being `dy`; tail: dy u du of the GELU and
+// dy x w b x_g w_g b_g of the layer ahead).  The first layer's two products can only share a launch where neither
+// overwrites what the other reads: its input gradient goes to the workspace, and the GELU's pass, which reads it anyway,
+// leaves it where it belongs.  A block's forward and backward pass on [64 x 256] 78.6 -> 76.1 us, on [78 x 1024]
+// 135.7 -> 135.0.  BR_ERR_TODO: not of that form, or not small; nothing has been done.
+int gelu_between(const Operand& dy, const tensor_t* low, const tensor_t* tail, int64_t n, int compute, const br_partial_sums* later) {
+    const tensor_t &x = low[0], &w = low[1], &x_g = low[3], &w_g = low[4], &u = tail[1], &du = tail[2];
+    const tensor_t* top = tail + 3;   // dy x w b x_g w_g b_g
+    const int native = compute == BR_GEMM_F16 ? BR_F16 : BR_BF16;
+    if (compute == BR_GEMM_F32 || dy.dtype != native || !dev(x) || code(x) != native || !same_tensor(x_g, x) || !same_tensor(tail[0], x) ||
+        !dev(u) || !dev(du) || code(u) != native || code(du) != native || u->items() != x->items() || du->items() != x->items() ||
+        !same_tensor(top[0], du) || du->shape().dim() != 3 || x->shape().dim() != 3)
+        return BR_ERR_TODO;
+    const int64_t mid = (int64_t)x->shape()[2], out = (int64_t)w->shape()[0], in = (int64_t)(top[1]->items()) / n;
+    if ((int64_t)w->items() != out * mid || (int64_t)du->shape()[2] != mid || mid % 8 != 0 || !dev(top[1]) || !dev(top[2]) ||
+        !dev(top[4]) || !dev(top[5]) || !dev_f32(top[6]) || top[1]->shape().dim() != 3 || (int64_t)top[1]->items() != n * in ||
+        (int64_t)top[2]->items() != mid * in || (int64_t)top[4]->items() != n * in || (int64_t)top[5]->items() != mid * in ||
+        (int64_t)top[6]->items() != mid || pick_compute({du, top[1], top[2]}) != compute)
+        return BR_ERR_TODO;
+    if (!(same_tensor(u, du) || apart(u, du)) || !apart(du, x) || !apart(u, x) || !apart(x, w) || !apart(x, w_g) || !apart(du, w_g) || !apart(u, w_g) ||
+        !apart(top[6], x) || !apart(top[6], u) || !apart(top[6], du))
+        return BR_ERR_TODO;
+    auto off = [](const tensor_t& t) { return (reinterpret_cast<uintptr_t>(t->data()) & 15) != 0; };
+    if (off(x) || off(u) || off(du) || !br_hip_bias_gelu_bwd_copies(n, mid) ||
+        br_hip_gemm_pair_kernel(out, mid, n, 1, n, mid, out, 1, compute) < 0)
+        return BR_ERR_TODO;
+    // partial sums that wait to be added up lie at the workspace's head
+    const size_t sums = later && later->partials ? (size_t)(later->arrays * later->parts * later->cols) * sizeof(float) : 0;
+    const size_t at = (sums + 255) / 256 * 256;
+    if (at + (size_t)(n * mid) * 2 > head_bytes()) return BR_ERR_TODO;
+    void* x_grad = static_cast<char*>(ComputingContext::workspace) + at;
+    int rc = two_products({1, 0, out, mid, n, unlift(), dy.ptr, dy.dtype, out, 0, x->data(), native, mid, 0, w_g->data(), code(w_g), mid, 0, 1},
+                          {0, 0, n, mid, out, 1.0f, dy.ptr, dy.dtype, out, 0, w->data(), code(w), mid, 0, x_grad, native, mid, 0, 1},
+                          nullptr, compute, later);
+    if (rc != BR_OK) return rc;
+    rc = br_hip_bias_gelu_bwd_copy(x_grad, u->data(), nullptr, du->data(), static_cast<float*>(top[6]->data()), x->data(), native, n,
+                                   mid, unlift(), stream());
+    if (rc != BR_OK) return rc;
+    return linear_backward_products(Operand{du->data(), native}, top[1], top[2], top[4], top[5], n, in, mid, compute);
+}
+}  // namespace
+
+ComputingReturn hip_linear_gelu_linear_backward(const tensor_t* lin, const tensor_t* tail) {
+    const tensor_t &dy = lin[0], &x = lin[1], &w = lin[2];
+    if (dev_f32(dy) && dy->shape().dim() == 3 && dev(x) && x->shape().dim() == 3 && dev(w) && w->shape().dim() == 2 && dev(lin[4]) &&
+        dev(lin[5]) && dev_f32(lin[6])) {
+        const int64_t n = (int64_t)(dy->shape()[0] * dy->shape()[1]), out = (int64_t)dy->shape()[2], in = (int64_t)x->shape()[2];
+        const int compute = pick_compute({dy, x, w});
+        if (compute != BR_GEMM_F32 && out % 8 == 0 && (int64_t)x->items() == n * in && (int64_t)w->items() == out * in &&
+            (int64_t)lin[5]->items() == out * in && (int64_t)lin[6]->items() == out &&
+            same_tensor(lin[4], x)) {
+            // (the first pass of op_linear_backward)
+            const int native = compute == BR_GEMM_F16 ? BR_F16 : BR_BF16;
+            const size_t need = br_hip_colsum_workspace(n, out);
+            void* ws = need <= head_bytes() ? ComputingContext::workspace : ComputingContext::scratch(need);
+            void* dy16 = ComputingContext::gemm_staging(1, (size_t)(n * out) * 2);
+            BR_OP(br_hip_colsum_cast(static_cast<const float*>(dy->data()), static_cast<float*>(lin[6]->data()), dy16, native, n, out,
+                                     unlift(), ws, need, stream()));
+            const int rc = gelu_between(Operand{dy16, native}, lin + 1, tail, n, compute, nullptr);
+            if (rc != BR_ERR_TODO) {
+                BR_OP(rc);
+                return OP_OK;
+            }
+            BR_OP(linear_backward_products(Operand{dy16, native}, x, w, lin[4], lin[5], n, in, out, compute));
+            return hip_gelu_linear_backward(tail[0], tail[1], tail[2], tail[4], tail[5], tail[6], tail[7], tail[8], tail[9]);
+        }
+    }
+    const ComputingReturn r = dy->op_linear_backward(dy, x, w, lin[3], lin[4], lin[5], lin[6]);
+    if (r != OP_OK) return r;
+    return hip_gelu_linear_backward(tail[0], tail[1], tail[2], tail[4], tail[5], tail[6], tail[7], tail[8], tail[9]);
+}
+
 // op_layernorm_backward(ln[0..7], eps) followed by op_add(add[0], add[1], add[2]) of its din and a residual, and, unless
 // lin is null, by op_linear_backward(lin[0..6]) of that sum.  One pass of the LayerNorm kernel leaves din, the sum, and for
 // the linear layer the sum's 16-bit image and its bias gradient; anything else runs as the operators.
@@ -1196,7 +1270,12 @@ ComputingReturn hip_layernorm_backward_add_linear_backward(
     const tensor_t& dy, const tensor_t& scale, const tensor_t& bias, const tensor_t& var, const tensor_t& y,
     const tensor_t& dscale, const tensor_t& dbias, const tensor_t& residual, const tensor_t& din, float eps,
     const tensor_t& x, const tensor_t& weight, const tensor_t& lbias, const tensor_t& x_g, const tensor_t& weight_g,
-    const tensor_t& bias_g) {
+    const tensor_t& bias_g, const tensor_t* tail) {
+    // what follows the linear layer's backward: a GELU's and that of the layer ahead of it, or nothing
+    auto rest = [&]() {
+        if (!tail) return OP_OK;
+        return hip_gelu_linear_backward(tail[0], tail[1], tail[2], tail[4], tail[5], tail[6], tail[7], tail[8], tail[9]);
+    };
     bool fast = dev_f32(dy) && dev_f32(scale) && dev_f32(bias) && dev_f32(var) && dev_f32(y) && dev_f32(dscale) &&
                 dev_f32(dbias) && dev_f32(residual) && dev_f32(din) && dy->shape().dim() == 3 && dev(x) &&
                 dev(weight) && dev(x_g) && dev(weight_g) && dev_f32(bias_g) && x->shape().dim() == 3 &&
@@ -1229,9 +1308,17 @@ ComputingReturn hip_layernorm_backward_add_linear_backward(
                 unlift(), &later, ws, need, stream());
             if (rc != BR_ERR_TODO) {
                 BR_OP(rc);
+                if (tail) {
+                    const tensor_t low[6] = {x, weight, lbias, x_g, weight_g, bias_g};
+                    const int rg = gelu_between(Operand{d16, native}, low, tail, rows, compute, &later);
+                    if (rg != BR_ERR_TODO) {
+                        BR_OP(rg);
+                        return OP_OK;
+                    }
+                }
                 BR_OP(linear_backward_products(Operand{d16, native}, x, weight, x_g, weight_g, rows, in, cols, compute, nullptr,
                                                &later));
-                return OP_OK;
+                return rest();
             }
         }
     }

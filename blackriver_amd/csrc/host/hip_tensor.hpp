@@ -118,6 +118,9 @@ ComputingReturn hip_layernorm_backward_add_linear_backward(
     const tensor_t& dy, const tensor_t& scale, const tensor_t& bias, const tensor_t& var, const tensor_t& y,
     const tensor_t& dscale, const tensor_t& dbias, const tensor_t& residual, const tensor_t& din, float eps,
     const tensor_t& x, const tensor_t& weight, const tensor_t& lbias, const tensor_t& x_g, const tensor_t& weight_g,
-    const tensor_t& bias_g);
+    const tensor_t& bias_g, const tensor_t* tail = nullptr);
+// op_linear_backward (lin: dy x w b x_g w_g b_g) followed by hip_gelu_linear_backward (tail: dy u du and dy x w b x_g w_g
+// b_g, the latter's dy being du); the function above takes such a tail too.
+ComputingReturn hip_linear_gelu_linear_backward(const tensor_t* lin, const tensor_t* tail);
 
 }  // namespace br

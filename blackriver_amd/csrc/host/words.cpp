@@ -438,6 +438,40 @@ BR_WORD(GeluLinearBackward,
         l[0]->op_linear_backward(l[0], l[1], l[2], l[3], l[4], l[5], l[6]);
     }
 )
+// The seven of a linear layer's backward, then the three of a GELU's and the seven of the layer ahead of it: the GELU's du
+// has to be the latter's dy.
+struct GeluBetween {
+    tensor_t t[10];
+    explicit GeluBetween(Stack& stack) {
+        Tensors<7> l(stack);
+        Tensors<3> g(stack);
+        for (int i = 0; i < 3; i++) t[i] = g[i];
+        for (int i = 0; i < 7; i++) t[3 + i] = l[i];
+    }
+    bool joined() const { return t[3]->data() == t[2]->data() && t[3]->items() == t[2]->items(); }
+    void run() const {
+        if (joined()) {
+            op_check_word(hip_gelu_linear_backward(t[0], t[1], t[2], t[4], t[5], t[6], t[7], t[8], t[9]),
+                          "op.gelu_backward + op.linear_backward");
+            return;
+        }
+        tensor_t dy = t[0], low = t[3];
+        dy->op_gelu_backward(t[0], t[1], t[2]);
+        low->op_linear_backward(t[3], t[4], t[5], t[6], t[7], t[8], t[9]);
+    }
+};
+// ( dy x w b x_g w_g b_g   dy' u du   du' x' w' b' x_g' w_g' b_g' -- )  `op.linear_backward`, `op.gelu_backward` and
+// `op.linear_backward` in a row
+BR_WORD(LinearGeluLinearBackward,
+    GeluBetween tail(stack);
+    Tensors<7> l(stack);
+    if (tail.joined()) {
+        op_check_word(hip_linear_gelu_linear_backward(l.t, tail.t), "op.linear_backward + op.gelu_backward + op.linear_backward");
+    } else {
+        l[0]->op_linear_backward(l[0], l[1], l[2], l[3], l[4], l[5], l[6]);
+        tail.run();
+    }
+)
 // ( x w b u y -- )   u = x . w^T + b,  y = gelu(u)      `op.linear` + `op.gelu`
 BR_WORD(LinearGelu,
     Tensors<5> a(stack);
@@ -475,6 +509,26 @@ BR_WORD(LayernormBackwardAddLinearBackward,
                       "op.layernorm_backward_add");
         l[0]->op_linear_backward(l[0], l[1], l[2], l[3], l[4], l[5], l[6]);
     }
+)
+
+// The same followed by `op.gelu_backward` and the `op.linear_backward` of the layer ahead of it
+BR_WORD(LayernormBackwardAddLinearGeluLinearBackward,
+    GeluBetween tail(stack);
+    Tensors<7> l(stack);
+    const float eps = (float)stack.pop_number();
+    Tensors<9> a(stack);
+    const bool linear = l[0]->data() == a[8]->data() && l[0]->items() == a[8]->items();
+    if (linear) {
+        op_check_word(hip_layernorm_backward_add_linear_backward(a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], eps,
+                                                                 l[1], l[2], l[3], l[4], l[5], l[6],
+                                                                 tail.joined() ? tail.t : nullptr),
+                      "op.layernorm_backward_add + op.linear_backward + op.gelu_backward + op.linear_backward");
+    } else {
+        op_check_word(hip_layernorm_backward_add(a[0], a[1], a[2], a[3], a[4], a[5], a[6], a[7], a[8], eps),
+                      "op.layernorm_backward_add");
+        l[0]->op_linear_backward(l[0], l[1], l[2], l[3], l[4], l[5], l[6]);
+    }
+    if (!linear || !tail.joined()) tail.run();
 )
 
 // ( dy scale bias var y dscale dbias din eps   a b c   dy' x w b x_g w_g b_g -- )  `op.layernorm_backward`, `op.add` and
@@ -662,6 +716,8 @@ void load_nn_words(Enviroment& env) {
         {"op.gelu_linear_then_add", GeluLinearThenAdd::creator},
         {"op.transpos_0213_x3", Transpos0213x3::creator},
         {"op.gelu_linear_backward", GeluLinearBackward::creator},
+        {"op.linear_gelu_linear_backward", LinearGeluLinearBackward::creator},
+        {"op.layernorm_backward_add_linear_gelu_linear_backward", LayernormBackwardAddLinearGeluLinearBackward::creator},
         {"op.linear_add", LinearAdd::creator},
         {"op.linear_gelu", LinearGelu::creator},
         {"op.linear_residual", LinearResidual::creator},
@@ -680,7 +736,6 @@ void load_nn_words(Enviroment& env) {
     env.insert_fusion({"op.add", "op.add", "op.softmax", "op.copy"}, "op.add_add_softmax_copy");
     env.insert_fusion({"op.add", "op.add", "op.softmax"}, "op.add_add_softmax");
     env.insert_fusion({"op.layernorm", "op.copy"}, "op.layernorm_copy");
-    env.insert_fusion({"op.gelu_backward", "op.linear_backward"}, "op.gelu_linear_backward");
     env.insert_fusion({"op.layernorm", "op.linear", "op.linear", "op.linear"}, "op.layernorm_linear_x3");
     env.insert_fusion({"op.linear", "op.linear", "op.linear"}, "op.linear_x3");
     env.insert_fusion({"op.gelu", "op.linear", "op.add"}, "op.gelu_linear_then_add");
@@ -690,7 +745,11 @@ void load_nn_words(Enviroment& env) {
     env.insert_fusion({"op.zero", "op.linear_backward", "op.add", "op.linear_backward", "op.add", "op.linear_backward", "op.add",
                        "op.layernorm_backward", "op.add"}, "op.qkv_backward_layernorm");
     env.insert_fusion({"op.layernorm_backward", "op.add", "op.linear_backward"}, "op.layernorm_backward_then_add_linear_backward");
-    // the pair also stands across a block boundary of a model program
+    // these two also stand across a block boundary of a model program
+    env.insert_fusion({"op.layernorm_backward_add", "op.linear_backward", "op.gelu_backward", "op.linear_backward"},
+                      "op.layernorm_backward_add_linear_gelu_linear_backward", true);
+    env.insert_fusion({"op.linear_backward", "op.gelu_backward", "op.linear_backward"}, "op.linear_gelu_linear_backward");
+    env.insert_fusion({"op.gelu_backward", "op.linear_backward"}, "op.gelu_linear_backward");
     env.insert_fusion({"op.layernorm_backward_add", "op.linear_backward"}, "op.layernorm_backward_add_linear_backward", true);
 }
 

@@ -750,6 +750,7 @@ struct OwnBiasGeluBwd {
     const T* x;
     const float* bias;
     T* dx;
+    T* dy_copy;   // null: none
     float b[V];
     static constexpr int VEC = V, NIN = 2;
     __device__ __forceinline__ void init(int64_t col) {
@@ -761,6 +762,7 @@ struct OwnBiasGeluBwd {
         VecIO<T, V>::load(x + at, in[1]);
     }
     __device__ __forceinline__ void finish(int64_t at, float (&in)[NIN][VEC]) const {
+        if (dy_copy) VecIO<T, V>::store_rounded(dy_copy + at, in[0]);   // exact: the values are of this type
 #pragma unroll
         for (int j = 0; j < V; j++) in[0][j] *= gelu_grad_one(in[1][j] + b[j]);
         VecIO<T, V>::store_rounded(dx + at, in[0]);
@@ -1480,6 +1482,31 @@ int br_hip_gelu_bwd(const void* dy, const void* x, void* dx, int dtype, int64_t 
 
 size_t br_hip_bias_gelu_bwd_workspace(int64_t rows, int64_t cols) { return br_hip_colsum_workspace(rows, cols); }
 
+// Rows and columns that a single launch owns with its sums (owner_lanes): the copy is one more store there, in the two
+// launches of larger sizes, where the products around fill the chip one at a time, nothing asks for it.
+int br_hip_bias_gelu_bwd_copies(int64_t rows, int64_t cols) {
+    return rows > 0 && cols > 0 && owner_lanes(rows, cols, 2, kOwnBiasGelu) != 0;
+}
+
+int br_hip_bias_gelu_bwd_copy(const void* dy, const void* x, const float* bias, void* dx, float* dbias, void* dy_copy, int dtype,
+                              int64_t rows, int64_t cols, float dbias_scale, br_stream_t stream) {
+    if (rows < 0 || cols <= 0) return BR_ERR_ATTR;
+    if (rows == 0) return BR_OK;
+    if (!dy || !x) return BR_ERR_INPUT;
+    if (!dx || !dbias || !dy_copy || dy_copy == dy || dy_copy == dx || dy_copy == x) return BR_ERR_OUTPUT;
+    if ((dtype != BR_F16 && dtype != BR_BF16) || !br_hip_bias_gelu_bwd_copies(rows, cols) || !aligned16(dy) || !aligned16(x) ||
+        !aligned16(dx) || !aligned16(dy_copy))
+        return BR_ERR_TODO;
+    const int lanes = owner_lanes(rows, cols, 2, kOwnBiasGelu);
+    hipStream_t st = as_stream(stream);
+    if (dtype == BR_F16)
+        return colsum_owner_launch<2>(lanes, OwnBiasGeluBwd<__half, 8>{(const __half*)dy, (const __half*)x, bias, (__half*)dx,
+                                                                       (__half*)dy_copy}, dbias, rows, cols, dbias_scale, st);
+    return colsum_owner_launch<2>(lanes, OwnBiasGeluBwd<__hip_bfloat16, 8>{(const __hip_bfloat16*)dy, (const __hip_bfloat16*)x, bias,
+                                                                           (__hip_bfloat16*)dx, (__hip_bfloat16*)dy_copy},
+                                  dbias, rows, cols, dbias_scale, st);
+}
+
 int br_hip_bias_gelu_bwd(const void* dy, const void* x, const float* bias, void* dx, float* dbias, int dtype,
                          int64_t rows, int64_t cols, float dbias_scale, void* workspace, size_t workspace_bytes,
                          br_stream_t stream) {
@@ -1500,13 +1527,13 @@ int br_hip_bias_gelu_bwd(const void* dy, const void* x, const float* bias, void*
     if (const int lanes = dbias && al ? owner_lanes(rows, cols, dtype == BR_F32 ? 4 : 2, kOwnBiasGelu) : 0) {
         // gradient and bias gradient from one launch
         if (dtype == BR_F32)
-            return colsum_owner_launch<2>(lanes, OwnBiasGeluBwd<float, 4>{(const float*)dy, (const float*)x, bias, (float*)dx},
+            return colsum_owner_launch<2>(lanes, OwnBiasGeluBwd<float, 4>{(const float*)dy, (const float*)x, bias, (float*)dx, nullptr},
                                           dbias, rows, cols, dbias_scale, st);
         if (dtype == BR_F16)
-            return colsum_owner_launch<2>(lanes, OwnBiasGeluBwd<__half, 8>{(const __half*)dy, (const __half*)x, bias, (__half*)dx},
+            return colsum_owner_launch<2>(lanes, OwnBiasGeluBwd<__half, 8>{(const __half*)dy, (const __half*)x, bias, (__half*)dx, nullptr},
                                           dbias, rows, cols, dbias_scale, st);
         return colsum_owner_launch<2>(lanes, OwnBiasGeluBwd<__hip_bfloat16, 8>{(const __hip_bfloat16*)dy, (const __hip_bfloat16*)x,
-                                                                        bias, (__hip_bfloat16*)dx},
+                                                                        bias, (__hip_bfloat16*)dx, nullptr},
                                       dbias, rows, cols, dbias_scale, st);
     }
     if (dtype == BR_F32 && al && cols % 4 == 0) {

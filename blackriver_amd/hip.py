@@ -71,6 +71,8 @@ SIGNATURES = {
     "br_hip_gelu_fwd_f32_to_16": (_int, [_vp, _vp, _int, _i64, _vp]),
     "br_hip_gelu_bwd": (_int, [_vp, _vp, _vp, _int, _i64, _vp]),
     "br_hip_bias_gelu_fwd": (_int, [_vp, _vp, _vp, _int, _i64, _i64, _vp]),
+    "br_hip_bias_gelu_bwd_copies": (_int, [_i64, _i64]),
+    "br_hip_bias_gelu_bwd_copy": (_int, [_vp] * 6 + [_int, _i64, _i64, _f32, _vp]),
     "br_hip_bias_gelu_bwd_workspace": (_sz, [_i64, _i64]),
     "br_hip_linear_gelu": (_int, [_vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _vp]),
     "br_hip_linear_group_workspace": (_sz, [_int, _i64, _i64, _i64, _int, _int]),

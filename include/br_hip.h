@@ -123,6 +123,11 @@ int br_hip_bias_gelu_fwd(const void* x, const float* bias, void* y, int dtype, i
  * workspace must hold br_hip_bias_gelu_bwd_workspace(rows, cols) bytes when
  * dbias != NULL. */
 size_t br_hip_bias_gelu_bwd_workspace(int64_t rows, int64_t cols);
+/* The same on 16-bit tensors at 16-byte addresses, with dy also copied to
+ * dy_copy.  One launch; BR_ERR_TODO where the sizes take two (_copies is 0). */
+int br_hip_bias_gelu_bwd_copies(int64_t rows, int64_t cols);
+int br_hip_bias_gelu_bwd_copy(const void* dy, const void* x, const float* bias, void* dx, float* dbias, void* dy_copy,
+                              int dtype, int64_t rows, int64_t cols, float dbias_scale, br_stream_t stream);
 int br_hip_bias_gelu_bwd(const void* dy, const void* x, const float* bias, void* dx,
                          float* dbias, int dtype, int64_t rows, int64_t cols, float dbias_scale,
                          void* workspace, size_t workspace_bytes, br_stream_t stream);

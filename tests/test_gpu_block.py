@@ -592,6 +592,76 @@ def test_fused_layernorm_backward_add_linear_backward_equals_the_two_words(runti
         env.close()
 
 
+@pytest.mark.parametrize("with_layernorm", [False, True])
+@pytest.mark.parametrize("mode", ["f16", "bf16"])
+@pytest.mark.parametrize("b,t,hidden,in_place", [
+    (1, 3, 8, True), (2, 24, 128, True), (1, 129, 264, True), (2, 250, 128, True), (1, 513, 384, True),
+    (1, 600, 640, True),      # a GELU backward of two launches: the words one by one
+    (2, 24, 128, False)])     # the first layer's input gradient not over its input: likewise
+def test_fused_backward_of_two_linear_layers_and_the_gelu_between_equals_the_words(runtime, b, t, hidden, in_place, mode,
+                                                                                   with_layernorm):
+    """4h -> h, GELU and h -> 4h of a block whose 4h activation is kept in the products' type.  The gradients that are
+    rounded on the way are small whole numbers, so the order of no sum shows: the same bits as the words one by one, except
+    in the last products, whose two kernels are the same on both sides."""
+    rng = np.random.default_rng(hidden + t)
+    mid = 4 * hidden
+    print("case %d x %d x %d %s in_place=%s layernorm=%s" % (b, t, hidden, mode, in_place, with_layernorm), flush=True)
+    env = host.Env(1)
+    try:
+        env.execute("'%s' op.gemm_precision" % mode)
+        for n, cols, dt in (("dy", hidden, "float"), ("ln", hidden, "float"), ("res", hidden, "float"), ("din", hidden, "float"),
+                            ("act", mid, mode), ("actg", mid, mode), ("u", mid, mode), ("x", hidden, mode), ("xg", hidden, "float")):
+            env.execute("%d %d %d 3 'cuda' '%s' op.create '%s' !" % (b, t, cols, dt, n))
+        for n, rows, cols, dt in (("w1", mid, hidden, mode), ("w1g", mid, hidden, "float"), ("w2", hidden, mid, mode),
+                                  ("w2g", hidden, mid, "float")):
+            env.execute("%d %d 2 'cuda' '%s' op.create '%s' !" % (rows, cols, dt, n))
+        for n, size in (("b1", mid), ("b1g", mid), ("b2", hidden), ("b2g", hidden), ("gam", hidden), ("bet", hidden), ("dgam", hidden),
+                        ("dbet", hidden), ("var", b * t)):
+            env.execute("%d 1 'cuda' 'float' op.create '%s' !" % (size, n))
+        whole = lambda *shape: rng.integers(-1, 2, shape).astype(np.float32)
+        for n in ("gam", "var"):
+            env.execute("'%s' @ 1.0 op.fill" % n)
+        for n in ("bet", "dy"):
+            env.execute("'%s' @ op.zero" % n)      # the LayerNorm's gradient is nothing: the sum is the residual
+        env.write("ln", rng.standard_normal((b, t, hidden)).astype(np.float32))
+        env.write("w1", (0.05 * rng.standard_normal((mid, hidden))).astype(np.float32))
+        env.write("w2", whole(hidden, mid))
+        env.write("x", rng.standard_normal((b, t, hidden)).astype(np.float32))
+        act, u = whole(b, t, mid), rng.standard_normal((b, t, mid)).astype(np.float32)
+        grad = "act" if in_place else "actg"
+        words = ["'res' @ 'act' @ 'w2' @ 'b2' @ '%s' @ 'w2g' @ 'b2g' @ op.linear_backward" % grad,
+                 "'%s' @ 'u' @ 'u' @ op.gelu_backward" % grad,
+                 "'u' @ 'x' @ 'w1' @ 'b1' @ 'xg' @ 'w1g' @ 'b1g' @ op.linear_backward"]
+        # (op.gelu_backward itself has no bf16 form: there the pair of words is what the three are compared with)
+        apart = [words[0], "  ".join(words[1:])]
+        name = "W:op.linear_gelu_linear_backward"
+        if with_layernorm:
+            head = "'dy' @ 'gam' @ 'bet' @ 'var' @ 'ln' @ 'dgam' @ 'dbet' @ 'res' @ 'din' @ 1e-5 op.layernorm_backward_add"
+            words[0] = apart[0] = words[0].replace("'res'", "'din'")
+            words, apart = [head + "  0 #"] + words, [head] + apart
+            name = "W:op.layernorm_backward_add_linear_gelu_linear_backward"
+        assert name in env.disassemble("  ".join(words), fused=True)
+        res = whole(b, t, hidden)
+        outs = ("u", grad, "xg", "w1g", "w2g", "b1g", "b2g") + (("din", "dgam", "dbet") if with_layernorm else ())
+
+        def run(programs):
+            for n in outs:
+                env.execute("'%s' @ op.zero" % n)
+            env.write("act", act)
+            env.write("u", u)
+            env.write("res", res)
+            for text in programs:
+                env.execute(text)
+            return {n: env.read(n) for n in outs}
+
+        want, got = run(apart), run(["  ".join(words)])
+        assert np.abs(want[grad]).max() <= 256 and np.any(want["xg"] != 0)
+        for n in outs:
+            assert np.array_equal(got[n], want[n]), n
+    finally:
+        env.close()
+
+
 def test_fused_attention_follows_the_mask_tables_prefix_rule(runtime):
     """A mask with a hole: the reference's table closes every key from the
     first zero on (train_bloom.cpp:73-90), so `bloom.valid` must report the
