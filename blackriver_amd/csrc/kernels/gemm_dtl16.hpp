@@ -635,6 +635,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64) void gemm_dtl_kern
 // from K = 512 99 -> 95 us, [4096 x 4096] 66.2 -> 64.6, h -> 4h forward 241 -> 237.
 // Memory operations complete in issue order on this target, which is what the partial waits rest on: after the 16
 // operand loads of the next tile come the wave's 128 stores, so "at most 63 outstanding" means the loads are in.
+// An fp32 C, 64 MB and more of it, is stored past the caches: a weight gradient [250880 x 4096] from K = 512 1480 -> 1270 us
+// (its 4.1 GB had pushed the operands out), [16384 x 4096] from K = 2048 259 -> 254, none slower.
 // Plain products only: 256 x 256 tiles, all of them interior (m, n multiples of 256), one batch, no bias, nothing
 // accumulated, no second output (walk_applies); everything else takes gemm_dtl_kernel.
 template <int CT, bool A_KSTR, bool B_KSTR, typename TC>
@@ -784,8 +786,8 @@ __global__ __launch_bounds__(512) void gemm_dtl_walk_kernel(GemmArgs g) {
             for (int v = 0; v < 16; v++) {
                 float o = alpha * acc[i][j][v] + 0.f;   // the plain epilogue's expression with its bias of zero
                 if (sizeof(TC) == 2) asm volatile("" : "+v"(o));   // one fp32 value, then one rounding (see gemm_dtl_kernel)
-                c_store<TC>(reinterpret_cast<TC*>(c_tile + (i * 32 + (v >> 2) * 8 + (v & 3)) * g.ldc * (long long)sizeof(TC) +
-                                                  j * 32 * sizeof(TC) + lane_bytes), o);
+                c_store_past<TC>(reinterpret_cast<TC*>(c_tile + (i * 32 + (v >> 2) * 8 + (v & 3)) * g.ldc * (long long)sizeof(TC) +
+                                                       j * 32 * sizeof(TC) + lane_bytes), o);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
