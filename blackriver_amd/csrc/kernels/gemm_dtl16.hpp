@@ -197,6 +197,10 @@ __device__ __forceinline__ void buffer_write(__amdgpu_buffer_rsrc_t r, unsigned 
     }
 }
 
+// Tiles of which a CU runs two at a time, each with 32-wide K steps: while one workgroup stores its tile the other
+// multiplies (see shared_applies).
+constexpr bool shared_tile(int bm, int bn, int kt) { return bm * bn == 128 * 256 && kt == 32; }
+
 // KW = 2: the sixteen-wide sub-steps of every K step are dealt to two groups of waves (group kw takes sub-steps
 // kw * KS/2 ..), each group covering the whole tile with wave tiles twice as large; the groups' accumulators are
 // added through LDS after the K loop (group 1 into group 0, which runs the epilogue).  For tiles too small to give
@@ -204,7 +208,7 @@ __device__ __forceinline__ void buffer_write(__amdgpu_buffer_rsrc_t r, unsigned 
 // from LDS, on two groups of four 64 x 128 waves 96 KB.
 template <int CT, int BM, int BN, int WM, int WN, int KT, int STAGES, bool A_KSTR, bool B_KSTR, typename TC,
           bool GELU = false, bool SPLIT = false, int KW = 1, bool RAG = false>
-__global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64) void gemm_dtl_kernel(GemmArgs g) {
+__global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64, (shared_tile(BM, BN, KT) ? 2 : 1)) void gemm_dtl_kernel(GemmArgs g) {
     constexpr int WAVES_MN = (BM / WM) * (BN / WN);
     constexpr int WAVES = WAVES_MN * KW;
     constexpr int FM = WM / 32, FN = WN / 32, KS = KT / 16 / KW;   // KS: sub-steps of a K step per wave
@@ -555,7 +559,8 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64) void gemm_dtl_kern
                     // of an fp32 C on loading it.  Left alone, the compiler merges the multiply-add and the
                     // narrowing into one mixed-precision instruction whose result differs in the last place.
                     if (sizeof(TC) == 2) asm volatile("" : "+v"(o));
-                    c_store<TC>(element(c_tile, blk, v), o);
+                    if (shared_tile(BM, BN, KT)) c_store_past<TC>(element(c_tile, blk, v), o);
+                    else c_store<TC>(element(c_tile, blk, v), o);
                     // the activation is taken of the fp32 value, not of its rounded copy
                     if (GELU) c_store<TC>(element(c2_tile, blk, v), gelu_one(o));
                 }
@@ -972,9 +977,45 @@ int launch_dtl_pair(GemmArgs g, const Problem& p, int kernel, int slot, hipStrea
     return launch_dtl_config<CT, 256, 128, 64, 64, 64, 3>(g, p, 1, st);
 }
 
+// A weight gradient from few tokens -- fp32 C, short K -- spends as long storing its tiles as multiplying, and one
+// workgroup per CU does the two in turn: 256 x 256 tiles take 56 us over a [16384 x 4096] gradient before the first K
+// value counts (48 us per 512 of them).  On tiles of half the size two workgroups share a CU, and the stores of one pass
+// under the products of the other.  One / two workgroups, us, by themselves, operands as a gradient's | A k-contiguous (the
+// sums are the same, and the bits):
+//                    K = 256         512          768          1024         1536
+//   [ 4096,  4096]   22.5 / 18.4    29.0 / 25.3   35.5 / 35.0   41.7 / 39.2    54.5 / 53.6  | 1024: 41.9 / 38.9
+//   [ 8192,  2048]   20.2 / 18.6    26.9 / 25.8   33.6 / 36.6   39.9 / 39.6    52.9 / 53.8  | 1024: 39.7 / 39.2
+//   [12288,  4096]   64.4 / 46.6    75.5 / 65.4   94.2 / 86.2  112.9 / 106.9  151.4 / 150.5 | 1024: 113 / 109
+//   [16384,  4096]   67.0 / 57.6    91.8 / 83.4  116.5 / 114   144.8 / 138    191.9 / 197   | 1024: 143 / 144
+//   [250880, 4096]   790 / 854      1204 / 1306   1818 / 2026   2259 / 2481
+// (the fewer the rounds of tiles, the more an end without products in it counts: a long walk evens out by itself).  In a
+// model's backward pass, its operands just written: [4096 x 4096] from 512 30.6 -> 26.0, [4096 x 16384] 98 -> 93,
+// [12288 x 4096] 73 -> 71, [16384 x 4096] 95 -> 95; there the long side of the tile has to lie along the long side of C
+// (across it the last is 103).  From 1024 on a block's step loses more elsewhere than it gains here (755 -> 760 us of
+// [1024 x 2048] as separate words).  With B k-contiguous, or a C of 16 bits, there is less to hide: [12288 x 4096] from 1024
+// 112 / 123 and 101 / 105.  Three K steps in flight instead of two: [16384 x 4096] from 512 91 -> 98.
+inline bool shared_applies(const GemmArgs& g, const Problem& p, long long batch) {
+    return batch == 1 && p.b_kstr && p.c_dtype == BR_F32 && g.k <= 768 && ceil_div(g.m, 256) * ceil_div(g.n, 256) <= 2048 &&
+           !g.bias && !g.accumulate && !g.c2 && !g.addend && g.splits == 1;
+}
+template <int CT>
+int launch_dtl_shared(GemmArgs g, const Problem& p, hipStream_t st) {
+    const bool tall = g.m >= g.n;
+    g.tiles_m = (int)ceil_div(g.m, tall ? 256 : 128);
+    g.tiles_n = (int)ceil_div(g.n, tall ? 128 : 256);
+    const unsigned grid = (unsigned)(g.tiles_m * g.tiles_n);
+    if (tall && p.a_kstr) gemm_dtl_kernel<CT, 256, 128, 64, 128, 32, 2, true, true, float><<<grid, 256, 0, st>>>(g);
+    else if (tall) gemm_dtl_kernel<CT, 256, 128, 64, 128, 32, 2, false, true, float><<<grid, 256, 0, st>>>(g);
+    else if (p.a_kstr) gemm_dtl_kernel<CT, 128, 256, 64, 128, 32, 2, true, true, float><<<grid, 256, 0, st>>>(g);
+    else gemm_dtl_kernel<CT, 128, 256, 64, 128, 32, 2, false, true, float><<<grid, 256, 0, st>>>(g);
+    BR_HIP_LAUNCH_CHECK();
+    return BR_OK;
+}
+
 // K a multiple of 64 (kTile128Half: of 32), one workgroup per tile and batch entry.
 template <int CT>
 int launch_dtl(const GemmArgs& g, const Problem& p, int kernel, long long batch, hipStream_t st) {
+    if (kernel == kTile256 && shared_applies(g, p, batch)) return launch_dtl_shared<CT>(g, p, st);
     if (kernel == kTile256 && walk_applies(g, batch)) return launch_dtl_walk<CT>(g, p, st);
     if (kernel == kTile256) return launch_dtl_config<CT, 256, 256, 64, 128, 64, 2>(g, p, batch, st);
     if (kernel == kTile256x128Groups) return launch_dtl_config<CT, 256, 128, 64, 128, 64, 3, 2>(g, p, batch, st);
