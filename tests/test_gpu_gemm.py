@@ -609,6 +609,34 @@ def test_gemm_staged_rows_too_far_apart_for_slices(a_wide):
     assert np.array_equal(to_host64(c), a.astype(np.float64) @ b.astype(np.float64).T)
 
 
+@pytest.mark.parametrize("c_dt", [F32, F16, BF16])
+@pytest.mark.parametrize("old", [0, 1])
+@pytest.mark.parametrize("off,gap", [(0, 0), (0, 3), (1, 4)])   # rows of C on 16-byte addresses, each row on another, none
+@pytest.mark.parametrize("slices,m,n,k", [(2, 488, 1024, 5120), (4, 40, 1024, 3072), (8, 40, 512, 3072), (15, 200, 1024, 8200),
+                                          (16, 40, 512, 12288)])
+def test_gemm_sum_of_slices_is_exact_on_integers(slices, m, n, k, off, gap, old, c_dt):
+    """The second launch of a product in slices of K: every number of slices, bias, an old C, and a C it can and cannot
+    write four elements at a time, with nothing beside it written."""
+    print("case slices=%d m=%d n=%d k=%d off=%d gap=%d c=%d" % (slices, m, n, k, off, gap, c_dt), flush=True)
+    assert hip.gemm_kernel(0, 1, m, n, k, staged=True)[1] == slices
+    torch.manual_seed(k)
+    dt = F16 if c_dt == F16 else BF16
+    a, b = whole_numbers((m, k), 2, dt), whole_numbers((n, k), 1, dt)
+    bias, before = whole_numbers((n,), 5, F32), whole_numbers((m, n), 9, c_dt)
+    buf = torch.full((off + m * (n + gap) + 8,), 77.0, device="cuda", dtype=TORCH_T[c_dt])
+    c = buf[off:off + m * (n + gap)].view(m, n + gap)
+    c[:, :n] = before
+    need = hip.load().br_hip_gemm_staged_workspace(0, 1, m, n, k, dt, dt, 1)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda").fill_(255)
+    call("br_hip_gemm_staged", 0, 1, m, n, k, 0.5, ptr(a), dt, k, 0, ptr(b), dt, k, 0, old, ptr(c), c_dt, n + gap, 0, ptr(bias), 1,
+         hip.GEMM_F16 if dt == F16 else hip.GEMM_BF16, ptr(ws), need, stream())
+    torch.cuda.synchronize()
+    want = 0.5 * (a.float() @ b.float().t()) + bias + (before.float() if old else 0)
+    assert torch.equal(c[:, :n], want.to(c.dtype))
+    c[:, :n] = 77
+    assert bool((buf == 77).all())
+
+
 @pytest.mark.parametrize("c_dt", [F32, F16])
 @pytest.mark.parametrize("kernel,m,n,k", [("256", 4000, 4096, 72), ("256x128 groups", 1000, 4104, 4160), ("128", 500, 4100, 72),
                                           ("flex 32", 40, 40, 72)])
