@@ -1265,17 +1265,14 @@ int hip_qkv_backward(const tensor_t& acc, const tensor_t* lin) {
 // `op.layernorm_backward_add` followed by the `op.linear_backward` whose dy is the LayerNorm's din: the
 // LayerNorm kernel has every row of din in registers, so it also writes the 16-bit image the two products read
 // and the partial column sums that make the bias gradient -- the pass over din that op.linear_backward starts
-// with does not run.  Anything the fused kernel declines runs as the two operators.
-ComputingReturn hip_layernorm_backward_add_linear_backward(
+// with does not run.  Anything the fused kernel declines runs as the two operators.  The GELU's and the next layer's
+// backward of `tail` (null: none) are joined to it where gelu_between takes them, which *tail_done says.
+namespace {
+ComputingReturn layernorm_backward_add_linear_backward(
     const tensor_t& dy, const tensor_t& scale, const tensor_t& bias, const tensor_t& var, const tensor_t& y,
     const tensor_t& dscale, const tensor_t& dbias, const tensor_t& residual, const tensor_t& din, float eps,
     const tensor_t& x, const tensor_t& weight, const tensor_t& lbias, const tensor_t& x_g, const tensor_t& weight_g,
-    const tensor_t& bias_g, const tensor_t* tail) {
-    // what follows the linear layer's backward: a GELU's and that of the layer ahead of it, or nothing
-    auto rest = [&]() {
-        if (!tail) return OP_OK;
-        return hip_gelu_linear_backward(tail[0], tail[1], tail[2], tail[4], tail[5], tail[6], tail[7], tail[8], tail[9]);
-    };
+    const tensor_t& bias_g, const tensor_t* tail, bool* tail_done) {
     bool fast = dev_f32(dy) && dev_f32(scale) && dev_f32(bias) && dev_f32(var) && dev_f32(y) && dev_f32(dscale) &&
                 dev_f32(dbias) && dev_f32(residual) && dev_f32(din) && dy->shape().dim() == 3 && dev(x) &&
                 dev(weight) && dev(x_g) && dev(weight_g) && dev_f32(bias_g) && x->shape().dim() == 3 &&
@@ -1313,18 +1310,32 @@ ComputingReturn hip_layernorm_backward_add_linear_backward(
                     const int rg = gelu_between(Operand{d16, native}, low, tail, rows, compute, &later);
                     if (rg != BR_ERR_TODO) {
                         BR_OP(rg);
+                        *tail_done = true;
                         return OP_OK;
                     }
                 }
                 BR_OP(linear_backward_products(Operand{d16, native}, x, weight, x_g, weight_g, rows, in, cols, compute, nullptr,
                                                &later));
-                return rest();
+                return OP_OK;
             }
         }
     }
     const ComputingReturn r = hip_layernorm_backward_add(dy, scale, bias, var, y, dscale, dbias, residual, din, eps);
     if (r != OP_OK) return r;
     return din->op_linear_backward(din, x, weight, lbias, x_g, weight_g, bias_g);
+}
+}  // namespace
+
+ComputingReturn hip_layernorm_backward_add_linear_backward(
+    const tensor_t& dy, const tensor_t& scale, const tensor_t& bias, const tensor_t& var, const tensor_t& y,
+    const tensor_t& dscale, const tensor_t& dbias, const tensor_t& residual, const tensor_t& din, float eps,
+    const tensor_t& x, const tensor_t& weight, const tensor_t& lbias, const tensor_t& x_g, const tensor_t& weight_g,
+    const tensor_t& bias_g, const tensor_t* tail) {
+    bool tail_done = false;
+    const ComputingReturn r = layernorm_backward_add_linear_backward(dy, scale, bias, var, y, dscale, dbias, residual, din, eps, x,
+                                                                     weight, lbias, x_g, weight_g, bias_g, tail, &tail_done);
+    if (r != OP_OK || !tail || tail_done) return r;
+    return hip_gelu_linear_backward(tail[0], tail[1], tail[2], tail[4], tail[5], tail[6], tail[7], tail[8], tail[9]);
 }
 
 template struct HIPTensor<DataType::Float>;

@@ -603,12 +603,27 @@ def test_fused_backward_of_two_linear_layers_and_the_gelu_between_equals_the_wor
     """4h -> h, GELU and h -> 4h of a block whose 4h activation is kept in the products' type.  The gradients that are
     rounded on the way are small whole numbers, so the order of no sum shows: the same bits as the words one by one, except
     in the last products, whose two kernels are the same on both sides."""
+    compare_linear_gelu_linear(b, t, hidden, 4 * hidden, in_place, mode, with_layernorm)
+
+
+@pytest.mark.parametrize("with_layernorm", [False, True])
+@pytest.mark.parametrize("hidden,mid,mode,odd", [
+    (256, 1024, "f32", False),   # fp32 products
+    (8192, 64, "f16", False), (5120, 64, "bf16", False),   # rows wider than the LayerNorm kernel's sums take
+    (128, 512, "f16", True),     # a gradient vector that starts at no multiple of 16 bytes
+    (132, 528, "f16", False)])   # a width that is no multiple of 8
+def test_fused_backward_of_two_linear_layers_runs_every_word_where_the_joined_form_is_declined(runtime, hidden, mid, mode, odd,
+                                                                                               with_layernorm):
+    compare_linear_gelu_linear(2, 24, hidden, mid, True, mode, with_layernorm, odd)
+
+
+def compare_linear_gelu_linear(b, t, hidden, mid, in_place, mode, with_layernorm, odd=False):
     rng = np.random.default_rng(hidden + t)
-    mid = 4 * hidden
     print("case %d x %d x %d %s in_place=%s layernorm=%s" % (b, t, hidden, mode, in_place, with_layernorm), flush=True)
+    products, mode = mode, "float" if mode == "f32" else mode
     env = host.Env(1)
     try:
-        env.execute("'%s' op.gemm_precision" % mode)
+        env.execute("'%s' op.gemm_precision" % products)
         for n, cols, dt in (("dy", hidden, "float"), ("ln", hidden, "float"), ("res", hidden, "float"), ("din", hidden, "float"),
                             ("act", mid, mode), ("actg", mid, mode), ("u", mid, mode), ("x", hidden, mode), ("xg", hidden, "float")):
             env.execute("%d %d %d 3 'cuda' '%s' op.create '%s' !" % (b, t, cols, dt, n))
@@ -618,6 +633,8 @@ def test_fused_backward_of_two_linear_layers_and_the_gelu_between_equals_the_wor
         for n, size in (("b1", mid), ("b1g", mid), ("b2", hidden), ("b2g", hidden), ("gam", hidden), ("bet", hidden), ("dgam", hidden),
                         ("dbet", hidden), ("var", b * t)):
             env.execute("%d 1 'cuda' 'float' op.create '%s' !" % (size, n))
+        if odd:
+            env.execute("%d 1 'cuda' 'float' op.create 'v' !  'v' @ 1 %d 1 op.view 'dgam' !" % (hidden + 1, hidden))
         whole = lambda *shape: rng.integers(-1, 2, shape).astype(np.float32)
         for n in ("gam", "var"):
             env.execute("'%s' @ 1.0 op.fill" % n)

@@ -119,6 +119,34 @@ def test_model_step_matches_oracle(runtime, mode, layers, batch, tokens, hidden,
         model.close()
 
 
+def test_step_of_a_model_wider_than_the_joined_layernorm_backward(runtime):
+    """Rows of more than 4096 values: the first block's backward pass, which the step's program joins to the last LayerNorm
+    of the second block's, against the same words each by itself.  The joined products sum in other orders, which a 16-bit
+    operand downstream rounds to a neighbour now and then."""
+    from test_gpu_block import GRADIENTS, apart_text
+    hidden, heads, batch, tokens, vocab = 5120, 40, 1, 16, 256
+    rng = np.random.default_rng(31)
+    model = host.BloomModel(2, batch, tokens, hidden, heads, vocab, 1e-5, "f16", "f16")
+    try:
+        model.init(31, 0.02)
+        ids = rng.integers(0, vocab, (batch, tokens)).astype(np.int32)
+        text = " ".join(["2 # layer_backward_flash", "1 # layer_backward_flash"])
+        assert "W:op.layernorm_backward_add_linear_gelu_linear_backward" in model.env.disassemble(text, fused=True)
+        model.step(ids, np.ones((batch, tokens), np.int32))
+        got = {n: model.read(1, n) for n in GRADIENTS}
+        assert all(np.any(g) for g in got.values())
+        # block 1 again from its input, which the step leaves, and the gradient block 2 left in its xa
+        model.env.execute("%g op.grad_lift  1 # layer_forward_flash" % model.grad_lift())
+        for n in GRADIENTS:
+            model.env.execute("1 # '%s' @ op.zero" % n)
+        model.env.execute("1 # " + apart_text("layer_backward_flash") + "  0 #  1 op.grad_lift  op.sync")
+        for n in GRADIENTS:
+            assert_close(got[n], model.read(1, n), 2e-3, n)
+    finally:
+        model.env.execute("1 op.grad_lift")
+        model.close()
+
+
 @pytest.mark.timeout(900)
 def test_full_depth_model_step_against_oracle(runtime):
     """BLOOM-7B1 at its real depth: 30 blocks, hidden 4096, 32 heads, the
