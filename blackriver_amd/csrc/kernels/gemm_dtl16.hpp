@@ -640,11 +640,10 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64, (shared_tile(BM, B
 // from K = 512 99 -> 95 us, [4096 x 4096] 66.2 -> 64.6, h -> 4h forward 241 -> 237.
 // Memory operations complete in issue order on this target, which is what the partial waits rest on: after the 16
 // operand loads of the next tile come the wave's 128 stores, so "at most 63 outstanding" means the loads are in.
-// An fp32 C, 64 MB and more of it, is stored past the caches: a weight gradient [250880 x 4096] from K = 512 1480 -> 1270 us
-// (its 4.1 GB had pushed the operands out), [16384 x 4096] from K = 2048 259 -> 254, none slower.
+// PAST: an fp32 C is stored past the caches (past_caches).
 // Plain products only: 256 x 256 tiles, all of them interior (m, n multiples of 256), one batch, no bias, nothing
 // accumulated, no second output (walk_applies); everything else takes gemm_dtl_kernel.
-template <int CT, bool A_KSTR, bool B_KSTR, typename TC>
+template <int CT, bool A_KSTR, bool B_KSTR, typename TC, bool PAST>
 __global__ __launch_bounds__(512) void gemm_dtl_walk_kernel(GemmArgs g) {
     constexpr int BM = 256, BN = 256, WM = 64, WN = 128, KT = 64, STAGES = 2;
     constexpr int WAVES = (BM / WM) * (BN / WN);
@@ -791,13 +790,25 @@ __global__ __launch_bounds__(512) void gemm_dtl_walk_kernel(GemmArgs g) {
             for (int v = 0; v < 16; v++) {
                 float o = alpha * acc[i][j][v] + 0.f;   // the plain epilogue's expression with its bias of zero
                 if (sizeof(TC) == 2) asm volatile("" : "+v"(o));   // one fp32 value, then one rounding (see gemm_dtl_kernel)
-                c_store_past<TC>(reinterpret_cast<TC*>(c_tile + (i * 32 + (v >> 2) * 8 + (v & 3)) * g.ldc * (long long)sizeof(TC) +
-                                                       j * 32 * sizeof(TC) + lane_bytes), o);
+                TC* const to = reinterpret_cast<TC*>(c_tile + (i * 32 + (v >> 2) * 8 + (v & 3)) * g.ldc * (long long)sizeof(TC) +
+                                                     j * 32 * sizeof(TC) + lane_bytes);
+                if (PAST) c_store_past<TC>(to, o);
+                else c_store<TC>(to, o);
             }
             __builtin_amdgcn_sched_barrier(0);
         }
     }
 }
+
+// Whether every row of an fp32 C starts on a 128-byte line: a wave's store of 32 columns is then one whole line.
+inline bool rows_on_lines(const GemmArgs& g) { return (reinterpret_cast<uintptr_t>(g.c) & 127) == 0 && g.ldc % 32 == 0; }
+
+// Whether the walking form stores an fp32 C past the caches: one that the 256 MB of the last level cannot hold, where it would
+// push the operands out, and that has products between its stores.  Ordinary stores / these, us: [250880 x 4096] from K = 512
+// 1480 / 1270, [32768 x 4096] from 1024 300 / 272, [8192 x 8192] from 1024 144 / 139, [5120 x 16384] from 2048 312 / 303; of a
+// C that fits the cache [2048 x 8192] from 1024, 2048 40.3 / 42.1, 66.3 / 68.2, [4096 x 8192] 76.4 / 77.6, 126.1 / 128.2; from
+// K = 64 [2048 x 8192] 14.6 / 17.5, [4096 x 32768] 111 / 114.
+inline bool past_caches(const GemmArgs& g) { return rows_on_lines(g) && g.m * g.n * 4 >= 256LL << 20 && g.k >= 128; }
 
 // Whether the walking form takes a product the plan has put on 256 x 256 tiles.
 inline bool walk_applies(const GemmArgs& g, long long batch) {
@@ -814,12 +825,14 @@ int launch_dtl_walk(GemmArgs g, const Problem& p, hipStream_t st) {
     using BF16 = __hip_bfloat16;
 #define BR_DTL_WALK_CASE(AK, BK_)                                                        \
     if (p.a_kstr == AK && p.b_kstr == BK_) {                                             \
-        if (p.c_dtype == BR_F32)                                                         \
-            gemm_dtl_walk_kernel<CT, AK, BK_, float><<<256, 512, 0, st>>>(g);            \
+        if (p.c_dtype == BR_F32 && past_caches(g))                                       \
+            gemm_dtl_walk_kernel<CT, AK, BK_, float, true><<<256, 512, 0, st>>>(g);      \
+        else if (p.c_dtype == BR_F32)                                                    \
+            gemm_dtl_walk_kernel<CT, AK, BK_, float, false><<<256, 512, 0, st>>>(g);     \
         else if (CT == BR_GEMM_F16)                                                      \
-            gemm_dtl_walk_kernel<CT, AK, BK_, F16><<<256, 512, 0, st>>>(g);              \
+            gemm_dtl_walk_kernel<CT, AK, BK_, F16, false><<<256, 512, 0, st>>>(g);       \
         else                                                                             \
-            gemm_dtl_walk_kernel<CT, AK, BK_, BF16><<<256, 512, 0, st>>>(g);             \
+            gemm_dtl_walk_kernel<CT, AK, BK_, BF16, false><<<256, 512, 0, st>>>(g);      \
     }
     BR_DTL_WALK_CASE(false, false)
     BR_DTL_WALK_CASE(false, true)

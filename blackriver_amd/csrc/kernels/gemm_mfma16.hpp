@@ -280,7 +280,8 @@ template <>
 __device__ __forceinline__ void c_store<__half>(__half* p, float v) { *p = __float2half_rn(v); }
 template <>
 __device__ __forceinline__ void c_store<__hip_bfloat16>(__hip_bfloat16* p, float v) { *p = __float2bfloat16(v); }
-// The same for a C that no cache can hold until somebody reads it: fp32 lines go past the ones the operands live in.
+// The same for an fp32 C of 37 MB and more (the smallest that 256 x 256 tiles are planned for) that is
+// written once and read much later, in whole 128-byte lines: they go past the ones the operands live in.
 template <typename T>
 __device__ __forceinline__ void c_store_past(T* p, float v) {
     if constexpr (sizeof(T) == 4) __builtin_nontemporal_store(v, p);

@@ -240,6 +240,24 @@ def test_gemm_two_workgroups_to_a_cu_for_a_short_k(ta, dt, m, n, k):
     assert torch.equal(c[:, :n], 0.5 * ((a.t() if ta else a).float() @ b.float())) and c[:, n:].isnan().all()
 
 
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("gap,off", [(32, 0), (4, 0), (0, 4)])
+def test_gemm_workgroups_that_walk_into_a_c_of_any_rows(ta, tb, gap, off):
+    """Rows of C that start on 128-byte lines, that do not, and a C that does not: four tiles a workgroup.  Exact."""
+    m, n, k = 4096, 16384, 832   # 256 MB: stored past the caches in whole lines
+    print("case ta=%d tb=%d gap=%d off=%d" % (ta, tb, gap, off), flush=True)
+    torch.manual_seed(gap)
+    a = torch.randint(-3, 4, (k, m) if ta else (m, k), device="cuda").half()
+    b = torch.randint(-2, 3, (n, k) if tb else (k, n), device="cuda").half()
+    buf = torch.full((m * (n + gap) + off,), float("nan"), device="cuda")
+    c = buf[off:].view(m, n + gap)
+    call("br_hip_gemm", ta, tb, m, n, k, 0.5, ptr(a), F16, m if ta else k, 0, ptr(b), F16, k if tb else n, 0, 0, ptr(c), F32, n + gap, 0,
+         None, 1, hip.GEMM_F16, stream())
+    torch.cuda.synchronize()
+    assert torch.equal(c[:, :n], 0.5 * ((a.t() if ta else a).float() @ (b.t() if tb else b).float()))
+    assert c[:, n:].isnan().all() and buf[:off].isnan().all()
+
+
 @pytest.mark.parametrize("k", [512, 2048])
 def test_gemm_walking_workgroups_at_the_weight_gradient_shape(k):
     """dW[16384, 4096] = dy[k, 16384]^T . x[k, 4096] (1024 tiles, four per
