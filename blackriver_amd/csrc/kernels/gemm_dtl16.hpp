@@ -993,33 +993,43 @@ int launch_dtl_pair(GemmArgs g, const Problem& p, int kernel, int slot, hipStrea
 // A weight gradient from few tokens -- fp32 C, short K -- spends as long storing its tiles as multiplying, and one
 // workgroup per CU does the two in turn: 256 x 256 tiles take 56 us over a [16384 x 4096] gradient before the first K
 // value counts (48 us per 512 of them).  On tiles of half the size two workgroups share a CU, and the stores of one pass
-// under the products of the other.  One / two workgroups, us, by themselves, operands as a gradient's | A k-contiguous (the
-// sums are the same, and the bits):
-//                    K = 256         512          768          1024         1536
-//   [ 4096,  4096]   22.5 / 18.4    29.0 / 25.3   35.5 / 35.0   41.7 / 39.2    54.5 / 53.6  | 1024: 41.9 / 38.9
-//   [ 8192,  2048]   20.2 / 18.6    26.9 / 25.8   33.6 / 36.6   39.9 / 39.6    52.9 / 53.8  | 1024: 39.7 / 39.2
-//   [12288,  4096]   64.4 / 46.6    75.5 / 65.4   94.2 / 86.2  112.9 / 106.9  151.4 / 150.5 | 1024: 113 / 109
-//   [16384,  4096]   67.0 / 57.6    91.8 / 83.4  116.5 / 114   144.8 / 138    191.9 / 197   | 1024: 143 / 144
-//   [250880, 4096]   790 / 854      1204 / 1306   1818 / 2026   2259 / 2481
-// (the fewer the rounds of tiles, the more an end without products in it counts: a long walk evens out by itself).  In a
-// model's backward pass, its operands just written: [4096 x 4096] from 512 30.6 -> 26.0, [4096 x 16384] 98 -> 93,
-// [12288 x 4096] 73 -> 71, [16384 x 4096] 95 -> 95; there the long side of the tile has to lie along the long side of C
-// (across it the last is 103).  From 1024 on a block's step loses more elsewhere than it gains here (755 -> 760 us of
-// [1024 x 2048] as separate words).  With B k-contiguous, or a C of 16 bits, there is less to hide: [12288 x 4096] from 1024
-// 112 / 123 and 101 / 105.  Three K steps in flight instead of two: [16384 x 4096] from 512 91 -> 98.
+// under the products of the other.  128 x 256 tiles, one / two workgroups to a CU, us, operands from memory (the sums are
+// the same, and the bits; A k-contiguous the same within 3 %):
+//                    K = 64          128            256            512            768
+//   [ 2048,  6144]   13.1 / 12.9    14.6 / 14.0    17.2 / 15.5    22.0 / 20.6    27.1 / 26.2
+//   [ 4096,  4096]   16.3 / 14.4    18.3 / 15.8    21.0 / 17.9    27.1 / 24.0    33.8 / 30.8
+//   [ 8192,  2048]   14.9 / 15.0    16.8 / 16.1    19.5 / 18.0    25.8 / 24.2    32.5 / 31.0
+//   [ 2048,  8192]   14.5 / 16.9    16.2 / 17.7    19.2 / 19.2    25.7 / 26.2    32.1 / 32.2
+//   [ 1024, 16384]   14.2 / 18.1    16.1 / 18.9    19.3 / 19.5    26.1 / 26.5    33.7 / 33.8
+//   [ 2560,  6400]   15.1 / 15.6    16.9 / 16.9    20.1 / 19.2    26.6 / 25.2    33.6 / 31.8
+//   [12288,  4096]   43.1 / 36.0    46.0 / 37.9    54.8 / 45.3    75.2 / 65.7    94.6 / 86.1
+//   [ 8192,  8192]   55.0 / 52.3    56.6 / 55.4    63.9 / 62.1    93.3 / 85.2   119.5 / 113
+//   [16384,  4096]   54.9 / 46.4    58.4 / 48.1    68.4 / 55.9    94.6 / 82.6   122.3 / 113
+//   [20480,  5120]   84.9 / 85.6    88.2 / 84.5    98.6 / 88.8   143.8 / 130    187.2 / 177
+//   [250880, 4096]                                 790 / 854     1204 / 1306    1818 / 2026
+// Where one round of 256 x 256 tiles holds all of C nothing follows a tile whose products its stores could pass under, and
+// rows 32 KB apart lose: such products stay there.  So do those of K = 64 within one round or past four, where either
+// way the stores are all there is (2-4 % lost), and any from K = 1024 on (a block's step loses more elsewhere than it gains:
+// 755 -> 760 us of [1024 x 2048] as separate words).
+// 256 x 128 tiles store columns of 256 rows: with rows 32 KB apart [8192 x 8192] 79.6, 100 and 121 us from K = 64, 512 and
+// 768, [4096 x 16384] 76, 104 and 127; elsewhere within 3 % of these, a model's step of 512 tokens 0-2 % slower.
+// Two workgroups' stores go past the caches, which takes whole 128-byte lines: a C of rows that start elsewhere waits for
+// memory at every line ([3000 x 5000] from K = 64, 512, 768 30.7, 40.6, 46.2 us, and 15.7, 26.6, 32.8 on 256 x 256 tiles).
+// With B k-contiguous, or a C of 16 bits, there is less to hide: [12288 x 4096] from 1024 112 / 123 and 101 / 105.  Three K
+// steps in flight instead of two: [16384 x 4096] from 512 91 -> 98.
 inline bool shared_applies(const GemmArgs& g, const Problem& p, long long batch) {
-    return batch == 1 && p.b_kstr && p.c_dtype == BR_F32 && g.k <= 768 && ceil_div(g.m, 256) * ceil_div(g.n, 256) <= 2048 &&
+    const long long tiles = ceil_div(g.m, 256) * ceil_div(g.n, 256);
+    const bool one_round = tiles <= 256;
+    return batch == 1 && p.b_kstr && p.c_dtype == BR_F32 && g.k <= 768 && tiles <= 2048 && rows_on_lines(g) &&
+           (one_round ? g.k >= 128 && g.ldc % 8192 != 0 : g.k >= 128 || tiles <= 1024) &&
            !g.bias && !g.accumulate && !g.c2 && !g.addend && g.splits == 1;
 }
 template <int CT>
 int launch_dtl_shared(GemmArgs g, const Problem& p, hipStream_t st) {
-    const bool tall = g.m >= g.n;
-    g.tiles_m = (int)ceil_div(g.m, tall ? 256 : 128);
-    g.tiles_n = (int)ceil_div(g.n, tall ? 128 : 256);
+    g.tiles_m = (int)ceil_div(g.m, 128);
+    g.tiles_n = (int)ceil_div(g.n, 256);
     const unsigned grid = (unsigned)(g.tiles_m * g.tiles_n);
-    if (tall && p.a_kstr) gemm_dtl_kernel<CT, 256, 128, 64, 128, 32, 2, true, true, float><<<grid, 256, 0, st>>>(g);
-    else if (tall) gemm_dtl_kernel<CT, 256, 128, 64, 128, 32, 2, false, true, float><<<grid, 256, 0, st>>>(g);
-    else if (p.a_kstr) gemm_dtl_kernel<CT, 128, 256, 64, 128, 32, 2, true, true, float><<<grid, 256, 0, st>>>(g);
+    if (p.a_kstr) gemm_dtl_kernel<CT, 128, 256, 64, 128, 32, 2, true, true, float><<<grid, 256, 0, st>>>(g);
     else gemm_dtl_kernel<CT, 128, 256, 64, 128, 32, 2, false, true, float><<<grid, 256, 0, st>>>(g);
     BR_HIP_LAUNCH_CHECK();
     return BR_OK;

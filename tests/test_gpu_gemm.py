@@ -224,17 +224,21 @@ def test_gemm_workgroups_that_walk_the_tiles(ta, tb, m, n, k, c_dt):
 @pytest.mark.parametrize("dt", [F16, BF16])
 @pytest.mark.parametrize("ta", [1, 0])
 @pytest.mark.parametrize("m,n,k", [(4096, 4096, 64), (4000, 4096, 64), (8192, 8200, 128), (8184, 8192, 192), (6144, 2048, 768),
-                                   (16384, 4096, 512), (4096, 16384, 512), (16384, 8192, 64)])
-def test_gemm_two_workgroups_to_a_cu_for_a_short_k(ta, dt, m, n, k):
-    """Plain products with an fp32 C, a row-contiguous B and K up to 768 run on tiles of 128 x 256 or 256 x 128: whole and partial ones,
-    two K steps and many, into a C whose rows lie apart.  Small integers, so exact."""
+                                   (16384, 4096, 512), (4096, 16384, 512), (16384, 8192, 64),
+                                   (4096, 4096, 128), (4000, 8184, 128), (4000, 8184, 64), (2048, 8160, 128), (8192, 2048, 768), (3000, 5000, 192)])
+@pytest.mark.parametrize("gap", [32, 4])
+def test_gemm_two_workgroups_to_a_cu_for_a_short_k(ta, dt, m, n, k, gap):
+    """Plain products with an fp32 C of rows on 128-byte lines, a row-contiguous B and K up to 768 run on tiles of 128 x 256,
+    two workgroups to a CU: whole and partial ones, four K steps and many, into a C whose rows lie apart.  Rows off such lines,
+    or all of C in one round of 256 x 256 tiles and a pitch of 32 KB or K = 64: on 256 x 256 tiles.  Small integers, so exact."""
+    gap += -n % 32
     assert hip.gemm_kernel(ta, 0, m, n, k, staged=True)[0] == "256"
     print("case ta=%d m=%d n=%d k=%d dt=%d" % (ta, m, n, k, dt), flush=True)
     torch.manual_seed(m + k)
     a = torch.randint(-3, 4, (k, m) if ta else (m, k), device="cuda").to(TORCH_T[dt])
     b = torch.randint(-2, 3, (k, n), device="cuda").to(TORCH_T[dt])
-    c = torch.full((m, n + 4), float("nan"), device="cuda")
-    call("br_hip_gemm", ta, 0, m, n, k, 0.5, ptr(a), dt, m if ta else k, 0, ptr(b), dt, n, 0, 0, ptr(c), F32, n + 4, 0, None, 1,
+    c = torch.full((m, n + gap), float("nan"), device="cuda")
+    call("br_hip_gemm", ta, 0, m, n, k, 0.5, ptr(a), dt, m if ta else k, 0, ptr(b), dt, n, 0, 0, ptr(c), F32, n + gap, 0, None, 1,
          hip.GEMM_F16 if dt == F16 else hip.GEMM_BF16, stream())
     torch.cuda.synchronize()
     assert torch.equal(c[:, :n], 0.5 * ((a.t() if ta else a).float() @ b.float())) and c[:, n:].isnan().all()
