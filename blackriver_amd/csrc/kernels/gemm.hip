@@ -456,13 +456,13 @@ struct StageJob {
     gemm16::u32x4* dst;
     long long ld, stride, total;   // total: 16-byte granules written
     unsigned rows, cols, granules; // granules: of a row
-    unsigned first;                // the first workgroup of this operand
     bool f32, flat;                // flat: rows follow each other without gaps, fp32 and aligned
 };
 constexpr int kStageJobs = 4;
 struct StageJobs {
-    StageJob job[kStageJobs];
+    unsigned first[kStageJobs];   // the first workgroup of each operand
     int count;
+    StageJob job[kStageJobs];
 };
 
 __device__ __forceinline__ gemm16::u32x4 pack16(const float (&v)[8], bool bf) {
@@ -484,23 +484,19 @@ __device__ __forceinline__ gemm16::u32x4 pack16(const float (&v)[8], bool bf) {
 // dO, P, V 5.3 + 11.2 + 6.2 / 13.5, dS, K, Q 10.5 + 5.2 + 5.4 / 12.
 template <bool BF>
 __global__ __launch_bounds__(256) void stage_kernel(StageJobs jobs) {
+    // every line of the arguments is on its way before the first is looked at
+    asm volatile("" ::"s"(jobs.count), "s"(jobs.job[0].src), "s"(jobs.job[1].src), "s"(jobs.job[2].src), "s"(jobs.job[3].src));
     int which = 0;
 #pragma unroll
     for (int i = 1; i < kStageJobs; i++)
-        if (i < jobs.count && blockIdx.x >= jobs.job[i].first) which = i;
+        if (i < jobs.count && blockIdx.x >= jobs.first[i]) which = i;
     which = __builtin_amdgcn_readfirstlane(which);
-    // picked field by field: the arguments stay where they are
-    auto pick = [&](auto field) {
-        auto v = field(jobs.job[0]);
-#pragma unroll
-        for (int i = 1; i < kStageJobs; i++) v = which == i ? field(jobs.job[i]) : v;
-        return v;
-    };
-    const void* const src = pick([](const StageJob& j) { return j.src; });
-    gemm16::u32x4* const dst = pick([](const StageJob& j) { return j.dst; });
-    const long long total = pick([](const StageJob& j) { return j.total; });
-    const unsigned first = pick([](const StageJob& j) { return j.first; });
-    const bool f32 = pick([](const StageJob& j) { return j.f32; }), flat = pick([](const StageJob& j) { return j.flat; });
+    const StageJob& job = jobs.job[which];
+    const void* const src = job.src;
+    gemm16::u32x4* const dst = job.dst;
+    const long long total = job.total;
+    const unsigned first = jobs.first[which];
+    const bool f32 = job.f32, flat = job.flat;
     const long long i = (long long)(blockIdx.x - first) * 256 + threadIdx.x;
     if (i >= total) return;
     if (flat) {
@@ -509,9 +505,8 @@ __global__ __launch_bounds__(256) void stage_kernel(StageJobs jobs) {
         dst[i] = pack16(v, BF);
         return;
     }
-    const unsigned rows = pick([](const StageJob& j) { return j.rows; }), cols = pick([](const StageJob& j) { return j.cols; });
-    const unsigned granules = pick([](const StageJob& j) { return j.granules; });
-    const long long ld = pick([](const StageJob& j) { return j.ld; }), stride = pick([](const StageJob& j) { return j.stride; });
+    const unsigned rows = job.rows, cols = job.cols, granules = job.granules;
+    const long long ld = job.ld, stride = job.stride;
     const unsigned c = (unsigned)(i % granules) * 8;
     const long long row = i / granules;
     const long long at = row / rows * stride + row % rows * ld + c;
@@ -575,8 +570,9 @@ struct Stager {
             const int rc = run();
             if (rc != BR_OK) return rc;
         }
+        jobs.first[jobs.count] = (unsigned)blocks;
         jobs.job[jobs.count++] = StageJob{src, static_cast<gemm16::u32x4*>(dst), ld, stride, total, (unsigned)rows, (unsigned)cols,
-                                          (unsigned)granules, (unsigned)blocks, f32, flat};
+                                          (unsigned)granules, f32, flat};
         blocks += need;
         return BR_OK;
     }

@@ -225,6 +225,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64, (shared_tile(BM, B
     const lds_byte* lds = (const lds_byte*)lds_raw;
     const unsigned lds0 = (unsigned)(unsigned long long)lds;
 
+    touch_args(g);
     long long batch;
     int tm, tn;
     tile_coords(g, batch, tm, tn);

@@ -369,6 +369,7 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
 template <int CT, int BM, int BN, int KW, int ST, bool A_KSTR, bool B_KSTR, typename TC, bool GELU = false, bool WORDS = false>
 __global__ __launch_bounds__(KW * 64, CT == BR_GEMM_F32 && !WORDS ? 2 : 1) void gemm_flex_kernel(GemmArgs g) {
     __shared__ __attribute__((aligned(1024))) unsigned char lds[flex_lds_bytes<BM, BN, KW, ST>()];
+    touch_args(g);
     flex_product<CT, BM, BN, KW, ST, A_KSTR, B_KSTR, TC, GELU, WORDS, true>(g, blockIdx.x, gridDim.x, lds);
 }
 

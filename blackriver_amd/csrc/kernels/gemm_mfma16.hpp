@@ -85,6 +85,14 @@ struct GemmArgs {
     int split_slot = 0;   // which set of the library's arrival counters the two slices of a tile meet through (one per stream)
 };
 
+// A word of each 64-byte line of the arguments, read ahead of everything else and all at once.  The compiler reads an argument
+// where it is first needed, and a line that is first needed behind the K loop is fetched there from memory with nothing
+// else to do: 32 x 32 tiles, [45 x 3448] from K = 424 7.37 us without, 7.05 with; 43 such products 1.048 and 1.007 of what they
+// took when the arguments had no bias stride and no second sum.
+__device__ __forceinline__ void touch_args(const GemmArgs& g) {
+    asm volatile("" ::"s"(g.a), "s"(g.ldb), "s"(g.c2), "s"(g.split_slot));
+}
+
 template <int CT>
 struct Cvt;
 template <>
