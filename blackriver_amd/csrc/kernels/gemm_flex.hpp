@@ -301,6 +301,23 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
                 if (kFold) held[kFold ? i : 0][kFold ? j : 0][v] = 0.f;
             }
 
+    // fp32 sums of 64 k-values go to a second set of registers, so that rounding errors grow with the number of such
+    // sums and not with K: against 64 bits, [512 x 1024] from K = 1024 2.9e-7 -> 1.6e-7, from 4096 5.7e-7 -> 1.7e-7.  That is an
+    // addition per 128 clocks of products, made while the next step's fragments come from LDS; the first product of the next
+    // 64 starts from zero by itself.  Without the second set / with it, us: [512 x 4096] from K = 1024 43.3 / 43.6, [1568 x
+    // 3504] from 1752 184 / 188, [342 x 216] from 8560 48.2 / 49.4, [1350 x 208] from 336 7.75 / 8.12 (behind the step's products,
+    // with a move to clear each: 45.7, 193, 51.4, 8.46; block by block between the products: twice the time).  It has
+    // to fit 256 registers, so that two waves share a SIMD (with one a block's step is 11 % slower), which it does not where
+    // values are loaded one by one (WORDS).
+    auto fold = [&]() {
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) held[kFold ? i : 0][kFold ? j : 0][v] += acc[i][j][v];
+    };
+
 #pragma unroll
     for (int s = 0; s < ST; s++)
         if (s < mine) issue(s);
@@ -320,6 +337,8 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
 #pragma unroll
             for (int j = 0; j < FN; j++) fb[ks][j] = TB::fragment(tile + TA::kBytes, TB::frag_offset(j * 32, ks, lane));
         }
+        const bool fresh = kFold && (t & 1) == 0;
+        if (fresh) fold();   // while the fragments are on their way
         // The step is in registers: its buffer takes the loads of step t + ST while the products run.  (In one
         // burst: dealt out between the products they measured 5-15 % slower.)
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -328,37 +347,26 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
         // Operands swapped: a lane then holds four consecutive columns of one row of C.  fp32: product s of a sub-step
         // multiplies slot s of both halves of the wave, two k-values; the blocks take turns, so that no product waits
         // for the one before it.
+        auto multiply = [&](int ks, int s, auto first) {
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+#pragma unroll
+                for (int j = 0; j < FN; j++) {
+                    if constexpr (CT == BR_GEMM_F32)
+                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fb[ks][j][s]), __uint_as_float(fa[ks][i][s]),
+                                                                         decltype(first)::value ? f32x16{} : acc[i][j], 0, 0, 0);
+                    else
+                        acc[i][j] = Cvt<CT>::mfma(fb[ks][j], fa[ks][i], acc[i][j]);
+                }
+        };
+        if (fresh) multiply(0, 0, std::true_type{});
+        else multiply(0, 0, std::false_type{});
 #pragma unroll
         for (int ks = 0; ks < 4; ks++)
 #pragma unroll
-            for (int s = 0; s < (CT == BR_GEMM_F32 ? 4 : 1); s++)
-#pragma unroll
-                for (int i = 0; i < FM; i++)
-#pragma unroll
-                    for (int j = 0; j < FN; j++) {
-                        if constexpr (CT == BR_GEMM_F32)
-                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fb[ks][j][s]), __uint_as_float(fa[ks][i][s]), acc[i][j], 0, 0, 0);
-                        else
-                            acc[i][j] = Cvt<CT>::mfma(fb[ks][j], fa[ks][i], acc[i][j]);
-                    }
-        // fp32 sums of 64 k-values go to a second set of registers, so that rounding errors grow with the number of such
-        // sums and not with K: against 64 bits, [512 x 1024] from K = 1024 2.9e-7 -> 1.6e-7, from 4096 5.7e-7 -> 1.7e-7.  An
-        // addition and a move per 128 clocks of products; it has to fit 256 registers, so that two waves share a SIMD (with
-        // one a block's step is 11 % slower), which it does not where values are loaded one by one (WORDS).
-        if constexpr (kFold) {
-            if ((t & 1) || t + 1 == mine) {
-#pragma unroll
-                for (int i = 0; i < FM; i++)
-#pragma unroll
-                    for (int j = 0; j < FN; j++)
-#pragma unroll
-                        for (int v = 0; v < 16; v++) {
-                            held[i][j][v] += acc[i][j][v];
-                            acc[i][j][v] = 0.f;
-                        }
-            }
-        }
+            for (int s = ks == 0 ? 1 : 0; s < (CT == BR_GEMM_F32 ? 4 : 1); s++) multiply(ks, s, std::false_type{});
     }
+    if constexpr (kFold) fold();
 
     if constexpr (kFold) flex_park<BM, BN>(held, mem, lane);
     else flex_park<BM, BN>(acc, mem, lane);
