@@ -174,6 +174,27 @@ inline int fp32_kernel(long long m, long long n, long long k, long long batch) {
     return best;
 }
 
+// What `batch` fp32 products of one size take in one launch: as fp32_kernel has it, with what a CU holds at a time (2 / 3 / 5
+// workgroups of each tile) put in.  Workgroups beyond a round of those start two or more to a CU, where the last round's
+// others have ended, so that part of a round takes most of a whole one; within a round the smaller tiles overlap.
+inline double fp32_batch_us(long long m, long long n, long long k, long long batch) {
+    const int kernel = fp32_kernel(m, n, k, batch);
+    if (kernel == kTile128) return 0.0;   // its rule compares whole launches
+    const KernelCost& c = kCost[kernel];
+    const bool wide = kernel == kFlex64, mid = kernel == kFlex32x64;
+    const double load = (double)(ceil_div(m, c.bm) * ceil_div(n, c.bn) * batch) / 256.0, held = wide ? 2.0 : mid ? 3.0 : 5.0;
+    const double whole = held * ceil(load / held), part = load + (wide ? 0.9 : mid ? 1.2 : 0.6);
+    const double rounds = load <= held ? ceil(load) : whole < part ? whole : part;
+    return 2.7 + rounds * (load <= 1.0 || wide ? 1.0 : mid ? 0.9 : 0.87) * (double)ceil_div(ceil_div(k, 32), 4) * (wide ? 2.45 : mid ? 1.4 : 0.78);
+}
+// Several fp32 products of one size: whether each gets a launch of its own.  Three linear layers of h features, one launch
+// each / one for all, us: 512 tokens, h = 2048 118 / 142, 1000 tokens, h = 1024 68.5 / 79.5, 1000 tokens, h = 1536 137 / 160;
+// 700 tokens, h = 1024 58.4 / 55.2, 1000 tokens, h = 512 28.2 / 22.2, 400 tokens, h = 2048 116 / 106.  Over 77 sizes (32-1200
+// tokens, h = 256-2048) the rule takes 2546 us, the better of both each time too, one launch always 2673.
+inline bool fp32_apart(long long m, long long n, long long k, long long batch) {
+    return (double)batch * fp32_batch_us(m, n, k, 1) < fp32_batch_us(m, n, k, batch);
+}
+
 // Two products as one launch of small tiles (gemm_pair.hpp): the tile, or -1 where they run one after the other.
 //
 //   us = start + max(longest walk * step, sum over both of workgroups * (steps + merge) * load / 256)

@@ -854,9 +854,9 @@ def test_two_products_keep_their_order_where_one_overwrites_the_others_operand(s
 @pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16, hip.GEMM_F32])
 @pytest.mark.parametrize("rows,out,inn,x_dt,y_dt", [
     (24, 256, 256, F32, F32), (65, 40, 72, None, None), (130, 1000, 136, None, F32), (1000, 1024, 64, F32, F32), (1000, 2048, 256, None, F32),
-    (2100, 1280, 128, F32, None), (33, 30, 20, F32, F32)])
+    (2100, 1280, 128, F32, None), (33, 30, 20, F32, F32), (512, 2048, 2048, None, None)])   # the last in fp32: one by one
 def test_linear_group_is_exact_on_integers(rows, out, inn, x_dt, y_dt, compute):
-    """Three layers of one x as a batch, each with a bias of its own; the kernels of small and of large tiles, sizes that
+    """Three layers of one x as a batch (or, fp32, where that is slower, one after the other), each with a bias of its own; the kernels of small and of large tiles, sizes that
     are no multiple of a granule among them."""
     dt = COMPUTE_T[compute]
     print("case rows=%d out=%d in=%d compute=%d" % (rows, out, inn, compute), flush=True)
