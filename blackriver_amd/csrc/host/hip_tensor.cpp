@@ -416,19 +416,22 @@ ComputingReturn HIPTensor<DT>::op_last_logits(tensor_t self, tensor_t mask_, ten
 }
 
 namespace {
-// What the newest op_loss_backward has its value from: log p(label) of every position in pinned memory (the context's
-// slot 0, there once the stream has been waited for) and which of them count.
+// What the newest op_loss_backward has its value from: which positions count and log p(label) of each, there once the
+// stream has been waited for.  They lie, behind the labels, in the context's pinned slot 0, which copies of a call that
+// left its value for later may still be reading or writing (`waiting`).
 struct LossRecord {
+    const int32_t* keep = nullptr;
     const float* logp = nullptr;
-    int64_t count = 0;
-    std::vector<int32_t> keep;
+    int64_t positions = 0, count = 0;
+    bool waiting = false;
 } g_loss;
 }  // namespace
 
 float hip_finish_loss() {
     double total = 0.0;
+    g_loss.waiting = false;
     if (g_loss.count > 0)
-        for (size_t i = 0; i < g_loss.keep.size(); i++)
+        for (int64_t i = 0; i < g_loss.positions; i++)
             if (g_loss.keep[i]) total += (double)g_loss.logp[i];
     const float ret = g_loss.count > 0 ? (float)(total / (double)g_loss.count) : 0.0f;
     ComputingContext::last_loss = ret;
@@ -466,9 +469,14 @@ TransformerComputing::loss_result_t HIPTensor<DT>::op_loss_backward(tensor_t sel
 
     const int* ids = static_cast<const int*>(ids_->data());
     const int* mask = static_cast<const int*>(mask_->data());
-    std::vector<int32_t> labels(2 * n, -100);
-    int32_t* const keep = labels.data() + n;
+    if (g_loss.waiting) ComputingContext::sync();
+    // pinned: labels and keep go to the device without a wait, and the values come back
+    int32_t* const labels = static_cast<int32_t*>(ComputingContext::pinned(0, (size_t)(3 * n) * sizeof(int32_t)));
+    int32_t* const keep = labels + n;
+    float* const logp = reinterpret_cast<float*>(keep + n);
+    std::fill(labels, labels + n, -100);
     std::fill(keep, keep + n, 0);
+    g_loss = LossRecord{keep, logp, n, 0, true};
     int64_t count = 0;
     for (int64_t b = 0; b < batch; b++) {
         for (int64_t t = 0; t + 1 < tokens; t++) {
@@ -504,9 +512,9 @@ TransformerComputing::loss_result_t HIPTensor<DT>::op_loss_backward(tensor_t sel
     float* d_result = d_logp + n;
     // labels and keep lie next to each other, here and on the device
     if (n <= 2048) {
-        BR_OP(br_hip_upload_words(d_labels, labels.data(), 2 * n, stream()));
+        BR_OP(br_hip_upload_words(d_labels, labels, 2 * n, stream()));
     } else {
-        BR_OP(br_hip_memcpy_h2d(d_labels, labels.data(), 2 * n * sizeof(int32_t), stream()));
+        BR_OP(br_hip_memcpy_h2d(d_labels, labels, 2 * n * sizeof(int32_t), stream()));
     }
 
     // weight gradient target: the tensor itself when it lives on the device,
@@ -584,11 +592,8 @@ TransformerComputing::loss_result_t HIPTensor<DT>::op_loss_backward(tensor_t sel
     if (overwrite && count > 0) BR_OP(br_hip_fill(d_wg, BR_F32, 0.f, vocab * hidden, stream()));
 
     // sum of log p(label) in fp64 on the host, as the reference accumulates it
-    float* logp = static_cast<float*>(ComputingContext::pinned(0, n * sizeof(float)));
     if (count > 0) BR_OP(br_hip_memcpy_d2h(logp, d_logp, n * sizeof(float), stream()));
-    g_loss.logp = logp;
     g_loss.count = count;
-    g_loss.keep.assign(keep, keep + n);
     const bool later = ComputingContext::loss_later && !staging;
     if (!later) ComputingContext::sync();
 

@@ -147,6 +147,32 @@ def test_step_of_a_model_wider_than_the_joined_layernorm_backward(runtime):
         model.close()
 
 
+@pytest.mark.parametrize("batch,tokens", [(4, 512), (4, 520)])   # labels as kernel arguments, and as a copy that is not waited for
+def test_loss_that_is_read_at_the_end_of_the_step_equals_the_words(runtime, batch, tokens):
+    """Two steps of more and of other labels, then the head's word by itself on what the step left: the same loss, and the same
+    gradient of the table in the rows no id of the batch has touched."""
+    hidden, vocab = 2176, 320
+    rng = np.random.default_rng(tokens)
+    model = host.BloomModel(1, batch, tokens, hidden, hidden // 128, vocab, 1e-5, "f16", "f16")
+    try:
+        model.init(5, 0.02)
+        for _ in range(2):
+            ids = rng.integers(0, vocab // 2, (batch, tokens)).astype(np.int32)
+            mask = np.ones((batch, tokens), np.int32)
+            for b in range(batch):
+                mask[b, rng.integers(tokens // 2, tokens):] = 0
+            loss = model.step(ids, mask)
+            got = model.read(0, "lm_head.weight_g")[vocab // 2:]
+            model.env.execute("0 #  %d %d %d 3 'cuda' 'float' op.create 'spare' !  %d %d 2 'cuda' 'float' op.create 'spare_g' !"
+                              % (batch, tokens, hidden, vocab, hidden))
+            model.env.execute("'xb' @ 'ids_' @ 'mask_' @ 'lm_head.weight' @ 'all_logits' @ 'spare' @ 'spare_g' @ op.loss_backward_set "
+                              "bloom.last_loss")
+            assert model.env.pop_number() == loss and np.isfinite(loss)
+            assert np.array_equal(model.read(0, "spare_g")[vocab // 2:], got) and np.any(got)
+    finally:
+        model.close()
+
+
 @pytest.mark.timeout(900)
 def test_full_depth_model_step_against_oracle(runtime):
     """BLOOM-7B1 at its real depth: 30 blocks, hidden 4096, 32 heads, the
