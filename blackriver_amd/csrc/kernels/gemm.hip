@@ -912,9 +912,17 @@ struct PairOperands {
     }
 };
 
-// Both products (and the column sums) as one launch; BR_ERR_TODO where they have to run one after the other.
-int pair_impl(const br_product& first, const br_product& second, const PairOperands& ops, const br_column_sums* sums,
-              const br_partial_sums* later, int compute, hipStream_t st) {
+// Both products (and the sums) as one launch.
+struct PairLaunch {
+    int kernel, w, x;   // w: the product with both operands row-contiguous
+    gemm16::GemmArgs g[2];
+    gemm16::Problem p[2];
+    gemm16::ColumnSums cs;
+    gemm16::PartialSums ps;
+};
+// BR_ERR_TODO where they have to run one after the other.
+int plan_pair(const br_product& first, const br_product& second, const PairOperands& ops, const br_column_sums* sums,
+              const br_partial_sums* later, int compute, PairLaunch& launch) {
     using namespace gemm16;
     const bool fp32 = compute == BR_GEMM_F32;
     const int native = compute == BR_GEMM_F16 ? BR_F16 : fp32 ? BR_F32 : BR_BF16;
@@ -929,7 +937,7 @@ int pair_impl(const br_product& first, const br_product& second, const PairOpera
     if (out[x].dtype != native && out[x].dtype != BR_F32) return BR_ERR_TODO;
     // nothing is written that another part reads or writes (what is copied first is read ahead of all writes)
     if (overlap(out[0], out[1]) || overlap(out[1], ops.now[0]) || overlap(out[1], ops.now[1])) return BR_ERR_TODO;
-    ColumnSums cs;
+    ColumnSums& cs = launch.cs;
     if (sums) {
         const Stored sx{sums->x, sums->dtype, sums->rows, sums->cols, sums->cols, 0, 1, false};
         const Stored so{sums->out, BR_F32, 1, sums->cols, sums->cols, 0, 1, false};
@@ -947,7 +955,7 @@ int pair_impl(const br_product& first, const br_product& second, const PairOpera
         cs.cols = (int)sums->cols;
         cs.scale = sums->scale;
     }
-    PartialSums ps;
+    PartialSums& ps = launch.ps;
     if (later && later->partials) {
         if (later->arrays < 1 || later->arrays > 3 || later->parts <= 0 || later->parts > 0x3fffffffLL || later->cols <= 0 ||
             later->cols % 4 != 0 || later->cols > 0x3fffffffLL || !aligned16(later->partials))
@@ -956,9 +964,18 @@ int pair_impl(const br_product& first, const br_product& second, const PairOpera
         for (int i = 0; i < later->arrays; i++) {
             if (!later->out[i] || !aligned16(later->out[i])) return BR_ERR_TODO;
             const Stored so{later->out[i], BR_F32, 1, later->cols, later->cols, 0, 1, false};
-            if (sums && overlap(so, Stored{sums->out, BR_F32, 1, sums->cols, sums->cols, 0, 1, false})) return BR_ERR_TODO;
-            for (const Stored& s : ops.now)
-                if (overlap(so, s)) return BR_ERR_TODO;
+            if (overlap(so, sp)) return BR_ERR_TODO;
+            for (int j = 0; j < i; j++)
+                if (overlap(so, Stored{later->out[j], BR_F32, 1, later->cols, later->cols, 0, 1, false})) return BR_ERR_TODO;
+            // the column sums come behind these, and read what they have written
+            if (sums) {
+                const Stored sx{sums->x, sums->dtype, sums->rows, sums->cols, sums->cols, 0, 1, false};
+                const Stored ss{sums->out, BR_F32, 1, sums->cols, sums->cols, 0, 1, false};
+                if (overlap(so, ss) || overlap(so, sx) || overlap(ss, sp)) return BR_ERR_TODO;
+            }
+            // so do the products, also what they read by way of a copy made ahead of everything
+            for (int j = 0; j < 4; j++)
+                if (overlap(so, ops.now[j]) || overlap(so, ops.before[j])) return BR_ERR_TODO;
             for (const Stored& s : out)
                 if (overlap(so, s) || overlap(sp, s)) return BR_ERR_TODO;
             ps.out[i] = reinterpret_cast<flex_f32x4*>(later->out[i]);
@@ -969,8 +986,8 @@ int pair_impl(const br_product& first, const br_product& second, const PairOpera
         ps.cols4 = (int)(later->cols / 4);
         ps.scale = later->scale;
     }
-    GemmArgs g[2];
-    Problem p[2];
+    GemmArgs(&g)[2] = launch.g;
+    Problem(&p)[2] = launch.p;
     for (int i = 0; i < 2; i++) {
         const Stored &a = ops.now[2 * i], &b = ops.now[2 * i + 1];
         const br_product& d = *products[i];
@@ -1004,10 +1021,22 @@ int pair_impl(const br_product& first, const br_product& second, const PairOpera
             return BR_ERR_TODO;
         }
     }
-    const int rc = ops.run(compute, st);
-    if (rc != BR_OK) return rc;
-    auto* const launch = fp32 ? gemm_pair_f32 : compute == BR_GEMM_F16 ? gemm_pair_f16 : gemm_pair_bf16;
-    return launch(g[w], p[w], products[w]->batch, g[x], p[x], products[x]->batch, kernel, cs, ps, st);
+    launch.kernel = kernel;
+    launch.w = w;
+    launch.x = x;
+    return BR_OK;
+}
+
+bool pair_types_ok(const br_product& p, int compute) {
+    const int native = compute == BR_GEMM_F16 ? BR_F16 : compute == BR_GEMM_BF16 ? BR_BF16 : BR_F32;
+    return (p.a_dtype == BR_F32 || p.a_dtype == native) && (p.b_dtype == BR_F32 || p.b_dtype == native) &&
+           (p.c_dtype == BR_F32 || p.c_dtype == native);
+}
+// Whether their operands may be copied ahead of both products: there is room, and the first does not write what the
+// second's copies are made of.
+bool copies_ahead(const br_product& first, const PairOperands& ops, const void* workspace, size_t workspace_bytes) {
+    return (ops.bytes == 0 || (workspace && aligned16(workspace) && ops.bytes <= workspace_bytes)) &&
+           !overlap(stored_c(first), ops.before[2]) && !overlap(stored_c(first), ops.before[3]);
 }
 
 }  // namespace
@@ -1032,6 +1061,18 @@ extern "C" int br_hip_gemm_pair_kernel(int64_t m1, int64_t n1, int64_t k1, int64
     return gemm16::pair_kernel({m1, n1, k1, batch1}, {m2, n2, k2, batch2}, compute == BR_GEMM_F32);
 }
 
+extern "C" int br_hip_gemm_pair_joined(const br_product* first, const br_product* second, const br_column_sums* sums,
+                                       const br_partial_sums* later, int compute, const void* workspace, size_t workspace_bytes) {
+    if (!first || !second) return BR_ERR_INPUT;
+    if (compute != BR_GEMM_F16 && compute != BR_GEMM_BF16 && compute != BR_GEMM_F32) return BR_ERR_ATTR;
+    if (!sizes_ok(*first) || !sizes_ok(*second) || !pair_types_ok(*first, compute) || !pair_types_ok(*second, compute)) return -1;
+    const PairOperands ops(*first, *second, compute, static_cast<char*>(const_cast<void*>(workspace)));
+    PairLaunch launch;
+    if (!copies_ahead(*first, ops, workspace, workspace_bytes) || plan_pair(*first, *second, ops, sums, later, compute, launch) != BR_OK)
+        return -1;
+    return launch.kernel;
+}
+
 extern "C" int br_hip_gemm_pair(const br_product* first, const br_product* second, const br_column_sums* sums,
                                 const br_partial_sums* later, int compute, void* workspace, size_t workspace_bytes,
                                 br_stream_t stream) {
@@ -1044,19 +1085,18 @@ extern "C" int br_hip_gemm_pair(const br_product* first, const br_product* secon
         return br_hip_colsum(sums->x, sums->dtype, sums->out, sums->rows, sums->cols, sums->scale, sums->workspace,
                              sums->workspace_bytes, stream);
     };
-    const int native = compute == BR_GEMM_F16 ? BR_F16 : compute == BR_GEMM_BF16 ? BR_BF16 : BR_F32;
-    auto types_ok = [&](const br_product& p) {
-        return (p.a_dtype == BR_F32 || p.a_dtype == native) && (p.b_dtype == BR_F32 || p.b_dtype == native) &&
-               (p.c_dtype == BR_F32 || p.c_dtype == native);
-    };
-    if (sizes_ok(*first) && sizes_ok(*second) && types_ok(*first) && types_ok(*second)) {
+    if (sizes_ok(*first) && sizes_ok(*second) && pair_types_ok(*first, compute) && pair_types_ok(*second, compute)) {
         char* ws = static_cast<char*>(workspace);
         const PairOperands ops(*first, *second, compute, ws);
-        const bool room = ops.bytes == 0 || (ws && aligned16(ws) && ops.bytes <= workspace_bytes);
-        // copies are made ahead of both products: the first must not write what the second's are made of
-        const bool apart = !overlap(stored_c(*first), ops.before[2]) && !overlap(stored_c(*first), ops.before[3]);
-        if (room && apart) {
-            const int rc = pair_impl(*first, *second, ops, sums, later, compute, st);
+        if (copies_ahead(*first, ops, workspace, workspace_bytes)) {
+            PairLaunch l;
+            int rc = plan_pair(*first, *second, ops, sums, later, compute, l);
+            if (rc == BR_OK) rc = ops.run(compute, st);
+            if (rc == BR_OK) {
+                auto* const launch = compute == BR_GEMM_F32 ? gemm_pair_f32 : compute == BR_GEMM_F16 ? gemm_pair_f16 : gemm_pair_bf16;
+                const br_product* const products[2] = {first, second};
+                rc = launch(l.g[l.w], l.p[l.w], products[l.w]->batch, l.g[l.x], l.p[l.x], products[l.x]->batch, l.kernel, l.cs, l.ps, st);
+            }
             if (rc != BR_ERR_TODO) return rc;
             if (ops.bytes > 0 && workspace_bytes >= ops.bytes) {
                 // one after the other, on copies made in one launch

@@ -114,6 +114,7 @@ SIGNATURES = {
                                   _int, _vp, _int, _i64, _i64, _vp, _i64, _int, _vp, ctypes.c_size_t, _vp]),
     "br_hip_gemm_pair_workspace": (ctypes.c_size_t, [_vp, _vp, _int]),
     "br_hip_gemm_pair": (_int, [_vp, _vp, _vp, _vp, _int, _vp, ctypes.c_size_t, _vp]),
+    "br_hip_gemm_pair_joined": (_int, [_vp, _vp, _vp, _vp, _int, _vp, ctypes.c_size_t]),
     "br_hip_gemm_pair_kernel": (_int, [_i64] * 8 + [_int]),
     "br_hip_gemm_kernel": (_int, [_int, _int, _i64, _i64, _i64, _int, _i64, _int, ctypes.POINTER(_int)]),
     "br_hip_flash_attn_fwd": (_int, [_vp, _vp, _vp, _int, _vp, _vp, _vp, _vp] + [_i64] * 9 + [_vp]),

@@ -404,8 +404,11 @@ int br_hip_gemm_staged(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k
  * C (trans_a = 1, trans_b = 0), the other has trans_a = 0, and none writes what
  * another reads or writes, all of it is ONE launch; results then differ from the
  * separate calls' in the order of the fp32 sums alone.  The same arguments
- * always take the same way.  br_hip_gemm_pair_kernel tells which kernel the one
- * launch runs on (BR_GEMM_FLEX_*), or -1 where there are several; sizes decide. */
+ * always take the same way.  br_hip_gemm_pair_kernel tells which kernel sizes
+ * alone would have the one launch run on (BR_GEMM_FLEX_*), or -1 where they make
+ * several; br_hip_gemm_pair_joined which one br_hip_gemm_pair runs these very
+ * operands on, or -1 (addresses are compared and nothing is read: it needs no
+ * GPU).  The outs of `later` lie apart from each other and from the partials. */
 typedef struct br_product {
     int trans_a, trans_b;
     int64_t m, n, k;
@@ -434,6 +437,8 @@ size_t br_hip_gemm_pair_workspace(const br_product* first, const br_product* sec
 int br_hip_gemm_pair(const br_product* first, const br_product* second, const br_column_sums* sums,
                      const br_partial_sums* later, int compute, void* workspace, size_t workspace_bytes,
                      br_stream_t stream);
+int br_hip_gemm_pair_joined(const br_product* first, const br_product* second, const br_column_sums* sums,
+                            const br_partial_sums* later, int compute, const void* workspace, size_t workspace_bytes);
 int br_hip_gemm_pair_kernel(int64_t m1, int64_t n1, int64_t k1, int64_t batch1, int64_t m2, int64_t n2, int64_t k2,
                             int64_t batch2, int compute);
 

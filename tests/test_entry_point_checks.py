@@ -82,3 +82,47 @@ def test_gemm_plan_reaches_every_kernel(kernel, slices, m, n, k, batch):
 @pytest.mark.parametrize("out", [(1 << 21) - 8, 1 << 21, (1 << 21) + 8, (1 << 26)])
 def test_linear_gelu_takes_wide_outputs(out):
     assert answer("br_hip_linear_gelu(4096, 8192, None, 1 << 40, 1 << 41, 2, 300, %d, 32, None)" % out) > 0
+
+
+MB = 1 << 20
+# addresses, a megabyte and more from each other: output gradient, input, weight, their gradients, sums
+PLACES = {"dy": 16 * MB, "x": 32 * MB, "w": 48 * MB, "dw": 64 * MB, "dx": 80 * MB, "sums.x": 96 * MB, "sums.out": 112 * MB,
+          "partials": 128 * MB, "out0": 144 * MB, "out1": 160 * MB, "ws": 176 * MB}
+
+
+def pair_joined(compute, x_f32=False, **moved):
+    """Kernel of a linear layer's backward products (64 tokens, 256 -> 256) with column sums and two arrays of partial sums
+    beside them, or -1; `moved`: tensors at other addresses."""
+    import ctypes
+    from blackriver_amd import hip
+    at = dict(PLACES, **{k.replace("_", "."): v for k, v in moved.items()})
+    dt = {hip.GEMM_F16: hip.F16, hip.GEMM_BF16: hip.BF16, hip.GEMM_F32: hip.F32}[compute]
+    xt = hip.F32 if x_f32 else dt
+    dw = hip.Product(1, 0, 256, 256, 64, 1.0, at["dy"], dt, 256, 0, at["x"], xt, 256, 0, at["dw"], hip.F32, 256, 0, 1)
+    dx = hip.Product(0, 0, 64, 256, 256, 1.0, at["dy"], dt, 256, 0, at["w"], dt, 256, 0, at["dx"], dt, 256, 0, 1)
+    sums = hip.ColumnSums(at["sums.x"], dt, at["sums.out"], 40, 256, 1.0, None, 0)
+    later = hip.PartialSums(at["partials"], 2, 7, 256, (ctypes.c_void_p * 3)(at["out0"], at["out1"]), 1.0)
+    lib, pair = hip.load(), (ctypes.byref(dw), ctypes.byref(dx))
+    return lib.br_hip_gemm_pair_joined(*pair, ctypes.byref(sums), ctypes.byref(later), compute, at["ws"],
+                                       lib.br_hip_gemm_pair_workspace(*pair, compute))
+
+
+@pytest.mark.parametrize("compute", [0, 1, 2])
+def test_two_products_and_sums_that_do_not_meet_are_one_launch(compute):
+    from blackriver_amd import hip
+    assert {hip.GEMM_F16, hip.GEMM_BF16, hip.GEMM_F32} == {0, 1, 2}
+    assert pair_joined(compute) == hip.load().br_hip_gemm_pair_kernel(256, 256, 64, 1, 64, 256, 256, 1, compute) >= 0
+    assert pair_joined(compute, x_f32=True) >= 0
+    assert pair_joined(compute, sums_x=PLACES["dy"]) >= 0            # a bias gradient: both are read
+    assert pair_joined(compute, x_f32=True, dx=PLACES["x"]) == (-1 if compute == 2 else pair_joined(compute))   # x is copied first
+
+
+@pytest.mark.parametrize("compute", [0, 1, 2])
+@pytest.mark.parametrize("moved,onto", [
+    ("dx", "dw"), ("dx", "dy"), ("dx", "x"), ("dw", "w"), ("dw", "dy"), ("sums_out", "dy"), ("sums_out", "x"), ("sums_out", "dw"),
+    ("dx", "sums.x"), ("sums_out", "partials"), ("sums_out", "out0"), ("out0", "sums.x"), ("out1", "sums.x"), ("out0", "partials"),
+    ("out1", "out0"), ("out0", "x"), ("out0", "dy"), ("out1", "w"), ("out0", "dw"), ("out1", "dx"), ("dw", "partials")])
+def test_two_products_and_sums_that_meet_keep_their_order(moved, onto, compute):
+    assert pair_joined(compute, **{moved: PLACES[onto] + 512}) == -1
+    if onto == "x" and moved != "dx":   # also where x is read by way of a copy
+        assert pair_joined(compute, x_f32=True, **{moved: PLACES[onto] + 512}) == -1

@@ -758,10 +758,12 @@ def run_pair(products, compute, sums=None, later=None):
     first, second = (ctypes.byref(d) for d in descs)
     need = hip.load().br_hip_gemm_pair_workspace(first, second, compute)
     ws = torch.full((max(need, 16),), 0x7f, dtype=torch.uint8, device="cuda")
-    call("br_hip_gemm_pair", first, second, ctypes.byref(sums) if sums else None, ctypes.byref(later) if later else None, compute,
-         ptr(ws), need, stream())
+    args = (first, second, ctypes.byref(sums) if sums else None, ctypes.byref(later) if later else None, compute, ptr(ws), need)
+    call("br_hip_gemm_pair", *args, stream())
     torch.cuda.synchronize()
-    return hip.load().br_hip_gemm_pair_kernel(*sizes, compute) >= 0
+    kernel = hip.load().br_hip_gemm_pair_joined(*args)
+    assert kernel in (-1, hip.load().br_hip_gemm_pair_kernel(*sizes, compute))
+    return kernel >= 0
 
 
 def pair_reference(ta, tb, a, b):
@@ -790,7 +792,7 @@ def test_two_products_of_a_linear_layer_in_one_launch_are_exact_on_integers(n, i
         need = hip.load().br_hip_colsum_workspace(n, out)
         ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
         sums = hip.ColumnSums(ptr(dy), dt, ptr(db), n, out, 0.5, ptr(ws), need)
-        assert run_pair([(1, 0, dy, x, dw), (0, 0, dy, w, dx)], compute, sums) == (n != 700) or compute == hip.GEMM_F32
+        assert run_pair([(1, 0, dy, x, dw), (0, 0, dy, w, dx)], compute, sums) == (n != 700 or compute == hip.GEMM_F32)
         assert torch.equal(dw, pair_reference(1, 0, dy, x).float())
         assert torch.equal(dx, pair_reference(0, 0, dy, w).to(dx.dtype))
         assert torch.equal(db, 0.5 * dy[0].float().sum(0))
@@ -831,10 +833,11 @@ def test_two_products_of_attention_in_one_launch_are_exact_on_integers(bh, t, hd
     p, d_o, v = whole_numbers((bh, t, t), 1, p_dt or dt), whole_numbers((bh, t, hd), 1, dt), whole_numbers((bh, t, hd), 1, p_dt or dt)
     dv, dq = (torch.full((bh, t, hd), float("nan"), device="cuda") for _ in range(2))
     dp = torch.full((bh, t, t), float("nan"), device="cuda")
-    assert run_pair([(1, 0, p, d_o, dv), (0, 1, d_o, v, dp)], compute)
+    joined = compute != hip.GEMM_F32 or t % 4 == 0   # fp32 rows have to start on 16-byte boundaries
+    assert run_pair([(1, 0, p, d_o, dv), (0, 1, d_o, v, dp)], compute) == joined
     assert torch.equal(dv, pair_reference(1, 0, p, d_o).float()) and torch.equal(dp, pair_reference(0, 1, d_o, v).float())
     dv.fill_(float("nan"))
-    assert run_pair([(0, 0, p, v, dq), (1, 0, p, d_o, dv)], compute)
+    assert run_pair([(0, 0, p, v, dq), (1, 0, p, d_o, dv)], compute) == joined
     assert torch.equal(dq, pair_reference(0, 0, p, v).float()) and torch.equal(dv, pair_reference(1, 0, p, d_o).float())
 
 
@@ -847,8 +850,36 @@ def test_two_products_keep_their_order_where_one_overwrites_the_others_operand(s
     x = whole_numbers((1, n, inn), 1, F32 if staged else F16)
     dw = torch.empty((1, out, inn), device="cuda")
     want = pair_reference(1, 0, dy, x).float()
-    assert run_pair([(1, 0, dy, x, dw), (0, 0, dy, w, x)], hip.GEMM_F16)   # one launch by its sizes
+    # a copy of x is out of dx's way, x itself is not
+    assert run_pair([(1, 0, dy, x, dw), (0, 0, dy, w, x)], hip.GEMM_F16) == staged
     assert torch.equal(dw, want) and torch.equal(x, pair_reference(0, 0, dy, w).to(x.dtype))
+
+
+@pytest.mark.parametrize("over", [None, "sums.x", "x"])
+@pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_F32])
+def test_sums_beside_two_products_keep_their_order_where_they_meet(over, compute):
+    """Partial sums, column sums and both products as the one-after-the-other calls leave them: the column sums are of what the
+    partial sums have written, and so are the products, also of an operand that is converted first."""
+    torch.manual_seed(9)
+    dt = COMPUTE_T[compute]
+    n, inn, out, rows, cols, parts = 64, 256, 256, 40, 256, 7
+    print("case over=%s compute=%d" % (over, compute), flush=True)
+    dy, x, w = whole_numbers((1, n, out), 1, dt), whole_numbers((1, n, inn), 1, F32), whole_numbers((1, out, inn), 1, dt)
+    z = whole_numbers((rows, cols), 3, F32)
+    partials = whole_numbers((2, parts, cols), 1, F32)
+    dw, dx = torch.empty((1, out, inn), device="cuda"), torch.empty((1, n, inn), device="cuda")
+    db, apart = torch.full((cols,), float("nan"), device="cuda"), torch.full((2, cols), float("nan"), device="cuda")
+    first = {None: apart[0], "sums.x": z[3], "x": x[0, 5]}[over]
+    outs = (ctypes.c_void_p * 3)(first.data_ptr(), apart[1].data_ptr())
+    later = hip.PartialSums(ptr(partials), 2, parts, cols, outs, 1.0)
+    need = hip.load().br_hip_colsum_workspace(rows, cols)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    sums = hip.ColumnSums(ptr(z), F32, ptr(db), rows, cols, 0.5, ptr(ws), need)
+    # (column sums of another type than the products' are a launch of their own)
+    assert run_pair([(1, 0, dy, x, dw), (0, 0, dy, w, dx)], compute, sums, later) == (over is None and compute == hip.GEMM_F32)
+    added = partials.sum(1)
+    assert torch.equal(first, added[0]) and torch.equal(apart[1], added[1]) and torch.equal(db, 0.5 * z.sum(0))
+    assert torch.equal(dw, pair_reference(1, 0, dy, x).float()) and torch.equal(dx, pair_reference(0, 0, dy, w).float())
 
 
 @pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16, hip.GEMM_F32])
