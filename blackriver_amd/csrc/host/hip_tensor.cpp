@@ -980,7 +980,8 @@ ComputingReturn linear_then_add(const Operand& x, const tensor_t* lin, const ten
     if (fast) {
         const bool first = same_tensor(add[0], y);
         const tensor_t &r = first ? add[1] : add[0], &sum = add[2];
-        fast = first != same_tensor(add[1], y) && same_shape(add[0], add[1]) && r->items() == y->items() && sum->items() == y->items() &&
+        fast = first != same_tensor(add[1], y) && same_shape(add[0], add[1]) && y->shape().dim() <= 4 && r->items() == y->items() &&
+               sum->items() == y->items() &&
                apart(y, r) && apart(y, sum) && (same_tensor(sum, r) || apart(sum, r)) && y->items() % 4 == 0;
         for (int k = 0; fast && k < 3; k++) fast = apart(y, lin[k]) && apart(sum, lin[k]);
         if (fast) {
@@ -1087,10 +1088,12 @@ int gelu_between(const Operand& dy, const tensor_t* low, const tensor_t* tail, i
         !dev(u) || !dev(du) || code(u) != native || code(du) != native || u->items() != x->items() || du->items() != x->items() ||
         !same_tensor(top[0], du) || du->shape().dim() != 3 || x->shape().dim() != 3)
         return BR_ERR_TODO;
-    const int64_t mid = (int64_t)x->shape()[2], out = (int64_t)w->shape()[0], in = (int64_t)(top[1]->items()) / n;
+    const int64_t mid = (int64_t)x->shape()[2], out = (int64_t)w->shape()[0];
     if ((int64_t)w->items() != out * mid || (int64_t)du->shape()[2] != mid || mid % 8 != 0 || !dev(top[1]) || !dev(top[2]) ||
-        !dev(top[4]) || !dev(top[5]) || !dev_f32(top[6]) || top[1]->shape().dim() != 3 || (int64_t)top[1]->items() != n * in ||
-        (int64_t)top[2]->items() != mid * in || (int64_t)top[4]->items() != n * in || (int64_t)top[5]->items() != mid * in ||
+        !dev(top[4]) || !dev(top[5]) || !dev_f32(top[6]) || top[1]->shape().dim() != 3)
+        return BR_ERR_TODO;
+    const int64_t in = (int64_t)top[1]->shape()[2];
+    if ((int64_t)top[1]->items() != n * in || (int64_t)top[2]->items() != mid * in || (int64_t)top[4]->items() != n * in || (int64_t)top[5]->items() != mid * in ||
         (int64_t)top[6]->items() != mid || pick_compute({du, top[1], top[2]}) != compute)
         return BR_ERR_TODO;
     if (!(same_tensor(u, du) || apart(u, du)) || !apart(du, x) || !apart(u, x) || !apart(x, w) || !apart(x, w_g) || !apart(du, w_g) || !apart(u, w_g) ||
@@ -1237,8 +1240,9 @@ int hip_qkv_backward(const tensor_t& acc, const tensor_t* lin) {
     for (int i = 0; i < 3; i++) {
         const tensor_t* l = lin + 7 * i;
         if (!dev_f32(l[0]) || l[0]->shape().dim() != 3 || (int64_t)(l[0]->shape()[0] * l[0]->shape()[1]) != n ||
-            (int64_t)l[0]->shape()[2] != out || !same_tensor(l[1], x) || !dev(l[2]) || !same_tensor(l[4], tmp) || !dev_f32(l[5]) ||
-            !dev_f32(l[6]) || (int64_t)l[2]->items() != out * in || (int64_t)l[5]->items() != out * in || (int64_t)l[6]->items() != out)
+            (int64_t)l[0]->shape()[2] != out || !same_tensor(l[1], x) || l[1]->shape().dim() != 3 ||
+            (int64_t)l[1]->shape()[2] != in || !dev(l[2]) || !same_tensor(l[4], tmp) || !dev_f32(l[5]) || !dev_f32(l[6]) ||
+            (int64_t)l[2]->items() != out * in || (int64_t)l[5]->items() != out * in || (int64_t)l[6]->items() != out)
             return BR_ERR_TODO;
         if (i > 0 && !(adjacent(lin[7 * i - 5], l[2]) && adjacent(lin[7 * i - 2], l[5]) && adjacent(lin[7 * i - 1], l[6])))
             return BR_ERR_TODO;

@@ -581,7 +581,10 @@ BR_WORD(QkvBackwardLayernorm,
             for (int j = 0; j < 7; j++) lin[7 * i + j] = (*layer[i])[j];
         const int rc = hip_qkv_backward(xa, lin);
         one = rc != BR_ERR_TODO;
-        if (one) BR_HIP_CHECK(rc);
+        if (one) {
+            BR_HIP_CHECK(rc);
+            xa->marker() = 0;   // as op_zero leaves it
+        }
     }
     if (!one) {
         xa->op_zero(xa);

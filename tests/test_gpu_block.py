@@ -826,6 +826,29 @@ def test_fused_block_words_against_the_words_one_by_one(runtime, mode, words, hi
         assert_close(out[True][n], out[False][n], tol, n)
 
 
+@pytest.mark.parametrize("word,name,line", [
+    ("plain", "W:op.qkv_backward_layernorm", "'xkey' @ 'odd' @ 'key.weight' @"),
+    ("flash", "W:op.linear_gelu_linear_backward", "'x4a.h' @ 'odd' @ 'dense_h_to_4h.weight' @")])
+def test_joined_backward_words_refuse_an_input_the_words_refuse(runtime, word, name, line):
+    """An input of a linear layer whose rows are half as long as the weight's, twice as many."""
+    b, t, h = 2, 24, 256
+    env, *_ = setup_block(runtime, h, 2, b, t, "f16")
+    env.execute("create_operand_buffers create_flash_buffers prepare_batch_flash")
+    x = "xattn_in" if word == "plain" else "xln2.h"
+    env.execute("'%s' @ 0 %d %d %d 3 op.view 'odd' !" % (x, b, 2 * t, h // 2))
+    forward, backward = ("layer_forward", "layer_backward_core") if word == "plain" else ("layer_forward_flash", "layer_backward_flash")
+    env.execute(forward)
+    text = host.words_text("bloom.words").split("%def " + backward + "\n")[1].split("%end")[0]
+    env.execute(" ".join(l for l in text.splitlines() if not l.strip().startswith(";;")))   # as it is
+    wrong = line.replace("'odd'", "'%s'" % x)
+    assert wrong in text
+    text = " ".join(l for l in text.replace(wrong, line).splitlines() if not l.strip().startswith(";;"))
+    assert name in env.disassemble(text, fused=True)
+    with pytest.raises(host.HostError):
+        env.execute(text)
+    env.close()
+
+
 GRADIENTS = ["input_layernorm.weight_g", "input_layernorm.bias_g", "post_attention_layernorm.weight_g",
              "post_attention_layernorm.bias_g", "query_key_value.weight_g", "query_key_value.bias_g", "dense.weight_g",
              "dense.bias_g", "dense_h_to_4h.weight_g", "dense_h_to_4h.bias_g", "dense_4h_to_h.weight_g", "dense_4h_to_h.bias_g"]
