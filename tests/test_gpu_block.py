@@ -8,6 +8,8 @@ Two modes:
   f16    weights stored as fp16, every product on the fp16 MFMA kernel with
          fp32 accumulation (bound 2e-2, the stated fp16-GEMM tolerance)
 """
+import ctypes
+
 import numpy as np
 import pytest
 import torch
@@ -15,7 +17,7 @@ import torch
 import oracle as orc
 from oracle import bloom_block as blk
 from conftest import assert_close, print_ledger
-from blackriver_amd import host
+from blackriver_amd import hip, host
 
 pytestmark = pytest.mark.gpu
 
@@ -675,6 +677,175 @@ def compare_linear_gelu_linear(b, t, hidden, mid, in_place, mode, with_layernorm
         assert np.abs(want[grad]).max() <= 256 and np.any(want["xg"] != 0)
         for n in outs:
             assert np.array_equal(got[n], want[n]), n
+    finally:
+        env.close()
+
+# ---- joined words one by one: operands they take as one, and operands for which each word has to run by itself
+def joined_operands(word, how):
+    """Tensors (name -> shape, type, base, offset) and lines of a program that the word machine makes one `word` of."""
+    b, t, h = 2, 24, 132 if how == "width of no granules" else 128
+    tensors, own = {}, lambda name, *shape, dt="float": tensors.update({name: (shape, dt, None, 0)})
+    part = lambda name, base, at, *shape: tensors.update({name: (shape, None, base, at)})
+    bth = (b, t, h)
+
+    def three(name, size, *shape, dt="float"):
+        own(name, 3 * size, dt=dt)
+        for i in range(3):
+            part(name + str(i), name, i * size, *shape)
+
+    def vectors(*names):
+        for n in names:
+            own(n, h)
+
+    def layernorm():
+        own("x", *bth), own("xn", *bth), own("mean", b * t), own("var", b * t), vectors("gam", "bet")
+        return "'x' @ 'mean' @ 'var' @ 'gam' @ 'bet' @ 'xn' @ 'eps' @ op.layernorm"
+
+    def linears(x):
+        three("w", h * h, h, h, dt="f16"), three("bias", h, h), three("y", b * t * h, *bth)
+        read, w, y = [x] * 3, ["w0", "w1", "w2"], ["y0", "y1", "y2"]
+        if how == "another input":
+            own("x2", *bth)
+            read[2] = "x2"
+        if how == "a weight elsewhere":
+            own("v", h, h, dt="f16")
+            w[1] = "v"
+        if how == "an output on the input":
+            y[0] = x
+        return ["'%s' @ '%s' @ 'bias%d' @ '%s' @ op.linear" % (read[i], w[i], i, y[i]) for i in range(3)]
+
+    def linear_add(x):
+        own("w", h, h, dt="f16"), vectors("bias"), own("y", *bth), own("r", *bth), own("s", *bth)
+        a, c = {"onto the residual": ("r", "r"), "onto the output": ("r", "y"), "twice itself": ("y", "s"),
+                "another input, onto the output": ("r", "y")}.get(how, ("r", "s"))
+        return ["'%s' @ 'w' @ 'bias' @ 'y' @ op.linear" % x, "'y' @ '%s' @ '%s' @ op.add" % (a, c)]
+
+    if word == "op.linear_x3":
+        own("x", *bth)
+        return tensors, linears("x")
+    if word == "op.layernorm_linear_x3":
+        ln = layernorm()
+        return tensors, [ln] + linears("x" if how == "not of the LayerNorm's output" else "xn")
+    if word == "op.layernorm_linear":
+        ln = layernorm()
+        own("w", h, h, dt="f16"), vectors("bias"), own("y", *bth)
+        return tensors, [ln, "'%s' @ 'w' @ 'bias' @ 'y' @ op.linear" % ("x" if how == "not of the LayerNorm's output" else "xn")]
+    if word == "op.linear_then_add":
+        own("x", *bth)
+        return tensors, linear_add("x")
+    if word == "op.gelu_linear_then_add":
+        own("u", *bth), own("v", *bth)
+        other = how.startswith("another input")
+        if other:
+            own("v2", *bth)
+        return tensors, ["'u' @ 'v' @ op.gelu"] + linear_add("v2" if other else "v")
+    if word == "op.transpos_0213_x3":
+        for n in "abcdef":
+            own(n, b, t, 4, h // 4)
+        if how == "of two shapes":
+            own("e", b, 4, t, h // 4)
+        pairs = ["ab", "bc", "ef"] if how == "one of another's output" else ["ab", "cd", "ef"]
+        return tensors, ["'%s' @ '%s' @ op.transpos_0213" % tuple(p) for p in pairs]
+    # the backward words
+    own("dy", *bth), own("x", *bth), own("out", *bth), own("res", *bth), own("var", b * t)
+    vectors("gam", "bet", "dgam", "dbet")
+    norm = "'%s' @ 'gam' @ 'bet' @ 'var' @ 'x' @ 'dgam' @ 'dbet' @ '%s' @ 'eps' @ op.layernorm_backward"
+    if word == "op.layernorm_backward_then_add_linear_backward":
+        own("w", h, h, dt="f16"), own("in", *bth), own("xg", *bth), own("wg", h, h), vectors("bias", "bg")
+        din = "dy" if how == "in place" else "out"
+        sum_ = "x" if how == "onto the LayerNorm's output" else "res"
+        lin = "dy" if how == "another gradient" else sum_
+        return tensors, [norm % ("dy", din), "'res' @ '%s' @ '%s' @ op.add" % (din, sum_),
+                         "'%s' @ 'in' @ 'w' @ 'bias' @ 'xg' @ 'wg' @ 'bg' @ op.linear_backward" % lin]
+    assert word == "op.qkv_backward_layernorm"
+    three("d", b * t * h, *bth), three("w", h * h, h, h, dt="f16"), three("bias", h, h)
+    three("wg", h * h, h, h), three("bg", h, h), own("xa", *bth)
+    w = ["w0", "w1", "w2"]
+    if how == "a weight elsewhere":
+        own("v", h, h, dt="f16")
+        w[1] = "v"
+    lines = ["'xa' @ op.zero"]
+    for i in range(3):
+        x = "xa" if how == "an input that is written" and i == 2 else "x"
+        lines += ["'d%d' @ '%s' @ '%s' @ 'bias%d' @ 'out' @ 'wg%d' @ 'bg%d' @ op.linear_backward" % (i, x, w[i], i, i, i),
+                  "'xa' @ 'out' @ 'xa' @ op.add"]
+    own("din", *bth)
+    din = "din" if how == "a gradient that is seen" else "out"
+    return tensors, lines + [norm % ("xa", din), "'%s' @ 'res' @ 'xa' @ op.add" % din]
+
+
+def kernels_of(env, text):
+    """Kernels that a program launches: recorded, not run, once the buffers it grows are there."""
+    lib, stream = hip.load(), ctypes.c_void_p(host.stream())
+    program = env.build(text)
+    env.run(program)
+    env.execute("op.sync")
+    graph, count = ctypes.c_void_p(), ctypes.c_size_t()
+    relaxed = 2
+    assert lib.hipStreamBeginCapture(stream, relaxed) == 0
+    try:
+        env.run(program)
+    finally:
+        assert lib.hipStreamEndCapture(stream, ctypes.byref(graph)) == 0
+    assert lib.hipGraphGetNodes(graph, None, ctypes.byref(count)) == 0 and lib.hipGraphDestroy(graph) == 0
+    return count.value
+
+
+@pytest.mark.parametrize("word,how,joined", [
+    ("op.linear_x3", "", True), ("op.linear_x3", "another input", False), ("op.linear_x3", "a weight elsewhere", False),
+    ("op.linear_x3", "an output on the input", False),
+    ("op.layernorm_linear_x3", "", True), ("op.layernorm_linear_x3", "another input", False),
+    ("op.layernorm_linear_x3", "a weight elsewhere", False), ("op.layernorm_linear_x3", "not of the LayerNorm's output", True),
+    ("op.layernorm_linear", "", True), ("op.layernorm_linear", "width of no granules", False),
+    ("op.layernorm_linear", "not of the LayerNorm's output", False),
+    ("op.linear_then_add", "", True), ("op.linear_then_add", "onto the residual", True),
+    ("op.linear_then_add", "onto the output", False), ("op.linear_then_add", "twice itself", False),
+    ("op.gelu_linear_then_add", "", True), ("op.gelu_linear_then_add", "width of no granules", True),
+    ("op.gelu_linear_then_add", "onto the output", True), ("op.gelu_linear_then_add", "another input", True),
+    ("op.gelu_linear_then_add", "another input, onto the output", False),
+    ("op.transpos_0213_x3", "", True), ("op.transpos_0213_x3", "one of another's output", False),
+    ("op.transpos_0213_x3", "of two shapes", False),
+    ("op.layernorm_backward_then_add_linear_backward", "", True),
+    ("op.layernorm_backward_then_add_linear_backward", "another gradient", True),
+    ("op.layernorm_backward_then_add_linear_backward", "width of no granules", True),
+    ("op.layernorm_backward_then_add_linear_backward", "in place", False),
+    ("op.layernorm_backward_then_add_linear_backward", "onto the LayerNorm's output", False),
+    ("op.qkv_backward_layernorm", "", True), ("op.qkv_backward_layernorm", "a weight elsewhere", True),
+    ("op.qkv_backward_layernorm", "an input that is written", True), ("op.qkv_backward_layernorm", "a gradient that is seen", True)])
+def test_joined_word_against_its_words_one_by_one(runtime, word, how, joined):
+    """Every tensor that a program of fp16 products leaves, as one word and with a `1 drop` between its words.  Where nothing is
+    joined they run the same kernels: as many, and the same bits.  Where something is (of several words it may be some), fewer,
+    and fp32 sums in another order."""
+    print("case", word, how, flush=True)
+    tensors, lines = joined_operands(word, how)
+    rng = np.random.default_rng(41)
+    data = {n: rng.integers(-2, 3, shape).astype(np.float32) for n, (shape, _, base, _) in tensors.items() if base is None}
+    for n in data:
+        if n in ("gam", "var"):
+            data[n] = np.abs(data[n]) + 1
+    env = host.Env(1)
+    try:
+        env.execute("'f16' op.gemm_precision  1e-5 'eps' !")
+        for n, (shape, dt, base, at) in tensors.items():
+            sizes = " ".join(str(s) for s in shape) + " %d" % len(shape)
+            env.execute("%s 'cuda' '%s' op.create '%s' !" % (sizes, dt, n) if base is None else
+                        "'%s' @ %d %s op.view '%s' !" % (base, at, sizes, n))
+        texts = {True: "  ".join(lines), False: "  1 drop  ".join(lines)}
+        assert "W:" + word in env.disassemble(texts[True], fused=True)
+        assert "W:" + word not in env.disassemble(texts[False], fused=True)
+        out = {}
+        for one in (True, False):
+            for n in data:
+                env.write(n, data[n])
+            env.execute(texts[one] + "  op.sync")
+            out[one] = {n: env.read(n) for n in data}
+        for n in data:
+            if joined:
+                assert_close(out[True][n], out[False][n], 1e-5, n)
+            else:
+                assert np.array_equal(out[True][n], out[False][n]), n
+        counts = [kernels_of(env, texts[one]) for one in (True, False)]
+        assert counts[0] < counts[1] if joined else counts[0] == counts[1], counts
     finally:
         env.close()
 

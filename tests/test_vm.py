@@ -206,3 +206,22 @@ def test_fusion_pass_folds_a_trailing_copy_into_the_producer(env):
     both = env.disassemble(sm + "  's.h' @ 's' @ op.copy  " + sm + " op.sync 's.h' @ 's' @ op.copy", fused=True)
     assert [x for x in both if x.startswith("W:")] == ["W:op.add_add_softmax_copy", "W:op.add_add_softmax",
                                                        "W:op.sync", "W:op.copy"]
+
+
+@pytest.mark.parametrize("word,joined", [
+    ("layer_forward", "layernorm_linear_x3 transpos_0213_x3 querykey add_add_softmax attn transpos_0213 linear_then_add "
+                      "layernorm_linear gelu_linear_then_add"),
+    ("layer_backward_core", "linear_gelu_linear_backward layernorm_backward_then_add_linear_backward transpos_0213 "
+                            "softmax_attn_backward qk_backward transpos_0213_x3 qkv_backward_layernorm"),
+    ("layer_forward_mixed", "layernorm_copy linear_x3 transpos_0213_x3 querykey add_add_softmax_copy attn transpos_0213 "
+                            "linear_then_add layernorm_copy linear gelu_linear_then_add"),
+    ("layer_backward_mixed", "linear_gelu_linear_backward layernorm_backward_then_add_linear_backward transpos_0213 attn_backward "
+                             "softmax_backward qk_backward transpos_0213_x3 qkv_backward_layernorm"),
+    ("layer_forward_flash", "layernorm_copy linear flash_attn_qkv linear_residual layernorm_copy linear_gelu linear_add"),
+    ("layer_backward_flash", "linear_gelu_linear_backward layernorm_backward_add_linear_backward flash_attn_qkv_backward "
+                             "linear_backward layernorm_backward_add")])
+def test_words_a_block_is_run_as(env, word, joined):
+    """The operators that the block's words come to once the fusion pass has been over them."""
+    env.execute(host.words_text("bloom.words"))
+    fused = env.disassemble(word, fused=True)
+    assert [x for x in fused if x.startswith("W:op.")] == ["W:op." + n for n in joined.split()]
