@@ -246,8 +246,11 @@ inline int pair_kernel(const PairSizes& a, const PairSizes& b, bool fp32) {
             all += groups * (steps + c.merge) * c.load / 256.0;
         }
         const double t = c.start + (all > longest ? all : longest);
-        // (a hurdle for the close ones: [1024 x 4096] from 74 tokens 14.3 in two launches, 14.8 in one)
-        if (t < 0.97 * us && t < best_us) best = kPairKernels[i], best_us = t;
+        // A hurdle for the close ones: [1024 x 4096] from 74 tokens 14.3 in two launches, 14.8 in one.  Not for fp32 on 32-row
+        // tiles, where two launches take 10 % more than these costs say: of 77 pairs priced at 0.97 to 1 of two launches one
+        // takes 0.90 of them, none more than they do (64 tokens, 2048 -> 6144 82 / 60 us; on 64 x 64 tiles 0.91 to 1.09).
+        const double hurdle = fp32 && kPairKernels[i] != kFlex64 ? 1.0 : 0.97;
+        if (t < hurdle * us && t < best_us) best = kPairKernels[i], best_us = t;
     }
     return best;
 }

@@ -79,6 +79,14 @@ def test_gemm_plan_reaches_every_kernel(kernel, slices, m, n, k, batch):
     assert {kernel for kernel, *_ in PLANNED} == set(hip.GEMM_KERNELS)
 
 
+@pytest.mark.parametrize("n,inn,out,name", [(64, 2048, 6144, "flex 32"), (200, 2048, 2048, "flex 32x64"), (250, 2048, 3072, None),
+                                            (65, 2048, 6144, None)])   # on 64 x 64 tiles; many whole 128 x 128 tiles: two launches
+def test_fp32_pairs_that_cost_about_two_launches_by_the_rule(n, inn, out, name):
+    from blackriver_amd import hip
+    kernel = hip.load().br_hip_gemm_pair_kernel(out, inn, n, 1, n, inn, out, 1, hip.GEMM_F32)
+    assert kernel == (-1 if name is None else hip.GEMM_KERNELS.index(name))
+
+
 @pytest.mark.parametrize("out", [(1 << 21) - 8, 1 << 21, (1 << 21) + 8, (1 << 26)])
 def test_linear_gelu_takes_wide_outputs(out):
     assert answer("br_hip_linear_gelu(4096, 8192, None, 1 << 40, 1 << 41, 2, 300, %d, 32, None)" % out) > 0
