@@ -384,7 +384,10 @@ int gemm_impl(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, float a
             }
         }
         const gemm16::Plan plan = planned ? *planned : gemm16::gemm_plan(m, n, k, batch, false);
-        if (gemm16::is_flex(plan.kernel) && c_dtype == BR_F32) sum_beside();
+        // On two waves to a tile a second output costs more than a launch that adds, from some K on: K <= 768 0.84 to 0.97 of two
+        // launches, 1024 0.93 to 1.03, 1536 to 3072 0.99 to 1.03 ([800 x 2560] from 1536 27.6 us in two, 28.4 in one).
+        const bool two_launches = plan.kernel == gemm16::kFlex64Short && k > 1024;
+        if (gemm16::is_flex(plan.kernel) && !two_launches && c_dtype == BR_F32) sum_beside();
         return run_plan(g, p, plan, batch, compute, st);
     }
     // the register-staged kernel; its fast form loads 128 bits at a time and never checks k

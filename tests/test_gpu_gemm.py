@@ -905,7 +905,8 @@ def test_linear_group_is_exact_on_integers(rows, out, inn, x_dt, y_dt, compute):
 
 
 @pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_F32])
-@pytest.mark.parametrize("rows,out,inn", [(24, 256, 256), (65, 44, 72), (78, 1024, 4096), (1000, 1024, 1024), (1000, 2048, 2048), (2048, 4096, 64), (33, 30, 20)])
+@pytest.mark.parametrize("rows,out,inn", [(24, 256, 256), (65, 44, 72), (78, 1024, 4096), (1000, 1024, 1024), (1000, 2048, 2048), (2048, 4096, 64), (33, 30, 20),
+                                          (500, 4096, 384), (800, 2560, 1536)])   # two waves to a tile: with the sum, and followed by it
 @pytest.mark.parametrize("over", [False, True])
 def test_linear_with_the_sum_beside_it_is_exact_on_integers(rows, out, inn, over, compute):
     """y and y + r, the sum over r or apart: small tiles, a ring of K steps, slices of K, and large tiles followed by an
