@@ -872,14 +872,14 @@ inline bool narrow_split_dkv(unsigned workgroups) { return workgroups < (unsigne
 // 105.7, 20 x 2000 160.1 / 140.4; 64 x 600 68.2 / 73.9, 64 x 1024 113 / 130, 32 x 2048 185 / 198).
 inline bool long_walk(unsigned workgroups, int64_t tokens) { return workgroups <= 320 && tokens >= 896; }
 
-// Both passes in one launch (of narrow workgroups, one to a CU): up to three rounds of them.  us as two launches / as one:
+// Both passes in one launch (of narrow workgroups, one to a CU): up to two rounds and a little, and up to three of short
+// sequences.  A third round starts behind the longest walks and, of long sequences, is one itself.  us as two launches / as one:
 // 2 heads x 32 tokens 16.1 / 9.8, 8 x 78 20.6 / 12.9, 32 x 256 26.5 / 17.1 (256 workgroups), 48 x 192 24.1 / 18.5 (288),
-// 32 x 512 37.1 / 32.1 (512), 48 x 334 34.5 / 32.7 (576), 320 x 64 32.4 / 27.1 (640), 96 x 200 37.8 / 34.8 (768), 48 x 550
+// 16 x 1024 55.4 / 46.1 (512), 8 x 2048 93.6 / 74.7 (512), 2 x 8192 321 / 261 (512), 12 x 1536 77.3 / 68.9 (576), 48 x 334
+// 34.5 / 32.7 (576), 320 x 64 32.4 / 27.1 (640), 96 x 250 38.2 / 35.4 (768), 48 x 500 46.5 / 46.5 (768); 24 x 800 50.9 / 51.5
+// (624), 32 x 760 54.3 / 57.2 (768), 24 x 1000 63.4 / 68.9 (768), 12 x 2000 98.3 / 111 (768), 8 x 3000 134 / 140 (752); 48 x 550
 // 51.3 / 56.7 (864), 224 x 128 35.5 / 39.5 (896), 96 x 300 43.9 / 47.8 (960).
-#ifndef BR_FA_BOTH_UP_TO
-#define BR_FA_BOTH_UP_TO 768
-#endif
-inline bool both_at_once(unsigned workgroups) { return workgroups <= (unsigned)BR_FA_BOTH_UP_TO; }
+inline bool both_at_once(unsigned workgroups, int64_t tokens) { return workgroups <= (tokens <= 512 ? 768 : 576); }
 
 bool flash_shape_ok(int64_t batch, int64_t heads, int64_t tokens, int64_t head_dim, int64_t row, int64_t head,
                     int64_t batch_stride, int64_t orow, int64_t obatch) {
@@ -988,7 +988,7 @@ int br_hip_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
     const unsigned tiles2 = (unsigned)(((tokens + 63) / 64) * batch * heads);
     const bool walk = long_walk(tiles, tokens);
     const bool split_q = walk || narrow_split(tiles), split_kv = walk || narrow_split_dkv(tiles);
-    if (both_at_once(2 * tiles2)) {
+    if (both_at_once(2 * tiles2, tokens)) {
         if (dtype == BR_F16) flash_bwd_both_kernel<BR_GEMM_F16><<<2 * tiles2, kThreads, 0, st>>>(a, tiles2);
         else flash_bwd_both_kernel<BR_GEMM_BF16><<<2 * tiles2, kThreads, 0, st>>>(a, tiles2);
         BR_HIP_LAUNCH_CHECK();
