@@ -984,7 +984,6 @@ int br_hip_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
     a.scale = (float)(1.0 / sqrt((double)head_dim));
     hipStream_t st = as_stream(stream);
     const unsigned tiles = (unsigned)(((tokens + kBQ - 1) / kBQ) * batch * heads);
-    // the dQ pass first: it leaves delta behind for the dK / dV pass
     const unsigned tiles2 = (unsigned)(((tokens + 63) / 64) * batch * heads);
     const bool walk = long_walk(tiles, tokens);
     const bool split_q = walk || narrow_split(tiles), split_kv = walk || narrow_split_dkv(tiles);
@@ -994,6 +993,7 @@ int br_hip_flash_attn_bwd(const void* q, const void* k, const void* v, const voi
         BR_HIP_LAUNCH_CHECK();
         return BR_OK;
     }
+    // the dQ pass first: it leaves delta behind for the dK / dV pass
     if (dtype == BR_F16) {
         if (split_q) flash_bwd_dq_kernel<BR_GEMM_F16, 2, 2><<<tiles2, kThreads, 0, st>>>(a);
         else flash_bwd_dq_kernel<BR_GEMM_F16, 4, 1><<<tiles, kThreads, 0, st>>>(a);

@@ -78,7 +78,8 @@ inline double kernel_us(int kernel, long long m, long long n, long long k, long 
     const double memory = 3.0 + ((double)m * k * 2.0 + (double)n * k * 2.0 + (double)m * n * 4.0) * batch / 5.5e6;
     return us > memory ? us : memory + 0.02 * us;   // between two that memory bounds, the one with less to do
 }
-// the pass that adds the partial sums of `slices` slices
+// The pass that adds the partial sums of `slices` slices.  (Fitted before it had all its loads in flight at once: four slices of
+// [1002 x 2048] 8.3 us by this, 10.2 measured then, 8.0 now.)
 inline double reduce_us(long long m, long long n, int slices) { return 3.16 + (double)(slices + 1) * m * n * 4.0 / 8.00e6; }
 
 constexpr int kMaxSplitTiles = 8192;   // the two-slice form's arrival counters per stream
@@ -153,7 +154,8 @@ inline int flex_kernel(long long m, long long n, long long k, long long batch) {
 
 // fp32 products (gemm_flex.hpp): the tile whose matrix instructions finish first.  A step of 32 k-values takes a wave
 // 64 / 32 / 16 instructions of 64 clocks; measured with everything around them 2.45 / 1.4 / 0.78 us per step and
-// workgroup of a CU, and 2.7 us besides.  A CU that holds one workgroup more than the others sets the time.
+// workgroup of a CU, and 2.7 us besides.  A CU that holds one workgroup more than the others sets the time.  (Measured, as
+// kPairCost32 is, before the sums of 64 k-values went to registers of their own, which is 2.3 % more on average.)
 inline int fp32_kernel(long long m, long long n, long long k, long long batch) {
     auto us = [&](int kernel, double per_step) {
         const KernelCost& c = kCost[kernel];

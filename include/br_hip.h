@@ -108,8 +108,12 @@ int br_hip_gelu_fwd(const void* x, void* y, int dtype, int64_t n, br_stream_t st
 /* The same forward with fp32 x and a 16-bit y (BR_F16 or BR_BF16; n % 8 == 0,
  * 16-byte aligned): for an activation that only feeds a 16-bit product, which
  * would round an fp32 y the same way. */
-int br_hip_gelu_fwd_copy16(const float* x, float* y, void* y16, int y16_dtype, int64_t n, br_stream_t stream);
 int br_hip_gelu_fwd_f32_to_16(const float* x, void* y, int y_dtype, int64_t n, br_stream_t stream);
+/* br_hip_gelu_fwd on fp32 and its 16-bit image (y16_dtype BR_F16 or BR_BF16) in
+ * one pass, y16 as br_hip_gelu_fwd_f32_to_16 leaves it: for an activation that
+ * is kept in fp32 and read by a 16-bit product.  y may alias x, y16 neither.
+ * BR_ERR_TODO unless n % 8 == 0 and all three are 16-byte aligned. */
+int br_hip_gelu_fwd_copy16(const float* x, float* y, void* y16, int y16_dtype, int64_t n, br_stream_t stream);
 int br_hip_gelu_bwd(const void* dy, const void* x, void* dx, int dtype, int64_t n,
                     br_stream_t stream);
 
@@ -123,24 +127,25 @@ int br_hip_bias_gelu_fwd(const void* x, const float* bias, void* y, int dtype, i
  * workspace must hold br_hip_bias_gelu_bwd_workspace(rows, cols) bytes when
  * dbias != NULL. */
 size_t br_hip_bias_gelu_bwd_workspace(int64_t rows, int64_t cols);
-/* The same on 16-bit tensors at 16-byte addresses, with dy also copied to
- * dy_copy.  One launch; BR_ERR_TODO where the sizes take two (_copies is 0). */
-int br_hip_bias_gelu_bwd_copies(int64_t rows, int64_t cols);
-int br_hip_bias_gelu_bwd_copy(const void* dy, const void* x, const float* bias, void* dx, float* dbias, void* dy_copy,
-                              int dtype, int64_t rows, int64_t cols, float dbias_scale, br_stream_t stream);
 int br_hip_bias_gelu_bwd(const void* dy, const void* x, const float* bias, void* dx,
                          float* dbias, int dtype, int64_t rows, int64_t cols, float dbias_scale,
                          void* workspace, size_t workspace_bytes, br_stream_t stream);
+/* br_hip_bias_gelu_bwd with dbias on 16-bit tensors at 16-byte addresses, with
+ * dy also copied to dy_copy.  One launch; BR_ERR_TODO where the sizes take two
+ * (_copies is 0). */
+int br_hip_bias_gelu_bwd_copies(int64_t rows, int64_t cols);
+int br_hip_bias_gelu_bwd_copy(const void* dy, const void* x, const float* bias, void* dx, float* dbias, void* dy_copy,
+                              int dtype, int64_t rows, int64_t cols, float dbias_scale, br_stream_t stream);
 
 /* kernels::launch_transform_0213<float>, kernels/transform_kernels.cu:56-65
  * (declared kernels/kernels.h:35), called at cuda_tensor.cpp:257-275: [s0,s1,s2,s3] -> [s0,s2,s1,s3].
  * elem_bytes is 2 or 4. */
-/* `count` of them, one after the other or, where none writes what another
- * reads, in one launch (up to 4 of one shape). */
-int br_hip_transpose_0213_group(const void* const* x, void* const* y, int count, int elem_bytes, int64_t s0,
-                                int64_t s1, int64_t s2, int64_t s3, br_stream_t stream);
 int br_hip_transpose_0213(const void* x, void* y, int elem_bytes, int64_t s0, int64_t s1,
                           int64_t s2, int64_t s3, br_stream_t stream);
+/* `count` of them over tensors of one shape, one after the other or, where none
+ * writes what another reads, in one launch (up to 4). */
+int br_hip_transpose_0213_group(const void* const* x, void* const* y, int count, int elem_bytes, int64_t s0,
+                                int64_t s1, int64_t s2, int64_t s3, br_stream_t stream);
 
 /* cudnnReduceTensor(ADD) of cuda_tensor.cpp:738-760: out[c] = sum_r x[r,c]
  * (x fp32, fp16 or bf16, out fp32), times out_scale (1 for the plain sum; a
@@ -150,13 +155,6 @@ int br_hip_transpose_0213(const void* x, void* y, int elem_bytes, int64_t s0, in
 size_t br_hip_colsum_workspace(int64_t rows, int64_t cols);
 int br_hip_colsum(const void* x, int dtype, float* out, int64_t rows, int64_t cols, float out_scale,
                   void* workspace, size_t workspace_bytes, br_stream_t stream);
-/* `count` (up to 4) fp32 matrices [rows, cols] side by side: packed[r, i * cols + c]
- * = x[i][r, c] in packed_dtype, and out[i * cols + c] = out_scale * sum_r x[i][r, c]:
- * the bias gradients of the query, key and value layers and the operand of
- * their products as one layer of 3 * cols outputs.  BR_ERR_TODO unless
- * cols % 8 == 0 and everything is 16-byte aligned. */
-int br_hip_pack_colsum(const float* const* x, int count, float* out, void* packed, int packed_dtype, int64_t rows,
-                       int64_t cols, float out_scale, br_stream_t stream);
 /* The same column sums of an fp32 x together with a 16-bit copy of x (x16,
  * BR_F16 or BR_BF16, dense [rows, cols]) in one pass: op_linear_backward
  * (cuda_tensor.cpp:730-812) needs the sums as the bias gradient and, with a
@@ -164,6 +162,13 @@ int br_hip_pack_colsum(const float* const* x, int count, float* out, void* packe
  * x 16-byte aligned; workspace as for br_hip_colsum. */
 int br_hip_colsum_cast(const float* x, float* out, void* x16, int x16_dtype, int64_t rows, int64_t cols,
                        float out_scale, void* workspace, size_t workspace_bytes, br_stream_t stream);
+/* `count` (up to 4) fp32 matrices [rows, cols] side by side: packed[r, i * cols + c]
+ * = x[i][r, c] in packed_dtype, and out[i * cols + c] = out_scale * sum_r x[i][r, c]:
+ * the bias gradients of the query, key and value layers and the operand of
+ * their products as one layer of 3 * cols outputs.  BR_ERR_TODO unless
+ * cols % 8 == 0 and everything is 16-byte aligned. */
+int br_hip_pack_colsum(const float* const* x, int count, float* out, void* packed, int packed_dtype, int64_t rows,
+                       int64_t cols, float out_scale, br_stream_t stream);
 
 /* br_hip_gelu_bwd (fp32) and br_hip_colsum_cast in one pass: dx = dy * gelu'(x)
  * is written as fp32 (dx may be x's or dy's own buffer), as a 16-bit copy dx16
@@ -234,6 +239,25 @@ int br_hip_layernorm_bwd_residual(const float* dy, const float* y, const float* 
                                   int64_t cols, float eps, float param_scale, void* workspace,
                                   size_t workspace_bytes, br_stream_t stream);
 
+/* The same followed by what the `op.linear_backward` of the layer below does to
+ * dx first (cuda_tensor.cpp:738-760: its bias gradient, the column sums of dx;
+ * and, for 16-bit products, the 16-bit image of dx both of its products read):
+ * dx16 = dx rounded to dx16_dtype (BR_F16 / BR_BF16), dx_sum[c] = param_scale *
+ * sum over rows of dx[r, c], the sums in a fixed order.  dx16 and dx are what
+ * br_hip_colsum_cast would make of dx; the sums agree with its to rounding (a
+ * different but equally fixed summation order).  Workspace:
+ * br_hip_layernorm_bwd_sums_workspace.  BR_ERR_TODO for rows wider than 4096
+ * columns, unaligned dgamma / dbeta / dx_sum / dx16 and whatever
+ * br_hip_layernorm_bwd_residual declines: callers then run the two steps.
+ * (The words call br_hip_layernorm_bwd_add, which can leave the sums to a later
+ * launch; this one is for callers that want all of it done.) */
+size_t br_hip_layernorm_bwd_sums_workspace(int64_t rows, int64_t cols);
+int br_hip_layernorm_bwd_residual_sums(const float* dy, const float* y, const float* gamma,
+                                       const float* beta, const float* var, const float* residual,
+                                       float* dgamma, float* dbeta, float* dx, void* dx16,
+                                       int dx16_dtype, float* dx_sum, int64_t rows, int64_t cols,
+                                       float eps, float param_scale, void* workspace,
+                                       size_t workspace_bytes, br_stream_t stream);
 /* op_layernorm_backward followed by op_add of a residual into a tensor of its
  * own: dx is what op_layernorm_backward leaves, sum = dx + residual (residual's
  * or dy's own buffer if need be), and, where asked for (both or neither), sum16 and
@@ -258,23 +282,6 @@ int br_hip_layernorm_bwd_add(const float* dy, const float* y, const float* gamma
                              size_t workspace_bytes, br_stream_t stream);
 /* Adds up what is described in *sums (nothing where its partials are null). */
 int br_hip_finish_sums(const br_partial_sums* sums, br_stream_t stream);
-/* The same followed by what the `op.linear_backward` of the layer below does to
- * dx first (cuda_tensor.cpp:738-760: its bias gradient, the column sums of dx;
- * and, for 16-bit products, the 16-bit image of dx both of its products read):
- * dx16 = dx rounded to dx16_dtype (BR_F16 / BR_BF16), dx_sum[c] = param_scale *
- * sum over rows of dx[r, c], the sums in a fixed order.  dx16 and dx are what
- * br_hip_colsum_cast would make of dx; the sums agree with its to rounding (a
- * different but equally fixed summation order).  Workspace:
- * br_hip_layernorm_bwd_sums_workspace.  BR_ERR_TODO for rows wider than 4096
- * columns, unaligned dgamma / dbeta / dx_sum / dx16 and whatever
- * br_hip_layernorm_bwd_residual declines: callers then run the two steps. */
-size_t br_hip_layernorm_bwd_sums_workspace(int64_t rows, int64_t cols);
-int br_hip_layernorm_bwd_residual_sums(const float* dy, const float* y, const float* gamma,
-                                       const float* beta, const float* var, const float* residual,
-                                       float* dgamma, float* dbeta, float* dx, void* dx16,
-                                       int dx16_dtype, float* dx_sum, int64_t rows, int64_t cols,
-                                       float eps, float param_scale, void* workspace,
-                                       size_t workspace_bytes, br_stream_t stream);
 
 /* ---- softmax family ---------------------------------------------------- */
 /* cudnnSoftmaxForward(ACCURATE, INSTANCE) at cuda_tensor.cpp:332-356 and
@@ -543,9 +550,10 @@ int br_hip_flash_attn_fwd(const void* q, const void* k, const void* v, int dtype
  * of the projection's backward would round them) with the element strides of
  * q, k, v.  delta: fp32 scratch of
  * batch * heads * tokens entries (receives rowsum(d_o * o)).  Deterministic: one
- * pass accumulates dq per query block (and forms delta on the way), a second one
- * dk / dv per key block.  dq, dk and dv must not be q, k, v, o or d_o themselves
- * (BR_ERR_OUTPUT): the second pass still reads all five.
+ * pass accumulates dq per query block (and forms delta on the way), another
+ * dk / dv per key block; they run one after the other, or in one launch where
+ * both together are small.  dq, dk and dv must not overlap q, k, v, o or d_o
+ * (BR_ERR_OUTPUT where they are the same): both passes read all five.
  * Same shape limits as the forward (BR_ERR_TODO otherwise). */
 int br_hip_flash_attn_bwd(const void* q, const void* k, const void* v, const void* o, const void* d_o,
                           int dtype, const float* alibi, const int32_t* valid, const float* lse,
