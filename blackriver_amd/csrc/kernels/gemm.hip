@@ -54,12 +54,12 @@ constexpr int kThreads = 256;
 
 // m varies fastest so that neighbouring workgroups share one panel of B
 __device__ __forceinline__ void tile_coords32(const GemmArgs& g, long long& batch, int& tm, int& tn) {
-    const long long per_batch = (long long)g.tiles_m * g.tiles_n;
-    const long long id = blockIdx.x;
-    batch = id / per_batch;
-    const int rem = (int)(id % per_batch);
-    tm = rem % g.tiles_m;
-    tn = rem / g.tiles_m;
+    const unsigned tiles_m = (unsigned)g.tiles_m, per_batch = tiles_m * (unsigned)g.tiles_n, id = blockIdx.x;
+    const unsigned entry = id < per_batch ? 0 : id / per_batch;
+    const unsigned rem = id - entry * per_batch;
+    batch = entry;
+    tn = (int)(rem / tiles_m);
+    tm = (int)(rem - tn * tiles_m);
 }
 
 // ---- fp32 operands on v_mfma_f32_32x32x2_f32 ------------------------------

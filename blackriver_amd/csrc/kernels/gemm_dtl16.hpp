@@ -277,7 +277,7 @@ __global__ __launch_bounds__((BM / WM) * (BN / WN) * KW * 64, (shared_tile(BM, B
     const int nk = SPLIT ? (slice + 1) * nk_all / 2 - k_begin
                    : RAG && g.splits > 1 && k_begin + g.k_slice / KT < nk_all ? g.k_slice / KT : nk_all - k_begin;
     // step `t` of the loop covers K step k_begin + (t + first) mod nk (see k_walk_start)
-    const int first = SPLIT || RAG ? (int)(k_walk_start(row0, col0, g.k) / KT) % nk : (int)(k_walk_start(row0, col0, g.k) / KT);
+    const int start = (int)(k_walk_start(row0, col0, g.k) / KT), first = (SPLIT || RAG) && start >= nk ? start % nk : start;
     a_src += (k_begin + first) * a_step;
     b_src += (k_begin + first) * b_step;
     int until_wrap = nk - first;  // issues left before the walk returns to K step 0

@@ -423,7 +423,7 @@ __global__ __launch_bounds__(512) void gemm_ring_kernel(GemmArgs g) {
     const int steps = (k_end - k_begin + KT - 1) / KT;
     const int padded = steps + (steps & 1);   // the multipliers take steps in pairs
     // step t of the loop covers K step (t + first) mod steps of the slice (see k_walk_start)
-    const int first = (int)(k_walk_start(row0, col0, g.k) / KT) % steps;
+    const int start = (int)(k_walk_start(row0, col0, g.k) / KT), first = start < steps ? start : start % steps;
     const int k0 = k_begin + first * KT;
     const long long a_at = (sliced ? 0 : b * g.sa) + (A_KSTR ? (long long)k0 * g.lda + row0 : (long long)row0 * g.lda + k0);
     const long long b_at = (sliced ? 0 : b * g.sb) + (B_KSTR ? (long long)k0 * g.ldb + col0 : (long long)col0 * g.ldb + k0);

@@ -319,29 +319,37 @@ __device__ __forceinline__ void c_store4<__hip_bfloat16>(__hip_bfloat16* p, cons
 // fastest: the ~32 workgroups an XCD runs at a time cover a GM x GN block and
 // share GM + GN operand strips in its L2 (8 x 4: 12 strips for 32 tiles; a
 // column-first walk down a tall product would touch 33).
-__device__ __forceinline__ void tile_in_order(const GemmArgs& g, int rem, int& tm, int& tn) {
-    const int GM = g.tiles_m < 8 ? g.tiles_m : 8;
-    const int GN = 32 / GM > 4 ? 32 / GM : 4;
-    const int group = rem / (GN * g.tiles_m);
-    const int first_n = group * GN;
-    const int gn = g.tiles_n - first_n < GN ? g.tiles_n - first_n : GN;
-    const int in_group = rem - group * GN * g.tiles_m;
-    const int blk = in_group / (GM * gn);
-    const int within = in_group - blk * GM * gn;
-    const int gm = g.tiles_m - blk * GM < GM ? g.tiles_m - blk * GM : GM;
-    tm = blk * GM + within % gm;
-    tn = first_n + within / gm;
+__device__ __forceinline__ void tile_in_order(const GemmArgs& g, int rem_, int& tm, int& tn) {
+    const unsigned rem = (unsigned)rem_, tiles_m = (unsigned)g.tiles_m, tiles_n = (unsigned)g.tiles_n;
+    const unsigned GM = tiles_m < 8 ? tiles_m : 8;
+    // max(32 / GM, 4): six bits each for GM = 1 .. 8
+    constexpr unsigned long long kWidths = 32ull | 16ull << 6 | 10ull << 12 | 8ull << 18 | 6ull << 24 | 5ull << 30 | 4ull << 36 | 4ull << 42;
+    const unsigned GN = (unsigned)(kWidths >> 6 * (GM - 1)) & 63;
+    const unsigned per_group = GN * tiles_m;
+    const unsigned group = rem < per_group ? 0 : rem / per_group;
+    const unsigned first_n = group * GN;
+    const unsigned gn = tiles_n - first_n < GN ? tiles_n - first_n : GN;
+    const unsigned in_group = rem - group * per_group, per_block = GM * gn;
+    const unsigned blk = per_block == 32 ? in_group >> 5 : in_group / per_block;
+    const unsigned within = in_group - blk * per_block;
+    const unsigned gm = tiles_m - blk * GM < GM ? tiles_m - blk * GM : GM;
+    const unsigned across = gm == 8 ? within >> 3 : within / gm;
+    tm = (int)(blk * GM + within - across * gm);
+    tn = (int)(first_n + across);
 }
 
-// Workgroup `id` of the `nb` a product has -> (batch, tile_m, tile_n).
-__device__ __forceinline__ void tile_coords(const GemmArgs& g, long long id, long long nb, long long& batch, int& tm, int& tn) {
+// Workgroup `id` of the `nb` a product has (fewer than 2^31) -> (batch, tile_m, tile_n).  In 32 bits, and without the divisions
+// that most products can do without: a division of scalars is a chain of twenty dependent instructions, of 64-bit ones a
+// hundred, and a kernel does nothing else meanwhile.  (A 78-token block step of 1024 features 129.7 us with 64-bit ones, 126.7
+// without; two blocks of 512 features and a head over 200 tokens 431.6 and 420.6; the same bits.)
+__device__ __forceinline__ void tile_coords(const GemmArgs& g, unsigned id, unsigned nb, long long& batch, int& tm, int& tn) {
     // ids are dealt to the 8 XCDs round-robin; make each XCD's share contiguous
-    const long long per_xcd = nb / 8;
-    if (per_xcd > 0 && id < per_xcd * 8) id = (id % 8) * per_xcd + id / 8;
-    const long long per_batch = (long long)g.tiles_m * g.tiles_n;
-    batch = id / per_batch;
-    const int rem = (int)(id % per_batch);
-    tile_in_order(g, rem, tm, tn);
+    const unsigned per_xcd = nb / 8;
+    if (id < per_xcd * 8) id = id % 8 * per_xcd + id / 8;
+    const unsigned per_batch = (unsigned)g.tiles_m * (unsigned)g.tiles_n;
+    const unsigned entry = id < per_batch ? 0 : id / per_batch;
+    batch = entry;
+    tile_in_order(g, (int)(id - entry * per_batch), tm, tn);
 }
 __device__ __forceinline__ void tile_coords(const GemmArgs& g, long long& batch, int& tm, int& tn) {
     tile_coords(g, blockIdx.x, gridDim.x, batch, tm, tn);
@@ -359,8 +367,8 @@ __device__ __forceinline__ void tile_coords(const GemmArgs& g, long long& batch,
 __device__ __forceinline__ long long k_walk_start(long long row0, long long col0, long long k) {
     const long long n64 = k >> 6;
     if (n64 < 2) return 0;
-    const long long phase = ((row0 >> 8) & 3) + ((col0 >> 8) & 3);
-    return 64 * (phase % n64);
+    const unsigned phase = ((unsigned)(row0 >> 8) & 3) + ((unsigned)(col0 >> 8) & 3);   // at most 6
+    return 64 * (n64 > 6 ? phase : phase % (unsigned)n64);
 }
 
 // The K loop.  STAGES register sets: the global loads of K steps t+1 ..
