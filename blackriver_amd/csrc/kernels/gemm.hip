@@ -1147,18 +1147,10 @@ extern "C" int br_hip_linear_group(const void* x, int x_dtype, const void* w, in
     if (rows == 0 || count == 0) return BR_OK;
     if (!x || !w) return BR_ERR_INPUT;
     if (!y) return BR_ERR_OUTPUT;
-    const bool apart = compute == BR_GEMM_F32 && count > 1 && gemm16::fp32_apart(rows, out, in, count);
-    const int launches = apart ? count : 1;
-    for (int i = 0; i < launches; i++) {
-        Extra extra;
-        extra.bias_stride = out;
-        const int rc = staged_impl(0, 1, rows, out, in, 1.0f, x, x_dtype, in, 0, static_cast<const char*>(w) + i * out * in * elem_size(w_dtype),
-                                   w_dtype, in, out * in, 0, nullptr, static_cast<char*>(y) + i * rows * out * elem_size(y_dtype), y_dtype,
-                                   out, rows * out, bias ? bias + i * out : nullptr, apart ? 1 : count, compute, workspace, workspace_bytes,
-                                   stream, false, &extra);
-        if (rc != BR_OK) return rc;
-    }
-    return BR_OK;
+    Extra extra;
+    extra.bias_stride = out;
+    return staged_impl(0, 1, rows, out, in, 1.0f, x, x_dtype, in, 0, w, w_dtype, in, out * in, 0, nullptr, y, y_dtype, out, rows * out, bias,
+                       count, compute, workspace, workspace_bytes, stream, false, &extra);
 }
 
 extern "C" int br_hip_linear_sum(const void* x, int x_dtype, const void* w, int w_dtype, const float* bias, const float* r,

@@ -34,12 +34,14 @@
 // for a 64 x 64 tile.  A second buffer per wave, or the loads dealt out between
 // the products, measured equal or 5-15 % slower on the 64 x 64 tile.
 //
-// fp32 products run on the same kernel with v_mfma_f32_32x32x2: 64 clocks for
-// two k-values, so the matrix cores bound anything but the smallest and what
-// counts is that all 1024 SIMDs have an equal share (before / after; before =
-// 128 x 128 tiles of four waves): [512 x 1024] K = 1024 97 -> 14.6 us, K = 4096
-// 345 -> 44, [512 x 4096] K = 1024 97 -> 45 (95 TFLOP/s), [1024 x 8192] K = 2048
-// 327 -> 290 (119 TFLOP/s; clock not yet settled in any of these).
+// fp32 products run on the same kernel, and on the 16-bit matrix instructions: a value is the sum of three bf16 values to 24
+// bits, and six of the nine products of such parts are all that a float holds of the whole.  They take 192 clocks for
+// 16 k-values of a 32 x 32 block, v_mfma_f32_32x32x2 512.  With those / with parts, us (and the error against 64 bits, 2-norm):
+// [512 x 1024] K = 1024 14.9 / 12.4 (1.6e-7 / 1.0e-7), K = 4096 43 / 33 (1.7e-7 / 1.4e-7), [512 x 4096] K = 1024 43.5 / 30.5 (1.6e-7 /
+// 1.0e-7), [1024 x 8192] K = 2048 282 / 198 (1.6e-7 / 1.3e-7), [342 x 216] K = 8560 47 / 38.6 (1.85e-7 / 1.75e-7); a launch of under
+// 6 us takes as long as before.  What bounds it: many tiles, the rate of the 16-bit instructions at the clock they leave (175
+// TFLOP/s are 1050 of theirs); one small tile to a CU, the loads into LDS, 25-30 B per clock whatever the tile and however many are
+// in flight (a second and a third buffer per wave measured equal or slower).
 #pragma once
 #include <type_traits>
 
@@ -215,6 +217,53 @@ __device__ __forceinline__ void flex_emit(const GemmArgs& g, const lds_byte* lds
     }
 }
 
+// The three bf16 parts of eight fp32 values of a lane, each the nearest to what the parts before it leave (those differences
+// are exact).  DOTS: the difference as a product of two pairs with -1 and 0, one instruction where shift or mask and
+// subtraction are two: 27.7 -> 25.1 us for a layer's backward products on 32 x 32 tiles, 2-3 % slower on 64 x 64.
+//
+// A fragment's products with those of the other operand, hi hi, hi mid, mid hi, mid mid, hi lo, lo hi:
+//   kAsParts        all but the first are added up in registers of their own: one rounding of the large sum for 16 k-values.
+//                   Up to 512 k-values a wave (kApartUpTo), from where the error passes that of
+//   kAsPartsFolded  all into one accumulator, which goes to a second one every 64 k-values, so that errors grow with the number
+//                   of such sums and not with K (3-10 % slower)
+//   kOneByOne       the fp32 instructions, folded likewise.  What is not a number or beyond bf16's range in an operand makes the
+//                   parts' sums something else than a number, and an operand below 2^-110, whose parts lose bits, a result below
+//                   2^-100 (unless the other operand is large): a wave that finds either in its sums walks once more, like this.
+enum FlexWalk { kInTheirType, kAsParts, kAsPartsFolded, kOneByOne };
+constexpr int kApartUpTo = 512;
+constexpr int kNotNumbers = 0x207, kSubnormals = 0x090;   // classes of v_cmp_class_f32: NaN and infinity, subnormal
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+typedef float f32x2 __attribute__((ext_vector_type(2)));
+template <bool DOTS>
+__device__ __forceinline__ void three_parts(const u32x4& first, const u32x4& second, u32x4& hi, u32x4& mid, u32x4& lo) {
+    // -1, 0 and 0, -1, in registers: as a constant the first becomes an inline -1.0, which the instruction takes for the second
+    unsigned x = 0x0000bf80u, y = 0xbf800000u;
+    asm("" : "+s"(x), "+s"(y));
+    auto without = [&](f32x2 v, bf16x2 h) {
+        if constexpr (DOTS) {
+            v.x = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(bf16x2, x), v.x, false);
+            v.y = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(bf16x2, y), v.y, false);
+        } else {
+            v.x -= __uint_as_float(__builtin_bit_cast(unsigned, h) << 16);
+            v.y -= __uint_as_float(__builtin_bit_cast(unsigned, h) & 0xffff0000u);
+        }
+        return v;
+    };
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        f32x2 v;
+        v.x = __uint_as_float(e < 2 ? first[2 * e] : second[2 * e - 4]);
+        v.y = __uint_as_float(e < 2 ? first[2 * e + 1] : second[2 * e - 3]);
+        const bf16x2 h = __builtin_convertvector(v, bf16x2);
+        v = without(v, h);
+        const bf16x2 m = __builtin_convertvector(v, bf16x2);
+        v = without(v, m);
+        hi[e] = __builtin_bit_cast(unsigned, h);
+        mid[e] = __builtin_bit_cast(unsigned, m);
+        lo[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+    }
+}
+
 // LDS of a workgroup of such tiles
 template <int BM, int BN, int KW, int ST>
 constexpr int flex_lds_bytes() { return KW * ST * (BM + BN) * 128; }
@@ -289,86 +338,133 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
     };
 
     f32x16 acc[FM][FN];
-    constexpr bool kFold = CT == BR_GEMM_F32 && !WORDS;   // see below
-    f32x16 held[kFold ? FM : 1][kFold ? FN : 1];
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++)
-#pragma unroll
-            for (int v = 0; v < 16; v++) {
-                acc[i][j][v] = 0.f;
-                if (kFold) held[kFold ? i : 0][kFold ? j : 0][v] = 0.f;
-            }
+    f32x16 low[CT == BR_GEMM_F32 ? FM : 1][CT == BR_GEMM_F32 ? FN : 1];   // fp32: what is added to `acc` at the end
 
-    // fp32 sums of 64 k-values go to a second set of registers, so that rounding errors grow with the number of such
-    // sums and not with K: against 64 bits, [512 x 1024] from K = 1024 2.9e-7 -> 1.6e-7, from 4096 5.7e-7 -> 1.7e-7.  That is an
-    // addition per 128 clocks of products, made while the next step's fragments come from LDS; the first product of the next
-    // 64 starts from zero by itself.  Without the second set / with it, us: [512 x 4096] from K = 1024 43.3 / 43.6, [1568 x
-    // 3504] from 1752 184 / 188, [342 x 216] from 8560 48.2 / 49.4, [1350 x 208] from 336 7.75 / 8.12 (behind the step's products,
-    // with a move to clear each: 45.7, 193, 51.4, 8.46; block by block between the products: twice the time).  It has
-    // to fit 256 registers, so that two waves share a SIMD (with one a block's step is 11 % slower), which it does not where
-    // values are loaded one by one (WORDS).
-    auto fold = [&]() {
+    // The wave's steps; `how`: see FlexWalk
+    auto walk = [&](auto how) {
+        constexpr int kHow = decltype(how)::value;
 #pragma unroll
         for (int i = 0; i < FM; i++)
 #pragma unroll
             for (int j = 0; j < FN; j++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) held[kFold ? i : 0][kFold ? j : 0][v] += acc[i][j][v];
-    };
-
-#pragma unroll
-    for (int s = 0; s < ST; s++)
-        if (s < mine) issue(s);
-    int stage = 0;
-    for (int t = 0; t < mine; t++) {
-        // the loads of step t are in once at most those of the steps after it are outstanding
-        const int after = mine - 1 - t;
-        if (ST > 1 && after >= ST - 1) wait_vmem<(ST - 1) * kLoads>();
-        else if (ST > 2 && after == 1) wait_vmem<kLoads>();
-        else wait_vmem<0>();
-        const lds_byte* tile = mem + stage * kStageBytes;
-        u32x4 fa[4][FM], fb[4][FN];
-#pragma unroll
-        for (int ks = 0; ks < 4; ks++) {
-#pragma unroll
-            for (int i = 0; i < FM; i++) fa[ks][i] = TA::fragment(tile, TA::frag_offset(i * 32, ks, lane));
-#pragma unroll
-            for (int j = 0; j < FN; j++) fb[ks][j] = TB::fragment(tile + TA::kBytes, TB::frag_offset(j * 32, ks, lane));
-        }
-        const bool fresh = kFold && (t & 1) == 0;
-        if (fresh) fold();   // while the fragments are on their way
-        // The step is in registers: its buffer takes the loads of step t + ST while the products run.  (In one
-        // burst: dealt out between the products they measured 5-15 % slower.)
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-        if (t + ST < mine) issue(stage);
-        stage = stage + 1 == ST ? 0 : stage + 1;
-        // Operands swapped: a lane then holds four consecutive columns of one row of C.  fp32: product s of a sub-step
-        // multiplies slot s of both halves of the wave, two k-values; the blocks take turns, so that no product waits
-        // for the one before it.
-        auto multiply = [&](int ks, int s, auto first) {
-#pragma unroll
-            for (int i = 0; i < FM; i++)
-#pragma unroll
-                for (int j = 0; j < FN; j++) {
-                    if constexpr (CT == BR_GEMM_F32)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fb[ks][j][s]), __uint_as_float(fa[ks][i][s]),
-                                                                         decltype(first)::value ? f32x16{} : acc[i][j], 0, 0, 0);
-                    else
-                        acc[i][j] = Cvt<CT>::mfma(fb[ks][j], fa[ks][i], acc[i][j]);
+                for (int v = 0; v < 16; v++) {
+                    acc[i][j][v] = 0.f;
+                    if constexpr (CT == BR_GEMM_F32) low[i][j][v] = 0.f;
                 }
+        auto fold = [&]() {
+            if constexpr (CT == BR_GEMM_F32) {
+#pragma unroll
+                for (int i = 0; i < FM; i++)
+#pragma unroll
+                    for (int j = 0; j < FN; j++)
+#pragma unroll
+                        for (int v = 0; v < 16; v++) low[i][j][v] += acc[i][j][v];
+            }
         };
-        if (fresh) multiply(0, 0, std::true_type{});
-        else multiply(0, 0, std::false_type{});
 #pragma unroll
-        for (int ks = 0; ks < 4; ks++)
+        for (int s = 0; s < ST; s++)
+            if (s < mine) issue(s);
+        int stage = 0;
+        for (int t = 0; t < mine; t++) {
+            // the loads of step t are in once at most those of the steps after it are outstanding
+            const int after = mine - 1 - t;
+            if (ST > 1 && after >= ST - 1) wait_vmem<(ST - 1) * kLoads>();
+            else if (ST > 2 && after == 1) wait_vmem<kLoads>();
+            else wait_vmem<0>();
+            const lds_byte* tile = mem + stage * kStageBytes;
+            u32x4 fa[4][FM], fb[4][FN];
 #pragma unroll
-            for (int s = ks == 0 ? 1 : 0; s < (CT == BR_GEMM_F32 ? 4 : 1); s++) multiply(ks, s, std::false_type{});
+            for (int ks = 0; ks < 4; ks++) {
+#pragma unroll
+                for (int i = 0; i < FM; i++) fa[ks][i] = TA::fragment(tile, TA::frag_offset(i * 32, ks, lane));
+#pragma unroll
+                for (int j = 0; j < FN; j++) fb[ks][j] = TB::fragment(tile + TA::kBytes, TB::frag_offset(j * 32, ks, lane));
+            }
+            const bool fresh = (kHow == kOneByOne || kHow == kAsPartsFolded) && (t & 1) == 0;
+            if (fresh) fold();   // sums of 64 k-values go to a second set of registers
+            // The step is in registers: its buffer takes the loads of step t + ST while the products run.  (In one
+            // burst: dealt out between the products they measured 5-15 % slower.)
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            if (t + ST < mine) issue(stage);
+            stage = stage + 1 == ST ? 0 : stage + 1;
+            // Operands swapped: a lane then holds four consecutive columns of one row of C.
+            if constexpr (kHow == kAsParts || kHow == kAsPartsFolded) {
+                constexpr bool kApart = kHow == kAsParts;
+#pragma unroll
+                for (int ks = 0; ks < 4; ks += 2) {
+                    u32x4 pa[3][FM], pb[3][FN];
+#pragma unroll
+                    for (int i = 0; i < FM; i++) three_parts<BM * BN == 1024>(fa[ks][i], fa[ks + 1][i], pa[0][i], pa[1][i], pa[2][i]);
+#pragma unroll
+                    for (int j = 0; j < FN; j++) three_parts<BM * BN == 1024>(fb[ks][j], fb[ks + 1][j], pb[0][j], pb[1][j], pb[2][j]);
+                    auto products = [&](int p, int q, f32x16 (&to)[FM][FN]) {
+#pragma unroll
+                        for (int i = 0; i < FM; i++)
+#pragma unroll
+                            for (int j = 0; j < FN; j++)
+                                to[i][j] = Cvt<BR_GEMM_BF16>::mfma(pb[q][j], pa[p][i], !kApart && fresh && ks + p + q == 0 ? f32x16{} : to[i][j]);
+                    };
+                    products(0, 0, acc);
+                    auto small_products = [&](f32x16 (&to)[FM][FN]) {
+                        products(0, 1, to);
+                        products(1, 0, to);
+                        products(1, 1, to);
+                        products(0, 2, to);
+                        products(2, 0, to);
+                    };
+                    if constexpr (!kApart) small_products(acc);
+                    else if constexpr (CT == BR_GEMM_F32) small_products(low);
+                }
+            } else if constexpr (kHow == kOneByOne) {
+                // product s of a sub-step multiplies slot s of both halves of the wave, two k-values; the blocks take
+                // turns, so that no product waits for the one before it
+#pragma unroll
+                for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+                    for (int s = 0; s < 4; s++)
+#pragma unroll
+                        for (int i = 0; i < FM; i++)
+#pragma unroll
+                            for (int j = 0; j < FN; j++)
+                                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(fb[ks][j][s]), __uint_as_float(fa[ks][i][s]),
+                                                                                 fresh && ks == 0 && s == 0 ? f32x16{} : acc[i][j], 0, 0, 0);
+            } else {
+#pragma unroll
+                for (int ks = 0; ks < 4; ks++)
+#pragma unroll
+                    for (int i = 0; i < FM; i++)
+#pragma unroll
+                        for (int j = 0; j < FN; j++) acc[i][j] = Cvt<kHow == kInTheirType ? CT : BR_GEMM_BF16>::mfma(fb[ks][j], fa[ks][i], acc[i][j]);
+            }
+        }
+        fold();
+    };
+    if constexpr (CT == BR_GEMM_F32) {
+        const unsigned char* const a_first = a_src;
+        const unsigned char* const b_first = b_src;
+        const long long a_all = a_left, b_all = b_left;
+        const int k_all = k_left;
+        if (k_end - k_begin <= kApartUpTo * KW) walk(std::integral_constant<int, kAsParts>{});
+        else walk(std::integral_constant<int, kAsPartsFolded>{});
+        bool odd = false;
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+#pragma unroll
+                for (int v = 0; v < 16; v++) odd |= __builtin_amdgcn_classf(low[i][j][v] * 0x1p-26f, kNotNumbers | kSubnormals);
+        if (__any(odd)) {
+            a_src = a_first; b_src = b_first;
+            a_left = a_all; b_left = b_all;
+            k_left = k_all;
+            walk(std::integral_constant<int, kOneByOne>{});
+        }
+    } else {
+        walk(std::integral_constant<int, kInTheirType>{});
     }
-    if constexpr (kFold) fold();
 
-    if constexpr (kFold) flex_park<BM, BN>(held, mem, lane);
+    if constexpr (CT == BR_GEMM_F32) flex_park<BM, BN>(low, mem, lane);
     else flex_park<BM, BN>(acc, mem, lane);
     __syncthreads();
     flex_emit<BM, BN, KW, KW * 64, TC, GELU>(g, (lds_byte*)lds_raw, kWaveBytes, row0, col0, b);
@@ -624,9 +720,8 @@ int launch_flex(const GemmArgs& g, const Problem& p, int kernel, long long batch
 
 // fp32 operands and C.  `words`: an operand's rows are not aligned to 16 bytes (or a k-contiguous one's do not end on
 // such a boundary), so it is loaded value by value.
-template <int BM, int BN, bool WORDS>
+template <int BM, int BN, int KW, bool WORDS>
 int launch_flex_fp32(GemmArgs g, const Problem& p, long long batch, hipStream_t st) {
-    constexpr int KW = 4;
     g.tiles_m = (int)((g.m + BM - 1) / BM);
     g.tiles_n = (int)((g.n + BN - 1) / BN);
     const long long blocks = (long long)g.tiles_m * g.tiles_n * batch;

@@ -152,49 +152,35 @@ inline int flex_kernel(long long m, long long n, long long k, long long batch) {
     return best;
 }
 
-// fp32 products (gemm_flex.hpp): the tile whose matrix instructions finish first.  A step of 32 k-values takes a wave
-// 64 / 32 / 16 instructions of 64 clocks; measured with everything around them 2.45 / 1.4 / 0.78 us per step and
-// workgroup of a CU, and 2.7 us besides.  A CU that holds one workgroup more than the others sets the time.  (Measured, as
-// kPairCost32 is, before the sums of 64 k-values went to registers of their own, which is 2.3 % more on average.)
+// fp32 products (gemm_flex.hpp): us = start + steps * max(step, load * workgroups of a CU) + merge * workgroups of a CU, a step
+// being 32 k-values of a wave; a CU that holds one workgroup more than the others sets the time.  Fitted to 80 products of 16 to
+// 4096 rows, each on every tile (median error 4-6 %); choosing by it takes 2140 us for all of them, the best of the measurements
+// 2128, the tiles as they were when matrix instructions of fp32 operands did the products 2697.
+struct Fp32Cost {
+    double start, step, load, merge;
+};
+constexpr Fp32Cost kFp32Cost64{4.21, 1.542, 1.341, 1.62}, kFp32Cost32x64{3.83, 0.83, 0.796, 0.61}, kFp32Cost32{3.38, 0.60, 0.509, 0.27};
+// 32 x 32 tiles of at most one to a CU: from here on K is dealt to eight waves instead of four (0.51 us per step of four)
+constexpr long long kFp32EightWaves = 512;
+inline double fp32_us(int kernel, long long m, long long n, long long k, long long batch) {
+    const KernelCost& c = kCost[kernel];
+    const Fp32Cost& f = kernel == kFlex64 ? kFp32Cost64 : kernel == kFlex32x64 ? kFp32Cost32x64 : kFp32Cost32;
+    const double per_cu = (double)(ceil_div(m, c.bm) * ceil_div(n, c.bn) * batch) / 256.0;
+    const double step = kernel == kFlex32 && per_cu <= 1.0 && k >= kFp32EightWaves ? 0.51 : f.step;
+    const double load = f.load * (per_cu < 4.0 ? ceil(per_cu) : per_cu);
+    return f.start + (double)ceil_div(ceil_div(k, 32), 4) * (load > step ? load : step) + f.merge * per_cu;
+}
 inline int fp32_kernel(long long m, long long n, long long k, long long batch) {
-    auto us = [&](int kernel, double per_step) {
-        const KernelCost& c = kCost[kernel];
-        const double load = (double)(ceil_div(m, c.bm) * ceil_div(n, c.bn) * batch) / 256.0;
-        return 2.7 + (load >= 4.0 ? load : ceil(load)) * (double)ceil_div(ceil_div(k, 32), 4) * per_step;
-    };
     int best = kFlex64;
-    double t = us(kFlex64, 2.45);
-    if (us(kFlex32x64, 1.4) < 0.98 * t) best = kFlex32x64, t = us(kFlex32x64, 1.4);
-    if (us(kFlex32, 0.78) < 0.98 * t) best = kFlex32;
-    // kTile128: 128 x 128 tiles of four waves (gemm.hip), three to a CU.  A short K gives a wave of the small tiles one
-    // step and an accumulator to merge; many whole tiles then go faster by rounds of these: [512 x 512] K = 128, 128
-    // products 126 us against 142 (1024 tiles, a round and a third, 80 against 67; 512 tiles 37 against 41).
+    for (int c : {kFlex32x64, kFlex32})
+        if (fp32_us(c, m, n, k, batch) < fp32_us(best, m, n, k, batch)) best = c;
+    // kTile128: 128 x 128 tiles of four waves (gemm.hip), three to a CU.  From a K of little more than 64 the small tiles pay for
+    // four waves' steps and multiply with two and a bit; many whole tiles then go faster by rounds of these: [512 x 512], 128
+    // products from K = 65 89.5 us against 94.4, 48 from 72 33.1 against 34.9; from 96, 64 products, 65.3 against 45.3.
     const long long tiles = m / 128 * (n / 128) * batch;
-    if (k > 64 && k <= 128 && m % 128 == 0 && n % 128 == 0 && tiles >= 512 &&
-        38.0 * (double)ceil_div(tiles, 768) * (double)k / 128.0 < 5.0 + 0.067 * (double)tiles)
+    if (k > 64 && k <= 80 && m % 128 == 0 && n % 128 == 0 && 30.0 * (double)ceil_div(tiles, 768) < 1.0 + 0.0447 * (double)tiles)
         return kTile128;
     return best;
-}
-
-// What `batch` fp32 products of one size take in one launch: as fp32_kernel has it, with what a CU holds at a time (2 / 3 / 5
-// workgroups of each tile) put in.  Workgroups beyond a round of those start two or more to a CU, where the last round's
-// others have ended, so that part of a round takes most of a whole one; within a round the smaller tiles overlap.
-inline double fp32_batch_us(long long m, long long n, long long k, long long batch) {
-    const int kernel = fp32_kernel(m, n, k, batch);
-    if (kernel == kTile128) return 0.0;   // its rule compares whole launches
-    const KernelCost& c = kCost[kernel];
-    const bool wide = kernel == kFlex64, mid = kernel == kFlex32x64;
-    const double load = (double)(ceil_div(m, c.bm) * ceil_div(n, c.bn) * batch) / 256.0, held = wide ? 2.0 : mid ? 3.0 : 5.0;
-    const double whole = held * ceil(load / held), part = load + (wide ? 0.9 : mid ? 1.2 : 0.6);
-    const double rounds = load <= held ? ceil(load) : whole < part ? whole : part;
-    return 2.7 + rounds * (load <= 1.0 || wide ? 1.0 : mid ? 0.9 : 0.87) * (double)ceil_div(ceil_div(k, 32), 4) * (wide ? 2.45 : mid ? 1.4 : 0.78);
-}
-// Several fp32 products of one size: whether each gets a launch of its own.  Three linear layers of h features, one launch
-// each / one for all, us: 512 tokens, h = 2048 118 / 142, 1000 tokens, h = 1024 68.5 / 79.5, 1000 tokens, h = 1536 137 / 160;
-// 700 tokens, h = 1024 58.4 / 55.2, 1000 tokens, h = 512 28.2 / 22.2, 400 tokens, h = 2048 116 / 106.  Over 77 sizes (32-1200
-// tokens, h = 256-2048) the rule takes 2546 us, the better of both each time too, one launch always 2673.
-inline bool fp32_apart(long long m, long long n, long long k, long long batch) {
-    return (double)batch * fp32_batch_us(m, n, k, 1) < fp32_batch_us(m, n, k, batch);
 }
 
 // Two products as one launch of small tiles (gemm_pair.hpp): the tile, or -1 where they run one after the other.
@@ -210,16 +196,10 @@ struct PairCost {
 };
 constexpr int kPairKernels[3] = {kFlex64, kFlex32x64, kFlex32};
 constexpr PairCost kPairCost16[3] = {{4.29, 0.884, 0.757, 1.80}, {3.47, 0.722, 0.596, 0.79}, {3.02, 0.542, 0.433, 1.47}};
-constexpr PairCost kPairCost32[3] = {{4.55, 2.392, 2.434, 0.54}, {3.72, 1.365, 0.962, 1.72}, {3.31, 0.807, 0.650, 0.65}};
+constexpr PairCost kPairCost32[3] = {{4.94, 1.637, 1.504, 1.10}, {4.24, 0.961, 0.867, 0.75}, {3.81, 0.655, 0.523, 0.28}};
 struct PairSizes {
     long long m, n, k, batch;
 };
-inline double fp32_us(int kernel, const PairSizes& s) {
-    const KernelCost& c = kCost[kernel];
-    const double load = (double)(ceil_div(s.m, c.bm) * ceil_div(s.n, c.bn) * s.batch) / 256.0;
-    const double step = kernel == kFlex64 ? 2.45 : kernel == kFlex32x64 ? 1.4 : 0.78;
-    return 2.7 + (load >= 4.0 ? load : ceil(load)) * (double)ceil_div(ceil_div(s.k, 32), 4) * step;
-}
 #ifndef BR_PAIR_FORCE
 #define BR_PAIR_FORCE -1   // a kernel: every pair of products on it, for measuring
 #endif
@@ -230,7 +210,7 @@ inline int pair_kernel(const PairSizes& a, const PairSizes& b, bool fp32) {
         if (fp32) {
             const int kernel = fp32_kernel(s->m, s->n, s->k, s->batch);
             if (kernel == kTile128) return -1;
-            us += fp32_us(kernel, *s);
+            us += fp32_us(kernel, s->m, s->n, s->k, s->batch);
         } else {
             us += gemm_plan(s->m, s->n, s->k, s->batch, true).us;
         }
@@ -240,18 +220,22 @@ inline int pair_kernel(const PairSizes& a, const PairSizes& b, bool fp32) {
     for (int i = 0; i < 3; i++) {
         const KernelCost& tile = kCost[kPairKernels[i]];
         const PairCost& c = fp32 ? kPairCost32[i] : kPairCost16[i];
-        double longest = 0.0, all = 0.0;
+        double longest = 0.0, all = 0.0, fewest = 1e30;
         for (const PairSizes* s : {&a, &b}) {
             const double groups = (double)(ceil_div(s->m, tile.bm) * ceil_div(s->n, tile.bn) * s->batch);
             const double steps = (double)ceil_div(ceil_div(s->k, fp32 ? 32 : 64), tile.k_waves);
             if (steps * c.step > longest) longest = steps * c.step;
+            if (groups < fewest) fewest = groups;
             all += groups * (steps + c.merge) * c.load / 256.0;
         }
         const double t = c.start + (all > longest ? all : longest);
-        // A hurdle for the close ones: [1024 x 4096] from 74 tokens 14.3 in two launches, 14.8 in one.  Not for fp32 on 32-row
-        // tiles, where two launches take 10 % more than these costs say: of 77 pairs priced at 0.97 to 1 of two launches one
-        // takes 0.90 of them, none more than they do (64 tokens, 2048 -> 6144 82 / 60 us; on 64 x 64 tiles 0.91 to 1.09).
-        const double hurdle = fp32 && kPairKernels[i] != kFlex64 ? 1.0 : 0.97;
+        // A hurdle for the close ones: [1024 x 4096] from 74 tokens 14.3 in two launches, 14.8 in one.  fp32: two launches
+        // take more than these costs say where the tiles are small or both products fill the chip (1000 tokens, 2048 -> 2048 on
+        // 64 x 64 tiles 106 us in one launch, 113 in two).  Over 79 pairs (16 to 1000 tokens of 256 to 6144 features, attention
+        // heads of 16 to 512) 2313 us by the rule, 2271 by the best of the measurements, 3187 when matrix instructions of fp32
+        // operands did the products.
+        const int tile_of = kPairKernels[i];
+        const double hurdle = !fp32 ? 0.97 : tile_of == kFlex32 ? 1.05 : tile_of == kFlex32x64 ? 0.98 : fewest >= 256.0 ? 1.1 : 0.95;
         if (t < hurdle * us && t < best_us) best = kPairKernels[i], best_us = t;
     }
     return best;

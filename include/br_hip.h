@@ -485,8 +485,7 @@ int br_hip_linear_gelu(const void* x, const void* w, const float* bias, void* u,
 
 /* `count` op_linear of one x (cuda_tensor.cpp:146-193; the query, key and value
  * layers of bloomz-7b/train.words:139-145) whose weights [out, in], biases [out]
- * and outputs [rows, out] lie one behind the other: one batch of products, or with
- * BR_GEMM_F32 one after the other where their tiles fill the chip better so, x
+ * and outputs [rows, out] lie one behind the other: one batch of products, x
  * converted once.  workspace: br_hip_linear_group_workspace() bytes. */
 size_t br_hip_linear_group_workspace(int count, int64_t rows, int64_t out, int64_t in, int x_dtype, int w_dtype);
 int br_hip_linear_group(const void* x, int x_dtype, const void* w, int w_dtype, const float* bias, void* y, int y_dtype,

@@ -3,6 +3,7 @@ layout, storage type and compute type, odd sizes, batching, bias, alpha and
 accumulation.  Tolerances: 2e-2 relative for fp16 / bf16 operands, 1e-5 for
 the fp32-operand kernel."""
 import ctypes
+import math
 
 import numpy as np
 import pytest
@@ -579,6 +580,50 @@ def test_gemm_fp32_rows_far_apart(ta, tb, wide):
          0, ptr(bias), 1, hip.GEMM_F32, stream())
     torch.cuda.synchronize()
     assert torch.equal(c, want)
+
+
+@pytest.mark.parametrize("m,n,k", [(64, 96, 40), (64, 96, 511), (200, 768, 512), (520, 1028, 2048), (520, 1028, 2052), (512, 1024, 3072),
+                                   (64, 256, 4096), (64, 256, 4100), (1000, 1100, 2120), (31, 65, 2049)])
+def test_gemm_fp32_error_against_64_bits(m, n, k):
+    """Products as sums of bf16 parts: apart and folded, four waves and eight, every tile, values one by one.  Rounding sums of 64
+    products of random sign to 24 bits one after the other leaves 2^-25 sqrt(64 / 2) = 1.7e-7 of the result."""
+    print("case m=%d n=%d k=%d" % (m, n, k), flush=True)
+    torch.manual_seed(k)
+    for ta, tb in ((0, 1), (1, 0)):
+        a, b = torch.randn((k, m) if ta else (m, k), device="cuda"), torch.randn((n, k) if tb else (k, n), device="cuda")
+        c = torch.full((m, n), float("nan"), device="cuda")
+        call("br_hip_gemm", ta, tb, m, n, k, 1.0, ptr(a), F32, a.shape[1], 0, ptr(b), F32, b.shape[1], 0, 0, ptr(c), F32, n, 0, None, 1,
+             hip.GEMM_F32, stream())
+        want = (a.t() if ta else a).double().contiguous() @ (b.t() if tb else b).double().contiguous()
+        assert ((c - want).norm() / want.norm()).item() <= 2.0e-7
+
+
+@pytest.mark.parametrize("k", [40, 512, 2100])
+@pytest.mark.parametrize("m,n", [(32, 64), (200, 768), (1000, 2100)])
+def test_gemm_fp32_values_that_parts_do_not_hold(m, n, k):
+    """Infinities, NaN, a value that rounds past bf16's largest and operands of some 2^-115 come out as from fp32 instructions."""
+    print("case m=%d n=%d k=%d" % (m, n, k), flush=True)
+    torch.manual_seed(k)
+    for odd in (True, False):
+        a, b = torch.randn((m, k), device="cuda"), torch.randn((n, k), device="cuda")
+        if odd:
+            a[3, 5], a[7, 9], b[11, 2], a[20, 30] = math.inf, math.nan, -math.inf, 3.4e38
+            b[:, 30] = 0.25
+            b[12, 5] = 0.0
+        else:
+            a *= 2.0 ** -115
+        c = torch.full((m, n), 5.0, device="cuda")
+        call("br_hip_gemm", 0, 1, m, n, k, 1.0, ptr(a), F32, k, 0, ptr(b), F32, k, 0, 0, ptr(c), F32, n, 0, None, 1, hip.GEMM_F32, stream())
+        want = (a.double() @ b.double().t().contiguous()).cpu()   # of bounded rows and columns: no sum is beyond fp32
+        got = c.double().cpu()
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+        assert torch.equal(got[want.isinf()], want[want.isinf()])
+        sure = want.isfinite()
+        sure[20] &= not odd   # one value outweighs the others
+        assert ((got - want)[sure].norm() / want[sure].norm()).item() <= 2.0e-7
+        if odd:
+            both = want[20].isfinite()
+            assert ((got[20] - want[20])[both].norm() / want[20][both].norm()).item() <= 2.0e-7
 
 
 def test_gemm_fp32_without_k_leaves_the_bias():
