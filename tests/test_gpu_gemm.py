@@ -843,6 +843,33 @@ def test_two_products_of_a_linear_layer_in_one_launch_are_exact_on_integers(n, i
         assert torch.equal(db, 0.5 * dy[0].float().sum(0))
 
 
+@pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16])
+@pytest.mark.parametrize("n,inn,out,x_dt", [(1, 1024, 1024, None), (64, 2056, 2040, None), (128, 1024, 4096, None), (200, 512, 2048, F32),
+                                            (257, 1024, 3080, None), (300, 520, 2056, F32)])
+def test_weight_gradients_on_wide_tiles_beside_the_other_product_are_exact_on_integers(n, inn, out, x_dt, compute):
+    """One K step of the wide tiles to five, whole tiles and remainders either way, eight waves with a step each and some without;
+    column sums and partial sums beside them, dx in either type and either product first."""
+    dt = COMPUTE_T[compute]
+    print("case n=%d in=%d out=%d compute=%d" % (n, inn, out, compute), flush=True)
+    assert hip.load().br_hip_gemm_pair_kernel(out, inn, n, 1, n, inn, out, 1, compute) == 10   # BR_GEMM_PAIR_WIDE
+    torch.manual_seed(n)
+    partials = whole_numbers((3, 65, 68), 1, F32)
+    for dx_dt, turned in ((dt, False), (F32, True)):
+        dy, x, w = whole_numbers((1, n, out), 1, dt), whole_numbers((1, n, inn), 1, x_dt or dt), whole_numbers((1, out, inn), 1, dt)
+        dw = torch.full((1, out, inn), float("nan"), device="cuda")
+        dx = torch.full((1, n, inn), float("nan"), device="cuda", dtype=TORCH_T[dx_dt])
+        db, added = torch.full((out,), float("nan"), device="cuda"), torch.full((3, 68), float("nan"), device="cuda")
+        need = hip.load().br_hip_colsum_workspace(n, out)
+        ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+        sums = hip.ColumnSums(ptr(dy), dt, ptr(db), n, out, 0.5, ptr(ws), need)
+        later = hip.PartialSums(ptr(partials), 3, 65, 68, (ctypes.c_void_p * 3)(*(added[i].data_ptr() for i in range(3))), 2.0)
+        products = [(1, 0, dy, x, dw), (0, 0, dy, w, dx)]
+        assert run_pair(products[::-1] if turned else products, compute, sums, later)
+        assert torch.equal(dw, pair_reference(1, 0, dy, x).float())
+        assert torch.equal(dx, pair_reference(0, 0, dy, w).to(dx.dtype))
+        assert torch.equal(db, 0.5 * dy[0].float().sum(0)) and torch.equal(added, 2 * partials.sum(1))
+
+
 @pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16, hip.GEMM_F32])
 @pytest.mark.parametrize("n", [64, 700])   # one launch, and (16-bit) two after the sums
 @pytest.mark.parametrize("arrays,parts,cols", [(2, 1, 4), (3, 7, 68), (3, 39, 256), (2, 64, 1000), (3, 65, 60), (3, 256, 4096)])
