@@ -129,6 +129,33 @@ def test_logsoftmax_nll_against_oracle(rows, vocab):
     assert np.array_equal(host(dl), g)
 
 
+@pytest.mark.parametrize("rows,vocab", [(9, 1), (9, 2), (9, 3), (7, 5), (6, 1023), (5, 4097), (8, 16389), (3, 16386), (4, 32003)])
+def test_logsoftmax_nll_of_rows_that_start_anywhere(rows, vocab):
+    """A vocabulary that is no multiple of four: labels on the first and last values of rows, in quads and around them, rows
+    without one; four quads of a thread at a time and fewer.  fp32, in place, fp16, logits off 16-byte boundaries."""
+    rng = np.random.default_rng(vocab)
+    logits = (2 * rng.standard_normal((rows, vocab))).astype(np.float32)
+    target = np.array([[0, vocab - 1, vocab // 2, min(4, vocab - 1), max(vocab - 4, 0)][r % 5] for r in range(rows)], np.int32)
+    keep = np.ones(rows, np.int32)
+    keep[rows // 2] = 0
+    loss_ref, lse_ref, dl_ref = orc.logsoftmax_nll(logits, target, keep)
+    loss, count, lse, g, dl, dt, dk, dlse = nll_run(logits, target, keep)
+    assert count == rows - 1 and abs(loss - loss_ref) <= RTOL * abs(loss_ref) + 1e-6
+    assert_close(lse, lse_ref, RTOL, "lse")
+    assert_close(g, dl_ref, RTOL, "dlogits")
+    _, _, _, g16, *_ = nll_run(logits, target, keep, F16)
+    assert_close_f16(g16, dl_ref, RTOL, "dlogits fp16")
+    room = torch.zeros(rows * vocab + 1, device="cuda")
+    room[1:] = dl.reshape(-1)
+    off, res, lse2, logp = room[1:], empty(2), empty(rows), empty(rows)
+    call("br_hip_logsoftmax_nll_fwd", ptr(off), ptr(dt), ptr(dk), ptr(lse2), ptr(logp), ptr(res), rows, vocab, stream())
+    assert_close(host(lse2), lse_ref, RTOL, "lse, off boundaries")
+    call("br_hip_logsoftmax_nll_bwd", ptr(off), ptr(dt), ptr(dk), ptr(dlse), ptr(off), F32, 1.0 / count, rows, vocab, stream())
+    assert np.array_equal(host(room)[1:].reshape(rows, vocab), g)
+    call("br_hip_logsoftmax_nll_bwd", ptr(dl), ptr(dt), ptr(dk), ptr(dlse), ptr(dl), F32, 1.0 / count, rows, vocab, stream())
+    assert np.array_equal(host(dl), g)
+
+
 def test_logsoftmax_nll_headline_shape_properties_and_sampled_rows():
     """logits[2048, 250880] fp32 ~N(0,2), targets uniform, mask Bernoulli(0.9),
     seed 2.  Too large for a full oracle pass in seconds: rows are independent,
