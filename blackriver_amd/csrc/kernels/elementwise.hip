@@ -965,8 +965,10 @@ __global__ __launch_bounds__(kOwnThreads) void pack_colsum_kernel(PackSet set, f
 }
 template <typename D>
 int pack_colsum(const PackSet& set, int count, float* out, void* packed, int64_t rows, int64_t cols, float scale, hipStream_t st) {
-    // lanes per row as in owner_lanes: the narrowest strips whose workgroups fit the chip
-    const int lanes = rows <= 128 ? 8 : count * cols / 8 <= 512 ? 2 : count * cols / 16 <= 512 ? 4 : 8;
+    // The widest strips that make 128 workgroups: with narrower ones a line of x is asked for by several.  Strips of 2 / 4 / 8
+    // quads, three matrices to fp16, us: [1000 x 512] 6.0 / 6.5 / 7.4, [1000 x 1024] 11.7 / 8.1 / 8.6, [1024 x 2048] 17.4 / 14.2 / 10.3,
+    // [500 x 1024] 6.3 / 4.8 / 5.2, [512 x 2048] 10.0 / 8.1 / 6.2, [300 x 1024] 4.1 / 3.7 / 3.8.
+    const int lanes = rows <= 128 || count * cols / 32 >= 128 ? 8 : count * cols / 16 >= 128 ? 4 : 2;
     const dim3 grid((unsigned)((cols + lanes * 4 - 1) / (lanes * 4)), (unsigned)count);
     D* const p = (D*)packed;
     if (lanes == 2) pack_colsum_kernel<2, D><<<grid, kOwnThreads, 0, st>>>(set, out, p, rows, cols, count * cols, scale);
