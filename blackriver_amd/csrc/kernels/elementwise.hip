@@ -1667,25 +1667,10 @@ int br_hip_pack_colsum(const float* const* x, int count, float* out, void* packe
     return BR_ERR_TODO;
 }
 
-int br_hip_gelu_bwd_colsum_cast(const float* dy, const float* x, float* dx, float* out, void* dx16, int dx16_dtype,
-                                int64_t rows, int64_t cols, float out_scale, void* workspace, size_t workspace_bytes,
-                                br_stream_t stream) {
-    if (rows <= 0 || cols <= 0) return BR_ERR_ATTR;
-    if (!dy || !x) return BR_ERR_INPUT;
-    if (!dx || !out || !dx16) return BR_ERR_OUTPUT;
-    if (dx16_dtype != BR_F16 && dx16_dtype != BR_BF16) return BR_ERR_TODO;
-    if (cols % 4 != 0 || !aligned16(dy) || !aligned16(x) || !aligned16(dx) ||
-        (reinterpret_cast<uintptr_t>(dx16) & 7u) != 0)
-        return BR_ERR_TODO;
-    if (!workspace || workspace_bytes < br_hip_colsum_workspace(rows, cols)) return BR_ERR_ATTR;
-    hipStream_t st = as_stream(stream);
-    if (const int lanes = owner_lanes(rows, cols, 4, kOwnSum)) {
-        if (dx16_dtype == BR_F16)
-            return colsum_owner_launch<2>(lanes, OwnGeluBwdCast<__half>{dy, x, dx, (__half*)dx16}, out, rows, cols, out_scale, st);
-        return colsum_owner_launch<2>(lanes, OwnGeluBwdCast<__hip_bfloat16>{dy, x, dx, (__hip_bfloat16*)dx16}, out, rows, cols,
-                                      out_scale, st);
-    }
-    float* partial = (float*)workspace;
+namespace {
+// The gradient and its copy with partial column sums of strips in `partial`; returns the number of strips.
+int gelu_bwd_strips(const float* dy, const float* x, float* dx, float* partial, void* dx16, int dx16_dtype, int64_t rows, int64_t cols,
+                    hipStream_t st) {
     // same strips as br_hip_colsum_cast, hence the same summation order
     const int64_t blocks_x = (cols / 4 + kBlock - 1) / kBlock;
     const int rpb = colsum_vec_rows_per_block(rows, blocks_x);
@@ -1694,10 +1679,57 @@ int br_hip_gelu_bwd_colsum_cast(const float* dy, const float* x, float* dx, floa
     if (dx16_dtype == BR_F16)
         gelu_bwd_colsum_cast_partial<__half><<<grid, kBlock, 0, st>>>(dy, x, dx, partial, (__half*)dx16, rows, cols, rpb);
     else
-        gelu_bwd_colsum_cast_partial<__hip_bfloat16><<<grid, kBlock, 0, st>>>(dy, x, dx, partial,
-                                                                             (__hip_bfloat16*)dx16, rows, cols, rpb);
+        gelu_bwd_colsum_cast_partial<__hip_bfloat16><<<grid, kBlock, 0, st>>>(dy, x, dx, partial, (__hip_bfloat16*)dx16, rows, cols, rpb);
+    return groups;
+}
+int gelu_bwd_cast_checks(const float* dy, const float* x, float* dx, float* out, void* dx16, int dx16_dtype, int64_t rows, int64_t cols,
+                         void* workspace, size_t workspace_bytes) {
+    if (rows <= 0 || cols <= 0) return BR_ERR_ATTR;
+    if (!dy || !x) return BR_ERR_INPUT;
+    if (!dx || !out || !dx16) return BR_ERR_OUTPUT;
+    if (dx16_dtype != BR_F16 && dx16_dtype != BR_BF16) return BR_ERR_TODO;
+    if (cols % 4 != 0 || !aligned16(dy) || !aligned16(x) || !aligned16(dx) || (reinterpret_cast<uintptr_t>(dx16) & 7u) != 0)
+        return BR_ERR_TODO;
+    if (!workspace || workspace_bytes < br_hip_colsum_workspace(rows, cols)) return BR_ERR_ATTR;
+    return BR_OK;
+}
+}  // namespace
+
+int br_hip_gelu_bwd_colsum_cast(const float* dy, const float* x, float* dx, float* out, void* dx16, int dx16_dtype,
+                                int64_t rows, int64_t cols, float out_scale, void* workspace, size_t workspace_bytes,
+                                br_stream_t stream) {
+    const int rc = gelu_bwd_cast_checks(dy, x, dx, out, dx16, dx16_dtype, rows, cols, workspace, workspace_bytes);
+    if (rc != BR_OK) return rc;
+    hipStream_t st = as_stream(stream);
+    if (const int lanes = owner_lanes(rows, cols, 4, kOwnSum)) {
+        if (dx16_dtype == BR_F16)
+            return colsum_owner_launch<2>(lanes, OwnGeluBwdCast<__half>{dy, x, dx, (__half*)dx16}, out, rows, cols, out_scale, st);
+        return colsum_owner_launch<2>(lanes, OwnGeluBwdCast<__hip_bfloat16>{dy, x, dx, (__hip_bfloat16*)dx16}, out, rows, cols,
+                                      out_scale, st);
+    }
+    float* partial = (float*)workspace;
+    const int groups = gelu_bwd_strips(dy, x, dx, partial, dx16, dx16_dtype, rows, cols, st);
     BR_HIP_LAUNCH_CHECK();
     return colsum_finish(partial, out, groups, cols, out_scale, st);
+}
+
+int br_hip_gelu_bwd_cast_sums(const float* dy, const float* x, float* dx, float* out, void* dx16, int dx16_dtype, int64_t rows,
+                              int64_t cols, float out_scale, br_partial_sums* later, void* workspace, size_t workspace_bytes,
+                              br_stream_t stream) {
+    if (!later) return BR_ERR_OUTPUT;
+    const int rc = gelu_bwd_cast_checks(dy, x, dx, out, dx16, dx16_dtype, rows, cols, workspace, workspace_bytes);
+    if (rc != BR_OK) return rc;
+    if (!aligned16(out) || !aligned16(workspace)) return BR_ERR_TODO;
+    *later = br_partial_sums{};
+    const int groups = gelu_bwd_strips(dy, x, dx, (float*)workspace, dx16, dx16_dtype, rows, cols, as_stream(stream));
+    BR_HIP_LAUNCH_CHECK();
+    later->partials = (const float*)workspace;
+    later->arrays = 1;
+    later->parts = groups;
+    later->cols = cols;
+    later->out[0] = out;
+    later->scale = out_scale;
+    return BR_OK;
 }
 
 int br_hip_transpose_0213_group(const void* const* x, void* const* y, int count, int elem_bytes, int64_t s0, int64_t s1,

@@ -282,6 +282,12 @@ int br_hip_layernorm_bwd_add(const float* dy, const float* y, const float* gamma
                              size_t workspace_bytes, br_stream_t stream);
 /* Adds up what is described in *sums (nothing where its partials are null). */
 int br_hip_finish_sums(const br_partial_sums* sums, br_stream_t stream);
+/* br_hip_gelu_bwd_colsum_cast whose column sums are left as partial sums in the
+ * workspace, described in *later, for br_hip_gemm_pair to add up beside its
+ * products or br_hip_finish_sums to out (16-byte aligned).  BR_ERR_TODO as there. */
+int br_hip_gelu_bwd_cast_sums(const float* dy, const float* x, float* dx, float* out, void* dx16, int dx16_dtype,
+                              int64_t rows, int64_t cols, float out_scale, br_partial_sums* later, void* workspace,
+                              size_t workspace_bytes, br_stream_t stream);
 
 /* ---- softmax family ---------------------------------------------------- */
 /* cudnnSoftmaxForward(ACCURATE, INSTANCE) at cuda_tensor.cpp:332-356 and

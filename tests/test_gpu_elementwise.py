@@ -472,6 +472,34 @@ def test_memset_of_more_granules_than_a_launch_has_work_items():
 
 
 @pytest.mark.parametrize("dtype,tdtype", [(F16, torch.float16), (BF16, torch.bfloat16)])
+@pytest.mark.parametrize("rows,cols", [(1, 4), (5, 1028), (257, 1024), (300, 72), (1000, 4096), (1023, 20)])
+def test_gelu_bwd_cast_sums_are_those_of_one_launch(rows, cols, dtype, tdtype):
+    """The gradient and its copy bit for bit; the column sums, finished by a launch of their own, to the rounding of `rows`
+    32-bit additions in another order, which is at most 2^-24 of the sum of magnitudes each."""
+    torch.manual_seed(rows)
+    dy, x = torch.randn(rows, cols, device="cuda"), torch.randn(rows, cols, device="cuda")
+    need = hip.load().br_hip_colsum_workspace(rows, cols)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    got = []
+    for apart in (False, True):
+        dx, x16 = torch.empty_like(x), torch.empty((rows, cols), dtype=tdtype, device="cuda")
+        out = torch.full((cols,), float("nan"), device="cuda")
+        if apart:
+            later = hip.PartialSums()
+            call("br_hip_gelu_bwd_cast_sums", ptr(dy), ptr(x), ptr(dx), ptr(out), ptr(x16), dtype, rows, cols, 0.5, ctypes.byref(later), ptr(ws),
+                 need, stream())
+            assert later.arrays == 1 and later.cols == cols
+            call("br_hip_finish_sums", ctypes.byref(later), stream())
+        else:
+            call("br_hip_gelu_bwd_colsum_cast", ptr(dy), ptr(x), ptr(dx), ptr(out), ptr(x16), dtype, rows, cols, 0.5, ptr(ws), need, stream())
+        torch.cuda.synchronize()
+        got.append((dx, x16, out))
+    assert torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
+    want, bound = 0.5 * got[0][0].double().sum(0), rows * 2.0 ** -24 * got[0][0].double().abs().sum(0)
+    assert all(((out - want).abs() <= bound).all() for _, _, out in got)
+
+
+@pytest.mark.parametrize("dtype,tdtype", [(F16, torch.float16), (BF16, torch.bfloat16)])
 @pytest.mark.parametrize("rows,cols", [(2048, 16384), (37, 64), (5, 1000), (512, 16384), (300, 3080), (700, 1000),
                                        (700, 1404), (1000, 4100)])
 def test_gelu_bwd_colsum_cast_equals_the_separate_kernels(rows, cols, dtype, tdtype):
