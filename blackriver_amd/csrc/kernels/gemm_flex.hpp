@@ -37,10 +37,10 @@
 // fp32 products run on the same kernel, and on the 16-bit matrix instructions: a value is the sum of three bf16 values to 24
 // bits, and six of the nine products of such parts are all that a float holds of the whole.  They take 192 clocks for
 // 16 k-values of a 32 x 32 block, v_mfma_f32_32x32x2 512.  With those / with parts, us (and the error against 64 bits, 2-norm):
-// [512 x 1024] K = 1024 14.9 / 12.4 (1.6e-7 / 1.0e-7), K = 4096 43 / 33 (1.7e-7 / 1.4e-7), [512 x 4096] K = 1024 43.5 / 30.5 (1.6e-7 /
-// 1.0e-7), [1024 x 8192] K = 2048 282 / 198 (1.6e-7 / 1.3e-7), [342 x 216] K = 8560 47 / 38.6 (1.85e-7 / 1.75e-7); a launch of under
-// 6 us takes as long as before.  What bounds it: many tiles, the rate of the 16-bit instructions at the clock they leave (175
-// TFLOP/s are 1050 of theirs); one small tile to a CU, the loads into LDS, 25-30 B per clock whatever the tile and however many are
+// [512 x 1024] K = 1024 15.0 / 12.6 (1.6e-7 / 1.0e-7), K = 4096 43 / 34 (1.7e-7 / 1.6e-7), [512 x 4096] K = 1024 44 / 30.5 (1.6e-7 /
+// 1.0e-7), [1024 x 8192] K = 2048 282 / 206 (1.6e-7 / 1.5e-7), [342 x 216] K = 8560 47 / 38.4 (1.9e-7 / 1.7e-7); a launch of under
+// 6 us takes as long as before.  What bounds it: many tiles, the rate of the 16-bit instructions at the clock they leave (167
+// TFLOP/s are 1000 of theirs); one small tile to a CU, the loads into LDS, 25-30 B per clock whatever the tile and however many are
 // in flight (a second and a third buffer per wave measured equal or slower).
 #pragma once
 #include <type_traits>
@@ -223,14 +223,15 @@ __device__ __forceinline__ void flex_emit(const GemmArgs& g, const lds_byte* lds
 //
 // A fragment's products with those of the other operand, hi hi, hi mid, mid hi, mid mid, hi lo, lo hi:
 //   kAsParts        all but the first are added up in registers of their own: one rounding of the large sum for 16 k-values.
-//                   Up to 512 k-values a wave (kApartUpTo), from where the error passes that of
+//                   Up to 256 k-values a wave (kApartUpTo): with 512 the largest entry's error passes that of the fp32
+//                   instructions ([1024 x 8192] from K = 2048 1.23e-6 of the rms, 1.04e-6), with 1024 the 2-norm's too
 //   kAsPartsFolded  all into one accumulator, which goes to a second one every 64 k-values, so that errors grow with the number
 //                   of such sums and not with K (3-10 % slower)
 //   kOneByOne       the fp32 instructions, folded likewise.  What is not a number or beyond bf16's range in an operand makes the
 //                   parts' sums something else than a number, and an operand below 2^-110, whose parts lose bits, a result below
 //                   2^-100 (unless the other operand is large): a wave that finds either in its sums walks once more, like this.
 enum FlexWalk { kInTheirType, kAsParts, kAsPartsFolded, kOneByOne };
-constexpr int kApartUpTo = 512;
+constexpr int kApartUpTo = 256;
 constexpr int kNotNumbers = 0x207, kSubnormals = 0x090;   // classes of v_cmp_class_f32: NaN and infinity, subnormal
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));

@@ -362,7 +362,7 @@ int br_hip_logsoftmax_nll_bwd(const float* logits, const int32_t* target, const 
 enum {
     BR_GEMM_F16 = 0,  /* operands rounded to fp16, v_mfma_f32_32x32x16_f16  */
     BR_GEMM_BF16 = 1, /* operands rounded to bf16, v_mfma_f32_32x32x16_bf16 */
-    BR_GEMM_F32 = 2   /* fp32 operands, v_mfma_f32_32x32x2_f32              */
+    BR_GEMM_F32 = 2   /* fp32 operands, to 24 bits: three bf16 parts each    */
 };
 
 /* kernels::LtSgemm, kernels/LtSgemm.cu:55-126 (declared kernels/kernels.h:528-543),

@@ -582,7 +582,8 @@ def test_gemm_fp32_rows_far_apart(ta, tb, wide):
     assert torch.equal(c, want)
 
 
-@pytest.mark.parametrize("m,n,k", [(64, 96, 40), (64, 96, 511), (200, 768, 512), (520, 1028, 2048), (520, 1028, 2052), (512, 1024, 3072),
+@pytest.mark.parametrize("m,n,k", [(64, 96, 40), (64, 96, 511), (200, 768, 512), (520, 1028, 1024), (520, 1028, 1028), (64, 256, 2048),
+                                   (64, 256, 2052), (512, 1024, 3072),
                                    (64, 256, 4096), (64, 256, 4100), (1000, 1100, 2120), (31, 65, 2049)])
 def test_gemm_fp32_error_against_64_bits(m, n, k):
     """Products as sums of bf16 parts: apart and folded, four waves and eight, every tile, values one by one.  Rounding sums of 64
