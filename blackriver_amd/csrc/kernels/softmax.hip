@@ -566,7 +566,8 @@ void launch_nll_bwd(const float* logits, const int32_t* target, const int32_t* k
                     float scale, int64_t rows, int64_t vocab, bool aligned, hipStream_t st) {
     const bool vec_ok = aligned && vocab % 4 == 0;
     const int64_t blocks_x = (vocab / 4 + (vocab % 4 ? 6 : 0) + kFlatBlock - 1) / kFlatBlock;
-    if (BR_NLL_BWD_FLAT && aligned && rows <= 65535 && blocks_x <= 0x7fffffff) {
+    // (a launch of 2^32 or more work items runs without those beyond, and without an error)
+    if (BR_NLL_BWD_FLAT && aligned && rows <= 65535 && blocks_x <= 0xffffffffLL / kFlatBlock / rows) {
         const dim3 grid((unsigned)blocks_x, (unsigned)rows);
         if (vocab % 4 == 0) nll_bwd_flat_kernel<OUT, true><<<grid, kFlatBlock, 0, st>>>(logits, target, keep, lse, dlogits, scale, vocab);
         else nll_bwd_flat_kernel<OUT, false><<<grid, kFlatBlock, 0, st>>>(logits, target, keep, lse, dlogits, scale, vocab);
