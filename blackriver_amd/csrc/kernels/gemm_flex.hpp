@@ -36,11 +36,11 @@
 //
 // fp32 products run on the same kernel, and on the 16-bit matrix instructions: a value is the sum of three bf16 values to 24
 // bits, and six of the nine products of such parts are all that a float holds of the whole.  They take 192 clocks for
-// 16 k-values of a 32 x 32 block, v_mfma_f32_32x32x2 512.  With those / with parts, us (and the error against 64 bits, 2-norm):
-// [512 x 1024] K = 1024 15.0 / 12.6 (1.6e-7 / 1.0e-7), K = 4096 43 / 34 (1.7e-7 / 1.6e-7), [512 x 4096] K = 1024 44 / 30.5 (1.6e-7 /
-// 1.0e-7), [1024 x 8192] K = 2048 282 / 206 (1.6e-7 / 1.5e-7), [342 x 216] K = 8560 47 / 38.4 (1.9e-7 / 1.7e-7); a launch of under
-// 6 us takes as long as before.  What bounds it: many tiles, the rate of the 16-bit instructions at the clock they leave (167
-// TFLOP/s are 1000 of theirs); one small tile to a CU, the loads into LDS, 25-30 B per clock whatever the tile and however many are
+// 16 k-values of a 32 x 32 block, v_mfma_f32_32x32x2_f32 512.  With those / with parts, us (and the error against 64 bits, 2-norm):
+// [512 x 1024] K = 1024 14.8 / 13.4 (1.6e-7 / 1.0e-7), K = 4096 47.8 / 38.9 (1.7e-7 / 1.6e-7), [512 x 4096] K = 1024 47.0 / 32.5 (1.6e-7 /
+// 1.0e-7), [1024 x 8192] K = 2048 313 / 230 (1.6e-7 / 1.5e-7), [64 x 2048] K = 8192 45.1 / 37.3 (1.8e-7 / 1.7e-7); a launch of under
+// 6 us takes as long as before.  What bounds it: many tiles, the rate of the 16-bit instructions at the clock they leave (150
+// TFLOP/s are 900 of theirs); one small tile to a CU, the loads into LDS, 25-30 B per clock whatever the tile and however many are
 // in flight (a second and a third buffer per wave measured equal or slower).
 #pragma once
 #include <type_traits>
@@ -217,9 +217,12 @@ __device__ __forceinline__ void flex_emit(const GemmArgs& g, const lds_byte* lds
     }
 }
 
-// The three bf16 parts of eight fp32 values of a lane, each the nearest to what the parts before it leave (those differences
-// are exact).  DOTS: the difference as a product of two pairs with -1 and 0, one instruction where shift or mask and
-// subtraction are two: 27.7 -> 25.1 us for a layer's backward products on 32 x 32 tiles, 2-3 % slower on 64 x 64.
+// The three bf16 parts of eight fp32 values of a lane times 2^24, each the nearest to what the parts before it leave (those
+// differences are exact).  bf16 has no bits below 2^-133: of a value below 2^-110 as it is the parts would hold fewer than 24, of
+// one of 2^-125 eight.  Times 2^24 the lowest bit there is lies at 2^-125, and whatever an fp32 operand holds, its parts hold too.
+// That multiplication is a fifth of the splitting (3 % of a launch, 4 to 7 % where one small tile is all a CU has).
+// All of a part ahead of the next one, so that no value waits for its own last step: value by value a layer's backward products
+// from 78 tokens take 31.0 us, so 28.6.
 //
 // A fragment's products with those of the other operand, hi hi, hi mid, mid hi, mid mid, hi lo, lo hi:
 //   kAsParts        all but the first are added up in registers of their own: one rounding of the large sum for 16 k-values.
@@ -227,42 +230,35 @@ __device__ __forceinline__ void flex_emit(const GemmArgs& g, const lds_byte* lds
 //                   instructions ([1024 x 8192] from K = 2048 1.23e-6 of the rms, 1.04e-6), with 1024 the 2-norm's too
 //   kAsPartsFolded  all into one accumulator, which goes to a second one every 64 k-values, so that errors grow with the number
 //                   of such sums and not with K (3-10 % slower)
-//   kOneByOne       the fp32 instructions, folded likewise.  What is not a number or beyond bf16's range in an operand makes the
-//                   parts' sums something else than a number, and an operand below 2^-110, whose parts lose bits, a result below
-//                   2^-100 (unless the other operand is large): a wave that finds either in its sums walks once more, like this.
+//   kOneByOne       the fp32 instructions, folded likewise.  An operand of 2^104 or more, infinite or not a number, and a sum of
+//                   2^80 or more make the parts' sums infinite or not a number: a wave that finds that in its sums walks once
+//                   more, like this.
 enum FlexWalk { kInTheirType, kAsParts, kAsPartsFolded, kOneByOne };
 constexpr int kApartUpTo = 256;
-constexpr int kNotNumbers = 0x207, kSubnormals = 0x090;   // classes of v_cmp_class_f32: NaN and infinity, subnormal
+constexpr float kPartsScale = 0x1p24f;
+constexpr int kNotNumbers = 0x207;   // classes of v_cmp_class_f32: NaN and infinity
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 typedef float f32x2 __attribute__((ext_vector_type(2)));
-template <bool DOTS>
 __device__ __forceinline__ void three_parts(const u32x4& first, const u32x4& second, u32x4& hi, u32x4& mid, u32x4& lo) {
-    // -1, 0 and 0, -1, in registers: as a constant the first becomes an inline -1.0, which the instruction takes for the second
-    unsigned x = 0x0000bf80u, y = 0xbf800000u;
-    asm("" : "+s"(x), "+s"(y));
-    auto without = [&](f32x2 v, bf16x2 h) {
-        if constexpr (DOTS) {
-            v.x = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(bf16x2, x), v.x, false);
-            v.y = __builtin_amdgcn_fdot2_f32_bf16(h, __builtin_bit_cast(bf16x2, y), v.y, false);
-        } else {
-            v.x -= __uint_as_float(__builtin_bit_cast(unsigned, h) << 16);
-            v.y -= __uint_as_float(__builtin_bit_cast(unsigned, h) & 0xffff0000u);
-        }
-        return v;
-    };
+    f32x2 v[4];
 #pragma unroll
     for (int e = 0; e < 4; e++) {
-        f32x2 v;
-        v.x = __uint_as_float(e < 2 ? first[2 * e] : second[2 * e - 4]);
-        v.y = __uint_as_float(e < 2 ? first[2 * e + 1] : second[2 * e - 3]);
-        const bf16x2 h = __builtin_convertvector(v, bf16x2);
-        v = without(v, h);
-        const bf16x2 m = __builtin_convertvector(v, bf16x2);
-        v = without(v, m);
-        hi[e] = __builtin_bit_cast(unsigned, h);
-        mid[e] = __builtin_bit_cast(unsigned, m);
-        lo[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(v, bf16x2));
+        v[e].x = __uint_as_float(e < 2 ? first[2 * e] : second[2 * e - 4]) * kPartsScale;
+        v[e].y = __uint_as_float(e < 2 ? first[2 * e + 1] : second[2 * e - 3]) * kPartsScale;
     }
+    auto next_part = [&](u32x4& to, bool last) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) to[e] = __builtin_bit_cast(unsigned, __builtin_convertvector(v[e], bf16x2));
+        if (last) return;
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            v[e].x -= __uint_as_float(to[e] << 16);
+            v[e].y -= __uint_as_float(to[e] & 0xffff0000u);
+        }
+    };
+    next_part(hi, false);
+    next_part(mid, false);
+    next_part(lo, true);
 }
 
 // LDS of a workgroup of such tiles
@@ -339,7 +335,7 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
     };
 
     f32x16 acc[FM][FN];
-    f32x16 low[CT == BR_GEMM_F32 ? FM : 1][CT == BR_GEMM_F32 ? FN : 1];   // fp32: what is added to `acc` at the end
+    f32x16 low[CT == BR_GEMM_F32 ? FM : 1][CT == BR_GEMM_F32 ? FN : 1];   // fp32: what `acc` is added to at the end
 
     // The wave's steps; `how`: see FlexWalk
     auto walk = [&](auto how) {
@@ -394,28 +390,30 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
                 constexpr bool kApart = kHow == kAsParts;
 #pragma unroll
                 for (int ks = 0; ks < 4; ks += 2) {
-                    u32x4 pa[3][FM], pb[3][FN];
+                    u32x4 pa[3][FM];
 #pragma unroll
-                    for (int i = 0; i < FM; i++) three_parts<BM * BN == 1024>(fa[ks][i], fa[ks + 1][i], pa[0][i], pa[1][i], pa[2][i]);
+                    for (int i = 0; i < FM; i++) three_parts(fa[ks][i], fa[ks + 1][i], pa[0][i], pa[1][i], pa[2][i]);
+                    // (the parts of all of B ahead of the products take more registers than 64 x 64 tiles have)
 #pragma unroll
-                    for (int j = 0; j < FN; j++) three_parts<BM * BN == 1024>(fb[ks][j], fb[ks + 1][j], pb[0][j], pb[1][j], pb[2][j]);
-                    auto products = [&](int p, int q, f32x16 (&to)[FM][FN]) {
+                    for (int j = 0; j < FN; j++) {
+                        u32x4 pb[3];
+                        three_parts(fb[ks][j], fb[ks + 1][j], pb[0], pb[1], pb[2]);
+                        auto products = [&](int p, int q, f32x16 (&to)[FM][FN]) {
 #pragma unroll
-                        for (int i = 0; i < FM; i++)
-#pragma unroll
-                            for (int j = 0; j < FN; j++)
-                                to[i][j] = Cvt<BR_GEMM_BF16>::mfma(pb[q][j], pa[p][i], !kApart && fresh && ks + p + q == 0 ? f32x16{} : to[i][j]);
-                    };
-                    products(0, 0, acc);
-                    auto small_products = [&](f32x16 (&to)[FM][FN]) {
-                        products(0, 1, to);
-                        products(1, 0, to);
-                        products(1, 1, to);
-                        products(0, 2, to);
-                        products(2, 0, to);
-                    };
-                    if constexpr (!kApart) small_products(acc);
-                    else if constexpr (CT == BR_GEMM_F32) small_products(low);
+                            for (int i = 0; i < FM; i++)
+                                to[i][j] = Cvt<BR_GEMM_BF16>::mfma(pb[q], pa[p][i], !kApart && fresh && ks + p + q == 0 ? f32x16{} : to[i][j]);
+                        };
+                        auto small_products = [&](f32x16 (&to)[FM][FN]) {
+                            products(0, 1, to);
+                            products(1, 0, to);
+                            products(1, 1, to);
+                            products(0, 2, to);
+                            products(2, 0, to);
+                        };
+                        products(0, 0, acc);
+                        if constexpr (!kApart) small_products(acc);
+                        else if constexpr (CT == BR_GEMM_F32) small_products(low);
+                    }
                 }
             } else if constexpr (kHow == kOneByOne) {
                 // product s of a sub-step multiplies slot s of both halves of the wave, two k-values; the blocks take
@@ -454,7 +452,10 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
 #pragma unroll
             for (int j = 0; j < FN; j++)
 #pragma unroll
-                for (int v = 0; v < 16; v++) odd |= __builtin_amdgcn_classf(low[i][j][v] * 0x1p-26f, kNotNumbers | kSubnormals);
+                for (int v = 0; v < 16; v++) {
+                    odd |= __builtin_amdgcn_classf(low[i][j][v], kNotNumbers);
+                    low[i][j][v] *= 1.0f / (kPartsScale * kPartsScale);
+                }
         if (__any(odd)) {
             a_src = a_first; b_src = b_first;
             a_left = a_all; b_left = b_all;

@@ -627,6 +627,59 @@ def test_gemm_fp32_values_that_parts_do_not_hold(m, n, k):
             assert ((got[20] - want[20])[both].norm() / want[20][both].norm()).item() <= 2.0e-7
 
 
+# 32 x 32 tiles (four waves, eight), 32 x 64, 64 x 64, apart and folded
+FP32_SIZES = [(32, 64, 40), (200, 768, 512), (1000, 2100, 2100), (500, 4100, 516), (500, 4100, 1032)]
+
+
+@pytest.mark.parametrize("front", [0, 1])   # values in front of A: 1 puts it off 16-byte boundaries
+@pytest.mark.parametrize("m,n,k", FP32_SIZES)
+def test_gemm_fp32_small_operands_keep_their_bits(m, n, k, front):
+    """Operands down to the smallest subnormal ones against such as bring the sums back to normal numbers, beside one of ordinary
+    size that meets zeros alone; the bound of test_gemm_fp32_error_against_64_bits.  And times one: every bit."""
+    print("case m=%d n=%d k=%d front=%d" % (m, n, k, front), flush=True)
+    rng = np.random.default_rng(k)
+
+    def product(a, b):
+        da, db = dev(np.concatenate([np.zeros(front, np.float32), a.ravel()])), dev(b)
+        c = torch.full((m, n), float("nan"), device="cuda")
+        call("br_hip_gemm", 0, 1, m, n, k, 1.0, ctypes.c_void_p(da.data_ptr() + 4 * front), F32, k, 0, ptr(db), F32, k, 0, 0, ptr(c), F32,
+             n, 0, None, 1, hip.GEMM_F32, stream())
+        return host(c)
+
+    for ea, eb in ((-115, 0), (-120, 30), (-125, 60), (-130, 10), (-140, 100), (40, -130)):
+        a, b = rng.standard_normal((m, k)) * 2.0 ** ea, rng.standard_normal((n, k)) * 2.0 ** eb
+        a[:, 0], b[:, 0] = 1, 0
+        a, b = a.astype(np.float32), b.astype(np.float32)
+        got, want = product(a, b), (dev(a).double() @ dev(b).double().t().contiguous()).cpu().numpy()
+        assert np.linalg.norm(got - want) / np.linalg.norm(want) <= 2.0e-7, (ea, eb)
+    if n >= k:
+        for e in (-124, -126, -135):
+            a = (rng.uniform(1, 4, (m, k)) * 2.0 ** e).astype(np.float32)
+            assert np.array_equal(product(a, np.eye(n, k, dtype=np.float32))[:, :k], a), e
+
+
+@pytest.mark.parametrize("n,inn,out,kernel", [(64, 256, 264, "flex 32"), (250, 1024, 3072, "flex 32x64"), (512, 1024, 1024, "flex 64")])
+def test_fp32_pairs_of_small_operands_and_of_values_that_parts_do_not_hold(n, inn, out, kernel):
+    print("case n=%d in=%d out=%d" % (n, inn, out), flush=True)
+    assert hip.load().br_hip_gemm_pair_kernel(out, inn, n, 1, n, inn, out, 1, hip.GEMM_F32) == hip.GEMM_KERNELS.index(kernel)
+    rng = np.random.default_rng(n)
+    for odd in (False, True):
+        dy, x, w = (rng.standard_normal(s) * 2.0 ** (0 if odd else e)
+                    for s, e in (((1, n, out), -125), ((1, n, inn), 60), ((1, out, inn), 60)))
+        if odd:
+            dy[0, 3, 5], dy[0, 20, 30], w[0, 11, 2], x[0, 9, 7] = math.inf, 3.0e38, math.nan, -math.inf
+            w[0, 30], x[0, 20] = 0.25, 0.25
+        dy, x, w = (dev(t.astype(np.float32)) for t in (dy, x, w))
+        dw, dx = torch.full((1, out, inn), float("nan"), device="cuda"), torch.full((1, n, inn), float("nan"), device="cuda")
+        assert run_pair([(1, 0, dy, x, dw), (0, 0, dy, w, dx)], hip.GEMM_F32)
+        for got, want in ((dw, pair_reference(1, 0, dy, x)), (dx, pair_reference(0, 0, dy, w))):
+            got, want = got.double(), torch.where(want.abs() >= 2.0 ** 128, want.sign() * math.inf, want)
+            assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got[want.isinf()], want[want.isinf()])
+            big = want.abs() > 1e30 if odd else want.isnan()   # one value outweighs the others
+            for part in (want.isfinite() & big, want.isfinite() & ~big):
+                assert not part.any() or ((got - want)[part].norm() / want[part].norm()).item() <= 2.0e-7
+
+
 def test_gemm_fp32_without_k_leaves_the_bias():
     bias, a = dev(np.arange(7, dtype=np.float32)), empty((5, 8))
     c = torch.full((5, 7), float("nan"), device="cuda")
