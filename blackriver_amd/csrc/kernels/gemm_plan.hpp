@@ -205,7 +205,7 @@ struct PairSizes {
 // shorter K), 32 x 32 tiles whose K is dealt to eight waves for the other.  Fitted to 193 linear layers of 16 to 700 tokens and
 // 256 to 8192 features (median error 7 %).  Taken where it beats everything else by these costs by 5 %, all of them together take
 // 2383 us instead of 2591, by the better of both each time 2360: from some 512 x 1536 features on and up to some 300 tokens
-// (16 tokens 4096 -> 1024 15.0 -> 9.3 us, 78 tokens 1024 -> 4096 16.0 -> 13.1, 200 tokens 512 -> 2048 9.2 -> 7.2; but 200 tokens
+// (16 tokens 4096 -> 1024 15.0 -> 9.3 us, 78 tokens 1024 -> 4096 16.0 -> 13.1, 200 tokens 512 -> 2048 9.2 -> 7.7; but 200 tokens
 // 512 -> 512 4.5, and 6.7 so).
 inline double wide_pair_us(const PairSizes& w, const PairSizes& x) {
     const double nw = (double)(ceil_div(w.m, 128) * ceil_div(w.n, 128)), nx = (double)(ceil_div(x.m, 32) * ceil_div(x.n, 32));

@@ -924,6 +924,25 @@ def test_weight_gradients_on_wide_tiles_beside_the_other_product_are_exact_on_in
         assert torch.equal(db, 0.5 * dy[0].float().sum(0)) and torch.equal(added, 2 * partials.sum(1))
 
 
+@pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16])
+@pytest.mark.parametrize("n,inn,out", [(200, 512, 2048), (257, 1024, 3080), (300, 1024, 4096)])
+def test_weight_gradients_on_wide_tiles_are_as_precise_as_on_small_ones(n, inn, out, compute):
+    """dW is four sums over every fourth 64 tokens, as a small tile's four waves leave them, added up at the end.  A matrix instruction
+    adds 16 products to a sum and is off by up to 0.65 x 2^-24 of what it leaves (2-norm; 0.6 measured from 16 tokens): all
+    roundings of the four and of the three additions, each times the variance the sum then has."""
+    dt, steps = COMPUTE_T[compute], -(-n // 64)
+    print("case n=%d in=%d out=%d compute=%d" % (n, inn, out, compute), flush=True)
+    assert hip.load().br_hip_gemm_pair_kernel(out, inn, n, 1, n, inn, out, 1, compute) == 10   # BR_GEMM_PAIR_WIDE
+    torch.manual_seed(n)
+    dy, x, w = (torch.randn(s, device="cuda").to(TORCH_T[dt]) for s in ((1, n, out), (1, n, inn), (1, out, inn)))
+    dw, dx = torch.empty((1, out, inn), device="cuda"), torch.empty((1, n, inn), device="cuda")
+    assert run_pair([(1, 0, dy, x, dw), (0, 0, dy, w, dx)], compute)
+    want = pair_reference(1, 0, dy, x)
+    waves = [[min(16, n - k) / n for t in range(w, steps, 4) for k in range(64 * t, min(64 * t + 64, n), 16)] for w in range(4)]
+    variance = sum(sum(np.cumsum(w)) for w in waves) + sum(np.cumsum([sum(w) for w in waves])[1:])
+    assert ((dw - want).norm() / want.norm()).item() <= 0.65 * 2.0 ** -24 * math.sqrt(variance)
+
+
 @pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16, hip.GEMM_F32])
 @pytest.mark.parametrize("n", [64, 700])   # one launch, and (16-bit) two after the sums
 @pytest.mark.parametrize("arrays,parts,cols", [(2, 1, 4), (3, 7, 68), (3, 39, 256), (2, 64, 1000), (3, 65, 60), (3, 256, 4096)])
