@@ -933,9 +933,10 @@ int plan_pair(const br_product& first, const br_product& second, const PairOpera
     auto wide = [](const br_product& p) { return p.trans_a && !p.trans_b && p.c_dtype == BR_F32; };
     const int w = wide(first) ? 0 : 1, x = 1 - w;
     if (!wide(w ? second : first) || (w ? first : second).trans_a) return BR_ERR_TODO;
-    const int kernel = pair_kernel({first.m, first.n, first.k, first.batch}, {second.m, second.n, second.k, second.batch}, fp32);
-    if (kernel < 0) return BR_ERR_TODO;
     const br_product* const products[2] = {&first, &second};
+    auto sizes = [&](int i) { return PairSizes{products[i]->m, products[i]->n, products[i]->k, products[i]->batch}; };
+    const int kernel = pair_kernel(sizes(w), sizes(x), fp32);
+    if (kernel < 0) return BR_ERR_TODO;
     const Stored out[2] = {stored_c(first), stored_c(second)};
     if (out[x].dtype != native && out[x].dtype != BR_F32) return BR_ERR_TODO;
     // nothing is written that another part reads or writes (what is copied first is read ahead of all writes)

@@ -27,6 +27,8 @@
 
 #include <math.h>
 
+#include <initializer_list>
+
 namespace brk {
 namespace gemm16 {
 
@@ -201,8 +203,8 @@ constexpr PairCost kPairCost32[3] = {{4.94, 1.637, 1.504, 1.10}, {4.24, 0.961, 0
 struct PairSizes {
     long long m, n, k, batch;
 };
-// Two 16-bit products as one launch of gemm_wide_pair_kernel: 128 x 128 tiles for the weight gradient `w` (the one with the
-// shorter K), 32 x 32 tiles whose K is dealt to eight waves for the other.  Fitted to 193 linear layers of 16 to 700 tokens and
+// Two 16-bit products as one launch of gemm_wide_pair_kernel: 128 x 128 tiles for the weight gradient `w`, 32 x 32 tiles whose K
+// is dealt to eight waves for the other.  Fitted to 193 linear layers of 16 to 700 tokens and
 // 256 to 8192 features (median error 7 %).  Taken where it beats everything else by these costs by 5 %, all of them together take
 // 2383 us instead of 2591, by the better of both each time 2360: from some 512 x 1536 features on and up to some 300 tokens
 // (16 tokens 4096 -> 1024 15.0 -> 9.3 us, 78 tokens 1024 -> 4096 16.0 -> 13.1, 200 tokens 512 -> 2048 9.2 -> 7.7; but 200 tokens
@@ -219,10 +221,11 @@ inline double wide_pair_us(const PairSizes& w, const PairSizes& x) {
 #ifndef BR_PAIR_FORCE
 #define BR_PAIR_FORCE -1   // a kernel: every pair of products on it, for measuring
 #endif
-inline int pair_kernel(const PairSizes& a, const PairSizes& b, bool fp32) {
+// `w`: the product whose operands are both row-contiguous, which alone can have the wide tiles.
+inline int pair_kernel(const PairSizes& w, const PairSizes& x, bool fp32) {
     if (BR_PAIR_FORCE >= 0) return BR_PAIR_FORCE;
     double us = 0.0;   // one after the other
-    for (const PairSizes* s : {&a, &b}) {
+    for (const PairSizes* s : {&w, &x}) {
         if (fp32) {
             const int kernel = fp32_kernel(s->m, s->n, s->k, s->batch);
             if (kernel == kTile128) return -1;
@@ -237,7 +240,7 @@ inline int pair_kernel(const PairSizes& a, const PairSizes& b, bool fp32) {
         const KernelCost& tile = kCost[kPairKernels[i]];
         const PairCost& c = fp32 ? kPairCost32[i] : kPairCost16[i];
         double longest = 0.0, all = 0.0, fewest = 1e30;
-        for (const PairSizes* s : {&a, &b}) {
+        for (const PairSizes* s : {&w, &x}) {
             const double groups = (double)(ceil_div(s->m, tile.bm) * ceil_div(s->n, tile.bn) * s->batch);
             const double steps = (double)ceil_div(ceil_div(s->k, fp32 ? 32 : 64), tile.k_waves);
             if (steps * c.step > longest) longest = steps * c.step;
@@ -254,10 +257,7 @@ inline int pair_kernel(const PairSizes& a, const PairSizes& b, bool fp32) {
         const double hurdle = !fp32 ? 0.97 : tile_of == kFlex32 ? 1.05 : tile_of == kFlex32x64 ? 0.98 : fewest >= 256.0 ? 1.1 : 0.95;
         if (t < hurdle * us && t < best_us) best = kPairKernels[i], best_us = t;
     }
-    if (!fp32 && a.batch == 1 && b.batch == 1) {
-        const double t = a.k <= b.k ? wide_pair_us(a, b) : wide_pair_us(b, a);
-        if (t < 0.95 * (best_us < us ? best_us : us)) best = kPairWide;
-    }
+    if (!fp32 && w.batch == 1 && x.batch == 1 && wide_pair_us(w, x) < 0.95 * (best_us < us ? best_us : us)) best = kPairWide;
     return best;
 }
 

@@ -418,7 +418,8 @@ int br_hip_gemm_staged(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k
  * another reads or writes, all of it is ONE launch; results then differ from the
  * separate calls' in the order of the fp32 sums alone.  The same arguments
  * always take the same way.  br_hip_gemm_pair_kernel tells which kernel sizes
- * alone would have the one launch run on (BR_GEMM_FLEX_*, BR_GEMM_PAIR_WIDE), or -1 where they make
+ * alone, first those of the product with both operands row-contiguous, would have
+ * the one launch run on (BR_GEMM_FLEX_*, BR_GEMM_PAIR_WIDE), or -1 where they make
  * several; br_hip_gemm_pair_joined which one br_hip_gemm_pair runs these very
  * operands on, or -1 (addresses are compared and nothing is read: it needs no
  * GPU).  The outs of `later` lie apart from each other and from the partials. */

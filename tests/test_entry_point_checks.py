@@ -87,6 +87,36 @@ def test_fp32_pairs_that_cost_about_two_launches_by_the_rule(n, inn, out, name):
     assert kernel == (-1 if name is None else hip.GEMM_KERNELS.index(name))
 
 
+def on_wide_tiles(*products):
+    """Whether two products, the weight gradient's (trans_a, trans_b, m, n, k) first, share a launch with wide tiles: by their sizes, and
+    as operands in either order."""
+    import ctypes
+    from blackriver_amd import hip
+    lib, wide = hip.load(), 10   # BR_GEMM_PAIR_WIDE
+    (_, _, m1, n1, k1), (_, _, m2, n2, k2) = products
+    by_size = lib.br_hip_gemm_pair_kernel(m1, n1, k1, 1, m2, n2, k2, 1, hip.GEMM_F16)
+    made = [hip.Product(ta, tb, m, n, k, 1.0, 64 * MB, hip.F16, m if ta else k, 0, at, hip.F16, k if tb else n, 0, 2 * at, hip.F32, n, 0, 1)
+            for at, (ta, tb, m, n, k) in zip((256 * MB, 1024 * MB), products)]
+    joined = [lib.br_hip_gemm_pair_joined(ctypes.byref(a), ctypes.byref(b), None, None, hip.GEMM_F16, None, 0)
+              for a, b in (made, made[::-1])]
+    assert joined[0] == joined[1] == by_size
+    return by_size == wide
+
+
+@pytest.mark.parametrize("n,inn,out,wide", [(78, 1024, 4096, True), (200, 512, 2048, True), (32, 8192, 400, True), (256, 512, 2048, True),
+                                            # more tokens than outputs: K of the gradient is the longer one
+                                            (400, 8192, 32, False), (256, 8192, 32, False), (2048, 512, 128, False),
+                                            (4096, 512, 256, False), (1024, 4096, 64, False)])
+def test_wide_pairs_are_priced_with_the_weight_gradient_on_the_wide_tiles(n, inn, out, wide):
+    assert on_wide_tiles((1, 0, out, inn, n), (0, 0, n, inn, out)) == wide
+
+
+@pytest.mark.parametrize("t,hd", [(776, 64), (1024, 64), (1024, 128), (400, 64)])
+def test_a_heads_backward_products_keep_off_wide_tiles(t, hd):
+    assert not on_wide_tiles((1, 0, t, hd, t), (0, 1, t, t, hd))   # of the values and the scores
+    assert not on_wide_tiles((1, 0, t, hd, t), (0, 0, t, hd, t))   # of the keys and the queries
+
+
 @pytest.mark.parametrize("out", [(1 << 21) - 8, 1 << 21, (1 << 21) + 8, (1 << 26)])
 def test_linear_gelu_takes_wide_outputs(out):
     assert answer("br_hip_linear_gelu(4096, 8192, None, 1 << 40, 1 << 41, 2, 300, %d, 32, None)" % out) > 0

@@ -853,7 +853,7 @@ def run_pair(products, compute, sums=None, later=None):
         m, n, k = c.shape[1], c.shape[2], a.shape[1] if ta else a.shape[2]
         descs.append(hip.Product(ta, tb, m, n, k, 2.0, ptr(a), code[a.dtype], a.shape[2], a[0].numel(), ptr(b), code[b.dtype],
                                  b.shape[2], b[0].numel(), ptr(c), code[c.dtype], n, m * n, c.shape[0]))
-        sizes += [m, n, k, c.shape[0]]
+        sizes = sizes + [m, n, k, c.shape[0]] if tb or not ta else [m, n, k, c.shape[0]] + sizes   # the weight gradient's first
     first, second = (ctypes.byref(d) for d in descs)
     need = hip.load().br_hip_gemm_pair_workspace(first, second, compute)
     ws = torch.full((max(need, 16),), 0x7f, dtype=torch.uint8, device="cuda")
