@@ -358,8 +358,7 @@ __device__ __forceinline__ MaxSum combine(MaxSum a, MaxSum b) {
     const float m = fmaxf(a.m, b.m);
     MaxSum r;
     r.m = m;
-    // a side that has seen nothing carries m = -inf and s = 0
-    r.s = (a.m == -INFINITY ? 0.f : a.s * __expf(a.m - m)) + (b.m == -INFINITY ? 0.f : b.s * __expf(b.m - m));
+    r.s = a.s * __expf(a.m - m) + b.s * __expf(b.m - m);
     return r;
 }
 
@@ -368,13 +367,15 @@ __device__ __forceinline__ MaxSum combine(MaxSum a, MaxSum b) {
 // quads of a thread are on their way at a time: four where a CU has one row, one where others fill the time.
 template <int AHEAD>
 __device__ __forceinline__ float row_logsumexp(const float* __restrict__ lr, int64_t vocab, MaxSum* lds) {
+    // The lowest number rather than minus infinity: what is masked with the latter then adds nothing, also where a thread has met
+    // nothing else yet, and no difference is one of infinities.
     MaxSum t;
-    t.m = -INFINITY;
+    t.m = -FLT_MAX;
     t.s = 0.f;
     auto quad = [&](const float4& v) {
         const float m4 = fmaxf(fmaxf(v.x, v.y), fmaxf(v.z, v.w));
         if (m4 > t.m) {
-            t.s *= __expf(t.m - m4);  // exp(-inf) = 0 on the first vector
+            t.s *= __expf(t.m - m4);
             t.m = m4;
         }
         t.s += (__expf(v.x - t.m) + __expf(v.y - t.m)) + (__expf(v.z - t.m) + __expf(v.w - t.m));

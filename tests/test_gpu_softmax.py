@@ -129,10 +129,10 @@ def test_logsoftmax_nll_against_oracle(rows, vocab):
     assert np.array_equal(host(dl), g)
 
 
-@pytest.mark.parametrize("rows,vocab", [(9, 1), (9, 2), (9, 3), (7, 5), (6, 1023), (5, 4097), (8, 16389), (3, 16386), (4, 32003)])
+@pytest.mark.parametrize("rows,vocab", [(9, 1), (9, 2), (9, 3), (7, 5), (6, 1023), (5, 4097), (8, 16389), (3, 16386), (4, 32003), (300, 1003)])
 def test_logsoftmax_nll_of_rows_that_start_anywhere(rows, vocab):
     """A vocabulary that is no multiple of four: labels on the first and last values of rows, in quads and around them, rows
-    without one; four quads of a thread at a time and fewer.  fp32, in place, fp16, logits off 16-byte boundaries."""
+    without one; four quads of a thread at a time and (beyond 256 rows) one.  fp32, in place, fp16, logits off 16-byte boundaries."""
     rng = np.random.default_rng(vocab)
     logits = (2 * rng.standard_normal((rows, vocab))).astype(np.float32)
     target = np.array([[0, vocab - 1, vocab // 2, min(4, vocab - 1), max(vocab - 4, 0)][r % 5] for r in range(rows)], np.int32)
@@ -154,6 +154,39 @@ def test_logsoftmax_nll_of_rows_that_start_anywhere(rows, vocab):
     assert np.array_equal(host(room)[1:].reshape(rows, vocab), g)
     call("br_hip_logsoftmax_nll_bwd", ptr(dl), ptr(dt), ptr(dk), ptr(dlse), ptr(dl), F32, 1.0 / count, rows, vocab, stream())
     assert np.array_equal(host(dl), g)
+
+
+@pytest.mark.parametrize("low", [-np.inf, np.finfo(np.float32).min])
+@pytest.mark.parametrize("rows,vocab", [(5, 4097), (9, 32001), (4, 20000), (300, 1003), (300, 5002)])
+def test_logsoftmax_nll_of_masked_words(rows, vocab, low):
+    """Words masked with minus infinity or the lowest number: single ones, the row's first or last five, runs of quads at its start and
+    behind, all but the label.  Against 64 bits; four quads of a thread at a time (up to 256 rows) and one."""
+    rng = np.random.default_rng(vocab)
+    logits = (2 * rng.standard_normal((rows, vocab))).astype(np.float32)
+    target = np.full(rows, vocab // 2, np.int32)
+    for r in range(rows):
+        kind = r % 5
+        if kind == 0:
+            logits[r, rng.integers(0, vocab, 40)] = low
+        elif kind == 1:
+            logits[r, :5] = logits[r, -5:] = low
+        elif kind == 2:
+            logits[r, :vocab // 3] = low
+        elif kind == 3:
+            logits[r, vocab // 4: vocab // 2] = low
+        else:
+            logits[r] = low
+        logits[r, target[r]] = rng.standard_normal()
+    keep = np.ones(rows, np.int32)
+    x = logits.astype(np.float64)
+    top = x.max(1, keepdims=True)
+    want = (top + np.log(np.exp(x - top).sum(1, keepdims=True)))[:, 0]
+    grad = np.exp(x - want[:, None])
+    grad[np.arange(rows), target] -= 1
+    loss, count, lse, g, *_ = nll_run(logits, target, keep)
+    assert count == rows
+    assert_close(lse, want, RTOL, "lse")
+    assert_close(g, grad / rows, RTOL, "dlogits")
 
 
 def test_logsoftmax_nll_headline_shape_properties_and_sampled_rows():
