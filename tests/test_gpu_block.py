@@ -525,6 +525,51 @@ def test_fused_gelu_backward_linear_backward_equals_the_two_words(runtime, mode)
         env.close()
 
 
+@pytest.mark.parametrize("weights", ["native", "float"])
+@pytest.mark.parametrize("mode", ["f16", "bf16"])
+@pytest.mark.parametrize("t,hidden,mid,in_place", [(257, 512, 2048, False), (300, 512, 2048, True), (600, 512, 1024, False),
+                                                   (1000, 256, 1032, False), (1000, 256, 1032, True)])
+def test_fused_gelu_backward_linear_backward_of_many_rows(runtime, t, hidden, mid, in_place, mode, weights):
+    """From 257 rows on the bias gradient is left as partial sums, which are added up beside the two products, behind the staging of
+    x and of fp32 weights; in place, dx lands on the 16-bit x that dW reads, so that the products are two launches and the sums
+    one ahead of them.  The products' bits are those of the two words; the bias gradient is within the rounding of its
+    additions: of n partial sums of some sqrt(n) values each, four times 2^-24 n rms for the furthest of mid."""
+    assert hip.load().br_hip_gemm_pair_kernel(mid, hidden, t, 1, t, hidden, mid, 1, {"f16": hip.GEMM_F16, "bf16": hip.GEMM_BF16}[mode]) >= 0
+    rng = np.random.default_rng(t)
+    env = host.Env(1)
+    try:
+        env.execute("'%s' op.gemm_precision" % mode)
+        wdt, xdt = mode if weights == "native" else "float", mode if in_place else "float"
+        env.execute("1 %d %d 3 'cuda' 'float' op.create 'dy' !  1 %d %d 3 'cuda' 'float' op.create 'u' !" % (t, mid, t, mid))
+        env.execute("1 %d %d 3 'cuda' '%s' op.create 'x' !  1 %d %d 3 'cuda' '%s' op.create 'xg' !" % (t, hidden, xdt, t, hidden, xdt))
+        env.execute("%d %d 2 'cuda' '%s' op.create 'w' !  %d %d 2 'cuda' 'float' op.create 'wg' !" % (mid, hidden, wdt, mid, hidden))
+        env.execute("%d 1 'cuda' 'float' op.create 'bias' !  %d 1 'cuda' 'float' op.create 'bg' !" % (mid, mid))
+        u0, x0 = 1.5 * rng.standard_normal((1, t, mid)), rng.standard_normal((1, t, hidden))
+        env.write("dy", rng.standard_normal((1, t, mid)).astype(np.float32))
+        env.write("w", (0.05 * rng.standard_normal((mid, hidden))).astype(np.float32))
+        dx = "x" if in_place else "xg"
+        gelu = "'dy' @ 'u' @ 'u' @ op.gelu_backward"
+        lin = "'u' @ 'x' @ 'w' @ 'bias' @ '%s' @ 'wg' @ 'bg' @ op.linear_backward" % dx
+        assert "W:op.gelu_linear_backward" in env.disassemble(gelu + "  " + lin, fused=True)
+        got = []
+        for texts in ([gelu, lin], [gelu + "  " + lin], [gelu + "  " + lin]):
+            env.write("u", u0.astype(np.float32))
+            env.write("x", x0.astype(np.float32))
+            env.execute("'xg' @ op.zero 'wg' @ op.zero 'bg' @ op.zero")
+            for text in texts:
+                env.execute(text)
+            got.append({n: env.read(n) for n in ("u", dx, "wg", "bg")})
+        for n in ("u", dx, "wg"):
+            assert np.array_equal(got[0][n], got[1][n]), n
+        du = got[0]["u"][0].astype(np.float64)
+        bound = 4 * 2.0 ** -24 * t * np.sqrt(np.mean(du * du, 0))
+        for run in got:
+            assert np.all(np.abs(run["bg"] - du.sum(0)) <= bound)
+        assert np.array_equal(got[1]["bg"], got[2]["bg"])
+    finally:
+        env.close()
+
+
 @pytest.mark.parametrize("mode,hidden", [("f16", 256), ("bf16", 256), ("f32", 256), ("f16", 8192)])
 def test_fused_layernorm_backward_add_linear_backward_equals_the_two_words(runtime, mode, hidden):
     """The fusion pass turns `op.layernorm_backward_add op.linear_backward` (the post-attention LayerNorm's
