@@ -62,6 +62,13 @@ struct FlexTile {
     static constexpr int kBytes = ROWS * 128;
     static constexpr int kInstr = kBytes / (WORDS ? 256 : 1024);  // wave-wide loads of a tile
     static constexpr int kGranulesPerK = ROWS / kPer;             // row contiguous: granules of a k-row
+    // Loads whose offsets a lane holds.  Value by value there are up to 32 of an operand, and the 64 registers of a 64 x 64 tile
+    // left one wave to a SIMD: held are eight, the others' lie kFar rows (row contiguous: k-rows) and a multiple of it further on.
+    // All held / eight, us, operands off 16-byte boundaries: [987 x 4608] from K = 1152 131 / 89, [501 x 501] from 65, 16 products,
+    // 38.4 / 19.0, [700 x 2049] from 513 29.7 / 19.1; one tile to a CU the same to within 5 %.
+    static constexpr int kHeld = WORDS ? 8 : kInstr;
+    static constexpr int kFar = kHeld * (WORDS ? 16 : 64) / (KSTR ? kGranulesPerK : 8);
+    static_assert(kInstr % kHeld == 0, "whole sets of loads");
     static_assert(!WORDS || kSize == 4, "single values are fp32");
 
     // Row contiguous, where things lie in LDS.  16-bit: the transposing read of a fragment touches 4 k-rows x 64
@@ -310,25 +317,33 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
     const long long a_step = (A_KSTR ? g.lda : 1) * ((long long)kSize * KT * KW);
     const long long b_step = (B_KSTR ? g.ldb : 1) * ((long long)kSize * KT * KW);
     int k_left = k_end - k0;
-    unsigned a_off[TA::kInstr], b_off[TB::kInstr];
+    const long long a_far = (long long)kSize * TA::kFar * g.lda, b_far = (long long)kSize * TB::kFar * g.ldb;
+    unsigned a_off[TA::kHeld], b_off[TB::kHeld];
 #pragma unroll
-    for (int q = 0; q < TA::kInstr; q++) a_off[q] = TA::source_offset(q, lane, g.lda);
+    for (int q = 0; q < TA::kHeld; q++) a_off[q] = TA::source_offset(q, lane, g.lda);
 #pragma unroll
-    for (int q = 0; q < TB::kInstr; q++) b_off[q] = TB::source_offset(q, lane, g.ldb);
+    for (int q = 0; q < TB::kHeld; q++) b_off[q] = TB::source_offset(q, lane, g.ldb);
     lds_byte* const mem = (lds_byte*)lds_raw + wave * kWaveBytes;
     const unsigned mem0 = (unsigned)(unsigned long long)mem;
 
     auto issue = [&](int stage) {
-        const buffer_rsrc ra = buffer_from(a_src, a_left), rb = buffer_from(b_src, b_left);
         const unsigned dst = mem0 + (unsigned)stage * kStageBytes;
         // a k-contiguous operand's last step: chunks past K are fetched from past the end of the operand
         const bool tail = k_left < KT;
 #pragma unroll
-        for (int q = 0; q < TA::kInstr; q++)
-            TA::load(dst, q, !A_KSTR && tail && TA::k_of(q, lane) >= k_left ? kPastEnd : a_off[q], ra);
+        for (int s = 0; s < TA::kInstr / TA::kHeld; s++) {
+            const buffer_rsrc r = buffer_from(a_src + s * a_far, a_left - s * a_far);
 #pragma unroll
-        for (int q = 0; q < TB::kInstr; q++)
-            TB::load(dst + TA::kBytes, q, !B_KSTR && tail && TB::k_of(q, lane) >= k_left ? kPastEnd : b_off[q], rb);
+            for (int q = 0; q < TA::kHeld; q++)
+                TA::load(dst, s * TA::kHeld + q, !A_KSTR && tail && TA::k_of(q, lane) >= k_left ? kPastEnd : a_off[q], r);
+        }
+#pragma unroll
+        for (int s = 0; s < TB::kInstr / TB::kHeld; s++) {
+            const buffer_rsrc r = buffer_from(b_src + s * b_far, b_left - s * b_far);
+#pragma unroll
+            for (int q = 0; q < TB::kHeld; q++)
+                TB::load(dst + TA::kBytes, s * TB::kHeld + q, !B_KSTR && tail && TB::k_of(q, lane) >= k_left ? kPastEnd : b_off[q], r);
+        }
         a_src += a_step; a_left -= a_step;
         b_src += b_step; b_left -= b_step;
         k_left -= KT * KW;
@@ -473,7 +488,7 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
 }
 
 template <int CT, int BM, int BN, int KW, int ST, bool A_KSTR, bool B_KSTR, typename TC, bool GELU = false, bool WORDS = false>
-__global__ __launch_bounds__(KW * 64, CT == BR_GEMM_F32 && !WORDS ? 2 : 1) void gemm_flex_kernel(GemmArgs g) {
+__global__ __launch_bounds__(KW * 64, CT == BR_GEMM_F32 ? 2 : 1) void gemm_flex_kernel(GemmArgs g) {
     __shared__ __attribute__((aligned(1024))) unsigned char lds[flex_lds_bytes<BM, BN, KW, ST>()];
     touch_args(g);
     flex_product<CT, BM, BN, KW, ST, A_KSTR, B_KSTR, TC, GELU, WORDS, true>(g, blockIdx.x, gridDim.x, lds);
