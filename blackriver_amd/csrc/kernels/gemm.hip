@@ -420,6 +420,14 @@ extern "C" int br_hip_gemm_kernel(int trans_a, int trans_b, int64_t m, int64_t n
     return plan.kernel;
 }
 
+extern "C" int br_hip_gemm_fp32_kernel(int64_t m, int64_t n, int64_t k, int64_t batch, int* waves) {
+    if (m <= 0 || n <= 0 || k <= 0 || batch <= 0) return BR_ERR_ATTR;
+    if (!waves) return BR_ERR_OUTPUT;
+    const int kernel = gemm16::fp32_kernel(m, n, k, batch);
+    *waves = gemm16::fp32_waves(kernel, m, n, k, batch);
+    return kernel;
+}
+
 extern "C" int br_hip_linear_gelu(const void* x, const void* w, const float* bias, void* u, void* y, int dtype,
                                   int64_t rows, int64_t out, int64_t in, br_stream_t stream) {
     if (rows < 0 || out <= 0 || in <= 0) return BR_ERR_ATTR;

@@ -163,13 +163,22 @@ struct Fp32Cost {
     double start, step, load, merge;
 };
 constexpr Fp32Cost kFp32Cost64{4.21, 1.542, 1.341, 1.62}, kFp32Cost32x64{3.83, 0.83, 0.796, 0.61}, kFp32Cost32{3.38, 0.60, 0.509, 0.27};
-// 32 x 32 tiles of at most one to a CU: from here on K is dealt to eight waves instead of four (0.51 us per step of four)
+// Waves that walk along K.  Where a CU has at most one workgroup of the small tiles they are eight, two to a SIMD.  Four / eight, us:
+// 32 x 32 tiles, [200 x 768] from 512 7.6 / 6.7, [64 x 2048] from 8192 49 / 37, value by value [31 x 1025] from 1025 12.1 / 9.2;
+// 32 x 64 tiles, [500 x 520] from 512 8.6 / 7.5, 1024 11.8 / 10.7, 2048 20.7 / 16.6, 8192 69.5 / 56.3, [512 x 1024], a workgroup to
+// each CU, 9.4 / 8.8, 13.8 / 12.9, 23.5 / 20.0, 76.5 / 69.9, value by value [333 x 1025] from 1025 17.7 / 13.3.  Below 512 a wave has less
+// than a step; with more tiles than CUs eight are 5-40 % slower.  (The price of 32 x 64 tiles is that of four: no choice among 142
+// products would be another with eight at 0.8 to 1 of it.)
 constexpr long long kFp32EightWaves = 512;
+inline int fp32_waves(int kernel, long long m, long long n, long long k, long long batch) {
+    if (kernel != kFlex32 && kernel != kFlex32x64) return 4;
+    return k >= kFp32EightWaves && ceil_div(m, kCost[kernel].bm) * ceil_div(n, kCost[kernel].bn) * batch <= 256 ? 8 : 4;
+}
 inline double fp32_us(int kernel, long long m, long long n, long long k, long long batch) {
     const KernelCost& c = kCost[kernel];
     const Fp32Cost& f = kernel == kFlex64 ? kFp32Cost64 : kernel == kFlex32x64 ? kFp32Cost32x64 : kFp32Cost32;
     const double per_cu = (double)(ceil_div(m, c.bm) * ceil_div(n, c.bn) * batch) / 256.0;
-    const double step = kernel == kFlex32 && per_cu <= 1.0 && k >= kFp32EightWaves ? 0.51 : f.step;
+    const double step = kernel == kFlex32 && fp32_waves(kernel, m, n, k, batch) == 8 ? 0.51 : f.step;
     const double load = f.load * (per_cu < 4.0 ? ceil(per_cu) : per_cu);
     return f.start + (double)ceil_div(ceil_div(k, 32), 4) * (load > step ? load : step) + f.merge * per_cu;
 }

@@ -118,6 +118,7 @@ SIGNATURES = {
     "br_hip_gemm_pair_joined": (_int, [_vp, _vp, _vp, _vp, _int, _vp, ctypes.c_size_t]),
     "br_hip_gemm_pair_kernel": (_int, [_i64] * 8 + [_int]),
     "br_hip_gemm_kernel": (_int, [_int, _int, _i64, _i64, _i64, _int, _i64, _int, ctypes.POINTER(_int)]),
+    "br_hip_gemm_fp32_kernel": (_int, [_i64, _i64, _i64, _i64, ctypes.POINTER(_int)]),
     "br_hip_flash_attn_fwd": (_int, [_vp, _vp, _vp, _int, _vp, _vp, _vp, _vp] + [_i64] * 9 + [_vp]),
     "br_hip_flash_attn_bwd": (_int, [_vp] * 5 + [_int] + [_vp] * 7 + [_int] + [_i64] * 9 + [_vp]),
     "br_hip_adamw": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _i64, _f32, _f32, _f32, _f32, _f32, _i64, _vp]),
@@ -163,6 +164,14 @@ def gemm_kernel(trans_a, trans_b, m, n, k, c_dtype=F32, batch=1, staged=False):
     code = load().br_hip_gemm_kernel(trans_a, trans_b, m, n, k, c_dtype, batch, int(staged), ctypes.byref(slices))
     check(min(code, 0), "br_hip_gemm_kernel")
     return GEMM_KERNELS[code], slices.value
+
+
+def gemm_fp32_kernel(m, n, k, batch=1):
+    """(kernel, waves along K) of an fp32 product: see br_hip_gemm_fp32_kernel."""
+    waves = _int(0)
+    code = load().br_hip_gemm_fp32_kernel(m, n, k, batch, ctypes.byref(waves))
+    check(min(code, 0), "br_hip_gemm_fp32_kernel")
+    return GEMM_KERNELS[code], waves.value
 
 
 def check(code: int, what: str = "") -> None:

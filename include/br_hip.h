@@ -478,6 +478,9 @@ enum {
 };
 int br_hip_gemm_kernel(int trans_a, int trans_b, int64_t m, int64_t n, int64_t k, int c_dtype, int64_t batch,
                        int staged, int* slices);
+/* ... and a BR_GEMM_F32 product, with the number of waves that walk along K, where
+ * rows lie close enough for 32-bit offsets. */
+int br_hip_gemm_fp32_kernel(int64_t m, int64_t n, int64_t k, int64_t batch, int* waves);
 
 /* op_linear followed by op_gelu (cuda_tensor.cpp:146-193 and :400-412; the pair
  * of bloomz-7b/train.words:188-189) in one product whose epilogue writes both

@@ -31,6 +31,18 @@ PLANNED = [
 ]
 
 
+# (kernel, waves along K, m, n, k, batch): fp32 products that reach every kernel in each of its forms -- K of one walk's parts added
+# apart (up to 256 k-values a wave) and folded, whole and partial steps, sizes that are loaded in quads and value by value
+FP32_PLANNED = [
+    ("flex 32", 4, 33, 36, 40, 2), ("flex 32", 4, 31, 65, 7, 2), ("flex 32", 4, 520, 1028, 1024, 1), ("flex 32", 4, 1000, 1100, 2120, 1),
+    ("flex 32", 8, 200, 768, 512, 1), ("flex 32", 8, 31, 1025, 1025, 1), ("flex 32", 8, 64, 256, 4100, 1),
+    ("flex 32x64", 4, 1000, 1028, 36, 4), ("flex 32x64", 4, 501, 501, 65, 16), ("flex 32x64", 4, 1000, 2100, 2100, 1),
+    ("flex 32x64", 8, 500, 520, 512, 1), ("flex 32x64", 8, 333, 1025, 1025, 1), ("flex 32x64", 8, 500, 520, 2052, 1),
+    ("flex 64", 4, 500, 2049, 200, 4), ("flex 64", 4, 500, 4096, 516, 1), ("flex 64", 4, 500, 2048, 1025, 2), ("flex 64", 4, 500, 2048, 2052, 1),
+    ("128", 4, 512, 512, 72, 48), ("128", 4, 256, 384, 65, 128),
+]
+
+
 def answer(call):
     """Return code of `L.<call>`, made without a GPU."""
     env = dict(os.environ, HIP_VISIBLE_DEVICES="-1", ROCR_VISIBLE_DEVICES="-1")
@@ -77,6 +89,22 @@ def test_gemm_plan_reaches_every_kernel(kernel, slices, m, n, k, batch):
     from blackriver_amd import hip
     assert hip.gemm_kernel(0, 1, m, n, k, batch=batch, staged=True) == (kernel, slices)
     assert {kernel for kernel, *_ in PLANNED} == set(hip.GEMM_KERNELS)
+
+
+@pytest.mark.parametrize("kernel,waves,m,n,k,batch", FP32_PLANNED)
+def test_fp32_products_run_on(kernel, waves, m, n, k, batch):
+    from blackriver_amd import hip
+    assert hip.gemm_fp32_kernel(m, n, k, batch) == (kernel, waves)
+
+
+@pytest.mark.parametrize("m,n", [(512, 1024), (32, 16384), (2048, 256), (513, 992)])
+def test_eight_waves_walk_along_k_where_a_cu_has_one_small_tile(m, n):
+    """Up to 256 of the small tiles, from a K of 512 on."""
+    from blackriver_amd import hip
+    for k in (511, 512, 1024, 3071, 3072, 8192):
+        kernel, waves = hip.gemm_fp32_kernel(m, n, k)
+        tiles = -(-m // 32) * -(-n // {"flex 32": 32, "flex 32x64": 64}[kernel])
+        assert waves == (8 if k >= 512 and tiles <= 256 else 4)
 
 
 @pytest.mark.parametrize("n,inn,out,name", [(64, 2048, 6144, "flex 32"), (200, 2048, 2048, "flex 32x64"), (250, 2048, 3072, None),

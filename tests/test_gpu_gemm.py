@@ -12,7 +12,7 @@ import torch
 from conftest import assert_close
 from gpu_util import BF16, F16, F32, call, dev, empty, host, ptr, stream
 from blackriver_amd import hip
-from test_entry_point_checks import PLANNED
+from test_entry_point_checks import FP32_PLANNED, PLANNED
 
 pytestmark = pytest.mark.gpu
 
@@ -539,11 +539,11 @@ def test_gemm_every_kernel_is_exact_on_integers(ta, tb, kernel, slices, m, n, k,
     (33, 36, 40, 2),         # 32 x 32 tiles, rows in 16-byte granules
     (64, 1024, 260, 1),      # K dealt unevenly to the four waves
     (512, 1028, 1024, 1),    # 32 x 64 tiles
-    (1000, 1028, 36, 4),     # 64 x 64 tiles
+    (1000, 1028, 36, 4),     # 32 x 64 tiles, many of them
     (31, 65, 7, 2),          # value by value: everything odd
     (333, 64, 333, 3),       # attention products of 333 tokens
-    (1001, 2050, 70, 2),     # 64 x 64 tiles, value by value
-    (128, 128, 128, 512),    # 128 x 128 tiles: a short K and 512 whole tiles
+    (1001, 2050, 70, 2),     # 32 x 64 tiles, value by value
+    (128, 128, 128, 512),
     (256, 384, 68, 90),
 ])
 def test_gemm_fp32_small_tiles_are_exact_on_integers(ta, tb, m, n, k, batch):
@@ -557,6 +557,13 @@ def test_gemm_fp32_small_tiles_are_exact_on_integers(ta, tb, m, n, k, batch):
     c0 = rng.integers(-9, 10, (batch, m, n)).astype(np.float32)
     got, ref = run_gemm(ta, tb, m, n, k, a, b, F32, F32, F32, hip.GEMM_F32, batch=batch, bias=bias, c0=c0)
     assert np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("kernel,waves,m,n,k,batch", FP32_PLANNED)
+def test_gemm_every_fp32_kernel_is_exact_on_integers(ta, tb, kernel, waves, m, n, k, batch):
+    assert hip.gemm_fp32_kernel(m, n, k, batch) == (kernel, waves)
+    test_gemm_fp32_small_tiles_are_exact_on_integers(ta, tb, m, n, k, batch)
 
 
 @pytest.mark.parametrize("wide", ["a", "b"])
@@ -586,7 +593,7 @@ def test_gemm_fp32_rows_far_apart(ta, tb, wide):
                                    (64, 256, 2052), (512, 1024, 3072),
                                    (64, 256, 4096), (64, 256, 4100), (1000, 1100, 2120), (31, 65, 2049)])
 def test_gemm_fp32_error_against_64_bits(m, n, k):
-    """Products as sums of bf16 parts: apart and folded, four waves and eight, every tile, values one by one.  Rounding sums of 64
+    """Products as sums of bf16 parts: apart and folded, four waves and eight, tiles of 32 rows, values one by one.  Rounding sums of 64
     products of random sign to 24 bits one after the other leaves 2^-25 sqrt(64 / 2) = 1.7e-7 of the result."""
     print("case m=%d n=%d k=%d" % (m, n, k), flush=True)
     torch.manual_seed(k)
@@ -597,6 +604,23 @@ def test_gemm_fp32_error_against_64_bits(m, n, k):
              hip.GEMM_F32, stream())
         want = (a.t() if ta else a).double().contiguous() @ (b.t() if tb else b).double().contiguous()
         assert ((c - want).norm() / want.norm()).item() <= 2.0e-7
+
+
+@pytest.mark.parametrize("front", [0, 1])   # values in front of A: 1 puts it off 16-byte boundaries
+@pytest.mark.parametrize("ta,tb", [(0, 1), (0, 0), (1, 0), (1, 1)])
+@pytest.mark.parametrize("kernel,waves,m,n,k,batch", FP32_PLANNED)
+def test_gemm_every_fp32_kernel_against_64_bits(kernel, waves, m, n, k, batch, ta, tb, front):
+    """The bound of test_gemm_fp32_error_against_64_bits; 128 x 128 tiles add up K one after the other, of at most 80 values."""
+    assert hip.gemm_fp32_kernel(m, n, k, batch) == (kernel, waves)
+    print("case ta=%d tb=%d m=%d n=%d k=%d batch=%d front=%d" % (ta, tb, m, n, k, batch, front), flush=True)
+    torch.manual_seed(k)
+    buf, b = torch.randn(front + batch * m * k, device="cuda"), torch.randn((batch, n, k) if tb else (batch, k, n), device="cuda")
+    a = buf[front:].view((batch, k, m) if ta else (batch, m, k))
+    c = torch.full((batch, m, n), float("nan"), device="cuda")
+    call("br_hip_gemm", ta, tb, m, n, k, 1.0, ptr(a), F32, a.shape[2], m * k, ptr(b), F32, b.shape[2], n * k, 0, ptr(c), F32, n, m * n, None,
+         batch, hip.GEMM_F32, stream())
+    want = torch.stack([(x.t() if ta else x).double().contiguous() @ (y.t() if tb else y).double().contiguous() for x, y in zip(a, b)])
+    assert ((c - want).norm() / want.norm()).item() <= 2.0e-7
 
 
 @pytest.mark.parametrize("k", [40, 512, 2100])
@@ -627,8 +651,16 @@ def test_gemm_fp32_values_that_parts_do_not_hold(m, n, k):
             assert ((got[20] - want[20])[both].norm() / want[20][both].norm()).item() <= 2.0e-7
 
 
-# 32 x 32 tiles (four waves, eight), 32 x 64, 64 x 64, apart and folded
-FP32_SIZES = [(32, 64, 40), (200, 768, 512), (1000, 2100, 2100), (500, 4100, 516), (500, 4100, 1032)]
+# 32 x 32 tiles (four waves, eight), 32 x 64 (four, eight) and 64 x 64, apart and folded; sizes that are loaded value by value too
+FP32_SIZES = [(32, 64, 40), (200, 768, 512), (500, 4100, 516), (1000, 2100, 2100), (500, 520, 512), (500, 520, 2052), (500, 4096, 516),
+              (500, 2048, 2052)]
+
+
+@pytest.mark.parametrize("kernel,m,n,k", [("flex 32x64", 333, 1025, 1025), ("flex 32x64", 500, 520, 2052), ("flex 64", 500, 4096, 333),
+                                          ("flex 64", 500, 4096, 516), ("flex 64", 500, 2048, 2052), ("flex 64", 500, 2048, 2053)])
+def test_gemm_fp32_values_that_parts_do_not_hold_on_the_larger_tiles(kernel, m, n, k):
+    assert hip.gemm_fp32_kernel(m, n, k)[0] == kernel
+    test_gemm_fp32_values_that_parts_do_not_hold(m, n, k)
 
 
 @pytest.mark.parametrize("front", [0, 1])   # values in front of A: 1 puts it off 16-byte boundaries
@@ -1030,10 +1062,10 @@ def test_sums_beside_two_products_keep_their_order_where_they_meet(over, compute
 @pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16, hip.GEMM_F32])
 @pytest.mark.parametrize("rows,out,inn,x_dt,y_dt", [
     (24, 256, 256, F32, F32), (65, 40, 72, None, None), (130, 1000, 136, None, F32), (1000, 1024, 64, F32, F32), (1000, 2048, 256, None, F32),
-    (2100, 1280, 128, F32, None), (33, 30, 20, F32, F32), (512, 2048, 2048, None, None)])   # the last in fp32: one by one
+    (2100, 1280, 128, F32, None), (33, 30, 20, F32, F32), (512, 2048, 2048, None, None)])
 def test_linear_group_is_exact_on_integers(rows, out, inn, x_dt, y_dt, compute):
-    """Three layers of one x as a batch (or, fp32, where that is slower, one after the other), each with a bias of its own; the kernels of small and of large tiles, sizes that
-    are no multiple of a granule among them."""
+    """Three layers of one x as a batch, each with a bias of its own; the kernels of small and of large tiles, sizes that are no multiple
+    of a granule among them."""
     dt = COMPUTE_T[compute]
     print("case rows=%d out=%d in=%d compute=%d" % (rows, out, inn, compute), flush=True)
     torch.manual_seed(rows)
