@@ -26,15 +26,17 @@ struct ColumnSums {
 };
 constexpr int kSumLanes = 8;   // 16-byte granules of a row one workgroup sums
 
-template <int CT, int THREADS>
+// The workgroup's first four waves add up the rows, whatever it has: with the rows dealt to eight waves, whose sums meet one after
+// the other, the result was up to 8 % further from 64 bits ([2048] from 200 rows 1.87e-8, from four waves 1.79e-8).
+template <int CT>
 __device__ __forceinline__ void sum_strip(const ColumnSums& s, int strip, float* lds) {
-    constexpr int kVec = CT == BR_GEMM_F32 ? 4 : 8, kRows = THREADS / kSumLanes, kAhead = 4;
+    constexpr int kVec = CT == BR_GEMM_F32 ? 4 : 8, kThreads = 256, kRows = kThreads / kSumLanes, kAhead = 4;
     const int lane = threadIdx.x % kSumLanes, first = threadIdx.x / kSumLanes;
     const int col = (strip * kSumLanes + lane) * kVec;
     float acc[kVec];
 #pragma unroll
     for (int j = 0; j < kVec; j++) acc[j] = 0.f;
-    if (col < s.cols) {
+    if (threadIdx.x < kThreads && col < s.cols) {
         const u32x4* x = static_cast<const u32x4*>(s.x) + col / kVec;
         const int pitch = s.cols / kVec;
         for (int r = first; r < s.rows; r += kAhead * kRows) {
@@ -66,7 +68,7 @@ __device__ __forceinline__ void sum_strip(const ColumnSums& s, int strip, float*
 #pragma unroll
         for (int j = 0; j < kVec; j++) acc[j] += __shfl_xor(acc[j], d);
     constexpr int kWidth = kSumLanes * kVec;
-    if ((threadIdx.x & 63) < kSumLanes) {
+    if (threadIdx.x < kThreads && (threadIdx.x & 63) < kSumLanes) {
 #pragma unroll
         for (int j = 0; j < kVec; j++) lds[(threadIdx.x >> 6) * kWidth + lane * kVec + j] = acc[j];
     }
@@ -75,7 +77,7 @@ __device__ __forceinline__ void sum_strip(const ColumnSums& s, int strip, float*
     if (threadIdx.x < kWidth && at < s.cols) {
         float sum = lds[threadIdx.x];
 #pragma unroll
-        for (int w = 1; w < THREADS / 64; w++) sum += lds[w * kWidth + threadIdx.x];
+        for (int w = 1; w < kThreads / 64; w++) sum += lds[w * kWidth + threadIdx.x];
         s.out[at] = sum * s.scale;
     }
 }
@@ -133,7 +135,7 @@ __global__ __launch_bounds__(KW * 64, CT == BR_GEMM_F32 ? 2 : 1) void gemm_flex_
     const unsigned id = blockIdx.x;
     if (id < n1) flex_product<CT, BM, BN, KW, ST, AK1, BK1, TC1, false, false, false>(a, id, n1, lds);
     else if (id < n1 + n2) flex_product<CT, BM, BN, KW, ST, AK2, BK2, TC2, false, false, false>(b, id - n1, n2, lds);
-    else if (id < n1 + n2 + n3) sum_strip<CT, KW * 64>(sums, (int)(id - n1 - n2), reinterpret_cast<float*>(lds));
+    else if (id < n1 + n2 + n3) sum_strip<CT>(sums, (int)(id - n1 - n2), reinterpret_cast<float*>(lds));
     else add_partials<KW * 64>(later, (int)(id - n1 - n2 - n3), reinterpret_cast<flex_f32x4*>(lds));
 }
 
@@ -303,7 +305,7 @@ __global__ __launch_bounds__(512, 4) void gemm_wide_pair_kernel(GemmArgs x, Gemm
     const unsigned id = blockIdx.x;
     if (id < nx) flex_product<CT, 32, 32, 8, 1, false, BK2, TC2, false, false, false>(x, id, nx, lds);
     else if (id < nx + nw) wide_product<CT>(w, id - nx, nw, lds);
-    else if (id < nx + nw + n3) sum_strip<CT, 512>(sums, (int)(id - nx - nw), reinterpret_cast<float*>(lds));
+    else if (id < nx + nw + n3) sum_strip<CT>(sums, (int)(id - nx - nw), reinterpret_cast<float*>(lds));
     else add_partials<512>(later, (int)(id - nx - nw - n3), reinterpret_cast<flex_f32x4*>(lds));
 }
 

@@ -975,6 +975,34 @@ def test_weight_gradients_on_wide_tiles_are_as_precise_as_on_small_ones(n, inn, 
     assert ((dw - want).norm() / want.norm()).item() <= 0.65 * 2.0 ** -24 * math.sqrt(variance)
 
 
+def sums_of_four_waves(x):
+    """Column sums in fp32 in the order that four waves of 8 rows at a time have: every 32nd row one after the other, the 8 rows of a wave
+    by halves, the waves one after the other."""
+    slots = np.zeros((32, x.shape[1]), np.float32)
+    for first in range(0, x.shape[0], 32):
+        rows = x[first:first + 32]
+        slots[:len(rows)] += rows
+    while len(slots) > 4:
+        slots = slots[0::2] + slots[1::2]
+    return ((slots[0] + slots[1]) + slots[2]) + slots[3]
+
+
+@pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16])
+@pytest.mark.parametrize("n,inn,out", [(1, 1024, 1024), (33, 1024, 4096), (78, 1024, 4096), (200, 512, 2048), (300, 1024, 4096), (78, 256, 264)])
+def test_column_sums_beside_two_products_have_one_order(n, inn, out, compute):
+    """Beside wide tiles as beside small ones (the last): the bits of four waves' sums."""
+    dt = COMPUTE_T[compute]
+    print("case n=%d in=%d out=%d compute=%d" % (n, inn, out, compute), flush=True)
+    assert (hip.load().br_hip_gemm_pair_kernel(out, inn, n, 1, n, inn, out, 1, compute) == 10) == (out > 264)   # BR_GEMM_PAIR_WIDE
+    torch.manual_seed(n)
+    dy, x, w = (torch.randn(s, device="cuda").to(TORCH_T[dt]) for s in ((1, n, out), (1, n, inn), (1, out, inn)))
+    dw, dx, db = (torch.empty(s, device="cuda") for s in ((1, out, inn), (1, n, inn), (out,)))
+    need = hip.load().br_hip_colsum_workspace(n, out)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    assert run_pair([(1, 0, dy, x, dw), (0, 0, dy, w, dx)], compute, hip.ColumnSums(ptr(dy), dt, ptr(db), n, out, 1.0, ptr(ws), need))
+    assert np.array_equal(host(db), sums_of_four_waves(host(dy[0].float())))
+
+
 @pytest.mark.parametrize("compute", [hip.GEMM_F16, hip.GEMM_BF16, hip.GEMM_F32])
 @pytest.mark.parametrize("n", [64, 700])   # one launch, and (16-bit) two after the sums
 @pytest.mark.parametrize("arrays,parts,cols", [(2, 1, 4), (3, 7, 68), (3, 39, 256), (2, 64, 1000), (3, 65, 60), (3, 256, 4096)])
