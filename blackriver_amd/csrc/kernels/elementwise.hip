@@ -955,12 +955,18 @@ __global__ __launch_bounds__(kOwnThreads) void pack_colsum_kernel(PackSet set, f
         for (int j = 0; j < VEC; j++) slots[threadIdx.x >> 6][lr * VEC + j] = acc[j];
     }
     __syncthreads();
+    // The waves' sums meet in pairs: one after the other, sixteen of them are most of a result's error ([1024] from 300 rows against
+    // 64 bits 9.9e-8, so 7.9e-8; [2048] from 1024 1.06e-7, 9.1e-8).
     if (threadIdx.x < CW) {
-        float z = 0.f;
+        float z[WAVES];
 #pragma unroll
-        for (int k = 0; k < WAVES; k++) z += slots[k][threadIdx.x];
+        for (int k = 0; k < WAVES; k++) z[k] = slots[k][threadIdx.x];
+#pragma unroll
+        for (int half = WAVES / 2; half > 0; half /= 2)
+#pragma unroll
+            for (int k = 0; k < half; k++) z[k] += z[k + half];
         const int64_t oc = strip * CW + threadIdx.x;
-        if (oc < cols) out[oc] = z * scale;
+        if (oc < cols) out[oc] = z[0] * scale;
     }
 }
 template <typename D>

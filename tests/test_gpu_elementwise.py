@@ -171,6 +171,29 @@ def test_pack_colsum_is_exact_on_integers(rows, cols, count, dtype):
     assert torch.equal(packed.float(), want) and torch.equal(out, 0.5 * want.sum(0))
 
 
+@pytest.mark.parametrize("rows,cols", [(100, 1024), (300, 512), (300, 1024), (512, 2048), (1000, 1024), (1024, 2048), (2000, 768)])
+def test_pack_colsum_against_64_bits(rows, cols):
+    """A thread adds up its rows, a wave's threads and then sixteen waves meet in pairs.  Each addition is off by up to 0.5 x 2^-24 of
+    the sum it leaves (2-norm over sums of random sign), whose variance is the number of rows in it; the widest strips, 8 quads,
+    leave the most rows to a thread.  Waves that met one after the other would be over the bound at 300 to 1024 rows."""
+    torch.manual_seed(rows)
+    parts, additions = [len(range(r, rows, 128)) for r in range(128)], 0
+    additions += sum(sum(range(2, n + 1)) for n in parts)
+    while len(parts) > 1:
+        pairs = list(zip(parts[0::2], parts[1::2]))
+        additions += sum(a + b for a, b in pairs if a and b)
+        parts = [a + b for a, b in pairs]
+    off = want = 0.0
+    for _ in range(3):
+        x = [torch.randn((rows, cols), device="cuda") for _ in range(3)]
+        out, packed = torch.empty((3, cols), device="cuda"), torch.empty((rows, 3 * cols), dtype=torch.float16, device="cuda")
+        call("br_hip_pack_colsum", (ctypes.c_void_p * 3)(*(t.data_ptr() for t in x)), 3, ptr(out), ptr(packed), F16, rows, cols, 1.0, stream())
+        torch.cuda.synchronize()
+        sums = torch.stack([t.double().sum(0) for t in x])
+        off, want = off + (out - sums).square().sum().item(), want + sums.square().sum().item()
+    assert (off / want) ** 0.5 <= 0.5 * 2.0 ** -24 * (additions / rows) ** 0.5
+
+
 @pytest.mark.parametrize("rows,cols", [(2048, 4096), (77, 130), (1, 8), (512, 4096), (1000, 3080)])
 def test_colsum(rows, cols):
     rng = np.random.default_rng(6)
