@@ -17,6 +17,7 @@ import torch
 import oracle as orc
 from oracle import bloom_block as blk
 from conftest import assert_close, print_ledger
+from gpu_util import call, dev, empty, host as gpu_host, ptr, stream
 from blackriver_amd import hip, host
 
 pytestmark = pytest.mark.gpu
@@ -527,10 +528,10 @@ def test_fused_gelu_backward_linear_backward_equals_the_two_words(runtime, mode)
 
 @pytest.mark.parametrize("weights", ["native", "float"])
 @pytest.mark.parametrize("mode", ["f16", "bf16"])
-@pytest.mark.parametrize("t,hidden,mid,in_place", [(257, 512, 2048, False), (300, 512, 2048, True), (600, 512, 1024, False),
+@pytest.mark.parametrize("t,hidden,mid,in_place", [(257, 512, 2056, False), (300, 512, 2304, True), (449, 512, 2048, False), (600, 512, 1024, False),
                                                    (1000, 256, 1032, False), (1000, 256, 1032, True)])
 def test_fused_gelu_backward_linear_backward_of_many_rows(runtime, t, hidden, mid, in_place, mode, weights):
-    """From 257 rows on the bias gradient is left as partial sums, which are added up beside the two products, behind the staging of
+    """From 257 rows on (449 of up to 2048 columns) the bias gradient is left as partial sums, which are added up beside the two products, behind the staging of
     x and of fp32 weights; in place, dx lands on the 16-bit x that dW reads, so that the products are two launches and the sums
     one ahead of them.  The products' bits are those of the two words; the bias gradient is within the rounding of its
     additions: of n partial sums of some sqrt(n) values each, four times 2^-24 n rms for the furthest of mid."""
@@ -568,6 +569,40 @@ def test_fused_gelu_backward_linear_backward_of_many_rows(runtime, t, hidden, mi
         assert np.array_equal(got[1]["bg"], got[2]["bg"])
     finally:
         env.close()
+
+
+@pytest.mark.parametrize("mode", ["f16", "bf16"])
+@pytest.mark.parametrize("t,hidden,mid", [(256, 512, 4096), (257, 512, 2048), (288, 512, 2048), (448, 512, 2048), (448, 256, 1032)])
+def test_fused_gelu_backward_linear_backward_of_fewer_rows_owns_its_column_sums(runtime, t, hidden, mid, mode):
+    """Where the GELU's pass rounds its column sums less often than partial sums beside the products would, the bias gradient has
+    that pass's bits."""
+    compute, dt = {"f16": (hip.GEMM_F16, hip.F16), "bf16": (hip.GEMM_BF16, hip.BF16)}[mode]
+    assert hip.load().br_hip_gemm_pair_kernel(mid, hidden, t, 1, t, hidden, mid, 1, compute) >= 0
+    rng = np.random.default_rng(t)
+    dy, u = (rng.standard_normal((1, t, mid)).astype(np.float32) for _ in range(2))
+    env = host.Env(1)
+    try:
+        env.execute("'%s' op.gemm_precision" % mode)
+        env.execute("1 %d %d 3 'cuda' 'float' op.create 'dy' !  1 %d %d 3 'cuda' 'float' op.create 'u' !" % (t, mid, t, mid))
+        env.execute("1 %d %d 3 'cuda' 'float' op.create 'x' !  1 %d %d 3 'cuda' 'float' op.create 'xg' !" % (t, hidden, t, hidden))
+        env.execute("%d %d 2 'cuda' '%s' op.create 'w' !  %d %d 2 'cuda' 'float' op.create 'wg' !" % (mid, hidden, mode, mid, hidden))
+        env.execute("%d 1 'cuda' 'float' op.create 'bias' !  %d 1 'cuda' 'float' op.create 'bg' !" % (mid, mid))
+        env.write("dy", dy)
+        env.write("u", u)
+        env.write("x", rng.standard_normal((1, t, hidden)).astype(np.float32))
+        env.write("w", (0.05 * rng.standard_normal((mid, hidden))).astype(np.float32))
+        text = "'dy' @ 'u' @ 'u' @ op.gelu_backward  'u' @ 'x' @ 'w' @ 'bias' @ 'xg' @ 'wg' @ 'bg' @ op.linear_backward"
+        assert "W:op.gelu_linear_backward" in env.disassemble(text, fused=True)
+        env.execute(text)
+        got = env.read("bg")
+    finally:
+        env.close()
+    d = [dev(dy[0]), dev(u[0])]
+    du, du16, bg = empty((t, mid)), empty((t, mid), torch.float16), empty(mid)
+    need = hip.load().br_hip_colsum_workspace(t, mid)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device="cuda")
+    call("br_hip_gelu_bwd_colsum_cast", ptr(d[0]), ptr(d[1]), ptr(du), ptr(bg), ptr(du16), dt, t, mid, 1.0, ptr(ws), need, stream())
+    assert np.array_equal(got, gpu_host(bg))
 
 
 @pytest.mark.parametrize("mode,hidden", [("f16", 256), ("bf16", 256), ("f32", 256), ("f16", 8192)])
