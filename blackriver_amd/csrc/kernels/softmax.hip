@@ -567,8 +567,16 @@ void launch_nll_bwd(const float* logits, const int32_t* target, const int32_t* k
                     float scale, int64_t rows, int64_t vocab, bool aligned, hipStream_t st) {
     const bool vec_ok = aligned && vocab % 4 == 0;
     const int64_t blocks_x = (vocab / 4 + (vocab % 4 ? 6 : 0) + kFlatBlock - 1) / kFlatBlock;
+    // Rows of an odd vocabulary that the caches hold (256 MB of them) stay a workgroup each, two to a CU, where they fill three
+    // quarters of such rounds: memory's order does not matter there, and starting a workgroup for every 4 KB does.  Flat / a
+    // workgroup a row, us: [512 x 32001] to fp16 21.2 / 17.1, [1024 x 16001] to fp32 22.6 / 21.1, in place [512 x 8001] 7.3 / 6.0,
+    // [2048 x 24001] 63.7 / 57.5; but [1024 x 50257] to fp32, 412 MB, 67 / 97, [300 x 32001], 0.59 of a round, 14.4 / 15.7, [2048 x
+    // 3001] to fp16 8.1 / 9.3.  (432 sizes of 3001 to 120001 words: 10028 flat, 9689 by this rule, 9672 by the best of each.)
+    const int64_t round = 512, rounds = (rows + round - 1) / round;
+    const int64_t touched = rows * vocab * (int64_t)(sizeof(float) + ((const void*)logits == (const void*)dlogits ? 0 : sizeof(OUT)));
+    const bool a_row_each = vocab % 4 != 0 && vocab >= 4096 && touched <= 1LL << 28 && 4 * rows >= 3 * rounds * round;
     // (a launch of 2^32 or more work items runs without those beyond, and without an error)
-    if (BR_NLL_BWD_FLAT && aligned && rows <= 65535 && blocks_x <= 0xffffffffLL / kFlatBlock / rows) {
+    if (BR_NLL_BWD_FLAT && aligned && !a_row_each && rows <= 65535 && blocks_x <= 0xffffffffLL / kFlatBlock / rows) {
         const dim3 grid((unsigned)blocks_x, (unsigned)rows);
         if (vocab % 4 == 0) nll_bwd_flat_kernel<OUT, true><<<grid, kFlatBlock, 0, st>>>(logits, target, keep, lse, dlogits, scale, vocab);
         else nll_bwd_flat_kernel<OUT, false><<<grid, kFlatBlock, 0, st>>>(logits, target, keep, lse, dlogits, scale, vocab);

@@ -189,6 +189,34 @@ def test_logsoftmax_nll_of_masked_words(rows, vocab, low):
     assert_close(g, grad / rows, RTOL, "dlogits")
 
 
+@pytest.mark.parametrize("rows,vocab", [(400, 4099), (512, 4097), (1536, 4098), (400, 4095)])   # the last: no workgroup a row
+def test_logsoftmax_nll_gradient_of_many_rows_has_the_bits_of_few(rows, vocab):
+    """Rows of an odd vocabulary, a workgroup each where the caches hold them and they fill the chip, against a quarter of them at a time;
+    to each type and in place, some without a label, the label on first, last and other values."""
+    torch.manual_seed(vocab)
+    logits = 2 * torch.randn((rows, vocab), device="cuda")
+    target = torch.tensor([[0, vocab - 1, vocab // 2, 4, vocab - 4][r % 5] for r in range(rows)], dtype=torch.int32, device="cuda")
+    keep = (torch.arange(rows, device="cuda") % 7 != 3).int()
+    lse = torch.logsumexp(logits, 1)
+    part = rows // 4
+    for code, dtype in ((hip.F32, torch.float32), (hip.F16, torch.float16), (hip.BF16, torch.bfloat16), (hip.F32, None)):
+        print("case rows=%d vocab=%d type=%d in place=%d" % (rows, vocab, code, dtype is None), flush=True)
+        got = []
+        for step in (rows, part):
+            src = logits.clone()
+            out = src if dtype is None else torch.full((rows, vocab), float("nan"), device="cuda", dtype=dtype)
+            for r in range(0, rows, step):
+                call("br_hip_logsoftmax_nll_bwd", ptr(src[r:]), ptr(target[r:]), ptr(keep[r:]), ptr(lse[r:]), ptr(out[r:]), code, 0.25, step, vocab,
+                     stream())
+            torch.cuda.synchronize()
+            got.append(out)
+        assert torch.equal(got[0], got[1])
+        want = torch.softmax(logits.double(), 1)
+        want[torch.arange(rows), target.long()] -= 1
+        want *= 0.25 * keep[:, None]
+        assert ((got[0].double() - want).norm() / want.norm()).item() <= {hip.F32: 1e-6, hip.F16: 2.0 ** -11, hip.BF16: 2.0 ** -8}[code]
+
+
 def test_logsoftmax_nll_headline_shape_properties_and_sampled_rows():
     """logits[2048, 250880] fp32 ~N(0,2), targets uniform, mask Bernoulli(0.9),
     seed 2.  Too large for a full oracle pass in seconds: rows are independent,
