@@ -798,11 +798,12 @@ ComputingReturn hip_gelu_linear_backward(const tensor_t& dy, const tensor_t& u, 
             void* dy16 = ComputingContext::gemm_staging(1, (size_t)(n * out) * 2);
             // Where the products share a launch the column sums are added up beside them, so that the GELU's pass need not own whole
             // columns.  In a step over [1000 x 4096]: 18.7 us with its sums and 35.7 for the products, 13.4 and 38.2 so.  Not where
-            // that pass adds up with fewer roundings: up to 256 rows, and 448 of up to 2048 columns (its narrowest strips), a thread
+            // that pass adds up with fewer roundings: up to 256 rows, and 512 of up to 2048 columns (its narrowest strips), a thread
             // has one position and few waves have any.  Against 64 bits, owned / beside: [2048] from 288 rows 8.5e-8 / 9.3e-8,
-            // from 416 9.3 / 9.4, from 512 9.9 / 9.4; [2304] from 257 9.6 / 9.0, [4096] from 1000 10.3 / 9.8.
+            // from 416 9.3 / 9.4, from 512 9.9 / 9.4; [2304] from 257 9.6 / 9.0, [4096] from 1000 10.3 / 9.8.  With the products, us:
+            // 512 -> 2048 features, 300 rows 13.1 / 13.6, 449 16.8 / 17.0, 600 21.4 / 19.0; 768 -> 3072, 257 rows 20.4 / 19.6.
             br_partial_sums later = {};
-            const bool beside = n > (out > 2048 ? 256 : 448) && br_hip_gemm_pair_kernel(out, in, n, 1, n, in, out, 1, compute) >= 0;
+            const bool beside = n > (out > 2048 ? 256 : 512) && br_hip_gemm_pair_kernel(out, in, n, 1, n, in, out, 1, compute) >= 0;
             int rc = beside ? br_hip_gelu_bwd_cast_sums(static_cast<const float*>(dy->data()), static_cast<const float*>(u->data()),
                                                         static_cast<float*>(du->data()), static_cast<float*>(bias_g->data()), dy16, native,
                                                         n, out, unlift(), &later, ws, need, stream())

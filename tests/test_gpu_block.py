@@ -528,10 +528,10 @@ def test_fused_gelu_backward_linear_backward_equals_the_two_words(runtime, mode)
 
 @pytest.mark.parametrize("weights", ["native", "float"])
 @pytest.mark.parametrize("mode", ["f16", "bf16"])
-@pytest.mark.parametrize("t,hidden,mid,in_place", [(257, 512, 2056, False), (300, 512, 2304, True), (449, 512, 2048, False), (600, 512, 1024, False),
+@pytest.mark.parametrize("t,hidden,mid,in_place", [(257, 512, 2056, False), (300, 512, 2304, True), (513, 512, 2048, False), (600, 512, 1024, False),
                                                    (1000, 256, 1032, False), (1000, 256, 1032, True)])
 def test_fused_gelu_backward_linear_backward_of_many_rows(runtime, t, hidden, mid, in_place, mode, weights):
-    """From 257 rows on (449 of up to 2048 columns) the bias gradient is left as partial sums, which are added up beside the two products, behind the staging of
+    """From 257 rows on (513 of up to 2048 columns) the bias gradient is left as partial sums, which are added up beside the two products, behind the staging of
     x and of fp32 weights; in place, dx lands on the 16-bit x that dW reads, so that the products are two launches and the sums
     one ahead of them.  The products' bits are those of the two words; the bias gradient is within the rounding of its
     additions: of n partial sums of some sqrt(n) values each, four times 2^-24 n rms for the furthest of mid."""
@@ -572,7 +572,7 @@ def test_fused_gelu_backward_linear_backward_of_many_rows(runtime, t, hidden, mi
 
 
 @pytest.mark.parametrize("mode", ["f16", "bf16"])
-@pytest.mark.parametrize("t,hidden,mid", [(256, 512, 4096), (257, 512, 2048), (288, 512, 2048), (448, 512, 2048), (448, 256, 1032)])
+@pytest.mark.parametrize("t,hidden,mid", [(256, 512, 4096), (257, 512, 2048), (288, 512, 2048), (512, 512, 2048), (512, 256, 1032)])
 def test_fused_gelu_backward_linear_backward_of_fewer_rows_owns_its_column_sums(runtime, t, hidden, mid, mode):
     """Where the GELU's pass rounds its column sums less often than partial sums beside the products would, the bias gradient has
     that pass's bits."""
