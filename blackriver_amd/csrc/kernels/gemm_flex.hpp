@@ -317,7 +317,12 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
     const long long a_step = (A_KSTR ? g.lda : 1) * ((long long)kSize * KT * KW);
     const long long b_step = (B_KSTR ? g.ldb : 1) * ((long long)kSize * KT * KW);
     int k_left = k_end - k0;
-    const long long a_far = (long long)kSize * TA::kFar * g.lda, b_far = (long long)kSize * TB::kFar * g.ldb;
+    const unsigned a_far = (unsigned)(kSize * TA::kFar * g.lda), b_far = (unsigned)(kSize * TB::kFar * g.ldb);
+    // (computed ahead of the walk, the sums would take the registers that the held offsets save)
+    auto here = [](unsigned v) {
+        asm volatile("" : "+s"(v));
+        return v;
+    };
     unsigned a_off[TA::kHeld], b_off[TB::kHeld];
 #pragma unroll
     for (int q = 0; q < TA::kHeld; q++) a_off[q] = TA::source_offset(q, lane, g.lda);
@@ -327,22 +332,23 @@ __device__ __forceinline__ void flex_product(const GemmArgs& g, unsigned id, uns
     const unsigned mem0 = (unsigned)(unsigned long long)mem;
 
     auto issue = [&](int stage) {
+        const buffer_rsrc ra = buffer_from(a_src, a_left), rb = buffer_from(b_src, b_left);
         const unsigned dst = mem0 + (unsigned)stage * kStageBytes;
         // a k-contiguous operand's last step: chunks past K are fetched from past the end of the operand
         const bool tail = k_left < KT;
 #pragma unroll
         for (int s = 0; s < TA::kInstr / TA::kHeld; s++) {
-            const buffer_rsrc r = buffer_from(a_src + s * a_far, a_left - s * a_far);
+            const unsigned far = s == 0 ? 0u : here(s * a_far);
 #pragma unroll
             for (int q = 0; q < TA::kHeld; q++)
-                TA::load(dst, s * TA::kHeld + q, !A_KSTR && tail && TA::k_of(q, lane) >= k_left ? kPastEnd : a_off[q], r);
+                TA::load(dst, s * TA::kHeld + q, !A_KSTR && tail && TA::k_of(q, lane) >= k_left ? kPastEnd : a_off[q] + far, ra);
         }
 #pragma unroll
         for (int s = 0; s < TB::kInstr / TB::kHeld; s++) {
-            const buffer_rsrc r = buffer_from(b_src + s * b_far, b_left - s * b_far);
+            const unsigned far = s == 0 ? 0u : here(s * b_far);
 #pragma unroll
             for (int q = 0; q < TB::kHeld; q++)
-                TB::load(dst + TA::kBytes, s * TB::kHeld + q, !B_KSTR && tail && TB::k_of(q, lane) >= k_left ? kPastEnd : b_off[q], r);
+                TB::load(dst + TA::kBytes, s * TB::kHeld + q, !B_KSTR && tail && TB::k_of(q, lane) >= k_left ? kPastEnd : b_off[q] + far, rb);
         }
         a_src += a_step; a_left -= a_step;
         b_src += b_step; b_left -= b_step;
