@@ -157,8 +157,8 @@ inline int flex_kernel(long long m, long long n, long long k, long long batch) {
 
 // fp32 products (gemm_flex.hpp): us = start + steps * max(step, load * workgroups of a CU) + merge * workgroups of a CU, a step
 // being 32 k-values of a wave; a CU that holds one workgroup more than the others sets the time.  Fitted to 80 products of 16 to
-// 4096 rows, each on every tile (median error 4-6 %); choosing by it takes 2140 us for all of them, the best of the measurements
-// 2128, the tiles as they were when matrix instructions of fp32 operands did the products 2697.
+// 4096 rows, each on every tile (median error 4-6 %; operands were split as they are then, which took 3-7 % less on every tile).
+// Choosing by it, 142 other products, 40 of them loaded value by value, take 3686 us, the best of the measurements 3633.
 struct Fp32Cost {
     double start, step, load, merge;
 };
@@ -166,8 +166,8 @@ constexpr Fp32Cost kFp32Cost64{4.21, 1.542, 1.341, 1.62}, kFp32Cost32x64{3.83, 0
 // Waves that walk along K.  Where a CU has at most one workgroup of the small tiles they are eight, two to a SIMD.  Four / eight, us:
 // 32 x 32 tiles, [200 x 768] from 512 7.6 / 6.7, [64 x 2048] from 8192 49 / 37, value by value [31 x 1025] from 1025 12.1 / 9.2;
 // 32 x 64 tiles, [500 x 520] from 512 8.6 / 7.5, 1024 11.8 / 10.7, 2048 20.7 / 16.6, 8192 69.5 / 56.3, [512 x 1024], a workgroup to
-// each CU, 9.4 / 8.8, 13.8 / 12.9, 23.5 / 20.0, 76.5 / 69.9, value by value [333 x 1025] from 1025 17.7 / 13.3.  Below 512 a wave has less
-// than a step; with more tiles than CUs eight are 5-40 % slower.  (The price of 32 x 64 tiles is that of four: no choice among 142
+// each CU, 9.4 / 8.8, 13.8 / 12.9, 23.5 / 20.0, 76.5 / 69.9, value by value [333 x 1025] from 1025 17.7 / 13.3.  Below 512 a wave of
+// eight has one step or two; with more tiles than CUs eight are 5-40 % slower.  (The price of 32 x 64 tiles is that of four: no choice among 142
 // products would be another with eight at 0.8 to 1 of it.)
 constexpr long long kFp32EightWaves = 512;
 inline int fp32_waves(int kernel, long long m, long long n, long long k, long long batch) {
